@@ -440,6 +440,26 @@ int pdw_convblock_bwd(const void *gy, const void *x, const void *a, const void *
                       void *gw_pool, void *gb_pool, void *gw_out, void *gb_out, void *workspace,
                       size_t workspace_bytes, int B, int H, int W, int D, int I, int K, int dtype, void *stream);
 
+/* The two-scale block (scales 1 and s: pooled extents h, w; conv_up without bias) on every shape and type that the
+ * library's dense and convolution kernels cover (fp32, odd extents, pooled sizes that are not exact halves, widths that
+ * are not multiples of 16), as one host call each way; the fused launches of pdw_convblock_* where those cover the
+ * shape.  Covered when pdw_block_supported.  `saved` is one device buffer of pdw_block_saved_bytes that the forward
+ * fills and the backward reads (its layout is the library's own: everything between the two calls is in it); a forward
+ * that no backward follows uses it as its workspace.  x, y, gy, dx[B,H,W,D]; weights and their gradients as for
+ * pdw_convblock_*; dx may be NULL (not wanted), gb_pool and gb_out too.  Status 3: case not covered, nothing launched.
+ * Replaces ConvBlock.forward, conv_block.py:36-49, and its autograd backward. */
+int pdw_block_supported(int B, int H, int W, int h, int w, int D, int I, int K, int dtype);
+size_t pdw_block_saved_bytes(int B, int H, int W, int h, int w, int D, int I, int K, int dtype);
+int pdw_block_fwd(const void *x, const void *w_up, const void *w_dw0, const void *w_dw1, const void *w_pool,
+                  const void *b_pool, const void *w_out, const void *b_out, void *y, void *saved, size_t saved_bytes,
+                  int B, int H, int W, int h, int w, int D, int I, int K, int dtype, void *stream);
+size_t pdw_block_bwd_workspace_bytes(int B, int H, int W, int h, int w, int D, int I, int K, int dtype);
+int pdw_block_bwd(const void *gy, const void *x, const void *saved, const void *w_up, const void *w_dw0,
+                  const void *w_dw1, const void *w_pool, const void *w_out, void *dx, void *gw_up, void *gw_dw0,
+                  void *gw_dw1, void *gw_pool, void *gb_pool, void *gw_out, void *gb_out, void *workspace,
+                  size_t workspace_bytes, int B, int H, int W, int h, int w, int D, int I, int K, int dtype,
+                  void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,4 +1,5 @@
-"""ctypes binding of libpdw.so, the C-ABI library of hand-written gfx950 kernels.
+"""Bindings of libpdw.so, the C-ABI library of hand-written gfx950 kernels: ctypes for every entry point, and the
+extension module whose native host path ``ConvBlock`` and ``OptimizedDepthwiseConv2d`` run.
 
 There is deliberately no fallback: if the library is missing and cannot be built, or a
 tensor is not on a HIP device, the operators raise.
@@ -45,6 +46,11 @@ _SIGS = {
     "pdw_convblock_infer": (c_int, [c_void_p] * 10 + [c_size_t] + [c_int] * 7 + [c_void_p]),
     "pdw_convblock_bwd_workspace_bytes": (c_size_t, [c_int] * 7),
     "pdw_convblock_bwd": (c_int, [c_void_p] * 22 + [c_size_t] + [c_int] * 7 + [c_void_p]),
+    "pdw_block_supported": (c_int, [c_int] * 9),
+    "pdw_block_saved_bytes": (c_size_t, [c_int] * 9),
+    "pdw_block_fwd": (c_int, [c_void_p] * 10 + [c_size_t] + [c_int] * 9 + [c_void_p]),
+    "pdw_block_bwd_workspace_bytes": (c_size_t, [c_int] * 9),
+    "pdw_block_bwd": (c_int, [c_void_p] * 17 + [c_size_t] + [c_int] * 9 + [c_void_p]),
     "pdw_avgpool_fwd": (c_int, [c_void_p] * 2 + [c_int] * 7 + [c_void_p]),
     "pdw_avgpool_bwd": (c_int, [c_void_p] * 2 + [c_int] * 8 + [c_void_p]),
     "pdw_bilinear_fwd": (c_int, [c_void_p] * 2 + [c_int] * 8 + [c_void_p]),
@@ -113,6 +119,24 @@ def lib():
             fn.restype, fn.argtypes = res, args
         _lib = L
     return _lib
+
+
+_ext = None
+
+
+def ext():
+    """The native host path of the operators (csrc/torch_ops.cpp), built beside libpdw.so."""
+    global _ext
+    if _ext is None:
+        lib()
+        if not os.path.exists(os.path.join(_HERE, "_pdw_torch.so")):
+            from . import build as _build
+
+            _build.build()
+        from . import _pdw_torch
+
+        _ext = _pdw_torch
+    return _ext
 
 
 def check(status: int, what: str = "libpdw") -> None:

@@ -3,7 +3,9 @@
     python -m pyramidconvblock_amd.build [--force]
 
 Every csrc/*.hip file is compiled to an object (in parallel) and linked into
-pyramidconvblock_amd/libpdw.so.  hipcc cross-compiles, so no GPU is needed.
+pyramidconvblock_amd/libpdw.so; csrc/torch_ops.cpp (the operators' host path, no device code) is
+compiled with the host compiler against torch's headers and linked to it as the extension module
+pyramidconvblock_amd/_pdw_torch.so.  hipcc cross-compiles, so no GPU is needed.
 With PDW_TUNE_BUILD=1 in the environment of the build the library is compiled with -DPDW_TUNE, which makes
 its planners honour the PDW_* override variables (for experiments; the product build reads no environment).
 """
@@ -19,6 +21,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "csrc", "build")
 LIB = os.path.join(HERE, "libpdw.so")
+EXT = os.path.join(HERE, "_pdw_torch.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = (["-DPDW_TUNE"] if os.environ.get("PDW_TUNE_BUILD") else []) + [
@@ -49,6 +52,28 @@ def _compile(src, headers, force):
     return obj
 
 
+def _build_ext(headers, force):
+    """The host extension: libpdw.so is found beside it ($ORIGIN), torch's libraries are loaded by `import torch`."""
+    import sysconfig
+
+    import torch
+
+    src = os.path.join(CSRC, "torch_ops.cpp")
+    if not (force or _stale(EXT, [src] + headers)):
+        return EXT
+    troot = os.path.dirname(torch.__file__)
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
+           "-D__HIP_PLATFORM_AMD__=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-isystem", os.path.join(troot, "include"), "-isystem", os.path.join(troot, "include/torch/csrc/api/include"),
+           "-isystem", "/opt/rocm/include", "-isystem", sysconfig.get_paths()["include"], src, "-o", EXT,
+           LIB, "-L" + os.path.join(troot, "lib"), "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10", "-lc10_hip",
+           "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("building _pdw_torch.so failed:\n" + r.stderr)
+    return EXT
+
+
 def build(force: bool = False, jobs: int | None = None) -> str:
     os.makedirs(OBJ, exist_ok=True)
     srcs = sorted(glob.glob(os.path.join(CSRC, "*.hip")))
@@ -57,10 +82,11 @@ def build(force: bool = False, jobs: int | None = None) -> str:
     with ThreadPoolExecutor(jobs) as ex:
         objs = list(ex.map(lambda s: _compile(s, headers, force), srcs))
     if force or _stale(LIB, objs):
-        cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-fno-gpu-rdc", "-o", LIB] + objs
+        cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-fno-gpu-rdc", "-Wl,-soname,libpdw.so", "-o", LIB] + objs
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError("link failed:\n" + r.stderr)
+    _build_ext(headers, force)
     return LIB
 
 

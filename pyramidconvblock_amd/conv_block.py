@@ -5,7 +5,10 @@ names, parameter shapes and ``[B,H,W,C]`` in/out contract
 ``state_dict`` keys match the reference: ``conv_up.weight``, ``gates.{i}.conv_spatial.weight``
 (``[k,k,inter_dim]``), ``conv_out.{weight,bias}``, ``conv_pool.{weight,bias}``.
 
-``ConvBlock.forward`` runs as ONE autograd node (``ConvBlockFunction``): the pooling, depthwise
+``ConvBlock.forward`` runs as ONE autograd node: in native code (``csrc/torch_ops.cpp`` over
+``pdw_block_fwd`` / ``_bwd``) for two scales wherever the library's dense layers cover the widths,
+as ``ConvBlockFunction``, the same launches made one by one from Python, for everything else (other
+scale tuples, a bias on ``conv_up``, mixed types).  The pooling, depthwise
 convolutions, gates and upsampling go through libpdw.so, the gate outputs are written straight
 into the halves of the concatenated buffer (no ``torch.cat``), the pooled branch is added in
 place, and the backward reuses one per-image column sum for both bias gradients and the
@@ -68,7 +71,7 @@ class SimpleGate(nn.Module):
 _BMM_FP32_OUT = [True]
 
 # Test hooks (module attributes, never read from the environment): run the block as one Python-level call per
-# launch instead of the library's single call per direction / run conv_up's two gradients as separate launches.
+# launch instead of the native path / run conv_up's two gradients as separate launches there.
 FORCE_STEPWISE = False
 NO_UP_PAIR = False
 
@@ -111,40 +114,11 @@ def _weight_grad(g2d: torch.Tensor, x2d: torch.Tensor, out_dtype=torch.float32) 
     return out
 
 
-def _block_call_ok(x, scales, w_up, b_up, w_out, b_out, w_pool, b_pool, w_dw) -> bool:
-    """Whether pdw_convblock_fwd / _bwd cover this call: scales (1, 1/2), no conv_up bias, everything contiguous and
-    of x's 16-bit dtype, one odd square depthwise filter shape, and shapes the library accepts."""
-    if FORCE_STEPWISE or b_up is not None or tuple(scales) != (1., 0.5) or x.dim() != 4:
-        return False
-    dt = x.dtype
-    tensors = [w_up, w_out, w_pool, *w_dw] + [b for b in (b_out, b_pool) if b is not None]
-    if len(w_dw) != 2 or any(t.dtype != dt or not t.is_contiguous() or t.device != x.device for t in tensors):
-        return False
-    B, H, W, D = x.shape
-    I, K = w_up.shape[0], w_dw[0].shape[0]
-    if (dt not in (torch.float16, torch.bfloat16) or tuple(w_up.shape) != (I, D) or tuple(w_out.shape) != (D, I)
-            or tuple(w_pool.shape) != (D, D) or any(tuple(w.shape) != (K, K, I) for w in w_dw)):
-        return False
-    return bool(_lib.lib().pdw_convblock_supported(B, H, W, D, I, K, _lib.dtype_code(dt)))
-
-
 def convblock_infer(x, w_up, w_out, b_out, w_pool, b_pool, w_dw):
     """Inference forward through pdw_convblock_infer: y only, neither convolution output written to HBM where the
-    fused convolution + gate covers the filter (conv_block.py:36-49 under no_grad).  The caller has checked
-    ``_block_call_ok``."""
-    dev = _lib.require_device(x)
-    B, H, W, D = x.shape
-    I, K = w_up.shape[0], w_dw[0].shape[0]
-    L, code = _lib.lib(), _lib.dtype_code(x.dtype)
-    y = torch.empty((B, H, W, D), device=dev, dtype=x.dtype)
-    ws = torch.empty(L.pdw_convblock_infer_workspace_bytes(B, H, W, D, I, K, code) // 4 + 1, device=dev,
-                     dtype=torch.float32)
-    _lib.check(L.pdw_convblock_infer(x.data_ptr(), w_up.data_ptr(), w_dw[0].data_ptr(), w_dw[1].data_ptr(),
-                                     w_pool.data_ptr(), b_pool.data_ptr() if b_pool is not None else None,
-                                     w_out.data_ptr(), b_out.data_ptr() if b_out is not None else None, y.data_ptr(),
-                                     ws.data_ptr(), ws.numel() * 4, B, H, W, D, I, K, code, _lib.stream_ptr(dev)),
-               "pdw_convblock_infer")
-    return y
+    fused convolution + gate covers the filter (conv_block.py:36-49 under no_grad), for the shapes that
+    pdw_convblock_supported."""
+    return _lib.ext().block_infer(x, w_up, w_out, b_out, w_pool, b_pool, w_dw[0], w_dw[1])
 
 
 def _is_pair(scales) -> bool:
@@ -173,29 +147,6 @@ class ConvBlockFunction(torch.autograd.Function):
         B, H, W, D = x.shape
         dt = x.dtype
         I = w_up.shape[0]
-        ctx.block_call = None
-        if _block_call_ok(x, scales, w_up, b_up, w_out, b_out, w_pool, b_pool, w_dw):
-            # the whole launch sequence below as one call of the library (same kernels, same order, same results)
-            K = w_dw[0].shape[0]
-            L, code = _lib.lib(), _lib.dtype_code(dt)
-            new = lambda *shape: torch.empty(shape, device=dev, dtype=dt)
-            a, c0, cat = new(B, H, W, I), new(B, H, W, I), new(B, H, W, I)
-            xp, c1 = new(B, H // 2, W // 2, I), new(B, H // 2, W // 2, I)
-            m, y = new(B, D), new(B, H, W, D)
-            ws = torch.empty(L.pdw_convblock_fwd_workspace_bytes(B, H, W, D, I, K, code) // 4 + 1, device=dev,
-                             dtype=torch.float32)
-            _lib.check(L.pdw_convblock_fwd(x.data_ptr(), w_up.data_ptr(), w_dw[0].data_ptr(), w_dw[1].data_ptr(),
-                                           w_pool.data_ptr(), b_pool.data_ptr() if b_pool is not None else None,
-                                           w_out.data_ptr(), b_out.data_ptr() if b_out is not None else None,
-                                           a.data_ptr(), c0.data_ptr(), xp.data_ptr(), c1.data_ptr(), cat.data_ptr(),
-                                           m.data_ptr(), y.data_ptr(), ws.data_ptr(), ws.numel() * 4, B, H, W, D, I, K,
-                                           code, _lib.stream_ptr(dev)), "pdw_convblock_fwd")
-            ctx.block_call = (B, H, W, D, I, K, code)
-            ctx.fast = (True, True)
-            ctx.scales = tuple(scales)
-            ctx.has_bias = (False, b_out is not None, b_pool is not None)
-            ctx.save_for_backward(x, a, cat, m, w_up, w_out, w_pool, *w_dw, c0, c1, xp)
-            return y
         fast_up = (ops.dense_supported(D, I, dt) and ops.dense_supported(I, D, dt) and w_up.dtype == dt
                    and (b_up is None or b_up.dtype == dt))
         same_dt = w_pool.dtype == dt and all(b is None or b.dtype == dt for b in (b_pool, b_out))
@@ -316,26 +267,6 @@ class ConvBlockFunction(torch.autograd.Function):
         N = B * H * W
         gy = gy.to(dt).contiguous()
         g2d = gy.view(N, D)
-        if ctx.block_call is not None:
-            dev = gy.device
-            L = _lib.lib()
-            shape = ctx.block_call
-            like = lambda t: torch.empty_like(t, memory_format=torch.contiguous_format)
-            dx, gw_up, gw_out, gw_pool = like(x), like(w_up), like(w_out), like(w_pool)
-            gw_dw = [like(w_dw[0]), like(w_dw[1])]
-            gb_out = torch.empty(D, device=dev, dtype=dt) if ctx.has_bias[1] else None
-            gb_pool = torch.empty(D, device=dev, dtype=dt) if ctx.has_bias[2] else None
-            ws = torch.empty(L.pdw_convblock_bwd_workspace_bytes(*shape) // 4 + 1, device=dev, dtype=torch.float32)
-            _lib.check(L.pdw_convblock_bwd(gy.data_ptr(), x.data_ptr(), a.data_ptr(), convs[0].data_ptr(),
-                                           pooled[1].data_ptr(), convs[1].data_ptr(), cat.data_ptr(), m.data_ptr(),
-                                           w_up.data_ptr(), w_dw[0].data_ptr(), w_dw[1].data_ptr(), w_pool.data_ptr(),
-                                           w_out.data_ptr(), dx.data_ptr(), gw_up.data_ptr(), gw_dw[0].data_ptr(),
-                                           gw_dw[1].data_ptr(), gw_pool.data_ptr(),
-                                           gb_pool.data_ptr() if gb_pool is not None else None, gw_out.data_ptr(),
-                                           gb_out.data_ptr() if gb_out is not None else None, ws.data_ptr(),
-                                           ws.numel() * 4, *shape, _lib.stream_ptr(dev)), "pdw_convblock_bwd")
-            return (dx, None, gw_up, None, gw_out, gb_out, gw_pool, gb_pool, *gw_dw)
-
         fast_up, fast_out = ctx.fast
         pool_fast = w_pool.dtype == dt and B > 0
         # the four weight gradients end in a small summation kernel each: they are run as one launch at the end
@@ -476,16 +407,15 @@ class ConvBlock(nn.Module):
         if x.dim() != 4 or x.shape[3] != self.conv_up.in_features:
             raise ValueError(f"expected [B,H,W,{self.conv_up.in_features}] input, got {tuple(x.shape)}")
         scales = tuple(float(g.scale_factor) for g in self.gates)
-        if not (torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in self.parameters()))):
-            # nothing to save for a backward: the inference form of the block, where the library covers the shape
-            xc = x.detach().contiguous()
-            args = (self.conv_up.weight.detach(), self.conv_up.bias, self.conv_out.weight.detach(),
-                    None if self.conv_out.bias is None else self.conv_out.bias.detach(), self.conv_pool.weight.detach(),
-                    None if self.conv_pool.bias is None else self.conv_pool.bias.detach(),
-                    [g.conv_spatial.weight.detach() for g in self.gates])
-            if _block_call_ok(xc, scales, *args):
-                with _lib.launch_scope(_lib.require_device(xc)):
-                    return convblock_infer(xc, args[0], args[2], args[3], args[4], args[5], args[6])
+        up, out, pool = self.conv_up, self.conv_out, self.conv_pool
+        if len(scales) == 2 and not FORCE_STEPWISE:
+            # two scales: the whole pass in native code (csrc/torch_ops.cpp), where the library's block calls cover it
+            w_dw = [g.conv_spatial.weight for g in self.gates]
+            y = _lib.ext().block(x, up.weight, up.bias, out.weight, out.bias, pool.weight, pool.bias, *w_dw, *scales)
+            if y is True:   # nothing to save for a backward, and the inference form of the block covers the shape
+                return convblock_infer(x, up.weight, out.weight, out.bias, pool.weight, pool.bias, w_dw)
+            if y is not None:
+                return y
         return ConvBlockFunction.apply(x, scales, self.conv_up.weight, self.conv_up.bias, self.conv_out.weight,
                                        self.conv_out.bias, self.conv_pool.weight, self.conv_pool.bias,
                                        *[g.conv_spatial.weight for g in self.gates])

@@ -1,0 +1,287 @@
+// The two-scale pyramid block of conv_block.py:25-49 (scales 1 and s) on any extents, widths and types that the
+// library's kernels cover, as one host call each way: what pdw_convblock_* is for the shapes of its fused launches,
+// for every other shape (fp32, odd extents, pooled sizes that are not exact halves, widths beyond 128).  Where
+// pdw_convblock_supported, these calls are those.  Everything the backward reads lies in one buffer of the caller, so a
+// binding keeps one tensor per pass.  Host code only: a launch sequence of the library's own entry points, chosen from
+// the arguments.
+#include <stdint.h>
+
+#include "../../include/pdw.h"
+#include "common.h"
+#include "kernels.h"
+
+namespace {
+
+using namespace pdw;
+
+size_t up256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+// Hands out 256-byte aligned pieces of a buffer; with a null base it only counts.
+struct Carver {
+    char* base;
+    size_t used = 0;
+    void* take(size_t bytes) {
+        void* r = base ? base + used : nullptr;
+        used += up256(bytes);
+        return r;
+    }
+};
+
+struct Shape {
+    int B, H, W, h, w, D, I, K, dtype, es, P;
+    long long N, n;       // pixels at full and at the pooled resolution
+    bool exact;           // the pooled extents are exact halves
+    bool single;          // the fused launches of pdw_convblock_* take it
+};
+
+Shape shape_of(int B, int H, int W, int h, int w, int D, int I, int K, int dtype) {
+    Shape s{B, H, W, h, w, D, I, K, dtype, dtype == kF32 ? 4 : 2, H * W, (long long)B * H * W, (long long)B * h * w, false, false};
+    s.exact = H == 2 * h && W == 2 * w;
+    s.single = s.exact && pdw_convblock_supported(B, H, W, D, I, K, dtype) != 0;
+    return s;
+}
+
+bool layer_ok(int K, int NO, int dtype) { return pdw_dense_supported(K, NO, dtype) != 0; }
+
+// What the forward leaves for the backward, then what only the forward needs.
+struct Saved {
+    void *a, *c0, *cat, *xp, *c1, *m;
+    float *xparts, *yp;
+    void* ws;
+    size_t ws_bytes, bytes;
+};
+
+Saved saved_layout(const Shape& s, void* base) {
+    Carver c{(char*)base};
+    Saved r{};
+    const size_t full = (size_t)s.N * s.I * s.es, half = (size_t)s.n * s.I * s.es;
+    r.a = c.take(full), r.c0 = c.take(full), r.cat = c.take(full);
+    r.xp = c.take(half), r.c1 = c.take(half);
+    r.m = c.take((size_t)s.B * s.D * s.es);
+    r.xparts = (float*)c.take((size_t)((s.N + 31) / 32) * s.D * 4);
+    r.yp = (float*)c.take((size_t)s.B * s.D * 4);   // (behind xparts: the workspace of pdw_convblock_fwd)
+    r.ws_bytes = up256(pdw_pool_branch_workspace_bytes(s.B, s.P, s.D));
+    r.ws = c.take(r.ws_bytes);
+    r.bytes = c.used;
+    return r;
+}
+
+struct BwdWork {
+    void *dcat, *gcf, *gch, *dxp, *da, *gbias;
+    float *gparts, *dmean;
+    void *ws_po, *ws_pool, *ws_w0, *ws_w1, *ws_pu;
+    size_t b_po, b_pool, b_w0, b_w1, b_pu, bytes;
+};
+
+BwdWork bwd_layout(const Shape& s, void* base) {
+    Carver c{(char*)base};
+    BwdWork r{};
+    const size_t full = (size_t)s.N * s.I * s.es, half = (size_t)s.n * s.I * s.es;
+    const int pad = s.K / 2;
+    r.dcat = c.take(full), r.gcf = c.take(full), r.da = c.take(full);
+    r.gch = c.take(half), r.dxp = c.take(half);
+    r.gbias = c.take((size_t)2 * s.D * s.es);
+    r.gparts = (float*)c.take((size_t)((s.N + 31) / 32) * s.D * 4);
+    r.dmean = (float*)c.take((size_t)s.B * s.D * 4);
+    r.b_po = up256(pdw_dense_wgrad_workspace_bytes(s.N, s.D, s.I)), r.ws_po = c.take(r.b_po);
+    r.b_pool = up256(pdw_pool_branch_workspace_bytes(s.B, s.P, s.D)), r.ws_pool = c.take(r.b_pool);
+    r.b_w0 = up256(pdw_dwconv_wgrad_workspace_bytes(s.B, s.H, s.W, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, s.dtype));
+    r.ws_w0 = c.take(r.b_w0);
+    r.b_w1 = up256(pdw_dwconv_wgrad_workspace_bytes(s.B, s.h, s.w, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, s.dtype));
+    r.ws_w1 = c.take(r.b_w1);
+    r.b_pu = up256(pdw_dense_wgrad_workspace_bytes(s.N, s.I, s.D)), r.ws_pu = c.take(r.b_pu);
+    r.bytes = c.used;
+    return r;
+}
+
+bool rows_whole_tiles(const Shape& s) { return s.P % pdw_dense_colsum_rows() == 0; }
+
+int forward(const Shape& s, const Saved& v, const void* x, const void* w_up, const void* w_dw0, const void* w_dw1,
+            const void* w_pool, const void* b_pool, const void* w_out, const void* b_out, void* y, void* stream) {
+    const int pad = s.K / 2, dt = s.dtype;
+    const bool two = s.exact && dt != kF32 && pdw_dwconv_fwd2_supported(s.B, s.H, s.W, s.I, s.K, dt);
+    // conv_up, where its kernel can with the sums of x per row tile (for the mean branch) and the 2x2 pool of its result
+    const float* parts = nullptr;
+    int nparts = 0;
+    bool pooled = false;
+    if (two) {
+        const int r = pdw_dense_fwd_colsum_pool(x, w_up, nullptr, v.a, v.xparts, v.xp, s.B, s.H, s.W, s.D, s.I, dt, stream);
+        if (r != 0 && r != 3) return r;
+        pooled = r == 0;
+    }
+    if (pooled) {
+        parts = v.xparts, nparts = s.P / 32;
+    } else if (rows_whole_tiles(s) && pdw_dense_colsum_supported(s.D, s.I, dt)) {
+        if (int e = pdw_dense_fwd_colsum(x, w_up, 0, nullptr, nullptr, v.a, v.xparts, s.N, s.D, s.I, s.P, dt, stream)) return e;
+        parts = v.xparts, nparts = s.P / pdw_dense_colsum_rows();
+    } else if (int e = pdw_dense_fwd(x, w_up, 0, nullptr, nullptr, v.a, s.N, s.D, s.I, s.P, dt, stream)) {
+        return e;
+    }
+    // the convolutions of both scales                                                         (conv_block.py:14-17)
+    bool convs = false, mean = false;
+    if (two) {
+        if (!pooled)
+            if (int e = pdw_avgpool_fwd(v.a, v.xp, s.B, s.H, s.W, s.I, s.h, s.w, dt, stream)) return e;
+        int r = 3;
+        if (parts) {
+            r = pdw_dwconv_fwd2_mean(v.a, w_dw0, v.c0, 0, 0, v.xp, w_dw1, v.c1, 0, 0, s.B, s.H, s.W, s.I, s.K, parts, nparts,
+                                     w_pool, b_pool, b_out, v.m, v.yp, s.P, s.D, dt, stream);
+            mean = r == 0;
+        }
+        if (r == 3) r = pdw_dwconv_fwd2(v.a, w_dw0, v.c0, v.xp, w_dw1, v.c1, s.B, s.H, s.W, s.I, s.K, dt, stream);
+        if (r != 0 && r != 3) return r;
+        convs = r == 0;
+        if (!convs)
+            if (int e = pdw_dwconv_fwd(v.a, w_dw0, v.c0, s.B, s.H, s.W, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, dt, stream)) return e;
+    } else if (int e = pdw_dwconv_fwd_pool(v.a, w_dw0, v.c0, v.xp, s.B, s.H, s.W, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, s.h,
+                                           s.w, dt, stream)) {
+        return e;
+    }
+    if (!convs)
+        if (int e = pdw_dwconv_fwd(v.xp, w_dw1, v.c1, s.B, s.h, s.w, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, dt, stream)) return e;
+    // both gates and the resize into the concatenation, the mean branch's row per image, conv_out (conv_block.py:18-21, 40-49)
+    if (mean) {
+        const int r = pdw_dense_fwd_gated(v.c0, v.c1, v.cat, w_out, nullptr, v.yp, y, s.B, s.H, s.W, s.I, s.D, 0, dt, stream);
+        if (r != 3) return r;
+        if (int e = pdw_gate_pair_fwd(v.c0, v.c1, v.cat, s.B, s.H, s.W, s.h, s.w, s.I, s.I, dt, stream)) return e;
+    } else if (parts) {
+        if (int e = pdw_block_mid_fwd(v.c0, v.c1, v.cat, s.B, s.H, s.W, s.h, s.w, s.I, s.I, parts, nparts, w_pool, b_pool,
+                                      b_out, v.m, v.yp, s.P, s.D, dt, stream))
+            return e;
+    } else {
+        if (int e = pdw_gate_pair_fwd(v.c0, v.c1, v.cat, s.B, s.H, s.W, s.h, s.w, s.I, s.I, dt, stream)) return e;
+        if (int e = pdw_pool_branch_fwd(x, w_pool, b_pool, b_out, v.m, v.yp, v.ws, v.ws_bytes, s.B, s.P, s.D, dt, stream)) return e;
+    }
+    return pdw_dense_fwd(v.cat, w_out, 0, nullptr, v.yp, y, s.N, s.I, s.D, s.P, dt, stream);
+}
+
+int backward(const Shape& s, const Saved& v, const BwdWork& g, const void* gy, const void* x, const void* w_up,
+             const void* w_dw0, const void* w_dw1, const void* w_pool, const void* w_out, void* dx, void* gw_up,
+             void* gw_dw0, void* gw_dw1, void* gw_pool, void* gb_pool, void* gw_out, void* gb_out, void* stream) {
+    const int pad = s.K / 2, dt = s.dtype;
+    // conv_out: gradient of the concatenation and of the weight, with the sums of gy per row tile where the kernel can
+    const bool colsum = rows_whole_tiles(s) && pdw_dense_colsum_supported(s.D, s.I, dt);
+    const bool pair_cs = colsum && pdw_dense_bwd_pair_colsum_supported(s.D, s.I, dt);
+    float* gparts = nullptr;
+    if (pair_cs || pdw_dense_bwd_pair_supported(s.D, s.I, dt)) {
+        if (pair_cs) gparts = g.gparts;
+        if (int e = pdw_dense_bwd_pair(gy, w_out, v.cat, g.dcat, gparts, gw_out, g.ws_po, g.b_po, nullptr, 1, s.N, s.D, s.I, dt, stream))
+            return e;
+    } else {
+        if (colsum) {
+            gparts = g.gparts;
+            if (int e = pdw_dense_fwd_colsum(gy, w_out, 1, nullptr, nullptr, g.dcat, gparts, s.N, s.D, s.I, 1, dt, stream)) return e;
+        } else if (int e = pdw_dense_fwd(gy, w_out, 1, nullptr, nullptr, g.dcat, s.N, s.D, s.I, 1, dt, stream)) {
+            return e;
+        }
+        if (int e = pdw_dense_wgrad(gy, v.cat, gw_out, g.ws_po, g.b_po, s.N, s.D, s.I, dt, stream)) return e;
+    }
+    // the gates and the mean branch
+    void* gb0 = gb_out ? gb_out : g.gbias;
+    void* gb1 = gb_pool ? gb_pool : (char*)g.gbias + (size_t)s.D * s.es;
+    const int nparts = s.P / pdw_dense_colsum_rows();
+    if (gparts && s.exact && s.h >= 2 && s.w >= 2) {
+        if (int e = pdw_block_mid_bwd(g.dcat, v.c0, v.c1, g.gcf, g.gch, s.B, s.H, s.W, s.h, s.w, s.I, s.I, gparts, nparts, v.m,
+                                      w_pool, gb0, gb1, gw_pool, g.dmean, g.ws_pool, g.b_pool, s.P, s.D, dt, stream))
+            return e;
+    } else {
+        if (gparts) {
+            if (int e = pdw_pool_branch_bwd_parts(gparts, nparts, v.m, w_pool, gb0, gb1, gw_pool, g.dmean, g.ws_pool, g.b_pool,
+                                                  s.B, s.P, s.D, dt, stream))
+                return e;
+        } else if (int e = pdw_pool_branch_bwd(gy, v.m, w_pool, gb0, gb1, gw_pool, g.dmean, g.ws_pool, g.b_pool, s.B, s.P, s.D,
+                                               dt, stream)) {
+            return e;
+        }
+        if (int e = pdw_gate_pair_bwd(g.dcat, v.c0, v.c1, g.gcf, g.gch, s.B, s.H, s.W, s.h, s.w, s.I, s.I, dt, stream)) return e;
+    }
+    // the convolutions: the pooled scale's input gradient, then the rest (one launch where that is covered)
+    if (int e = pdw_dwconv_dgrad(g.gch, w_dw1, g.dxp, s.B, s.h, s.w, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, dt, stream)) return e;
+    int r = 3;
+    if (s.exact && dt != kF32) {
+        r = pdw_dwconv_bwd3(g.gcf, w_dw0, g.dxp, g.da, v.a, gw_dw0, g.ws_w0, g.b_w0, v.xp, g.gch, gw_dw1, g.ws_w1, g.b_w1, s.B,
+                            s.H, s.W, s.I, s.K, dt, stream);
+        if (r != 0 && r != 3) return r;
+    }
+    if (r == 3) {
+        if (int e = pdw_dwconv_wgrad_pair(v.a, g.gcf, gw_dw0, g.ws_w0, g.b_w0, s.H, s.W, v.xp, g.gch, gw_dw1, g.ws_w1, g.b_w1,
+                                          s.h, s.w, s.B, s.I, s.K, dt, stream))
+            return e;
+        if (int e = pdw_dwconv_dgrad_addpool(g.gcf, w_dw0, g.dxp, g.da, s.B, s.H, s.W, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, s.h,
+                                             s.w, dt, stream))
+            return e;
+    }
+    // conv_up: input gradient (plus the mean branch's per-image term) and weight gradient
+    if (dx && s.P >= 32 && pdw_dense_bwd_pair_supported(s.I, s.D, dt))
+        return pdw_dense_bwd_pair(g.da, w_up, x, dx, nullptr, gw_up, g.ws_pu, g.b_pu, g.dmean, s.P, s.N, s.I, s.D, dt, stream);
+    if (int e = pdw_dense_wgrad(g.da, x, gw_up, g.ws_pu, g.b_pu, s.N, s.I, s.D, dt, stream)) return e;
+    if (!dx) return 0;
+    // (the summations recorded so far ride in the last kernel of the pass)
+    return pdw_dense_fwd_flush(g.da, w_up, 1, nullptr, g.dmean, dx, s.N, s.I, s.D, s.P, dt, stream);
+}
+
+}  // namespace
+
+extern "C" {
+
+int pdw_block_supported(int B, int H, int W, int h, int w, int D, int I, int K, int dtype) {
+    if (dtype != kF32 && dtype != kF16 && dtype != kBF16) return 0;
+    if (B < 1 || H < 1 || W < 1 || h < 1 || w < 1 || K < 1 || !(K & 1) || D < 4 || I < 4 || (I & 1)) return 0;
+    if ((long long)B * H * W * (D > I ? D : I) > 0x7fffffffLL || (long long)H * h > 0x7fffffffLL) return 0;
+    if ((long long)B * h * w * I > 0x7fffffffLL) return 0;
+    return layer_ok(D, I, dtype) && layer_ok(I, D, dtype) ? 1 : 0;
+}
+
+size_t pdw_block_saved_bytes(int B, int H, int W, int h, int w, int D, int I, int K, int dtype) {
+    if (!pdw_block_supported(B, H, W, h, w, D, I, K, dtype)) return 0;
+    return saved_layout(shape_of(B, H, W, h, w, D, I, K, dtype), nullptr).bytes;
+}
+
+int pdw_block_fwd(const void* x, const void* w_up, const void* w_dw0, const void* w_dw1, const void* w_pool,
+                  const void* b_pool, const void* w_out, const void* b_out, void* y, void* saved, size_t saved_bytes, int B,
+                  int H, int W, int h, int w, int D, int I, int K, int dtype, void* stream) {
+    if (!pdw_block_supported(B, H, W, h, w, D, I, K, dtype))
+        return set_error("pdw_block_fwd: case not covered (B=%d H=%d W=%d h=%d w=%d D=%d I=%d K=%d dtype=%d)", B, H, W, h, w, D,
+                         I, K, dtype), 3;
+    for (const void* p : {x, w_up, w_dw0, w_dw1, w_pool, w_out, (const void*)y, (const void*)saved})
+        if (!p) return set_error("pdw_block_fwd: null pointer"), 1;
+    const Shape s = shape_of(B, H, W, h, w, D, I, K, dtype);
+    const Saved v = saved_layout(s, saved);
+    if (saved_bytes < v.bytes)
+        return set_error("pdw_block_fwd: buffer of %zu bytes given, %zu needed", saved_bytes, v.bytes), 1;
+    if (s.single)
+        return pdw_convblock_fwd(x, w_up, w_dw0, w_dw1, w_pool, b_pool, w_out, b_out, v.a, v.c0, v.xp, v.c1, v.cat, v.m, y,
+                                 v.xparts, (size_t)((char*)v.ws - (char*)v.xparts), B, H, W, D, I, K, dtype, stream);
+    return forward(s, v, x, w_up, w_dw0, w_dw1, w_pool, b_pool, w_out, b_out, y, stream);
+}
+
+size_t pdw_block_bwd_workspace_bytes(int B, int H, int W, int h, int w, int D, int I, int K, int dtype) {
+    if (!pdw_block_supported(B, H, W, h, w, D, I, K, dtype)) return 0;
+    const Shape s = shape_of(B, H, W, h, w, D, I, K, dtype);
+    return bwd_layout(s, nullptr).bytes;
+}
+
+int pdw_block_bwd(const void* gy, const void* x, const void* saved, const void* w_up, const void* w_dw0, const void* w_dw1,
+                  const void* w_pool, const void* w_out, void* dx, void* gw_up, void* gw_dw0, void* gw_dw1, void* gw_pool,
+                  void* gb_pool, void* gw_out, void* gb_out, void* workspace, size_t workspace_bytes, int B, int H, int W,
+                  int h, int w, int D, int I, int K, int dtype, void* stream) {
+    if (!pdw_block_supported(B, H, W, h, w, D, I, K, dtype))
+        return set_error("pdw_block_bwd: case not covered (B=%d H=%d W=%d h=%d w=%d D=%d I=%d K=%d dtype=%d)", B, H, W, h, w, D,
+                         I, K, dtype), 3;
+    for (const void* p : {gy, x, saved, w_up, w_dw0, w_dw1, w_pool, w_out, (const void*)gw_up, (const void*)gw_dw0,
+                          (const void*)gw_dw1, (const void*)gw_pool, (const void*)gw_out, (const void*)workspace})
+        if (!p) return set_error("pdw_block_bwd: null pointer"), 1;
+    const Shape s = shape_of(B, H, W, h, w, D, I, K, dtype);
+    const Saved v = saved_layout(s, const_cast<void*>(saved));
+    const BwdWork g = bwd_layout(s, workspace);
+    if (workspace_bytes < g.bytes)
+        return set_error("pdw_block_bwd: workspace of %zu bytes given, %zu needed", workspace_bytes, g.bytes), 1;
+    // the final summations of all weight gradients run as one launch at the end of the pass
+    if (int e = pdw_reduce_defer_begin()) return e;
+    const int e = backward(s, v, g, gy, x, w_up, w_dw0, w_dw1, w_pool, w_out, dx, gw_up, gw_dw0, gw_dw1, gw_pool, gb_pool,
+                           gw_out, gb_out, stream);
+    const int f = pdw_reduce_defer_flush(stream);   // also ends the deferral after an error
+    return e ? e : f;
+}
+
+}  // extern "C"

@@ -1,0 +1,335 @@
+// The operators' host path in native code: allocation of results, argument checks, autograd nodes and the calls of
+// libpdw.so for ConvBlock and OptimizedDepthwiseConv2d.  From Python, with torch.autograd.Function and ctypes, one
+// training step of a block cost 250-900 us of host time (one interpreter-level call per launch, 10-20 us each, where the
+// library's kernels run 3-30 us each); a Node here is entered by the autograd engine without the interpreter lock.
+// Plain C++ (no device code): built with the host compiler against torch's headers and linked to libpdw.so beside it.
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/autograd/saved_variable.h>
+
+#include "../../include/pdw.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+
+int dtype_code(at::ScalarType t) {
+    switch (t) {
+        case at::kFloat: return PDW_F32;
+        case at::kHalf: return PDW_F16;
+        case at::kBFloat16: return PDW_BF16;
+        default: return -1;
+    }
+}
+
+void check(int status, const char* what) {
+    TORCH_CHECK(status == 0, what, ": ", pdw_last_error(), " (status ", status, ")");
+}
+
+void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+// Contiguous and 16-byte aligned (the kernels move 16-byte pieces; a view at an odd storage offset is copied).
+Tensor dense(const Tensor& t) {
+    Tensor c = t.is_contiguous() ? t : t.contiguous();
+    return reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 == 0 ? c : c.clone(at::MemoryFormat::Contiguous);
+}
+
+void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+
+Tensor bytes(size_t n, const Tensor& like) { return at::empty({(int64_t)n}, like.options().dtype(at::kByte)); }
+
+// ---------------------------------------------------------------------------------------------------------------
+// The block
+
+struct BlockShape {
+    int B, H, W, h, w, D, I, K, dtype;
+};
+
+#define PDW_SHAPE(s) (s).B, (s).H, (s).W, (s).h, (s).w, (s).D, (s).I, (s).K, (s).dtype
+
+enum { kX, kUp, kOut, kBOut, kPool, kBPool, kDw0, kDw1, kBlockInputs };   // order of a block's differentiable inputs
+
+struct BlockNode : public torch::autograd::Node {
+    SavedVariable x, w_up, w_out, w_pool, w_dw0, w_dw1, saved;
+    BlockShape s;
+    bool has_b_out, has_b_pool;
+
+    std::string name() const override { return "ConvBlockBackward"; }
+
+    void release_variables() override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        for (SavedVariable* v : {&x, &w_up, &w_out, &w_pool, &w_dw0, &w_dw1, &saved}) v->reset_data();
+    }
+
+    variable_list apply(variable_list&& grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        variable_list out(kBlockInputs);
+        if (!grads[0].defined()) return out;
+        at::AutoDispatchBelowADInplaceOrView below;
+        auto take = [&](const SavedVariable& v) { return dense(v.unpack(shared_from_this())); };
+        const Tensor xs = take(x), wu = take(w_up), wo = take(w_out), wp = take(w_pool), d0 = take(w_dw0), d1 = take(w_dw1);
+        const Tensor keep = saved.unpack(shared_from_this());
+        const Tensor gy = dense(grads[0].to(xs.scalar_type()));
+        const c10::DeviceGuard guard(xs.device());
+        auto like = [](const Tensor& t) { return at::empty(t.sizes(), t.options()); };
+        if (task_should_compute_output(kX)) out[kX] = like(xs);
+        out[kUp] = like(wu), out[kOut] = like(wo), out[kPool] = like(wp), out[kDw0] = like(d0), out[kDw1] = like(d1);
+        if (has_b_out) out[kBOut] = at::empty({s.D}, xs.options());
+        if (has_b_pool) out[kBPool] = at::empty({s.D}, xs.options());
+        const Tensor ws = bytes(pdw_block_bwd_workspace_bytes(PDW_SHAPE(s)), xs);
+        check(pdw_block_bwd(ptr(gy), ptr(xs), ptr(keep), ptr(wu), ptr(d0), ptr(d1), ptr(wp), ptr(wo), ptr(out[kX]),
+                            ptr(out[kUp]), ptr(out[kDw0]), ptr(out[kDw1]), ptr(out[kPool]), ptr(out[kBPool]),
+                            ptr(out[kOut]), ptr(out[kBOut]), ptr(ws), ws.numel(), PDW_SHAPE(s), stream_of(xs)),
+              "pdw_block_bwd");
+        return out;
+    }
+};
+
+// Whether the library's block calls take this: everything on x's device in x's type, conv_up without bias, two square
+// odd filters of one shape, and extents and widths that pdw_block_supported.
+bool block_shape(const Tensor* in, const Tensor& b_up, double s0, double s1, BlockShape* s) {
+    const Tensor& x = in[kX];
+    if (b_up.defined() || s0 != 1.0 || s1 == 1.0 || x.dim() != 4 || !x.is_cuda()) return false;
+    const int dt = dtype_code(x.scalar_type());
+    if (dt < 0) return false;
+    for (int i = 1; i < kBlockInputs; ++i)
+        if (in[i].defined() && (in[i].scalar_type() != x.scalar_type() || in[i].device() != x.device())) return false;
+    const Tensor &up = in[kUp], &out = in[kOut], &pool = in[kPool], &d0 = in[kDw0], &d1 = in[kDw1];
+    if (up.dim() != 2 || out.dim() != 2 || pool.dim() != 2 || d0.dim() != 3 || d0.sizes() != d1.sizes()) return false;
+    const int64_t D = x.size(3), I = up.size(0), K = d0.size(0);
+    if (up.size(1) != D || d0.size(1) != K || d0.size(2) != I || out.size(0) != D || out.size(1) != I || (I & 1) ||
+        pool.size(0) != D || pool.size(1) != D)
+        return false;
+    for (int64_t e : x.sizes())
+        if (e > 0x7fffffff) return false;
+    const int H = (int)x.size(1), W = (int)x.size(2);
+    *s = {(int)x.size(0), H, W, (int)(H * s1), (int)(W * s1), (int)D, (int)I, (int)K, dt};
+    return pdw_block_supported(PDW_SHAPE(*s)) != 0;
+}
+
+Tensor block_train_or_infer(const Tensor* in, const BlockShape& s, bool grad) {
+    const c10::DeviceGuard guard(in[kX].device());
+    Tensor d[kBlockInputs], y, saved;
+    std::shared_ptr<BlockNode> node;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        for (int i = 0; i < kBlockInputs; ++i)
+            if (in[i].defined()) d[i] = dense(in[i]);
+        y = at::empty(d[kX].sizes(), d[kX].options());
+        saved = bytes(pdw_block_saved_bytes(PDW_SHAPE(s)), d[kX]);
+        check(pdw_block_fwd(ptr(d[kX]), ptr(d[kUp]), ptr(d[kDw0]), ptr(d[kDw1]), ptr(d[kPool]), ptr(d[kBPool]),
+                            ptr(d[kOut]), ptr(d[kBOut]), ptr(y), ptr(saved), saved.numel(), PDW_SHAPE(s), stream_of(y)),
+              "pdw_block_fwd");
+    }
+    if (grad) {
+        node = std::shared_ptr<BlockNode>(new BlockNode(), torch::autograd::deleteNode);
+        node->set_next_edges(torch::autograd::collect_next_edges(in[kX], in[kUp], in[kOut], in[kBOut], in[kPool],
+                                                                 in[kBPool], in[kDw0], in[kDw1]));
+        // (the input itself where it went to the kernels as it is, so that a later change of it in place is noticed)
+        auto save = [&](int i) { return SavedVariable(d[i].is_same(in[i]) ? in[i] : d[i], false); };
+        node->x = save(kX), node->w_up = save(kUp), node->w_out = save(kOut), node->w_pool = save(kPool);
+        node->w_dw0 = save(kDw0), node->w_dw1 = save(kDw1), node->saved = SavedVariable(saved, false);
+        node->s = s, node->has_b_out = in[kBOut].defined(), node->has_b_pool = in[kBPool].defined();
+        torch::autograd::set_history(y, node);
+    }
+    return y;
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// The depthwise convolution
+
+struct ConvGeo {
+    int sh, sw, ph, pw, dh, dw;
+};
+
+#define PDW_CONV(x, w, g)                                                                                         \
+    (int)(x)[0], (int)(x)[1], (int)(x)[2], (int)(x)[3], (int)(w)[0], (int)(w)[1], (g).sh, (g).sw, (g).ph, (g).pw, \
+        (g).dh, (g).dw
+
+struct ConvNode : public torch::autograd::Node {
+    SavedVariable x, w;
+    ConvGeo g;
+    at::ScalarType x_type;
+
+    std::string name() const override { return "DepthwiseConv2DBackward"; }
+
+    void release_variables() override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        x.reset_data(), w.reset_data();
+    }
+
+    variable_list apply(variable_list&& grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        variable_list out(2);
+        if (!grads[0].defined()) return out;
+        at::AutoDispatchBelowADInplaceOrView below;
+        const Tensor wd = dense(w.unpack(shared_from_this()));
+        const Tensor xd = dense(x.unpack(shared_from_this()).to(wd.scalar_type()));
+        const Tensor gy = dense(grads[0].to(wd.scalar_type()));
+        const c10::DeviceGuard guard(xd.device());
+        const int dt = dtype_code(wd.scalar_type());
+        void* const stream = stream_of(xd);
+        const auto xs = xd.sizes(), ws = wd.sizes();
+        const bool empty = xd.numel() == 0 || gy.numel() == 0;
+        if (task_should_compute_output(0)) {
+            Tensor dx = at::empty(xs, xd.options());
+            if (empty)
+                dx.zero_();
+            else
+                check(pdw_dwconv_dgrad(ptr(gy), ptr(wd), ptr(dx), PDW_CONV(xs, ws, g), dt, stream), "pdw_dwconv_dgrad");
+            out[0] = dx.to(x_type);
+        }
+        if (task_should_compute_output(1)) {
+            Tensor dw = at::empty(ws, wd.options());
+            if (empty) {
+                dw.zero_();
+            } else {
+                const Tensor work = bytes(pdw_dwconv_wgrad_workspace_bytes(PDW_CONV(xs, ws, g), dt) + 4, xd);
+                check(pdw_dwconv_wgrad(ptr(xd), ptr(gy), ptr(dw), ptr(work), work.numel(), PDW_CONV(xs, ws, g), dt, stream),
+                      "pdw_dwconv_wgrad");
+            }
+            out[1] = dw;
+        }
+        return out;
+    }
+};
+
+Tensor conv_forward(const Tensor& x, const Tensor& w, const ConvGeo& g) {
+    TORCH_CHECK_VALUE(x.dim() == 4 && w.dim() == 3 && x.size(3) == w.size(2),
+                      "expected input [B,H,W,C] and weight [k1,k2,C], got ", x.sizes(), " and ", w.sizes());
+    TORCH_CHECK(x.is_cuda() && w.is_cuda(), "pyramid dwconv kernels run on a HIP device only (tensor is on ",
+                (x.is_cuda() ? w : x).device(), "); there is no CPU path");
+    TORCH_CHECK(x.device() == w.device(), "tensors on different devices: ", x.device(), " vs ", w.device());
+    TORCH_CHECK_TYPE(dtype_code(w.scalar_type()) >= 0, "pyramid dwconv kernels support float32/float16/bfloat16, got ",
+                     w.scalar_type());
+    const c10::DeviceGuard guard(x.device());
+    const bool grad = at::GradMode::is_enabled() && (x.requires_grad() || w.requires_grad());
+    Tensor y, xc;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        xc = x.scalar_type() == w.scalar_type() ? x : x.to(w.scalar_type());
+        const Tensor xd = dense(xc), wd = dense(w);
+        const auto xs = xd.sizes(), ws = wd.sizes();
+        const int oh = pdw_conv_out_size((int)xs[1], (int)ws[0], g.sh, g.ph, g.dh);
+        const int ow = pdw_conv_out_size((int)xs[2], (int)ws[1], g.sw, g.pw, g.dw);
+        y = at::empty({xs[0], oh, ow, xs[3]}, xd.options());
+        if (y.numel())
+            check(pdw_dwconv_fwd(ptr(xd), ptr(wd), ptr(y), PDW_CONV(xs, ws, g), dtype_code(wd.scalar_type()), stream_of(xd)),
+                  "pdw_dwconv_fwd");
+    }
+    if (grad) {
+        auto node = std::shared_ptr<ConvNode>(new ConvNode(), torch::autograd::deleteNode);
+        node->set_next_edges(torch::autograd::collect_next_edges(x, w));
+        node->x = SavedVariable(xc, false), node->w = SavedVariable(w, false);
+        node->g = g, node->x_type = x.scalar_type();
+        torch::autograd::set_history(y, node);
+    }
+    return y;
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// Python entry points
+
+bool tensor_arg(PyObject* o, Tensor* t) {
+    if (o == Py_None) return true;
+    if (!THPVariable_Check(o)) {
+        PyErr_Format(PyExc_TypeError, "expected a Tensor or None, got %s", Py_TYPE(o)->tp_name);
+        return false;
+    }
+    *t = THPVariable_Unpack(o);
+    return true;
+}
+
+// block(x, w_up, b_up, w_out, b_out, w_pool, b_pool, w_dw0, w_dw1, s0, s1): the block's output; None where the library's
+// block calls do not cover the case; True where no gradient is wanted and its inference call (block_infer) covers it.
+PyObject* py_block(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    TORCH_CHECK(n == 11, "block: 11 arguments expected");
+    Tensor in[kBlockInputs], b_up;
+    Tensor* const slot[9] = {&in[kX], &in[kUp], &b_up, &in[kOut], &in[kBOut], &in[kPool], &in[kBPool], &in[kDw0], &in[kDw1]};
+    for (int i = 0; i < 9; ++i)
+        if (!tensor_arg(args[i], slot[i])) return nullptr;
+    const double s0 = PyFloat_AsDouble(args[9]), s1 = PyFloat_AsDouble(args[10]);
+    if (PyErr_Occurred()) return nullptr;
+    BlockShape s;
+    if (!block_shape(in, b_up, s0, s1, &s)) Py_RETURN_NONE;
+    bool grad = false;
+    if (at::GradMode::is_enabled())
+        for (const Tensor& t : in) grad = grad || (t.defined() && t.requires_grad());
+    if (!grad && s.H == 2 * s.h && s.W == 2 * s.w && pdw_convblock_supported(s.B, s.H, s.W, s.D, s.I, s.K, s.dtype))
+        Py_RETURN_TRUE;
+    Tensor y;
+    {
+        pybind11::gil_scoped_release no_gil;
+        y = block_train_or_infer(in, s, grad);
+    }
+    return THPVariable_Wrap(std::move(y));
+    END_HANDLE_TH_ERRORS
+}
+
+// block_infer(x, w_up, w_out, b_out, w_pool, b_pool, w_dw0, w_dw1): pdw_convblock_infer (the caller has asked block()).
+PyObject* py_block_infer(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    TORCH_CHECK(n == kBlockInputs, "block_infer: 8 arguments expected");
+    Tensor in[kBlockInputs];
+    for (int i = 0; i < kBlockInputs; ++i) {
+        if (!tensor_arg(args[i], &in[i])) return nullptr;
+    }
+    Tensor y;
+    {
+        pybind11::gil_scoped_release no_gil;
+        at::AutoDispatchBelowADInplaceOrView below;
+        const c10::DeviceGuard guard(in[kX].device());
+        for (Tensor& t : in)
+            if (t.defined()) t = dense(t);
+        const Tensor& x = in[kX];
+        const int B = x.size(0), H = x.size(1), W = x.size(2), D = x.size(3), I = in[kUp].size(0), K = in[kDw0].size(0);
+        const int dt = dtype_code(x.scalar_type());
+        y = at::empty(x.sizes(), x.options());
+        const Tensor ws = bytes(pdw_convblock_infer_workspace_bytes(B, H, W, D, I, K, dt), x);
+        check(pdw_convblock_infer(ptr(x), ptr(in[kUp]), ptr(in[kDw0]), ptr(in[kDw1]), ptr(in[kPool]), ptr(in[kBPool]),
+                                  ptr(in[kOut]), ptr(in[kBOut]), ptr(y), ptr(ws), ws.numel(), B, H, W, D, I, K, dt, stream_of(x)),
+              "pdw_convblock_infer");
+    }
+    return THPVariable_Wrap(std::move(y));
+    END_HANDLE_TH_ERRORS
+}
+
+// dwconv(x, w, (sh, sw), (ph, pw), (dh, dw))
+PyObject* py_dwconv(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    TORCH_CHECK(n == 5, "dwconv: 5 arguments expected");
+    Tensor x, w;
+    if (!tensor_arg(args[0], &x) || !tensor_arg(args[1], &w)) return nullptr;
+    int v[6];
+    for (int i = 0; i < 3; ++i)
+        if (!PyArg_ParseTuple(args[2 + i], "ii", &v[2 * i], &v[2 * i + 1])) return nullptr;
+    Tensor y;
+    {
+        pybind11::gil_scoped_release no_gil;
+        y = conv_forward(x, w, {v[0], v[1], v[2], v[3], v[4], v[5]});
+    }
+    return THPVariable_Wrap(std::move(y));
+    END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef kMethods[] = {
+    {"block", (PyCFunction)(void (*)(void))py_block, METH_FASTCALL, nullptr},
+    {"block_infer", (PyCFunction)(void (*)(void))py_block_infer, METH_FASTCALL, nullptr},
+    {"dwconv", (PyCFunction)(void (*)(void))py_dwconv, METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_pdw_torch", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__pdw_torch(void) { return PyModule_Create(&kModule); }

@@ -1,0 +1,63 @@
+"""The native host path of the operators (csrc/torch_ops.cpp) at the edges of what autograd may ask of it."""
+import pytest
+import torch
+
+from parity import assert_close, randn
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dim,k,shape,dtype", [
+    (128, 13, (2, 24, 32, 128), torch.bfloat16),    # the fused launches
+    (64, 7, (2, 13, 18, 64), torch.float32),        # the general sequence, pooled size not an exact half
+    (200, 9, (1, 9, 7, 200), torch.float16),
+])
+def test_block_node_partial_gradients(oracle, dim, k, shape, dtype):
+    """An input without gradient, frozen parameters, views as parameters and inputs, a second backward."""
+    import pyramid_dwconv
+
+    torch.manual_seed(7)
+    m = pyramid_dwconv.ConvBlock(dim=dim, kernel_size=k).to(dtype)
+    gen = torch.Generator().manual_seed(7)
+    x, g = randn(gen, *shape).to(dtype), randn(gen, *shape).to(dtype)
+    params = {n: p.detach().double().numpy() for n, p in m.state_dict().items()}
+    yo, cache = oracle.convblock_fwd(x.double().numpy(), params)
+    dxo, go = oracle.convblock_bwd(cache, g.double().numpy())
+    m = m.cuda()
+    m.conv_pool.weight.requires_grad_(False)
+    base = torch.zeros(dim * dim + 1, dtype=dtype, device="cuda")      # conv_up's weight at an odd storage offset
+    base[1:1 + m.conv_up.weight.numel()] = m.conv_up.weight.detach().flatten()
+    m.conv_up.weight = torch.nn.Parameter(base[1:1 + m.conv_up.weight.numel()].view_as(m.conv_up.weight))
+    xd = x.cuda().transpose(1, 2).contiguous().transpose(1, 2)           # not contiguous, no gradient
+    y = m(xd)
+    assert_close(y, yo, dtype, "y")
+    torch.autograd.backward(y, g.cuda(), retain_graph=True)
+    first = {n: p.grad.clone() for n, p in m.named_parameters() if p.grad is not None}
+    assert set(first) == set(go) - {"conv_pool.weight"}
+    for n, v in first.items():
+        assert_close(v, go[n], dtype, "grad " + n)
+    torch.autograd.backward(y, g.cuda())                                 # the kept graph once more: same bits, added
+    for n, p in m.named_parameters():
+        if p.grad is not None:
+            assert torch.equal(p.grad, first[n] + first[n]), n
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.backward(y, g.cuda())
+    xd = xd.requires_grad_()
+    y = m(xd)
+    torch.autograd.backward(y, g.cuda())
+    assert_close(xd.grad, dxo, dtype, "dx")
+
+
+def test_changed_in_place_is_noticed():
+    import pyramid_dwconv
+    import pyramidconvblock_amd
+
+    m = pyramid_dwconv.ConvBlock(dim=64, kernel_size=5).bfloat16().cuda()
+    conv = pyramidconvblock_amd.OptimizedDepthwiseConv2d(64, 5, padding=2).bfloat16().cuda()
+    x = torch.randn(1, 8, 8, 64, device="cuda").bfloat16().requires_grad_()
+    for layer, w in ((m, m.conv_up.weight), (conv, conv.weight)):
+        y = layer(x)
+        with torch.no_grad():
+            w.add_(1)
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            y.sum().backward()
