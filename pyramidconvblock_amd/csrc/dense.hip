@@ -992,8 +992,11 @@ static bool dense_dims_ok(int K, int NO, int dtype) {
     return dtype != kF32 && K >= 8 && K <= 16 * kKT && K % 8 == 0 && NO >= 8 && NO <= 32 * kNT && NO % 8 == 0;
 }
 
-// (the tiled kernels of this file, or the one-tile-per-wavefront kernels of dense_any.hip: fp32, other widths)
-int dense_rows_supported(int K, int NO, int dtype) { return (dense_dims_ok(K, NO, dtype) || dense_any_dims_ok(K, NO)) ? 1 : 0; }
+// (the tiled kernels of this file, the 128 x 128 tiles of dense_wide.hip beyond their widths, or the
+// one-tile-per-wavefront kernels of dense_any.hip: fp32, widths off multiples of 8)
+int dense_rows_supported(int K, int NO, int dtype) {
+    return (dense_dims_ok(K, NO, dtype) || dense_wide_ok(K, NO, dtype) || dense_any_dims_ok(K, NO)) ? 1 : 0;
+}
 
 int dense_colsum_rows() { return 32; }
 
@@ -1005,9 +1008,12 @@ int dense_rows_launch(const void* x, const void* w, int w_kmajor, const void* bi
     if (!dense_dims_ok(K, NO, dtype)) {
         // fp32 and the widths the tiled kernels do not take: no tile sums there, and summations that were to ride
         // in this launch get one of their own
-        if (colsum || !dense_any_dims_ok(K, NO)) return -1;
+        if (colsum || !dense_rows_supported(K, NO, dtype)) return -1;
         if (rider)
             if (int e = reduce_jobs_launch(*rider, s)) return e;
+        // (wide against any, 16-bit, us: [10431,200] -> 112 7.0 / 12.7, [50000,256] -> 128 9.7 / 24)
+        const int r = dense_wide_rows_launch(x, w, w_kmajor, bias, rowbias, y, N, K, NO, P, dtype, s);
+        if (r != -1) return r;
         return dense_any_rows_launch(x, w, w_kmajor, bias, rowbias, y, N, K, NO, P, dtype, s);
     }
     if (rider && colsum) return -1;
@@ -1210,13 +1216,22 @@ static bool dense_wgrad_tiled_ok(int M, int NO, int dtype) {
 }
 
 int dense_wgrad_supported(int M, int NO, int dtype) {
-    return (dense_wgrad_tiled_ok(M, NO, dtype) || dense_any_wgrad_dims_ok(M, NO)) ? 1 : 0;
+    return (dense_wgrad_tiled_ok(M, NO, dtype) || dense_wide_ok(M, NO, dtype) || dense_any_wgrad_dims_ok(M, NO)) ? 1 : 0;
+}
+
+// Partials that the tiled and the any-width kernels may leave: one per workgroup of the plan, fewer where each is large
+// (widths beyond 256, where 256 partials would be hundreds of megabytes).
+static int dense_wgrad_parts(long long N, int M, int NO) {
+    int blocks, spb;
+    dense_wgrad_plan(N, &blocks, &spb);
+    if (M <= 256 && NO <= 256) return blocks;
+    const long long most = ((long long)64 << 20) / ((long long)M * NO * (long long)sizeof(float));
+    return most < 1 ? 1 : most < blocks ? (int)most : blocks;
 }
 
 size_t dense_wgrad_workspace(long long N, int M, int NO) {
-    int blocks, spb;
-    dense_wgrad_plan(N, &blocks, &spb);
-    return (size_t)blocks * M * NO * sizeof(float);
+    const size_t wide = dense_wide_wgrad_workspace(N, M, NO), rest = (size_t)dense_wgrad_parts(N, M, NO) * M * NO * sizeof(float);
+    return wide > rest ? wide : rest;
 }
 
 template <typename T, int MT, int NT, bool EXACT>
@@ -1255,9 +1270,9 @@ static int dense_wgrad_t(const void* a, const void* b, void* dw, void* ws, long 
 int dense_wgrad_launch(const void* a, const void* b, void* dw, void* ws, long long N, int M, int NO, int dtype,
                        hipStream_t s) {
     if (!dense_wgrad_tiled_ok(M, NO, dtype)) {   // fp32, other widths: at most as many partials as the workspace holds
-        int blocks, spb;
-        dense_wgrad_plan(N, &blocks, &spb);
-        return dense_any_wgrad_launch(a, b, dw, ws, N, M, NO, dtype, blocks, s);
+        const int r = dense_wide_wgrad_launch(a, b, dw, ws, N, M, NO, dtype, s);
+        if (r != -1) return r;
+        return dense_any_wgrad_launch(a, b, dw, ws, N, M, NO, dtype, dense_wgrad_parts(N, M, NO), s);
     }
     if ((reinterpret_cast<uintptr_t>(a) & 15) || (reinterpret_cast<uintptr_t>(b) & 15)) return -1;
     if (dtype == kF16) return dense_wgrad_t<f16_t>(a, b, dw, ws, N, M, NO, s);

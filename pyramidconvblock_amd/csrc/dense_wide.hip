@@ -1,0 +1,321 @@
+// Dense layers of wide blocks (16-bit types, widths that are multiples of 8): all three products of an nn.Linear on
+// tiles of 128 x 128 (or 64) results, the products of conv_block.py:37, 44 for any dim.
+//
+//   rows:   Y[n,o]  = sum_k X[n,k] W(o,k) + bias[o] + rowbias[n / P][o]     (W stored [o][k], or [k][o] for the input gradient)
+//   wgrad:  dW[m,o] = sum_n A[n,m] B[n,o]                                    (fp32 partials over row ranges)
+//
+// What bounds it: the matrix pipe from a width of about 600 on, HBM below.  A stage is 64 values of the inner dimension
+// of both operands, moved by the direct global-to-LDS loads (16 bytes a lane, no registers in between) into one of two
+// buffers while the other is multiplied; one barrier a stage.  Operands whose inner dimension is not the contiguous one
+// (both of the weight gradient, the weight of the input gradient) are staged as they lie and read with
+// ds_read_b64_tr_b16, which hands every lane four values down a column, so there is no transposing pass over memory and
+// no byte shuffling.  The 16-byte pieces of a staged row are permuted by the row (the loads' lanes choose the global piece,
+// since their LDS side is fixed to lane order), so that the fragment reads of both kinds fall on all 64 banks once.
+// Measured (bf16, us; in brackets the library product it replaces): [16384,1152] -> 576 35 (34), its input gradient 35
+// (48), its weight gradient 32 + its share of the summation (a batched product over 128 slabs and their sum: 160 + 150).
+// Out-of-range rows, columns and the inner tail read as zero through the buffer descriptors; nothing is branched around.
+#include <stdint.h>
+
+#include "common.h"
+#include "kernels.h"
+#include "reduce_parts.h"
+#include "tile_common.h"
+
+namespace pdw {
+
+namespace {
+
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef short v4s __attribute__((ext_vector_type(4)));
+typedef short v8s __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) char lds_char;
+
+constexpr int kBK = 64;                     // inner values per stage
+constexpr uint32_t kPast = 0x80000000u;     // an offset past the end of any descriptor used here
+
+__device__ __forceinline__ v16f mfma(v8s a, v8s b, v16f c, bf16_t) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ v16f mfma(v8s a, v8s b, v16f c, f16_t) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, b), c, 0, 0, 0);
+}
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
+}
+
+// One operand of a tile: R results wide, kBK inner values per stage, staged by the workgroup's 256 threads.
+// TR = false: stored [result][inner] (pitch ld): LDS rows of 64 values, 8 pieces each, piece c of row r at c ^ (r / 2 % 8).
+// TR = true: stored [inner][result]: LDS rows of R values; pieces moved in groups of four (64 bytes) by the row, so that the
+// four rows that a transposing read takes together lie on different banks.
+template <int R, bool TR>
+struct Operand {
+    static constexpr int NL = R * kBK / 8 / 256;     // loads per thread and stage
+    static constexpr int CPR = TR ? R / 8 : 8;       // pieces per LDS row
+    static constexpr int BYTES = R * kBK * 2;
+    __amdgpu_buffer_rsrc_t rsrc;
+    uint32_t off[NL];
+    int kc[NL];          // first inner value of the piece (TR: its row)
+    uint32_t step;       // bytes per stage
+
+    static __device__ __forceinline__ int swz(int row, int c) {
+        if constexpr (!TR) return c ^ ((row >> 1) & 7);
+        else if constexpr (R == 128) return c ^ (4 * (row & 3));
+        else return c ^ (4 * ((row >> 1) & 1));
+    }
+    // r0: first result; nres: results of the whole operand; inner values [kb, ke)
+    __device__ __forceinline__ void init(const char* p, int ld, long long r0, long long nres, long long kb, long long ke) {
+        const int tid = threadIdx.x;
+        if constexpr (!TR) {
+            const long long rows = nres - r0 < R ? nres - r0 : R;
+            rsrc = rsrc_of(p + (r0 * ld + kb) * 2, (uint32_t)((rows - 1) * ld + (ke - kb)) * 2);
+            step = kBK * 2;
+        } else {
+            rsrc = rsrc_of(p + (kb * ld + r0) * 2, (uint32_t)((ke - kb - 1) * ld + (nres - r0)) * 2);
+            step = (uint32_t)ld * kBK * 2;
+        }
+#pragma unroll
+        for (int j = 0; j < NL; ++j) {
+            const int slot = j * 256 + tid, row = slot / CPR, c = swz(row, slot % CPR);
+            if constexpr (!TR) {
+                kc[j] = c * 8;
+                off[j] = r0 + row < nres ? (uint32_t)(row * ld + c * 8) * 2 : kPast;
+            } else {
+                kc[j] = row;
+                off[j] = r0 + c * 8 < nres ? (uint32_t)(row * ld + c * 8) * 2 : kPast;
+            }
+        }
+    }
+    // requests stage `st` (inner values left from its start: left) into buf
+    __device__ __forceinline__ void request(lds_char* buf, int st, int left) const {
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+#pragma unroll
+        for (int j = 0; j < NL; ++j) {
+            const uint32_t o = kc[j] < left ? off[j] + (uint32_t)st * step : kPast;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(buf + (j * 256 + wave * 64) * 16),
+                                                     16, (int)o, 0, 0, 0);
+        }
+    }
+    // this lane's 8 inner values (16 kk + 8 (lane / 32) ..) of result 32 t + lane % 32
+    static __device__ __forceinline__ v8s frag(const lds_char* buf, int t, int kk, int lane) {
+        if constexpr (!TR) {
+            const int row = 32 * t + (lane & 31), c = swz(row, 2 * kk + (lane >> 5));
+            return *(const __attribute__((address_space(3))) v8s*)(buf + row * 128 + c * 16);
+        } else {
+            const int g = lane >> 4, i = lane & 15;
+            const int col = 32 * t + 16 * (g & 1) + 4 * (i & 3);
+            v4s h[2];
+#pragma unroll
+            for (int hh = 0; hh < 2; ++hh) {
+                const int row = 16 * kk + 8 * (g >> 1) + 4 * hh + (i >> 2);
+                h[hh] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (__attribute__((address_space(3))) v4s*)(buf + row * (R * 2) + swz(row, col >> 3) * 16 + (col & 7) * 2));
+            }
+            return __builtin_shufflevector(h[0], h[1], 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+    }
+};
+
+struct WideArgs {
+    const void *a, *b, *bias;
+    const float* rowbias;
+    void* y;              // T, or the fp32 partials
+    long long M, Kd;      // results along a; inner extent
+    int N, lda, ldb, P;   // results along b
+    int mt, nt, splits;
+    long long kper;       // inner values per split (a multiple of kBK)
+};
+
+// Results [M][N] = sum over k of a(m,k) b(n,k).  The b operand is the matrix instruction's first, so that a lane holds
+// four consecutive n of one m.  Wavefronts 2 x 2 over the tile.
+template <typename T, int BM, int BN, bool TA, bool TB, bool PART>
+__global__ __launch_bounds__(256, 2) void wide_gemm_k(WideArgs g) {
+    typedef Operand<BM, TA> OpA;
+    typedef Operand<BN, TB> OpB;
+    constexpr int STAGE = OpA::BYTES + OpB::BYTES;
+    constexpr int FM = BM / 64, FN = BN / 64;   // 32-result fragments per wavefront
+    extern __shared__ __align__(16) char dsm[];
+    lds_char* const sm = (lds_char*)dsm;
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave & 1, wn = wave >> 1;
+    // tiles of one row range next to each other on one XCD: they read the same rows
+    int id = xcd_remap(blockIdx.x, gridDim.x);
+    const int tn = id % g.nt;
+    id /= g.nt;
+    const int tm = id % g.mt, sp = id / g.mt;
+    const long long m0 = (long long)tm * BM;
+    const int n0 = tn * BN;
+    const long long kb = sp * g.kper, ke = kb + g.kper < g.Kd ? kb + g.kper : g.Kd;
+    OpA a;
+    OpB b;
+    a.init((const char*)g.a, g.lda, m0, g.M, kb, ke);
+    b.init((const char*)g.b, g.ldb, n0, g.N, kb, ke);
+    const int left = (int)(ke - kb), nst = (left + kBK - 1) / kBK;
+    v16f acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    a.request(sm, 0, left);
+    b.request(sm + OpA::BYTES, 0, left);
+    for (int st = 0; st < nst; ++st) {
+        lds_char* const cur = sm + (st & 1) * STAGE;
+        lds_char* const nxt = sm + ((st & 1) ^ 1) * STAGE;
+        // this stage has arrived, and every wavefront is done with the buffer that the next one goes to
+        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+        // all fragments of the stage first, then the next stage's requests, then the products: an LDS read behind a
+        // request in program order would wait for it (the compiler cannot tell the two buffers apart)
+        v8s fa[kBK / 16][FM], fb[kBK / 16][FN];
+#pragma unroll
+        for (int kk = 0; kk < kBK / 16; ++kk) {
+#pragma unroll
+            for (int i = 0; i < FM; ++i) fa[kk][i] = OpA::frag(cur, wm * FM + i, kk, lane);
+#pragma unroll
+            for (int j = 0; j < FN; ++j) fb[kk][j] = OpB::frag(cur + OpA::BYTES, wn * FN + j, kk, lane);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (st + 1 < nst) {
+            a.request(nxt, st + 1, left - (st + 1) * kBK);
+            b.request(nxt + OpA::BYTES, st + 1, left - (st + 1) * kBK);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int kk = 0; kk < kBK / 16; ++kk)
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j) acc[i][j] = mfma(fb[kk][j], fa[kk][i], acc[i][j], T());
+    }
+    if constexpr (PART) {
+        float* const out = (float*)g.y + (size_t)sp * g.M * g.N;
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+            const long long m = m0 + (wm * FM + i) * 32 + l32;
+            if (m >= g.M) continue;
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int n = n0 + (wn * FN + j) * 32 + 8 * q + 4 * h;
+                    if (n < g.N)
+                        *reinterpret_cast<float4*>(out + m * g.N + n) =
+                            make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+                }
+        }
+    } else {
+        // bias and per-image row in fp32, then through LDS so that the stores are whole 16-byte pieces in order
+        constexpr int TP = BN + 8;
+        __syncthreads();
+        T* const tile = reinterpret_cast<T*>(dsm);
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+            const int mr = (wm * FM + i) * 32 + l32;
+            const long long m = m0 + mr < g.M ? m0 + mr : g.M - 1;
+            const float* const rb = g.rowbias ? g.rowbias + (size_t)((uint32_t)m / (uint32_t)g.P) * g.N : nullptr;
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int nr = (wn * FN + j) * 32 + 8 * q + 4 * h, n = n0 + nr < g.N ? n0 + nr : 0;
+                    float v[4] = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+                    float add[4] = {0.f, 0.f, 0.f, 0.f};
+                    if (g.bias) load_f32<T, 4>((const T*)g.bias + n, add);
+                    if (rb) {
+                        const float4 t = *reinterpret_cast<const float4*>(rb + n);
+                        add[0] += t.x, add[1] += t.y, add[2] += t.z, add[3] += t.w;
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] += add[e];
+                    store_f32<T, 4>(tile + mr * TP + nr, v);
+                }
+        }
+        __syncthreads();
+        constexpr int CPR = BN / 8;
+#pragma unroll
+        for (int j = 0; j < BM * CPR / 256; ++j) {
+            const int s = j * 256 + tid, row = s / CPR, c = s % CPR;
+            if (m0 + row < g.M && n0 + c * 8 < g.N)
+                *reinterpret_cast<uint4*>((T*)g.y + (m0 + row) * g.N + n0 + c * 8) =
+                    *reinterpret_cast<const uint4*>(tile + row * TP + c * 8);
+        }
+    }
+}
+
+template <typename T, int BM, int BN, bool TA, bool TB, bool PART>
+int wide_go(const WideArgs& g, hipStream_t s) {
+    constexpr size_t stages = (size_t)2 * (BM + BN) * kBK * 2, out = PART ? 0 : (size_t)BM * (BN + 8) * 2;
+    constexpr size_t lds = stages > out ? stages : out;
+    hipLaunchKernelGGL((wide_gemm_k<T, BM, BN, TA, TB, PART>), dim3((unsigned)(g.mt * g.nt * g.splits)), dim3(256), lds, s, g);
+    return check_launch("wide_gemm");
+}
+
+// Tiles and row ranges of the weight gradient: tiles of 64 where a width is no more than that, and enough ranges for
+// two workgroups on every compute unit, of at least four stages each, whose partials (written and read once more in
+// fp32) are not more traffic than the operands.
+struct WgradPlan {
+    int bm, bn, mt, nt, splits;
+    long long kper;
+};
+WgradPlan wgrad_plan(long long N, int M, int NO) {
+    WgradPlan p{M <= 64 ? 64 : 128, NO <= 64 ? 64 : 128, 0, 0, 0, 0};
+    p.mt = cdiv(M, p.bm), p.nt = cdiv(NO, p.bn);
+    long long s = 512 / ((long long)p.mt * p.nt);
+    const long long by_rows = N / (4 * kBK), by_traffic = N * (M + NO) / (4LL * M * NO);
+    if (s > by_rows) s = by_rows;
+    if (s > by_traffic) s = by_traffic;
+    if (s < 1) s = 1;
+    p.kper = ((N + s - 1) / s + kBK - 1) / kBK * kBK;
+    p.splits = (int)((N + p.kper - 1) / p.kper);
+    return p;
+}
+
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+}  // namespace
+
+bool dense_wide_ok(int K, int NO, int dtype) { return dtype != kF32 && K >= 8 && NO >= 8 && K % 8 == 0 && NO % 8 == 0; }
+
+// -1: not covered (widths, alignment, offsets of 2^31 bytes within a tile or a weight).
+int dense_wide_rows_launch(const void* x, const void* w, int w_kmajor, const void* bias, const float* rowbias, void* y,
+                           long long N, int K, int NO, int P, int dtype, hipStream_t s) {
+    if (!dense_wide_ok(K, NO, dtype) || N > 0x7fffffffLL || (long long)K * NO * 2 > 0x7fffffffLL || K > (1 << 22) || NO > (1 << 22))
+        return -1;
+    if (!aligned16(x) || !aligned16(w) || !aligned16(y) || !aligned16(rowbias) || (reinterpret_cast<uintptr_t>(bias) & 7)) return -1;
+    if (N == 0) return 0;
+    WideArgs g{x, w, bias, rowbias, y, N, K, NO, K, w_kmajor ? NO : K, P > 0 ? P : 1, 0, 0, 1, (long long)cdiv(K, kBK) * kBK};
+    // tiles of 64 rows where 128-row tiles would leave compute units without work
+    const bool small = (long long)cdiv(N, 128) * cdiv(NO, 128) < 256;
+    const int bm = small ? 64 : 128, bn = NO <= 64 ? 64 : 128;
+    g.mt = cdiv(N, bm), g.nt = cdiv(NO, bn);
+#define PDW_WIDE_T(T, BM, BN) (w_kmajor ? wide_go<T, BM, BN, false, true, false>(g, s) : wide_go<T, BM, BN, false, false, false>(g, s))
+#define PDW_WIDE(BM, BN) (dtype == kF16 ? PDW_WIDE_T(f16_t, BM, BN) : PDW_WIDE_T(bf16_t, BM, BN))
+    if (bm == 64) return bn == 64 ? PDW_WIDE(64, 64) : PDW_WIDE(64, 128);
+    return bn == 64 ? PDW_WIDE(128, 64) : PDW_WIDE(128, 128);
+#undef PDW_WIDE
+#undef PDW_WIDE_T
+}
+
+size_t dense_wide_wgrad_workspace(long long N, int M, int NO) {
+    return N < 1 || M < 1 || NO < 1 ? 0 : (size_t)wgrad_plan(N, M, NO).splits * M * NO * sizeof(float);
+}
+
+int dense_wide_wgrad_launch(const void* a, const void* b, void* dw, void* ws, long long N, int M, int NO, int dtype, hipStream_t s) {
+    if (!dense_wide_ok(M, NO, dtype) || N < 1 || !aligned16(a) || !aligned16(b) || !aligned16(ws)) return -1;
+    const WgradPlan p = wgrad_plan(N, M, NO);
+    if (p.kper * (M > NO ? M : NO) * 2 > 0x7fffffffLL) return -1;
+    WideArgs g{a, b, nullptr, nullptr, ws, M, N, NO, M, NO, 1, p.mt, p.nt, p.splits, p.kper};
+#define PDW_WIDE_W(BM, BN) \
+    (dtype == kF16 ? wide_go<f16_t, BM, BN, true, true, true>(g, s) : wide_go<bf16_t, BM, BN, true, true, true>(g, s))
+    const int e = p.bm == 64 ? (p.bn == 64 ? PDW_WIDE_W(64, 64) : PDW_WIDE_W(64, 128))
+                             : (p.bn == 64 ? PDW_WIDE_W(128, 64) : PDW_WIDE_W(128, 128));
+#undef PDW_WIDE_W
+    if (e) return e;
+    if (dtype == kF16) return wgrad_reduce_launch<f16_t>((const float*)ws, dw, p.splits, M * NO, s);
+    return wgrad_reduce_launch<bf16_t>((const float*)ws, dw, p.splits, M * NO, s);
+}
+
+}  // namespace pdw

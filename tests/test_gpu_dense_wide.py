@@ -1,0 +1,28 @@
+"""The 128 x 128-tile dense kernels (csrc/dense_wide.hip: 16-bit layers wider than 128) against float64, at the edges of
+their tiles, stages and row ranges."""
+import pytest
+import torch
+
+from parity import assert_close, randn
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K,NO", [(136, 8), (8, 264), (200, 112), (256, 128), (520, 264), (64, 192), (1152, 576)])
+@pytest.mark.parametrize("N,P", [(1, 1), (63, 7), (130, 65), (1000, 250), (4097, 4097)])
+def test_dense_wide_layers(dtype, K, NO, N, P):
+    from pyramidconvblock_amd import ops
+
+    assert ops.dense_supported(K, NO, dtype) and ops.dense_supported(NO, K, dtype)
+    gen = torch.Generator().manual_seed(K + NO + N)
+    x, g = randn(gen, N, K).to(dtype), randn(gen, N, NO).to(dtype)
+    w, b = (randn(gen, NO, K) / K ** 0.5).to(dtype), randn(gen, NO).to(dtype)
+    rb = randn(gen, (N + P - 1) // P, NO)
+    y = ops.dense_forward(x.cuda(), w.cuda(), bias=b.cuda(), rowbias=rb.cuda(), rows_per_image=P)
+    ref = x.double() @ w.double().t() + b.double() + rb.double().repeat_interleave(P, 0)[:N]
+    assert_close(y, ref.numpy(), dtype, "forward", 0.5)
+    dx = ops.dense_forward(g.cuda(), w.cuda(), w_kmajor=True)
+    assert_close(dx, (g.double() @ w.double()).numpy(), dtype, "input gradient", 0.5)
+    dw = ops.dense_wgrad(g.cuda(), x.cuda())
+    assert_close(dw, (g.double().t() @ x.double()).numpy(), dtype, "weight gradient", 0.5)
