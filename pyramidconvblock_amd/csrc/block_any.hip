@@ -2,8 +2,14 @@
 // library's kernels cover, as one host call each way: what pdw_convblock_* is for the shapes of its fused launches,
 // for every other shape (fp32, odd extents, pooled sizes that are not exact halves, widths beyond 128).  Where
 // pdw_convblock_supported, these calls are those.  Everything the backward reads lies in one buffer of the caller, so a
-// binding keeps one tensor per pass.  Host code only: a launch sequence of the library's own entry points, chosen from
-// the arguments.
+// binding keeps one tensor per pass.  A launch sequence of the library's own entry points, chosen from the arguments.
+//
+// 16-bit blocks whose inner width I is not a multiple of 8 run on channels padded with zeros: both halves of the
+// inner channels are laid out G = I / 2 rounded up to 8 wide, so that the matrix-core convolutions (slices of 8 or 16
+// channels), the 128 x 128 dense tiles and the 16-byte gate kernels take them; the vector-ALU kernels that take the
+// widths as they are cost two to five times as much ([34,55,55,168], filter 15: 693 us for a training step, 1.14 times
+// the channels on the matrix cores 230).  The weights are packed into that layout by one launch per forward, and the summations
+// of the weight gradients leave the padding out again.
 #include <stdint.h>
 
 #include "../../include/pdw.h"
@@ -28,24 +34,84 @@ struct Carver {
 };
 
 struct Shape {
-    int B, H, W, h, w, D, I, K, dtype, es, P;
+    int B, H, W, h, w, D, I, K, dtype, es, P;   // I: the inner channels as they are laid out
+    int G, Gp;            // width of a gate, and of a half of the inner channels
     long long N, n;       // pixels at full and at the pooled resolution
     bool exact;           // the pooled extents are exact halves
     bool single;          // the fused launches of pdw_convblock_* take it
+    bool padded() const { return Gp != G; }
+    int gw() const { return padded() ? G : 0; }
 };
 
+// Width of a half of the inner channels.  Inner widths that are multiples of 8 run as they are: the convolutions and the
+// dense tiles take them, and the packing launch and the padding would cost more than 8-byte instead of 16-byte gates (108
+// against 101 us for a training step at [41,16,17,80]).  So do tensors small enough for the packing launch to outweigh what
+// the vector-ALU convolutions lose (inference at [2,59,56,40], filter 3, 1.2 M products a scale: 42 against 38 us; a
+// training step at [4,13,13,40], filter 15, 3 M products: 98 against 129 us).
+int padded_half(long long N, int D, int I, int K, int dtype) {
+    const bool as_is = dtype == kF32 || D % 8 != 0 || I % 8 == 0 || (D <= 256 && N * I * K * K < 2000000);
+    return as_is ? I / 2 : (I / 2 + 7) / 8 * 8;
+}
+
 Shape shape_of(int B, int H, int W, int h, int w, int D, int I, int K, int dtype) {
-    Shape s{B, H, W, h, w, D, I, K, dtype, dtype == kF32 ? 4 : 2, H * W, (long long)B * H * W, (long long)B * h * w, false, false};
+    const int G = I / 2, Gp = padded_half((long long)B * H * W, D, I, K, dtype);
+    Shape s{B, H, W, h, w, D, 2 * Gp, K, dtype, dtype == kF32 ? 4 : 2, H * W, G, Gp, (long long)B * H * W, (long long)B * h * w, false, false};
     s.exact = H == 2 * h && W == 2 * w;
-    s.single = s.exact && pdw_convblock_supported(B, H, W, D, I, K, dtype) != 0;
+    s.single = s.exact && !s.padded() && pdw_convblock_supported(B, H, W, D, I, K, dtype) != 0;
     return s;
 }
 
 bool layer_ok(int K, int NO, int dtype) { return pdw_dense_supported(K, NO, dtype) != 0; }
 
+// The four weights with inner channels in the padded layout, eight values to a thread: conv_up's rows, conv_out's
+// columns, the filters' channels.  A few hundred KB at most: launch latency.
+struct PackArgs {
+    const uint16_t *up, *out, *dw0, *dw1;
+    uint16_t *up_p, *out_p, *dw0_p, *dw1_p;
+    int D, G, Gp, KK;
+    int n_up, n_out, n_dw;   // vectors of 8 in each region
+};
+
+__global__ __launch_bounds__(256) void pack_weights_k(const PackArgs g) {
+    int v = blockIdx.x * 256 + threadIdx.x;
+    const int I = 2 * g.G, Ip = 2 * g.Gp;
+    if (v < g.n_up) {
+        const int per = g.D / 8, row = v / per, c = v - row * per;
+        const int hi = row >= g.Gp, r = row - hi * g.Gp;
+        uint4 x = make_uint4(0, 0, 0, 0);
+        if (r < g.G) x = *reinterpret_cast<const uint4*>(g.up + (long long)(hi * g.G + r) * g.D + c * 8);
+        *reinterpret_cast<uint4*>(g.up_p + (long long)v * 8) = x;
+        return;
+    }
+    v -= g.n_up;
+    const uint16_t* src = g.out;
+    uint16_t* dst = g.out_p;
+    if (v >= g.n_out) {
+        v -= g.n_out;
+        src = g.dw0, dst = g.dw0_p;
+        if (v >= g.n_dw) {
+            v -= g.n_dw;
+            src = g.dw1, dst = g.dw1_p;
+            if (v >= g.n_dw) return;
+        }
+    }
+    const int per = Ip / 8, row = v / per, c = (v - row * per) * 8;
+    const int hi = c >= g.Gp, r = c - hi * g.Gp;
+    ChanVec<uint16_t, 8> o;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o.v[i] = r + i < g.G ? src[(long long)row * I + hi * g.G + r + i] : (uint16_t)0;
+    *reinterpret_cast<ChanVec<uint16_t, 8>*>(dst + (long long)v * 8) = o;
+}
+
+// The block's inner weights as its kernels read them.
+struct Weights {
+    const void *up, *out, *dw0, *dw1;
+};
+
 // What the forward leaves for the backward, then what only the forward needs.
 struct Saved {
     void *a, *c0, *cat, *xp, *c1, *m;
+    void *up_p, *out_p, *dw0_p, *dw1_p;   // packed weights (padded widths)
     float *xparts, *yp;
     void* ws;
     size_t ws_bytes, bytes;
@@ -58,6 +124,10 @@ Saved saved_layout(const Shape& s, void* base) {
     r.a = c.take(full), r.c0 = c.take(full), r.cat = c.take(full);
     r.xp = c.take(half), r.c1 = c.take(half);
     r.m = c.take((size_t)s.B * s.D * s.es);
+    if (s.padded()) {
+        const size_t layer = (size_t)s.I * s.D * s.es, filter = (size_t)s.K * s.K * s.I * s.es;
+        r.up_p = c.take(layer), r.out_p = c.take(layer), r.dw0_p = c.take(filter), r.dw1_p = c.take(filter);
+    }
     r.xparts = (float*)c.take((size_t)((s.N + 31) / 32) * s.D * 4);
     r.yp = (float*)c.take((size_t)s.B * s.D * 4);   // (behind xparts: the workspace of pdw_convblock_fwd)
     r.ws_bytes = up256(pdw_pool_branch_workspace_bytes(s.B, s.P, s.D));
@@ -94,10 +164,22 @@ BwdWork bwd_layout(const Shape& s, void* base) {
     return r;
 }
 
+int pack_weights(const Shape& s, const Saved& v, Weights* w, hipStream_t stream) {
+    PackArgs g{(const uint16_t*)w->up, (const uint16_t*)w->out, (const uint16_t*)w->dw0, (const uint16_t*)w->dw1,
+               (uint16_t*)v.up_p,      (uint16_t*)v.out_p,      (uint16_t*)v.dw0_p,      (uint16_t*)v.dw1_p,
+               s.D,                    s.G,                     s.Gp,                    s.K * s.K,
+               s.I * s.D / 8,          s.I * s.D / 8,           s.K * s.K * s.I / 8};
+    hipLaunchKernelGGL(pack_weights_k, dim3(cdiv(g.n_up + g.n_out + 2 * g.n_dw, 256)), dim3(256), 0, stream, g);
+    *w = {v.up_p, v.out_p, v.dw0_p, v.dw1_p};
+    return check_launch("pack_weights");
+}
+
 bool rows_whole_tiles(const Shape& s) { return s.P % pdw_dense_colsum_rows() == 0; }
 
-int forward(const Shape& s, const Saved& v, const void* x, const void* w_up, const void* w_dw0, const void* w_dw1,
-            const void* w_pool, const void* b_pool, const void* w_out, const void* b_out, void* y, void* stream) {
+int forward(const Shape& s, const Saved& v, const void* x, const Weights& wt, const void* w_pool, const void* b_pool,
+            const void* b_out, void* y, void* stream) {
+    const void *const w_up = wt.up, *const w_out = wt.out, *const w_dw0 = wt.dw0, *const w_dw1 = wt.dw1;
+    const hipStream_t st = (hipStream_t)stream;
     const int pad = s.K / 2, dt = s.dtype;
     const bool two = s.exact && dt != kF32 && pdw_dwconv_fwd2_supported(s.B, s.H, s.W, s.I, s.K, dt);
     // conv_up, where its kernel can with the sums of x per row tile (for the mean branch) and the 2x2 pool of its result
@@ -140,25 +222,35 @@ int forward(const Shape& s, const Saved& v, const void* x, const void* w_up, con
     if (!convs)
         if (int e = pdw_dwconv_fwd(v.xp, w_dw1, v.c1, s.B, s.h, s.w, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, dt, stream)) return e;
     // both gates and the resize into the concatenation, the mean branch's row per image, conv_out (conv_block.py:18-21, 40-49)
-    if (mean) {
+    if (mean && !s.padded()) {
         const int r = pdw_dense_fwd_gated(v.c0, v.c1, v.cat, w_out, nullptr, v.yp, y, s.B, s.H, s.W, s.I, s.D, 0, dt, stream);
         if (r != 3) return r;
-        if (int e = pdw_gate_pair_fwd(v.c0, v.c1, v.cat, s.B, s.H, s.W, s.h, s.w, s.I, s.I, dt, stream)) return e;
-    } else if (parts) {
-        if (int e = pdw_block_mid_fwd(v.c0, v.c1, v.cat, s.B, s.H, s.W, s.h, s.w, s.I, s.I, parts, nparts, w_pool, b_pool,
-                                      b_out, v.m, v.yp, s.P, s.D, dt, stream))
-            return e;
-    } else {
-        if (int e = pdw_gate_pair_fwd(v.c0, v.c1, v.cat, s.B, s.H, s.W, s.h, s.w, s.I, s.I, dt, stream)) return e;
-        if (int e = pdw_pool_branch_fwd(x, w_pool, b_pool, b_out, v.m, v.yp, v.ws, v.ws_bytes, s.B, s.P, s.D, dt, stream)) return e;
     }
+    bool gates = false;
+    if (!mean && parts) {
+        const int r = block_mid_fwd_launch(v.c0, v.c1, v.cat, s.B, s.H, s.W, s.h, s.w, s.I, s.I, parts, nparts, w_pool, b_pool,
+                                           b_out, v.m, v.yp, s.P, s.D, dt, st, s.gw());
+        if (r != 0 && r != -1) return r;
+        mean = gates = r == 0;
+    }
+    if (!gates)
+        if (int e = gate_pair_fwd_launch(v.c0, v.c1, v.cat, s.B, s.H, s.W, s.h, s.w, s.I, s.I, dt, st, s.gw())) return e;
+    if (!mean)
+        if (int e = pool_branch_fwd_launch(parts ? nullptr : x, w_pool, b_pool, b_out, v.m, v.yp, (float*)v.ws, s.B, s.P, s.D, dt,
+                                           st, parts, nparts))
+            return e;
     return pdw_dense_fwd(v.cat, w_out, 0, nullptr, v.yp, y, s.N, s.I, s.D, s.P, dt, stream);
 }
 
-int backward(const Shape& s, const Saved& v, const BwdWork& g, const void* gy, const void* x, const void* w_up,
-             const void* w_dw0, const void* w_dw1, const void* w_pool, const void* w_out, void* dx, void* gw_up,
-             void* gw_dw0, void* gw_dw1, void* gw_pool, void* gb_pool, void* gw_out, void* gb_out, void* stream) {
+int backward(const Shape& s, const Saved& v, const BwdWork& g, const void* gy, const void* x, const Weights& wt,
+             const void* w_pool, void* dx, void* gw_up, void* gw_dw0, void* gw_dw1, void* gw_pool, void* gb_pool,
+             void* gw_out, void* gb_out, void* stream) {
     const int pad = s.K / 2, dt = s.dtype;
+    const void *const w_up = wt.up, *const w_out = wt.out, *const w_dw0 = wt.dw0, *const w_dw1 = wt.dw1;
+    const hipStream_t st = (hipStream_t)stream;
+    // gradients of the inner weights leave the padding out: the halves of a row of channels, or of conv_up's rows
+    const int seg = s.padded() ? s.Gp : 0, val = s.G;
+    reduce_defer_compact(seg, val);
     // conv_out: gradient of the concatenation and of the weight, with the sums of gy per row tile where the kernel can
     const bool colsum = rows_whole_tiles(s) && pdw_dense_colsum_supported(s.D, s.I, dt);
     const bool pair_cs = colsum && pdw_dense_bwd_pair_colsum_supported(s.D, s.I, dt);
@@ -177,25 +269,24 @@ int backward(const Shape& s, const Saved& v, const BwdWork& g, const void* gy, c
         if (int e = pdw_dense_wgrad(gy, v.cat, gw_out, g.ws_po, g.b_po, s.N, s.D, s.I, dt, stream)) return e;
     }
     // the gates and the mean branch
+    reduce_defer_compact(0, 0);
     void* gb0 = gb_out ? gb_out : g.gbias;
     void* gb1 = gb_pool ? gb_pool : (char*)g.gbias + (size_t)s.D * s.es;
     const int nparts = s.P / pdw_dense_colsum_rows();
-    if (gparts && s.exact && s.h >= 2 && s.w >= 2) {
-        if (int e = pdw_block_mid_bwd(g.dcat, v.c0, v.c1, g.gcf, g.gch, s.B, s.H, s.W, s.h, s.w, s.I, s.I, gparts, nparts, v.m,
-                                      w_pool, gb0, gb1, gw_pool, g.dmean, g.ws_pool, g.b_pool, s.P, s.D, dt, stream))
+    int mid = -1;
+    if (gparts) {
+        mid = block_mid_bwd_launch(g.dcat, v.c0, v.c1, g.gcf, g.gch, s.B, s.H, s.W, s.h, s.w, s.I, s.I, gparts, nparts, v.m, w_pool,
+                                   gb0, gb1, gw_pool, g.dmean, (float*)g.ws_pool, s.P, s.D, dt, st, s.gw());
+        if (mid != 0 && mid != -1) return mid;
+    }
+    if (mid == -1) {
+        if (int e = pool_branch_bwd_launch(gparts ? nullptr : gy, v.m, w_pool, gb0, gb1, gw_pool, g.dmean, (float*)g.ws_pool, s.B,
+                                           s.P, s.D, dt, st, gparts, nparts))
             return e;
-    } else {
-        if (gparts) {
-            if (int e = pdw_pool_branch_bwd_parts(gparts, nparts, v.m, w_pool, gb0, gb1, gw_pool, g.dmean, g.ws_pool, g.b_pool,
-                                                  s.B, s.P, s.D, dt, stream))
-                return e;
-        } else if (int e = pdw_pool_branch_bwd(gy, v.m, w_pool, gb0, gb1, gw_pool, g.dmean, g.ws_pool, g.b_pool, s.B, s.P, s.D,
-                                               dt, stream)) {
-            return e;
-        }
-        if (int e = pdw_gate_pair_bwd(g.dcat, v.c0, v.c1, g.gcf, g.gch, s.B, s.H, s.W, s.h, s.w, s.I, s.I, dt, stream)) return e;
+        if (int e = gate_pair_bwd_launch(g.dcat, v.c0, v.c1, g.gcf, g.gch, s.B, s.H, s.W, s.h, s.w, s.I, s.I, dt, st, s.gw())) return e;
     }
     // the convolutions: the pooled scale's input gradient, then the rest (one launch where that is covered)
+    reduce_defer_compact(seg, val);
     if (int e = pdw_dwconv_dgrad(g.gch, w_dw1, g.dxp, s.B, s.h, s.w, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, dt, stream)) return e;
     int r = 3;
     if (s.exact && dt != kF32) {
@@ -212,6 +303,7 @@ int backward(const Shape& s, const Saved& v, const BwdWork& g, const void* gy, c
             return e;
     }
     // conv_up: input gradient (plus the mean branch's per-image term) and weight gradient
+    reduce_defer_compact(seg * s.D, val * s.D);
     if (dx && s.P >= 32 && pdw_dense_bwd_pair_supported(s.I, s.D, dt))
         return pdw_dense_bwd_pair(g.da, w_up, x, dx, nullptr, gw_up, g.ws_pu, g.b_pu, g.dmean, s.P, s.N, s.I, s.D, dt, stream);
     if (int e = pdw_dense_wgrad(g.da, x, gw_up, g.ws_pu, g.b_pu, s.N, s.I, s.D, dt, stream)) return e;
@@ -229,7 +321,9 @@ int pdw_block_supported(int B, int H, int W, int h, int w, int D, int I, int K, 
     if (B < 1 || H < 1 || W < 1 || h < 1 || w < 1 || K < 1 || !(K & 1) || D < 4 || I < 4 || (I & 1)) return 0;
     if ((long long)B * H * W * (D > I ? D : I) > 0x7fffffffLL || (long long)H * h > 0x7fffffffLL) return 0;
     if ((long long)B * h * w * I > 0x7fffffffLL) return 0;
-    return layer_ok(D, I, dtype) && layer_ok(I, D, dtype) ? 1 : 0;
+    const int Il = 2 * padded_half((long long)B * H * W, D, I, K, dtype);
+    if (Il * (long long)B * H * W > 0x7fffffffLL) return 0;
+    return layer_ok(D, Il, dtype) && layer_ok(Il, D, dtype) ? 1 : 0;
 }
 
 size_t pdw_block_saved_bytes(int B, int H, int W, int h, int w, int D, int I, int K, int dtype) {
@@ -252,7 +346,10 @@ int pdw_block_fwd(const void* x, const void* w_up, const void* w_dw0, const void
     if (s.single)
         return pdw_convblock_fwd(x, w_up, w_dw0, w_dw1, w_pool, b_pool, w_out, b_out, v.a, v.c0, v.xp, v.c1, v.cat, v.m, y,
                                  v.xparts, (size_t)((char*)v.ws - (char*)v.xparts), B, H, W, D, I, K, dtype, stream);
-    return forward(s, v, x, w_up, w_dw0, w_dw1, w_pool, b_pool, w_out, b_out, y, stream);
+    Weights wt{w_up, w_out, w_dw0, w_dw1};
+    if (s.padded())
+        if (int e = pack_weights(s, v, &wt, (hipStream_t)stream)) return e;
+    return forward(s, v, x, wt, w_pool, b_pool, b_out, y, stream);
 }
 
 size_t pdw_block_bwd_workspace_bytes(int B, int H, int W, int h, int w, int D, int I, int K, int dtype) {
@@ -278,8 +375,8 @@ int pdw_block_bwd(const void* gy, const void* x, const void* saved, const void* 
         return set_error("pdw_block_bwd: workspace of %zu bytes given, %zu needed", workspace_bytes, g.bytes), 1;
     // the final summations of all weight gradients run as one launch at the end of the pass
     if (int e = pdw_reduce_defer_begin()) return e;
-    const int e = backward(s, v, g, gy, x, w_up, w_dw0, w_dw1, w_pool, w_out, dx, gw_up, gw_dw0, gw_dw1, gw_pool, gb_pool,
-                           gw_out, gb_out, stream);
+    const Weights wt = s.padded() ? Weights{v.up_p, v.out_p, v.dw0_p, v.dw1_p} : Weights{w_up, w_out, w_dw0, w_dw1};
+    const int e = backward(s, v, g, gy, x, wt, w_pool, dx, gw_up, gw_dw0, gw_dw1, gw_pool, gb_pool, gw_out, gb_out, stream);
     const int f = pdw_reduce_defer_flush(stream);   // also ends the deferral after an error
     return e ? e : f;
 }

@@ -1318,7 +1318,8 @@ int dense_bwd_pair_launch(const void* gy, const void* w, const void* xin, void* 
     const int nnt = cdiv(I, 32);
     const size_t lds_rows = ((size_t)nnt * 32 * ((O > 64 ? 128 : 64) + 8) + 4 * 32 * ((O > I ? O : I) + 8)) * 2 +
                             (rowbias ? (size_t)4 * 2 * nnt * 32 * sizeof(float) : 0);
-    const size_t lds_wg = (size_t)2 * kWgRows * (O + 8 + I + 8) * 2;
+    size_t lds_wg = (size_t)2 * kWgRows * (O + 8 + I + 8) * 2;
+    if (lds_wg < 4 * 16 * 64 * sizeof(float)) lds_wg = 4 * 16 * 64 * sizeof(float);   // the wavefronts' sums (narrow layers)
     const size_t lds = lds_rows > lds_wg ? lds_rows : lds_wg;
     const dim3 grid((unsigned)(nwg + nrows));
 #define PDW_PAIR(T, CS, OO, II)                                                                                      \

@@ -136,6 +136,9 @@ __global__ __launch_bounds__(256) void wgrad_reduce_many(const ReduceJobs jobs) 
 // recorded; the flush runs them all in one launch.
 static thread_local bool t_defer = false;
 static thread_local ReduceJobs t_jobs;
+static thread_local int t_seg = 0, t_val = 0;
+
+void reduce_defer_compact(int seg, int val) { t_seg = t_defer ? seg : 0, t_val = val; }
 
 // Part lanes of a stand-alone summation: 32 when 8 would need more than one round of loads.
 static int standalone_part_lanes(int nparts) { return nparts > 128 ? 32 : 8; }
@@ -160,6 +163,7 @@ int reduce_jobs_launch(const ReduceJobs& recorded, hipStream_t s) {
 int reduce_defer_begin() {
     if (t_defer) return set_error("pdw_reduce_defer_begin: already deferring on this thread"), 1;
     t_defer = true;
+    t_seg = 0;
     t_jobs.njobs = 0;
     t_jobs.first_block[0] = 0;
     return 0;
@@ -183,7 +187,7 @@ int reduce_defer_outer(const float* g, const void* m, void* out, int B, int D, i
     if (reduce_defer_room() < 1 || dtype == kF32 || D % 4 != 0) return -1;
     const int j = t_jobs.njobs++;
     t_jobs.part[j] = g, t_jobs.aux[j] = m, t_jobs.out[j] = out, t_jobs.nparts[j] = B, t_jobs.n[j] = D * D;
-    t_jobs.dtype[j] = dtype, t_jobs.vec[j] = 0, t_jobs.ql[j] = 8, t_jobs.dim[j] = D;
+    t_jobs.dtype[j] = dtype, t_jobs.vec[j] = 0, t_jobs.ql[j] = 8, t_jobs.dim[j] = D, t_jobs.seg[j] = 0;
     t_jobs.first_block[j + 1] = t_jobs.first_block[j] + cdiv((long long)D * D, kOuterBlock);
     return 0;
 }
@@ -274,12 +278,17 @@ size_t dwconv_wgrad_direct_workspace(int B, int H, int W, int C, int KH, int KW,
 
 template <typename T>
 int wgrad_reduce_launch(const float* part, void* dw, int nparts, int n, hipStream_t s) {
-    const int vec = reduce_vec_ok(part, dw, n, (int)sizeof(T)) ? kReduceVec : 1;
+    // (packed outputs are stored one by one: only the partials have to be aligned for four of them to a lane)
+    const int vec = reduce_vec_ok(part, t_seg ? nullptr : dw, n, (int)sizeof(T)) ? kReduceVec : 1;
+    if (t_defer && t_seg && t_jobs.njobs == kMaxReduceJobs) {   // only a table can carry the packing: make room
+        if (int e = reduce_jobs_launch(t_jobs, s)) return e;
+        t_jobs.njobs = 0;
+    }
     if (t_defer && t_jobs.njobs < kMaxReduceJobs) {
         const int j = t_jobs.njobs++;
         t_jobs.part[j] = part, t_jobs.out[j] = dw, t_jobs.nparts[j] = nparts, t_jobs.n[j] = n;
         t_jobs.dtype[j] = dtype_of<T>();
-        t_jobs.vec[j] = vec, t_jobs.ql[j] = 8;
+        t_jobs.vec[j] = vec, t_jobs.ql[j] = 8, t_jobs.seg[j] = t_seg, t_jobs.val[j] = t_val;
         t_jobs.first_block[j + 1] = t_jobs.first_block[j] + cdiv(n, reduce_block_outputs(vec, 8));
         return 0;
     }

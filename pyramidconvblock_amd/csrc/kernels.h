@@ -30,6 +30,9 @@ bool reduce_deferring();  // between reduce_defer_begin and the flush on this th
 int reduce_defer_room();  // jobs that can still be recorded (0 when not deferring)
 int reduce_defer_outer(const float* g, const void* m, void* out, int B, int D, int dtype);  // -1: not recorded
 int reduce_defer_flush(hipStream_t s);
+// Summations recorded (while deferring) from here on drop padding on the way out: of every `seg` outputs only the first
+// `val` exist in the result, which is packed; seg a multiple of 4.  seg = 0: results as they are.
+void reduce_defer_compact(int seg, int val);
 
 // dwconv_tiled.hip: LDS-tiled forward / input gradient for stride 1, dilation 1, odd KW <= 17.
 // Returns -1 if the case is not covered (the caller then uses the direct kernel).
@@ -67,20 +70,21 @@ int bilinear_fwd_launch(const void* x, void* y, int B, int h, int w, int C, int 
 int bilinear_bwd_launch(const void* gy, void* gx, int B, int h, int w, int C, int H, int W, int ldg, int dtype,
                         hipStream_t s);
 int gate_fwd_launch(const void* x, void* y, long long M, int I, int ldy, int dtype, hipStream_t s);
+// (gw, here and below: the gate's width where it is not I / 2, halves padded with zero channels; 0 otherwise)
 int gate_pair_fwd_launch(const void* xf, const void* xh, void* y, int B, int H, int W, int h, int w, int I, int ldy,
-                         int dtype, hipStream_t s);
+                         int dtype, hipStream_t s, int gw = 0);
 int gate_pair_bwd_launch(const void* gy, const void* xf, const void* xh, void* gxf, void* gxh, int B, int H, int W, int h,
-                         int w, int I, int ldg, int dtype, hipStream_t s);
+                         int w, int I, int ldg, int dtype, hipStream_t s, int gw = 0);
 int bilinear_pool_fwd_launch(const void* x, void* y, int B, int h, int w, int C, int H, int W, int ldy, const float* parts,
                              int nparts, const void* wp, const void* bp, const void* bo, void* m, float* rowbias, int P,
                              int D, int dtype, hipStream_t s);
 int block_mid_fwd_launch(const void* xf, const void* xh, void* y, int B, int H, int W, int h, int w, int I, int ldy,
                          const float* parts, int nparts, const void* wp, const void* bp, const void* bo, void* m,
-                         float* rowbias, int P, int D, int dtype, hipStream_t s);
+                         float* rowbias, int P, int D, int dtype, hipStream_t s, int gw = 0);
 int block_mid_bwd_launch(const void* gy, const void* xf, const void* xh, void* gxf, void* gxh, int B, int H, int W, int h,
                          int w, int I, int ldg, const float* parts, int nparts, const void* m, const void* wp,
                          void* gbias, void* gbias2, void* gwp, float* dmean, float* ws, int P, int D, int dtype,
-                         hipStream_t s);
+                         hipStream_t s, int gw = 0);
 int gate_bilinear_fwd_launch(const void* x, void* y, int B, int h, int w, int I, int H, int W, int ldy, int dtype,
                              hipStream_t s);
 int bilinear_gate_bwd_launch(const void* gy, const void* x, void* gx, int B, int h, int w, int I, int H, int W, int ldg,

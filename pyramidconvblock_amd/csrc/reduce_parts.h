@@ -17,7 +17,7 @@ constexpr int kReduceLds = 8 * 32 * kReduceVec;  // floats of LDS a workgroup ne
 
 template <typename T, int V, int QL>
 __device__ __forceinline__ void reduce_parts_block(const float* __restrict__ part, T* __restrict__ dw, int nparts, int n,
-                                                   int blk, float* red) {
+                                                   int blk, float* red, int seg, int val) {
     constexpr int EL = 256 / QL, ROW = EL * V;  // red[QL][ROW]
     const int el = threadIdx.x % EL, q = threadIdx.x / EL;
     const int e = (blk * EL + el) * V;
@@ -89,7 +89,14 @@ __device__ __forceinline__ void reduce_parts_block(const float* __restrict__ par
             o[i] = ((red[c] + red[ROW + c]) + (red[2 * ROW + c] + red[3 * ROW + c])) +
                    ((red[4 * ROW + c] + red[5 * ROW + c]) + (red[6 * ROW + c] + red[7 * ROW + c]));
         }
-        store_f32<T, V>(dw + e, o);
+        if (seg == 0) {
+            store_f32<T, V>(dw + e, o);
+        } else {   // of every seg outputs the first val exist (seg % 4 == 0: the V are of one segment)
+            const int sg = e / seg, r = e - sg * seg;
+#pragma unroll
+            for (int i = 0; i < V; ++i)
+                if (r + i < val) dw[(long long)sg * val + r + i] = from_f32<T>(o[i]);
+        }
     }
 }
 
@@ -104,13 +111,13 @@ inline int reduce_block_outputs(int vec, int ql) { return 256 / ql * vec; }
 
 template <typename T>
 __device__ __forceinline__ void reduce_parts_any(const float* part, T* dw, int nparts, int n, int blk, int vec, int ql,
-                                                 float* red) {
+                                                 float* red, int seg = 0, int val = 0) {
     if (vec == kReduceVec) {
-        if (ql == 32) reduce_parts_block<T, kReduceVec, 32>(part, dw, nparts, n, blk, red);
-        else reduce_parts_block<T, kReduceVec, 8>(part, dw, nparts, n, blk, red);
+        if (ql == 32) reduce_parts_block<T, kReduceVec, 32>(part, dw, nparts, n, blk, red, seg, val);
+        else reduce_parts_block<T, kReduceVec, 8>(part, dw, nparts, n, blk, red, seg, val);
     } else {
-        if (ql == 32) reduce_parts_block<T, 1, 32>(part, dw, nparts, n, blk, red);
-        else reduce_parts_block<T, 1, 8>(part, dw, nparts, n, blk, red);
+        if (ql == 32) reduce_parts_block<T, 1, 32>(part, dw, nparts, n, blk, red, seg, val);
+        else reduce_parts_block<T, 1, 8>(part, dw, nparts, n, blk, red, seg, val);
     }
 }
 
@@ -161,6 +168,7 @@ struct ReduceJobs {
     int vec[kMaxReduceJobs];  // outputs per lane: kReduceVec or 1; 0 = outer product (n = D * D, nparts = B)
     int ql[kMaxReduceJobs];   // part lanes: 8 or 32
     int dim[kMaxReduceJobs];  // outer products: D
+    int seg[kMaxReduceJobs], val[kMaxReduceJobs];  // outputs without their padding (reduce_defer_compact); seg = 0: all of them
     int first_block[kMaxReduceJobs + 1];
     int njobs;
 };
@@ -172,6 +180,7 @@ __device__ __forceinline__ void reduce_jobs_block(const ReduceJobs& jobs, int wg
     const int blk = wg - jobs.first_block[j];
     const float* part = jobs.part[j];
     const int nparts = jobs.nparts[j], n = jobs.n[j], vec = jobs.vec[j], ql = jobs.ql[j];
+    const int seg = jobs.seg[j], val = jobs.val[j];
     if (vec == 0) {  // outer product; fp32 outputs are not produced this way
         if (jobs.dtype[j] == kF16)
             outer_sum_block<f16_t>(part, (const f16_t*)jobs.aux[j], (f16_t*)jobs.out[j], nparts, jobs.dim[j], blk, threadIdx.x);
@@ -180,9 +189,9 @@ __device__ __forceinline__ void reduce_jobs_block(const ReduceJobs& jobs, int wg
         return;
     }
     switch (jobs.dtype[j]) {
-        case kF32: reduce_parts_any<float>(part, (float*)jobs.out[j], nparts, n, blk, vec, ql, red); break;
-        case kF16: reduce_parts_any<f16_t>(part, (f16_t*)jobs.out[j], nparts, n, blk, vec, ql, red); break;
-        default: reduce_parts_any<bf16_t>(part, (bf16_t*)jobs.out[j], nparts, n, blk, vec, ql, red); break;
+        case kF32: reduce_parts_any<float>(part, (float*)jobs.out[j], nparts, n, blk, vec, ql, red, seg, val); break;
+        case kF16: reduce_parts_any<f16_t>(part, (f16_t*)jobs.out[j], nparts, n, blk, vec, ql, red, seg, val); break;
+        default: reduce_parts_any<bf16_t>(part, (bf16_t*)jobs.out[j], nparts, n, blk, vec, ql, red, seg, val); break;
     }
 }
 

@@ -1386,7 +1386,7 @@ int bilinear_gate_bwd_launch(const void* gy, const void* x, void* gx, int B, int
 }
 
 int gate_pair_fwd_launch(const void* xf, const void* xh, void* y, int B, int H, int W, int h, int w, int I, int ldy,
-                         int dtype, hipStream_t s) {
+                         int dtype, hipStream_t s, int gw) {
     const void* ptrs[3] = {xf, xh, y};
     const int vec = pick_vec(gcd_int(I / 2, ldy), esize(dtype), ptrs, 3);
     const long long tf = (long long)B * H * W * (I / 2 / vec);
@@ -1396,7 +1396,7 @@ int gate_pair_fwd_launch(const void* xf, const void* xh, void* y, int B, int H, 
     if (!grid_for((tf + kGateItems - 1) / kGateItems, &bf) || !grid_for(th, &bh) ||
         (unsigned long long)bf + bh > 0x7fffffffULL)
         return 1;
-    const float sy = (float)h / (float)H, sx = (float)w / (float)W, sc = sqrtf((float)(I / 2));
+    const float sy = (float)h / (float)H, sx = (float)w / (float)W, sc = sqrtf((float)(gw > 0 ? gw : I / 2));
 #define CALL(T, V) hipLaunchKernelGGL((gate_pair_fwd_k<T, V>), dim3(bf + bh), dim3(256), 0, s, (const T*)xf, (const T*)xh, (T*)y, h, w, I, H, W, ldy, sy, sx, sc, bf, tf, th);
     PDW_TYPE_SWITCH(dtype, vec, CALL)
 #undef CALL
@@ -1405,7 +1405,7 @@ int gate_pair_fwd_launch(const void* xf, const void* xh, void* y, int B, int H, 
 
 // -1: extents are not exactly doubled (the caller runs the separate kernels).
 int gate_pair_bwd_launch(const void* gy, const void* xf, const void* xh, void* gxf, void* gxh, int B, int H, int W, int h,
-                         int w, int I, int ldg, int dtype, hipStream_t s) {
+                         int w, int I, int ldg, int dtype, hipStream_t s, int gw) {
     const void* ptrs[5] = {gy, xf, xh, gxf, gxh};
     const int vec = pick_vec(gcd_int(I / 2, ldg), esize(dtype), ptrs, 5);
     const long long tf = (long long)B * H * W * (I / 2 / vec), th = (long long)B * h * w * (I / 2 / vec);
@@ -1414,7 +1414,7 @@ int gate_pair_bwd_launch(const void* gy, const void* xf, const void* xh, void* g
     if (!grid_for((tf + kGateItems - 1) / kGateItems, &bf) || !grid_for(th, &bh) ||
         (unsigned long long)bf + bh > 0x7fffffffULL)
         return 1;
-    const float sc = sqrtf((float)(I / 2));
+    const float sc = sqrtf((float)(gw > 0 ? gw : I / 2));
     if (H != 2 * h || W != 2 * w || h < 2 || w < 2) {   // any ratio of extents
         const float sy = (float)h / (float)H, sx = (float)w / (float)W;
 #define CALL(T, V) hipLaunchKernelGGL((gate_pair_bwd_gen_k<T, V>), dim3(bf + bh), dim3(256), 0, s, (const T*)gy, (const T*)xf, (const T*)xh, (T*)gxf, (T*)gxh, h, w, H, W, I, ldg, sc, sy, sx, bf, tf, th);
@@ -1433,7 +1433,7 @@ int gate_pair_bwd_launch(const void* gy, const void* xf, const void* xh, void* g
 
 int block_mid_fwd_launch(const void* xf, const void* xh, void* y, int B, int H, int W, int h, int w, int I, int ldy,
                          const float* parts, int nparts, const void* wp, const void* bp, const void* bo, void* m,
-                         float* rowbias, int P, int D, int dtype, hipStream_t s) {
+                         float* rowbias, int P, int D, int dtype, hipStream_t s, int gw) {
     const void* ptrs[3] = {xf, xh, y};
     if (pick_vec(gcd_int(I / 2, ldy), esize(dtype), ptrs, 3) != 8 || !pool_branch_v8_ok(wp, nullptr, parts, B, D, dtype))
         return -1;
@@ -1444,7 +1444,7 @@ int block_mid_fwd_launch(const void* xf, const void* xh, void* y, int B, int H, 
     if (!grid_for((tf + kGateItems - 1) / kGateItems, &bf) || !grid_for(th, &bh) ||
         (unsigned long long)bf + bh + B > 0x7fffffffULL)
         return 1;
-    const float sy = (float)h / (float)H, sx = (float)w / (float)W, sc = sqrtf((float)(I / 2));
+    const float sy = (float)h / (float)H, sx = (float)w / (float)W, sc = sqrtf((float)(gw > 0 ? gw : I / 2));
     const PoolFwdJob job{parts, nparts, B, D, 1.f / (float)P, wp, bp, bo, m, rowbias};
     const size_t lds = (size_t)9 * D * sizeof(float);
     if (dtype == kF16)
@@ -1482,7 +1482,7 @@ int bilinear_pool_fwd_launch(const void* x, void* y, int B, int h, int w, int C,
 int block_mid_bwd_launch(const void* gy, const void* xf, const void* xh, void* gxf, void* gxh, int B, int H, int W, int h,
                          int w, int I, int ldg, const float* parts, int nparts, const void* m, const void* wp,
                          void* gbias, void* gbias2, void* gwp, float* dmean, float* ws, int P, int D, int dtype,
-                         hipStream_t s) {
+                         hipStream_t s, int gw) {
     if (H != 2 * h || W != 2 * w || h < 2 || w < 2) return -1;
     const void* ptrs[5] = {gy, xf, xh, gxf, gxh};
     if (pick_vec(gcd_int(I / 2, ldg), esize(dtype), ptrs, 5) != 8 || !pool_branch_v8_ok(wp, m, parts, B, D, dtype)) return -1;
@@ -1492,7 +1492,7 @@ int block_mid_bwd_launch(const void* gy, const void* xf, const void* xh, void* g
     if (!grid_for((tf + kGateItems - 1) / kGateItems, &bf) || !grid_for(th, &bh) ||
         (unsigned long long)bf + bh + B + D > 0x7fffffffULL)
         return 1;
-    const float sc = sqrtf((float)(I / 2));
+    const float sc = sqrtf((float)(gw > 0 ? gw : I / 2));
     float* gs = ws + spatial_sum_workspace(B, P, D) / sizeof(float);
     const PoolBwdJob job{parts, nparts, B, D, 1.f / (float)P, wp, m, gs, dmean, gbias, gbias2, gwp};
     const size_t la = (size_t)17 * D * sizeof(float), lb = (size_t)(B + 16 * D) * sizeof(float);
