@@ -15,6 +15,7 @@
 #include "../../include/pdw.h"
 #include "common.h"
 #include "kernels.h"
+#include "mean_any.h"
 
 namespace {
 
@@ -114,8 +115,15 @@ struct Saved {
     void *up_p, *out_p, *dw0_p, *dw1_p;   // packed weights (padded widths)
     float *xparts, *yp;
     void* ws;
-    size_t ws_bytes, bytes;
+    size_t bytes;
 };
+
+// The mean branch: column sums, and (backward) the sums per image, in the layout of pdw_pool_branch_*.
+size_t mean_workspace(const Shape& s) {
+    const ColsumJob j = colsum_plan(nullptr, nullptr, s.B, s.P, s.D, s.es);
+    const size_t own = up256((size_t)s.B * j.n * s.D * 4) + (size_t)s.B * s.D * 4, old = pdw_pool_branch_workspace_bytes(s.B, s.P, s.D);
+    return own > old ? own : old;
+}
 
 Saved saved_layout(const Shape& s, void* base) {
     Carver c{(char*)base};
@@ -130,8 +138,7 @@ Saved saved_layout(const Shape& s, void* base) {
     }
     r.xparts = (float*)c.take((size_t)((s.N + 31) / 32) * s.D * 4);
     r.yp = (float*)c.take((size_t)s.B * s.D * 4);   // (behind xparts: the workspace of pdw_convblock_fwd)
-    r.ws_bytes = up256(pdw_pool_branch_workspace_bytes(s.B, s.P, s.D));
-    r.ws = c.take(r.ws_bytes);
+    r.ws = c.take(mean_workspace(s));
     r.bytes = c.used;
     return r;
 }
@@ -140,7 +147,7 @@ struct BwdWork {
     void *dcat, *gcf, *gch, *dxp, *da, *gbias;
     float *gparts, *dmean;
     void *ws_po, *ws_pool, *ws_w0, *ws_w1, *ws_pu;
-    size_t b_po, b_pool, b_w0, b_w1, b_pu, bytes;
+    size_t b_po, b_w0, b_w1, b_pu, bytes;
 };
 
 BwdWork bwd_layout(const Shape& s, void* base) {
@@ -154,7 +161,7 @@ BwdWork bwd_layout(const Shape& s, void* base) {
     r.gparts = (float*)c.take((size_t)((s.N + 31) / 32) * s.D * 4);
     r.dmean = (float*)c.take((size_t)s.B * s.D * 4);
     r.b_po = up256(pdw_dense_wgrad_workspace_bytes(s.N, s.D, s.I)), r.ws_po = c.take(r.b_po);
-    r.b_pool = up256(pdw_pool_branch_workspace_bytes(s.B, s.P, s.D)), r.ws_pool = c.take(r.b_pool);
+    r.ws_pool = c.take(mean_workspace(s));
     r.b_w0 = up256(pdw_dwconv_wgrad_workspace_bytes(s.B, s.H, s.W, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, s.dtype));
     r.ws_w0 = c.take(r.b_w0);
     r.b_w1 = up256(pdw_dwconv_wgrad_workspace_bytes(s.B, s.h, s.w, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, s.dtype));
@@ -199,11 +206,19 @@ int forward(const Shape& s, const Saved& v, const void* x, const Weights& wt, co
     } else if (int e = pdw_dense_fwd(x, w_up, 0, nullptr, nullptr, v.a, s.N, s.D, s.I, s.P, dt, stream)) {
         return e;
     }
+    // the pool, with the sums of x where conv_up's kernel did not leave any
+    const bool any_mean = mean_any_ok(x, w_pool, v.m, s.D, s.es);
+    auto pool = [&]() -> int {
+        if (parts || !any_mean) return avgpool_fwd_launch(v.a, v.xp, s.B, s.H, s.W, s.I, s.h, s.w, dt, st);
+        const ColsumJob sums = colsum_plan(x, (float*)v.ws, s.B, s.P, s.D, s.es);
+        parts = sums.part, nparts = sums.n;
+        return avgpool_colsum_launch(v.a, v.xp, s.B, s.H, s.W, s.I, s.h, s.w, sums, dt, st);
+    };
     // the convolutions of both scales                                                         (conv_block.py:14-17)
     bool convs = false, mean = false;
     if (two) {
         if (!pooled)
-            if (int e = pdw_avgpool_fwd(v.a, v.xp, s.B, s.H, s.W, s.I, s.h, s.w, dt, stream)) return e;
+            if (int e = pool()) return e;
         int r = 3;
         if (parts) {
             r = pdw_dwconv_fwd2_mean(v.a, w_dw0, v.c0, 0, 0, v.xp, w_dw1, v.c1, 0, 0, s.B, s.H, s.W, s.I, s.K, parts, nparts,
@@ -215,9 +230,12 @@ int forward(const Shape& s, const Saved& v, const void* x, const Weights& wt, co
         convs = r == 0;
         if (!convs)
             if (int e = pdw_dwconv_fwd(v.a, w_dw0, v.c0, s.B, s.H, s.W, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, dt, stream)) return e;
-    } else if (int e = pdw_dwconv_fwd_pool(v.a, w_dw0, v.c0, v.xp, s.B, s.H, s.W, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, s.h,
-                                           s.w, dt, stream)) {
-        return e;
+    } else if (parts || !any_mean) {
+        if (int e = pdw_dwconv_fwd_pool(v.a, w_dw0, v.c0, v.xp, s.B, s.H, s.W, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, s.h, s.w, dt, stream))
+            return e;
+    } else {
+        if (int e = pool()) return e;
+        if (int e = pdw_dwconv_fwd(v.a, w_dw0, v.c0, s.B, s.H, s.W, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, dt, stream)) return e;
     }
     if (!convs)
         if (int e = pdw_dwconv_fwd(v.xp, w_dw1, v.c1, s.B, s.h, s.w, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, dt, stream)) return e;
@@ -232,6 +250,11 @@ int forward(const Shape& s, const Saved& v, const void* x, const Weights& wt, co
                                            b_out, v.m, v.yp, s.P, s.D, dt, st, s.gw());
         if (r != 0 && r != -1) return r;
         mean = gates = r == 0;
+    }
+    if (!mean && parts && any_mean) {
+        const MeanJob job{parts, nparts, s.B, s.D, 1.f / (float)s.P, w_pool, b_pool, b_out, v.m, v.yp, nullptr, nullptr};
+        if (int e = gate_pair_mean_fwd_launch(v.c0, v.c1, v.cat, s.B, s.H, s.W, s.h, s.w, s.I, s.I, job, dt, st, s.gw())) return e;
+        mean = gates = true;
     }
     if (!gates)
         if (int e = gate_pair_fwd_launch(v.c0, v.c1, v.cat, s.B, s.H, s.W, s.h, s.w, s.I, s.I, dt, st, s.gw())) return e;
@@ -279,7 +302,16 @@ int backward(const Shape& s, const Saved& v, const BwdWork& g, const void* gy, c
                                    gb0, gb1, gw_pool, g.dmean, (float*)g.ws_pool, s.P, s.D, dt, st, s.gw());
         if (mid != 0 && mid != -1) return mid;
     }
-    if (mid == -1) {
+    if (mid == -1 && mean_any_ok(gy, w_pool, v.m, s.D, s.es) && reduce_defer_room() >= 3) {
+        ColsumJob sums = colsum_plan(gy, (float*)g.ws_pool, s.B, s.P, s.D, s.es);
+        float* const gs = (float*)((char*)g.ws_pool + up256((size_t)s.B * sums.n * s.D * 4));
+        if (int e = gparts ? gate_pair_bwd_launch(g.dcat, v.c0, v.c1, g.gcf, g.gch, s.B, s.H, s.W, s.h, s.w, s.I, s.I, dt, st, s.gw())
+                           : gate_pair_colsum_bwd_launch(g.dcat, v.c0, v.c1, g.gcf, g.gch, s.B, s.H, s.W, s.h, s.w, s.I, s.I, sums, dt, st, s.gw()))
+            return e;
+        const MeanJob job{gparts ? gparts : sums.part, gparts ? nparts : sums.n, s.B, s.D, 1.f / (float)s.P, w_pool, nullptr, nullptr, v.m,
+                          nullptr, gs, g.dmean};
+        if (int e = mean_bwd_launch(job, gb0, gb1, gw_pool, dt, st)) return e;
+    } else if (mid == -1) {
         if (int e = pool_branch_bwd_launch(gparts ? nullptr : gy, v.m, w_pool, gb0, gb1, gw_pool, g.dmean, (float*)g.ws_pool, s.B,
                                            s.P, s.D, dt, st, gparts, nparts))
             return e;

@@ -184,7 +184,7 @@ int reduce_defer_room() { return t_defer ? kMaxReduceJobs - t_jobs.njobs : 0; }
 
 // Records out[o * D + d] = sum_b g[b * D + o] * m[b * D + d] (see outer_sum_block); only while deferring.
 int reduce_defer_outer(const float* g, const void* m, void* out, int B, int D, int dtype) {
-    if (reduce_defer_room() < 1 || dtype == kF32 || D % 4 != 0) return -1;
+    if (reduce_defer_room() < 1 || D % 4 != 0) return -1;
     const int j = t_jobs.njobs++;
     t_jobs.part[j] = g, t_jobs.aux[j] = m, t_jobs.out[j] = out, t_jobs.nparts[j] = B, t_jobs.n[j] = D * D;
     t_jobs.dtype[j] = dtype, t_jobs.vec[j] = 0, t_jobs.ql[j] = 8, t_jobs.dim[j] = D, t_jobs.seg[j] = 0;

@@ -1,0 +1,239 @@
+// The global-mean branch of a block (conv_block.py:46-49) for any width, as workgroup bodies of 256 threads that ride in
+// the grids of the resampling launches around them: column sums of a tensor over ranges of an image's positions, and
+// the two small products (mean -> conv_pool -> a row per image; its transpose).  16-byte vectors: widths that are
+// multiples of 16 bytes.  Bandwidth for the sums, latency for the products: a product's workgroup takes 64 features of
+// one image and adds up the image's partial sums itself, so that nothing has to wait for a summation launch; the plan
+// keeps the partials few (32 an image at most) because every such workgroup reads them all.  At [4,64,64,1152] the four
+// launches that this replaces (two sums, two products with up to 128 partials an image) took 10 + 24 + 10 + 52 us.
+#pragma once
+#include "common.h"
+
+namespace pdw {
+
+struct ColsumJob {
+    const void* x;   // [B][P][C]
+    float* part;     // [B][n][C]
+    int B, P, C, n, len;      // n ranges of len positions
+    int lanes_log, slices;    // 1 << lanes_log vectors of a row to a workgroup, slices of them
+};
+
+inline int colsum_workgroups(const ColsumJob& j) { return j.B * j.n * j.slices; }
+
+// part = nullptr: only the plan (for the size of the partials).
+inline ColsumJob colsum_plan(const void* x, float* part, int B, int P, int C, int esize) {
+    const int V = 16 / esize, vecs = C / V;
+    ColsumJob j{x, part, B, P, C, 1, P, 3, 1};
+    while (j.lanes_log < 5 && (1 << j.lanes_log) < vecs) ++j.lanes_log;
+    j.slices = cdiv(vecs, 1 << j.lanes_log);
+    const int pl = 256 >> j.lanes_log;
+    int n = cdiv(512, (long long)B * j.slices);   // two workgroups per compute unit ...
+    if (n > P / (pl * 8)) n = P / (pl * 8);       // ... of at least eight positions a thread
+    if (n > 32) n = 32;
+    if (n < 1) n = 1;
+    j.len = cdiv(P, n), j.n = cdiv(P, j.len);
+    return j;
+}
+
+// red: 256 * V floats of LDS (V = values per 16 bytes).
+template <typename T>
+__device__ __forceinline__ void colsum_body(const ColsumJob& j, int wg, float* red) {
+    constexpr int V = 16 / (int)sizeof(T);
+    const int sl = wg % j.slices, rest = wg / j.slices, ch = rest % j.n, b = rest / j.n;
+    const int tid = threadIdx.x, lanes = 1 << j.lanes_log, cv = tid & (lanes - 1), pl = tid >> j.lanes_log, PL = 256 >> j.lanes_log;
+    const int c = (sl * lanes + cv) * V;
+    const int p1 = min((ch + 1) * j.len, j.P);
+    float acc[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) acc[v] = 0.f;
+    if (c < j.C) {
+        const T* xb = (const T*)j.x + (long long)b * j.P * j.C + c;
+        int p = ch * j.len + pl;
+        for (; p + 7 * PL < p1; p += 8 * PL) {   // eight loads in flight
+            ChanVec<T, V> xv[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) xv[u] = *reinterpret_cast<const ChanVec<T, V>*>(xb + (long long)(p + u * PL) * j.C);
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+#pragma unroll
+                for (int v = 0; v < V; ++v) acc[v] += to_f32(xv[u].v[v]);
+        }
+        for (; p < p1; p += PL) {
+            float xv[V];
+            load_f32<T, V>(xb + (long long)p * j.C, xv);
+#pragma unroll
+            for (int v = 0; v < V; ++v) acc[v] += xv[v];
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < V; v += 4) *reinterpret_cast<float4*>(red + tid * V + v) = make_float4(acc[v], acc[v + 1], acc[v + 2], acc[v + 3]);
+    __syncthreads();
+    const int cols = lanes * V;   // <= 256
+    if (tid < cols && sl * cols + tid < j.C) {
+        float s = 0.f;
+        for (int q = 0; q < PL; ++q) s += red[q * cols + tid];
+        j.part[((long long)b * j.n + ch) * j.C + sl * cols + tid] = s;
+    }
+}
+
+// sm[c] = sum over the n partials of an image, c < D; D % 4 == 0.  red: 256 float4 of LDS.  Ends with a barrier.
+__device__ __forceinline__ void image_sums(const float* __restrict__ pp, int n, int D, float* sm, float4* red) {
+    const int tid = threadIdx.x, d4 = D / 4;
+    int L = 16;
+    while (L < 256 && L < d4) L <<= 1;
+    const int cl = tid & (L - 1), ql = tid / L, QL = 256 / L;
+    for (int c0 = 0; c0 < d4; c0 += L) {   // (more than once only where QL = 1)
+        const int c = c0 + cl;
+        float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (c < d4) {
+            const float* p = pp + c * 4;
+            int q = ql;
+            for (; q + 7 * QL < n; q += 8 * QL) {
+                float4 v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const float4*>(p + (long long)(q + u * QL) * D);
+#pragma unroll
+                for (int u = 0; u < 8; ++u) s.x += v[u].x, s.y += v[u].y, s.z += v[u].z, s.w += v[u].w;
+            }
+            for (; q < n; q += QL) {
+                const float4 v = *reinterpret_cast<const float4*>(p + (long long)q * D);
+                s.x += v.x, s.y += v.y, s.z += v.z, s.w += v.w;
+            }
+        }
+        if (QL == 1) {
+            if (c < d4) *reinterpret_cast<float4*>(sm + c * 4) = s;
+        } else {
+            red[ql * L + cl] = s;
+            __syncthreads();
+            if (ql == 0 && c < d4) {
+                for (int q = 1; q < QL; ++q) {
+                    const float4 v = red[q * L + cl];
+                    s.x += v.x, s.y += v.y, s.z += v.z, s.w += v.w;
+                }
+                *reinterpret_cast<float4*>(sm + c * 4) = s;
+            }
+        }
+    }
+    __syncthreads();
+}
+
+constexpr int kMeanOut = 64;   // features of a workgroup of the products
+
+struct MeanJob {
+    const float* part;   // [B][n][D]
+    int n, B, D;
+    float inv_p;
+    const void *wp, *bp, *bo;
+    void* m;             // forward: the mean
+    float* rowbias;      // forward: m Wp^T + bp + bo
+    float *gs, *dmean;   // backward: the sums of the gradient, their product with Wp over P
+};
+
+inline int mean_slices(int D) { return cdiv(D, kMeanOut); }
+inline size_t mean_lds(int D) { return (size_t)D * sizeof(float) + 2048 * sizeof(float); }   // sums; scratch of 8 KB
+
+template <typename T>
+__device__ __forceinline__ void mean_fwd_body(const MeanJob& j, int wg, float* sm) {
+    constexpr int V = 16 / (int)sizeof(T);
+    const int slices = (j.D + kMeanOut - 1) / kMeanOut, b = wg / slices, sl = wg - b * slices, D = j.D, tid = threadIdx.x;
+    image_sums(j.part + (long long)b * j.n * D, j.n, D, sm, reinterpret_cast<float4*>(sm + D));
+    for (int c = tid; c < D; c += 256) {
+        const T mv = from_f32<T>(sm[c] * j.inv_p);
+        if (sl == 0) ((T*)j.m)[(long long)b * D + c] = mv;
+        sm[c] = to_f32(mv);
+    }
+    __syncthreads();
+    const int sub = tid & 7, nv = D / V;
+#pragma unroll
+    for (int pass = 0; pass < kMeanOut / 32; ++pass) {   // eight lanes to a feature
+        const int o = sl * kMeanOut + pass * 32 + (tid >> 3);
+        float acc = 0.f;
+        if (o < D) {
+            const T* wr = (const T*)j.wp + (long long)o * D;
+            int v = sub;
+            for (; v + 24 < nv; v += 32) {
+                ChanVec<T, V> wv[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) wv[u] = *reinterpret_cast<const ChanVec<T, V>*>(wr + (v + 8 * u) * V);
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int e = 0; e < V; ++e) acc = fmaf(sm[(v + 8 * u) * V + e], to_f32(wv[u].v[e]), acc);
+            }
+            for (; v < nv; v += 8) {
+                float wv[V];
+                load_f32<T, V>(wr + v * V, wv);
+#pragma unroll
+                for (int e = 0; e < V; ++e) acc = fmaf(sm[v * V + e], wv[e], acc);
+            }
+        }
+        acc += __shfl_xor(acc, 1);
+        acc += __shfl_xor(acc, 2);
+        acc += __shfl_xor(acc, 4);
+        if (sub == 0 && o < D) {
+            if (j.bp) acc += to_f32(((const T*)j.bp)[o]);
+            if (j.bo) acc += to_f32(((const T*)j.bo)[o]);
+            j.rowbias[(long long)b * D + o] = acc;
+        }
+    }
+}
+
+template <typename T>
+__device__ __forceinline__ void mean_bwd_body(const MeanJob& j, int wg, float* sm) {
+    constexpr int V = 16 / (int)sizeof(T), CL = kMeanOut / V, OL = 256 / CL;   // column lanes, row lanes
+    const int slices = (j.D + kMeanOut - 1) / kMeanOut, b = wg / slices, sl = wg - b * slices, D = j.D, tid = threadIdx.x;
+    float* red = sm + D;   // [OL][64]
+    image_sums(j.part + (long long)b * j.n * D, j.n, D, sm, reinterpret_cast<float4*>(red));
+    if (sl == 0)
+        for (int c = tid; c < D; c += 256) j.gs[(long long)b * D + c] = sm[c];
+    const int cv = tid % CL, ol = tid / CL, c = sl * kMeanOut + cv * V;
+    float acc[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) acc[e] = 0.f;
+    if (c < D) {
+        const T* wc = (const T*)j.wp + c;
+        int o = ol;
+        for (; o + 7 * OL < D; o += 8 * OL) {
+            ChanVec<T, V> wv[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) wv[u] = *reinterpret_cast<const ChanVec<T, V>*>(wc + (long long)(o + u * OL) * D);
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+#pragma unroll
+                for (int e = 0; e < V; ++e) acc[e] = fmaf(sm[o + u * OL], to_f32(wv[u].v[e]), acc[e]);
+        }
+        for (; o < D; o += OL) {
+            float wv[V];
+            load_f32<T, V>(wc + (long long)o * D, wv);
+#pragma unroll
+            for (int e = 0; e < V; ++e) acc[e] = fmaf(sm[o], wv[e], acc[e]);
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < V; ++e) red[ol * kMeanOut + cv * V + e] = acc[e];
+    __syncthreads();
+    if (tid < kMeanOut && sl * kMeanOut + tid < D) {
+        float t = 0.f;
+        for (int q = 0; q < OL; ++q) t += red[q * kMeanOut + tid];
+        j.dmean[(long long)b * D + sl * kMeanOut + tid] = t * j.inv_p;
+    }
+}
+
+// Whether the bodies take the case (host side).
+inline bool mean_any_ok(const void* x, const void* wp, const void* m, int D, int esize) {
+    return D % (16 / esize) == 0 && D <= 8192 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(wp) & 15) == 0 &&
+           (reinterpret_cast<uintptr_t>(m) & 15) == 0;
+}
+
+// resample.hip: the launches that they ride in.
+// xp = adaptive average pool of a to (h, w), with the column sums
+int avgpool_colsum_launch(const void* a, void* xp, int B, int H, int W, int C, int h, int w, const ColsumJob& sums, int dtype, hipStream_t s);
+// gate_pair_fwd_launch with the mean branch's forward
+int gate_pair_mean_fwd_launch(const void* xf, const void* xh, void* y, int B, int H, int W, int h, int w, int I, int ldy,
+                              const MeanJob& mean, int dtype, hipStream_t s, int gw);
+// gate_pair_bwd_launch with the column sums
+int gate_pair_colsum_bwd_launch(const void* gy, const void* xf, const void* xh, void* gxf, void* gxh, int B, int H, int W, int h,
+                                int w, int I, int ldg, const ColsumJob& sums, int dtype, hipStream_t s, int gw);
+// the mean branch's backward; the gradients of the pooled layer's weight and biases join the deferred summations
+int mean_bwd_launch(const MeanJob& mean, void* gbias, void* gbias2, void* gwp, int dtype, hipStream_t s);
+
+}  // namespace pdw

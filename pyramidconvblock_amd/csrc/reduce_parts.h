@@ -181,8 +181,10 @@ __device__ __forceinline__ void reduce_jobs_block(const ReduceJobs& jobs, int wg
     const float* part = jobs.part[j];
     const int nparts = jobs.nparts[j], n = jobs.n[j], vec = jobs.vec[j], ql = jobs.ql[j];
     const int seg = jobs.seg[j], val = jobs.val[j];
-    if (vec == 0) {  // outer product; fp32 outputs are not produced this way
-        if (jobs.dtype[j] == kF16)
+    if (vec == 0) {  // outer product
+        if (jobs.dtype[j] == kF32)
+            outer_sum_block<float>(part, (const float*)jobs.aux[j], (float*)jobs.out[j], nparts, jobs.dim[j], blk, threadIdx.x);
+        else if (jobs.dtype[j] == kF16)
             outer_sum_block<f16_t>(part, (const f16_t*)jobs.aux[j], (f16_t*)jobs.out[j], nparts, jobs.dim[j], blk, threadIdx.x);
         else
             outer_sum_block<bf16_t>(part, (const bf16_t*)jobs.aux[j], (bf16_t*)jobs.out[j], nparts, jobs.dim[j], blk, threadIdx.x);

@@ -6,6 +6,7 @@
 // no atomics and results are bit-reproducible.
 #include "common.h"
 #include "kernels.h"
+#include "mean_any.h"
 #include "bilinear.h"
 #include "pool_branch.h"
 
@@ -46,10 +47,8 @@ __device__ __forceinline__ int bin_end(int i, int in, int out) {
 }
 
 template <typename T, int VEC>
-__global__ __launch_bounds__(256) void avgpool_fwd_k(const T* __restrict__ x, T* __restrict__ y, int H, int W, int C,
-                                                     int h, int w, long long total) {
-    const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= total) return;
+__device__ __forceinline__ void avgpool_fwd_item(const T* __restrict__ x, T* __restrict__ y, int H, int W, int C, int h,
+                                                 int w, long long idx) {
     const int CV = C / VEC;
     int cq, j, i;
     long long b;
@@ -81,6 +80,23 @@ __global__ __launch_bounds__(256) void avgpool_fwd_k(const T* __restrict__ x, T*
 #pragma unroll
     for (int v = 0; v < VEC; ++v) acc[v] *= inv;
     store_f32<T, VEC>(y + ((b * h + i) * w + j) * C + c, acc);
+}
+
+template <typename T, int VEC>
+__global__ __launch_bounds__(256) void avgpool_fwd_k(const T* __restrict__ x, T* __restrict__ y, int H, int W, int C,
+                                                     int h, int w, long long total) {
+    const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx < total) avgpool_fwd_item<T, VEC>(x, y, H, W, C, h, w, idx);
+}
+
+// The same with the column sums of another tensor (mean_any.h) in the first workgroups: both are bandwidth.
+template <typename T, int VEC>
+__global__ __launch_bounds__(256) void avgpool_colsum_k(const T* __restrict__ x, T* __restrict__ y, int H, int W, int C,
+                                                        int h, int w, long long total, const ColsumJob sums, int nsums) {
+    extern __shared__ float sm[];
+    if ((int)blockIdx.x < nsums) return colsum_body<T>(sums, blockIdx.x, sm);
+    const long long idx = (long long)(blockIdx.x - nsums) * blockDim.x + threadIdx.x;
+    if (idx < total) avgpool_fwd_item<T, VEC>(x, y, H, W, C, h, w, idx);
 }
 
 // Input row ih lies in bins i with floor(ih*h/H) <= i <= ceil((ih+1)*h/H) - 1.
@@ -612,15 +628,15 @@ __device__ __forceinline__ void gate_bilinear_fwd_x2_item(const T* __restrict__ 
 // Both branches of a two-scale block in one launch: workgroups below nblk_full gate the full-resolution tensor into
 // channels [0, G) of y, the others gate and resize the pooled one into channels [G, 2G).
 template <typename T, int VEC>
-__global__ __launch_bounds__(256) void gate_pair_fwd_k(const T* __restrict__ xf, const T* __restrict__ xh,
-                                                       T* __restrict__ y, int h, int w, int I, int H, int W, int ldy,
-                                                       float sy, float sx, float s, unsigned nblk_full,
-                                                       long long total_full, long long total_half) {
-    if (blockIdx.x < nblk_full) {
-        const long long first = (long long)blockIdx.x * (kGateItems * 256) + threadIdx.x;
+__device__ __forceinline__ void gate_pair_fwd_body(const T* __restrict__ xf, const T* __restrict__ xh, T* __restrict__ y,
+                                                   int h, int w, int I, int H, int W, int ldy, float sy, float sx, float s,
+                                                   unsigned nblk_full, long long total_full, long long total_half,
+                                                   unsigned bid) {
+    if (bid < nblk_full) {
+        const long long first = (long long)bid * (kGateItems * 256) + threadIdx.x;
         if (first < total_full) gate_fwd_items<T, VEC, kGateItems>(xf, y, I, ldy, s, first, 256, total_full);
     } else {
-        const long long idx = (long long)(blockIdx.x - nblk_full) * blockDim.x + threadIdx.x;
+        const long long idx = (long long)(bid - nblk_full) * blockDim.x + threadIdx.x;
         if (idx < total_half) {
             if (H == 2 * h && W == 2 * w)  // total_half then counts 2 x 2 output blocks
                 gate_bilinear_fwd_x2_item<T, VEC>(xh, y + I / 2, h, w, I, ldy, s, idx);
@@ -628,6 +644,26 @@ __global__ __launch_bounds__(256) void gate_pair_fwd_k(const T* __restrict__ xf,
                 gate_bilinear_fwd_item<T, VEC>(xh, y + I / 2, h, w, I, H, W, ldy, sy, sx, s, idx);
         }
     }
+}
+
+template <typename T, int VEC>
+__global__ __launch_bounds__(256) void gate_pair_fwd_k(const T* __restrict__ xf, const T* __restrict__ xh,
+                                                       T* __restrict__ y, int h, int w, int I, int H, int W, int ldy,
+                                                       float sy, float sx, float s, unsigned nblk_full,
+                                                       long long total_full, long long total_half) {
+    gate_pair_fwd_body<T, VEC>(xf, xh, y, h, w, I, H, W, ldy, sy, sx, s, nblk_full, total_full, total_half, blockIdx.x);
+}
+
+// The same with the mean branch (mean_any.h) in the first workgroups.
+template <typename T, int VEC>
+__global__ __launch_bounds__(256) void gate_pair_mean_fwd_k(const T* __restrict__ xf, const T* __restrict__ xh,
+                                                            T* __restrict__ y, int h, int w, int I, int H, int W, int ldy,
+                                                            float sy, float sx, float s, unsigned nblk_full,
+                                                            long long total_full, long long total_half, const MeanJob mean,
+                                                            unsigned nmean) {
+    extern __shared__ float sm[];
+    if (blockIdx.x < nmean) return mean_fwd_body<T>(mean, blockIdx.x, sm);
+    gate_pair_fwd_body<T, VEC>(xf, xh, y, h, w, I, H, W, ldy, sy, sx, s, nblk_full, total_full, total_half, blockIdx.x - nmean);
 }
 
 // Backward of the pair for exactly doubled extents: the bilinear gather of bilinear_bwd_x2_k (rounded to T),
@@ -714,18 +750,9 @@ __global__ __launch_bounds__(256) void gate_pair_bwd_k(const T* __restrict__ gy,
 // The same for any ratio of extents: the half-resolution items gather their gradient with bilinear_bwd_gather
 // (rounded to T, as the separate kernel stores it) and apply the gate's gradient.
 template <typename T, int VEC>
-__global__ __launch_bounds__(256) void gate_pair_bwd_gen_k(const T* __restrict__ gy, const T* __restrict__ xf,
-                                                           const T* __restrict__ xh, T* __restrict__ gxf,
-                                                           T* __restrict__ gxh, int h, int w, int H, int W, int I, int ldg,
-                                                           float s, float sy, float sx, unsigned nblk_full,
-                                                           long long total_full, long long total_half) {
-    if (blockIdx.x < nblk_full) {
-        const long long first = (long long)blockIdx.x * (kGateItems * 256) + threadIdx.x;
-        if (first < total_full) gate_bwd_items<T, VEC, kGateItems>(xf, gy, gxf, I, ldg, s, first, 256, total_full);
-        return;
-    }
-    const long long idx = (long long)(blockIdx.x - nblk_full) * blockDim.x + threadIdx.x;
-    if (idx >= total_half) return;
+__device__ __forceinline__ void gate_pair_bwd_gen_item(const T* __restrict__ gy, const T* __restrict__ xh, T* __restrict__ gxh,
+                                                       int h, int w, int H, int W, int I, int ldg, float s, float sy, float sx,
+                                                       long long idx) {
     const int G = I / 2, GV = G / VEC;
     int cq, n, m;
     long long b;
@@ -746,6 +773,50 @@ __global__ __launch_bounds__(256) void gate_pair_bwd_gen_k(const T* __restrict__
     T* op = gxh + ((b * h + m) * w + n) * I + c;
     store_f32<T, VEC>(op, ga);
     store_f32<T, VEC>(op + G, gbv);
+}
+
+template <typename T, int VEC>
+__global__ __launch_bounds__(256) void gate_pair_bwd_gen_k(const T* __restrict__ gy, const T* __restrict__ xf,
+                                                           const T* __restrict__ xh, T* __restrict__ gxf,
+                                                           T* __restrict__ gxh, int h, int w, int H, int W, int I, int ldg,
+                                                           float s, float sy, float sx, unsigned nblk_full,
+                                                           long long total_full, long long total_half) {
+    if (blockIdx.x < nblk_full) {
+        const long long first = (long long)blockIdx.x * (kGateItems * 256) + threadIdx.x;
+        if (first < total_full) gate_bwd_items<T, VEC, kGateItems>(xf, gy, gxf, I, ldg, s, first, 256, total_full);
+        return;
+    }
+    const long long idx = (long long)(blockIdx.x - nblk_full) * blockDim.x + threadIdx.x;
+    if (idx < total_half) gate_pair_bwd_gen_item<T, VEC>(gy, xh, gxh, h, w, H, W, I, ldg, s, sy, sx, idx);
+}
+
+// Either form with the column sums of another tensor (mean_any.h); the half-resolution workgroups, whose gathers take
+// longest, first, then the sums.
+template <typename T, int VEC, bool X2>
+__global__ __launch_bounds__(256) void gate_pair_colsum_bwd_k(const T* __restrict__ gy, const T* __restrict__ xf,
+                                                              const T* __restrict__ xh, T* __restrict__ gxf,
+                                                              T* __restrict__ gxh, int h, int w, int H, int W, int I, int ldg,
+                                                              float s, float sy, float sx, unsigned nblk_half, unsigned nsums,
+                                                              long long total_full, long long total_half, const ColsumJob sums) {
+    extern __shared__ float sm[];
+    unsigned bid = blockIdx.x;
+    if (bid < nblk_half) {
+        const long long idx = (long long)bid * blockDim.x + threadIdx.x;
+        if (idx >= total_half) return;
+        if constexpr (X2) bilinear_gate_bwd_x2_item<T, VEC>(gy + I / 2, xh, gxh, h, w, I, ldg, s, idx);
+        else gate_pair_bwd_gen_item<T, VEC>(gy, xh, gxh, h, w, H, W, I, ldg, s, sy, sx, idx);
+        return;
+    }
+    bid -= nblk_half;
+    if (bid < nsums) return colsum_body<T>(sums, (int)bid, sm);
+    const long long first = (long long)(bid - nsums) * (kGateItems * 256) + threadIdx.x;
+    if (first < total_full) gate_bwd_items<T, VEC, kGateItems>(xf, gy, gxf, I, ldg, s, first, 256, total_full);
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void mean_bwd_k(const MeanJob mean) {
+    extern __shared__ float sm[];
+    mean_bwd_body<T>(mean, blockIdx.x, sm);
 }
 
 // ---------------------------------------------------------------- per-image column sums and broadcast add
@@ -1285,6 +1356,21 @@ int avgpool_fwd_launch(const void* x, void* y, int B, int H, int W, int C, int h
     return check_launch("avgpool_fwd");
 }
 
+int avgpool_colsum_launch(const void* a, void* xp, int B, int H, int W, int C, int h, int w, const ColsumJob& sums, int dtype,
+                          hipStream_t s) {
+    const void* ptrs[2] = {a, xp};
+    const int vec = pick_vec(C, esize(dtype), ptrs, 2);
+    const long long total = (long long)B * h * w * (C / vec);
+    const int nsums = colsum_workgroups(sums);
+    unsigned blocks;
+    if (!grid_for(total, &blocks) || (unsigned long long)blocks + nsums > 0x7fffffffULL) return 1;
+    const size_t lds = 256 * 16 / esize(dtype) * sizeof(float);
+#define CALL(T, V) hipLaunchKernelGGL((avgpool_colsum_k<T, V>), dim3(blocks + nsums), dim3(256), lds, s, (const T*)a, (T*)xp, H, W, C, h, w, total, sums, nsums);
+    PDW_TYPE_SWITCH(dtype, vec, CALL)
+#undef CALL
+    return check_launch("avgpool_colsum");
+}
+
 int avgpool_bwd_launch(const void* gy, void* gx, int B, int H, int W, int C, int h, int w, int accumulate, int dtype,
                        hipStream_t s) {
     const void* ptrs[2] = {gy, gx};
@@ -1401,6 +1487,66 @@ int gate_pair_fwd_launch(const void* xf, const void* xh, void* y, int B, int H, 
     PDW_TYPE_SWITCH(dtype, vec, CALL)
 #undef CALL
     return check_launch("gate_pair_fwd");
+}
+
+int gate_pair_mean_fwd_launch(const void* xf, const void* xh, void* y, int B, int H, int W, int h, int w, int I, int ldy,
+                              const MeanJob& mean, int dtype, hipStream_t s, int gw) {
+    const void* ptrs[3] = {xf, xh, y};
+    const int vec = pick_vec(gcd_int(I / 2, ldy), esize(dtype), ptrs, 3);
+    const long long tf = (long long)B * H * W * (I / 2 / vec);
+    const long long th = (H == 2 * h && W == 2 * w) ? (long long)B * h * w * (I / 2 / vec) : tf;
+    unsigned bf, bh;
+    const unsigned nmean = (unsigned)(B * mean_slices(mean.D));
+    if (!grid_for((tf + kGateItems - 1) / kGateItems, &bf) || !grid_for(th, &bh) ||
+        (unsigned long long)bf + bh + nmean > 0x7fffffffULL)
+        return 1;
+    const float sy = (float)h / (float)H, sx = (float)w / (float)W, sc = sqrtf((float)(gw > 0 ? gw : I / 2));
+#define CALL(T, V) hipLaunchKernelGGL((gate_pair_mean_fwd_k<T, V>), dim3(bf + bh + nmean), dim3(256), mean_lds(mean.D), s, (const T*)xf, (const T*)xh, (T*)y, h, w, I, H, W, ldy, sy, sx, sc, bf, tf, th, mean, nmean);
+    PDW_TYPE_SWITCH(dtype, vec, CALL)
+#undef CALL
+    return check_launch("gate_pair_mean_fwd");
+}
+
+int gate_pair_colsum_bwd_launch(const void* gy, const void* xf, const void* xh, void* gxf, void* gxh, int B, int H, int W, int h,
+                                int w, int I, int ldg, const ColsumJob& sums, int dtype, hipStream_t s, int gw) {
+    const void* ptrs[5] = {gy, xf, xh, gxf, gxh};
+    const int vec = pick_vec(gcd_int(I / 2, ldg), esize(dtype), ptrs, 5);
+    const long long tf = (long long)B * H * W * (I / 2 / vec), th = (long long)B * h * w * (I / 2 / vec);
+    const unsigned nsums = (unsigned)colsum_workgroups(sums);
+    unsigned bf, bh;
+    if (!grid_for((tf + kGateItems - 1) / kGateItems, &bf) || !grid_for(th, &bh) ||
+        (unsigned long long)bf + bh + nsums > 0x7fffffffULL)
+        return 1;
+    const float sc = sqrtf((float)(gw > 0 ? gw : I / 2)), sy = (float)h / (float)H, sx = (float)w / (float)W;
+    const size_t lds = 256 * 16 / esize(dtype) * sizeof(float);
+    const bool x2 = H == 2 * h && W == 2 * w && h >= 2 && w >= 2;
+#define GO(T, V, X2) hipLaunchKernelGGL((gate_pair_colsum_bwd_k<T, V, X2>), dim3(bf + bh + nsums), dim3(256), lds, s, (const T*)gy, (const T*)xf, (const T*)xh, (T*)gxf, (T*)gxh, h, w, H, W, I, ldg, sc, sy, sx, bh, nsums, tf, th, sums)
+#define CALL(T, V) if (x2) GO(T, V, true); else GO(T, V, false);
+    PDW_TYPE_SWITCH(dtype, vec, CALL)
+#undef CALL
+#undef GO
+    return check_launch("gate_pair_colsum_bwd");
+}
+
+int mean_bwd_launch(const MeanJob& mean, void* gbias, void* gbias2, void* gwp, int dtype, hipStream_t s) {
+    const int B = mean.B, D = mean.D;
+    if (reduce_defer_room() < 3) return set_error("mean_bwd: no room among the deferred summations"), 1;
+    const dim3 grid((unsigned)(B * mean_slices(D)));
+    switch (dtype) {
+        case kF32: hipLaunchKernelGGL((mean_bwd_k<float>), grid, dim3(256), mean_lds(D), s, mean); break;
+        case kF16: hipLaunchKernelGGL((mean_bwd_k<f16_t>), grid, dim3(256), mean_lds(D), s, mean); break;
+        default: hipLaunchKernelGGL((mean_bwd_k<bf16_t>), grid, dim3(256), mean_lds(D), s, mean);
+    }
+    if (int e = check_launch("mean_bwd")) return e;
+    if (reduce_defer_outer(mean.gs, mean.m, gwp, B, D, dtype) != 0) return set_error("mean_bwd: deferred job refused"), 1;
+    for (void* g : {gbias, gbias2}) {
+        if (!g) continue;
+        const int e = dtype == kF32   ? wgrad_reduce_launch<float>(mean.gs, g, B, D, s)
+                      : dtype == kF16 ? wgrad_reduce_launch<f16_t>(mean.gs, g, B, D, s)
+                                      : wgrad_reduce_launch<bf16_t>(mean.gs, g, B, D, s);
+        if (e) return e;
+    }
+    return 0;
 }
 
 // -1: extents are not exactly doubled (the caller runs the separate kernels).

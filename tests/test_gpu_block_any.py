@@ -16,3 +16,13 @@ pytestmark = pytest.mark.gpu
 ])
 def test_padded_inner_channels(oracle, dtype, dim, k, shape):
     _block_case(oracle, dim, k, shape, dtype)
+
+
+@pytest.mark.parametrize("dtype,dim,k,shape", [
+    (torch.bfloat16, 16, 5, (5, 11, 13, 16)), (torch.float16, 72, 3, (2, 90, 90, 72)), (torch.bfloat16, 1032, 3, (1, 7, 9, 1032)),
+    (torch.float32, 36, 5, (3, 17, 12, 36)), (torch.float32, 252, 3, (40, 9, 8, 252)), (torch.float16, 256, 3, (70, 6, 6, 256)),
+])
+def test_mean_branch_of_any_width(oracle, dtype, dim, k, shape):
+    """The mean branch riding in the pool's and the gates' launches (csrc/mean_any.h): widths of less than one, of several
+    and of more than 256 vectors of four sums, one and many ranges of positions, batches beyond its plan's."""
+    _block_case(oracle, dim, k, shape, dtype)
