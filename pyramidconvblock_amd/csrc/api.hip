@@ -169,9 +169,13 @@ int pdw_dwconv_dgrad_addpool(const void* gy, const void* w, const void* gp, void
         return e;
     if (int e = check_resample("pdw_dwconv_dgrad_addpool", gp, dx, B, H, W, C, h, wp, dtype)) return e;
     if (B == 0) return 0;
-    if (SH == 1 && SW == 1 && DH == 1 && DW == 1 && PH <= KH - 1 && PW <= KW - 1 && H == 2 * h && W == 2 * wp) {
+    if (SH == 1 && SW == 1 && DH == 1 && DW == 1 && PH <= KH - 1 && PW <= KW - 1) {
         const int OH = conv_out_size(H, KH, 1, PH, 1), OW = conv_out_size(W, KW, 1, PW, 1);
-        if (OH > 0 && OW > 0) {
+        if (OH > 0 && OW > 0 && dtype == kF32 && KH == KW) {   // any ratio
+            const int r = dwconv_f32t_launch(gy, w, gp, dx, B, OH, OW, C, KW, KH - 1 - PH, KW - 1 - PW, true, h, wp,
+                                             (hipStream_t)stream);
+            if (r != -1) return r;
+        } else if (OH > 0 && OW > 0 && H == 2 * h && W == 2 * wp) {
             const int r = dwconv_tiled_launch(gy, w, dx, B, OH, OW, C, KH, KW, KH - 1 - PH, KW - 1 - PW, true, dtype,
                                               (hipStream_t)stream, gp);
             if (r != -1) return r;

@@ -8,7 +8,7 @@
 // inner channels are laid out G = I / 2 rounded up to 8 wide, so that the matrix-core convolutions (slices of 8 or 16
 // channels), the 128 x 128 dense tiles and the 16-byte gate kernels take them; the vector-ALU kernels that take the
 // widths as they are cost two to five times as much ([34,55,55,168], filter 15: 693 us for a training step, 1.14 times
-// the channels on the matrix cores 230).  The weights are packed into that layout by one launch per forward, and the summations
+// the channels on the matrix cores 324).  The weights are packed into that layout by one launch per forward, and the summations
 // of the weight gradients leave the padding out again.
 #include <stdint.h>
 

@@ -1,0 +1,416 @@
+// Depthwise convolution in fp32 on the fp32 matrix cores: forward and input gradient, stride 1, dilation 1, odd square
+// filters 3 .. 17 (the input gradient is the same kernel on gy with the rotated filter and padding k-1-p).
+//
+// The block-Toeplitz product of dwconv_tz.h on v_mfma_f32_16x16x4_f32: for one channel m = the 16 outputs of a 4 x 4 patch,
+// n = 16 patches four columns apart (in NI = 16 / NPC images), k = 4 consecutive columns of one window row.
+//     A[(di,dj)][(r, 4j+g)] = w[r - di][4j + g - dj]     in registers, IC * JB of them (IC = K+3 rows, JB column blocks)
+//     B[(r, 4j+g)][n]       = window[r][4n + 4j + g]      64 consecutive floats of a staged row: one conflict-free LDS read
+// A window row belongs to up to PER = ceil(IC/4) patch rows, whose accumulators are all live: a B operand is read once and
+// feeds PER products of 32 cycles each, so the matrix pipe is what bounds the kernel (LDS is under 10 % busy), a row
+// is dead after its step, and the window in LDS is two groups of four rows whatever the filter (20 KB).
+//
+// A workgroup (8 wavefronts, one channel each) owns a band of output rows x 4 NPC columns x NI images of 8 channels.  A step is
+// four window rows: the wavefronts multiply them, commit the next four from registers (16 bytes = 4 channels of a pixel,
+// written channel-major), request the rows two steps ahead, and store the patch row that the previous step finished
+// (through a pixel-major tile in LDS, 16 bytes a thread).  One barrier a step; wavefronts 0-3 multiply first and 4-7 last, so
+// that of a SIMD's two wavefronts one always feeds the matrix pipe.
+//
+// Measured at [32,56,56,64] against the vector-ALU kernel (dwconv_tiled.h): filter 9 28 us for 37, 13 40 for 77, 17 57 for 90
+// (the products of filter 13 alone 24); [32,28,28,64]: filter 13 15 for 41; [4,112,112,128]: filter 9 28 for 49, 13 39 for 75.
+//
+// ADD: the input gradient of a tensor that was also average-pooled to (AH, AW): y += the pool's gradient, from the one bin of
+// a pixel where the pool halved both extents (1), gathered from the at most 2 x 2 bins that a pixel lies in (2).
+#pragma once
+#include <mutex>
+
+#include "common.h"
+#include "kernels.h"
+#include "tile_common.h"
+
+namespace pdw {
+
+template <int K, int NPC>
+struct F32Shape {
+    static constexpr int NT = 512, CS = 8;
+    static constexpr int IC = K + 3, JB = (IC + 3) / 4, PER = (IC + 3) / 4, NI = 16 / NPC, TW = 4 * NPC;
+    static constexpr int WCOLS = 4 * (NPC - 1) + 4 * JB;          // window columns of an image
+    static constexpr int RP = 4 * WCOLS;                           // bytes per window row of a channel
+    // bytes per channel plane (8 rows): images of an operand read and channel quads of a staging write on other banks
+    static constexpr int plane() {
+        int p = 8 * RP;
+        const int want = NI == 1 ? 32 : NI == 2 ? 16 : 8, mod = NI == 1 ? 64 : 32;
+        while (p % mod != want) p += 8;
+        return p;
+    }
+    static constexpr int CHP = plane();
+    static constexpr int OROWP = TW * 32 + NPC * 4;                // result tile: row pitch (4 bytes more every 4 pixels)
+    static constexpr int OLB = NI * 4 * OROWP;
+    static constexpr int WTH = K + 6, WTW = 4 * JB + 4;            // zero-bordered filter table of a channel
+    static constexpr int R2B = (2 * OLB > CS * WTH * WTW * 4 ? 2 * OLB : CS * WTH * WTW * 4 + 15) / 16 * 16;
+    static constexpr size_t lds_bytes = (size_t)NI * CS * CHP + R2B;
+    static constexpr int NLD = (4 * NI * WCOLS * 2 + NT - 1) / NT; // staging items per thread and step
+    static_assert(lds_bytes <= 80 * 1024 && NLD <= 2, "sizes");
+};
+
+struct F32Geom {
+    int B, H, W, C, OH, OW, PH, PW, BR, nbands, ncolt, nslices, flip, AH, AW;
+};
+
+// Bins of an adaptive average pool of `in` values to `out` <= in that value i lies in: the first, and the weights (one
+// over the bin's length; 0: no second bin).
+__device__ __forceinline__ void pool_bins(int i, int in, int out, int& b0, float& w0, float& w1) {
+    b0 = (int)((unsigned)(i * out) / (unsigned)in);
+    const int b1 = (int)((unsigned)((i + 1) * out + in - 1) / (unsigned)in) - 1;
+    auto len = [&](int b) {
+        return (int)((unsigned)((b + 1) * in + out - 1) / (unsigned)out) - (int)((unsigned)(b * in) / (unsigned)out);
+    };
+    w0 = 1.f / (float)len(b0);
+    w1 = b1 > b0 ? 1.f / (float)len(b1) : 0.f;
+}
+
+template <int K, int NPC, int ADD>
+__device__ __forceinline__ void dwconv_f32_body(const float* __restrict__ x, const float* __restrict__ w,
+                                                const float* __restrict__ add, float* __restrict__ y, const F32Geom& g, int blk,
+                                                int nblk) {
+    using Sh = F32Shape<K, NPC>;
+    constexpr int NT = Sh::NT, IC = Sh::IC, JB = Sh::JB, PER = Sh::PER, NI = Sh::NI, TW = Sh::TW, RP = Sh::RP, CHP = Sh::CHP;
+    constexpr int OROWP = Sh::OROWP, OLB = Sh::OLB, WTH = Sh::WTH, WTW = Sh::WTW, NLD = Sh::NLD, WCOLS = Sh::WCOLS, CS = Sh::CS;
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    extern __shared__ uint32_t smem[];
+    char* const xl = reinterpret_cast<char*>(smem);
+    char* const r2 = xl + NI * CS * CHP;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    int bid = xcd_remap(blk, nblk);
+    const int sl = bid % g.nslices;
+    bid /= g.nslices;
+    const int ct = bid % g.ncolt;
+    bid /= g.ncolt;
+    const int band = bid % g.nbands, b0 = bid / g.nbands * NI;
+    const int c0 = sl * CS, ocol0 = ct * TW, orow0 = band * g.BR;
+    const int rows_valid = min(g.BR, g.OH - orow0), cols_valid = min(TW, g.OW - ocol0);
+    const int npr = (rows_valid + 3) >> 2, nsteps = npr + PER - 1;   // patch rows; groups of four window rows
+    const long long img_in = (long long)g.H * g.W * g.C, img_out = (long long)g.OH * g.OW * g.C;
+
+    // ---- filter slice to registers (before the window's loads), then to the zero-bordered table
+    constexpr int NWL = (K * K * 2 + NT - 1) / NT;
+    f4 wval[NWL];
+#pragma unroll
+    for (int i = 0; i < NWL; ++i) {
+        const int idx = min(tid + i * NT, K * K * 2 - 1);
+        wval[i] = *reinterpret_cast<const f4*>(w + (idx >> 1) * g.C + min(c0 + 4 * (idx & 1), g.C - 4));
+    }
+    // ---- staging: offsets past the descriptor's end (images beyond the batch, the markers) read as zero
+    constexpr uint32_t kNoCol = 0x40000000u, kNoRow = 0x80000000u;
+    const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(x + (long long)b0 * img_in), (short)0, (int)(min(NI, g.B - b0) * img_in * 4), 0x00020000);
+    uint32_t icol[NLD];
+    int irow[NLD], idst[NLD];
+#pragma unroll
+    for (int l = 0; l < NLD; ++l) {
+        const int idx = tid + l * NT, q = idx & 1, col = (idx >> 1) % WCOLS, img = (idx >> 1) / WCOLS % NI;
+        irow[l] = (idx >> 1) / WCOLS / NI;
+        const int ic = ocol0 - g.PW + col;
+        const bool ok = irow[l] < 4 && c0 + 4 * q < g.C && ic >= 0 && ic < g.W;
+        icol[l] = ok ? ((uint32_t)img * (uint32_t)img_in + (uint32_t)(ic * g.C + c0 + 4 * q)) * 4u : kNoCol;
+        idst[l] = (img * CS + 4 * q) * CHP + (irow[l] & 3) * RP + col * 4;
+    }
+    f4 buf[2][NLD];
+    auto issue = [&](f4 (&bf)[NLD], int s) {
+#pragma unroll
+        for (int l = 0; l < NLD; ++l) {
+            const int ir = orow0 - g.PH + 4 * s + irow[l];
+            const uint32_t r = s < nsteps && ir >= 0 && ir < g.H ? (uint32_t)(ir * g.W * g.C) * 4u : kNoRow;
+            bf[l] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(xrsrc, (int)(r + icol[l]), 0, 0));
+        }
+    };
+    auto commit = [&](const f4 (&bf)[NLD], int s) {
+        char* const half = xl + (s & 1) * 4 * RP;
+#pragma unroll
+        for (int l = 0; l < NLD; ++l) {
+            if (irow[l] < 4) {
+                const float e0 = bf[l].x, e1 = bf[l].y, e2 = bf[l].z, e3 = bf[l].w;
+                char* d = half + idst[l];
+                *reinterpret_cast<float*>(d) = e0;
+                *reinterpret_cast<float*>(d + CHP) = e1;
+                *reinterpret_cast<float*>(d + 2 * CHP) = e2;
+                *reinterpret_cast<float*>(d + 3 * CHP) = e3;
+            }
+        }
+    };
+    issue(buf[0], 0);
+    issue(buf[1], 1);
+    auto lds_barrier = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    float* const wt = reinterpret_cast<float*>(r2);   // [channel][3 + u][3 + v]
+    for (int i = tid; i < CS * WTH * WTW / 4; i += NT) reinterpret_cast<f4*>(wt)[i] = f4{0.f, 0.f, 0.f, 0.f};
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < NWL; ++i) {
+        const int idx = tid + i * NT, q = idx & 1, uv = idx >> 1, u = uv / K, v = uv - u * K;
+        if (idx < K * K * 2 && c0 + 4 * q < g.C) {
+            const int uu = g.flip ? K - 1 - u : u, vv = g.flip ? K - 1 - v : v;
+            float* wp = wt + (4 * q * WTH + 3 + uu) * WTW + 3 + vv;
+            const float e0 = wval[i].x, e1 = wval[i].y, e2 = wval[i].z, e3 = wval[i].w;
+            wp[0] = e0, wp[WTH * WTW] = e1, wp[2 * WTH * WTW] = e2, wp[3 * WTH * WTW] = e3;
+        }
+    }
+    commit(buf[0], 0);
+    issue(buf[0], 2);
+    lds_barrier();
+    // ---- this wavefront's A operands
+    const int ln = lane & 15, kg = lane >> 4;
+    float A[IC][JB];
+    {
+        const int di = ln >> 2, dj = ln & 3;
+        const float* wp = wt + (wv * WTH + 3 - di) * WTW + 3 + kg - dj;
+#pragma unroll
+        for (int r = 0; r < IC; ++r)
+#pragma unroll
+            for (int j = 0; j < JB; ++j) A[r][j] = wp[r * WTW + 4 * j];
+    }
+    lds_barrier();   // (the table's space becomes the result tiles)
+    const int pimg = ln / NPC, pc = ln % NPC;
+    const char* const xb = xl + (pimg * CS + wv) * CHP + (4 * pc + kg) * 4;
+    // result of a lane: patch ln, row kg, columns 4 pc .. + 3 (the four registers)
+    char* const olw = r2 + (pimg * 4 + kg) * OROWP + pc * (4 * 32 + 4) + wv * 4;
+    const int sq = tid & 1, scol = (tid >> 1) % TW, srow = (tid >> 1) / TW % 4, simg = (tid >> 1) / TW / 4;
+    const bool s_ok = scol < cols_valid && c0 + 4 * sq < g.C;
+    const char* const olr = r2 + (simg * 4 + srow) * OROWP + scol * 32 + (scol >> 2) * 4 + 16 * sq;
+    const __amdgpu_buffer_rsrc_t yrsrc = __builtin_amdgcn_make_buffer_rsrc(
+        y + (long long)b0 * img_out, (short)0, (int)(min(NI, g.B - b0) * img_out * 4), 0x00020000);
+    const uint32_t ycol = (uint32_t)simg * (uint32_t)img_out + (uint32_t)((ocol0 + scol) * g.C + c0 + 4 * sq);
+    __amdgpu_buffer_rsrc_t arsrc = xrsrc;
+    int jb0 = 0;
+    float wj0 = 0.f, wj1 = 0.f, wi0 = 0.f, wi1 = 0.f;
+    f4 addv[ADD == 2 ? 4 : 1];
+    if constexpr (ADD) {
+        arsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(add + (long long)b0 * g.AH * g.AW * g.C), (short)0,
+                                                  (int)((long long)min(NI, g.B - b0) * g.AH * g.AW * g.C * 4), 0x00020000);
+        if constexpr (ADD == 2) pool_bins(min(ocol0 + scol, g.OW - 1), g.OW, g.AW, jb0, wj0, wj1);
+        else jb0 = (ocol0 + scol) >> 1;
+    }
+    auto add_fetch = [&](int pr) {   // the bins of patch row pr's pixels
+        if constexpr (ADD == 1) {
+            const bool ok = s_ok && pr >= 0 && 4 * pr + srow < rows_valid;
+            const uint32_t off = ok ? ((uint32_t)((simg * g.AH + ((orow0 + 4 * pr + srow) >> 1)) * g.AW + jb0) * (uint32_t)g.C + (uint32_t)(c0 + 4 * sq)) * 4u : kNoRow;
+            addv[0] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(arsrc, (int)off, 0, 0));
+        } else if constexpr (ADD == 2) {
+            int ib0;
+            const int row = orow0 + 4 * pr + srow;
+            pool_bins(min(max(row, 0), g.OH - 1), g.OH, g.AH, ib0, wi0, wi1);
+            const bool ok = s_ok && pr >= 0 && 4 * pr + srow < rows_valid;
+            const uint32_t o = ((uint32_t)((simg * g.AH + ib0) * g.AW + jb0) * (uint32_t)g.C + (uint32_t)(c0 + 4 * sq)) * 4u;
+            const uint32_t dx = (uint32_t)g.C * 4u, dy = (uint32_t)(g.AW * g.C) * 4u;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const bool in = ok && ((t & 1) == 0 || wj1 != 0.f) && ((t & 2) == 0 || wi1 != 0.f);
+                const uint32_t off = in ? o + (t & 1 ? dx : 0u) + (t & 2 ? dy : 0u) : kNoRow;
+                addv[t] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(arsrc, (int)off, 0, 0));
+            }
+        }
+    };
+    auto store = [&](int pr) {   // patch row pr from its tile (outside the band: nothing)
+        const char* src = olr + (pr & 1) * OLB;
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = *reinterpret_cast<const float*>(src + 4 * e);
+        if constexpr (ADD == 1) {
+            const float a0 = addv[0].x, a1 = addv[0].y, a2 = addv[0].z, a3 = addv[0].w;
+            v[0] += 0.25f * a0, v[1] += 0.25f * a1, v[2] += 0.25f * a2, v[3] += 0.25f * a3;
+        } else if constexpr (ADD == 2) {
+            const float k00 = wi0 * wj0, k01 = wi0 * wj1, k10 = wi1 * wj0, k11 = wi1 * wj1;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                v[e] += fmaf(k11, addv[3][e], fmaf(k10, addv[2][e], fmaf(k01, addv[1][e], k00 * addv[0][e])));
+        }
+        const bool ok = s_ok && pr >= 0 && 4 * pr + srow < rows_valid;
+        const uint32_t off = ok ? (ycol + (uint32_t)((orow0 + 4 * pr + srow) * g.OW * g.C)) * 4u : kNoRow;
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, f4{v[0], v[1], v[2], v[3]}), yrsrc, (int)off, 0, 0);
+    };
+    f4 acc[PER];
+#pragma unroll
+    for (int q = 0; q < PER; ++q) acc[q] = f4{0.f, 0.f, 0.f, 0.f};
+    // step s multiplies window rows 4 s .. 4 s + 3 (for patch rows s - PER + 1 .. s) and finishes patch row s - PER + 1
+    auto compute = [&](int ps, int s) {   // ps = s mod PER
+        const char* rowp = xb + (s & 1) * 4 * RP;
+        float bv[2][JB];   // the next row's operands are read while a row is multiplied
+        auto fetch = [&](int r) {
+#pragma unroll
+            for (int j = 0; j < JB; ++j) bv[r & 1][j] = *reinterpret_cast<const float*>(rowp + r * RP + 16 * j);
+        };
+        fetch(0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (r < 3) fetch(r + 1);
+#pragma unroll
+            for (int q = 0; q < PER; ++q) {
+                if (4 * q + r >= IC) continue;
+                if (s - q >= 0 && s - q < npr) {   // (uniform)
+                    f4& a = acc[(ps - q + PER) % PER];
+#pragma unroll
+                    for (int j = 0; j < JB; ++j) a = __builtin_amdgcn_mfma_f32_16x16x4f32(A[4 * q + r < IC ? 4 * q + r : 0][j], bv[r & 1][j], a, 0, 0, 0);
+                }
+            }
+        }
+        f4& done = acc[(ps + 1) % PER];
+        const int pr = s - PER + 1;
+        if (pr >= 0) {
+            char* d = olw + (pr & 1) * OLB;
+            const float e0 = done.x, e1 = done.y, e2 = done.z, e3 = done.w;
+            *reinterpret_cast<float*>(d) = e0;
+            *reinterpret_cast<float*>(d + 32) = e1;
+            *reinterpret_cast<float*>(d + 64) = e2;
+            *reinterpret_cast<float*>(d + 96) = e3;
+        }
+        done = f4{0.f, 0.f, 0.f, 0.f};
+    };
+    auto stage = [&](int par, int s) {   // par: the buffer that the rows of step s came from
+        store(s - PER);                      // (finished by step s - 1)
+        add_fetch(s - PER + 1);              // for the next step's store
+        commit(buf[par ^ 1], s + 1);
+        issue(buf[par ^ 1], s + 3);
+    };
+    // trips of PER steps: accumulators and buffers by constant index (an odd trip leaves the two buffers swapped)
+    add_fetch(-1);
+    bool left = false;
+    for (int s0 = 0; !left; s0 += PER) {
+#pragma unroll
+        for (int t = 0; t < PER; ++t) {
+            const int s = s0 + t;
+            if (s >= nsteps) {   // (uniform)
+                left = true;
+                break;
+            }
+            lds_barrier();   // the rows of step s are in place, and everybody is done with those of s - 1
+            if (wv < 4) {
+                compute(t, s);
+                stage(t & 1, s);
+            } else {
+                stage(t & 1, s);
+                compute(t, s);
+            }
+        }
+        if constexpr (PER % 2 == 1) {
+#pragma unroll
+            for (int l = 0; l < NLD; ++l) {
+                const f4 v = buf[0][l];
+                buf[0][l] = buf[1][l], buf[1][l] = v;
+            }
+        }
+    }
+    lds_barrier();
+    store(nsteps - PER);
+}
+
+// Register bound: two workgroups on a compute unit where the filter's operands leave room, so that one's start-up
+// overlaps the other's products.
+template <int K, int ADD>
+constexpr int f32t_waves() {
+    return (K + 3) * ((K + 6) / 4) <= (ADD ? 36 : 56) ? 4 : 2;
+}
+
+template <int K, int NPC, int ADD>
+__global__ __launch_bounds__(512, (f32t_waves<K, ADD>())) void dwconv_f32t_k(const float* __restrict__ x, const float* __restrict__ w,
+                                                                     const float* __restrict__ add, float* __restrict__ y,
+                                                                     const F32Geom g) {
+    dwconv_f32_body<K, NPC, ADD>(x, w, add, y, g, blockIdx.x, gridDim.x);
+}
+
+// ------------------------------------------------------------------------------------------------
+// Host side
+
+// Patches side by side (16, or 8 or 4 in two or four images): the width whose padding of (columns x images) is smallest.
+inline int f32t_npc(int B, int OW) {
+    int best = 16;
+    long long least = -1;
+    for (int npc = 16; npc >= 4; npc /= 2) {
+        const int tw = 4 * npc, ni = 16 / npc;
+        const long long pad = (long long)cdiv(OW, tw) * tw * cdiv(B, ni) * ni;
+        if (least < 0 || pad < least) least = pad, best = npc;
+    }
+    return best;
+}
+
+// Band height: the fewest cycles for rounds of workgroups over 256 compute units (products of the band; start-up and the
+// window's first rows, which two workgroups of a unit overlap).
+template <int K>
+int f32t_band(long long per_band, int OH) {
+    constexpr int NA = (K + 3) * ((K + 6) / 4);
+    if (const char* e = tune_env("PDW_F32_BR")) return atoi(e);
+    int best = 4;
+    double cost = -1;
+    for (int br = 4; br <= (OH + 3) / 4 * 4; br += 4) {
+        const long long wgs = per_band * cdiv(OH, br);
+        const double c = (double)cdiv(wgs, 256) * (br / 4) * NA * 64 + (double)cdiv(wgs, f32t_waves<K, 0>() == 4 ? 512 : 256) * 9000;
+        if (cost < 0 || c <= cost) cost = c, best = br;
+    }
+    return best;
+}
+
+// Where the vector-ALU kernel (dwconv_tiled.h) stays, unless the pooled gradient rides here (which saves a pass over y):
+// - filters 3 and 7 once the tensor is more than a round of workgroups ([32,28,28,64]: 8.3 and 11.1 us here, 7.4 and 10.3
+//   there; [40,112,112,64]: 86 and 98, 69 and 87; [4,16,37,32]: 5.6 and 6.8, 5.9 and 7.7), 5 there unless the images fill
+//   the tiles ([40,70,70,64]: 32 here, 45 there);
+// - filters 9 and 11 on images that leave half of a tile's columns empty ([100,7,7,1152] filter 9: 66 here, 47 there; filter
+//   13 130 and 144).
+template <int K>
+bool f32t_pays(long long outputs, int OW, int npc, bool add) {
+    if (K >= 13 || add) return true;
+    const int tw = 4 * npc, filled = OW * 100 / (cdiv(OW, tw) * tw);   // per cent of the columns
+    if (K <= 7 && outputs <= 350000) return true;
+    return K == 5 ? filled >= 82 : K > 7 && filled >= 55;
+}
+
+// false: not covered
+template <int K>
+bool f32t_geom(F32Geom& g, int& npc, long long& nblocks, int B, int H, int W, int C, int PH, int PW, bool flip) {
+    g = F32Geom{B, H, W, C, H + 2 * PH - K + 1, W + 2 * PW - K + 1, PH, PW, 0, 0, 0, 0, flip ? 1 : 0, 0, 0};
+    if (g.OH < 1 || g.OW < 1 || C % 4 != 0 || B < 1) return false;
+    npc = f32t_npc(B, g.OW);
+    const int ni = 16 / npc;
+    if ((long long)H * W * C * ni > 0x0fffffffLL || (long long)g.OH * g.OW * C * ni > 0x0fffffffLL) return false;
+    g.ncolt = cdiv(g.OW, 4 * npc), g.nslices = cdiv(C, 8);
+    const long long per_band = (long long)cdiv(B, ni) * g.ncolt * g.nslices;
+    g.BR = f32t_band<K>(per_band, g.OH), g.nbands = cdiv(g.OH, g.BR);
+    nblocks = per_band * g.nbands;
+    return nblocks <= 0x7fffffffLL;
+}
+
+// -1: not covered.  add (optional): [B, AH, AW, C], AH <= OH, AW <= OW.
+template <int K>
+int launch_f32t(const void* x, const void* w, const void* add, void* y, int B, int H, int W, int C, int PH, int PW, bool flip,
+                int AH, int AW, hipStream_t s) {
+    F32Geom g;
+    int npc;
+    long long nblocks;
+    if (!f32t_geom<K>(g, npc, nblocks, B, H, W, C, PH, PW, flip)) return -1;
+    if (!f32t_pays<K>((long long)B * g.OH * g.OW * C, g.OW, npc, add != nullptr)) return -1;
+    for (const void* p : {x, w, (const void*)y, add})
+        if (reinterpret_cast<uintptr_t>(p) & 15) return -1;
+    if (add && (AH > g.OH || AW > g.OW || AH < 1 || AW < 1)) return -1;
+    g.AH = AH, g.AW = AW;
+#define PDW_F32T(NPC, A)                                                                                                   \
+    {                                                                                                                      \
+        auto kern = dwconv_f32t_k<K, NPC, A>;                                                                              \
+        static std::once_flag once;                                                                                        \
+        std::call_once(once, [&] { (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); }); \
+        constexpr size_t lds = F32Shape<K, NPC>::lds_bytes;                                                                \
+        hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(512), lds, s, (const float*)x, (const float*)w,             \
+                           (const float*)add, (float*)y, g);                                                               \
+    }
+    const int mode = !add ? 0 : g.OH == 2 * AH && g.OW == 2 * AW ? 1 : 2;
+#define PDW_F32T_M(NPC) \
+    if (mode == 0) PDW_F32T(NPC, 0) else if (mode == 1) PDW_F32T(NPC, 1) else PDW_F32T(NPC, 2)
+    if (npc == 16) {
+        PDW_F32T_M(16)
+    } else if (npc == 8) {
+        PDW_F32T_M(8)
+    } else {
+        PDW_F32T_M(4)
+    }
+#undef PDW_F32T_M
+#undef PDW_F32T
+    return check_launch("dwconv_f32t");
+}
+
+}  // namespace pdw

@@ -1,0 +1,19 @@
+// fp32 depthwise convolution on the fp32 matrix cores, 11x11 filter: the instantiations of the kernel templates in
+// dwconv_f32t.h (forward / input gradient) and dwconv_wgrad_f32t.h (weight gradient) for this size, one translation unit per
+// size so the build compiles them in parallel.
+#include "dwconv_f32t.h"
+#include "dwconv_wgrad_f32t.h"
+
+namespace pdw {
+
+int dwconv_f32t_k11(const void* x, const void* w, const void* add, void* y, int B, int H, int W, int C, int PH, int PW, bool flip,
+                   int AH, int AW, hipStream_t s) {
+    return launch_f32t<11>(x, w, add, y, B, H, W, C, PH, PW, flip, AH, AW, s);
+}
+
+int dwconv_wgrad_f32t_k11(const void* x, const void* gy, void* dw, void* ws, int B, int H, int W, int C, int PH, int PW,
+                         hipStream_t s) {
+    return launch_wgrad_f32t<11>(x, gy, dw, ws, B, H, W, C, PH, PW, s);
+}
+
+}  // namespace pdw

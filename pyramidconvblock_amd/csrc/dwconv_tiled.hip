@@ -111,8 +111,8 @@ int dwconv_tiled_launch(const void* x, const void* w, void* y, int B, int H, int
         const int r = dwconv_mfma_launch(x, w, add, pool, y, B, H, W, C, KH, KW, PH, PW, flip, dtype, s);
         if (r != -1 || add || pool) return r;   // only the matrix-core kernel has the fused forms
     }
-    if (dtype == kF32) {   // fp32 matrix cores (square odd filters 5 .. 17, C % 4 == 0)
-        const int r = dwconv_f32m_launch(x, w, y, B, H, W, C, KH, KW, PH, PW, flip, s);
+    if (dtype == kF32 && KH == KW) {
+        const int r = dwconv_f32t_launch(x, w, nullptr, y, B, H, W, C, KW, PH, PW, flip, 0, 0, s);
         if (r != -1) return r;
     }
     switch (KW) {

@@ -164,6 +164,7 @@ size_t dwconv_wgrad_tiled_workspace(int B, int H, int W, int C, int KH, int KW, 
     size_t wm = wgrad_mfma_workspace(B, H, W, C, KH, PH, PW, dtype);
     const size_t wz = wgrad_tz_enabled() ? dwconv_wgrad_tz_workspace(B, H, W, C, KH, PH, PW, dtype) : 0;
     if (wz > wm) wm = wz;
+    if (dtype == kF32) wm = dwconv_wgrad_f32t_workspace(B, H, W, C, KH, PH, PW);
     size_t wt = 0;
     switch (KH) {
         case 3: wt = dwconv_wgrad_tiled_ws_k3(B, H, W, C, PH, PW, dtype); break;
@@ -183,6 +184,10 @@ size_t dwconv_wgrad_tiled_workspace(int B, int H, int W, int C, int KH, int KW, 
 int dwconv_wgrad_tiled_launch(const void* x, const void* gy, void* dw, void* ws, int B, int H, int W, int C, int KH,
                               int KW, int PH, int PW, int dtype, hipStream_t s) {
     if (KH != KW) return -1;
+    if (dtype == kF32) {
+        const int r = dwconv_wgrad_f32t_launch(x, gy, dw, ws, B, H, W, C, KH, PH, PW, s);
+        if (r != -1) return r;
+    }
     if (wgrad_tz_enabled()) {
         const int r = dwconv_wgrad_tz_launch(x, gy, dw, ws, B, H, W, C, KH, PH, PW, dtype, s);
         if (r != -1) return r;

@@ -1,0 +1,33 @@
+"""The fp32 convolutions on the fp32 matrix cores (csrc/dwconv_f32t.h, csrc/dwconv_wgrad_f32t.h) against float64, at the edges
+of their tiles (columns, images side by side, row bands, channel slices) and with pooled gradients of any ratio."""
+import pytest
+import torch
+
+from parity import assert_close, randn
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("k", [3, 5, 7, 9, 11, 13, 15, 17])
+@pytest.mark.parametrize("shape,hw", [((1, 5, 1, 4), (2, 1)), ((5, 9, 8, 12), (4, 4)), ((3, 12, 33, 20), (6, 16)), ((2, 37, 64, 8), (37, 30)),
+                                      ((3, 21, 24, 16), (10, 12)), ((1, 50, 65, 36), (25, 32)), ((9, 18, 16, 8), (9, 8))])
+def test_f32_matrix_core_convolutions(oracle, k, shape, hw):
+    from pyramidconvblock_amd.dwconv import dwconv_dgrad, dwconv_forward, dwconv_wgrad
+
+    B, H, W, C = shape
+    gen = torch.Generator().manual_seed(k * H + W)
+    w = randn(gen, k, k, C) / k
+    for pad in (k // 2, min(k - 1, k // 2 + 2)):
+        x, gp = randn(gen, B, H, W, C), randn(gen, B, *hw, C)
+        geo = ((1, 1), (pad, pad), (1, 1))
+        y = dwconv_forward(x.cuda(), w.cuda(), *geo)
+        xn, wn = x.double().numpy(), w.double().numpy()
+        assert_close(y, oracle.dwconv_fwd(xn, wn, 1, pad, 1), torch.float32, "y")
+        g = randn(gen, *y.shape)
+        gn = g.double().numpy()
+        dx_ref = oracle.dwconv_dgrad(gn, wn, (H, W), 1, pad, 1)
+        assert_close(dwconv_dgrad(g.cuda(), w.cuda(), x.shape, *geo), dx_ref, torch.float32, "dx")
+        dx = dwconv_dgrad(g.cuda(), w.cuda(), x.shape, *geo, pooled_grad=gp.cuda())
+        assert_close(dx, dx_ref + oracle.avgpool_bwd(gp.double().numpy(), (H, W)), torch.float32, "dx + pooled")
+        dw = dwconv_wgrad(x.cuda(), g.cuda(), (k, k, C), *geo)
+        assert_close(dw, oracle.dwconv_wgrad(xn, gn, (k, k), 1, pad, 1), torch.float32, "dw")
