@@ -293,8 +293,9 @@ int pdw_dwconv_bwd3(const void* gy0, const void* w0, const void* gp, void* dx, c
         return set_error("pdw_dwconv_bwd3: workspaces of %zu and %zu bytes given, %zu and %zu needed", workspace0_bytes,
                          workspace1_bytes, need0, need1), 1;
     if (B == 0) return 0;
-    const int r = dwconv_bwd3_launch(gy0, w0, gp, dx, x0, dw0, workspace0, x1, gy1, dw1, workspace1, B, H, W, C, K, dtype,
-                                     (hipStream_t)stream);
+    const int r = !dwconv_bwd3_covers(B, W, C) ? -1
+                                               : dwconv_bwd3_launch(gy0, w0, gp, dx, x0, dw0, workspace0, x1, gy1, dw1, workspace1,
+                                                                    B, H, W, H / 2, W / 2, C, K, dtype, (hipStream_t)stream);
     if (r == -1) return set_error("pdw_dwconv_bwd3: case not covered (B=%d H=%d W=%d C=%d K=%d dtype=%d)", B, H, W, C, K, dtype), 3;
     return r;
 }
@@ -302,8 +303,9 @@ int pdw_dwconv_bwd3(const void* gy0, const void* w0, const void* gp, void* dx, c
 int pdw_dwconv_bwd3_plan(int B, int H, int W, int C, int K, int dtype, int* bands) {
     if (!bands || !valid_dtype(dtype) || B < 1 || H < 2 || W < 2 || C < 1 || K < 1 || !(K & 1) || (H & 1) || (W & 1))
         return set_error("pdw_dwconv_bwd3_plan: bad arguments (B=%d H=%d W=%d C=%d K=%d dtype=%d)", B, H, W, C, K, dtype), 1;
-    const int r = dwconv_bwd3_launch(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
-                                     nullptr, nullptr, B, H, W, C, K, dtype, nullptr, bands);
+    const int r = !dwconv_bwd3_covers(B, W, C) ? -1
+                                               : dwconv_bwd3_launch(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
+                                                                    nullptr, nullptr, nullptr, B, H, W, H / 2, W / 2, C, K, dtype, nullptr, bands);
     if (r == -1) return set_error("pdw_dwconv_bwd3_plan: case not covered"), 3;
     return r;
 }
@@ -320,7 +322,9 @@ int pdw_dwconv_fwd2(const void* x0, const void* w0, void* y0, const void* x1, co
     if (int e = check_conv("pdw_dwconv_fwd2", x0, w0, y0, B, H, W, C, K, K, 1, 1, P, P, 1, 1, dtype)) return e;
     if (int e = check_conv("pdw_dwconv_fwd2", x1, w1, y1, B, H / 2, W / 2, C, K, K, 1, 1, P, P, 1, 1, dtype)) return e;
     if (B == 0) return 0;
-    const int r = dwconv_fwd2_launch(x0, w0, y0, x1, w1, y1, B, H, W, C, K, dtype, (hipStream_t)stream);
+    const int r = !dwconv_fwd2_covers(B, H, W, C, K, dtype)
+                      ? -1
+                      : dwconv_fwd2_launch(x0, w0, y0, x1, w1, y1, B, H, W, H / 2, W / 2, C, K, dtype, (hipStream_t)stream);
     if (r == -1) return set_error("pdw_dwconv_fwd2: case not covered (B=%d H=%d W=%d C=%d K=%d dtype=%d)", B, H, W, C, K, dtype), 3;
     return r;
 }
@@ -342,9 +346,9 @@ int pdw_dwconv_fwd2_mean(const void* x0, const void* w0, void* y0, int ldy0, int
         return set_error("pdw_dwconv_fwd2_mean: gated stores need even C and ych + C/2 <= ldy for both scales (C=%d ldy=%d,%d "
                          "ych=%d,%d)", C, ldy0, ldy1, ych0, ych1), 1;
     int r = -1;
-    if (pool_branch_v8_ok(w_pool, m, parts, B, D, dtype) && !(reinterpret_cast<uintptr_t>(rowbias) & 15)) {
+    if (dwconv_fwd2_covers(B, H, W, C, K, dtype) && pool_branch_v8_ok(w_pool, m, parts, B, D, dtype) && !(reinterpret_cast<uintptr_t>(rowbias) & 15)) {
         const PoolFwdJob job{parts, nparts, B, D, 1.f / (float)P, w_pool, b_pool, b_out, m, rowbias};
-        r = dwconv_fwd2_launch(x0, w0, y0, x1, w1, y1, B, H, W, C, K, dtype, (hipStream_t)stream, ldy0, ych0, ldy1, ych1,
+        r = dwconv_fwd2_launch(x0, w0, y0, x1, w1, y1, B, H, W, H / 2, W / 2, C, K, dtype, (hipStream_t)stream, ldy0, ych0, ldy1, ych1,
                                &job);
     }
     if (r == -1)
@@ -366,7 +370,9 @@ int pdw_dwconv_fwd2_gate(const void* x0, const void* w0, void* y0, int ldy0, int
         return set_error("pdw_dwconv_fwd2_gate: need even C and ych + C/2 <= ldy (C=%d ldy=%d,%d ych=%d,%d)", C, ldy0, ldy1,
                          ych0, ych1), 1;
     if (B == 0) return 0;
-    const int r = dwconv_fwd2_launch(x0, w0, y0, x1, w1, y1, B, H, W, C, K, dtype, (hipStream_t)stream, ldy0, ych0, ldy1, ych1);
+    const int r = !dwconv_fwd2_covers(B, H, W, C, K, dtype) ? -1
+                                                            : dwconv_fwd2_launch(x0, w0, y0, x1, w1, y1, B, H, W, H / 2, W / 2, C, K, dtype,
+                                                                                 (hipStream_t)stream, ldy0, ych0, ldy1, ych1);
     if (r == -1)
         return set_error("pdw_dwconv_fwd2_gate: case not covered (B=%d H=%d W=%d C=%d K=%d dtype=%d)", B, H, W, C, K, dtype), 3;
     return r;

@@ -235,7 +235,11 @@ int forward(const Shape& s, const Saved& v, const void* x, const Weights& wt, co
             return e;
     } else {
         if (int e = pool()) return e;
-        if (int e = pdw_dwconv_fwd(v.a, w_dw0, v.c0, s.B, s.H, s.W, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, dt, stream)) return e;
+        const int r = dwconv_fwd2_launch(v.a, w_dw0, v.c0, v.xp, w_dw1, v.c1, s.B, s.H, s.W, s.h, s.w, s.I, s.K, dt, st);
+        if (r != 0 && r != -1) return r;
+        convs = r == 0;
+        if (!convs)
+            if (int e = pdw_dwconv_fwd(v.a, w_dw0, v.c0, s.B, s.H, s.W, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, dt, stream)) return e;
     }
     if (!convs)
         if (int e = pdw_dwconv_fwd(v.xp, w_dw1, v.c1, s.B, s.h, s.w, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, dt, stream)) return e;
@@ -297,36 +301,43 @@ int backward(const Shape& s, const Saved& v, const BwdWork& g, const void* gy, c
     void* gb1 = gb_pool ? gb_pool : (char*)g.gbias + (size_t)s.D * s.es;
     const int nparts = s.P / pdw_dense_colsum_rows();
     int mid = -1;
+    MeanJob mean{};
+    bool waiting = false;   // the mean branch's backward still has to run
     if (gparts) {
         mid = block_mid_bwd_launch(g.dcat, v.c0, v.c1, g.gcf, g.gch, s.B, s.H, s.W, s.h, s.w, s.I, s.I, gparts, nparts, v.m, w_pool,
                                    gb0, gb1, gw_pool, g.dmean, (float*)g.ws_pool, s.P, s.D, dt, st, s.gw());
         if (mid != 0 && mid != -1) return mid;
     }
-    if (mid == -1 && mean_any_ok(gy, w_pool, v.m, s.D, s.es) && reduce_defer_room() >= 3) {
+    if (mid == -1 && mean_any_ok(gy, w_pool, v.m, s.D, s.es) && reduce_defer_room() >= 5) {
         ColsumJob sums = colsum_plan(gy, (float*)g.ws_pool, s.B, s.P, s.D, s.es);
         float* const gs = (float*)((char*)g.ws_pool + up256((size_t)s.B * sums.n * s.D * 4));
         if (int e = gparts ? gate_pair_bwd_launch(g.dcat, v.c0, v.c1, g.gcf, g.gch, s.B, s.H, s.W, s.h, s.w, s.I, s.I, dt, st, s.gw())
                            : gate_pair_colsum_bwd_launch(g.dcat, v.c0, v.c1, g.gcf, g.gch, s.B, s.H, s.W, s.h, s.w, s.I, s.I, sums, dt, st, s.gw()))
             return e;
-        const MeanJob job{gparts ? gparts : sums.part, gparts ? nparts : sums.n, s.B, s.D, 1.f / (float)s.P, w_pool, nullptr, nullptr, v.m,
-                          nullptr, gs, g.dmean};
-        if (int e = mean_bwd_launch(job, gb0, gb1, gw_pool, dt, st)) return e;
+        mean = MeanJob{gparts ? gparts : sums.part, gparts ? nparts : sums.n, s.B, s.D, 1.f / (float)s.P, w_pool, nullptr, nullptr, v.m,
+                       nullptr, gs, g.dmean};
+        waiting = true;
     } else if (mid == -1) {
         if (int e = pool_branch_bwd_launch(gparts ? nullptr : gy, v.m, w_pool, gb0, gb1, gw_pool, g.dmean, (float*)g.ws_pool, s.B,
                                            s.P, s.D, dt, st, gparts, nparts))
             return e;
         if (int e = gate_pair_bwd_launch(g.dcat, v.c0, v.c1, g.gcf, g.gch, s.B, s.H, s.W, s.h, s.w, s.I, s.I, dt, st, s.gw())) return e;
     }
-    // the convolutions: the pooled scale's input gradient, then the rest (one launch where that is covered)
+    // the convolutions: the pooled scale's input gradient, then the rest (one launch where that is covered, the mean branch in it)
     reduce_defer_compact(seg, val);
     if (int e = pdw_dwconv_dgrad(g.gch, w_dw1, g.dxp, s.B, s.h, s.w, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, dt, stream)) return e;
-    int r = 3;
-    if (s.exact && dt != kF32) {
-        r = pdw_dwconv_bwd3(g.gcf, w_dw0, g.dxp, g.da, v.a, gw_dw0, g.ws_w0, g.b_w0, v.xp, g.gch, gw_dw1, g.ws_w1, g.b_w1, s.B,
-                            s.H, s.W, s.I, s.K, dt, stream);
-        if (r != 0 && r != 3) return r;
+    const int r = dwconv_bwd3_launch(g.gcf, w_dw0, s.exact ? g.dxp : nullptr, g.da, v.a, gw_dw0, g.ws_w0, v.xp, g.gch, gw_dw1, g.ws_w1,
+                                     s.B, s.H, s.W, s.h, s.w, s.I, s.K, dt, st, nullptr, waiting ? &mean : nullptr);
+    if (r != 0 && r != -1) return r;
+    if (waiting) {
+        reduce_defer_compact(0, 0);
+        if (int e = r == 0 ? mean_bwd_defer(mean, gb0, gb1, gw_pool, dt, st) : mean_bwd_launch(mean, gb0, gb1, gw_pool, dt, st)) return e;
+        reduce_defer_compact(seg, val);
     }
-    if (r == 3) {
+    if (r == 0) {
+        if (!s.exact)
+            if (int e = avgpool_bwd_launch(g.dxp, g.da, s.B, s.H, s.W, s.I, s.h, s.w, 1, dt, st)) return e;
+    } else {
         if (int e = pdw_dwconv_wgrad_pair(v.a, g.gcf, gw_dw0, g.ws_w0, g.b_w0, s.H, s.W, v.xp, g.gch, gw_dw1, g.ws_w1, g.b_w1,
                                           s.h, s.w, s.B, s.I, s.K, dt, stream))
             return e;

@@ -1,8 +1,10 @@
 // The three convolution launches at the end of a two-scale block's backward pass that do not depend on one another
-// (the full-scale input gradient with the pooled branch's gradient added, and the weight gradients of both scales) as
-// one launch: on a compute unit a band of each runs back to back, without two drains and launch gaps in between.
+// (the full-scale input gradient, with the pooled branch's gradient added where the pool halved the extents, and the weight
+// gradients of both scales) as one launch: on a compute unit a band of each runs back to back, without two drains and
+// launch gaps in between.  Every problem runs in the tile that its width fills better, chosen per problem at run time.
 // The kernel template and its per-filter-size launcher; dwconv_bwd3_k<K>.hip instantiate it, one file per size.
 #pragma once
+#include "dwconv_fwd2.h"
 #include "dwconv_tz.h"
 #include "dwconv_wgrad_tz.h"
 #include <algorithm>
@@ -11,32 +13,52 @@
 #include <tuple>
 #include <vector>
 
+#include "mean_any.h"
 #include "reduce_parts.h"
 
 namespace pdw {
 
+struct Bwd3Wgrad {
+    const void *x, *gy;
+    float* part;
+    WgTzGeom g;
+    int ncb;       // column blocks of a tile (8 or 5)
+    int start, n;  // first workgroup and number of workgroups
+};
+
 struct Bwd3Args {
-    const void *gy, *w, *add;   // input gradient: dx = conv^T(gy, w) + add / 4 (2x2 blocks)
+    const void *gy, *w, *add;   // input gradient: dx = conv^T(gy, w) (+ add / 4 over 2x2 blocks)
     void* dx;
-    const void *x0, *gy0, *x1, *gy1;   // weight gradients
-    float *part0, *part1;
     TzGeom gd;
-    WgTzGeom g0, g1;
-    int sd, nd, s1, n1, s0, n0;   // first workgroup and number of workgroups of the input gradient, the half scale's
-                                  // and the full scale's weight gradient
+    int npcd;                   // patches of its tile side by side (16 or 8)
+    int sd, nd;
+    Bwd3Wgrad p[2];             // full scale, pooled scale
+    MeanJob mean;               // nmean workgroups behind the others: the backward of the block's mean branch, which needs
+    int nmean;                  // nothing of this launch and whose result is read after it
 };
 
 // Each problem's workgroups are a contiguous range of the grid, in the order the launcher chose.
-template <typename T, int K, int CS, int NGA, int NCB1, int NB>
+template <typename T, int K, int CS, int NGA, int NB, int MODE>
 __global__ __launch_bounds__(512, 1) void dwconv_bwd3_k(const Bwd3Args a) {
-    const unsigned blk = blockIdx.x;
-    if (blk - (unsigned)a.sd < (unsigned)a.nd)
-        dwconv_tz_body<T, K, 16, CS, 1>((const T*)a.gy, (const T*)a.w, (const T*)a.add, nullptr, (T*)a.dx, a.gd,
-                                        (int)blk - a.sd, a.nd);
-    else if (blk - (unsigned)a.s1 < (unsigned)a.n1)
-        dwconv_wgrad_tz_body<T, NGA, NCB1, NB>((const T*)a.x1, (const T*)a.gy1, a.part1, a.g1, (int)blk - a.s1, a.n1);
-    else
-        dwconv_wgrad_tz_body<T, NGA, 8, NB>((const T*)a.x0, (const T*)a.gy0, a.part0, a.g0, (int)blk - a.s0, a.n0);
+    const int blk = blockIdx.x;
+    if (blk >= a.nd + a.p[0].n + a.p[1].n) {
+        extern __shared__ uint32_t smem[];
+        mean_bwd_body<T, 512>(a.mean, blk - a.nd - a.p[0].n - a.p[1].n, reinterpret_cast<float*>(smem));
+        return;
+    }
+    if ((unsigned)(blk - a.sd) < (unsigned)a.nd) {
+        const T *gy = (const T*)a.gy, *w = (const T*)a.w, *add = (const T*)a.add;
+        if (a.npcd == 16) dwconv_tz_body<T, K, 16, CS, MODE>(gy, w, add, nullptr, (T*)a.dx, a.gd, blk - a.sd, a.nd);
+        else dwconv_tz_body<T, K, 8, CS, MODE>(gy, w, add, nullptr, (T*)a.dx, a.gd, blk - a.sd, a.nd);
+        return;
+    }
+    const bool full = (unsigned)(blk - a.p[0].start) < (unsigned)a.p[0].n;
+    const T *x = (const T*)(full ? a.p[0].x : a.p[1].x), *gy = (const T*)(full ? a.p[0].gy : a.p[1].gy);
+    float* const part = full ? a.p[0].part : a.p[1].part;
+    const WgTzGeom g = full ? a.p[0].g : a.p[1].g;
+    const int at = blk - (full ? a.p[0].start : a.p[1].start), n = full ? a.p[0].n : a.p[1].n;
+    if ((full ? a.p[0].ncb : a.p[1].ncb) == 8) dwconv_wgrad_tz_body<T, NGA, 8, NB>(x, gy, part, g, at, n);
+    else dwconv_wgrad_tz_body<T, NGA, 5, NB>(x, gy, part, g, at, n);
 }
 
 // Band heights and grid order of the three problems.  A compute unit holds one workgroup of this launch at a time, and a
@@ -67,24 +89,24 @@ inline double bwd3_makespan(const double (&cost)[3], const long long (&count)[3]
 }
 
 template <int K, int CS>
-static Bwd3Plan bwd3_plan(int B, const TzGeom& gd, const WgTzPlan& p0, const WgTzPlan& p1) {
+static Bwd3Plan bwd3_plan(int B, const TzGeom& gd, int npcd, const WgTzPlan& p0, const WgTzPlan& p1) {
     static std::mutex mu;
     struct Key {
-        int B, H, W, C;
-        bool operator<(const Key& o) const { return std::tie(B, H, W, C) < std::tie(o.B, o.H, o.W, o.C); }
+        int B, H, W, h, w, C;
+        bool operator<(const Key& o) const { return std::tie(B, H, W, h, w, C) < std::tie(o.B, o.H, o.W, o.h, o.w, o.C); }
     };
     static std::map<Key, Bwd3Plan> cache;
-    const Key key{B, gd.OH, gd.OW, gd.C};
+    const Key key{B, gd.OH, gd.OW, p1.g.OH, p1.g.OW, gd.C};
     std::lock_guard<std::mutex> lock(mu);
     if (auto it = cache.find(key); it != cache.end()) return it->second;
     const int oh[3] = {gd.OH, p0.g.OH, p1.g.OH};
-    const long long per_band[3] = {(long long)cdiv(B, TzShape<K, 16, CS>::NI) * gd.ncolt * gd.nslices,
+    const long long per_band[3] = {(long long)cdiv(B, 16 / npcd) * gd.ncolt * gd.nslices,
                                    (long long)B * p0.g.ncolt * p0.g.nslices, (long long)B * p1.g.ncolt * p1.g.nslices};
     const int standalone[3] = {gd.nbands, p0.g.nbands, p1.g.nbands};
     constexpr int nmf = K == 17 ? 2 : 1;
     auto band_rows = [&](int i, int nb) { return (cdiv(oh[i], nb) + 3) / 4 * 4; };
     auto band_cost = [&](int i, int br) {
-        if (i == 0) return (CS == 16 ? 9.6 : 7.0) + 0.045 * br * (TzShape<K, 16, CS>::NM / 8.0);
+        if (i == 0) return tz_band_cost<K, CS>(npcd, br);
         const int ncb = i == 1 ? p0.ncb : p1.ncb;
         return 3.0 + 1.5 * nmf * (ncb == 8 ? 1.0 : 0.9) * ((br + 4) / 4);
     };
@@ -129,27 +151,30 @@ static Bwd3Plan bwd3_plan(int B, const TzGeom& gd, const WgTzPlan& p0, const WgT
     return best;
 }
 
-// -1: not covered (the caller makes the three launches).  16-bit types, C % 16 == 0, padding K / 2, the second scale
-// exactly half the first, the full scale in the wide tiles of both kernels.
+// -1: not covered (the caller makes the three launches).  16-bit types, C % 8 == 0, padding K / 2; the full scale
+// [B, H, W, C], the pooled one [B, h, w, C].  addp (optional, H = 2 h and W = 2 w): the pooled branch's gradient.
 template <int K>
 static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* dx, const void* x0, void* dw0, void* ws0,
-                       const void* x1, const void* gy1, void* dw1, void* ws1, int B, int H, int W, int C, int dtype,
-                       hipStream_t s, int* plan_out) {
+                       const void* x1, const void* gy1, void* dw1, void* ws1, int B, int H, int W, int h, int w, int C, int dtype,
+                       hipStream_t s, int* plan_out, const MeanJob* mean) {
     constexpr int CS = (2 * 4 * TzShape<K, 16, 16>::NM + 2 * 4 * TzShape<K, 16, 16>::RING) <= 160 ? 16 : 8;
     constexpr int NGA0 = (4 + 2 * ((K - 1) / 2) + 3) / 4, NGA = NGA0 < 2 ? 2 : NGA0, NB = K == 17 ? 3 : 2;
-    if (dtype == kF32 || C % 16 != 0 || (H & 1) || (W & 1) || B < 1) return -1;
-    const int P = K / 2, h = H / 2, wd = W / 2;
+    if (dtype == kF32 || C % 8 != 0 || B < 1 || H < 1 || W < 1 || h < 1 || w < 1) return -1;
+    if (addp && (H != 2 * h || W != 2 * w)) return -1;
+    const int P = K / 2;
     if (!plan_out)
-        for (const void* p : {gyf, w0, addp, (const void*)dx, x0, (const void*)ws0, x1, gy1, (const void*)ws1})
+        for (const void* p : {gyf, w0, (const void*)dx, x0, (const void*)ws0, x1, gy1, (const void*)ws1})
             if (!p || (reinterpret_cast<uintptr_t>(p) & 15)) return -1;
-    const long long pad16 = (long long)cdiv(W, 64) * 64 * B, pad8 = (long long)cdiv(W, 32) * 32 * cdiv(B, 2) * 2;
-    if (pad16 > pad8) return -1;   // the input gradient's wide tile only
-    Bwd3Args a;
+    if (reinterpret_cast<uintptr_t>(addp) & 15) return -1;
+    Bwd3Args a{};
     long long nd;
-    if (!tz_make_geom<K, 16, CS>(a.gd, nd, true, B, H, W, C, K - 1 - P, K - 1 - P, true, nullptr)) return -1;
-    WgTzPlan p0 = wgrad_tz_plan(B, H, W, C, K, P, P), p1 = wgrad_tz_plan(B, h, wd, C, K, P, P);
+    a.npcd = tz_wide_tile(B, W) ? 16 : 8;
+    if (!(a.npcd == 16 ? tz_make_geom<K, 16, CS>(a.gd, nd, true, B, H, W, C, K - 1 - P, K - 1 - P, true, nullptr)
+                       : tz_make_geom<K, 8, CS>(a.gd, nd, true, B, H, W, C, K - 1 - P, K - 1 - P, true, nullptr)))
+        return -1;
+    WgTzPlan p0 = wgrad_tz_plan(B, H, W, C, K, P, P), p1 = wgrad_tz_plan(B, h, w, C, K, P, P);
     if (!p0.ok || !p1.ok) return -1;
-    Bwd3Plan plan = bwd3_plan<K, CS>(B, a.gd, p0, p1);
+    Bwd3Plan plan = bwd3_plan<K, CS>(B, a.gd, a.npcd, p0, p1);
     if (const char* e = tune_env("PDW_BWD3_BANDS")) {   // e.g. "2,2,1,DHF": bands of D, F, H and the grid order
         if (sscanf(e, "%d,%d,%d,%3s", &plan.nb[0], &plan.nb[1], &plan.nb[2], plan.order) != 4) return -1;
     }
@@ -159,47 +184,50 @@ static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* 
     if (plan.nb[0] < 1 || plan.nb[1] < 1 || plan.nb[2] < 1) return -1;
     auto rows_of = [](int oh, int nb) { return (cdiv(oh, nb) + 3) / 4 * 4; };
     a.gd.BR = rows_of(a.gd.OH, plan.nb[0]), a.gd.nbands = cdiv(a.gd.OH, a.gd.BR);
-    nd = (long long)cdiv(B, TzShape<K, 16, CS>::NI) * a.gd.nbands * a.gd.ncolt * a.gd.nslices;
+    nd = (long long)cdiv(B, 16 / a.npcd) * a.gd.nbands * a.gd.ncolt * a.gd.nslices;
     p0.g.BR = rows_of(p0.g.OH, plan.nb[1]), p0.g.nbands = cdiv(p0.g.OH, p0.g.BR);
     p0.nblocks = (long long)B * p0.g.nslices * p0.g.ncolt * p0.g.nbands;
     p1.g.BR = rows_of(p1.g.OH, plan.nb[2]), p1.g.nbands = cdiv(p1.g.OH, p1.g.BR);
     p1.nblocks = (long long)B * p1.g.nslices * p1.g.ncolt * p1.g.nbands;
-    if (!p0.ok || !p1.ok || p0.ncb != 8 || wgrad_tz_nga(K) != NGA) return -1;
-    if (nd + p0.nblocks + p1.nblocks > 0x7fffffffLL) return -1;
+    if (wgrad_tz_nga(K) != NGA) return -1;
+    const int nmean = mean ? mean->B * mean_slices(mean->D) : 0;
+    if (nd + p0.nblocks + p1.nblocks + nmean > 0x7fffffffLL) return -1;
     if (plan_out) {
         plan_out[0] = a.gd.nbands, plan_out[1] = p0.g.nbands, plan_out[2] = p1.g.nbands;
         return 0;
     }
     a.gy = gyf, a.w = w0, a.add = addp, a.dx = dx;
-    a.x0 = x0, a.gy0 = gyf, a.x1 = x1, a.gy1 = gy1, a.part0 = (float*)ws0, a.part1 = (float*)ws1;
-    a.g0 = p0.g, a.g1 = p1.g, a.nd = (int)nd, a.n1 = (int)p1.nblocks, a.n0 = (int)p0.nblocks;
+    a.p[0] = Bwd3Wgrad{x0, gyf, (float*)ws0, p0.g, p0.ncb, 0, (int)p0.nblocks};
+    a.p[1] = Bwd3Wgrad{x1, gy1, (float*)ws1, p1.g, p1.ncb, 0, (int)p1.nblocks};
+    a.nd = (int)nd, a.nmean = nmean;
+    if (mean) a.mean = *mean;
     {
         // order of the three problems in the grid: a permutation of D (input gradient), H (half scale), F (full scale)
         const char* ord = plan.order;
         int at = 0;
         for (int i = 0; i < 3; ++i) {
             if (ord[i] == 'D') a.sd = at, at += a.nd;
-            if (ord[i] == 'H') a.s1 = at, at += a.n1;
-            if (ord[i] == 'F') a.s0 = at, at += a.n0;
+            if (ord[i] == 'H') a.p[1].start = at, at += a.p[1].n;
+            if (ord[i] == 'F') a.p[0].start = at, at += a.p[0].n;
         }
     }
-    size_t lds = TzShape<K, 16, CS>::lds_bytes;
-    if (WgTzShape<NGA, 8, NB>::lds_bytes > lds) lds = WgTzShape<NGA, 8, NB>::lds_bytes;
-    if (WgTzShape<NGA, 5, NB>::lds_bytes > lds) lds = WgTzShape<NGA, 5, NB>::lds_bytes;
-    const unsigned grid = (unsigned)(nd + p0.nblocks + p1.nblocks);
+    size_t lds = a.npcd == 16 ? TzShape<K, 16, CS>::lds_bytes : TzShape<K, 8, CS>::lds_bytes;
+    for (const Bwd3Wgrad& p : a.p) lds = std::max(lds, p.ncb == 8 ? WgTzShape<NGA, 8, NB>::lds_bytes : WgTzShape<NGA, 5, NB>::lds_bytes);
+    if (nmean) lds = std::max(lds, mean_lds(mean->D, 512));
+    const unsigned grid = (unsigned)(nd + p0.nblocks + p1.nblocks + nmean);
     static std::once_flag once[4];
-#define PDW_BWD3_GO(T, NCB1, SLOT)                                                                                        \
+#define PDW_BWD3_GO(T, MODE, SLOT)                                                                                        \
     {                                                                                                                     \
-        auto kern = dwconv_bwd3_k<T, K, CS, NGA, NCB1, NB>;                                                               \
+        auto kern = dwconv_bwd3_k<T, K, CS, NGA, NB, MODE>;                                                               \
         std::call_once(once[SLOT], [&] {                                                                                  \
             (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);         \
         });                                                                                                               \
         hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, s, a);                                                       \
     }
     if (dtype == kF16) {
-        if (p1.ncb == 8) PDW_BWD3_GO(f16_t, 8, 0) else PDW_BWD3_GO(f16_t, 5, 1)
+        if (addp) PDW_BWD3_GO(f16_t, 1, 0) else PDW_BWD3_GO(f16_t, 0, 1)
     } else {
-        if (p1.ncb == 8) PDW_BWD3_GO(bf16_t, 8, 2) else PDW_BWD3_GO(bf16_t, 5, 3)
+        if (addp) PDW_BWD3_GO(bf16_t, 1, 2) else PDW_BWD3_GO(bf16_t, 0, 3)
     }
 #undef PDW_BWD3_GO
     if (int e = check_launch("dwconv_bwd3")) return e;

@@ -545,6 +545,11 @@ static int tz_pick_band(int B, int OH, int OW, int C) {
     return best;
 }
 
+// Patches per image row, 16 (true) or 8 in two images: the width whose padding of (columns x images) is smaller, wider on ties.
+inline bool tz_wide_tile(int B, int OW) {
+    return (long long)cdiv(OW, 64) * 64 * B <= (long long)cdiv(OW, 32) * 32 * cdiv(B, 2) * 2;
+}
+
 // The geometry of a launch (false: not covered) and its number of workgroups.
 template <int K, int NPC, int CS>
 static bool tz_make_geom(TzGeom& g, long long& nblocks, bool add, int B, int H, int W, int C, int PH, int PW, bool flip,
@@ -599,9 +604,7 @@ static int launch_tz_best(const void* x, const void* w, const void* add, void* p
     if (add && ((OH | OW) & 1 || (reinterpret_cast<uintptr_t>(add) & 15) != 0)) return -1;
     if (pool && (add || flip || OH != H || OW != W || ((H | W | PH | PW) & 1) || (reinterpret_cast<uintptr_t>(pool) & 15) != 0))
         return -1;
-    // patches per image row: the width whose padding of (columns x images) is smaller, wider on ties
-    const long long pad16 = (long long)cdiv(OW, 64) * 64 * B, pad8 = (long long)cdiv(OW, 32) * 32 * cdiv(B, 2) * 2;
-    const bool wide_tile = pad16 <= pad8;
+    const bool wide_tile = tz_wide_tile(B, OW);
     // 16 channels per workgroup (two per wavefront) while the operand registers allow it, else 8
     constexpr int CS = (2 * 4 * TzShape<K, 16, 16>::NM + 2 * 4 * TzShape<K, 16, 16>::RING) <= 160 ? 16 : 8;
     if (wide_tile) return launch_tz<T, K, 16, CS>(x, w, add, pool, y, B, H, W, C, PH, PW, flip, gate, s);

@@ -78,7 +78,7 @@ __device__ __forceinline__ void dwconv_wgrad_f32_body(const float* __restrict__ 
     const int sl = bid % g.nslices, chunk = bid / g.nslices, c0 = sl * CS;
     const int u0 = chunk * g.U, u1 = min(u0 + g.U, g.units);
     const long long img_x = (long long)g.H * g.W * g.C, img_g = (long long)g.OH * g.OW * g.C;
-    constexpr uint32_t kNoCol = 0x40000000u, kNoRow = 0x80000000u;
+    constexpr uint32_t kNoRow = 0x80000000u;
 
     // ---- a thread's items: NLX of x, one of gy; (row of the group, image, column, channel quad)
     int xrow[NLX], xcol[NLX], xdst[NLX];

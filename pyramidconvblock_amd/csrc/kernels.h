@@ -151,19 +151,21 @@ int dense_bwd_pair_colsum_supported(int O, int I, int dtype);
 int dense_bwd_pair_launch(const void* gy, const void* w, const void* xin, void* dx, float* colsum, void* dw, void* ws,
                           const float* rowbias, int P, long long N, int O, int I, int dtype, hipStream_t s);
 
-// dwconv_bwd3.hip: input gradient (+ pooled branch's) of the full scale and the weight gradients of both scales of a
-// two-scale block in one launch; -1 = not covered
+// dwconv_bwd3.hip: input gradient (+ pooled branch's where the pool halved the extents, else addp = nullptr) of the full scale
+// and the weight gradients of both scales of a two-scale block in one launch, with the backward of its mean branch
+// (optional); -1 = not covered
+bool dwconv_bwd3_covers(int B, int W, int C);
 int dwconv_bwd3_launch(const void* gyf, const void* w0, const void* addp, void* dx, const void* x0, void* dw0, void* ws0,
-                       const void* x1, const void* gy1, void* dw1, void* ws1, int B, int H, int W, int C, int K, int dtype,
-                       hipStream_t s, int* plan_out = nullptr);
+                       const void* x1, const void* gy1, void* dw1, void* ws1, int B, int H, int W, int h, int w, int C, int K,
+                       int dtype, hipStream_t s, int* plan_out = nullptr, const struct MeanJob* mean = nullptr);
 
-// dwconv_fwd2.hip: the forward convolutions of both scales of a two-scale block (the second at half the extents, its
+// dwconv_fwd2.hip: the forward convolutions of both scales of a two-scale block (the second at the pooled extents h, w, its
 // own input) in one launch; -1 = not covered
 bool dwconv_fwd2_covers(int B, int H, int W, int C, int K, int dtype);
 // (ldy0 > 0: each convolution with the gate applied in its store, written at pixel strides ldy0 / ldy1 from channels
 // ych0 / ych1)
 int dwconv_fwd2_launch(const void* x0, const void* w0, void* y0, const void* x1, const void* w1, void* y1, int B, int H,
-                       int W, int C, int K, int dtype, hipStream_t s, int ldy0 = 0, int ych0 = 0, int ldy1 = 0,
+                       int W, int h, int w, int C, int K, int dtype, hipStream_t s, int ldy0 = 0, int ych0 = 0, int ldy1 = 0,
                        int ych1 = 0, const struct PoolFwdJob* mean = nullptr);
 
 }  // namespace pdw

@@ -75,12 +75,13 @@ __device__ __forceinline__ void colsum_body(const ColsumJob& j, int wg, float* r
     }
 }
 
-// sm[c] = sum over the n partials of an image, c < D; D % 4 == 0.  red: 256 float4 of LDS.  Ends with a barrier.
+// sm[c] = sum over the n partials of an image, c < D; D % 4 == 0.  red: NT float4 of LDS.  Ends with a barrier.
+template <int NT>
 __device__ __forceinline__ void image_sums(const float* __restrict__ pp, int n, int D, float* sm, float4* red) {
     const int tid = threadIdx.x, d4 = D / 4;
     int L = 16;
-    while (L < 256 && L < d4) L <<= 1;
-    const int cl = tid & (L - 1), ql = tid / L, QL = 256 / L;
+    while (L < NT && L < d4) L <<= 1;
+    const int cl = tid & (L - 1), ql = tid / L, QL = NT / L;
     for (int c0 = 0; c0 < d4; c0 += L) {   // (more than once only where QL = 1)
         const int c = c0 + cl;
         float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -129,13 +130,14 @@ struct MeanJob {
 };
 
 inline int mean_slices(int D) { return cdiv(D, kMeanOut); }
-inline size_t mean_lds(int D) { return (size_t)D * sizeof(float) + 2048 * sizeof(float); }   // sums; scratch of 8 KB
+// sums; scratch of 32 bytes a thread (backward, 16-bit) or less
+inline size_t mean_lds(int D, int nt = 256) { return (size_t)D * sizeof(float) + (size_t)nt * 32; }
 
 template <typename T>
 __device__ __forceinline__ void mean_fwd_body(const MeanJob& j, int wg, float* sm) {
     constexpr int V = 16 / (int)sizeof(T);
     const int slices = (j.D + kMeanOut - 1) / kMeanOut, b = wg / slices, sl = wg - b * slices, D = j.D, tid = threadIdx.x;
-    image_sums(j.part + (long long)b * j.n * D, j.n, D, sm, reinterpret_cast<float4*>(sm + D));
+    image_sums<256>(j.part + (long long)b * j.n * D, j.n, D, sm, reinterpret_cast<float4*>(sm + D));
     for (int c = tid; c < D; c += 256) {
         const T mv = from_f32<T>(sm[c] * j.inv_p);
         if (sl == 0) ((T*)j.m)[(long long)b * D + c] = mv;
@@ -177,14 +179,15 @@ __device__ __forceinline__ void mean_fwd_body(const MeanJob& j, int wg, float* s
     }
 }
 
-template <typename T>
+// By a workgroup of NT threads.
+template <typename T, int NT>
 __device__ __forceinline__ void mean_bwd_body(const MeanJob& j, int wg, float* sm) {
-    constexpr int V = 16 / (int)sizeof(T), CL = kMeanOut / V, OL = 256 / CL;   // column lanes, row lanes
+    constexpr int V = 16 / (int)sizeof(T), CL = kMeanOut / V, OL = NT / CL;   // column lanes, row lanes
     const int slices = (j.D + kMeanOut - 1) / kMeanOut, b = wg / slices, sl = wg - b * slices, D = j.D, tid = threadIdx.x;
     float* red = sm + D;   // [OL][64]
-    image_sums(j.part + (long long)b * j.n * D, j.n, D, sm, reinterpret_cast<float4*>(red));
+    image_sums<NT>(j.part + (long long)b * j.n * D, j.n, D, sm, reinterpret_cast<float4*>(red));
     if (sl == 0)
-        for (int c = tid; c < D; c += 256) j.gs[(long long)b * D + c] = sm[c];
+        for (int c = tid; c < D; c += NT) j.gs[(long long)b * D + c] = sm[c];
     const int cv = tid % CL, ol = tid / CL, c = sl * kMeanOut + cv * V;
     float acc[V];
 #pragma unroll
@@ -233,7 +236,9 @@ int gate_pair_mean_fwd_launch(const void* xf, const void* xh, void* y, int B, in
 // gate_pair_bwd_launch with the column sums
 int gate_pair_colsum_bwd_launch(const void* gy, const void* xf, const void* xh, void* gxf, void* gxh, int B, int H, int W, int h,
                                 int w, int I, int ldg, const ColsumJob& sums, int dtype, hipStream_t s, int gw);
-// the mean branch's backward; the gradients of the pooled layer's weight and biases join the deferred summations
+// the mean branch's backward: what its launch leaves to the deferred summations (the gradients of the pooled layer's weight
+// and biases), and the launch of its own with that
+int mean_bwd_defer(const MeanJob& mean, void* gbias, void* gbias2, void* gwp, int dtype, hipStream_t s);
 int mean_bwd_launch(const MeanJob& mean, void* gbias, void* gbias2, void* gwp, int dtype, hipStream_t s);
 
 }  // namespace pdw

@@ -816,7 +816,7 @@ __global__ __launch_bounds__(256) void gate_pair_colsum_bwd_k(const T* __restric
 template <typename T>
 __global__ __launch_bounds__(256) void mean_bwd_k(const MeanJob mean) {
     extern __shared__ float sm[];
-    mean_bwd_body<T>(mean, blockIdx.x, sm);
+    mean_bwd_body<T, 256>(mean, blockIdx.x, sm);
 }
 
 // ---------------------------------------------------------------- per-image column sums and broadcast add
@@ -1530,7 +1530,6 @@ int gate_pair_colsum_bwd_launch(const void* gy, const void* xf, const void* xh, 
 
 int mean_bwd_launch(const MeanJob& mean, void* gbias, void* gbias2, void* gwp, int dtype, hipStream_t s) {
     const int B = mean.B, D = mean.D;
-    if (reduce_defer_room() < 3) return set_error("mean_bwd: no room among the deferred summations"), 1;
     const dim3 grid((unsigned)(B * mean_slices(D)));
     switch (dtype) {
         case kF32: hipLaunchKernelGGL((mean_bwd_k<float>), grid, dim3(256), mean_lds(D), s, mean); break;
@@ -1538,6 +1537,12 @@ int mean_bwd_launch(const MeanJob& mean, void* gbias, void* gbias2, void* gwp, i
         default: hipLaunchKernelGGL((mean_bwd_k<bf16_t>), grid, dim3(256), mean_lds(D), s, mean);
     }
     if (int e = check_launch("mean_bwd")) return e;
+    return mean_bwd_defer(mean, gbias, gbias2, gwp, dtype, s);
+}
+
+int mean_bwd_defer(const MeanJob& mean, void* gbias, void* gbias2, void* gwp, int dtype, hipStream_t s) {
+    const int B = mean.B, D = mean.D;
+    if (reduce_defer_room() < 3) return set_error("mean_bwd: no room among the deferred summations"), 1;
     if (reduce_defer_outer(mean.gs, mean.m, gwp, B, D, dtype) != 0) return set_error("mean_bwd: deferred job refused"), 1;
     for (void* g : {gbias, gbias2}) {
         if (!g) continue;

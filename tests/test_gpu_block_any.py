@@ -26,3 +26,14 @@ def test_mean_branch_of_any_width(oracle, dtype, dim, k, shape):
     """The mean branch riding in the pool's and the gates' launches (csrc/mean_any.h): widths of less than one, of several
     and of more than 256 vectors of four sums, one and many ranges of positions, batches beyond its plan's."""
     _block_case(oracle, dim, k, shape, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("dim,k,shape", [
+    (16, 13, (3, 9, 70, 16)), (32, 17, (2, 33, 31, 32)), (48, 3, (5, 65, 33, 48)), (144, 9, (1, 12, 66, 144)), (80, 15, (3, 14, 32, 80)),
+    (176, 11, (9, 8, 8, 176)),
+])
+def test_convolutions_of_any_two_scales(oracle, dtype, dim, k, shape):
+    """Both scales' convolutions in one launch, forward and backward (csrc/dwconv_fwd2.h, dwconv_bwd3.h): wide and narrow tiles
+    of either scale, odd batches in two-image tiles, pooled extents that are exact halves and not, a last slice of 8 channels."""
+    _block_case(oracle, dim, k, shape, dtype)
