@@ -46,6 +46,15 @@ void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 
 Tensor bytes(size_t n, const Tensor& like) { return at::empty({(int64_t)n}, like.options().dtype(at::kByte)); }
 
+// Whether a call under these transforms belongs to the nodes below: they have no forward-mode derivative and no batching
+// rule, so such calls go on to the torch.autograd.Function forms, which refuse them.
+bool plain_call(const Tensor* in, int n) {
+    if (c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode)) return false;
+    for (int i = 0; i < n; ++i)
+        if (in[i].defined() && in[i]._fw_grad(0).defined()) return false;
+    return true;
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // The block
 
@@ -73,10 +82,12 @@ struct BlockNode : public torch::autograd::Node {
         std::lock_guard<std::mutex> lock(mutex_);
         variable_list out(kBlockInputs);
         if (!grads[0].defined()) return out;
+        // (unpacked first: a saved-tensor hook may run a whole recorded forward, as checkpointing does)
+        auto take = [&](const SavedVariable& v) { return v.unpack(shared_from_this()); };
+        Tensor xs = take(x), wu = take(w_up), wo = take(w_out), wp = take(w_pool), d0 = take(w_dw0), d1 = take(w_dw1);
+        const Tensor keep = take(saved);
         at::AutoDispatchBelowADInplaceOrView below;
-        auto take = [&](const SavedVariable& v) { return dense(v.unpack(shared_from_this())); };
-        const Tensor xs = take(x), wu = take(w_up), wo = take(w_out), wp = take(w_pool), d0 = take(w_dw0), d1 = take(w_dw1);
-        const Tensor keep = saved.unpack(shared_from_this());
+        for (Tensor* t : {&xs, &wu, &wo, &wp, &d0, &d1}) *t = dense(*t);
         const Tensor gy = dense(grads[0].to(xs.scalar_type()));
         const c10::DeviceGuard guard(xs.device());
         auto like = [](const Tensor& t) { return at::empty(t.sizes(), t.options()); };
@@ -108,6 +119,8 @@ bool block_shape(const Tensor* in, const Tensor& b_up, double s0, double s1, Blo
     if (up.size(1) != D || d0.size(1) != K || d0.size(2) != I || out.size(0) != D || out.size(1) != I || (I & 1) ||
         pool.size(0) != D || pool.size(1) != D)
         return false;
+    for (int i : {kBOut, kBPool})
+        if (in[i].defined() && (in[i].dim() != 1 || in[i].size(0) != D)) return false;
     for (int64_t e : x.sizes())
         if (e > 0x7fffffff) return false;
     const int H = (int)x.size(1), W = (int)x.size(2);
@@ -170,9 +183,9 @@ struct ConvNode : public torch::autograd::Node {
         std::lock_guard<std::mutex> lock(mutex_);
         variable_list out(2);
         if (!grads[0].defined()) return out;
+        const Tensor w_saved = w.unpack(shared_from_this()), x_saved = x.unpack(shared_from_this());   // (first, as in BlockNode)
         at::AutoDispatchBelowADInplaceOrView below;
-        const Tensor wd = dense(w.unpack(shared_from_this()));
-        const Tensor xd = dense(x.unpack(shared_from_this()).to(wd.scalar_type()));
+        const Tensor wd = dense(w_saved), xd = dense(x_saved.to(wd.scalar_type()));
         const Tensor gy = dense(grads[0].to(wd.scalar_type()));
         const c10::DeviceGuard guard(xd.device());
         const int dt = dtype_code(wd.scalar_type());
@@ -260,7 +273,7 @@ PyObject* py_block(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const double s0 = PyFloat_AsDouble(args[9]), s1 = PyFloat_AsDouble(args[10]);
     if (PyErr_Occurred()) return nullptr;
     BlockShape s;
-    if (!block_shape(in, b_up, s0, s1, &s)) Py_RETURN_NONE;
+    if (!plain_call(in, kBlockInputs) || !block_shape(in, b_up, s0, s1, &s)) Py_RETURN_NONE;
     bool grad = false;
     if (at::GradMode::is_enabled())
         for (const Tensor& t : in) grad = grad || (t.defined() && t.requires_grad());
@@ -303,12 +316,14 @@ PyObject* py_block_infer(PyObject*, PyObject* const* args, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// dwconv(x, w, (sh, sw), (ph, pw), (dh, dw))
+// dwconv(x, w, (sh, sw), (ph, pw), (dh, dw)): the convolution's output; None where DepthwiseConv2DFunction has to answer.
 PyObject* py_dwconv(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     TORCH_CHECK(n == 5, "dwconv: 5 arguments expected");
-    Tensor x, w;
-    if (!tensor_arg(args[0], &x) || !tensor_arg(args[1], &w)) return nullptr;
+    Tensor in[2];
+    if (!tensor_arg(args[0], &in[0]) || !tensor_arg(args[1], &in[1])) return nullptr;
+    const Tensor &x = in[0], &w = in[1];
+    if (!plain_call(in, 2)) Py_RETURN_NONE;
     int v[6];
     for (int i = 0; i < 3; ++i)
         if (!PyArg_ParseTuple(args[2 + i], "ii", &v[2 * i], &v[2 * i + 1])) return nullptr;

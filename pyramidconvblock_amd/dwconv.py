@@ -269,7 +269,10 @@ class OptimizedDepthwiseConv2d(torch.nn.Module):
     def forward(self, x):
         assert x.dim() == 4 and x.shape[3] == self.channels, "input must be [B,H,W,C] with matching channels"
         # DepthwiseConv2DFunction in native code (csrc/torch_ops.cpp)
-        return _lib.ext().dwconv(x, self.weight, self.stride, self.padding, self.dilation)
+        y = _lib.ext().dwconv(x, self.weight, self.stride, self.padding, self.dilation)
+        if y is None:   # under forward-mode differentiation or a functorch transform
+            y = DepthwiseConv2DFunction.apply(x, self.weight, self.stride, self.padding, self.dilation, self.weight.dtype)
+        return y
 
     def extra_repr(self):
         return (f"channels={self.channels}, kernel_size={self.kernel_size}, stride={self.stride}, "

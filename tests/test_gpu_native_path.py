@@ -61,3 +61,40 @@ def test_changed_in_place_is_noticed():
             w.add_(1)
         with pytest.raises(RuntimeError, match="modified by an inplace operation"):
             y.sum().backward()
+
+
+def _layers():
+    import pyramid_dwconv
+    import pyramidconvblock_amd
+
+    torch.manual_seed(3)
+    return [pyramid_dwconv.ConvBlock(dim=64, kernel_size=5).cuda(),
+            pyramidconvblock_amd.OptimizedDepthwiseConv2d(64, 5, padding=2).cuda()]
+
+
+@pytest.mark.parametrize("which", [0, 1])
+def test_recomputed_under_a_checkpoint(which):
+    """The unpacking of what the node saved runs the checkpointed forward again, recorded, layers of torch's own among it."""
+    from torch.utils.checkpoint import checkpoint
+
+    layer = _layers()[which]
+    m = torch.nn.Sequential(torch.nn.Linear(64, 64), torch.nn.GELU(), layer).cuda()
+    x = torch.randn(2, 8, 8, 64, device="cuda", requires_grad=True)
+    inputs = [x, *m.parameters()]
+    g = torch.randn(2, 8, 8, 64, device="cuda")
+    plain = torch.autograd.grad(m(x), inputs, g)
+    again = torch.autograd.grad(checkpoint(m, x, use_reentrant=False), inputs, g)
+    for a, b in zip(plain, again):
+        assert (a - b).abs().max() <= 1e-6 * a.abs().max()
+
+
+@pytest.mark.parametrize("which", [0, 1])
+def test_transforms_without_a_rule_are_refused(which):
+    import torch.autograd.forward_ad as fwad
+
+    layer = _layers()[which]
+    x = torch.randn(2, 8, 8, 64, device="cuda")
+    with fwad.dual_level(), pytest.raises(RuntimeError):
+        layer(fwad.make_dual(x, torch.ones_like(x)))
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(layer)(x[None])
