@@ -62,7 +62,7 @@ Shape shape_of(int B, int H, int W, int h, int w, int D, int I, int K, int dtype
     return s;
 }
 
-bool layer_ok(int K, int NO, int dtype) { return pdw_dense_supported(K, NO, dtype) != 0; }
+bool layer_ok(int K, int NO, int dtype) { return pdw_dense_supported(K, NO, dtype) != 0 || dense_wide_ok(K, NO, dtype); }
 
 // The four weights with inner channels in the padded layout, eight values to a thread: conv_up's rows, conv_out's
 // columns, the filters' channels.  A few hundred KB at most: launch latency.

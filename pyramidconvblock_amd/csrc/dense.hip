@@ -993,9 +993,10 @@ static bool dense_dims_ok(int K, int NO, int dtype) {
 }
 
 // (the tiled kernels of this file, the 128 x 128 tiles of dense_wide.hip beyond their widths, or the
-// one-tile-per-wavefront kernels of dense_any.hip: fp32, widths off multiples of 8)
+// one-tile-per-wavefront kernels of dense_any.hip: widths off multiples of 8.  fp32 of inner widths up to 256: the tiles of
+// dense_wide.hip take any, but callers of this answer have library products for the rest; block_any.hip asks dense_wide_ok)
 int dense_rows_supported(int K, int NO, int dtype) {
-    return (dense_dims_ok(K, NO, dtype) || dense_wide_ok(K, NO, dtype) || dense_any_dims_ok(K, NO)) ? 1 : 0;
+    return (dense_dims_ok(K, NO, dtype) || (dtype != kF32 && dense_wide_ok(K, NO, dtype)) || dense_any_dims_ok(K, NO)) ? 1 : 0;
 }
 
 int dense_colsum_rows() { return 32; }
@@ -1008,7 +1009,7 @@ int dense_rows_launch(const void* x, const void* w, int w_kmajor, const void* bi
     if (!dense_dims_ok(K, NO, dtype)) {
         // fp32 and the widths the tiled kernels do not take: no tile sums there, and summations that were to ride
         // in this launch get one of their own
-        if (colsum || !dense_rows_supported(K, NO, dtype)) return -1;
+        if (colsum || (!dense_rows_supported(K, NO, dtype) && !dense_wide_ok(K, NO, dtype))) return -1;
         if (rider)
             if (int e = reduce_jobs_launch(*rider, s)) return e;
         // (wide against any, 16-bit, us: [10431,200] -> 112 7.0 / 12.7, [50000,256] -> 128 9.7 / 24)

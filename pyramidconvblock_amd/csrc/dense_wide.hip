@@ -1,11 +1,11 @@
-// Dense layers of wide blocks (16-bit types, widths that are multiples of 8): all three products of an nn.Linear on
-// tiles of 128 x 128 (or 64) results, the products of conv_block.py:37, 44 for any dim.
+// Dense layers of wide blocks (16-bit types, widths that are multiples of 8) and of fp32 blocks (multiples of 4): all three
+// products of an nn.Linear on tiles of 128 x 128 (or 64) results, the products of conv_block.py:37, 44 for any dim.
 //
 //   rows:   Y[n,o]  = sum_k X[n,k] W(o,k) + bias[o] + rowbias[n / P][o]     (W stored [o][k], or [k][o] for the input gradient)
 //   wgrad:  dW[m,o] = sum_n A[n,m] B[n,o]                                    (fp32 partials over row ranges)
 //
-// What bounds it: the matrix pipe from a width of about 600 on, HBM below.  A stage is 64 values of the inner dimension
-// of both operands, moved by the direct global-to-LDS loads (16 bytes a lane, no registers in between) into one of two
+// What bounds it: the matrix pipe from a width of about 600 on, HBM below.  A stage is 128 bytes of the inner dimension
+// (64 values, in fp32 32) of both operands, moved by the direct global-to-LDS loads (16 bytes a lane, no registers in between) into one of two
 // buffers while the other is multiplied; one barrier a stage.  Operands whose inner dimension is not the contiguous one
 // (both of the weight gradient, the weight of the input gradient) are staged as they lie and read with
 // ds_read_b64_tr_b16, which hands every lane four values down a column, so there is no transposing pass over memory and
@@ -13,8 +13,13 @@
 // since their LDS side is fixed to lane order), so that the fragment reads of both kinds fall on all 64 banks once.
 // Measured (bf16, us; in brackets the library product it replaces): [16384,1152] -> 576 35 (34), its input gradient 35
 // (48), its weight gradient 32 + its share of the summation (a batched product over 128 slabs and their sum: 160 + 150).
+// fp32 (v_mfma_f32_32x32x2_f32, a sixteenth of the rate, so that the LDS and its reads down a column value by value are no
+// matter), us, dense_any.hip -> here: [100352,128] -> 64 28.7 -> 22.8, its input gradient 32.3 -> 25.6 (77 MB, 10.5 us of matrix
+// pipe); [10431,200] -> 100 16.0 -> 11.4; [20000,256] -> 128 26.5 -> 18.7; [2048,64] -> 32 5.1 -> 3.8.
 // Out-of-range rows, columns and the inner tail read as zero through the buffer descriptors; nothing is branched around.
 #include <stdint.h>
+
+#include <mutex>
 
 #include "common.h"
 #include "kernels.h"
@@ -28,11 +33,14 @@ namespace {
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef short v8s __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) char lds_char;
 
-constexpr int kBK = 64;                     // inner values per stage
+constexpr int kRowBytes = 128;              // inner bytes per stage: 64 values of 16 bits, 32 of fp32
+template <typename T>
+constexpr int kBK = kRowBytes / (int)sizeof(T);
 constexpr uint32_t kPast = 0x80000000u;     // an offset past the end of any descriptor used here
 
 __device__ __forceinline__ v16f mfma(v8s a, v8s b, v16f c, bf16_t) {
@@ -41,20 +49,30 @@ __device__ __forceinline__ v16f mfma(v8s a, v8s b, v16f c, bf16_t) {
 __device__ __forceinline__ v16f mfma(v8s a, v8s b, v16f c, f16_t) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, b), c, 0, 0, 0);
 }
+// (a lane's four values are inner values 8 kk + 4 (lane / 32) + t, of both operands: the order of a sum's terms)
+__device__ __forceinline__ v16f mfma(v8s a, v8s b, v16f c, float) {
+    const v4f x = __builtin_bit_cast(v4f, a), y = __builtin_bit_cast(v4f, b);
+    const float x0 = x.x, x1 = x.y, x2 = x.z, x3 = x.w, y0 = y.x, y1 = y.y, y2 = y.z, y3 = y.w;
+    c = __builtin_amdgcn_mfma_f32_32x32x2f32(x0, y0, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_32x32x2f32(x1, y1, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_32x32x2f32(x2, y2, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x2f32(x3, y3, c, 0, 0, 0);
+}
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void* p, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
 }
 
 // One operand of a tile: R results wide, kBK inner values per stage, staged by the workgroup's 256 threads.
-// TR = false: stored [result][inner] (pitch ld): LDS rows of 64 values, 8 pieces each, piece c of row r at c ^ (r / 2 % 8).
-// TR = true: stored [inner][result]: LDS rows of R values; pieces moved in groups of four (64 bytes) by the row, so that the
-// four rows that a transposing read takes together lie on different banks.
-template <int R, bool TR>
+// TR = false: stored [result][inner] (pitch ld): LDS rows of 128 bytes, 8 pieces each, piece c of row r at c ^ (r / 2 % 8).
+// TR = true: stored [inner][result]: LDS rows of R values; pieces moved in groups (64 bytes; fp32 128) by the row, so that the
+// rows that a read takes together (the four of a transposing read; in fp32 two, four apart) lie on different banks.
+template <typename T, int R, bool TR>
 struct Operand {
-    static constexpr int NL = R * kBK / 8 / 256;     // loads per thread and stage
-    static constexpr int CPR = TR ? R / 8 : 8;       // pieces per LDS row
-    static constexpr int BYTES = R * kBK * 2;
+    static constexpr int ES = (int)sizeof(T), VE = 16 / ES;
+    static constexpr int NL = R * kRowBytes / 16 / 256;   // loads per thread and stage
+    static constexpr int CPR = TR ? R / VE : 8;           // pieces per LDS row
+    static constexpr int BYTES = R * kRowBytes;
     __amdgpu_buffer_rsrc_t rsrc;
     uint32_t off[NL];
     int kc[NL];          // first inner value of the piece (TR: its row)
@@ -62,6 +80,7 @@ struct Operand {
 
     static __device__ __forceinline__ int swz(int row, int c) {
         if constexpr (!TR) return c ^ ((row >> 1) & 7);
+        else if constexpr (ES == 4) return c ^ (8 * ((row >> 2) & 1));
         else if constexpr (R == 128) return c ^ (4 * (row & 3));
         else return c ^ (4 * ((row >> 1) & 1));
     }
@@ -70,21 +89,21 @@ struct Operand {
         const int tid = threadIdx.x;
         if constexpr (!TR) {
             const long long rows = nres - r0 < R ? nres - r0 : R;
-            rsrc = rsrc_of(p + (r0 * ld + kb) * 2, (uint32_t)((rows - 1) * ld + (ke - kb)) * 2);
-            step = kBK * 2;
+            rsrc = rsrc_of(p + (r0 * ld + kb) * ES, (uint32_t)((rows - 1) * ld + (ke - kb)) * ES);
+            step = kRowBytes;
         } else {
-            rsrc = rsrc_of(p + (kb * ld + r0) * 2, (uint32_t)((ke - kb - 1) * ld + (nres - r0)) * 2);
-            step = (uint32_t)ld * kBK * 2;
+            rsrc = rsrc_of(p + (kb * ld + r0) * ES, (uint32_t)((ke - kb - 1) * ld + (nres - r0)) * ES);
+            step = (uint32_t)ld * kRowBytes;
         }
 #pragma unroll
         for (int j = 0; j < NL; ++j) {
             const int slot = j * 256 + tid, row = slot / CPR, c = swz(row, slot % CPR);
             if constexpr (!TR) {
-                kc[j] = c * 8;
-                off[j] = r0 + row < nres ? (uint32_t)(row * ld + c * 8) * 2 : kPast;
+                kc[j] = c * VE;
+                off[j] = r0 + row < nres ? (uint32_t)(row * ld + c * VE) * ES : kPast;
             } else {
                 kc[j] = row;
-                off[j] = r0 + c * 8 < nres ? (uint32_t)(row * ld + c * 8) * 2 : kPast;
+                off[j] = r0 + c * VE < nres ? (uint32_t)(row * ld + c * VE) * ES : kPast;
             }
         }
     }
@@ -98,11 +117,19 @@ struct Operand {
                                                      16, (int)o, 0, 0, 0);
         }
     }
-    // this lane's 8 inner values (16 kk + 8 (lane / 32) ..) of result 32 t + lane % 32
+    // this lane's 16 bytes of inner values (2 VE kk + VE (lane / 32) ..) of result 32 t + lane % 32
     static __device__ __forceinline__ v8s frag(const lds_char* buf, int t, int kk, int lane) {
         if constexpr (!TR) {
             const int row = 32 * t + (lane & 31), c = swz(row, 2 * kk + (lane >> 5));
-            return *(const __attribute__((address_space(3))) v8s*)(buf + row * 128 + c * 16);
+            return *(const __attribute__((address_space(3))) v8s*)(buf + row * kRowBytes + c * 16);
+        } else if constexpr (ES == 4) {
+            const int col = 32 * t + (lane & 31), row = 8 * kk + 4 * (lane >> 5);
+            const lds_char* const p = buf + row * (R * 4) + swz(row, col >> 2) * 16 + (col & 3) * 4;
+            float e[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) e[i] = *(const __attribute__((address_space(3))) float*)(p + i * (R * 4));
+            const v4f v = {e[0], e[1], e[2], e[3]};
+            return __builtin_bit_cast(v8s, v);
         } else {
             const int g = lane >> 4, i = lane & 15;
             const int col = 32 * t + 16 * (g & 1) + 4 * (i & 3);
@@ -125,15 +152,20 @@ struct WideArgs {
     long long M, Kd;      // results along a; inner extent
     int N, lda, ldb, P;   // results along b
     int mt, nt, splits;
-    long long kper;       // inner values per split (a multiple of kBK)
+    long long kper;       // inner values per split (a multiple of 64)
 };
 
 // Results [M][N] = sum over k of a(m,k) b(n,k).  The b operand is the matrix instruction's first, so that a lane holds
 // four consecutive n of one m.  Wavefronts 2 x 2 over the tile.
+// Workgroups of a compute unit: fp32 has registers and LDS for more than two of the smaller tiles.
+template <typename T, int BM, int BN>
+constexpr int kWideOccupancy = sizeof(T) == 4 ? (BM * BN <= 64 * 64 ? 4 : BM * BN <= 128 * 64 ? 3 : 2) : 2;
+
 template <typename T, int BM, int BN, bool TA, bool TB, bool PART>
-__global__ __launch_bounds__(256, 2) void wide_gemm_k(WideArgs g) {
-    typedef Operand<BM, TA> OpA;
-    typedef Operand<BN, TB> OpB;
+__global__ __launch_bounds__(256, (kWideOccupancy<T, BM, BN>)) void wide_gemm_k(WideArgs g) {
+    typedef Operand<T, BM, TA> OpA;
+    typedef Operand<T, BN, TB> OpB;
+    constexpr int BK = kBK<T>, KK = 4;          // inner values of a stage; fragments of it
     constexpr int STAGE = OpA::BYTES + OpB::BYTES;
     constexpr int FM = BM / 64, FN = BN / 64;   // 32-result fragments per wavefront
     extern __shared__ __align__(16) char dsm[];
@@ -152,7 +184,7 @@ __global__ __launch_bounds__(256, 2) void wide_gemm_k(WideArgs g) {
     OpB b;
     a.init((const char*)g.a, g.lda, m0, g.M, kb, ke);
     b.init((const char*)g.b, g.ldb, n0, g.N, kb, ke);
-    const int left = (int)(ke - kb), nst = (left + kBK - 1) / kBK;
+    const int left = (int)(ke - kb), nst = (left + BK - 1) / BK;
     v16f acc[FM][FN];
 #pragma unroll
     for (int i = 0; i < FM; ++i)
@@ -169,9 +201,9 @@ __global__ __launch_bounds__(256, 2) void wide_gemm_k(WideArgs g) {
         asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
         // all fragments of the stage first, then the next stage's requests, then the products: an LDS read behind a
         // request in program order would wait for it (the compiler cannot tell the two buffers apart)
-        v8s fa[kBK / 16][FM], fb[kBK / 16][FN];
+        v8s fa[KK][FM], fb[KK][FN];
 #pragma unroll
-        for (int kk = 0; kk < kBK / 16; ++kk) {
+        for (int kk = 0; kk < KK; ++kk) {
 #pragma unroll
             for (int i = 0; i < FM; ++i) fa[kk][i] = OpA::frag(cur, wm * FM + i, kk, lane);
 #pragma unroll
@@ -179,12 +211,12 @@ __global__ __launch_bounds__(256, 2) void wide_gemm_k(WideArgs g) {
         }
         __builtin_amdgcn_sched_barrier(0);
         if (st + 1 < nst) {
-            a.request(nxt, st + 1, left - (st + 1) * kBK);
-            b.request(nxt + OpA::BYTES, st + 1, left - (st + 1) * kBK);
+            a.request(nxt, st + 1, left - (st + 1) * BK);
+            b.request(nxt + OpA::BYTES, st + 1, left - (st + 1) * BK);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int kk = 0; kk < kBK / 16; ++kk)
+        for (int kk = 0; kk < KK; ++kk)
 #pragma unroll
             for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -208,7 +240,7 @@ __global__ __launch_bounds__(256, 2) void wide_gemm_k(WideArgs g) {
         }
     } else {
         // bias and per-image row in fp32, then through LDS so that the stores are whole 16-byte pieces in order
-        constexpr int TP = BN + 8;
+        constexpr int VE = 16 / (int)sizeof(T), TP = BN + VE;
         __syncthreads();
         T* const tile = reinterpret_cast<T*>(dsm);
 #pragma unroll
@@ -234,21 +266,27 @@ __global__ __launch_bounds__(256, 2) void wide_gemm_k(WideArgs g) {
                 }
         }
         __syncthreads();
-        constexpr int CPR = BN / 8;
+        constexpr int CPR = BN / VE;
 #pragma unroll
         for (int j = 0; j < BM * CPR / 256; ++j) {
             const int s = j * 256 + tid, row = s / CPR, c = s % CPR;
-            if (m0 + row < g.M && n0 + c * 8 < g.N)
-                *reinterpret_cast<uint4*>((T*)g.y + (m0 + row) * g.N + n0 + c * 8) =
-                    *reinterpret_cast<const uint4*>(tile + row * TP + c * 8);
+            if (m0 + row < g.M && n0 + c * VE < g.N)
+                *reinterpret_cast<uint4*>((T*)g.y + (m0 + row) * g.N + n0 + c * VE) =
+                    *reinterpret_cast<const uint4*>(tile + row * TP + c * VE);
         }
     }
 }
 
 template <typename T, int BM, int BN, bool TA, bool TB, bool PART>
 int wide_go(const WideArgs& g, hipStream_t s) {
-    constexpr size_t stages = (size_t)2 * (BM + BN) * kBK * 2, out = PART ? 0 : (size_t)BM * (BN + 8) * 2;
+    constexpr size_t stages = (size_t)2 * (BM + BN) * kRowBytes, out = PART ? 0 : (size_t)BM * (BN * sizeof(T) + 16);
     constexpr size_t lds = stages > out ? stages : out;
+    if constexpr (lds > 64 * 1024) {
+        static std::once_flag once;
+        std::call_once(once, [] {
+            (void)hipFuncSetAttribute((const void*)wide_gemm_k<T, BM, BN, TA, TB, PART>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        });
+    }
     hipLaunchKernelGGL((wide_gemm_k<T, BM, BN, TA, TB, PART>), dim3((unsigned)(g.mt * g.nt * g.splits)), dim3(256), lds, s, g);
     return check_launch("wide_gemm");
 }
@@ -260,15 +298,20 @@ struct WgradPlan {
     int bm, bn, mt, nt, splits;
     long long kper;
 };
-WgradPlan wgrad_plan(long long N, int M, int NO) {
+WgradPlan wgrad_plan(long long N, int M, int NO, int es) {
     WgradPlan p{M <= 64 ? 64 : 128, NO <= 64 ? 64 : 128, 0, 0, 0, 0};
-    p.mt = cdiv(M, p.bm), p.nt = cdiv(NO, p.bn);
-    long long s = 512 / ((long long)p.mt * p.nt);
-    const long long by_rows = N / (4 * kBK), by_traffic = N * (M + NO) / (4LL * M * NO);
-    if (s > by_rows) s = by_rows;
-    if (s > by_traffic) s = by_traffic;
-    if (s < 1) s = 1;
-    p.kper = ((N + s - 1) / s + kBK - 1) / kBK * kBK;
+    const long long by_rows = es == 4 ? N / 128 : N / 256, by_traffic = es * N * (M + NO) / (8LL * M * NO);
+    auto cut = [&] {
+        p.mt = cdiv(M, p.bm), p.nt = cdiv(NO, p.bn);
+        long long s = 512 / ((long long)p.mt * p.nt);
+        if (s > by_rows) s = by_rows;
+        if (s > by_traffic) s = by_traffic;
+        return s < 1 ? 1 : s;
+    };
+    long long s = cut();
+    // fp32, bound by the matrix pipe and not by what the tiles read: smaller ones where these would be too few
+    if (es == 4 && s * p.mt * p.nt < 512) p.bm = p.bn = 64, s = cut();
+    p.kper = ((N + s - 1) / s + 63) / 64 * 64;
     p.splits = (int)((N + p.kper - 1) / p.kper);
     return p;
 }
@@ -277,43 +320,67 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 
 }  // namespace
 
-bool dense_wide_ok(int K, int NO, int dtype) { return dtype != kF32 && K >= 8 && NO >= 8 && K % 8 == 0 && NO % 8 == 0; }
+bool dense_wide_ok(int K, int NO, int dtype) {
+    const int v = dtype == kF32 ? 4 : 8;   // values of 16 bytes
+    return K >= v && NO >= v && K % v == 0 && NO % v == 0;
+}
 
 // -1: not covered (widths, alignment, offsets of 2^31 bytes within a tile or a weight).
 int dense_wide_rows_launch(const void* x, const void* w, int w_kmajor, const void* bias, const float* rowbias, void* y,
                            long long N, int K, int NO, int P, int dtype, hipStream_t s) {
-    if (!dense_wide_ok(K, NO, dtype) || N > 0x7fffffffLL || (long long)K * NO * 2 > 0x7fffffffLL || K > (1 << 22) || NO > (1 << 22))
+    const int es = dtype == kF32 ? 4 : 2;
+    if (!dense_wide_ok(K, NO, dtype) || N > 0x7fffffffLL || (long long)K * NO * es > 0x7fffffffLL || K > (1 << 21) || NO > (1 << 21))
         return -1;
-    if (!aligned16(x) || !aligned16(w) || !aligned16(y) || !aligned16(rowbias) || (reinterpret_cast<uintptr_t>(bias) & 7)) return -1;
+    if (!aligned16(x) || !aligned16(w) || !aligned16(y) || !aligned16(rowbias) || (reinterpret_cast<uintptr_t>(bias) & (es == 4 ? 15 : 7)))
+        return -1;
     if (N == 0) return 0;
-    WideArgs g{x, w, bias, rowbias, y, N, K, NO, K, w_kmajor ? NO : K, P > 0 ? P : 1, 0, 0, 1, (long long)cdiv(K, kBK) * kBK};
-    // tiles of 64 rows where 128-row tiles would leave compute units without work
-    const bool small = (long long)cdiv(N, 128) * cdiv(NO, 128) < 256;
-    const int bm = small ? 64 : 128, bn = NO <= 64 ? 64 : 128;
+    WideArgs g{x, w, bias, rowbias, y, N, K, NO, K, w_kmajor ? NO : K, P > 0 ? P : 1, 0, 0, 1, (long long)cdiv(K, 64) * 64};
+    int bm, bn;
+    if (es == 4) {
+        // small tiles, four to a compute unit ([100352,128] -> 64: 22.8 us, 128 x 64 26.9, 128 x 128 41.7; never slower where
+        // it matters), but not for many rows of a short sum, which is a stream ([50000,16] -> 32: 6.4 here, 5.6 in dense_any.hip)
+        if (K < 32 && N >= 16384 && NO <= 256) return -1;
+        bm = bn = 64;
+    } else {
+        // tiles of 64 rows where 128-row tiles would leave compute units without work
+        bm = (long long)cdiv(N, 128) * cdiv(NO, 128) < 256 ? 64 : 128, bn = NO <= 64 ? 64 : 128;
+    }
     g.mt = cdiv(N, bm), g.nt = cdiv(NO, bn);
+    if ((long long)g.mt * g.nt > 0x7fffffffLL) return -1;
 #define PDW_WIDE_T(T, BM, BN) (w_kmajor ? wide_go<T, BM, BN, false, true, false>(g, s) : wide_go<T, BM, BN, false, false, false>(g, s))
 #define PDW_WIDE(BM, BN) (dtype == kF16 ? PDW_WIDE_T(f16_t, BM, BN) : PDW_WIDE_T(bf16_t, BM, BN))
+    if (es == 4) return PDW_WIDE_T(float, 64, 64);
     if (bm == 64) return bn == 64 ? PDW_WIDE(64, 64) : PDW_WIDE(64, 128);
     return bn == 64 ? PDW_WIDE(128, 64) : PDW_WIDE(128, 128);
 #undef PDW_WIDE
 #undef PDW_WIDE_T
 }
 
+// (of either type)
 size_t dense_wide_wgrad_workspace(long long N, int M, int NO) {
-    return N < 1 || M < 1 || NO < 1 ? 0 : (size_t)wgrad_plan(N, M, NO).splits * M * NO * sizeof(float);
+    if (N < 1 || M < 1 || NO < 1) return 0;
+    const int a = wgrad_plan(N, M, NO, 2).splits, b = wgrad_plan(N, M, NO, 4).splits;
+    return (size_t)(a > b ? a : b) * M * NO * sizeof(float);
 }
 
 int dense_wide_wgrad_launch(const void* a, const void* b, void* dw, void* ws, long long N, int M, int NO, int dtype, hipStream_t s) {
     if (!dense_wide_ok(M, NO, dtype) || N < 1 || !aligned16(a) || !aligned16(b) || !aligned16(ws)) return -1;
-    const WgradPlan p = wgrad_plan(N, M, NO);
-    if (p.kper * (M > NO ? M : NO) * 2 > 0x7fffffffLL) return -1;
+    const int es = dtype == kF32 ? 4 : 2;
+    // (fp32 widths up to 256: one 32 x 32 tile a wavefront, dense_any.hip, needs no LDS and is as fast or faster, [100352] rows of
+    // 128 x 64 24.3 us with its summation against 27.9, [784] of 248 x 124 7.1 against 9.6)
+    if (es == 4 && M <= 256 && NO <= 256) return -1;
+    const WgradPlan p = wgrad_plan(N, M, NO, es);
+    if (p.kper * (M > NO ? M : NO) * es > 0x7fffffffLL) return -1;
     WideArgs g{a, b, nullptr, nullptr, ws, M, N, NO, M, NO, 1, p.mt, p.nt, p.splits, p.kper};
-#define PDW_WIDE_W(BM, BN) \
-    (dtype == kF16 ? wide_go<f16_t, BM, BN, true, true, true>(g, s) : wide_go<bf16_t, BM, BN, true, true, true>(g, s))
+#define PDW_WIDE_W(BM, BN)                                                 \
+    (dtype == kF32   ? wide_go<float, BM, BN, true, true, true>(g, s)      \
+     : dtype == kF16 ? wide_go<f16_t, BM, BN, true, true, true>(g, s)      \
+                     : wide_go<bf16_t, BM, BN, true, true, true>(g, s))
     const int e = p.bm == 64 ? (p.bn == 64 ? PDW_WIDE_W(64, 64) : PDW_WIDE_W(64, 128))
                              : (p.bn == 64 ? PDW_WIDE_W(128, 64) : PDW_WIDE_W(128, 128));
 #undef PDW_WIDE_W
     if (e) return e;
+    if (dtype == kF32) return wgrad_reduce_launch<float>((const float*)ws, dw, p.splits, M * NO, s);
     if (dtype == kF16) return wgrad_reduce_launch<f16_t>((const float*)ws, dw, p.splits, M * NO, s);
     return wgrad_reduce_launch<bf16_t>((const float*)ws, dw, p.splits, M * NO, s);
 }

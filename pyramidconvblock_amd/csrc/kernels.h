@@ -140,7 +140,7 @@ int dense_any_rows_launch(const void* x, const void* w, int w_kmajor, const void
 bool dense_any_wgrad_dims_ok(int M, int NO);
 int dense_any_wgrad_launch(const void* a, const void* b, void* dw, void* ws, long long N, int M, int NO, int dtype,
                            int max_chunks, hipStream_t s);
-// dense_wide.hip: tiles of 128 x 128 results, 16-bit types, widths that are multiples of 8; -1 = not covered
+// dense_wide.hip: tiles of 128 x 128 results, widths that are multiples of 16 bytes; -1 = not covered
 bool dense_wide_ok(int K, int NO, int dtype);
 int dense_wide_rows_launch(const void* x, const void* w, int w_kmajor, const void* bias, const float* rowbias, void* y,
                            long long N, int K, int NO, int P, int dtype, hipStream_t s);

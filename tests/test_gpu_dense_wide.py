@@ -1,5 +1,5 @@
-"""The 128 x 128-tile dense kernels (csrc/dense_wide.hip: 16-bit layers wider than 128) against float64, at the edges of
-their tiles, stages and row ranges."""
+"""The 128 x 128-tile dense kernels (csrc/dense_wide.hip: 16-bit layers wider than 128, fp32 layers) against float64, at the
+edges of their tiles, stages and row ranges."""
 import pytest
 import torch
 
@@ -8,13 +8,10 @@ from parity import assert_close, randn
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("K,NO", [(136, 8), (8, 264), (200, 112), (256, 128), (520, 264), (64, 192), (1152, 576)])
-@pytest.mark.parametrize("N,P", [(1, 1), (63, 7), (130, 65), (1000, 250), (4097, 4097)])
-def test_dense_wide_layers(dtype, K, NO, N, P):
+def _layers(dtype, K, NO, N, P):
     from pyramidconvblock_amd import ops
 
-    assert ops.dense_supported(K, NO, dtype) and ops.dense_supported(NO, K, dtype)
+    assert dtype == torch.float32 or (ops.dense_supported(K, NO, dtype) and ops.dense_supported(NO, K, dtype))
     gen = torch.Generator().manual_seed(K + NO + N)
     x, g = randn(gen, N, K).to(dtype), randn(gen, N, NO).to(dtype)
     w, b = (randn(gen, NO, K) / K ** 0.5).to(dtype), randn(gen, NO).to(dtype)
@@ -26,3 +23,17 @@ def test_dense_wide_layers(dtype, K, NO, N, P):
     assert_close(dx, (g.double() @ w.double()).numpy(), dtype, "input gradient", 0.5)
     dw = ops.dense_wgrad(g.cuda(), x.cuda())
     assert_close(dw, (g.double().t() @ x.double()).numpy(), dtype, "weight gradient", 0.5)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K,NO", [(136, 8), (8, 264), (200, 112), (256, 128), (520, 264), (64, 192), (1152, 576)])
+@pytest.mark.parametrize("N,P", [(1, 1), (63, 7), (130, 65), (1000, 250), (4097, 4097)])
+def test_dense_wide_layers(dtype, K, NO, N, P):
+    _layers(dtype, K, NO, N, P)
+
+
+@pytest.mark.parametrize("K,NO", [(4, 4), (132, 36), (100, 200), (128, 64), (64, 128), (260, 576)])
+@pytest.mark.parametrize("N,P", [(1, 1), (63, 7), (1000, 250), (4097, 4097), (70001, 35001)])
+def test_dense_wide_fp32_layers(K, NO, N, P):
+    """Every tile (70001 rows: 128 high), remainders of 4 in both widths, ranges of rows that end within a stage."""
+    _layers(torch.float32, K, NO, N, P)
