@@ -311,7 +311,8 @@ inline WgF32Plan wgrad_f32t_plan(int B, int H, int W, int C, int K, int PH, int 
     const int ni = p.nbi > 2 ? 1 : 4 / p.nbi;
     if ((long long)H * W * C * ni > 0x1fffffffLL || (long long)g.OH * g.OW * C * ni > 0x1fffffffLL) return p;
     g.ncolt = cdiv(g.OW, 16 * p.nbi - 8), g.nslices = cdiv(C, 8);
-    // two workgroups for every compute unit: several units each, or row bands of at least 12 rows
+    // two workgroups for every compute unit: several units each, or row bands of at least 12 rows (5 where those would not
+    // give every compute unit one: the chain of a band's steps is all there is to wait for)
     const int want = 512;
     const long long whole = (long long)cdiv(B, ni) * g.ncolt * g.nslices;
     g.BR = g.OH;
@@ -319,7 +320,8 @@ inline WgF32Plan wgrad_f32t_plan(int B, int H, int W, int C, int K, int PH, int 
         g.U = (int)(whole / want);
     } else if (whole < want) {
         int nb = (int)(want / whole);
-        if (nb > g.OH / 12) nb = g.OH / 12;
+        const int least_rows = whole * (g.OH / 12) >= 256 ? 12 : 5;
+        if (nb > g.OH / least_rows) nb = g.OH / least_rows;
         if (nb > 1) g.BR = (cdiv(g.OH, nb) + 1 + 3) / 4 * 4 - 1;   // (rows + 1 whole groups of four)
     }
     g.nbands = cdiv(g.OH, g.BR);
