@@ -37,3 +37,10 @@ def test_dense_wide_layers(dtype, K, NO, N, P):
 def test_dense_wide_fp32_layers(K, NO, N, P):
     """Every tile (70001 rows: 128 high), remainders of 4 in both widths, ranges of rows that end within a stage."""
     _layers(torch.float32, K, NO, N, P)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K,NO", [(264, 136), (320, 200), (256, 384)])
+def test_dense_wide_columns_of_192(dtype, K, NO):
+    """Tiles of 128 x 192: rows enough for one round of them to save one of the narrower ones, remainders in both."""
+    _layers(dtype, K, NO, 257 * 128 + 5, 257 * 128 + 5)
