@@ -358,4 +358,80 @@ int launch_wgrad_f32t(const void* x, const void* gy, void* dw, void* ws, int B, 
     return wgrad_reduce_launch<float>((const float*)ws, (float*)dw, p.nchunks, K * K * C, s);
 }
 
+// The weight gradients of two problems (a block's scales) in one grid, each in the tile of its plan: neither depends on the
+// other, and at the sizes where one of them leaves compute units without work the launch takes as long as the longer one
+// ([2,32,32,32] and its half scale, filter 7, us: 10.6 + 12.4 -> 12.6; [3,57,61,100], filter 15: 25.2 + 12.0 -> 26.0;
+// [32,56,56,64], filter 13, where both fill the chip: 57.5 + 25.6 -> 76.1).
+struct WgF32Problem {
+    const float *x, *gy;
+    float* part;
+    WgF32Geom g;
+    int nbi, n;   // 16-column blocks of a tile; workgroups
+};
+struct WgF32Pair {
+    WgF32Problem p[2];
+};
+
+// Tiles that leave room for two workgroups on a compute unit: the pair is for those.
+template <int K>
+constexpr bool wg_f32t_pairs(int nbi) {
+    return (nbi == 4   ? wg_f32t_waves<K, 4, 1>()
+            : nbi == 3 ? wg_f32t_waves<K, 3, 1>()
+            : nbi == 2 ? wg_f32t_waves<K, 2, 2>()
+                       : wg_f32t_waves<K, 1, 4>()) == 4;
+}
+
+template <int K>
+__global__ __launch_bounds__(512, 4) void dwconv_wgrad_f32t_pair_k(const WgF32Pair a) {
+    const bool first = (int)blockIdx.x < a.p[0].n;
+    const float *x = first ? a.p[0].x : a.p[1].x, *gy = first ? a.p[0].gy : a.p[1].gy;
+    float* const part = first ? a.p[0].part : a.p[1].part;
+    const WgF32Geom g = first ? a.p[0].g : a.p[1].g;
+    const int nbi = first ? a.p[0].nbi : a.p[1].nbi, at = (int)blockIdx.x - (first ? 0 : a.p[0].n), n = first ? a.p[0].n : a.p[1].n;
+    if constexpr (wg_f32t_pairs<K>(4))
+        if (nbi == 4) return dwconv_wgrad_f32_body<K, 4, 1>(x, gy, part, g, at, n);
+    if constexpr (wg_f32t_pairs<K>(3))
+        if (nbi == 3) return dwconv_wgrad_f32_body<K, 3, 1>(x, gy, part, g, at, n);
+    if constexpr (wg_f32t_pairs<K>(2))
+        if (nbi == 2) return dwconv_wgrad_f32_body<K, 2, 2>(x, gy, part, g, at, n);
+    if constexpr (wg_f32t_pairs<K>(1))
+        if (nbi == 1) return dwconv_wgrad_f32_body<K, 1, 4>(x, gy, part, g, at, n);
+}
+
+// -1: not covered (the caller makes two launches).
+template <int K>
+int launch_wgrad_f32t_pair(const void* x0, const void* gy0, void* dw0, void* ws0, int H0, int W0, const void* x1, const void* gy1,
+                           void* dw1, void* ws1, int H1, int W1, int B, int C, int P, hipStream_t s) {
+    const WgF32Plan plan[2] = {wgrad_f32t_plan(B, H0, W0, C, K, P, P), wgrad_f32t_plan(B, H1, W1, C, K, P, P)};
+    const void *const x[2] = {x0, x1}, *const gy[2] = {gy0, gy1};
+    void *const dw[2] = {dw0, dw1}, *const ws[2] = {ws0, ws1};
+    WgF32Pair a{};
+    size_t lds = 0;
+    long long n = 0;
+    for (int i = 0; i < 2; ++i) {
+        const WgF32Plan& p = plan[i];
+        if (!p.ok || !wg_f32t_pairs<K>(p.nbi)) return -1;
+        for (const void* q : {x[i], gy[i], (const void*)ws[i]})
+            if (reinterpret_cast<uintptr_t>(q) & 15) return -1;
+        const int mine = p.nchunks * p.g.nslices;
+        a.p[i] = WgF32Problem{(const float*)x[i], (const float*)gy[i], (float*)ws[i], p.g, p.nbi, mine};
+        n += mine;
+        const size_t need = p.nbi == 4   ? WgF32Shape<K, 4, 1>::lds_bytes
+                            : p.nbi == 3 ? WgF32Shape<K, 3, 1>::lds_bytes
+                            : p.nbi == 2 ? WgF32Shape<K, 2, 2>::lds_bytes
+                                         : WgF32Shape<K, 1, 4>::lds_bytes;
+        if (need > lds) lds = need;
+    }
+    if (n > 0x7fffffffLL) return -1;
+    static std::once_flag once;
+    std::call_once(once, [] {
+        (void)hipFuncSetAttribute((const void*)dwconv_wgrad_f32t_pair_k<K>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    });
+    hipLaunchKernelGGL(dwconv_wgrad_f32t_pair_k<K>, dim3((unsigned)n), dim3(512), lds, s, a);
+    if (int e = check_launch("dwconv_wgrad_f32t_pair")) return e;
+    for (int i = 0; i < 2; ++i)
+        if (int e = wgrad_reduce_launch<float>((const float*)ws[i], (float*)dw[i], plan[i].nchunks, K * K * C, s)) return e;
+    return 0;
+}
+
 }  // namespace pdw

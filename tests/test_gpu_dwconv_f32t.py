@@ -31,3 +31,18 @@ def test_f32_matrix_core_convolutions(oracle, k, shape, hw):
         assert_close(dx, dx_ref + oracle.avgpool_bwd(gp.double().numpy(), (H, W)), torch.float32, "dx + pooled")
         dw = dwconv_wgrad(x.cuda(), g.cuda(), (k, k, C), *geo)
         assert_close(dw, oracle.dwconv_wgrad(xn, gn, (k, k), 1, pad, 1), torch.float32, "dw")
+
+
+@pytest.mark.parametrize("k", [3, 9, 13, 15, 17])
+@pytest.mark.parametrize("shape,hw", [((2, 32, 32, 32), (16, 16)), ((3, 57, 61, 100), (28, 30)), ((5, 13, 18, 12), (6, 9)), ((9, 40, 56, 8), (20, 28))])
+def test_weight_gradients_of_two_scales_in_one_launch(k, shape, hw):
+    """The pair launch's results are bitwise the single launches'."""
+    from pyramidconvblock_amd.dwconv import dwconv_wgrad, dwconv_wgrad_pair
+
+    B, H, W, C = shape
+    gen = torch.Generator().manual_seed(k + W)
+    x0, g0 = (randn(gen, B, H, W, C).cuda() for _ in range(2))
+    x1, g1 = (randn(gen, B, *hw, C).cuda() for _ in range(2))
+    geo = ((1, 1), (k // 2, k // 2), (1, 1))
+    d0, d1 = dwconv_wgrad_pair(x0, g0, x1, g1, (k, k, C))
+    assert torch.equal(d0, dwconv_wgrad(x0, g0, (k, k, C), *geo)) and torch.equal(d1, dwconv_wgrad(x1, g1, (k, k, C), *geo))
