@@ -235,7 +235,8 @@ int forward(const Shape& s, const Saved& v, const void* x, const Weights& wt, co
             return e;
     } else {
         if (int e = pool()) return e;
-        const int r = dwconv_fwd2_launch(v.a, w_dw0, v.c0, v.xp, w_dw1, v.c1, s.B, s.H, s.W, s.h, s.w, s.I, s.K, dt, st);
+        const int r = dt == kF32 ? dwconv_f32t_pair_launch(v.a, w_dw0, v.c0, s.H, s.W, v.xp, w_dw1, v.c1, s.h, s.w, s.B, s.I, s.K, st)
+                                 : dwconv_fwd2_launch(v.a, w_dw0, v.c0, v.xp, w_dw1, v.c1, s.B, s.H, s.W, s.h, s.w, s.I, s.K, dt, st);
         if (r != 0 && r != -1) return r;
         convs = r == 0;
         if (!convs)

@@ -413,4 +413,62 @@ int launch_f32t(const void* x, const void* w, const void* add, void* y, int B, i
     return check_launch("dwconv_f32t");
 }
 
+// The forward convolutions of two problems (a block's scales, the second on the pooled input) in one grid, each in its own
+// tiles and bands, as the separate launches would run them: where those leave compute units without work, the pair takes as
+// long as the longer one (us: [2,32,32,32] and its half scale, filter 7, 7.1 + 5.8 -> 6.4; [3,57,61,100], filter 15, 17.6 +
+// 10.7 -> 25.4; [32,56,56,64], filter 13, 39.9 + 16.0 -> 52.7).
+struct F32Problem {
+    const float *x, *w;
+    float* y;
+    F32Geom g;
+    int npc, n;   // patches of a tile side by side; workgroups
+};
+struct F32Pair {
+    F32Problem p[2];
+};
+
+template <int K>
+__global__ __launch_bounds__(512, (f32t_waves<K, 0>())) void dwconv_f32t_pair_k(const F32Pair a) {
+    const bool first = (int)blockIdx.x < a.p[0].n;
+    const float *x = first ? a.p[0].x : a.p[1].x, *w = first ? a.p[0].w : a.p[1].w;
+    float* const y = first ? a.p[0].y : a.p[1].y;
+    const F32Geom g = first ? a.p[0].g : a.p[1].g;
+    const int npc = first ? a.p[0].npc : a.p[1].npc, at = (int)blockIdx.x - (first ? 0 : a.p[0].n), n = first ? a.p[0].n : a.p[1].n;
+    if (npc == 16) dwconv_f32_body<K, 16, 0>(x, w, nullptr, y, g, at, n);
+    else if (npc == 8) dwconv_f32_body<K, 8, 0>(x, w, nullptr, y, g, at, n);
+    else dwconv_f32_body<K, 4, 0>(x, w, nullptr, y, g, at, n);
+}
+
+// -1: not covered (the caller makes two launches).  Padding K / 2.
+template <int K>
+int launch_f32t_pair(const void* x0, const void* w0, void* y0, int H0, int W0, const void* x1, const void* w1, void* y1, int H1,
+                     int W1, int B, int C, hipStream_t s) {
+    const void *const x[2] = {x0, x1}, *const w[2] = {w0, w1};
+    void* const y[2] = {y0, y1};
+    const int H[2] = {H0, H1}, W[2] = {W0, W1};
+    F32Pair a{};
+    size_t lds = 0;
+    long long total = 0;
+    for (int i = 0; i < 2; ++i) {
+        long long n;
+        F32Problem& p = a.p[i];
+        if (!f32t_geom<K>(p.g, p.npc, n, B, H[i], W[i], C, K / 2, K / 2, false)) return -1;
+        if (!f32t_pays<K>((long long)B * H[i] * W[i] * C, W[i], p.npc, false)) return -1;
+        for (const void* q : {x[i], w[i], (const void*)y[i]})
+            if (reinterpret_cast<uintptr_t>(q) & 15) return -1;
+        p.x = (const float*)x[i], p.w = (const float*)w[i], p.y = (float*)y[i];
+        total += n;
+        if (total > 0x7fffffffLL) return -1;
+        p.n = (int)n;
+        const size_t need = p.npc == 16 ? F32Shape<K, 16>::lds_bytes : p.npc == 8 ? F32Shape<K, 8>::lds_bytes : F32Shape<K, 4>::lds_bytes;
+        if (need > lds) lds = need;
+    }
+    static std::once_flag once;
+    std::call_once(once, [] {
+        (void)hipFuncSetAttribute((const void*)dwconv_f32t_pair_k<K>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    });
+    hipLaunchKernelGGL(dwconv_f32t_pair_k<K>, dim3((unsigned)total), dim3(512), lds, s, a);
+    return check_launch("dwconv_f32t_pair");
+}
+
 }  // namespace pdw

@@ -6,6 +6,8 @@ namespace pdw {
 #define PDW_DECL(K)                                                                                                        \
     int dwconv_f32t_k##K(const void* x, const void* w, const void* add, void* y, int B, int H, int W, int C, int PH,       \
                          int PW, bool flip, int AH, int AW, hipStream_t s);                                                \
+    int dwconv_f32t_pair_k##K(const void* x0, const void* w0, void* y0, int H0, int W0, const void* x1, const void* w1,    \
+                              void* y1, int H1, int W1, int B, int C, hipStream_t s);                                      \
     int dwconv_wgrad_f32t_k##K(const void* x, const void* gy, void* dw, void* ws, int B, int H, int W, int C, int PH,      \
                                int PW, hipStream_t s);                                                                     \
     int dwconv_wgrad_f32t_pair_k##K(const void* x0, const void* gy0, void* dw0, void* ws0, int H0, int W0, const void* x1, \
@@ -29,6 +31,13 @@ PDW_DECL(3) PDW_DECL(5) PDW_DECL(7) PDW_DECL(9) PDW_DECL(11) PDW_DECL(13) PDW_DE
 int dwconv_f32t_launch(const void* x, const void* w, const void* add, void* y, int B, int H, int W, int C, int K, int PH, int PW,
                        bool flip, int AH, int AW, hipStream_t s) {
 #define CALL(N) dwconv_f32t_k##N(x, w, add, y, B, H, W, C, PH, PW, flip, AH, AW, s)
+    PDW_BY_SIZE(CALL)
+#undef CALL
+}
+
+int dwconv_f32t_pair_launch(const void* x0, const void* w0, void* y0, int H0, int W0, const void* x1, const void* w1, void* y1, int H1,
+                            int W1, int B, int C, int K, hipStream_t s) {
+#define CALL(N) dwconv_f32t_pair_k##N(x0, w0, y0, H0, W0, x1, w1, y1, H1, W1, B, C, s)
     PDW_BY_SIZE(CALL)
 #undef CALL
 }

@@ -11,6 +11,11 @@ int dwconv_f32t_k11(const void* x, const void* w, const void* add, void* y, int 
     return launch_f32t<11>(x, w, add, y, B, H, W, C, PH, PW, flip, AH, AW, s);
 }
 
+int dwconv_f32t_pair_k11(const void* x0, const void* w0, void* y0, int H0, int W0, const void* x1, const void* w1, void* y1, int H1,
+                        int W1, int B, int C, hipStream_t s) {
+    return launch_f32t_pair<11>(x0, w0, y0, H0, W0, x1, w1, y1, H1, W1, B, C, s);
+}
+
 int dwconv_wgrad_f32t_k11(const void* x, const void* gy, void* dw, void* ws, int B, int H, int W, int C, int PH, int PW,
                          hipStream_t s) {
     return launch_wgrad_f32t<11>(x, gy, dw, ws, B, H, W, C, PH, PW, s);

@@ -130,6 +130,9 @@ int dense_wgrad_launch(const void* a, const void* b, void* dw, void* ws, long lo
 // add (optional): y += the gradient of an average pool of y's pixels to [AH, AW]
 int dwconv_f32t_launch(const void* x, const void* w, const void* add, void* y, int B, int H, int W, int C, int K, int PH, int PW,
                        bool flip, int AH, int AW, hipStream_t s);
+// the forward of two problems of one batch and channel count, padding K / 2, in one launch
+int dwconv_f32t_pair_launch(const void* x0, const void* w0, void* y0, int H0, int W0, const void* x1, const void* w1, void* y1, int H1,
+                            int W1, int B, int C, int K, hipStream_t s);
 size_t dwconv_wgrad_f32t_workspace(int B, int H, int W, int C, int K, int PH, int PW);
 int dwconv_wgrad_f32t_launch(const void* x, const void* gy, void* dw, void* ws, int B, int H, int W, int C, int K, int PH, int PW,
                              hipStream_t s);

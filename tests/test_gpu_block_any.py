@@ -37,3 +37,11 @@ def test_convolutions_of_any_two_scales(oracle, dtype, dim, k, shape):
     """Both scales' convolutions in one launch, forward and backward (csrc/dwconv_fwd2.h, dwconv_bwd3.h): wide and narrow tiles
     of either scale, odd batches in two-image tiles, pooled extents that are exact halves and not, a last slice of 8 channels."""
     _block_case(oracle, dim, k, shape, dtype)
+
+
+@pytest.mark.parametrize("k", [3, 9, 13, 17])
+@pytest.mark.parametrize("dim,shape", [(16, (1, 12, 64, 16)), (24, (3, 33, 31, 24)), (8, (5, 17, 16, 8)), (40, (2, 9, 130, 40))])
+def test_fp32_convolutions_of_two_scales(oracle, k, dim, shape):
+    """Both scales' fp32 convolutions in one launch (csrc/dwconv_f32t.h): tiles of one, two and four images, two column tiles,
+    odd batches and extents, slices of 4 channels."""
+    _block_case(oracle, dim, k, shape, torch.float32)
