@@ -1,5 +1,6 @@
-// Dense layers for the shapes that the tiled matrix-core kernels of dense.hip do not take: fp32, and 16-bit layers
-// whose widths are multiples of 4 only or wider than 128 (nn.Linear of conv_block.py:37, 44 on any dim and in fp32).
+// Dense layers for the shapes that the tiled matrix-core kernels of dense.hip and dense_wide.hip do not take: 16-bit layers
+// whose widths are multiples of 4 only, fp32 weight gradients up to 256 wide, fp32 rows of short sums and of pointers off 16
+// bytes (nn.Linear of conv_block.py:37, 44 on any dim).
 //
 //   rows:  Y[n,o] = sum_k X[n,k] * W(o,k) + bias[o] + rowbias[n / P][o]
 //   wgrad: dW[m,o] = sum_n A[n,m] * B[n,o]
