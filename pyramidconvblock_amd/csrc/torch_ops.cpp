@@ -12,6 +12,7 @@
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include "../../include/pdw.h"
 
@@ -46,9 +47,11 @@ void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 
 Tensor bytes(size_t n, const Tensor& like) { return at::empty({(int64_t)n}, like.options().dtype(at::kByte)); }
 
-// Whether a call under these transforms belongs to the nodes below: they have no forward-mode derivative and no batching
-// rule, so such calls go on to the torch.autograd.Function forms, which refuse them.
+// Whether a call belongs to the nodes below.  They have no forward-mode derivative and no batching rule, so such calls go
+// on to the torch.autograd.Function forms, which refuse them; and a trace (torch.jit.trace) would record of them the
+// allocation of the result alone, where a Function becomes a node of the graph that calls it again.
 bool plain_call(const Tensor* in, int n) {
+    if (torch::jit::tracer::isTracing()) return false;
     if (c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode)) return false;
     for (int i = 0; i < n; ++i)
         if (in[i].defined() && in[i]._fw_grad(0).defined()) return false;
@@ -261,8 +264,8 @@ bool tensor_arg(PyObject* o, Tensor* t) {
     return true;
 }
 
-// block(x, w_up, b_up, w_out, b_out, w_pool, b_pool, w_dw0, w_dw1, s0, s1): the block's output; None where the library's
-// block calls do not cover the case; True where no gradient is wanted and its inference call (block_infer) covers it.
+// block(x, w_up, b_up, w_out, b_out, w_pool, b_pool, w_dw0, w_dw1, s0, s1): the block's output; None where ConvBlockFunction
+// has to answer (a case that the library's block calls do not cover, a transform, a trace); True where no gradient is wanted and its inference call (block_infer) covers it.
 PyObject* py_block(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     TORCH_CHECK(n == 11, "block: 11 arguments expected");

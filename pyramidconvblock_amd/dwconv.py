@@ -270,7 +270,7 @@ class OptimizedDepthwiseConv2d(torch.nn.Module):
         assert x.dim() == 4 and x.shape[3] == self.channels, "input must be [B,H,W,C] with matching channels"
         # DepthwiseConv2DFunction in native code (csrc/torch_ops.cpp)
         y = _lib.ext().dwconv(x, self.weight, self.stride, self.padding, self.dilation)
-        if y is None:   # under forward-mode differentiation or a functorch transform
+        if y is None:   # under forward-mode differentiation, a functorch transform or a trace
             y = DepthwiseConv2DFunction.apply(x, self.weight, self.stride, self.padding, self.dilation, self.weight.dtype)
         return y
 

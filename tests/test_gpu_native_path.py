@@ -98,3 +98,30 @@ def test_transforms_without_a_rule_are_refused(which):
         layer(fwad.make_dual(x, torch.ones_like(x)))
     with pytest.raises(RuntimeError):
         torch.func.vmap(layer)(x[None])
+
+
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.parametrize("kind,dim,k,shape,dtype", [
+    ("block", 128, 13, (2, 24, 32, 128), torch.bfloat16),   # the fused launches, with an inference form
+    ("block", 64, 7, (2, 13, 18, 64), torch.float32),       # the general sequence
+    ("conv", 64, 5, (2, 9, 12, 64), torch.float16),
+])
+def test_a_trace_computes_again(kind, dim, k, shape, dtype, grad):
+    """A module recorded by torch.jit.trace, on another input than the one it was traced with: the module's own result,
+    and its gradients."""
+    import pyramidconvblock_amd
+
+    torch.manual_seed(3)
+    layer = (pyramidconvblock_amd.ConvBlock(dim=dim, kernel_size=k) if kind == "block"
+             else pyramidconvblock_amd.OptimizedDepthwiseConv2d(dim, k, padding=k // 2)).to(dtype).cuda()
+    gen = torch.Generator().manual_seed(4)
+    first, x, g = (randn(gen, *shape).to(dtype).cuda() for _ in range(3))
+    x.requires_grad_(grad)
+    with torch.set_grad_enabled(grad):
+        traced = torch.jit.trace(layer, (first.requires_grad_(grad),), check_trace=False)
+        want, got = layer(x), traced(x)
+    assert_close(got, want.detach().double().cpu().numpy(), dtype, "y")
+    if grad:
+        inputs = [x, *layer.parameters()]
+        for a, b in zip(torch.autograd.grad(got, inputs, g), torch.autograd.grad(want, inputs, g)):
+            assert_close(a, b.double().cpu().numpy(), dtype, "gradient")
