@@ -43,6 +43,10 @@ Tensor dense(const Tensor& t) {
     return reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 == 0 ? c : c.clone(at::MemoryFormat::Contiguous);
 }
 
+// What a node keeps of an input: the input itself where it went to the kernels as it is, so that a later change of it in
+// place is noticed, else the copy that they read.
+SavedVariable save(const Tensor& in, const Tensor& read) { return SavedVariable(read.is_same(in) ? in : read, false); }
+
 void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 
 Tensor bytes(size_t n, const Tensor& like) { return at::empty({(int64_t)n}, like.options().dtype(at::kByte)); }
@@ -149,10 +153,9 @@ Tensor block_train_or_infer(const Tensor* in, const BlockShape& s, bool grad) {
         node = std::shared_ptr<BlockNode>(new BlockNode(), torch::autograd::deleteNode);
         node->set_next_edges(torch::autograd::collect_next_edges(in[kX], in[kUp], in[kOut], in[kBOut], in[kPool],
                                                                  in[kBPool], in[kDw0], in[kDw1]));
-        // (the input itself where it went to the kernels as it is, so that a later change of it in place is noticed)
-        auto save = [&](int i) { return SavedVariable(d[i].is_same(in[i]) ? in[i] : d[i], false); };
-        node->x = save(kX), node->w_up = save(kUp), node->w_out = save(kOut), node->w_pool = save(kPool);
-        node->w_dw0 = save(kDw0), node->w_dw1 = save(kDw1), node->saved = SavedVariable(saved, false);
+        auto keep = [&](int i) { return save(in[i], d[i]); };
+        node->x = keep(kX), node->w_up = keep(kUp), node->w_out = keep(kOut), node->w_pool = keep(kPool);
+        node->w_dw0 = keep(kDw0), node->w_dw1 = keep(kDw1), node->saved = SavedVariable(saved, false);
         node->s = s, node->has_b_out = in[kBOut].defined(), node->has_b_pool = in[kBPool].defined();
         torch::autograd::set_history(y, node);
     }
@@ -228,11 +231,10 @@ Tensor conv_forward(const Tensor& x, const Tensor& w, const ConvGeo& g) {
                      w.scalar_type());
     const c10::DeviceGuard guard(x.device());
     const bool grad = at::GradMode::is_enabled() && (x.requires_grad() || w.requires_grad());
-    Tensor y, xc;
+    Tensor y, xd, wd;
     {
         at::AutoDispatchBelowADInplaceOrView below;
-        xc = x.scalar_type() == w.scalar_type() ? x : x.to(w.scalar_type());
-        const Tensor xd = dense(xc), wd = dense(w);
+        xd = dense(x.scalar_type() == w.scalar_type() ? x : x.to(w.scalar_type())), wd = dense(w);
         const auto xs = xd.sizes(), ws = wd.sizes();
         const int oh = pdw_conv_out_size((int)xs[1], (int)ws[0], g.sh, g.ph, g.dh);
         const int ow = pdw_conv_out_size((int)xs[2], (int)ws[1], g.sw, g.pw, g.dw);
@@ -244,7 +246,9 @@ Tensor conv_forward(const Tensor& x, const Tensor& w, const ConvGeo& g) {
     if (grad) {
         auto node = std::shared_ptr<ConvNode>(new ConvNode(), torch::autograd::deleteNode);
         node->set_next_edges(torch::autograd::collect_next_edges(x, w));
-        node->x = SavedVariable(xc, false), node->w = SavedVariable(w, false);
+        // (what the kernels read, as in block_train_or_infer: a copy is not made again by the backward, and stays valid
+        // when its source is changed in place)
+        node->x = save(x, xd), node->w = save(w, wd);
         node->g = g, node->x_type = x.scalar_type();
         torch::autograd::set_history(y, node);
     }

@@ -63,6 +63,35 @@ def test_changed_in_place_is_noticed():
             y.sum().backward()
 
 
+@pytest.mark.parametrize("which", ["block", "conv"])
+def test_a_copied_input_is_kept_as_copied(which):
+    """An input that the kernels read from a dense copy: the backward uses that copy, whatever becomes of the input."""
+    import pyramidconvblock_amd
+
+    torch.manual_seed(5)
+    layer = (pyramidconvblock_amd.ConvBlock(dim=64, kernel_size=5) if which == "block"
+             else pyramidconvblock_amd.OptimizedDepthwiseConv2d(64, 5, padding=2)).float().cuda()
+    flat = torch.randn(2 * 8 * 9 * 64 + 1, device="cuda")
+    for x in (flat[:-1].view(2, 9, 8, 64).transpose(1, 2), flat[1:].view(2, 8, 9, 64)):   # strides, alignment
+        leaves = [x.requires_grad_(), *layer.parameters()]
+        y = layer(x)
+        g = torch.randn_like(y)
+        want = torch.autograd.grad(y, leaves, g, retain_graph=True)
+        before = torch.cuda.memory_stats()["allocated_bytes.all.allocated"]
+        got = torch.autograd.grad(y, leaves, g, retain_graph=True)
+        again = torch.cuda.memory_stats()["allocated_bytes.all.allocated"] - before
+        dense = x.detach().contiguous().clone().requires_grad_()
+        yd = layer(dense)
+        torch.autograd.grad(yd, [dense, *leaves[1:]], g, retain_graph=True)
+        before = torch.cuda.memory_stats()["allocated_bytes.all.allocated"]
+        torch.autograd.grad(yd, [dense, *leaves[1:]], g)
+        assert again == torch.cuda.memory_stats()["allocated_bytes.all.allocated"] - before   # no second copy
+        with torch.no_grad():
+            flat.mul_(3)
+        for a, b, c in zip(want, got, torch.autograd.grad(y, leaves, g)):
+            assert torch.equal(a, b) and torch.equal(a, c)
+
+
 def _layers():
     import pyramid_dwconv
     import pyramidconvblock_amd
