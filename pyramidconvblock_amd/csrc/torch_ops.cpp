@@ -47,6 +47,12 @@ Tensor dense(const Tensor& t) {
 // place is noticed, else the copy that they read.
 SavedVariable save(const Tensor& in, const Tensor& read) { return SavedVariable(read.is_same(in) ? in : read, false); }
 
+// The gradient of a node's only output; zeros where the engine has none (a later node's backward returned none), as
+// torch.autograd.Function gives them, so that inputs and parameters get gradients of zero and not none.
+Tensor output_gradient(const torch::autograd::Node& node, const variable_list& grads) {
+    return grads[0].defined() ? grads[0] : node.input_metadata(0).zeros_like();
+}
+
 void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 
 Tensor bytes(size_t n, const Tensor& like) { return at::empty({(int64_t)n}, like.options().dtype(at::kByte)); }
@@ -88,14 +94,14 @@ struct BlockNode : public torch::autograd::Node {
     variable_list apply(variable_list&& grads) override {
         std::lock_guard<std::mutex> lock(mutex_);
         variable_list out(kBlockInputs);
-        if (!grads[0].defined()) return out;
+        const Tensor grad = output_gradient(*this, grads);
         // (unpacked first: a saved-tensor hook may run a whole recorded forward, as checkpointing does)
         auto take = [&](const SavedVariable& v) { return v.unpack(shared_from_this()); };
         Tensor xs = take(x), wu = take(w_up), wo = take(w_out), wp = take(w_pool), d0 = take(w_dw0), d1 = take(w_dw1);
         const Tensor keep = take(saved);
         at::AutoDispatchBelowADInplaceOrView below;
         for (Tensor* t : {&xs, &wu, &wo, &wp, &d0, &d1}) *t = dense(*t);
-        const Tensor gy = dense(grads[0].to(xs.scalar_type()));
+        const Tensor gy = dense(grad.to(xs.scalar_type()));
         const c10::DeviceGuard guard(xs.device());
         auto like = [](const Tensor& t) { return at::empty(t.sizes(), t.options()); };
         if (task_should_compute_output(kX)) out[kX] = like(xs);
@@ -188,11 +194,11 @@ struct ConvNode : public torch::autograd::Node {
     variable_list apply(variable_list&& grads) override {
         std::lock_guard<std::mutex> lock(mutex_);
         variable_list out(2);
-        if (!grads[0].defined()) return out;
+        const Tensor grad = output_gradient(*this, grads);
         const Tensor w_saved = w.unpack(shared_from_this()), x_saved = x.unpack(shared_from_this());   // (first, as in BlockNode)
         at::AutoDispatchBelowADInplaceOrView below;
         const Tensor wd = dense(w_saved), xd = dense(x_saved.to(wd.scalar_type()));
-        const Tensor gy = dense(grads[0].to(wd.scalar_type()));
+        const Tensor gy = dense(grad.to(wd.scalar_type()));
         const c10::DeviceGuard guard(xd.device());
         const int dt = dtype_code(wd.scalar_type());
         void* const stream = stream_of(xd);

@@ -92,6 +92,29 @@ def test_a_copied_input_is_kept_as_copied(which):
             assert torch.equal(a, b) and torch.equal(a, c)
 
 
+class _NoGradient(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x):
+        return x.clone()
+
+    @staticmethod
+    def backward(ctx, g):
+        return None
+
+
+@pytest.mark.parametrize("kind,dim,shape,dtype", [("block", 128, (1, 8, 32, 128), torch.bfloat16), ("block", 64, (2, 7, 9, 64), torch.float32),
+                                                  ("conv", 64, (2, 7, 9, 64), torch.float16)])
+def test_no_gradient_from_behind_is_a_gradient_of_zero(kind, dim, shape, dtype):
+    import pyramidconvblock_amd
+
+    layer = (pyramidconvblock_amd.ConvBlock(dim=dim, kernel_size=5) if kind == "block"
+             else pyramidconvblock_amd.OptimizedDepthwiseConv2d(dim, 5, padding=2)).to(dtype).cuda()
+    x = torch.randn(shape, device="cuda").to(dtype).requires_grad_()
+    _NoGradient.apply(layer(x)).sum().backward()
+    for t in (x, *layer.parameters()):
+        assert t.grad is not None and not t.grad.any()
+
+
 def _layers():
     import pyramid_dwconv
     import pyramidconvblock_amd
