@@ -301,7 +301,8 @@ PyObject* py_block(PyObject*, PyObject* const* args, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// block_infer(x, w_up, w_out, b_out, w_pool, b_pool, w_dw0, w_dw1): pdw_convblock_infer (the caller has asked block()).
+// block_infer(x, w_up, w_out, b_out, w_pool, b_pool, w_dw0, w_dw1): pdw_convblock_infer, refused where block() would not
+// name it.
 PyObject* py_block_infer(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     TORCH_CHECK(n == kBlockInputs, "block_infer: 8 arguments expected");
@@ -309,6 +310,15 @@ PyObject* py_block_infer(PyObject*, PyObject* const* args, Py_ssize_t n) {
     for (int i = 0; i < kBlockInputs; ++i) {
         if (!tensor_arg(args[i], &in[i])) return nullptr;
     }
+    // (the kernels take addresses: a tensor of another device, type or size must not get that far)
+    for (int i = 0; i < kBlockInputs; ++i)
+        TORCH_CHECK(in[i].defined() ? in[i].is_cuda() : i == kBOut || i == kBPool,
+                    "convblock_infer: tensors on a HIP device expected (the biases may be None)");
+    BlockShape s;
+    TORCH_CHECK(plain_call(in, kBlockInputs) && block_shape(in, Tensor(), 1.0, 0.5, &s) && s.H == 2 * s.h && s.W == 2 * s.w &&
+                    pdw_convblock_supported(s.B, s.H, s.W, s.D, s.I, s.K, s.dtype),
+                "convblock_infer: not a call that pdw_convblock_infer covers (input ", in[kX].sizes(), " ",
+                in[kX].scalar_type(), ", filters ", in[kDw0].sizes(), ")");
     Tensor y;
     {
         pybind11::gil_scoped_release no_gil;
@@ -317,12 +327,10 @@ PyObject* py_block_infer(PyObject*, PyObject* const* args, Py_ssize_t n) {
         for (Tensor& t : in)
             if (t.defined()) t = dense(t);
         const Tensor& x = in[kX];
-        const int B = x.size(0), H = x.size(1), W = x.size(2), D = x.size(3), I = in[kUp].size(0), K = in[kDw0].size(0);
-        const int dt = dtype_code(x.scalar_type());
         y = at::empty(x.sizes(), x.options());
-        const Tensor ws = bytes(pdw_convblock_infer_workspace_bytes(B, H, W, D, I, K, dt), x);
+        const Tensor ws = bytes(pdw_convblock_infer_workspace_bytes(s.B, s.H, s.W, s.D, s.I, s.K, s.dtype), x);
         check(pdw_convblock_infer(ptr(x), ptr(in[kUp]), ptr(in[kDw0]), ptr(in[kDw1]), ptr(in[kPool]), ptr(in[kBPool]),
-                                  ptr(in[kOut]), ptr(in[kBOut]), ptr(y), ptr(ws), ws.numel(), B, H, W, D, I, K, dt, stream_of(x)),
+                                  ptr(in[kOut]), ptr(in[kBOut]), ptr(y), ptr(ws), ws.numel(), s.B, s.H, s.W, s.D, s.I, s.K, s.dtype, stream_of(x)),
               "pdw_convblock_infer");
     }
     return THPVariable_Wrap(std::move(y));

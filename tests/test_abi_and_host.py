@@ -125,3 +125,10 @@ def test_no_cpu_path():
         conv(torch.zeros(1, 4, 4, 9))
     with pytest.raises(RuntimeError, match="HIP device"):
         P.ConvBlock(8, kernel_size=3)(torch.zeros(1, 4, 4, 8))
+    from pyramidconvblock_amd.conv_block import convblock_infer
+
+    m = P.ConvBlock(128, kernel_size=3).bfloat16()
+    args = [m.conv_up.weight, m.conv_out.weight, m.conv_out.bias, m.conv_pool.weight, m.conv_pool.bias]
+    for x, a in ((torch.zeros(1, 4, 8, 128).bfloat16(), args), (None, args), (torch.zeros(1, 4, 8, 128).bfloat16(), [None] * 5)):
+        with pytest.raises(RuntimeError, match="HIP device"):
+            convblock_infer(x, *a, [g.conv_spatial.weight for g in m.gates])

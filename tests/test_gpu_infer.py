@@ -186,3 +186,20 @@ def test_block_inference_other_shapes_use_the_stepwise_path(oracle, dim, kw):
         conv_block.convblock_infer = orig
     assert not calls, "the single-call inference entry point was taken for a configuration it does not cover"
     assert_close(y, yo, torch.float16, "y")
+
+
+def test_block_inference_refuses_what_does_not_fit():
+    """convblock_infer passes addresses on: tensors that do not belong together are refused before any launch."""
+    import pyramid_dwconv
+    from pyramidconvblock_amd.conv_block import convblock_infer
+
+    m = pyramid_dwconv.ConvBlock(dim=128, kernel_size=5).bfloat16().cuda()
+    x = torch.randn(1, 8, 32, 128, device="cuda").bfloat16()
+    good = [x, m.conv_up.weight, m.conv_out.weight, m.conv_out.bias, m.conv_pool.weight, m.conv_pool.bias,
+            [g.conv_spatial.weight for g in m.gates]]
+    with torch.no_grad():
+        assert torch.equal(convblock_infer(*good), m(x))
+    for i, bad in ((0, x[:, :7]), (0, x.float()), (0, x[..., :64]), (0, x[0]), (1, m.conv_up.weight[:32]), (3, m.conv_out.bias[:64]),
+                   (4, m.conv_pool.weight.cpu()), (6, [good[6][0], good[6][1][:3, :3]])):
+        with pytest.raises(RuntimeError, match="convblock_infer"):
+            convblock_infer(*good[:i], bad, *good[i + 1:])
