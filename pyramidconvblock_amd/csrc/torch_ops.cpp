@@ -47,6 +47,16 @@ Tensor dense(const Tensor& t) {
 // place is noticed, else the copy that they read.
 SavedVariable save(const Tensor& in, const Tensor& read) { return SavedVariable(read.is_same(in) ? in : read, false); }
 
+// What a node has saved, as it comes back: a saved-tensor hook may have put another tensor in its place, and the kernels
+// take addresses.  (Of another type: converted.)
+Tensor restored(const SavedVariable& v, const std::shared_ptr<torch::autograd::Node>& node, at::IntArrayRef sizes,
+                at::ScalarType type, c10::Device device) {
+    Tensor t = v.unpack(node);
+    TORCH_CHECK(t.defined() && t.sizes() == sizes && t.device() == device, node->name(),
+                ": a saved tensor came back as another one (", sizes, " on ", device, " was saved)");
+    return t.scalar_type() == type ? t : t.to(type);
+}
+
 // The gradient of a node's only output; zeros where the engine has none (a later node's backward returned none), as
 // torch.autograd.Function gives them, so that inputs and parameters get gradients of zero and not none.
 Tensor output_gradient(const torch::autograd::Node& node, const variable_list& grads) {
@@ -82,6 +92,7 @@ enum { kX, kUp, kOut, kBOut, kPool, kBPool, kDw0, kDw1, kBlockInputs };   // ord
 struct BlockNode : public torch::autograd::Node {
     SavedVariable x, w_up, w_out, w_pool, w_dw0, w_dw1, saved;
     BlockShape s;
+    int64_t saved_bytes;
     bool has_b_out, has_b_pool;
 
     std::string name() const override { return "ConvBlockBackward"; }
@@ -96,12 +107,15 @@ struct BlockNode : public torch::autograd::Node {
         variable_list out(kBlockInputs);
         const Tensor grad = output_gradient(*this, grads);
         // (unpacked first: a saved-tensor hook may run a whole recorded forward, as checkpointing does)
-        auto take = [&](const SavedVariable& v) { return v.unpack(shared_from_this()); };
-        Tensor xs = take(x), wu = take(w_up), wo = take(w_out), wp = take(w_pool), d0 = take(w_dw0), d1 = take(w_dw1);
-        const Tensor keep = take(saved);
+        const auto self = shared_from_this();
+        const auto type = grad.scalar_type();   // (the engine has cast it to the output's type and checked its sizes)
+        auto take = [&](const SavedVariable& v, std::initializer_list<int64_t> n) { return restored(v, self, n, type, grad.device()); };
+        Tensor xs = take(x, {s.B, s.H, s.W, s.D}), wu = take(w_up, {s.I, s.D}), wo = take(w_out, {s.D, s.I}),
+               wp = take(w_pool, {s.D, s.D}), d0 = take(w_dw0, {s.K, s.K, s.I}), d1 = take(w_dw1, {s.K, s.K, s.I});
+        Tensor keep = restored(saved, self, {saved_bytes}, at::kByte, grad.device());
         at::AutoDispatchBelowADInplaceOrView below;
-        for (Tensor* t : {&xs, &wu, &wo, &wp, &d0, &d1}) *t = dense(*t);
-        const Tensor gy = dense(grad.to(xs.scalar_type()));
+        for (Tensor* t : {&xs, &wu, &wo, &wp, &d0, &d1, &keep}) *t = dense(*t);
+        const Tensor gy = dense(grad);
         const c10::DeviceGuard guard(xs.device());
         auto like = [](const Tensor& t) { return at::empty(t.sizes(), t.options()); };
         if (task_should_compute_output(kX)) out[kX] = like(xs);
@@ -162,7 +176,7 @@ Tensor block_train_or_infer(const Tensor* in, const BlockShape& s, bool grad) {
         auto keep = [&](int i) { return save(in[i], d[i]); };
         node->x = keep(kX), node->w_up = keep(kUp), node->w_out = keep(kOut), node->w_pool = keep(kPool);
         node->w_dw0 = keep(kDw0), node->w_dw1 = keep(kDw1), node->saved = SavedVariable(saved, false);
-        node->s = s, node->has_b_out = in[kBOut].defined(), node->has_b_pool = in[kBPool].defined();
+        node->s = s, node->saved_bytes = saved.numel(), node->has_b_out = in[kBOut].defined(), node->has_b_pool = in[kBPool].defined();
         torch::autograd::set_history(y, node);
     }
     return y;
@@ -181,6 +195,7 @@ struct ConvGeo {
 
 struct ConvNode : public torch::autograd::Node {
     SavedVariable x, w;
+    at::DimVector x_sizes, w_sizes;
     ConvGeo g;
     at::ScalarType x_type;
 
@@ -195,10 +210,11 @@ struct ConvNode : public torch::autograd::Node {
         std::lock_guard<std::mutex> lock(mutex_);
         variable_list out(2);
         const Tensor grad = output_gradient(*this, grads);
-        const Tensor w_saved = w.unpack(shared_from_this()), x_saved = x.unpack(shared_from_this());   // (first, as in BlockNode)
+        const auto self = shared_from_this();   // (unpacked first, as in BlockNode)
+        const Tensor w_saved = restored(w, self, w_sizes, grad.scalar_type(), grad.device()),
+                     x_saved = restored(x, self, x_sizes, grad.scalar_type(), grad.device());
         at::AutoDispatchBelowADInplaceOrView below;
-        const Tensor wd = dense(w_saved), xd = dense(x_saved.to(wd.scalar_type()));
-        const Tensor gy = dense(grad.to(wd.scalar_type()));
+        const Tensor wd = dense(w_saved), xd = dense(x_saved), gy = dense(grad);
         const c10::DeviceGuard guard(xd.device());
         const int dt = dtype_code(wd.scalar_type());
         void* const stream = stream_of(xd);
@@ -255,6 +271,7 @@ Tensor conv_forward(const Tensor& x, const Tensor& w, const ConvGeo& g) {
         // (what the kernels read, as in block_train_or_infer: a copy is not made again by the backward, and stays valid
         // when its source is changed in place)
         node->x = save(x, xd), node->w = save(w, wd);
+        node->x_sizes = x.sizes(), node->w_sizes = w.sizes();
         node->g = g, node->x_type = x.scalar_type();
         torch::autograd::set_history(y, node);
     }

@@ -115,6 +115,31 @@ def test_no_gradient_from_behind_is_a_gradient_of_zero(kind, dim, shape, dtype):
         assert t.grad is not None and not t.grad.any()
 
 
+@pytest.mark.parametrize("which", ["block", "conv"])
+def test_a_hook_that_returns_another_tensor_is_refused(which):
+    """The backward's kernels take addresses of what was saved: a saved-tensor hook that gives back something else (left on
+    the host, cut short) ends in an error and not in a read out of bounds; one of another type is converted."""
+    import pyramidconvblock_amd
+
+    layer = (pyramidconvblock_amd.ConvBlock(dim=64, kernel_size=5) if which == "block"
+             else pyramidconvblock_amd.OptimizedDepthwiseConv2d(64, 5, padding=2)).float().cuda()
+    x = torch.randn(2, 7, 9, 64, device="cuda", requires_grad=True)
+    for unpack in (lambda t: t.cpu(), lambda t: t[:-1], lambda t: t.flatten()[::2]):
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            y = layer(x)
+        with pytest.raises(RuntimeError, match="came back as another one"):
+            y.sum().backward()
+    inputs = [x, *layer.parameters()]
+    want = torch.autograd.grad(layer(x).sum(), inputs)
+    with torch.autograd.graph.save_on_cpu():   # the hook in use: another tensor of the same kind
+        y = layer(x)
+    assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(y.sum(), inputs), want))
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.half(), lambda t: t):   # x and the weights in 16 bits
+        y = layer(x)
+    for a, b in zip(torch.autograd.grad(y.sum(), inputs), want):
+        assert_close(a, b.double().cpu().numpy(), torch.float16, "gradient")
+
+
 def _layers():
     import pyramid_dwconv
     import pyramidconvblock_amd
