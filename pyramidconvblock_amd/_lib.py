@@ -7,6 +7,7 @@ tensor is not on a HIP device, the operators raise.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import threading
 import os
 from ctypes import c_char_p, c_int, c_longlong, c_size_t, c_void_p
@@ -125,17 +126,20 @@ _ext = None
 
 
 def ext():
-    """The native host path of the operators (csrc/torch_ops.cpp), built beside libpdw.so."""
+    """The native host path of the operators (csrc/torch_ops.cpp), built beside libpdw.so for this torch (if it has
+    not been yet)."""
     global _ext
     if _ext is None:
         lib()
-        if not os.path.exists(os.path.join(_HERE, "_pdw_torch.so")):
-            from . import build as _build
+        from . import build as _build
 
-            _build.build()
-        from . import _pdw_torch
-
-        _ext = _pdw_torch
+        path = _build.ext_path(torch.__version__)
+        if not os.path.exists(path):
+            _build.build_ext()
+        spec = importlib.util.spec_from_file_location(__package__ + "._pdw_torch", path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _ext = module
     return _ext
 
 

@@ -3,6 +3,8 @@ and the host-side mirror keeps the reference's module structure, names and init.
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -132,3 +134,40 @@ def test_no_cpu_path():
     for x, a in ((torch.zeros(1, 4, 8, 128).bfloat16(), args), (None, args), (torch.zeros(1, 4, 8, 128).bfloat16(), [None] * 5)):
         with pytest.raises(RuntimeError, match="HIP device"):
             convblock_infer(x, *a, [g.conv_spatial.weight for g in m.gates])
+
+
+def test_the_library_builds_without_torch(tmp_path):
+    """build.py as a script in an interpreter without torch (the compiler stands in by a script that writes its output):
+    libpdw.so is linked, the host extension is left out, and nothing raises."""
+    hipcc = tmp_path / "hipcc"
+    hipcc.write_text('#!/bin/sh\nwhile [ "$1" != -o ]; do shift; done\necho built > "$2"\n')
+    hipcc.chmod(0o755)
+    code = ("import sys, importlib.util as u; sys.modules['torch'] = None\n"
+            f"spec = u.spec_from_file_location('b', {os.path.join(ROOT, 'pyramidconvblock_amd', 'build.py')!r})\n"
+            "b = u.module_from_spec(spec); spec.loader.exec_module(b)\n"
+            f"b.HERE = {str(tmp_path)!r}; b.OBJ = b.HERE + '/obj'; b.LIB = b.HERE + '/libpdw.so'; b._headers = lambda: []\n"
+            "b.build()")
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, env={**os.environ, "HIPCC": str(hipcc)})
+    assert r.returncode == 0, r.stderr
+    assert (tmp_path / "libpdw.so").read_text() == "built\n" and not list(tmp_path.glob("_pdw_torch*"))
+
+
+def test_the_host_extension_is_bound_to_its_torch(monkeypatch):
+    """Another torch than the one the extension was compiled against: that file is not loaded, one is built."""
+    from pyramidconvblock_amd import _lib, build
+
+    assert os.path.exists(build.ext_path(torch.__version__)) and _lib.ext()
+    asked = []
+
+    def build_ext():
+        asked.append(torch.__version__)
+        raise RuntimeError("no compiler")
+
+    monkeypatch.setattr(_lib, "_ext", None)
+    monkeypatch.setattr(build, "build_ext", build_ext)
+    monkeypatch.setattr(torch, "__version__", "99.1.0+rocm9")
+    with pytest.raises(RuntimeError, match="no compiler"):
+        _lib.ext()
+    assert asked == ["99.1.0+rocm9"]
+    names = {build.ext_path(v) for v in ("2.10.0+rocm7.0", "2.10.0", "2.11.0+rocm7.0")}
+    assert len(names) == 3 and all(os.path.dirname(n) == build.HERE for n in names)
