@@ -445,7 +445,8 @@ int pdw_convblock_bwd(const void *gy, const void *x, const void *a, const void *
  * are not multiples of 16), as one host call each way; the fused launches of pdw_convblock_* where those cover the
  * shape.  Covered when pdw_block_supported.  `saved` is one device buffer of pdw_block_saved_bytes that the forward
  * fills and the backward reads (its layout is the library's own: everything between the two calls is in it); a forward
- * that no backward follows uses it as its workspace.  x, y, gy, dx[B,H,W,D]; weights and their gradients as for
+ * that no backward follows uses it as its workspace.  y is scratch of the forward until its last launch writes it, so it must
+ * not overlap x.  x, y, gy, dx[B,H,W,D]; weights and their gradients as for
  * pdw_convblock_*; dx may be NULL (not wanted), gb_pool and gb_out too.  Status 3: case not covered, nothing launched.
  * Replaces ConvBlock.forward, conv_block.py:36-49, and its autograd backward. */
 int pdw_block_supported(int B, int H, int W, int h, int w, int D, int I, int K, int dtype);

@@ -46,40 +46,13 @@ Shape shape_of(int B, int H, int W, int D, int I, int K, int dtype) {
 
 }  // namespace
 
-extern "C" {
+namespace pdw {
 
-int pdw_convblock_supported(int B, int H, int W, int D, int I, int K, int dtype) {
-    if (dtype != kF16 && dtype != kBF16) return 0;
-    if (B < 1 || H < 4 || W < 4 || (H & 1) || (W & 1) || K < 1 || !(K & 1) || D < 8 || I < 16 || (I & 15)) return 0;
-    if ((long long)B * H * W * (D > I ? D : I) > 0x7fffffffLL) return 0;
-    if ((H * W) % pdw_dense_colsum_rows()) return 0;
-    return pdw_dense_supported(D, I, dtype) && pdw_dense_supported(I, D, dtype) && pdw_dense_colsum_supported(D, I, dtype) &&
-           pdw_dense_bwd_pair_colsum_supported(D, I, dtype) && pdw_dense_bwd_pair_supported(I, D, dtype);
-}
-
-size_t pdw_convblock_fwd_workspace_bytes(int B, int H, int W, int D, int I, int K, int dtype) {
-    if (!pdw_convblock_supported(B, H, W, D, I, K, dtype)) return 0;
+int convblock_fwd_launch(const void* x, const void* w_up, const void* w_dw0, const void* w_dw1, const void* w_pool,
+                         const void* b_pool, const void* w_out, const void* b_out, void* a, void* c0, void* xp, void* c1,
+                         void* cat, void* m, void* y, float* xparts, float* yp, int B, int H, int W, int D, int I, int K,
+                         int dtype, void* stream) {
     const Shape s = shape_of(B, H, W, D, I, K, dtype);
-    return up256((size_t)s.nt * D * 4) + up256((size_t)B * D * 4);
-}
-
-int pdw_convblock_fwd(const void* x, const void* w_up, const void* w_dw0, const void* w_dw1, const void* w_pool,
-                      const void* b_pool, const void* w_out, const void* b_out, void* a, void* c0, void* xp, void* c1,
-                      void* cat, void* m, void* y, void* workspace, size_t workspace_bytes, int B, int H, int W, int D,
-                      int I, int K, int dtype, void* stream) {
-    if (!pdw_convblock_supported(B, H, W, D, I, K, dtype))
-        return set_error("pdw_convblock_fwd: shape not covered (B=%d H=%d W=%d D=%d I=%d K=%d dtype=%d)", B, H, W, D, I, K,
-                         dtype), 1;
-    for (const void* ptr : {x, w_up, w_dw0, w_dw1, w_pool, w_out, (const void*)a, (const void*)c0, (const void*)xp,
-                            (const void*)c1, (const void*)cat, (const void*)m, (const void*)y, (const void*)workspace})
-        if (!ptr) return set_error("pdw_convblock_fwd: null pointer"), 1;
-    const Shape s = shape_of(B, H, W, D, I, K, dtype);
-    if (workspace_bytes < pdw_convblock_fwd_workspace_bytes(B, H, W, D, I, K, dtype))
-        return set_error("pdw_convblock_fwd: workspace of %zu bytes given, %zu needed", workspace_bytes,
-                         pdw_convblock_fwd_workspace_bytes(B, H, W, D, I, K, dtype)), 1;
-    Carver ws{(char*)workspace, workspace_bytes};
-    float* xparts = (float*)ws.take((size_t)s.nt * D * 4);  // sums of x over each row tile
-    float* yp = (float*)ws.take((size_t)B * D * 4);         // mean branch: one row per image
     const int pad = K / 2;
     // conv_up, with the tile sums of x for the mean branch                                   (conv_block.py:37, 46)
     // (where the layer's kernel can also pool its result for the second scale, the convolutions need no pooling launch)
@@ -126,6 +99,46 @@ int pdw_convblock_fwd(const void* x, const void* w_up, const void* w_dw0, const 
         return e;
     // conv_out plus the per-image row                                                        (conv_block.py:44, 49)
     return pdw_dense_fwd(cat, w_out, 0, nullptr, yp, y, s.N, I, D, s.P, dtype, stream);
+}
+
+}  // namespace pdw
+
+extern "C" {
+
+int pdw_convblock_supported(int B, int H, int W, int D, int I, int K, int dtype) {
+    if (dtype != kF16 && dtype != kBF16) return 0;
+    if (B < 1 || H < 4 || W < 4 || (H & 1) || (W & 1) || K < 1 || !(K & 1) || D < 8 || I < 16 || (I & 15)) return 0;
+    if ((long long)B * H * W * (D > I ? D : I) > 0x7fffffffLL) return 0;
+    if ((H * W) % pdw_dense_colsum_rows()) return 0;
+    return pdw_dense_supported(D, I, dtype) && pdw_dense_supported(I, D, dtype) && pdw_dense_colsum_supported(D, I, dtype) &&
+           pdw_dense_bwd_pair_colsum_supported(D, I, dtype) && pdw_dense_bwd_pair_supported(I, D, dtype);
+}
+
+size_t pdw_convblock_fwd_workspace_bytes(int B, int H, int W, int D, int I, int K, int dtype) {
+    if (!pdw_convblock_supported(B, H, W, D, I, K, dtype)) return 0;
+    const Shape s = shape_of(B, H, W, D, I, K, dtype);
+    return up256((size_t)s.nt * D * 4) + up256((size_t)B * D * 4);
+}
+
+int pdw_convblock_fwd(const void* x, const void* w_up, const void* w_dw0, const void* w_dw1, const void* w_pool,
+                      const void* b_pool, const void* w_out, const void* b_out, void* a, void* c0, void* xp, void* c1,
+                      void* cat, void* m, void* y, void* workspace, size_t workspace_bytes, int B, int H, int W, int D,
+                      int I, int K, int dtype, void* stream) {
+    if (!pdw_convblock_supported(B, H, W, D, I, K, dtype))
+        return set_error("pdw_convblock_fwd: shape not covered (B=%d H=%d W=%d D=%d I=%d K=%d dtype=%d)", B, H, W, D, I, K,
+                         dtype), 1;
+    for (const void* ptr : {x, w_up, w_dw0, w_dw1, w_pool, w_out, (const void*)a, (const void*)c0, (const void*)xp,
+                            (const void*)c1, (const void*)cat, (const void*)m, (const void*)y, (const void*)workspace})
+        if (!ptr) return set_error("pdw_convblock_fwd: null pointer"), 1;
+    const Shape s = shape_of(B, H, W, D, I, K, dtype);
+    if (workspace_bytes < pdw_convblock_fwd_workspace_bytes(B, H, W, D, I, K, dtype))
+        return set_error("pdw_convblock_fwd: workspace of %zu bytes given, %zu needed", workspace_bytes,
+                         pdw_convblock_fwd_workspace_bytes(B, H, W, D, I, K, dtype)), 1;
+    Carver ws{(char*)workspace, workspace_bytes};
+    float* xparts = (float*)ws.take((size_t)s.nt * D * 4);  // sums of x over each row tile
+    float* yp = (float*)ws.take((size_t)B * D * 4);         // mean branch: one row per image
+    return convblock_fwd_launch(x, w_up, w_dw0, w_dw1, w_pool, b_pool, w_out, b_out, a, c0, xp, c1, cat, m, y, xparts, yp, B, H,
+                                W, D, I, K, dtype, stream);
 }
 
 // The convolution with the gate in its store, for the widths conv_out's made-rows kernel does not cover: images small

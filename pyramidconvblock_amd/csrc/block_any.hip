@@ -109,11 +109,12 @@ struct Weights {
     const void *up, *out, *dw0, *dw1;
 };
 
-// What the forward leaves for the backward, then what only the forward needs.
+// What the forward leaves for the backward, and what only the forward needs.
 struct Saved {
     void *a, *c0, *cat, *xp, *c1, *m;
     void *up_p, *out_p, *dw0_p, *dw1_p;   // packed weights (padded widths)
-    float *xparts, *yp;
+    float* yp;   // (forward only, like xparts and ws, but read by the launch that writes y; a row per image)
+    float* xparts;
     void* ws;
     size_t bytes;
 };
@@ -125,7 +126,9 @@ size_t mean_workspace(const Shape& s) {
     return own > old ? own : old;
 }
 
-Saved saved_layout(const Shape& s, void* base) {
+// The sums of x live until conv_out, the last launch, writes y: they lie in y itself, so that the buffer kept for the
+// backward holds no scratch (a sixteenth of a 16-bit x).  In that buffer only where y is too small, images of a few pixels.
+Saved saved_layout(const Shape& s, void* base, void* y) {
     Carver c{(char*)base};
     Saved r{};
     const size_t full = (size_t)s.N * s.I * s.es, half = (size_t)s.n * s.I * s.es;
@@ -136,15 +139,17 @@ Saved saved_layout(const Shape& s, void* base) {
         const size_t layer = (size_t)s.I * s.D * s.es, filter = (size_t)s.K * s.K * s.I * s.es;
         r.up_p = c.take(layer), r.out_p = c.take(layer), r.dw0_p = c.take(filter), r.dw1_p = c.take(filter);
     }
-    r.xparts = (float*)c.take((size_t)((s.N + 31) / 32) * s.D * 4);
-    r.yp = (float*)c.take((size_t)s.B * s.D * 4);   // (behind xparts: the workspace of pdw_convblock_fwd)
-    r.ws = c.take(mean_workspace(s));
+    r.yp = (float*)c.take((size_t)s.B * s.D * 4);
+    const size_t sums = up256((size_t)((s.N + 31) / 32) * s.D * 4), ws = up256(mean_workspace(s));
+    char* scratch = (char*)up256((uintptr_t)y);
+    if (sums + ws + 255 > (size_t)s.N * s.D * s.es) scratch = (char*)c.take(sums + ws);
+    r.xparts = (float*)scratch, r.ws = scratch + sums;
     r.bytes = c.used;
     return r;
 }
 
 struct BwdWork {
-    void *dcat, *gcf, *gch, *dxp, *da, *gbias;
+    void *dcat, *gcf, *gch, *dxp, *da, *gbias;   // (da lies where dcat was: the gates read that before the convolutions write this)
     float *gparts, *dmean;
     void *ws_po, *ws_pool, *ws_w0, *ws_w1, *ws_pu;
     size_t b_po, b_w0, b_w1, b_pu, bytes;
@@ -155,7 +160,7 @@ BwdWork bwd_layout(const Shape& s, void* base) {
     BwdWork r{};
     const size_t full = (size_t)s.N * s.I * s.es, half = (size_t)s.n * s.I * s.es;
     const int pad = s.K / 2;
-    r.dcat = c.take(full), r.gcf = c.take(full), r.da = c.take(full);
+    r.dcat = r.da = c.take(full), r.gcf = c.take(full);
     r.gch = c.take(half), r.dxp = c.take(half);
     r.gbias = c.take((size_t)2 * s.D * s.es);
     r.gparts = (float*)c.take((size_t)((s.N + 31) / 32) * s.D * 4);
@@ -372,7 +377,7 @@ int pdw_block_supported(int B, int H, int W, int h, int w, int D, int I, int K, 
 
 size_t pdw_block_saved_bytes(int B, int H, int W, int h, int w, int D, int I, int K, int dtype) {
     if (!pdw_block_supported(B, H, W, h, w, D, I, K, dtype)) return 0;
-    return saved_layout(shape_of(B, H, W, h, w, D, I, K, dtype), nullptr).bytes;
+    return saved_layout(shape_of(B, H, W, h, w, D, I, K, dtype), nullptr, nullptr).bytes;
 }
 
 int pdw_block_fwd(const void* x, const void* w_up, const void* w_dw0, const void* w_dw1, const void* w_pool,
@@ -384,12 +389,15 @@ int pdw_block_fwd(const void* x, const void* w_up, const void* w_dw0, const void
     for (const void* p : {x, w_up, w_dw0, w_dw1, w_pool, w_out, (const void*)y, (const void*)saved})
         if (!p) return set_error("pdw_block_fwd: null pointer"), 1;
     const Shape s = shape_of(B, H, W, h, w, D, I, K, dtype);
-    const Saved v = saved_layout(s, saved);
+    const Saved v = saved_layout(s, saved, y);
     if (saved_bytes < v.bytes)
         return set_error("pdw_block_fwd: buffer of %zu bytes given, %zu needed", saved_bytes, v.bytes), 1;
+    const size_t nx = (size_t)s.N * D * s.es;
+    if ((uintptr_t)x < (uintptr_t)y + nx && (uintptr_t)y < (uintptr_t)x + nx)
+        return set_error("pdw_block_fwd: y overlaps x (it holds sums of x until it is written)"), 1;
     if (s.single)
-        return pdw_convblock_fwd(x, w_up, w_dw0, w_dw1, w_pool, b_pool, w_out, b_out, v.a, v.c0, v.xp, v.c1, v.cat, v.m, y,
-                                 v.xparts, (size_t)((char*)v.ws - (char*)v.xparts), B, H, W, D, I, K, dtype, stream);
+        return convblock_fwd_launch(x, w_up, w_dw0, w_dw1, w_pool, b_pool, w_out, b_out, v.a, v.c0, v.xp, v.c1, v.cat, v.m, y,
+                                    v.xparts, v.yp, B, H, W, D, I, K, dtype, stream);
     Weights wt{w_up, w_out, w_dw0, w_dw1};
     if (s.padded())
         if (int e = pack_weights(s, v, &wt, (hipStream_t)stream)) return e;
@@ -413,7 +421,7 @@ int pdw_block_bwd(const void* gy, const void* x, const void* saved, const void* 
                           (const void*)gw_dw1, (const void*)gw_pool, (const void*)gw_out, (const void*)workspace})
         if (!p) return set_error("pdw_block_bwd: null pointer"), 1;
     const Shape s = shape_of(B, H, W, h, w, D, I, K, dtype);
-    const Saved v = saved_layout(s, const_cast<void*>(saved));
+    const Saved v = saved_layout(s, const_cast<void*>(saved), nullptr);   // (none of the forward's scratch is read)
     const BwdWork g = bwd_layout(s, workspace);
     if (workspace_bytes < g.bytes)
         return set_error("pdw_block_bwd: workspace of %zu bytes given, %zu needed", workspace_bytes, g.bytes), 1;

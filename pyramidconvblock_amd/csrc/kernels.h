@@ -174,4 +174,11 @@ int dwconv_fwd2_launch(const void* x0, const void* w0, void* y0, const void* x1,
                        int W, int h, int w, int C, int K, int dtype, hipStream_t s, int ldy0 = 0, int ych0 = 0, int ldy1 = 0,
                        int ych1 = 0, const struct PoolFwdJob* mean = nullptr);
 
+// block.hip: the launches of pdw_convblock_fwd, arguments checked; xparts: the sums of x per row tile of
+// pdw_dense_colsum_rows() rows, read before anything writes y; yp: one row per image
+int convblock_fwd_launch(const void* x, const void* w_up, const void* w_dw0, const void* w_dw1, const void* w_pool,
+                         const void* b_pool, const void* w_out, const void* b_out, void* a, void* c0, void* xp, void* c1,
+                         void* cat, void* m, void* y, float* xparts, float* yp, int B, int H, int W, int D, int I, int K,
+                         int dtype, void* stream);
+
 }  // namespace pdw

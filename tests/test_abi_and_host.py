@@ -75,6 +75,35 @@ def test_single_call_block_host_logic_without_gpu():
     assert b"not covered" in L.pdw_last_error()
 
 
+@pytest.mark.parametrize("B,H,W,D,K,dtype", [(32, 56, 56, 128, 13, 2), (3, 57, 61, 200, 9, 2), (32, 56, 56, 128, 13, 0),
+                                             (4, 64, 64, 1152, 13, 1), (8, 7, 7, 512, 3, 1)])
+def test_block_buffers_hold_no_scratch_beyond_its_use(B, H, W, D, K, dtype):
+    """pdw_block_*: the buffer between the passes holds what the backward reads and one row per image (the sums of x lie in
+    y until it is written); the backward's workspace holds two gradients at full resolution, two pooled ones and partial
+    sums (the gradient of the concatenation makes room for conv_up's)."""
+    from pyramidconvblock_amd import _lib
+
+    L = _lib.lib()
+    es, I, h, w = (4 if dtype == 0 else 2), D // 2, H // 2, W // 2
+    Il = I if I % 8 == 0 or dtype == 0 else 2 * ((I // 2 + 7) // 8 * 8)
+    up = lambda b: (b + 255) // 256 * 256
+    full, half = up(B * H * W * Il * es), up(B * h * w * Il * es)
+    packed = 0 if Il == I else 2 * up(Il * D * es) + 2 * up(K * K * Il * es)
+    shape = (B, H, W, h, w, D, I, K, dtype)
+    assert L.pdw_block_supported(*shape)
+    assert L.pdw_block_saved_bytes(*shape) == 3 * full + 2 * half + up(B * D * es) + packed + up(B * D * 4)
+    wgrads = sum(up(L.pdw_dwconv_wgrad_workspace_bytes(B, *hw, Il, K, K, 1, 1, K // 2, K // 2, 1, 1, dtype)) for hw in ((H, W), (h, w)))
+    n = B * H * W
+    wgrads += up(L.pdw_dense_wgrad_workspace_bytes(n, D, Il)) + up(L.pdw_dense_wgrad_workspace_bytes(n, Il, D))
+    sums = up((n + 31) // 32 * D * 4) + up(2 * D * es) + up(B * D * 4)
+    mean = max(B * 33 * D * 4 + 512, up(L.pdw_pool_branch_workspace_bytes(B, H * W, D)))   # (at most 32 partial sums an image)
+    assert L.pdw_block_bwd_workspace_bytes(*shape) <= 2 * full + 2 * half + wgrads + sums + mean
+    # y is written early: it must not be x
+    for y in (1 << 20, (1 << 20) + B * H * W * D * es - 16):
+        assert L.pdw_block_fwd(1 << 20, *([1 << 40] * 7), y, 1 << 40, 1 << 60, *shape, None) == 1
+        assert b"overlaps" in L.pdw_last_error()
+
+
 @pytest.mark.parametrize("shape", [(128, 2, 64, 64, 3), (128, 4, 64, 64, 3), (128, 6, 64, 64, 13), (96, 2, 34, 16, 5),
                                    (512, 6, 40, 128, 17), (32, 56, 56, 64, 13), (8, 56, 56, 64, 13), (1, 8, 36, 16, 9),
                                    (8, 112, 112, 48, 17), (128, 56, 56, 64, 13)])

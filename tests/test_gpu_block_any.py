@@ -45,3 +45,10 @@ def test_fp32_convolutions_of_two_scales(oracle, k, dim, shape):
     """Both scales' fp32 convolutions in one launch (csrc/dwconv_f32t.h): tiles of one, two and four images, two column tiles,
     odd batches and extents, slices of 4 channels."""
     _block_case(oracle, dim, k, shape, torch.float32)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("shape", [(2, 2, 2, 16), (1, 2, 3, 64), (5, 4, 4, 32), (1, 6, 6, 8), (64, 4, 8, 64), (3, 8, 8, 136)])
+def test_sums_of_x_in_the_result_or_behind_the_saved(oracle, dtype, shape):
+    """The forward's sums of x, in y until it is written, or (images of a few pixels) in the buffer of the saved tensors."""
+    _block_case(oracle, shape[3], 3, shape, dtype)
