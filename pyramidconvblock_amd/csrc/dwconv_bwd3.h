@@ -1,7 +1,10 @@
 // The three convolution launches at the end of a two-scale block's backward pass that do not depend on one another
 // (the full-scale input gradient, with the pooled branch's gradient added where the pool halved the extents, and the weight
 // gradients of both scales) as one launch: on a compute unit a band of each runs back to back, without two drains and
-// launch gaps in between.  Every problem runs in the tile that its width fills better, chosen per problem at run time.
+// launch gaps in between.  Every problem runs in the tile that its width fills better: by template where both full-scale
+// problems' are the wide ones, the pool halved the extents and no mean branch rides along (each workgroup starts with one
+// problem's arguments; chosen at run time as for the others, us: [32,56,56,64] filter 13 30.8 for 30.6, 9 32.4 for 31.6,
+// 17 50.1 for 49.6; [128,56,56,64] filter 13 98.8 for 97.6), at run time per problem elsewhere.
 // The kernel template and its per-filter-size launcher; dwconv_bwd3_k<K>.hip instantiate it, one file per size.
 #pragma once
 #include "dwconv_fwd2.h"
@@ -38,27 +41,40 @@ struct Bwd3Args {
 };
 
 // Each problem's workgroups are a contiguous range of the grid, in the order the launcher chose.
-template <typename T, int K, int CS, int NGA, int NB, int MODE>
+// NCB1: column blocks of the pooled scale's tile, those of the full scale being 16 patches and 8 blocks, and no mean branch;
+// 0: all as the arguments say.
+template <typename T, int K, int CS, int NGA, int NCB1, int NB, int MODE>
 __global__ __launch_bounds__(512, 1) void dwconv_bwd3_k(const Bwd3Args a) {
     const int blk = blockIdx.x;
-    if (blk >= a.nd + a.p[0].n + a.p[1].n) {
-        extern __shared__ uint32_t smem[];
-        mean_bwd_body<T, 512>(a.mean, blk - a.nd - a.p[0].n - a.p[1].n, reinterpret_cast<float*>(smem));
-        return;
+    if constexpr (NCB1 != 0) {
+        if ((unsigned)(blk - a.sd) < (unsigned)a.nd)
+            dwconv_tz_body<T, K, 16, CS, MODE>((const T*)a.gy, (const T*)a.w, (const T*)a.add, nullptr, (T*)a.dx, a.gd, blk - a.sd, a.nd);
+        else if ((unsigned)(blk - a.p[1].start) < (unsigned)a.p[1].n)
+            dwconv_wgrad_tz_body<T, NGA, NCB1, NB>((const T*)a.p[1].x, (const T*)a.p[1].gy, a.p[1].part, a.p[1].g,
+                                                   blk - a.p[1].start, a.p[1].n);
+        else
+            dwconv_wgrad_tz_body<T, NGA, 8, NB>((const T*)a.p[0].x, (const T*)a.p[0].gy, a.p[0].part, a.p[0].g,
+                                                blk - a.p[0].start, a.p[0].n);
+    } else {
+        if (blk >= a.nd + a.p[0].n + a.p[1].n) {
+            extern __shared__ uint32_t smem[];
+            mean_bwd_body<T, 512>(a.mean, blk - a.nd - a.p[0].n - a.p[1].n, reinterpret_cast<float*>(smem));
+            return;
+        }
+        if ((unsigned)(blk - a.sd) < (unsigned)a.nd) {
+            const T *gy = (const T*)a.gy, *w = (const T*)a.w, *add = (const T*)a.add;
+            if (a.npcd == 16) dwconv_tz_body<T, K, 16, CS, MODE>(gy, w, add, nullptr, (T*)a.dx, a.gd, blk - a.sd, a.nd);
+            else dwconv_tz_body<T, K, 8, CS, MODE>(gy, w, add, nullptr, (T*)a.dx, a.gd, blk - a.sd, a.nd);
+            return;
+        }
+        const bool full = (unsigned)(blk - a.p[0].start) < (unsigned)a.p[0].n;
+        const T *x = (const T*)(full ? a.p[0].x : a.p[1].x), *gy = (const T*)(full ? a.p[0].gy : a.p[1].gy);
+        float* const part = full ? a.p[0].part : a.p[1].part;
+        const WgTzGeom g = full ? a.p[0].g : a.p[1].g;
+        const int at = blk - (full ? a.p[0].start : a.p[1].start), n = full ? a.p[0].n : a.p[1].n;
+        if ((full ? a.p[0].ncb : a.p[1].ncb) == 8) dwconv_wgrad_tz_body<T, NGA, 8, NB>(x, gy, part, g, at, n);
+        else dwconv_wgrad_tz_body<T, NGA, 5, NB>(x, gy, part, g, at, n);
     }
-    if ((unsigned)(blk - a.sd) < (unsigned)a.nd) {
-        const T *gy = (const T*)a.gy, *w = (const T*)a.w, *add = (const T*)a.add;
-        if (a.npcd == 16) dwconv_tz_body<T, K, 16, CS, MODE>(gy, w, add, nullptr, (T*)a.dx, a.gd, blk - a.sd, a.nd);
-        else dwconv_tz_body<T, K, 8, CS, MODE>(gy, w, add, nullptr, (T*)a.dx, a.gd, blk - a.sd, a.nd);
-        return;
-    }
-    const bool full = (unsigned)(blk - a.p[0].start) < (unsigned)a.p[0].n;
-    const T *x = (const T*)(full ? a.p[0].x : a.p[1].x), *gy = (const T*)(full ? a.p[0].gy : a.p[1].gy);
-    float* const part = full ? a.p[0].part : a.p[1].part;
-    const WgTzGeom g = full ? a.p[0].g : a.p[1].g;
-    const int at = blk - (full ? a.p[0].start : a.p[1].start), n = full ? a.p[0].n : a.p[1].n;
-    if ((full ? a.p[0].ncb : a.p[1].ncb) == 8) dwconv_wgrad_tz_body<T, NGA, 8, NB>(x, gy, part, g, at, n);
-    else dwconv_wgrad_tz_body<T, NGA, 5, NB>(x, gy, part, g, at, n);
 }
 
 // Band heights and grid order of the three problems.  A compute unit holds one workgroup of this launch at a time, and a
@@ -151,6 +167,14 @@ static Bwd3Plan bwd3_plan(int B, const TzGeom& gd, int npcd, const WgTzPlan& p0,
     return best;
 }
 
+template <typename T, int K, int CS, int NGA, int NCB1, int NB, int MODE>
+static void bwd3_go(const Bwd3Args& a, unsigned grid, size_t lds, hipStream_t s) {
+    auto kern = dwconv_bwd3_k<T, K, CS, NGA, NCB1, NB, MODE>;
+    static std::once_flag once;
+    std::call_once(once, [&] { (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); });
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, s, a);
+}
+
 // -1: not covered (the caller makes the three launches).  16-bit types, C % 8 == 0, padding K / 2; the full scale
 // [B, H, W, C], the pooled one [B, h, w, C].  addp (optional, H = 2 h and W = 2 w): the pooled branch's gradient.
 template <int K>
@@ -215,21 +239,16 @@ static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* 
     for (const Bwd3Wgrad& p : a.p) lds = std::max(lds, p.ncb == 8 ? WgTzShape<NGA, 8, NB>::lds_bytes : WgTzShape<NGA, 5, NB>::lds_bytes);
     if (nmean) lds = std::max(lds, mean_lds(mean->D, 512));
     const unsigned grid = (unsigned)(nd + p0.nblocks + p1.nblocks + nmean);
-    static std::once_flag once[4];
-#define PDW_BWD3_GO(T, MODE, SLOT)                                                                                        \
-    {                                                                                                                     \
-        auto kern = dwconv_bwd3_k<T, K, CS, NGA, NB, MODE>;                                                               \
-        std::call_once(once[SLOT], [&] {                                                                                  \
-            (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);         \
-        });                                                                                                               \
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, s, a);                                                       \
-    }
-    if (dtype == kF16) {
-        if (addp) PDW_BWD3_GO(f16_t, 1, 0) else PDW_BWD3_GO(f16_t, 0, 1)
-    } else {
-        if (addp) PDW_BWD3_GO(bf16_t, 1, 2) else PDW_BWD3_GO(bf16_t, 0, 3)
-    }
-#undef PDW_BWD3_GO
+    const bool wide = a.npcd == 16 && p0.ncb == 8 && nmean == 0;
+    auto go = [&](auto t) {
+        using T = decltype(t);
+        if (!addp) bwd3_go<T, K, CS, NGA, 0, NB, 0>(a, grid, lds, s);
+        else if (!wide) bwd3_go<T, K, CS, NGA, 0, NB, 1>(a, grid, lds, s);
+        else if (p1.ncb == 8) bwd3_go<T, K, CS, NGA, 8, NB, 1>(a, grid, lds, s);
+        else bwd3_go<T, K, CS, NGA, 5, NB, 1>(a, grid, lds, s);
+    };
+    if (dtype == kF16) go(f16_t{});
+    else go(bf16_t{});
     if (int e = check_launch("dwconv_bwd3")) return e;
     const int n0 = B * p0.g.nbands * p0.g.ncolt, n1 = B * p1.g.nbands * p1.g.ncolt;
     if (dtype == kF16) {

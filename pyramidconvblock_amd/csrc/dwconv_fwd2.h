@@ -4,13 +4,17 @@
 // that does not depend on its height, so a launch of its own cuts a problem into enough bands to fill the chip; here
 // the full scale runs as whole-image bands on half of the compute units while the half scale's workgroups run on the
 // others (14.8 us against 13.9 + 7.9 us and a launch gap at [32,56,56,64], K = 13).  Each scale runs in the tile
-// (16 or 8 patches side by side) that its width fills better.
+// (16 or 8 patches side by side) that its width fills better: by template where the full scale's is the wide one and slices
+// are 16 channels (each workgroup starts with one problem's arguments and no choice between the fields of two; at run time,
+// us: filter 13 14.2 for 14.0; [128,56,56,64] filter 13 36.0 for 35.7), at run time elsewhere (with the mean branch, filters
+// 15 and 17: 24.7 and 24.6, by template 24.9 and 24.8).
 // The kernel template and its per-filter-size launcher; dwconv_fwd2_k<K>.hip instantiate it, one file per size.
 #pragma once
 #include <algorithm>
 #include <map>
 #include <queue>
 #include <tuple>
+#include <type_traits>
 #include <vector>
 
 #include "dwconv_tz.h"
@@ -32,10 +36,23 @@ struct Fwd2Args {
 };
 
 // MODE 0: the convolutions; 4: each with the gate applied in its store (dwconv_tz.h).
-template <typename T, int K, int CS, int MODE>
+// NPC0, NPC1: patches side by side of the two problems' tiles; 0: as the arguments say.
+template <typename T, int K, int CS, int NPC0, int NPC1, int MODE>
 __global__ __launch_bounds__(512, 1) void dwconv_fwd2_k(const Fwd2Args a) {
     const int blk = blockIdx.x;
-    if (blk >= a.p[0].n + a.p[1].n) {
+    if constexpr (NPC0 != 0) {
+        if ((unsigned)(blk - a.p[0].start) < (unsigned)a.p[0].n) {
+            dwconv_tz_body<T, K, NPC0, CS, MODE>((const T*)a.p[0].x, (const T*)a.p[0].w, nullptr, nullptr, (T*)a.p[0].y, a.p[0].g,
+                                                 blk - a.p[0].start, a.p[0].n);
+            return;
+        }
+        if ((unsigned)(blk - a.p[1].start) < (unsigned)a.p[1].n) {
+            dwconv_tz_body<T, K, NPC1, CS, MODE>((const T*)a.p[1].x, (const T*)a.p[1].w, nullptr, nullptr, (T*)a.p[1].y, a.p[1].g,
+                                                 blk - a.p[1].start, a.p[1].n);
+            return;
+        }
+    }
+    if (NPC0 != 0 || blk >= a.p[0].n + a.p[1].n) {
         // The mean branch (per-image mean -> conv_pool -> the row added to every output row of the image) needs a
         // launch whose memory system is not saturated, and its inputs are ready when this one starts: last in the
         // grid, its short workgroups go to compute units the convolutions leave free or have finished with.
@@ -45,16 +62,18 @@ __global__ __launch_bounds__(512, 1) void dwconv_fwd2_k(const Fwd2Args a) {
                                    blk - a.p[0].n - a.p[1].n, reinterpret_cast<float*>(smem));
         return;
     }
-    const bool first = (unsigned)(blk - a.p[0].start) < (unsigned)a.p[0].n;
-    const T* const x = (const T*)(first ? a.p[0].x : a.p[1].x);
-    const T* const w = (const T*)(first ? a.p[0].w : a.p[1].w);
-    T* const y = (T*)(first ? a.p[0].y : a.p[1].y);
-    const TzGeom g = first ? a.p[0].g : a.p[1].g;
-    const int at = blk - (first ? a.p[0].start : a.p[1].start), n = first ? a.p[0].n : a.p[1].n;
-    if ((first ? a.p[0].npc : a.p[1].npc) == 16)
-        dwconv_tz_body<T, K, 16, CS, MODE>(x, w, nullptr, nullptr, y, g, at, n);
-    else
-        dwconv_tz_body<T, K, 8, CS, MODE>(x, w, nullptr, nullptr, y, g, at, n);
+    if constexpr (NPC0 == 0) {
+        const bool first = (unsigned)(blk - a.p[0].start) < (unsigned)a.p[0].n;
+        const T* const x = (const T*)(first ? a.p[0].x : a.p[1].x);
+        const T* const w = (const T*)(first ? a.p[0].w : a.p[1].w);
+        T* const y = (T*)(first ? a.p[0].y : a.p[1].y);
+        const TzGeom g = first ? a.p[0].g : a.p[1].g;
+        const int at = blk - (first ? a.p[0].start : a.p[1].start), n = first ? a.p[0].n : a.p[1].n;
+        if ((first ? a.p[0].npc : a.p[1].npc) == 16)
+            dwconv_tz_body<T, K, 16, CS, MODE>(x, w, nullptr, nullptr, y, g, at, n);
+        else
+            dwconv_tz_body<T, K, 8, CS, MODE>(x, w, nullptr, nullptr, y, g, at, n);
+    }
 }
 
 // Workgroups dealt in grid order to the earliest free of 256 compute units: the time the last one ends.
@@ -131,9 +150,17 @@ static Fwd2Plan fwd2_plan(int B, const TzGeom& g0, int npc0, const TzGeom& g1, i
     return best;
 }
 
+template <typename T, int K, int CS, int NPC0, int NPC1, int MODE>
+static void fwd2_go(const Fwd2Args& a, unsigned grid, size_t lds, hipStream_t s) {
+    auto kern = dwconv_fwd2_k<T, K, CS, NPC0, NPC1, MODE>;
+    static std::once_flag once;
+    std::call_once(once, [&] { (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); });
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, s, a);
+}
+
 // -1: not covered (the caller makes the two launches).  16-bit types, C % 8 == 0, padding K / 2; the full scale
 // [B, H, W, C], the pooled one [B, h, w, C].
-// gate0, gate1 (both or neither): the gate in the store of each scale, y0 / y1 then being the gated tensors with the
+// gate0, gate1 (both or neither, the full scale in the wide tile): the gate in the store of each scale, y0 / y1 then being the gated tensors with the
 // strides and channel offsets the gates name.
 template <int K>
 static int launch_fwd2(const void* x0, const void* w0, void* y0, const void* x1, const void* w1, void* y1, int B, int H,
@@ -141,7 +168,7 @@ static int launch_fwd2(const void* x0, const void* w0, void* y0, const void* x1,
                        const TzGate* gate1 = nullptr, const PoolFwdJob* mean = nullptr) {
     constexpr int CS = (2 * 4 * TzShape<K, 16, 16>::NM + 2 * 4 * TzShape<K, 16, 16>::RING) <= 160 ? 16 : 8;
     if (dtype == kF32 || C % 8 != 0 || B < 1 || H < 1 || W < 1 || h < 1 || w < 1) return -1;
-    if ((gate0 != nullptr) != (gate1 != nullptr)) return -1;
+    if ((gate0 != nullptr) != (gate1 != nullptr) || (gate0 && !tz_wide_tile(B, W))) return -1;
     const int P = K / 2;
     for (const void* p : {x0, w0, (const void*)y0, x1, w1, (const void*)y1})
         if (!p || (reinterpret_cast<uintptr_t>(p) & 15)) return -1;
@@ -175,21 +202,19 @@ static int launch_fwd2(const void* x0, const void* w0, void* y0, const void* x1,
     for (const Fwd2Problem& p : a.p) lds = std::max(lds, p.npc == 16 ? TzShape<K, 16, CS>::lds_bytes : TzShape<K, 8, CS>::lds_bytes);
     if (nmean > 0) lds = std::max(lds, (size_t)9 * mean->D * sizeof(float));
     const unsigned grid = (unsigned)(n[0] + n[1] + nmean);
-    static std::once_flag once[4];
-#define PDW_FWD2_GO(T, MODE, SLOT)                                                                                    \
-    {                                                                                                                 \
-        auto kern = dwconv_fwd2_k<T, K, CS, MODE>;                                                                    \
-        std::call_once(once[SLOT], [&] {                                                                              \
-            (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);     \
-        });                                                                                                           \
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, s, a);                                                   \
-    }
-    if (gate0) {
-        if (dtype == kF16) PDW_FWD2_GO(f16_t, 4, 0) else PDW_FWD2_GO(bf16_t, 4, 1)
-    } else {
-        if (dtype == kF16) PDW_FWD2_GO(f16_t, 0, 2) else PDW_FWD2_GO(bf16_t, 0, 3)
-    }
-#undef PDW_FWD2_GO
+    auto go = [&](auto t, auto mode) {
+        using T = decltype(t);
+        constexpr int MODE = decltype(mode)::value;
+        if constexpr (CS == 16) {
+            if (f.npc == 16 && q.npc == 16) return fwd2_go<T, K, CS, 16, 16, MODE>(a, grid, lds, s);
+            if (f.npc == 16) return fwd2_go<T, K, CS, 16, 8, MODE>(a, grid, lds, s);
+        }
+        if constexpr (CS != 16 || MODE == 0) fwd2_go<T, K, CS, 0, 0, MODE>(a, grid, lds, s);
+    };
+    using Plain = std::integral_constant<int, 0>;
+    using Gated = std::integral_constant<int, 4>;
+    if (gate0) dtype == kF16 ? go(f16_t{}, Gated{}) : go(bf16_t{}, Gated{});
+    else dtype == kF16 ? go(f16_t{}, Plain{}) : go(bf16_t{}, Plain{});
     return check_launch("dwconv_fwd2");
 }
 
