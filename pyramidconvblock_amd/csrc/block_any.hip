@@ -368,7 +368,11 @@ extern "C" {
 int pdw_block_supported(int B, int H, int W, int h, int w, int D, int I, int K, int dtype) {
     if (dtype != kF32 && dtype != kF16 && dtype != kBF16) return 0;
     if (B < 1 || H < 1 || W < 1 || h < 1 || w < 1 || K < 1 || !(K & 1) || D < 4 || I < 4 || (I & 1)) return 0;
-    if ((long long)B * H * W * (D > I ? D : I) > 0x7fffffffLL || (long long)H * h > 0x7fffffffLL) return 0;
+    if ((long long)B * H * W * (D > I ? D : I) > 0x7fffffffLL) return 0;
+    // the pool's bins are found in 32-bit products of the extents (the fused launches, on exact halves, need none)
+    if (((long long)H * h >= 0x7fffffffLL || (long long)W * w >= 0x7fffffffLL) &&
+        !(H == 2 * h && W == 2 * w && pdw_convblock_supported(B, H, W, D, I, K, dtype)))
+        return 0;
     if ((long long)B * h * w * I > 0x7fffffffLL) return 0;
     const int Il = 2 * padded_half((long long)B * H * W, D, I, K, dtype);
     if (Il * (long long)B * H * W > 0x7fffffffLL) return 0;

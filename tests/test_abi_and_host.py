@@ -104,6 +104,21 @@ def test_block_buffers_hold_no_scratch_beyond_its_use(B, H, W, D, K, dtype):
         assert b"overlaps" in L.pdw_last_error()
 
 
+def test_block_extents_beyond_the_pools_bins():
+    """pdw_block_supported: extents whose products do not fit the pool's 32-bit bins, of rows and of columns, are not taken
+    (the single calls refuse them), unless the fused launches do, which have no bins."""
+    from pyramidconvblock_amd import _lib
+
+    L = _lib.lib()
+    for dtype in (0, 1, 2):
+        for H, W in ((2, 70001), (70001, 2), (2, 70000), (70000, 2)):
+            assert L.pdw_block_supported(1, H, W, H // 2, W // 2, 8, 4, 3, dtype) == 0
+            assert L.pdw_avgpool_fwd(1 << 20, 1 << 21, 1, H, W, 4, H // 2, W // 2, dtype, None) == 1
+            assert b"too large" in L.pdw_last_error()
+        assert L.pdw_block_supported(1, 2, 65535, 1, 32767, 8, 4, 3, dtype) == 1
+    assert L.pdw_block_supported(1, 4, 70000, 2, 35000, 64, 32, 3, 2) == 1
+
+
 @pytest.mark.parametrize("shape", [(128, 2, 64, 64, 3), (128, 4, 64, 64, 3), (128, 6, 64, 64, 13), (96, 2, 34, 16, 5),
                                    (512, 6, 40, 128, 17), (32, 56, 56, 64, 13), (8, 56, 56, 64, 13), (1, 8, 36, 16, 9),
                                    (8, 112, 112, 48, 17), (128, 56, 56, 64, 13)])
