@@ -104,8 +104,8 @@ def _block(oracle, dim, k, shape, dtype, seed=0, **kw):
 @pytest.mark.parametrize("scales", [(1.,), (0.5,), (1., 0.5, 0.25), (0.5, 1.), (1., 1.), (1., 0.75)])
 @pytest.mark.parametrize("shape", [(2, 16, 24, 64), (2, 13, 18, 64)])
 def test_block_scales(oracle, dtype, scales, shape):
-    """Every combination of scales the constructor accepts runs the single-branch launches of the block
-    (one gate per branch, pooled gradients accumulated into the full-resolution one)."""
+    """Every combination of scales the constructor accepts: (1, s) on the two-scale launches, the others on the single-branch
+    ones (one gate per branch, pooled gradients accumulated into the full-resolution one)."""
     _block(oracle, 64, 7, shape, dtype, scales=scales)
 
 

@@ -3,8 +3,71 @@ import pytest
 import torch
 
 from parity import assert_close, randn
+from test_gpu_block import _block_case
+from test_gpu_modules import _block
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def native_only(monkeypatch):
+    """The block's Python form is out of reach."""
+    from pyramidconvblock_amd import conv_block
+
+    class Refuse:
+        @staticmethod
+        def apply(*a):
+            raise AssertionError("the block went to its Python form")
+
+    monkeypatch.setattr(conv_block, "ConvBlockFunction", Refuse)
+
+
+@pytest.mark.parametrize("dim,k,shape", [(264, 5, (2, 9, 12, 264)), (512, 3, (3, 16, 16, 512)), (1032, 7, (1, 7, 9, 1032))])
+def test_fp32_blocks_wider_than_256(oracle, native_only, dim, k, shape):
+    _block_case(oracle, dim, k, shape, torch.float32)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("s", [2., 1.5, 0.75, 0.3])
+@pytest.mark.parametrize("dim,shape", [(64, (2, 13, 18, 64)), (40, (3, 16, 34, 40)), (200, (1, 8, 9, 200))])
+def test_second_scales_below_and_above_one(oracle, native_only, dtype, s, dim, shape):
+    """Second scales that are not a half, enlarging ones among them (bins that overlap, a resize down)."""
+    _block(oracle, dim, 7, shape, dtype, scales=(1., s))
+
+
+@pytest.mark.parametrize("kind,dim,shape,dtype", [("block", 128, (2, 16, 32, 128), torch.bfloat16), ("block", 64, (2, 13, 18, 64), torch.float32),
+                                                  ("conv", 64, (2, 13, 18, 64), torch.float16)])
+def test_on_a_side_stream(kind, dim, shape, dtype):
+    """Input and gradient written late on a side stream, the forward there, the backward asked for from the default stream:
+    every kernel has to run on the forward's stream, behind what it reads."""
+    import pyramidconvblock_amd
+
+    torch.manual_seed(9)
+    layer = (pyramidconvblock_amd.ConvBlock(dim=dim, kernel_size=5) if kind == "block"
+             else pyramidconvblock_amd.OptimizedDepthwiseConv2d(dim, 5, padding=2)).to(dtype).cuda()
+    x, g = (torch.randn(shape, device="cuda").to(dtype) for _ in range(2))
+    x.requires_grad_()
+    y = layer(x)
+    want = [y, *torch.autograd.grad(y, [x, *layer.parameters()], g)]
+    with torch.no_grad():
+        plain = layer(x)
+    late, late_g = torch.zeros_like(x, requires_grad=True), torch.zeros_like(g)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(20_000_000)
+        with torch.no_grad():
+            late.copy_(x)
+            inferred = layer(late)
+        y = layer(late)
+        torch.cuda._sleep(20_000_000)
+        late_g.copy_(g)
+    torch.cuda.current_stream().wait_stream(side)
+    got = [y, *torch.autograd.grad(y, [late, *layer.parameters()], late_g)]
+    torch.cuda.synchronize()
+    assert torch.equal(inferred, plain)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("dim,k,shape,dtype", [
@@ -145,8 +208,8 @@ def _layers():
     import pyramidconvblock_amd
 
     torch.manual_seed(3)
-    return [pyramid_dwconv.ConvBlock(dim=64, kernel_size=5).cuda(),
-            pyramidconvblock_amd.OptimizedDepthwiseConv2d(64, 5, padding=2).cuda()]
+    return [pyramid_dwconv.ConvBlock(dim=64, kernel_size=5).float().cuda(),
+            pyramidconvblock_amd.OptimizedDepthwiseConv2d(64, 5, padding=2).float().cuda()]
 
 
 @pytest.mark.parametrize("which", [0, 1])
