@@ -6,16 +6,20 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("dim", [64, 128])  # 128: the block runs as one library call per direction
-def test_graph_replays_match_eager(dim):
+@pytest.mark.parametrize("dim,hw,dtype", [
+    (64, (28, 32), torch.bfloat16), (128, (28, 32), torch.bfloat16),   # the fused launches
+    (200, (29, 33), torch.bfloat16),                                   # the general ones: packed weights, odd extents,
+    (64, (28, 32), torch.float32), (264, (13, 18), torch.float16),     # fp32, wide layers
+])
+def test_graph_replays_match_eager(dim, hw, dtype):
     import pyramid_dwconv
     from pyramidconvblock_amd.graphs import GraphedStep
 
     torch.manual_seed(0)
-    m = pyramid_dwconv.ConvBlock(dim, kernel_size=9).to(torch.bfloat16).cuda()
+    m = pyramid_dwconv.ConvBlock(dim, kernel_size=9).to(dtype).cuda()
     gen = torch.Generator().manual_seed(1)
-    x = torch.randn(4, 28, 32, dim, generator=gen).to(torch.bfloat16).cuda()
-    g = torch.randn(4, 28, 32, dim, generator=gen).to(torch.bfloat16).cuda()
+    x = torch.randn(4, *hw, dim, generator=gen).to(dtype).cuda()
+    g = torch.randn(4, *hw, dim, generator=gen).to(dtype).cuda()
     step = GraphedStep(m, x, g)
     graph_grads = [step.x.grad] + step.param_grads
 
@@ -32,7 +36,7 @@ def test_graph_replays_match_eager(dim):
 
     for rep in range(4):
         if rep == 2:  # new input data through the static buffers
-            step.x.data.copy_(torch.randn(4, 28, 32, dim, generator=gen).to(torch.bfloat16))
+            step.x.data.copy_(torch.randn(4, *hw, dim, generator=gen).to(dtype))
         ref = eager(step.x)
         step.y.zero_()
         for t in graph_grads:
