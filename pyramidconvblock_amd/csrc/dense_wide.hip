@@ -311,6 +311,9 @@ WgradPlan wgrad_plan(long long N, int M, int NO, int es) {
     long long s = cut();
     // fp32, bound by the matrix pipe and not by what the tiles read: smaller ones where these would be too few
     if (es == 4 && s * p.mt * p.nt < 512) p.bm = p.bn = 64, s = cut();
+    // no range longer than its 32-bit offsets reach (operands of more than 2 GiB, widths that alone fill the chip)
+    const long long most = 0x7fffffffLL / ((long long)(M > NO ? M : NO) * es) / 64 * 64;
+    if (most > 0 && s < (N + most - 1) / most) s = (N + most - 1) / most;
     p.kper = ((N + s - 1) / s + 63) / 64 * 64;
     p.splits = (int)((N + p.kper - 1) / p.kper);
     return p;

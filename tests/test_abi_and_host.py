@@ -104,6 +104,17 @@ def test_block_buffers_hold_no_scratch_beyond_its_use(B, H, W, D, K, dtype):
         assert b"overlaps" in L.pdw_last_error()
 
 
+@pytest.mark.parametrize("N,M,NO", [(458752, 4096, 2048), (458752, 2048, 4096), (1 << 20, 2040, 1020), (1 << 17, 16376, 64)])
+def test_wide_weight_gradient_ranges_fit_32_bit_offsets(N, M, NO):
+    """pdw_dense_wgrad of wide layers cuts the rows into ranges whose operands 32-bit offsets reach, also where the layer's
+    tiles alone fill the chip: the workspace holds a partial result for each."""
+    from pyramidconvblock_amd import _lib
+
+    parts = _lib.lib().pdw_dense_wgrad_workspace_bytes(N, M, NO) // (M * NO * 4)
+    reach = (2**31 - 1) // (max(M, NO) * 4) // 64 * 64   # (the larger of the types; the workspace is for either)
+    assert parts * reach >= N
+
+
 def test_block_extents_beyond_the_pools_bins():
     """pdw_block_supported: extents whose products do not fit the pool's 32-bit bins, of rows and of columns, are not taken
     (the single calls refuse them), unless the fused launches do, which have no bins."""

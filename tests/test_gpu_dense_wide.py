@@ -44,3 +44,19 @@ def test_dense_wide_fp32_layers(K, NO, N, P):
 def test_dense_wide_columns_of_192(dtype, K, NO):
     """Tiles of 128 x 192: rows enough for one round of them to save one of the narrower ones, remainders in both."""
     _layers(dtype, K, NO, 257 * 128 + 5, 257 * 128 + 5)
+
+
+@pytest.mark.parametrize("dtype,N", [(torch.bfloat16, 270000), (torch.float32, 140000)])
+def test_weight_gradient_of_more_than_2_gib(dtype, N):
+    """A layer whose tiles alone fill the chip, over operands that one range's 32-bit offsets do not reach."""
+    from pyramidconvblock_amd import ops
+
+    M, NO = 4096, 2048
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    a = torch.randn(N, M, generator=gen, device="cuda").to(dtype)
+    b = torch.randn(N, NO, generator=gen, device="cuda").to(dtype)
+    assert a.numel() * a.element_size() > 2**31
+    got = ops.dense_wgrad(a, b)
+    cols = torch.tensor([0, 127, 128, 2047, 4095], device="cuda")
+    want = sum(a[i:i + 20000, cols].double().t() @ b[i:i + 20000].double() for i in range(0, N, 20000))
+    assert_close(got[cols], want.cpu().numpy(), dtype, "dw")
