@@ -326,10 +326,12 @@ int pdw_block_mid_infer(const void *xh, void *y, int B, int H, int W, int h, int
                         void *m, float *rowbias, int P, int D, int dtype, void *stream);
 
 /* Dense layers of the block on the matrix cores.  bf16/fp16 with K <= 128, NO <= 128, K % 8 == 0, NO % 8 == 0 run the
- * tiled kernels (persistent workgroups, weights in LDS, a 32-row tile per wavefront over all features); fp32 and
- * every other width with K % 4 == 0, NO % 4 == 0, K <= 256 run one 32 x 32 result tile per wavefront
- * (v_mfma_f32_32x32x2_f32 in fp32), forward, input gradient and weight gradient alike.  pdw_dense_supported says
- * whether a shape is covered - callers use a library GEMM otherwise.
+ * tiled kernels (persistent workgroups, weights in LDS, a 32-row tile per wavefront over all features); wider ones
+ * (K % 8 == 0, NO % 8 == 0) run tiles of 128 x 128 results, fp32 layers (K % 4 == 0, NO % 4 == 0) tiles of 64 x 64,
+ * and fp32 weight gradients and other 16-bit widths (K % 4 == 0, NO % 4 == 0, K <= 256) one 32 x 32 result tile per
+ * wavefront.  pdw_dense_supported says whether a shape is covered, forward, input gradient and weight gradient
+ * alike - callers use a library GEMM otherwise; it answers no for fp32 with K > 256, which pdw_dense_fwd and
+ * pdw_dense_wgrad take all the same.
  *   y[n,o] = sum_k x[n,k] * W(o,k) + bias[o] + rowbias[n / P][o]        x[N,K] -> y[N,NO]
  * W(o,k) = w[o*K + k] (w_kmajor == 0, the nn.Linear layout) or w[k*NO + o] (w_kmajor != 0, which gives the
  * input gradient of a layer from its own weight without a transpose).  bias (element type) and rowbias

@@ -8,15 +8,16 @@ names, parameter shapes and ``[B,H,W,C]`` in/out contract
 ``ConvBlock.forward`` runs as ONE autograd node: in native code (``csrc/torch_ops.cpp`` over
 ``pdw_block_fwd`` / ``_bwd``) for two scales wherever the library's dense layers cover the widths,
 as ``ConvBlockFunction``, the same launches made one by one from Python, for everything else (other
-scale tuples, a bias on ``conv_up``, mixed types).  The pooling, depthwise
+scale tuples, a bias on ``conv_up``, mixed types, calls under torch.jit.trace).  The pooling, depthwise
 convolutions, gates and upsampling go through libpdw.so, the gate outputs are written straight
 into the halves of the concatenated buffer (no ``torch.cat``), the pooled branch is added in
 place, and the backward reuses one per-image column sum for both bias gradients and the
 gradient of the mean.  The dense layers run on the matrix-core kernels of libpdw.so (bias /
 broadcast add fused into the store, deterministic split reduction for the weight gradients):
-16-bit layers up to 128 wide in the tiled kernels, wider ones in tiles of 128 x 128 results, fp32 and
-widths that are multiples of 4 only (inner width up to 256) one result tile per wavefront; anything else
-uses library GEMMs, with the weight gradients as a batched split-K product.
+16-bit layers up to 128 wide in the tiled kernels, wider ones in tiles of 128 x 128 results (inner widths off
+multiples of 8 on zero-padded channels), fp32 ones in tiles of 64 x 64 with weight gradients up to 256 wide one result
+tile per wavefront.  Widths that none of them take (and, launch by launch from Python, fp32 inner widths above 256) use
+library GEMMs, with the weight gradients as a batched split-K product.
 """
 from __future__ import annotations
 

@@ -235,7 +235,8 @@ def add_rowbias_(y, v):
 def dense_supported(K, NO, dtype):
     """True when the matrix-core dense kernels cover an inner size K, output size NO layer of this dtype (forward,
     input gradient and weight gradient): 16-bit layers up to 128 wide in the tiled kernels, any wider ones (multiples of
-    8) in 128 x 128 tiles, and fp32 or other widths (multiples of 4, inner width up to 256) one result tile per wavefront."""
+    8) in 128 x 128 tiles, other 16-bit widths (multiples of 4, inner width up to 256) one result tile per wavefront; fp32
+    (multiples of 4, inner width up to 256) in 64 x 64 tiles, the weight gradient one result tile per wavefront."""
     if dtype not in _lib._DTYPES:
         return False
     return bool(_lib.lib().pdw_dense_supported(int(K), int(NO), _lib.dtype_code(dtype)))
