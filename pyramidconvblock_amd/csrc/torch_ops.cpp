@@ -131,9 +131,9 @@ struct BlockNode : public torch::autograd::Node {
     }
 };
 
-// Whether the library's block calls take this: everything on x's device in x's type, conv_up without bias, two square
-// odd filters of one shape, and extents and widths that pdw_block_supported.
-bool block_shape(const Tensor* in, const Tensor& b_up, double s0, double s1, BlockShape* s) {
+// Whether these are a block of the library's calls: everything on x's device in x's type, conv_up without bias, two square
+// filters of one shape, widths that fit together.  (Which extents, widths and filters are covered, the library says.)
+bool block_args(const Tensor* in, const Tensor& b_up, double s0, double s1, BlockShape* s) {
     const Tensor& x = in[kX];
     if (b_up.defined() || s0 != 1.0 || s1 == 1.0 || x.dim() != 4 || !x.is_cuda()) return false;
     const int dt = dtype_code(x.scalar_type());
@@ -152,7 +152,12 @@ bool block_shape(const Tensor* in, const Tensor& b_up, double s0, double s1, Blo
         if (e > 0x7fffffff) return false;
     const int H = (int)x.size(1), W = (int)x.size(2);
     *s = {(int)x.size(0), H, W, (int)(H * s1), (int)(W * s1), (int)D, (int)I, (int)K, dt};
-    return pdw_block_supported(PDW_SHAPE(*s)) != 0;
+    return true;
+}
+
+// Whether the inference call of the fused launches takes it.
+bool infer_shape(const BlockShape& s) {
+    return s.H == 2 * s.h && s.W == 2 * s.w && pdw_convblock_supported(s.B, s.H, s.W, s.D, s.I, s.K, s.dtype);
 }
 
 Tensor block_train_or_infer(const Tensor* in, const BlockShape& s, bool grad) {
@@ -303,12 +308,12 @@ PyObject* py_block(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const double s0 = PyFloat_AsDouble(args[9]), s1 = PyFloat_AsDouble(args[10]);
     if (PyErr_Occurred()) return nullptr;
     BlockShape s;
-    if (!plain_call(in, kBlockInputs) || !block_shape(in, b_up, s0, s1, &s)) Py_RETURN_NONE;
+    if (!plain_call(in, kBlockInputs) || !block_args(in, b_up, s0, s1, &s)) Py_RETURN_NONE;
     bool grad = false;
     if (at::GradMode::is_enabled())
         for (const Tensor& t : in) grad = grad || (t.defined() && t.requires_grad());
-    if (!grad && s.H == 2 * s.h && s.W == 2 * s.w && pdw_convblock_supported(s.B, s.H, s.W, s.D, s.I, s.K, s.dtype))
-        Py_RETURN_TRUE;
+    if (!grad && infer_shape(s)) Py_RETURN_TRUE;
+    if (!pdw_block_supported(PDW_SHAPE(s))) Py_RETURN_NONE;
     Tensor y;
     {
         pybind11::gil_scoped_release no_gil;
@@ -332,8 +337,7 @@ PyObject* py_block_infer(PyObject*, PyObject* const* args, Py_ssize_t n) {
         TORCH_CHECK(in[i].defined() ? in[i].is_cuda() : i == kBOut || i == kBPool,
                     "convblock_infer: tensors on a HIP device expected (the biases may be None)");
     BlockShape s;
-    TORCH_CHECK(plain_call(in, kBlockInputs) && block_shape(in, Tensor(), 1.0, 0.5, &s) && s.H == 2 * s.h && s.W == 2 * s.w &&
-                    pdw_convblock_supported(s.B, s.H, s.W, s.D, s.I, s.K, s.dtype),
+    TORCH_CHECK(plain_call(in, kBlockInputs) && block_args(in, Tensor(), 1.0, 0.5, &s) && infer_shape(s),
                 "convblock_infer: not a call that pdw_convblock_infer covers (input ", in[kX].sizes(), " ",
                 in[kX].scalar_type(), ", filters ", in[kDw0].sizes(), ")");
     Tensor y;
