@@ -211,7 +211,7 @@ def test_the_host_extension_is_bound_to_its_torch(monkeypatch):
     """Another torch than the one the extension was compiled against: that file is not loaded, one is built."""
     from pyramidconvblock_amd import _lib, build
 
-    assert os.path.exists(build.ext_path(torch.__version__)) and _lib.ext()
+    assert _lib.ext() and os.path.exists(build.ext_path(torch.__version__))
     asked = []
 
     def build_ext():
