@@ -177,7 +177,7 @@ size_t dwconv_wgrad_tiled_workspace(int B, int H, int W, int C, int KH, int KW, 
         case 13: wt = dwconv_wgrad_tiled_ws_k13(B, H, W, C, PH, PW, dtype); break;
         case 15: wt = dwconv_wgrad_tiled_ws_k15(B, H, W, C, PH, PW, dtype); break;
         case 17: wt = dwconv_wgrad_tiled_ws_k17(B, H, W, C, PH, PW, dtype); break;
-        default: return 0;
+        default: break;   // (even filters: the dense matrix-core kernel's partials alone)
     }
     return wt > wm ? wt : wm;
 }
