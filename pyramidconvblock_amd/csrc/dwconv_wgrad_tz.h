@@ -1,19 +1,18 @@
-// Depthwise-convolution weight gradient on the dense matrix cores (16-bit types, stride 1, dilation 1, square
-// filters up to 17):     dw[u,v,c] = sum_{b,i,j} gy[b,i,j,c] * xw[b, i+u, j+v, c],   xw[r][s] = x[r-PH][s-PW].
+// Depthwise-convolution weight gradient on the dense matrix cores for the filters 16 and 17 (16-bit types, stride 1,
+// dilation 1; smaller ones: dwconv_wgrad_ph.h):
+//     dw[u,v,c] = sum_{b,i,j} gy[b,i,j,c] * xw[b, i+u, j+v, c],   xw[r][s] = x[r-PH][s-PW].
 //
 // With u = 2a + du, v = 8b + dv and the position p = (i + du, j + dv) the sum for one channel is
 //     dw[2a+du][8b+dv] = sum_p  xw[p + (2a, 8b)] * gy[p - (du, dv)],
-// which is one v_mfma_f32_16x16x32_{bf16,f16} product D[m][n] += sum_k A[m][k] B[k][n] with m = (a, b) = 2a + b,
-// n = (du, dv) = 8 du + dv and k running over a block of 4 rows x 8 columns of positions (a lane holds 8 consecutive
-// columns of one row: lane = m + 16 * row for A, n + 16 * row for B):
+// a v_mfma_f32_16x16x32_{bf16,f16} product D[m][n] += sum_k A[m][k] B[k][n] with m = (a, b), n = (du, dv) = 8 du + dv and k
+// running over a block of 4 rows x 8 columns of positions (a lane holds 8 consecutive columns of one row: lane = m + 16 * row
+// for A, n + 16 * row for B):
 //     A[(a,b)][(kr,e)]   = xw[R + kr + 2a][Cc + e + 8b]
 //     B[(kr,e)][(du,dv)] = gy[R + kr - du][Cc + e - dv]        (zero outside the band's own rows and columns)
-// One accumulator of 4 registers holds all 16 x 16 taps of a channel (169 of 256 used at K = 13), and a band of
-// BR x 56 positions takes ceil((BR+1)/4) x 8 instructions per channel.  K = 17 has 9 x 3 tap blocks (a, b): they are
-// numbered a * NB + b over two instructions that share the gy operand.  Both operands are data, so nothing is kept
-// per channel but the accumulator: a wavefront owns 2 of the workgroup's 16 channels for the whole band and
-// writes their taps to the fp32 partial of the band at the end; the partials are summed in a fixed order by
-// wgrad_reduce_parts (no atomics: bit-reproducible).
+// The 9 x 3 tap blocks (a, b) are numbered 3 a + b over two instructions that share the gy operand: two accumulators of 4
+// registers hold all taps of a channel.  Both operands are data, so nothing is kept per channel but the accumulators: a
+// wavefront owns 2 of the workgroup's 16 channels for the whole band and writes their taps to the fp32 partial of the band
+// at the end; the partials are summed in a fixed order by wgrad_reduce_parts (no atomics: bit-reproducible).
 //
 // The kernel is bound by LDS reads (two 1 KB operands per instruction, no reuse).  Aligned 16-byte reads run at
 // twice the rate of narrower ones on this part (measured: 256 against 128 bytes per clock), which is why the
@@ -37,13 +36,14 @@
 
 namespace pdw {
 
-// NGA: row groups (of 4 rows) the xw operand of a step spans (rows kr + 2a, a <= (K-1)/2); NCB: column blocks of 8
-// positions per band row (8: bands of 56 columns, 5: of 32); NB: tap column blocks (2: K <= 16, 3: K = 17).
-template <int NGA, int NCB, int NB>
+// NCB: column blocks of 8 positions per band row (8: bands of 56 columns, 5: of 32).
+template <int NCB>
 struct WgTzShape {
     static constexpr int NT = 512, CS = 16, CPW = 2, NH = 2;
     static constexpr int TWG = 8 * NCB - 8;                 // gy columns of a workgroup: TWG + 7 <= 8 NCB positions
-    static constexpr int NMF = NB == 3 ? 2 : 1;             // instructions per position block and channel
+    static constexpr int NGA = 5;                           // row groups (of 4 rows) the xw operand of a step spans (rows kr + 2a, a <= 8)
+    static constexpr int NB = 3;                            // tap column blocks
+    static constexpr int NMF = 2;                           // instructions per position block and channel
     static constexpr int WCX = 8 * NCB + 8 * (NB - 1);      // xw window columns the operands touch
     static constexpr int WCG = 8 * NCB + 8;                 // gy window columns: 8 of padding on the left
     // LDS pitches, chosen by measurement of the operands' access patterns on this part.  xw (ds_read_b128, lane (a, b, kr)
@@ -54,16 +54,15 @@ struct WgTzShape {
     static constexpr int RPX = (2 * WCX - 32 + 127) / 128 * 128 + 32;
     static constexpr int RPG = (2 * WCG - 40 + 127) / 128 * 128 + 40;
     // ring slots (row groups).  xw: the NGA groups a step reads and the two the pass committed meanwhile covers; even,
-    // so that a pass never wraps.  gy: a step reads groups t-1 and t while a whole pass (groups t+1, t+2) is committed;
-    // where LDS is short (NGA = 5) a step commits only group t+1, one half of a pass, and 3 slots do.
-    static constexpr int NSX = NGA + 2 + (NGA % 2), NSG = NGA == 5 ? 3 : 4;
+    // so that a pass never wraps.  gy: a step reads groups t-1 and t and commits group t+1, one half of a pass (LDS is short).
+    static constexpr int NSX = NGA + 2 + (NGA % 2), NSG = 3;
     static constexpr int GBX = 4 * RPX, GBG = 4 * RPG;      // bytes per row group of a channel
     static constexpr int CHPX = NSX * GBX + 16, CHPG = NSG * GBG + 8;   // channel planes
     static constexpr int XHALF = 64;                        // channels 8..15 sit 16 banks further: the two 8-channel
                                                             // pieces of a staging pass write different banks
     static constexpr int XB = CS * CHPX + XHALF, GCB = (CS * CHPG + 127) / 128 * 128 + 24;  // xw window; one gy copy
     static constexpr size_t lds_bytes = (size_t)XB + 2 * GCB;
-    static_assert(NGA >= 2 && NGA <= 5 && (NCB == 8 || NCB == 5) && (NB == 2 || NB == 3), "row groups spanned, column blocks");
+    static_assert(NCB == 8 || NCB == 5, "column blocks");
     static_assert(RPX % 128 == 32 && RPX >= 2 * WCX && RPG % 128 == 40 && RPG >= 2 * WCG && CHPX % 16 == 0 && GCB % 128 == 24,
                   "operand alignment / bank spread");
     // gy staging item: 4 consecutive columns of one window row x an 8-channel piece; a window row is GLPR consecutive
@@ -84,11 +83,12 @@ struct WgTzGeom {
 };
 
 // One workgroup's band: `blk` of the problem's `nblk` workgroups.
-template <typename T, int NGA, int NCB, int NB>
+template <typename T, int NCB>
 __device__ __forceinline__ void dwconv_wgrad_tz_body(const T* __restrict__ x, const T* __restrict__ gy,
                                                      float* __restrict__ part, const WgTzGeom& g, int blk, int nblk) {
-    using Sh = WgTzShape<NGA, NCB, NB>;
+    using Sh = WgTzShape<NCB>;
     constexpr int NT = Sh::NT, CS = Sh::CS, CPW = Sh::CPW, NH = Sh::NH, TWG = Sh::TWG, RPX = Sh::RPX, RPG = Sh::RPG, NMF = Sh::NMF;
+    constexpr int NGA = Sh::NGA, NB = Sh::NB;
     constexpr int NSX = Sh::NSX, NSG = Sh::NSG, GBX = Sh::GBX, GBG = Sh::GBG, CHPX = Sh::CHPX, CHPG = Sh::CHPG;
     constexpr int WCPX = Sh::WCX / 2;
     extern __shared__ uint32_t smem[];
@@ -185,13 +185,13 @@ __device__ __forceinline__ void dwconv_wgrad_tz_body(const T* __restrict__ x, co
         v = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x130, 0xf, 0xf, true);   // wave_shl:1: lane i takes lane i + 1
         return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x130, 0xf, 0xf, true);
     };
-    auto commit_g = [&](const uint4 (&bf)[4], int pass, int half) {   // half 0 / 1: one row group of the pass; -1: both
+    auto commit_g = [&](const uint4 (&bf)[4], int pass, int half) {   // half 0 / 1: one row group of the pass
         const uint32_t a0[4] = {bf[0].x, bf[0].y, bf[0].z, bf[0].w}, a1[4] = {bf[1].x, bf[1].y, bf[1].z, bf[1].w};
         const uint32_t a2[4] = {bf[2].x, bf[2].y, bf[2].z, bf[2].w}, a3[4] = {bf[3].x, bf[3].y, bf[3].z, bf[3].w};
         uint32_t a4[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) a4[j] = from_right(a0[j]);   // every lane takes part in the shift
-        if (!gact || (half >= 0 && (grow >> 2) != half)) return;
+        if (!gact || (grow >> 2) != half) return;
         char* dst = gl + gdst + ((2 * pass + (grow >> 2)) % NSG) * GBG;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {   // channels 2 j (low halves) and 2 j + 1 (high halves) of the piece
@@ -247,20 +247,13 @@ __device__ __forceinline__ void dwconv_wgrad_tz_body(const T* __restrict__ x, co
     for (int p = 0; p < P0X; ++p) {
         commit_x(bx[p % 2], p);
         issue_x(bx[p % 2], p + 2);
-        if (p == 0) {
-            if constexpr (NSG == 4) {
-                commit_g(bg[0], 0, -1);
-                issue_g(bg[0], 2);
-            } else {
-                commit_g(bg[0], 0, 0);
-            }
-        }
+        if (p == 0) commit_g(bg[0], 0, 0);
     }
     auto read_a = [&](const char* p) { return *reinterpret_cast<const uint4*>(p); };   // 16-byte aligned
     // Steps in trips of 4, left after the band's last step (a uniform exit between steps: the loads of passes past the
     // band's end, requested on the way, move nothing).  A step first commits what the NEXT step adds to the windows (an
-    // 8-row pass of xw or of gy on alternating steps; with 3 gy slots one row group of gy every step, the pass's
-    // registers being requested again once both of its groups are in LDS), behind the barrier that ends the previous step's reads of the ring slots it
+    // 8-row pass of xw every other step, one row group of gy every step, the pass's registers being requested again once
+    // both of its groups are in LDS), behind the barrier that ends the previous step's reads of the ring slots it
     // overwrites; no condition depends on data, so the loads keep their exact in-flight counts.
     constexpr int UNR = 4;
     for (int s0 = 0; s0 < nsteps; s0 += UNR) {
@@ -273,13 +266,7 @@ __device__ __forceinline__ void dwconv_wgrad_tz_body(const T* __restrict__ x, co
                 commit_x(bx[bi], pass);
                 issue_x(bx[bi], pass + 2);
             }
-            if constexpr (NSG == 4) {
-                if (j % 2 == 1) {       // gy row group t + 1 opens a pass
-                    const int bi = ((j + 1) / 2) % 2, pass = (t + 1) / 2;
-                    commit_g(bg[bi], pass, -1);
-                    issue_g(bg[bi], pass + 2);
-                }
-            } else {                    // gy row group t + 1: half (t + 1) % 2 of pass (t + 1) / 2
+            {                           // gy row group t + 1: half (t + 1) % 2 of pass (t + 1) / 2
                 const int bi = ((j + 1) / 2) % 2, pass = (t + 1) / 2;
                 commit_g(bg[bi], pass, (j + 1) % 2);
                 if ((j + 1) % 2 == 1) issue_g(bg[bi], pass + 2);
@@ -332,30 +319,28 @@ __device__ __forceinline__ void dwconv_wgrad_tz_body(const T* __restrict__ x, co
     }
 }
 
-template <typename T, int NGA, int NCB, int NB>
+template <typename T, int NCB>
 __global__ __launch_bounds__(512, 1) void dwconv_wgrad_tz_k(const T* __restrict__ x, const T* __restrict__ gy,
                                                             float* __restrict__ part, const WgTzGeom g) {
-    dwconv_wgrad_tz_body<T, NGA, NCB, NB>(x, gy, part, g, blockIdx.x, gridDim.x);
+    dwconv_wgrad_tz_body<T, NCB>(x, gy, part, g, blockIdx.x, gridDim.x);
 }
 
 // Two problems of the same filter size in one launch (the two scales of a block): the second problem's nblk1
 // workgroups come first in the grid.  With one workgroup per compute unit and two problems that each fill the chip
 // once, a compute unit runs one band of each back to back, without the drain and the launch between two kernels.
-template <typename T, int NGA, int NCB0, int NCB1, int NB>
+template <typename T, int NCB0, int NCB1>
 __global__ __launch_bounds__(512, 1) void dwconv_wgrad_tz_pair_k(const T* __restrict__ x0, const T* __restrict__ gy0,
                                                                  float* __restrict__ part0, const WgTzGeom g0,
                                                                  const T* __restrict__ x1, const T* __restrict__ gy1,
                                                                  float* __restrict__ part1, const WgTzGeom g1, int nblk1) {
     if ((int)blockIdx.x < nblk1)
-        dwconv_wgrad_tz_body<T, NGA, NCB1, NB>(x1, gy1, part1, g1, blockIdx.x, nblk1);
+        dwconv_wgrad_tz_body<T, NCB1>(x1, gy1, part1, g1, blockIdx.x, nblk1);
     else
-        dwconv_wgrad_tz_body<T, NGA, NCB0, NB>(x0, gy0, part0, g0, blockIdx.x - nblk1, gridDim.x - nblk1);
+        dwconv_wgrad_tz_body<T, NCB0>(x0, gy0, part0, g0, blockIdx.x - nblk1, gridDim.x - nblk1);
 }
 
 // ------------------------------------------------------------------------------------------------
 // Host side
-
-inline int wgrad_tz_nga(int K) { return (4 + 2 * ((K - 1) / 2) + 3) / 4 < 2 ? 2 : (4 + 2 * ((K - 1) / 2) + 3) / 4; }
 
 struct WgTzPlan {
     bool ok = false;
@@ -364,16 +349,16 @@ struct WgTzPlan {
     long long nblocks = 0;
 };
 
-// Covered: 16-bit types (the caller checks), C % 8 == 0, K <= 17, 16-byte aligned tensors.
+// Covered: 16-bit types (the caller checks), C % 8 == 0, K = 16 and 17, 16-byte aligned tensors.
 inline WgTzPlan wgrad_tz_plan(int B, int H, int W, int C, int K, int PH, int PW) {
     WgTzPlan p;
     WgTzGeom& g = p.g;
     g.B = B, g.H = H, g.W = W, g.C = C, g.PH = PH, g.PW = PW, g.K = K;
     g.OH = H + 2 * PH - K + 1, g.OW = W + 2 * PW - K + 1;
-    if (K < 1 || K > 17 || C % 8 != 0 || B < 1 || g.OH < 1 || g.OW < 1) return p;
+    if (K < 16 || K > 17 || C % 8 != 0 || B < 1 || g.OH < 1 || g.OW < 1) return p;
     if ((long long)H * W * C > 0x1fffffffLL || (long long)g.OH * g.OW * C > 0x1fffffffLL) return p;
     p.ncb = g.OW <= 32 ? 5 : 8;
-    const int twg = 8 * p.ncb - 8, ta = wgrad_tz_nga(K);
+    const int twg = 8 * p.ncb - 8, ta = WgTzShape<8>::NGA;
     g.ncolt = cdiv(g.OW, twg), g.nslices = cdiv(C, 16);
     // band height: shortest estimated run, rounds of workgroups over 256 compute units times the rows one moves
     const long long per_band = (long long)B * g.nslices * g.ncolt;
@@ -397,22 +382,22 @@ inline size_t wgrad_tz_workspace(int B, int H, int W, int C, int K, int PH, int 
     return p.ok ? (size_t)B * p.g.nbands * p.g.ncolt * K * K * C * sizeof(float) : 0;
 }
 
-template <typename T, int NGA, int NCB, int NB>
+template <typename T, int NCB>
 static int launch_wgrad_tz(const WgTzPlan& p, const void* x, const void* gy, void* ws, hipStream_t s) {
-    using Sh = WgTzShape<NGA, NCB, NB>;
-    auto kern = dwconv_wgrad_tz_k<T, NGA, NCB, NB>;
+    using Sh = WgTzShape<NCB>;
+    auto kern = dwconv_wgrad_tz_k<T, NCB>;
     static std::once_flag attr_once;
     std::call_once(attr_once, [&] { (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); });
     hipLaunchKernelGGL(kern, dim3((unsigned)p.nblocks), dim3(Sh::NT), Sh::lds_bytes, s, (const T*)x, (const T*)gy, (float*)ws, p.g);
     return check_launch("dwconv_wgrad_tz");
 }
 
-template <typename T, int NGA, int NCB0, int NCB1, int NB>
+template <typename T, int NCB0, int NCB1>
 static int launch_wgrad_tz_pair(const WgTzPlan& p0, const void* x0, const void* gy0, void* ws0, const WgTzPlan& p1,
                                 const void* x1, const void* gy1, void* ws1, hipStream_t s) {
-    using Sh0 = WgTzShape<NGA, NCB0, NB>;
-    using Sh1 = WgTzShape<NGA, NCB1, NB>;
-    auto kern = dwconv_wgrad_tz_pair_k<T, NGA, NCB0, NCB1, NB>;
+    using Sh0 = WgTzShape<NCB0>;
+    using Sh1 = WgTzShape<NCB1>;
+    auto kern = dwconv_wgrad_tz_pair_k<T, NCB0, NCB1>;
     static std::once_flag attr_once;
     std::call_once(attr_once, [&] { (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); });
     if (p0.nblocks + p1.nblocks > 0x7fffffffLL) return -1;

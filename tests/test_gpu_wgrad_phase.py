@@ -39,3 +39,19 @@ def _check(oracle, shape, k, pad, dtype, seed):
                                      ((2, 24, 28, 16), 16)])
 def test_even_filters(oracle, shape, k, dtype):
     _check(oracle, shape, k, (k // 2, k // 2), dtype, 10 * k)
+
+
+# one tile column of 64, two, and columns of 32 in two images (an odd number of them); rows off and on multiples of the passes
+# of 8; channels off the slices of 16; runs of rows that start and end inside an image; images smaller than the filter
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape,k", [((1, 8, 64, 16), 3), ((2, 9, 65, 24), 9), ((3, 57, 61, 8), 13), ((5, 16, 32, 40), 15),
+                                     ((3, 7, 7, 16), 11), ((4, 33, 31, 16), 5), ((2, 15, 112, 24), 7), ((7, 24, 63, 16), 13),
+                                     ((1, 1, 1, 8), 15), ((9, 3, 33, 8), 1), ((40, 28, 28, 32), 13), ((2, 70, 20, 136), 9)])
+def test_tiles_and_runs(oracle, shape, k, dtype):
+    _check(oracle, shape, k, (k // 2, k // 2), dtype, k + shape[1])
+
+
+@pytest.mark.parametrize("shape,k,pad", [((3, 20, 40, 16), 13, (0, 0)), ((2, 18, 34, 24), 9, (8, 8)), ((2, 17, 33, 8), 5, (7, 6)),
+                                         ((3, 16, 70, 16), 15, (14, 3)), ((2, 13, 13, 16), 11, (1, 10))])
+def test_paddings_other_than_same(oracle, shape, k, pad):
+    _check(oracle, shape, k, pad, torch.bfloat16, k + pad[0])
