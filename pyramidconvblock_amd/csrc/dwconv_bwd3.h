@@ -97,108 +97,87 @@ __global__ __launch_bounds__(512, 1) void dwconv_bwd3_k(const Bwd3Args<K> a) {
 
 // Cuts and grid order of the three problems.  A compute unit holds one workgroup of this launch at a time, and a workgroup
 // costs a start-up (first rows, operand set-up) that does not depend on how many rows it takes, so unlike a launch of its
-// own, which has to fill the chip, a problem here is best cut into as few pieces as the other problems leave room for: each
-// candidate (bands per image: 1, 2, 4 or the stand-alone planner's number; runs of dwconv_wgrad_ph.h: eighths of the
-// stand-alone number) is priced by dealing its workgroups, longest problem first (the grid order), to the earliest free of
-// 256 compute units.  Costs in microseconds, fitted to traces of this launch at [32,56,56,64]; beside runs of the phase-major
-// weight gradient a band of the input gradient takes a quarter longer than beside bands (it shares the memory with faster
-// neighbours): without that factor the plan there had 288 workgroups in two rounds, 33.6 us against 31.0 for 244 in one.
-struct Bwd3Cut {
-    int n;             // bands per image, or runs
-    double cost;       // of a workgroup
-    long long count;   // workgroups
-};
+// own, which has to fill the chip, a problem here is best cut into as few pieces as the other problems leave room for: all
+// three in one round of the chip, ending together, where that is possible; else each candidate (runs of several lengths; bands
+// per image for the weight gradients of dwconv_wgrad_tz.h)
+// is priced by dealing its workgroups, longest problem first (the grid order), to the compute units.  us with the summations,
+// against whole-image bands of one image: [32,56,56,64] filter 13 31 -> 27, 15 42 -> 32.5, 9 32 -> 25; [128,56,56,64] 98 -> 73.
 struct Bwd3Plan {
-    int n[3];         // of the input gradient, the full scale's and the half scale's weight gradient
+    int n[3];         // rows of the input gradient's runs; runs or bands of the full scale's and the half scale's weight gradient
     char order[4];    // 'D', 'F', 'H' in grid order
 };
 
-// The time the last of `cuts`' workgroups ends, dealt problem by problem in the order `ord`.
-inline double bwd3_makespan(const Bwd3Cut* const (&cuts)[3], const int (&ord)[3]) {
-    std::map<double, long long> free_at{{0.0, 256}};   // compute units by the time they are free at
-    double end = 0;
-    for (int o : ord) {
-        const Bwd3Cut& c = *cuts[o];
-        std::map<double, long long> busy;
-        for (long long left = c.count; left > 0;) {
-            if (free_at.empty()) std::swap(free_at, busy);
-            const auto first = free_at.begin();
-            if (!busy.empty() && busy.begin()->first < first->first) {   // some units of this problem are done before
-                for (const auto& [t, n] : busy) free_at[t] += n;
-                busy.clear();
-                continue;
-            }
-            const double t = first->first + c.cost;
-            const long long n = std::min(left, first->second);
-            left -= n, busy[t] += n, end = std::max(end, t);
-            if ((first->second -= n) == 0) free_at.erase(first);
-        }
-        for (const auto& [t, n] : busy) free_at[t] += n;
-    }
-    return end;
-}
-
 template <int K, int CS, typename P>
-static Bwd3Plan bwd3_plan(int B, const TzGeom& gd, int npcd, const P& p0, const P& p1) {
+static Bwd3Plan bwd3_plan(int B, const TzGeom& gd, int npcd, const P& p0, const P& p1, int nmean) {
     static std::mutex mu;
     struct Key {
-        int B, H, W, h, w, C;
-        bool operator<(const Key& o) const { return std::tie(B, H, W, h, w, C) < std::tie(o.B, o.H, o.W, o.h, o.w, o.C); }
+        int B, H, W, h, w, C, nmean;
+        bool operator<(const Key& o) const {
+            return std::tie(B, H, W, h, w, C, nmean) < std::tie(o.B, o.H, o.W, o.h, o.w, o.C, o.nmean);
+        }
     };
     static std::map<Key, Bwd3Plan> cache;
-    const Key key{B, gd.OH, gd.OW, p1.g.OH, p1.g.OW, gd.C};
+    const Key key{B, gd.OH, gd.OW, p1.g.OH, p1.g.OW, gd.C, nmean};
     std::lock_guard<std::mutex> lock(mu);
     if (auto it = cache.find(key); it != cache.end()) return it->second;
-    std::vector<Bwd3Cut> cuts[3];
-    const int oh[3] = {gd.OH, p0.g.OH, p1.g.OH};
-    long long per_band[3] = {(long long)cdiv(B, 16 / npcd) * gd.ncolt * gd.nslices, 0, 0};
-    int standalone[3] = {gd.nbands, 1, 1};
-    auto bands = [&](int i, auto cost_of) {   // candidates of a problem that is cut into bands
-        // with many times more whole-image bands than compute units the chip is full whatever the cut: fewest start-ups
-        const bool plenty = per_band[i] > 1024;
-        for (int pick : {1, 2, 4, 0}) {   // 0: the stand-alone planner's number
-            if (plenty && pick != 1) continue;
-            int nb = pick ? pick : standalone[i];
-            // (a weight gradient's partials must fit the workspace sized for the stand-alone plan)
-            if (pick && (nb > std::max(1, oh[i] / 4) || (i > 0 && nb > standalone[i]))) continue;
-            const int br = (cdiv(oh[i], nb) + 3) / 4 * 4;
-            nb = cdiv(oh[i], br);
-            cuts[i].push_back({nb, cost_of(br), per_band[i] * nb});
-        }
-    };
-    bands(0, [&](int br) { return (bwd3_phases(K) ? 1.25 : 1.0) * tz_band_cost<K, CS>(npcd, br); });
-    for (int i = 1; i < 3; ++i) {
-        P p = i == 1 ? p0 : p1;
-        if constexpr (bwd3_phases(K)) {
-            const int most = p.g.nchunks;
-            for (int e = 8; e >= 1; --e) {
-                const int n = std::max(1, most * e / 8);
-                if (!wgrad_ph_cut(p, n) || (!cuts[i].empty() && cuts[i].back().n == p.g.nchunks)) continue;
-                cuts[i].push_back({p.g.nchunks, wgrad_ph_run_cost(K, p.g.passes), p.nblocks});
-            }
-        } else {
-            per_band[i] = (long long)B * p.g.ncolt * p.g.nslices, standalone[i] = p.g.nbands;
-            bands(i, [&](int br) { return 3.0 + 3.0 * (p.ncb == 8 ? 1.0 : 0.9) * ((br + 4) / 4); });
+    constexpr double kStart = 5.0, kStep = 1.15;   // of the input gradient here (its store adds the pooled gradient)
+    const int ni = 16 / npcd;
+    Bwd3Plan best{{8, 1, 1}, "DFH"};
+    bool balanced = false;
+    if constexpr (bwd3_phases(K)) {
+        auto part = [](const P& p) { return LaunchPart{kWgPhStart, wgrad_ph_step(K), p.total, p.g.passes, [p](int s) { return p.per_chunk * cdiv(p.total, s); }}; };
+        const LaunchPart parts[3] = {tz_part(gd, ni, kStart, kStep), part(p0), part(p1)};
+        int steps[3];
+        if ((balanced = launch_balance(parts, nmean, steps))) {
+            TzGeom c = gd;
+            tz_cut_steps(c, ni, steps[0]);
+            best = Bwd3Plan{{c.run, cdiv(p0.total, steps[1]), cdiv(p1.total, steps[2])}, "DFH"};
         }
     }
-    Bwd3Plan best{{cuts[0].back().n, cuts[1].back().n, cuts[2].back().n}, "DFH"};
-    double best_t = 0;
-    for (const Bwd3Cut& d : cuts[0])
-        for (const Bwd3Cut& f : cuts[1])
-            for (const Bwd3Cut& q : cuts[2]) {
-                const Bwd3Cut* const pick[3] = {&d, &f, &q};
-                int ord[3] = {0, 1, 2};
-                // longest first; the input gradient ahead of a weight gradient of similar length (its band is mostly
-                // start-up, memory latency that overlaps best with the other problems' arithmetic: 29.1 against 30.2 us)
-                auto rank = [&](int x) { return pick[x]->cost * (x == 0 ? 1.25 : 1.0); };
-                std::sort(ord, ord + 3, [&](int x, int y) { return rank(x) > rank(y); });
-                const double t = bwd3_makespan(pick, ord);
-                if (best_t == 0 || t < best_t - 1e-9) {
-                    best_t = t;
-                    for (int i = 0; i < 3; ++i) best.n[i] = pick[i]->n, best.order[i] = "DFH"[ord[i]];
-                    best.order[3] = 0;
+    if (!balanced) {
+        std::vector<LaunchCut> cuts[3];
+        tz_cuts(cuts[0], gd, ni, kStart, kStep);
+        for (int i = 1; i < 3; ++i) {
+            P p = i == 1 ? p0 : p1;
+            if constexpr (bwd3_phases(K)) {
+                const int most = p.g.nchunks;
+                for (int e = 8; e >= 1; --e) {
+                    if (!wgrad_ph_cut(p, std::max(1, most * e / 8)) || (!cuts[i].empty() && cuts[i].back().n == p.g.nchunks)) continue;
+                    cuts[i].push_back({p.g.nchunks, wgrad_ph_run_cost(K, p.g.passes), p.nblocks});
+                }
+            } else {
+                const long long per_band = (long long)B * p.g.ncolt * p.g.nslices;
+                for (int pick : {1, 2, 4, 0}) {   // 0: the stand-alone planner's number
+                    // with many times more whole-image bands than compute units the chip is full whatever the cut: fewest start-ups
+                    if (per_band > 1024 && pick != 1) continue;
+                    int nb = pick ? pick : p.g.nbands;
+                    // (the partials must fit the workspace sized for the stand-alone plan)
+                    if (pick && (nb > std::max(1, p.g.OH / 4) || nb > p.g.nbands)) continue;
+                    const int br = (cdiv(p.g.OH, nb) + 3) / 4 * 4;
+                    nb = cdiv(p.g.OH, br);
+                    cuts[i].push_back({nb, 3.0 + 3.0 * (p.ncb == 8 ? 1.0 : 0.9) * ((br + 4) / 4), per_band * nb});
                 }
             }
+        }
+        const LaunchCut mean{0, kMeanCost, nmean};
+        double best_t = 0;
+        for (const LaunchCut& d : cuts[0])
+            for (const LaunchCut& f : cuts[1])
+                for (const LaunchCut& q : cuts[2]) {
+                    const LaunchCut* const pick[4] = {&d, &f, &q, &mean};
+                    int ord[4] = {0, 1, 2, 3};   // (the mean branch's workgroups are the last of the grid)
+                    // longest first; the input gradient ahead of a weight gradient of similar length (its run is mostly
+                    // start-up, memory latency that overlaps best with the other problems' arithmetic: 29.1 against 30.2 us)
+                    auto rank = [&](int x) { return pick[x]->cost * (x == 0 ? 1.25 : 1.0); };
+                    std::sort(ord, ord + 3, [&](int x, int y) { return rank(x) > rank(y); });
+                    const double t = launch_makespan(pick, ord);
+                    if (best_t == 0 || t < best_t - 1e-9) {
+                        best_t = t;
+                        for (int i = 0; i < 3; ++i) best.n[i] = pick[i]->n, best.order[i] = "DFH"[ord[i]];
+                        best.order[3] = 0;
+                    }
+                }
+    }
     if (cache.size() >= kPlanCacheMax) cache.clear();   // callers with ever-changing shapes: a plan is cheap to redo
     cache[key] = best;
     return best;
@@ -227,10 +206,9 @@ static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* 
             if (!p || (reinterpret_cast<uintptr_t>(p) & 15)) return -1;
     if (reinterpret_cast<uintptr_t>(addp) & 15) return -1;
     Bwd3Args<K> a{};
-    long long nd;
     a.npcd = tz_wide_tile(B, W) ? 16 : 8;
-    if (!(a.npcd == 16 ? tz_make_geom<K, 16, CS>(a.gd, nd, true, B, H, W, C, K - 1 - P, K - 1 - P, true, nullptr)
-                       : tz_make_geom<K, 8, CS>(a.gd, nd, true, B, H, W, C, K - 1 - P, K - 1 - P, true, nullptr)))
+    if (!(a.npcd == 16 ? tz_make_geom<K, 16, CS>(a.gd, true, B, H, W, C, K - 1 - P, K - 1 - P, true, nullptr)
+                       : tz_make_geom<K, 8, CS>(a.gd, true, B, H, W, C, K - 1 - P, K - 1 - P, true, nullptr)))
         return -1;
     auto plan_of = [&](int hh, int ww) {
         if constexpr (bwd3_phases(K)) return wgrad_ph_plan(B, hh, ww, C, K, P, P);
@@ -238,17 +216,17 @@ static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* 
     };
     auto p0 = plan_of(H, W), p1 = plan_of(h, w);
     if (!p0.ok || !p1.ok) return -1;
-    Bwd3Plan plan = bwd3_plan<K, CS>(B, a.gd, a.npcd, p0, p1);
-    if (const char* e = tune_env("PDW_BWD3_BANDS")) {   // e.g. "2,2,1,DHF": cuts of D, F, H and the grid order
+    const int nmean = mean ? mean->B * mean_slices(mean->D) : 0;
+    Bwd3Plan plan = bwd3_plan<K, CS>(B, a.gd, a.npcd, p0, p1, nmean);
+    if (const char* e = tune_env("PDW_BWD3_BANDS")) {   // e.g. "64,31,8,DHF": cuts of D, F, H and the grid order
         if (sscanf(e, "%d,%d,%d,%3s", &plan.n[0], &plan.n[1], &plan.n[2], plan.order) != 4) return -1;
     }
     if (tune_env("PDW_BWD3_PRINT"))
         fprintf(stderr, "bwd3 plan B=%d H=%d W=%d C=%d K=%d: cuts D %d F %d H %d order %s\n", B, H, W, C, K, plan.n[0],
                 plan.n[1], plan.n[2], plan.order);
     if (plan.n[0] < 1 || plan.n[1] < 1 || plan.n[2] < 1) return -1;
-    auto rows_of = [](int oh, int nb) { return (cdiv(oh, nb) + 3) / 4 * 4; };
-    a.gd.BR = rows_of(a.gd.OH, plan.n[0]), a.gd.nbands = cdiv(a.gd.OH, a.gd.BR);
-    nd = (long long)cdiv(B, 16 / a.npcd) * a.gd.nbands * a.gd.ncolt * a.gd.nslices;
+    if (!tz_cut(a.gd, 16 / a.npcd, plan.n[0])) return -1;
+    const long long nd = tz_blocks(a.gd);
     int parts[2], per_image[2];   // partials of the weight gradients, pieces of an image
     for (int i = 0; i < 2; ++i) {
         auto& p = i == 0 ? p0 : p1;
@@ -256,17 +234,16 @@ static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* 
             if (!wgrad_ph_cut(p, plan.n[1 + i])) return -1;
             parts[i] = p.parts(), per_image[i] = cdiv(p.g.nchunks, cdiv(B, p.g.ni));
         } else {
-            p.g.BR = rows_of(p.g.OH, plan.n[1 + i]), p.g.nbands = cdiv(p.g.OH, p.g.BR);
+            p.g.BR = (cdiv(p.g.OH, plan.n[1 + i]) + 3) / 4 * 4, p.g.nbands = cdiv(p.g.OH, p.g.BR);
             p.nblocks = (long long)B * p.g.nslices * p.g.ncolt * p.g.nbands;
             parts[i] = B * p.g.nbands * p.g.ncolt, per_image[i] = p.g.nbands;
             a.p[i].ncb = p.ncb;
         }
         a.p[i].g = p.g, a.p[i].n = (int)p.nblocks;
     }
-    const int nmean = mean ? mean->B * mean_slices(mean->D) : 0;
     if (nd + p0.nblocks + p1.nblocks + nmean > 0x7fffffffLL) return -1;
     if (plan_out) {
-        plan_out[0] = a.gd.nbands, plan_out[1] = per_image[0], plan_out[2] = per_image[1];
+        plan_out[0] = cdiv(a.gd.nruns, cdiv(B, 16 / a.npcd)), plan_out[1] = per_image[0], plan_out[2] = per_image[1];
         return 0;
     }
     a.gy = gyf, a.w = w0, a.add = addp, a.dx = dx;

@@ -1,18 +1,18 @@
 // The forward convolutions of both scales of a two-scale block as one launch: y0 = conv(x0, w0) at the full scale and
 // y1 = conv(x1, w1) at the pooled one (x1 being the average pool of x0, made before the launch), neither
-// depending on the other.  A compute unit holds one workgroup of these kernels at a time and a band costs a start-up
-// that does not depend on its height, so a launch of its own cuts a problem into enough bands to fill the chip; here
-// the full scale runs as whole-image bands on half of the compute units while the half scale's workgroups run on the
-// others (14.8 us against 13.9 + 7.9 us and a launch gap at [32,56,56,64], K = 13).  Each scale runs in the tile
+// depending on the other.  A compute unit holds one workgroup of these kernels at a time and a run of rows costs a start-up
+// that does not depend on its length, so a launch of its own cuts a problem into enough runs to fill the chip; here each
+// scale gets the part of the chip that lets both end together (us at [32,56,56,64], filter 13: 14.0 for the launch against 13.9
+// + 7.9 and a gap; [128,56,56,64] 31; with bands of one image instead of runs 14.4 and 36.3).  Each scale runs in the tile
 // (16 or 8 patches side by side) that its width fills better: by template where the full scale's is the wide one and slices
 // are 16 channels (each workgroup starts with one problem's arguments and no choice between the fields of two; at run time,
-// us: filter 13 14.2 for 14.0; [128,56,56,64] filter 13 36.0 for 35.7), at run time elsewhere (with the mean branch, filters
-// 15 and 17: 24.7 and 24.6, by template 24.9 and 24.8).
+// us: filter 13 14.2 for 14.0), at run time elsewhere (with the mean branch, filters 15 and 17: 24.7 and 24.6, by template 24.9
+// and 24.8).
 // The kernel template and its per-filter-size launcher; dwconv_fwd2_k<K>.hip instantiate it, one file per size.
 #pragma once
 #include <algorithm>
+#include <functional>
 #include <map>
-#include <queue>
 #include <tuple>
 #include <type_traits>
 #include <vector>
@@ -76,75 +76,130 @@ __global__ __launch_bounds__(512, 1) void dwconv_fwd2_k(const Fwd2Args a) {
     }
 }
 
-// Workgroups dealt in grid order to the earliest free of 256 compute units: the time the last one ends.
-inline double tz_makespan(int nproblems, const double* cost, const long long* count, const int* ord) {
-    constexpr int kCU = 256;
-    std::priority_queue<double, std::vector<double>, std::greater<double>> free_at;
-    for (int c = 0; c < kCU; ++c) free_at.push(0.0);
+// One way of cutting a problem of a shared launch: pieces (runs of rows, bands per image), time and number of its workgroups.
+struct LaunchCut {
+    int n;
+    double cost;
+    long long count;
+};
+
+// The time the last workgroup ends when the problems' workgroups, in the order `ord`, go to the earliest free of 256 compute
+// units (these kernels' workgroups have one to themselves).
+template <int N>
+inline double launch_makespan(const LaunchCut* const (&cuts)[N], const int (&ord)[N]) {
+    std::map<double, long long> free_at{{0.0, 256}};   // compute units by the time they are free at
     double end = 0;
-    for (int o = 0; o < nproblems; ++o)
-        for (long long n = 0; n < count[ord[o]]; ++n) {
-            const double t = free_at.top() + cost[ord[o]];
-            free_at.pop();
-            free_at.push(t);
-            end = std::max(end, t);
+    long long total = 0;
+    for (int o : ord) {
+        const LaunchCut& c = *cuts[o];
+        total += c.count;
+        for (long long left = c.count; left > 0;) {
+            const auto first = free_at.begin();
+            const double t = first->first + c.cost;
+            const long long n = std::min(left, first->second);
+            left -= n, end = std::max(end, t);
+            if ((first->second -= n) == 0) free_at.erase(first);
+            free_at[t] += n;
         }
-    return end;
+    }
+    return total > 256 ? 1.05 * end : end;   // (several rounds end later than that: see launch_balance)
+}
+
+// A problem that can be cut into runs of at most a number of steps: time of a run = start + step x its steps.
+struct LaunchPart {
+    double start, step;
+    int total, least;                        // steps of the whole problem; fewest of a run
+    std::function<long long(int)> blocks;    // workgroups when cut so
+};
+constexpr double kMeanCost = 5.0;   // us of one of the mean branch's workgroups
+
+// (Measured against plans in several rounds that are estimated equal: backward of [128,56,56,64], filter 13, 72.7 us in 252
+// workgroups, 80.2 in 428.  The mean branch's count too: forward of [8,112,112,48], filter 17, 17 us with units left for its 8
+// workgroups, 21.8 without.)
+// Steps per run with which all problems end together, as early as 256 compute units with one workgroup each allow, the mean
+// branch's nmean short workgroups one after another on the units left over; false: they do not fit in one round.
+template <int N>
+inline bool launch_balance(const LaunchPart (&p)[N], int nmean, int (&steps)[N]) {
+    auto fits = [&](double t, int (&s)[N]) {
+        double units = nmean * kMeanCost / t;
+        for (int i = 0; i < N; ++i) {
+            const double most = (t - p[i].start) / p[i].step;
+            s[i] = most >= p[i].total ? p[i].total : (int)most;
+            if (s[i] < p[i].least) return false;
+            units += (double)p[i].blocks(s[i]);
+        }
+        return units <= 256.0;
+    };
+    double lo = 0, hi = kMeanCost;
+    for (const LaunchPart& q : p) hi = std::max(hi, q.start + q.step * (q.total + 0.5));
+    if (!fits(hi, steps)) return false;
+    for (int i = 0; i < 24; ++i) {
+        const double t = 0.5 * (lo + hi);
+        int s[N];
+        if (fits(t, s)) hi = t;
+        else lo = t;
+    }
+    return fits(hi, steps);
+}
+
+// (a tile of two images starts later)
+inline LaunchPart tz_part(const TzGeom& g, int ni, double start, double step) {
+    return {start + 1.3 * (ni - 1), step, cdiv((long long)(cdiv(g.B, ni) - 1) * g.per + g.OH, 8), 1, [g, ni](int steps) {
+                TzGeom c = g;
+                return tz_cut_steps(c, ni, steps) ? tz_blocks(c) : 1LL << 40;
+            }};
+}
+
+// Candidates of a problem of dwconv_tz.h where that does not apply: n is the rows of the runs.
+inline void tz_cuts(std::vector<LaunchCut>& out, TzGeom g, int ni, double start, double step) {
+    auto add = [&](int steps) {
+        if (steps >= 1 && tz_cut_steps(g, ni, steps)) out.push_back({g.run, start + step * tz_steps(g), tz_blocks(g)});
+    };
+    if (!tz_cut_alone(g, ni)) return;
+    const int alone = tz_steps(g);
+    for (int e : {1, 2, 4, 8}) add(alone * e);
+    add(cdiv(g.OH, 8));
 }
 
 struct Fwd2Plan {
-    int nb[2];    // bands of the full and of the half scale
+    int n[2];     // rows of the runs of the full and of the half scale
     int first;    // problem whose workgroups come first in the grid
 };
 
-// Band costs in microseconds fitted to traces at [32,56,56,64]: a 64-column band of one image 9.6 + 0.045 per row
-// (K = 13), a 32-column band of two images 3.7 + 0.175 per row.
 template <int K, int CS>
-inline double tz_band_cost(int npc, int br) {
-    const double work = TzShape<K, 16, CS>::NM / 8.0;
-    if (npc == 16) return (CS == 16 ? 9.6 : 7.0) + 0.045 * br * work;
-    return (CS == 16 ? 3.7 : 3.0) + 0.175 * br * work;
-}
-
-template <int K, int CS>
-static Fwd2Plan fwd2_plan(int B, const TzGeom& g0, int npc0, const TzGeom& g1, int npc1) {
+static Fwd2Plan fwd2_plan(int B, const TzGeom& g0, int npc0, const TzGeom& g1, int npc1, int nmean) {
     static std::mutex mu;
     struct Key {
-        int B, H, W, h, w, C;
-        bool operator<(const Key& o) const { return std::tie(B, H, W, h, w, C) < std::tie(o.B, o.H, o.W, o.h, o.w, o.C); }
+        int B, H, W, h, w, C, nmean;
+        bool operator<(const Key& o) const {
+            return std::tie(B, H, W, h, w, C, nmean) < std::tie(o.B, o.H, o.W, o.h, o.w, o.C, o.nmean);
+        }
     };
     static std::map<Key, Fwd2Plan> cache;
-    const Key key{B, g0.OH, g0.OW, g1.OH, g1.OW, g0.C};
+    const Key key{B, g0.OH, g0.OW, g1.OH, g1.OW, g0.C, nmean};
     std::lock_guard<std::mutex> lock(mu);
     if (auto it = cache.find(key); it != cache.end()) return it->second;
-    const int oh[2] = {g0.OH, g1.OH}, npc[2] = {npc0, npc1};
-    const long long per_band[2] = {(long long)cdiv(B, 16 / npc0) * g0.ncolt * g0.nslices,
-                                   (long long)cdiv(B, 16 / npc1) * g1.ncolt * g1.nslices};
-    const int standalone[2] = {g0.nbands, g1.nbands};
-    Fwd2Plan best{{standalone[0], standalone[1]}, 0};
-    double best_t = 0;
-    const bool plenty = per_band[0] + per_band[1] > 1536;   // the chip is full whatever the cut: fewest start-ups
-    const int cand[4] = {1, 2, 4, 0};                       // 0: the stand-alone planner's count
-    for (int a = 0; a < 4; ++a)
-        for (int b = 0; b < 4; ++b) {
-            if (plenty && (a | b) != 0) continue;
-            const int pick[2] = {cand[a], cand[b]};
-            int nb[2];
-            double cost[2];
-            long long count[2];
-            bool ok = true;
-            for (int i = 0; i < 2; ++i) {
-                nb[i] = pick[i] ? pick[i] : standalone[i];
-                if (pick[i] && nb[i] > std::max(1, oh[i] / 4)) ok = false;
-                const int br = (cdiv(oh[i], nb[i]) + 3) / 4 * 4;
-                nb[i] = cdiv(oh[i], br);
-                cost[i] = tz_band_cost<K, CS>(npc[i], br), count[i] = per_band[i] * nb[i];
+    Fwd2Plan best{{8, 8}, 0};
+    const int ni[2] = {16 / npc0, 16 / npc1};
+    const LaunchPart parts[2] = {tz_part(g0, ni[0], kTzStart, kTzStep), tz_part(g1, ni[1], kTzStart, kTzStep)};
+    int steps[2];
+    if (launch_balance(parts, nmean, steps)) {
+        TzGeom c0 = g0, c1 = g1;
+        tz_cut_steps(c0, ni[0], steps[0]), tz_cut_steps(c1, ni[1], steps[1]);
+        best = Fwd2Plan{{c0.run, c1.run}, 0};
+    } else {
+        std::vector<LaunchCut> cuts[2];
+        tz_cuts(cuts[0], g0, ni[0], kTzStart, kTzStep), tz_cuts(cuts[1], g1, ni[1], kTzStart, kTzStep);
+        const LaunchCut mean{0, kMeanCost, nmean};
+        double best_t = 0;
+        for (const LaunchCut& f : cuts[0])
+            for (const LaunchCut& q : cuts[1]) {
+                const LaunchCut* const pick[3] = {&f, &q, &mean};
+                const int ord[3] = {f.cost >= q.cost ? 0 : 1, f.cost >= q.cost ? 1 : 0, 2};   // longest first
+                const double t = launch_makespan(pick, ord);
+                if (best_t == 0 || t < best_t - 1e-9) best_t = t, best = Fwd2Plan{{f.n, q.n}, ord[0]};
             }
-            if (!ok) continue;
-            const int ord[2] = {cost[0] >= cost[1] ? 0 : 1, cost[0] >= cost[1] ? 1 : 0};   // longest first
-            const double t = plenty ? 1.0 : tz_makespan(2, cost, count, ord);
-            if (best_t == 0 || t < best_t - 1e-9) best_t = t, best = Fwd2Plan{{nb[0], nb[1]}, ord[0]};
-        }
+    }
     if (cache.size() >= kPlanCacheMax) cache.clear();   // callers with ever-changing shapes: a plan is cheap to redo
     cache[key] = best;
     return best;
@@ -176,22 +231,20 @@ static int launch_fwd2(const void* x0, const void* w0, void* y0, const void* x1,
     Fwd2Problem &f = a.p[0], &q = a.p[1];
     f.npc = tz_wide_tile(B, W) ? 16 : 8, q.npc = tz_wide_tile(B, w) ? 16 : 8;
     auto geom = [&](Fwd2Problem& p, int hh, int ww, const TzGate* gate) {
-        long long n;
-        return p.npc == 16 ? tz_make_geom<K, 16, CS>(p.g, n, false, B, hh, ww, C, P, P, false, gate)
-                           : tz_make_geom<K, 8, CS>(p.g, n, false, B, hh, ww, C, P, P, false, gate);
+        return p.npc == 16 ? tz_make_geom<K, 16, CS>(p.g, false, B, hh, ww, C, P, P, false, gate)
+                           : tz_make_geom<K, 8, CS>(p.g, false, B, hh, ww, C, P, P, false, gate);
     };
     if (!geom(f, H, W, gate0) || !geom(q, h, w, gate1)) return -1;
-    Fwd2Plan plan = fwd2_plan<K, CS>(B, f.g, f.npc, q.g, q.npc);
-    if (const char* e = tune_env("PDW_FWD2_BANDS")) {   // "bands of the full scale, of the half scale, first problem"
-        if (sscanf(e, "%d,%d,%d", &plan.nb[0], &plan.nb[1], &plan.first) != 3) return -1;
+    Fwd2Plan plan = fwd2_plan<K, CS>(B, f.g, f.npc, q.g, q.npc, mean ? mean->B : 0);
+    if (const char* e = tune_env("PDW_FWD2_BANDS")) {   // "rows of the runs of the full scale, of the half scale, first problem"
+        if (sscanf(e, "%d,%d,%d", &plan.n[0], &plan.n[1], &plan.first) != 3) return -1;
     }
     if (tune_env("PDW_FWD2_PRINT"))
-        fprintf(stderr, "fwd2 plan B=%d H=%d W=%d C=%d K=%d: bands %d %d first %d\n", B, H, W, C, K, plan.nb[0], plan.nb[1], plan.first);
+        fprintf(stderr, "fwd2 plan B=%d H=%d W=%d C=%d K=%d: runs %d %d first %d\n", B, H, W, C, K, plan.n[0], plan.n[1], plan.first);
     long long n[2];
     for (int i = 0; i < 2; ++i) {
-        TzGeom& g = a.p[i].g;
-        g.BR = (cdiv(g.OH, plan.nb[i]) + 3) / 4 * 4, g.nbands = cdiv(g.OH, g.BR);
-        n[i] = (long long)cdiv(B, 16 / a.p[i].npc) * g.nbands * g.ncolt * g.nslices;
+        if (!tz_cut(a.p[i].g, 16 / a.p[i].npc, plan.n[i])) return -1;
+        n[i] = tz_blocks(a.p[i].g);
     }
     const int nmean = mean ? mean->B : 0;
     if (n[0] + n[1] + nmean > 0x7fffffffLL) return -1;

@@ -17,14 +17,23 @@
 // operands live in a register ring: a step reads only the 4 new window rows from LDS (ICB operands of 16 bytes per
 // lane) for NM instructions.  That is what makes the kernel a stream: per step and channel 2 LDS reads, 8 MFMAs.
 //
-// A workgroup (8 wavefronts, CS = 8 CPW channels) owns a band of BR output rows x 4 NPC columns of NI images.  Its
-// input window is staged once in LDS, channel-major: xl[image][channel][row][column] as 16-bit values, so that 8
-// consecutive columns of a channel are 16 contiguous bytes.  Threads load 2 x 2 pixels x 8 channels (four 16-byte
-// loads), interleave column pairs with byte permutes and write dwords; the passes of this copy are requested two
-// ahead and committed only as far as the next step needs, so steps start while the lower rows are still on their
-// way and the loads, the MFMAs and the stores of a band overlap.  Results are rounded once, transposed through a
-// small double-buffered LDS tile (pixel-major, one dword of padding per 4 pixels keeps the 4-byte scatter free of
-// bank conflicts) and leave as 16-byte stores, one step behind the MFMAs.
+// A workgroup (8 wavefronts, CS = 8 CPW channels) owns 4 NPC columns of NI images side by side and a run of output rows.  The
+// images of a batch are stacked into one column of rows, `per` rows apart with at least PH rows of zeros between them, and a
+// run starts and ends anywhere (at multiples of 8 rows): as many workgroups as the chip holds at once, whatever the extents,
+// each with one start-up.  The input window is streamed through LDS, channel-major: xl[image][channel][row][column] as 16-bit
+// values, so that 8 consecutive columns of a channel are 16 contiguous bytes.  Threads load 4 pixels of a row x 8 channels (four
+// 16-byte loads), interleave columns with byte permutes and write 8 bytes per channel; the passes of this copy are requested two
+// ahead and committed only as far as the next step needs.  Results are rounded once, transposed through a small
+// double-buffered LDS tile (pixel-major, one dword of padding per 4 pixels keeps the 4-byte scatter free of bank conflicts) and
+// leave as 16-byte stores, one step behind the MFMAs.
+//
+// What bounds it: the instructions that move data.  A step of 8 rows (of 64 columns and 16 channels) is 1024 cycles of products
+// on a SIMD, about 1100 of LDS accesses on the compute unit and, with two wavefronts to a SIMD that wait for one another,
+// whatever vector arithmetic a wavefront has: dependent instructions are 8 cycles apart.  Hence rows are counted with scalars
+// (images a multiple of 8 rows apart, so that a step or pass meets a boundary as a whole), LDS writes are 8 bytes with constant
+// offsets, and the pieces that move data are written between the products.  115 vector instructions a step became 64 and
+// [8,56,56,64], filter 13, in 8 long runs 1.15 us a step 0.97; what does not overlap yet is the LDS round trips either side of
+// the barrier.
 //
 // MODE is a set of bits.
 // 1 (input gradient of a tensor that was also average-pooled 2x2): y += add[i/2, j/2] / 4 in the store.
@@ -41,6 +50,7 @@
 // Zero entries of A multiply real pixels of the window (and the window is wider than K+3 where (K+3) % 8 != 0), so a
 // non-finite input value reaches outputs up to 3 + 8 ICB - (K+3) pixels beyond its K x K footprint as NaN.
 #pragma once
+#include <algorithm>
 #include <mutex>
 
 #include "common.h"
@@ -72,7 +82,9 @@ struct TzShape {
     static constexpr int NI = 16 / NPC;               // images side by side in one instruction
     static constexpr int TW = 4 * NPC;                // output columns of a workgroup
     static constexpr int NH = CS / 8;                 // 8-channel pieces per pixel
-    static constexpr int CPW = CS / 8;                // channels per wavefront
+    static constexpr int CPW = CS / NWV;              // channels per wavefront
+    static constexpr int PIECES = TW * 4 * NI * NH;   // 16-byte pieces of a result tile
+    static constexpr int TPT = NT / PIECES < 2 ? 1 : 2, NG = 2 / TPT;   // tiles stored side by side, and one after the other
     static constexpr int WCOLS = 4 * (NPC - 1) + 8 * ICB;  // window columns the operands touch
     static constexpr int RP = (2 * WCOLS + 7) / 8 * 8;     // bytes per window row of a channel
     static constexpr int OPX = 2 * CS;                     // bytes per pixel of the result tile
@@ -84,23 +96,32 @@ struct TzShape {
     static_assert(K % 2 == 1 && K >= 3 && K <= 17, "odd filters up to 17");
     static_assert(NPC == 16 || NPC == 8, "patches per image row");
     static_assert(CS == 8 || CS == 16, "channels per workgroup");
-    static constexpr int win_rows(int BR) { return BR + 4 * (PER - 1); }  // window rows of a band; BR % 4 == 0
     // The window lives in LDS as a ring of NR row groups (of 4 rows), window row r at ring row r % NRR: a step reads
     // the two row groups it adds to the operand registers while the next step's two are being written, and the
     // first step needs PER + 1 row groups in place before it starts.
     static constexpr int NR = PER + 1 > 4 ? PER + 1 : 4;
     static constexpr int NRR = 4 * NR;
     static constexpr int CHP = NRR * RP % 16 == 8 ? NRR * RP : NRR * RP + 8;  // bytes per channel plane, = 8 mod 16
-    static constexpr size_t lds_bytes = (size_t)NI * CS * CHP + R2B;
+    // behind the planes and the result tiles: where staging lanes without an item write (8 planes apart like an item)
+    static constexpr int SPARE = NI * CS * CHP + R2B;
+    static constexpr size_t lds_bytes = (size_t)SPARE + 7 * CHP + RP + 16;
     static_assert(lds_bytes <= 160 * 1024, "LDS");
 };
+
+// 2^32 / d rounded up (0 for 1): n / d = the high half of n times this while n d < 2^32.  (A division costs a wavefront about
+// 150 cycles, and a workgroup cannot request its first rows before it has made a handful.)
+inline uint32_t tz_inverse(int d) { return d == 1 ? 0u : (uint32_t)(((1ULL << 32) + d - 1) / (uint32_t)d); }
+__device__ __forceinline__ int tz_quotient(int n, uint32_t inverse) { return inverse ? (int)__umulhi((uint32_t)n, inverse) : n; }
 
 struct TzGeom {
     int B, H, W, C;    // input extents
     int OH, OW;        // output extents
     int PH, PW;        // padding
-    int BR;            // output rows of a band (multiple of 4)
-    int nbands, ncolt, nslices;
+    int per;           // rows from one image to the next in the stack of a batch's images (a multiple of 8)
+    int run;           // stacked rows of a workgroup (a multiple of 8)
+    int rpi;           // 0: runs follow one another; else they start anew with every image, rpi of them to one
+    int nruns, ncolt, nslices;
+    uint32_t per_inv, rpi_inv, ncolt_inv, nslices_inv;   // tz_inverse of these
     int flip;          // 1: 180-degree rotated filter (input gradient)
     int AH, AW;        // extents of the half-resolution addend / pooled output
     int YC, ych;       // output pixel stride in channels, first output channel
@@ -133,13 +154,13 @@ __device__ __forceinline__ uint2 tz_gate(uint2 a, uint2 b, float s) {
     return uo.u;
 }
 
-// One workgroup's band: `blk` of the problem's `nblk` workgroups.
+// One workgroup's run: `blk` of the problem's `nblk` workgroups.
 template <typename T, int K, int NPC, int CS, int MODE>
 __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T* __restrict__ w,
                                                const T* __restrict__ add, T* __restrict__ pool, T* __restrict__ y,
                                                const TzGeom& g, int blk, int nblk) {
     using Sh = TzShape<K, NPC, CS>;
-    constexpr int NT = Sh::NT, ICB = Sh::ICB, NKG = Sh::NKG, NM = Sh::NM, PER = Sh::PER, RING = Sh::RING;
+    constexpr int NT = Sh::NT, NG = Sh::NG, ICB = Sh::ICB, NKG = Sh::NKG, NM = Sh::NM, PER = Sh::PER, RING = Sh::RING;
     constexpr int NI = Sh::NI, TW = Sh::TW, NH = Sh::NH, CPW = Sh::CPW, RP = Sh::RP, OPX = Sh::OPX, OROWP = Sh::OROWP;
     constexpr int OLB = Sh::OLB, WTH = Sh::WTH, WTW = Sh::WTW, NR = Sh::NR, NRR = Sh::NRR, CHP = Sh::CHP;
     constexpr bool ADD = (MODE & 1) != 0, POOL = (MODE & 2) != 0, GATE = (MODE & 4) != 0;
@@ -154,16 +175,28 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
 
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     int bid = xcd_remap(blk, nblk);
-    const int sl = bid % g.nslices;
-    bid /= g.nslices;
-    const int ct = bid % g.ncolt;
-    bid /= g.ncolt;
-    const int band = bid % g.nbands, ig = bid / g.nbands;
-    const int c0 = sl * CS, ocol0 = ct * TW, orow0 = band * g.BR, b0 = ig * NI;
-    const int rows_valid = min(g.BR, g.OH - orow0), cols_valid = min(TW, g.OW - ocol0);
+    int rest = tz_quotient(bid, g.nslices_inv);
+    const int sl = bid - rest * g.nslices;
+    bid = tz_quotient(rest, g.ncolt_inv);
+    const int ct = rest - bid * g.ncolt;
+    const int c0 = sl * CS, ocol0 = ct * TW;
+    auto images_in = [&](int v) { return tz_quotient(v, g.per_inv); };   // (v >= 0)
+    // the run's output rows: g.run of the stack, without the rows between images at its ends
+    int b0, orow0, rows_valid;
+    {
+        const int image = g.rpi ? tz_quotient(bid, g.rpi_inv) : 0;
+        const int first = g.rpi ? image * g.per + (bid - image * g.rpi) * g.run : bid * g.run;
+        b0 = g.rpi ? image : images_in(first), orow0 = first - b0 * g.per;
+        int end = orow0 + min(g.run, ((g.B + NI - 1) / NI - 1) * g.per + g.OH - first);   // (from image b0's first row on)
+        if (orow0 >= g.OH) ++b0, orow0 = 0, end -= g.per;
+        if (end <= 0) return;     // (uniform) all of them between two images
+        const int over = images_in(end - 1) * g.per;
+        rows_valid = min(end, over + g.OH) - orow0;
+        b0 *= NI;
+    }
+    const int cols_valid = min(TW, g.OW - ocol0);
     const int nsteps = (rows_valid + 3) >> 2;
     const int NROWS = 4 * (nsteps + PER - 1);              // window rows the steps read
-    const int WCP = (4 * ((cols_valid + 3) / 4 - 1) + 8 * ICB) / 2;  // column pairs the used patches read
     const long long img_in = (long long)g.H * g.W * g.C, img_out = (long long)g.OH * g.OW * g.YC;
     // first channel of the slice's 8-channel piece h
     auto chof = [&](int h) { return G8 ? 4 * sl : GATE ? 8 * sl + h * (g.C >> 1) : c0 + 8 * h; };
@@ -186,24 +219,27 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
 
     // ---- staging.  The window arrives in passes, requested two ahead into two register buffers.  Passes 0 and 1
     // are halves of the PER + 1 row groups (of 4 rows) the first step reads, every later pass the two row groups the
-    // next step adds, so step f is preceded by the commit of pass f + 1.  A thread's item is (row pair of the pass,
-    // image, column pair cp, 8-channel piece h), h fastest, the same in every pass.
-    constexpr int RP01 = PER + 1;                                // row pairs of pass 0 and of pass 1
-    constexpr int RPMAX = RP01 > 4 ? RP01 : 4;
-    constexpr int NLD = (RPMAX * NI * (Sh::WCOLS / 2) * NH + NT - 1) / NT;  // items per thread and pass
+    // next step adds, so step f is preceded by the commit of pass f + 1.  A thread's item is (IR rows of the pass,
+    // image, IC columns cq, 8-channel piece h), h fastest, the same in every pass.
+    constexpr int IR = POOL ? 2 : 1, IC = POOL ? 2 : 4;          // (the pool's windows are 2 x 2)
+    constexpr int RW01 = 2 * PER + 2;                            // rows of pass 0 and of pass 1
+    constexpr int RWMAX = RW01 > 8 ? RW01 : 8;
+    constexpr int WCQ = Sh::WCOLS / IC;
+    constexpr int NLD = (RWMAX / IR * NI * (Sh::WCOLS / IC) * NH + NT - 1) / NT;  // items per thread and pass
     constexpr int UNRF = PER % 4 == 0 ? PER / 2 : (PER % 2 == 0 ? PER : 2 * PER);  // steps per trip: even, PER | 2 UNRF
-    auto first_rowpair = [&](int pass) { return pass < 2 ? pass * RP01 : 2 * RP01 + 4 * (pass - 2); };
-    auto rowpair_count = [&](int pass) { return pass < 2 ? RP01 : 4; };
+    auto first_row = [&](int pass) { return pass < 2 ? pass * RW01 : 2 * RW01 + 8 * (pass - 2); };
     // Loads go through a buffer descriptor over the workgroup's images: an offset past its end (an image beyond the
     // batch, or one of the markers for a row / column / channel outside the tensor) reads as zero and moves no
-    // data, which is the zero padding.  NI * H * W * C < 2^29 elements (guarded on the host), so valid byte
-    // offsets stay below 2^30 and any sum with a marker stays past the end.
+    // data, which is the zero padding.  The images of a run hold less than 2^29 elements (guarded on the host), so valid
+    // byte offsets stay below 2^30 and any sum with a marker stays past the end.
     constexpr uint32_t kNoCol = 0x40000000u, kNoRow = 0x80000000u;
+    // images the run reaches (all of its offsets are from b0 on)
+    const int images = min((images_in(orow0 + rows_valid + K + 24) + 1) * NI, g.B - b0);
     const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<T*>(x + (long long)b0 * img_in), (short)0, (int)(min(NI, g.B - b0) * img_in * 2), 0x00020000);
-    auto xload_from = [&](const __amdgpu_buffer_rsrc_t& r, uint32_t off) {
+        const_cast<T*>(x + (long long)b0 * img_in), (short)0, (int)(images * img_in * 2), 0x00020000);
+    auto xload_from = [&](const __amdgpu_buffer_rsrc_t& r, uint32_t off, uint32_t soff = 0) {
         typedef unsigned v4u __attribute__((ext_vector_type(4)));
-        const v4u v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0);
+        const v4u v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, (int)soff, 0);
         return make_uint4(v.x, v.y, v.z, v.w);
     };
     auto xload = [&](uint32_t off) {
@@ -216,71 +252,125 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
             return xload_from(xrsrc, off);
         }
     };
-    uint32_t icol[NLD][2];  // byte offsets of the item's two columns (image and channel piece included), or kNoCol
-    int irpw[NLD];          // row pair within a pass
-    int idst[NLD];          // LDS byte offset of the item's plane and column pair
+    uint32_t icol[NLD][IC];  // byte offsets of the item's columns (image and channel piece included), or kNoCol
+    int irw[NLD];           // (first) row within a pass
+    int idst[NLD];          // LDS byte offset of the item's plane and columns
 #pragma unroll
     for (int l = 0; l < NLD; ++l) {
         const int idx = tid + l * NT;
-        const int h = idx % NH, cp = (idx / NH) % WCP, img = (idx / NH / WCP) % NI, rpw = idx / NH / WCP / NI;
-        irpw[l] = rpw;
-        const int ic = ocol0 - g.PW + 2 * cp;
-        const bool any = (G8 || chof(h) < g.C) && rpw < RPMAX;
+        const int h = idx % NH, cq = (idx / NH) % WCQ, img = (idx / NH / WCQ) % NI, rw = idx / NH / WCQ / NI * IR;
+        irw[l] = rw;
+        const int ic = ocol0 - g.PW + IC * cq;
+        const bool any = (G8 || chof(h) < g.C) && rw < RWMAX;
         const uint32_t ioff = (uint32_t)img * (uint32_t)img_in + (uint32_t)chof(h);
-        icol[l][0] = any && ic >= 0 && ic < g.W ? (ioff + (uint32_t)(ic * g.C)) * 2u : kNoCol;
-        icol[l][1] = any && ic + 1 >= 0 && ic + 1 < g.W ? (ioff + (uint32_t)((ic + 1) * g.C)) * 2u : kNoCol;
-        idst[l] = (img * CS + 8 * h) * CHP + 4 * cp;
+#pragma unroll
+        for (int k = 0; k < IC; ++k) icol[l][k] = any && ic + k >= 0 && ic + k < g.W ? (ioff + (uint32_t)((ic + k) * g.C)) * 2u : kNoCol;
+        idst[l] = (img * CS + 8 * h) * CHP + 2 * IC * cq;
     }
     // the 2x2 average pool of x (MODE 2) leaves through a buffer descriptor as well: a store past its end is dropped
     __amdgpu_buffer_rsrc_t prsrc = xrsrc;
     if constexpr (POOL)
         prsrc = __builtin_amdgcn_make_buffer_rsrc(pool + (long long)b0 * g.AH * g.AW * g.C, (short)0,
-                                                  (int)((long long)min(NI, g.B - b0) * g.AH * g.AW * g.C * 2), 0x00020000);
-    uint4 buf[2][NLD][4];
-    auto issue = [&](uint4 (&bf)[NLD][4], int pass) {  // rows beyond the pass or the window read nothing
-        const int wr0 = 2 * first_rowpair(pass), nrp = rowpair_count(pass);
+                                                  (int)((long long)images * g.AH * g.AW * g.C * 2), 0x00020000);
+    // Window row r of the run is stacked row orow0 - PH + r, counted from b0's first: where it lies (image group, row in it).
+    // Rows between images and above the first are zeros; per >= H + PH keeps the windows of neighbouring images apart.
+    const uint32_t row_in = (uint32_t)(g.W * g.C) * 2u, group_in = (uint32_t)img_in * (uint32_t)NI * 2u;
+    auto locate = [&](int v, int& group, int& row) {
+        group = images_in(max(v, 0)), row = v - group * g.per;   // (v < 0: row < 0)
+    };
+    // From pass 2 on a pass's 8 rows lie in two aligned groups of 8 stacked rows; images are a multiple of 8 rows apart, so a
+    // group's place is uniform: row in the image and byte offset of groups a and b = a + 1, moved on by one each pass.
+    const int row_w = orow0 - g.PH + 2 * RW01;   // (first row of pass 2)
+    int ra, rb;
+    uint32_t oa, ob;
+    auto next_group = [&](int r, uint32_t o, int& rn, uint32_t& on) {
+        const bool wrap = r + 8 >= g.per;
+        rn = wrap ? 0 : r + 8, on = wrap ? o - (uint32_t)r * row_in + group_in : o + 8u * row_in;
+    };
+    {
+        const int first = (row_w >> 3) * 8;   // (negative with paddings beyond the filter: rows above the image)
+        const int group = images_in(max(first, 0));
+        ra = first - group * g.per, oa = (uint32_t)group * group_in + (uint32_t)ra * row_in;
+        next_group(ra, oa, rb, ob);
+    }
+    int lrow[NLD];          // the item's (first) row within its group
+    bool inb[NLD];          // ... which is b
 #pragma unroll
-        for (int l = 0; l < NLD; ++l) {
-            const int wr = wr0 + 2 * irpw[l];  // window row
-            const int ir = orow0 - g.PH + wr;
-            const bool ok = irpw[l] < nrp && wr < NROWS;
-            const uint32_t r0 = ok && ir >= 0 && ir < g.H ? (uint32_t)(ir * g.W * g.C) * 2u : kNoRow;
-            const uint32_t r1 = ok && ir + 1 >= 0 && ir + 1 < g.H ? (uint32_t)((ir + 1) * g.W * g.C) * 2u : kNoRow;
-            bf[l][0] = xload(r0 + icol[l][0]);
-            bf[l][1] = xload(r0 + icol[l][1]);
-            bf[l][2] = xload(r1 + icol[l][0]);
-            bf[l][3] = xload(r1 + icol[l][1]);
+    for (int l = 0; l < NLD; ++l) {
+        const int r = (row_w & 7) + irw[l];
+        inb[l] = r >= 8, lrow[l] = irw[l] < 8 ? r & 7 : 0x40000000;   // (no item in these passes)
+    }
+    uint4 buf[2][NLD][IC * IR];
+    auto load_item = [&](uint4 (&bf)[IC * IR], int l, bool ok, uint32_t off, bool ok1) {
+#pragma unroll
+        for (int r = 0; r < IR; ++r) {
+            const uint32_t r0 = (r == 0 ? ok : ok1) ? off + (uint32_t)r * row_in : kNoRow;
+#pragma unroll
+            for (int k = 0; k < IC; ++k) bf[IC * r + k] = xload(r0 + icol[l][k]);
         }
     };
-    auto commit = [&](const uint4 (&bf)[NLD][4], int pass) {
-        const int wr0 = 2 * first_rowpair(pass), nrp = rowpair_count(pass);
+    auto issue_first = [&](uint4 (&bf)[NLD][IC * IR], int pass) {   // passes 0 and 1
 #pragma unroll
         for (int l = 0; l < NLD; ++l) {
-            const int wr = wr0 + 2 * irpw[l];
-            if (irpw[l] < nrp && wr < NROWS) {
-                const uint32_t a0[4] = {bf[l][0].x, bf[l][0].y, bf[l][0].z, bf[l][0].w};
-                const uint32_t a1[4] = {bf[l][1].x, bf[l][1].y, bf[l][1].z, bf[l][1].w};
-                const uint32_t a2[4] = {bf[l][2].x, bf[l][2].y, bf[l][2].z, bf[l][2].w};
-                const uint32_t a3[4] = {bf[l][3].x, bf[l][3].y, bf[l][3].z, bf[l][3].w};
-                int rr = wr0 % NRR + 2 * irpw[l];   // ring row of the item's first row (a pair never wraps: both even)
-                rr -= rr >= NRR ? NRR : 0;
-                char* dst = xl + idst[l] + rr * RP;
+            int group, row;
+            locate(orow0 - g.PH + pass * RW01 + irw[l], group, row);
+            const bool ok = irw[l] < RW01;
+            load_item(bf[l], l, ok && row >= 0 && row < g.H, (uint32_t)group * group_in + (uint32_t)row * row_in,
+                      ok && row + 1 >= 0 && row + 1 < g.H);
+        }
+    };
+    auto issue = [&](uint4 (&bf)[NLD][IC * IR], int pass) {   // passes from 2 on, in order; those past the window read nothing
+        const bool any = first_row(pass) < NROWS;
+        const int la = any && ra >= 0 ? g.H - ra : 0, lb = any && rb >= 0 ? g.H - rb : 0;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    // column pair of channels 2j and 2j+1, the item's two rows
-                    *reinterpret_cast<uint32_t*>(dst + (2 * j) * CHP) = __builtin_amdgcn_perm(a1[j], a0[j], 0x05040100u);
-                    *reinterpret_cast<uint32_t*>(dst + (2 * j + 1) * CHP) = __builtin_amdgcn_perm(a1[j], a0[j], 0x07060302u);
-                    *reinterpret_cast<uint32_t*>(dst + (2 * j) * CHP + RP) = __builtin_amdgcn_perm(a3[j], a2[j], 0x05040100u);
-                    *reinterpret_cast<uint32_t*>(dst + (2 * j + 1) * CHP + RP) = __builtin_amdgcn_perm(a3[j], a2[j], 0x07060302u);
+        for (int l = 0; l < NLD; ++l) {
+            const int lim = inb[l] ? lb : la;
+            load_item(bf[l], l, lrow[l] < lim, (inb[l] ? ob : oa) + (uint32_t)(lrow[l] & 7) * row_in, lrow[l] + 1 < lim);
+        }
+        ra = rb, oa = ob;
+        next_group(rb, ob, rb, ob);
+    };
+    // A pass into the window: the columns of channels 2j and 2j + 1 of the items' rows at ring byte offset cring[l].  No
+    // branch, so that the products around it can be interleaved: lanes without an item write behind the planes.
+    int cring[NLD];
+    auto commit_part = [&](const uint4 (&bf)[NLD][IC * IR], int j) {
+#pragma unroll
+        for (int l = 0; l < NLD; ++l)
+#pragma unroll
+            for (int r = 0; r < IR; ++r) {
+                auto d = [&](int k) { const uint4& u = bf[l][IC * r + k]; return j == 0 ? u.x : j == 1 ? u.y : j == 2 ? u.z : u.w; };
+                char* const dst = xl + cring[l] + r * RP;   // (a pair of rows never wraps: both even)
+#pragma unroll
+                for (int odd = 0; odd < 2; ++odd) {
+                    const uint32_t sel = odd ? 0x07060302u : 0x05040100u;
+                    const uint32_t lo = __builtin_amdgcn_perm(d(1), d(0), sel);
+                    if constexpr (IC == 4)
+                        *reinterpret_cast<uint2*>(dst + (2 * j + odd) * CHP) = make_uint2(lo, __builtin_amdgcn_perm(d(3), d(2), sel));
+                    else
+                        *reinterpret_cast<uint32_t*>(dst + (2 * j + odd) * CHP) = lo;
                 }
             }
-            if constexpr (POOL) {
-                // the thread holds one window of the 2x2 pool (H, W, PH, PW even): the band that owns these rows writes it
+    };
+    auto commit_next = [&]() {   // 8 rows on (passes from 2 on)
+#pragma unroll
+        for (int l = 0; l < NLD; ++l) {
+            cring[l] += irw[l] < 8 ? 8 * RP : 0;
+            cring[l] -= irw[l] < 8 && cring[l] - idst[l] >= NRR * RP ? NRR * RP : 0;
+        }
+    };
+    auto write_pool = [&](const uint4 (&bf)[NLD][IC * IR], int pass) {
+        if constexpr (POOL) {
+            const int wr0 = first_row(pass), nrw = pass < 2 ? RW01 : 8;
+#pragma unroll
+            for (int l = 0; l < NLD; ++l) {
+                // the thread holds one window of the 2x2 pool (H, W, PH, PW even): the run that owns these rows writes it
                 const int idx = tid + l * NT;
-                const int h = idx % NH, cp = (idx / NH) % WCP, img = (idx / NH / WCP) % NI;
-                const int ir = orow0 - g.PH + wr, ic = ocol0 - g.PW + 2 * cp;
-                const bool mine = irpw[l] < nrp && chof(h) < g.C && ir >= orow0 && ir < orow0 + rows_valid && ic >= ocol0 &&
-                                  ic < ocol0 + cols_valid;
+                const int h = idx % NH, cq = (idx / NH) % WCQ, img = (idx / NH / WCQ) % NI;
+                const int v = orow0 - g.PH + wr0 + irw[l], ic = ocol0 - g.PW + 2 * cq;
+                int group, ir;
+                locate(v, group, ir);
+                const bool mine = irw[l] < nrw && chof(h) < g.C && v >= orow0 && v < orow0 + rows_valid && ir < g.H &&
+                                  ic >= ocol0 && ic < ocol0 + cols_valid;
                 union U {
                     uint4 u;
                     T t[8];
@@ -289,14 +379,21 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
                     o.t[e] = from_f32<T>((((to_f32(p0.t[e]) + to_f32(p1.t[e])) + to_f32(p2.t[e])) + to_f32(p3.t[e])) * 0.25f);
-                const uint32_t off = mine ? (uint32_t)(((img * g.AH + (ir >> 1)) * g.AW + (ic >> 1)) * g.C + chof(h)) * 2u : kNoRow;
+                const uint32_t off = mine ? (uint32_t)((((group * NI + img) * g.AH + (ir >> 1)) * g.AW + (ic >> 1)) * g.C + chof(h)) * 2u : kNoRow;
                 typedef unsigned v4u __attribute__((ext_vector_type(4)));
                 __builtin_amdgcn_raw_buffer_store_b128(v4u{o.u.x, o.u.y, o.u.z, o.u.w}, prsrc, (int)off, 0, 0);
             }
         }
     };
-    issue(buf[0], 0);
-    issue(buf[1], 1);
+    auto commit_first = [&](const uint4 (&bf)[NLD][IC * IR], int pass) {   // passes 0 and 1
+#pragma unroll
+        for (int l = 0; l < NLD; ++l) cring[l] = irw[l] < RW01 ? idst[l] + (pass * RW01 + irw[l]) % NRR * RP : Sh::SPARE;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) commit_part(bf, j);
+        write_pool(bf, pass);
+    };
+    issue_first(buf[0], 0);
+    issue_first(buf[1], 1);
 
     // LDS accesses of this wavefront complete, then the workgroup barrier; global loads and stores stay in flight
     auto lds_barrier = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
@@ -345,54 +442,71 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
     // store phase: one 16-byte piece (image, row, column, h) of each 4-row result tile per thread, through buffer
     // descriptors (an offset past the end: nothing stored / zero loaded), so that no vector memory instruction of the
     // kernel sits behind a branch and the in-flight counts the staging waits rely on stay exact
-    const int sh = tid % NH, scol = (tid / NH) % TW, srow = (tid / NH / TW) % 4, simg = tid / NH / TW / 4;
-    const bool s_ok = simg < NI && scol < cols_valid && (GATE || c0 + 8 * sh < g.C);
-    const char* const olr = r2 + (min(simg, NI - 1) * 4 + srow) * OROWP + scol * OPX + (scol >> 2) * 4 + 16 * sh;
+    const int sh = tid % NH, scol = (tid / NH) % TW, srow = (tid / NH / TW) % 4, simg = tid / NH / TW / 4 % NI;
+    const int stile = tid / Sh::PIECES;   // (with TPT = 2: the tile of the step's two that the thread stores)
+    auto tile_of = [&](int n) { return Sh::TPT == 2 ? stile : n; };
+    const bool s_ok = stile < Sh::TPT && scol < cols_valid && (GATE || c0 + 8 * sh < g.C);
+    const char* const olr = r2 + (simg * 4 + srow) * OROWP + scol * OPX + (scol >> 2) * 4 + 16 * sh;
     const __amdgpu_buffer_rsrc_t yrsrc = __builtin_amdgcn_make_buffer_rsrc(
-        y + (long long)b0 * img_out, (short)0, (int)(min(NI, g.B - b0) * img_out * 2), 0x00020000);
+        y + (long long)b0 * img_out, (short)0, (int)(images * img_out * 2), 0x00020000);
     const uint32_t ycol = (uint32_t)simg * (uint32_t)img_out +
                           (uint32_t)((ocol0 + scol) * g.YC + g.ych + (G8 ? 4 * sl : GATE ? 8 * sl + 4 * sh : c0 + 8 * sh));
     __amdgpu_buffer_rsrc_t arsrc = xrsrc;
     if constexpr (ADD)
         arsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(add + (long long)b0 * g.AH * g.AW * g.C), (short)0,
-                                                  (int)((long long)min(NI, g.B - b0) * g.AH * g.AW * g.C * 2), 0x00020000);
-    uint4 addv[2] = {make_uint4(0u, 0u, 0u, 0u), make_uint4(0u, 0u, 0u, 0u)};
-    auto add_fetch = [&](int f) {   // the addends of step f's two tiles
-        if constexpr (ADD) {
+                                                  (int)((long long)images * g.AH * g.AW * g.C * 2), 0x00020000);
+    uint4 addv[NG];
+    // a step's 8 rows lie in one image (group): its first row there, and the byte offsets of that row in y and the addend
+    int orow = orow0, rleft = rows_valid;   // rleft: rows of the run from this step on
+    const uint32_t row_out = (uint32_t)(g.OW * g.YC) * 2u, group_out = (uint32_t)img_out * (uint32_t)NI * 2u;
+    const uint32_t row_add = (uint32_t)(g.AW * g.C) * 2u, group_add = (uint32_t)(NI * g.AH) * row_add;
+    uint32_t ooff = (uint32_t)orow * row_out, aoff = (uint32_t)(orow >> 1) * row_add, stored = 0;   // stored: ooff of the step before
+    uint32_t ylane[NG], alane[NG], yoff[NG];   // the thread's piece from there (rows srow or srow + 4); yoff: or the marker
 #pragma unroll
-            for (int gi = 0; gi < 2; ++gi) {
-                const int row = 4 * (2 * f + gi) + srow;
-                const bool ok = s_ok && row < rows_valid;
-                const uint32_t off = ok ? (uint32_t)(((simg * g.AH + ((orow0 + row) >> 1)) * g.AW + ((ocol0 + scol) >> 1)) * g.C + c0 + 8 * sh) * 2u : kNoRow;
-                addv[gi] = xload_from(arsrc, off);
-            }
+    for (int n = 0; n < NG; ++n) {
+        const int r = 4 * tile_of(n) + srow;
+        ylane[n] = s_ok ? ycol * 2u + (uint32_t)r * row_out : kNoRow;
+        alane[n] = s_ok ? (uint32_t)(((simg * g.AH + (r >> 1)) * g.AW + ((ocol0 + scol) >> 1)) * g.C + c0 + 8 * sh) * 2u : kNoRow;
+        yoff[n] = kNoRow, addv[n] = make_uint4(0u, 0u, 0u, 0u);
+    }
+    auto place = [&]() {   // the next step: the offsets its tiles are stored at, and the addends
+        const int lim = min(g.OH - orow, rleft);
+#pragma unroll
+        for (int n = 0; n < NG; ++n) {
+            const bool ok = 4 * tile_of(n) + srow < lim;
+            yoff[n] = ok ? ylane[n] : kNoRow;
+            if constexpr (ADD) addv[n] = xload_from(arsrc, ok ? alane[n] : kNoRow, aoff);
+        }
+        stored = ooff;
+        rleft -= 8, orow += 8;
+        const bool wrap = orow >= g.per;
+        ooff += wrap ? group_out - (uint32_t)(orow - 8) * row_out : 8u * row_out;
+        aoff += wrap ? group_add - (uint32_t)((orow - 8) >> 1) * row_add : 4u * row_add;
+        orow = wrap ? 0 : orow;
+    };
+    auto tile_read = [&](int f, int n) {
+        const char* src = olr + (2 * (f & 1) + min(tile_of(n), 1)) * OLB;   // (f: or anything of its parity)
+        if constexpr (GATE) {
+            // the thread gates 4 channel pairs of the pixel: values 4 sh .. 4 sh + 3 of both 8-channel pieces, or
+            // the two halves of an 8-channel slice's one piece
+            const char* sg = G8 ? src : src - 8 * sh;   // (src points 16 sh into the pixel)
+            constexpr int PB = G8 ? 8 : 16;             // bytes between a pair's two values
+            return make_uint4(*reinterpret_cast<const uint32_t*>(sg), *reinterpret_cast<const uint32_t*>(sg + 4),
+                              *reinterpret_cast<const uint32_t*>(sg + PB), *reinterpret_cast<const uint32_t*>(sg + PB + 4));
+        } else {
+            return make_uint4(*reinterpret_cast<const uint32_t*>(src), *reinterpret_cast<const uint32_t*>(src + 4),
+                              *reinterpret_cast<const uint32_t*>(src + 8), *reinterpret_cast<const uint32_t*>(src + 12));
         }
     };
-    auto store = [&](int f) {   // f = -1: nothing
-#pragma unroll
-        for (int gi = 0; gi < 2; ++gi) {
-            const char* src = olr + (2 * (f & 1) + gi) * OLB;
-            uint4 v;
-            v.x = *reinterpret_cast<const uint32_t*>(src), v.y = *reinterpret_cast<const uint32_t*>(src + 4);
-            v.z = *reinterpret_cast<const uint32_t*>(src + 8), v.w = *reinterpret_cast<const uint32_t*>(src + 12);
-            if constexpr (ADD) v = tz_add_quarter<T>(v, addv[gi]);
-            const int row = 4 * (2 * f + gi) + srow;
-            const bool ok = s_ok && f >= 0 && row < rows_valid;
-            const uint32_t off = ok ? (ycol + (uint32_t)((orow0 + row) * g.OW * g.YC)) * 2u : kNoRow;
-            if constexpr (GATE) {
-                // the thread gates 4 channel pairs of the pixel: values 4 sh .. 4 sh + 3 of both 8-channel pieces, or
-                // the two halves of an 8-channel slice's one piece
-                const char* sg = G8 ? src : src - 8 * sh;   // (src points 16 sh into the pixel)
-                constexpr int PB = G8 ? 8 : 16;             // bytes between a pair's two values
-                const uint2 a = make_uint2(*reinterpret_cast<const uint32_t*>(sg), *reinterpret_cast<const uint32_t*>(sg + 4));
-                const uint2 b = make_uint2(*reinterpret_cast<const uint32_t*>(sg + PB), *reinterpret_cast<const uint32_t*>(sg + PB + 4));
-                const uint2 o = tz_gate<T>(a, b, g.gs);
-                typedef unsigned v2u __attribute__((ext_vector_type(2)));
-                __builtin_amdgcn_raw_buffer_store_b64(v2u{o.x, o.y}, yrsrc, (int)off, 0, 0);
-            } else {
-                typedef unsigned v4u __attribute__((ext_vector_type(4)));
-                __builtin_amdgcn_raw_buffer_store_b128(v4u{v.x, v.y, v.z, v.w}, yrsrc, (int)off, 0, 0);
-            }
+    auto tile_store = [&](uint4 v, int n) {   // where place() put it
+        if constexpr (ADD) v = tz_add_quarter<T>(v, addv[n]);
+        if constexpr (GATE) {
+            const uint2 o = tz_gate<T>(make_uint2(v.x, v.y), make_uint2(v.z, v.w), g.gs);
+            typedef unsigned v2u __attribute__((ext_vector_type(2)));
+            __builtin_amdgcn_raw_buffer_store_b64(v2u{o.x, o.y}, yrsrc, (int)yoff[n], (int)stored, 0);
+        } else {
+            typedef unsigned v4u __attribute__((ext_vector_type(4)));
+            __builtin_amdgcn_raw_buffer_store_b128(v4u{v.x, v.y, v.z, v.w}, yrsrc, (int)yoff[n], (int)stored, 0);
         }
     };
 
@@ -408,10 +522,12 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
             for (int i = 0; i < ICB; ++i) ring[q][slotgroup * ICB + i] = read16(xb[q][i] + byteoff);
     };
     // the passes the first step reads, then the ring's first PER - 1 row groups
-    commit(buf[0], 0);
+    commit_first(buf[0], 0);
     issue(buf[0], 2);
-    commit(buf[1], 1);
+    commit_first(buf[1], 1);
     issue(buf[1], 3);
+#pragma unroll
+    for (int l = 0; l < NLD; ++l) cring[l] = irw[l] < 8 ? idst[l] + (2 * RW01 + irw[l]) % NRR * RP : Sh::SPARE;
     lds_barrier();
     // ---- this wavefront's A operands: lane = (m = 4 di + dj, k group kg); operand t covers k groups 4t .. 4t+3
     uint4 A[CPW][NM];
@@ -434,50 +550,73 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
 
 #pragma unroll
     for (int j = 0; j < PER - 1; ++j) load_group(j, 4 * j * RP);
-    // A step is two row groups (8 output rows).  Trips of UNRF steps (the ring's period in steps), left after the
-    // band's last step by a uniform exit between steps.  Besides its products a step
-    // stores the previous step's tiles and commits the pass the NEXT step needs; the wavefronts 0-3 do the products
-    // first and the others last, so that of the two wavefronts a SIMD holds one feeds the matrix pipe while the
-    // other moves data (both make the same memory requests in the same order: the in-flight counts stay exact).
+    // A step is two row groups (8 output rows).  Trips of UNRF steps (the ring's period in steps), left after the run's last step
+    // by a uniform exit between steps.
     const int nfat = (nsteps + 1) >> 1;
     int fdone = 0;
     bool left = false;
-    auto stage_step = [&](int jf, int f) {
-        store(f - 1);
-        add_fetch(f);
-        commit(buf[jf % 2], f + 2);   // pass f + 2 sits in buffer f % 2 = jf % 2 (UNRF is even)
-        issue(buf[jf % 2], f + 4);
-    };
-    auto compute_step = [&](int jf, int f) {
-        // the two row groups this step adds to the ring; the second goes to the slot of the step's own first
-        // group, which the first tile still reads, so it waits in registers until the products are issued
+    auto step = [&](int jf, int f) {
+        // the two row groups this step adds to the ring; the second goes to the slot of the step's own first group, once the
+        // first tile's products with that are issued (LATE), or waits in registers where those are nearly all there are
+        constexpr bool LATE = PER >= 3;
         load_group((2 * jf + PER - 1) % PER, ((2 * f + PER - 1) % NR) * (4 * RP));
         const int late_off = ((2 * f + PER) % NR) * (4 * RP);
         uint4 late[CPW][ICB];
+        if constexpr (!LATE) {
 #pragma unroll
-        for (int q = 0; q < CPW; ++q)
+            for (int q = 0; q < CPW; ++q)
 #pragma unroll
-            for (int i = 0; i < ICB; ++i) late[q][i] = read16(xb[q][i] + late_off);
+                for (int i = 0; i < ICB; ++i) late[q][i] = read16(xb[q][i] + late_off);
+        }
+        uint4 out[NG];
+#pragma unroll
+        for (int n = 0; n < NG; ++n) out[n] = tile_read(jf + 1, n);
         tz_f32x4 acc[2][CPW];
 #pragma unroll
         for (int gi = 0; gi < 2; ++gi)
 #pragma unroll
             for (int q = 0; q < CPW; ++q) acc[gi][q] = tz_f32x4{0.f, 0.f, 0.f, 0.f};
+        // The products, and between them what moves data: the previous step's tiles out, the pass the NEXT step needs into
+        // the window, the one two steps on requested.  (One after the other they leave the matrix pipe idle two thirds of
+        // a step; left to itself the compiler puts them one after the other.)
+        constexpr int MOVE = NM < 7 ? 1 : NM / 7;   // products per channel and tile between two pieces
 #pragma unroll
-        for (int t = 0; t < NM; ++t)
+        for (int t = 0; t < NM; ++t) {
 #pragma unroll
             for (int q = 0; q < CPW; ++q) {
                 acc[0][q] = mfma16(A[q][t], ring[q][(ICB * 2 * jf + t) % RING], acc[0][q], T());
-                const uint4 b1 = t < ICB * (PER - 1) ? ring[q][(ICB * (2 * jf + 1) + t) % RING] : late[q][t - ICB * (PER - 1) < ICB ? t - ICB * (PER - 1) : 0];
+                const uint4 b1 = LATE || t < ICB * (PER - 1) ? ring[q][(ICB * (2 * jf + 1) + t) % RING] : late[q][t - ICB * (PER - 1) < ICB ? t - ICB * (PER - 1) : 0];
                 acc[1][q] = mfma16(A[q][t], b1, acc[1][q], T());
             }
+            if constexpr (LATE) {
+                if (t == ICB - 1) load_group((2 * jf) % PER, late_off);
+            }
 #pragma unroll
-        for (int q = 0; q < CPW; ++q)
+            for (int piece = 0; piece < 7; ++piece) {
+                if (t != (piece * MOVE < NM - 1 ? piece * MOVE : NM - 1)) continue;
+                if (piece >= 2 && piece < 6) commit_part(buf[jf % 2], piece - 2);   // pass f + 2 sits in buffer f % 2 = jf % 2 (UNRF is even)
+                if (piece == 6) {
+                    commit_next();
+                    write_pool(buf[jf % 2], f + 2);
+                    issue(buf[jf % 2], f + 4);
+                }
+                if (piece == 0) {
 #pragma unroll
-            for (int i = 0; i < ICB; ++i) ring[q][((2 * jf) % PER) * ICB + i] = late[q][i];
+                    for (int n = 0; n < NG; ++n) tile_store(out[n], n);
+                }
+                if (piece == 1) place();
+                __builtin_amdgcn_sched_barrier(0x6);   // (vector and scalar arithmetic may cross)
+            }
+        }
+        if constexpr (!LATE) {
+#pragma unroll
+            for (int q = 0; q < CPW; ++q)
+#pragma unroll
+                for (int i = 0; i < ICB; ++i) ring[q][((2 * jf) % PER) * ICB + i] = late[q][i];
+        }
 #pragma unroll
         for (int gi = 0; gi < 2; ++gi) {
-            char* dst = olw + (2 * (f & 1) + gi) * OLB;
+            char* dst = olw + (2 * (jf & 1) + gi) * OLB;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 if constexpr (CPW == 2) {
@@ -498,14 +637,8 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
         for (int jf = 0; jf < UNRF; ++jf) {
             const int f = f0 + jf;
             lds_barrier();  // the previous step's tiles are complete, its window reads done
-            if (wv < 4) {
-                if (f < nfat) compute_step(jf, f);
-                stage_step(jf, f);
-            } else {
-                stage_step(jf, f);
-                if (f < nfat) compute_step(jf, f);
-            }
-            if (f + 1 >= nfat) {   // the band's last step (uniform): its tiles are stored after the loop
+            step(jf, f);
+            if (f + 1 >= nfat) {   // the run's last step (uniform): its tiles are stored after the loop
                 left = true;
                 fdone = f + 1;
                 break;
@@ -515,7 +648,8 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
         fdone = f0 + UNRF;
     }
     lds_barrier();
-    store(fdone - 1);
+#pragma unroll
+    for (int n = 0; n < NG; ++n) tile_store(tile_read(fdone - 1, n), n);
 }
 
 template <typename T, int K, int NPC, int CS, int MODE>
@@ -528,32 +662,92 @@ __global__ __launch_bounds__(512, 1) void dwconv_tz_k(const T* __restrict__ x, c
 // ------------------------------------------------------------------------------------------------
 // Host side
 
-// Band height: the choice with the shortest estimated run, rounds of workgroups over 256 compute units times the
-// rows a workgroup moves (window rows plus a fixed cost of about 8 rows' worth).
-template <int K, int NPC, int CS>
-static int tz_pick_band(int B, int OH, int OW, int C) {
-    using Sh = TzShape<K, NPC, CS>;
-    const long long per_band = (long long)cdiv(B, Sh::NI) * cdiv(C, CS) * cdiv(OW, Sh::TW);
-    if (const char* e = tune_env("PDW_TZ_BR")) return atoi(e);
-    int best = 0;
-    double best_cost = 0;
-    for (int br = 4; br <= ((OH + 3) / 4) * 4; br += 4) {
-        const long long wgs = per_band * cdiv(OH, br);
-        const double cost = (double)cdiv(wgs, 256) * (Sh::win_rows(br) + 8);
-        if (best == 0 || cost <= best_cost) best = br, best_cost = cost;
-    }
-    return best;
-}
-
 // Patches per image row, 16 (true) or 8 in two images: the width whose padding of (columns x images) is smaller, wider on ties.
 inline bool tz_wide_tile(int B, int OW) {
     return (long long)cdiv(OW, 64) * 64 * B <= (long long)cdiv(OW, 32) * 32 * cdiv(B, 2) * 2;
 }
 
-// The geometry of a launch (false: not covered) and its number of workgroups.
+// Cuts the stack into runs of `run` rows (a multiple of 8), by the image where that divides an image's part of the stack; false:
+// a run's images are beyond 32-bit offsets.
+inline bool tz_cut(TzGeom& g, int ni, long long run) {
+    const int images = cdiv(g.B, ni), total = (images - 1) * g.per + g.OH;
+    if (run > total) run = (total + 7) / 8 * 8;
+    g.run = (int)run, g.rpi = g.per % g.run == 0 ? cdiv(g.OH, g.run) : 0;
+    if ((long long)images * g.rpi > 0x7fffffffLL) return false;
+    g.nruns = g.rpi ? images * g.rpi : cdiv(total, g.run);
+    const long long reach = ((long long)(g.per + g.run + 64) / g.per + 1) * ni, most = reach < g.B ? reach : g.B;
+    const long long in = (long long)g.H * g.W * g.C, out = (long long)g.OH * g.OW * g.YC;
+    // the kernel's quotients: rows of the stack by per, workgroups by slices, tiles and runs
+    const int by = std::max(std::max(g.nslices, g.ncolt), g.rpi);
+    if ((long long)(total + g.run + g.per + 128) * g.per > 0xffffffffLL || (long long)g.nruns * g.ncolt * g.nslices * by > 0xffffffffLL) return false;
+    g.per_inv = tz_inverse(g.per), g.rpi_inv = tz_inverse(std::max(g.rpi, 1));
+    g.ncolt_inv = tz_inverse(g.ncolt), g.nslices_inv = tz_inverse(g.nslices);
+    return most * (in > out ? in : out) <= 0x1fffffffLL;
+}
+inline long long tz_blocks(const TzGeom& g) { return (long long)g.nruns * g.ncolt * g.nslices; }
+
+// Steps of 8 rows of the longest run: those between images at a run's end are left out.
+inline int tz_steps(const TzGeom& g) {
+    if (g.run % g.per == 0) return (g.run - g.per + g.OH + 7) / 8;
+    return (g.rpi && g.OH < g.run ? g.OH + 7 : g.run) / 8;
+}
+
+// Estimated time of a workgroup, us, on a chip full of them: a start-up (first windows, filter table, operand set-up), then
+// steps of 8 rows.
+constexpr double kTzStart = 7.0, kTzStep = 0.9;
+inline double tz_run_cost(const TzGeom& g) { return kTzStart + kTzStep * tz_steps(g); }
+
+// The cut with the fewest workgroups whose runs have at most `steps` steps (of equal ones the shorter runs): runs of any length,
+// whole images, or equal parts of an image (those that start with an image need no steps for the rows between two).
+inline bool tz_cut_steps(TzGeom& g, int ni, int steps) {
+    long long best = 0, best_blocks = 0;
+    int best_steps = 0;
+    auto look = [&](long long run) {
+        if (run < 8 || !tz_cut(g, ni, run) || tz_steps(g) > steps) return;
+        const long long n = tz_blocks(g);
+        if (best == 0 || n < best_blocks || (n == best_blocks && tz_steps(g) < best_steps)) best = run, best_blocks = n, best_steps = tz_steps(g);
+    };
+    const int per_image = cdiv(g.OH, 8), group = g.per / 8;
+    look(8LL * steps);
+    if (steps >= per_image) look((long long)((steps - per_image) / group + 1) * g.per);
+    for (int j = 2; j <= group; ++j)
+        if (group % j == 0 && group / j <= steps) {
+            look(g.per / j);
+            break;
+        }
+    return best != 0 && tz_cut(g, ni, best);
+}
+
+// Runs of a launch of its own: the shortest with which 256 compute units are filled 1..4 times, whichever number is estimated to
+// end first; false: not covered.  (Each call plans anew: a handful of cuts, a fraction of a microsecond.)
+inline bool tz_cut_alone(TzGeom& g, int ni) {
+    const long long per_run = (long long)g.ncolt * g.nslices;
+    const int images = cdiv(g.B, ni), total = cdiv((long long)(images - 1) * g.per + g.OH, 8), group = g.per / 8;
+    long long best = 0;
+    double best_cost = 0;
+    auto look = [&](long long run, long long most) {
+        if (!tz_cut(g, ni, run) || (tz_blocks(g) > most && most >= per_run)) return;
+        const double cost = cdiv(tz_blocks(g), 256) * tz_run_cost(g);
+        if (best == 0 || cost < best_cost) best = run, best_cost = cost;
+    };
+    for (int rounds = 1; rounds <= 4; ++rounds) {
+        const long long most = 256LL * rounds, want = most / per_run, n = want < 1 ? 1 : want > total ? total : want;
+        look(8LL * cdiv(total, n), most);
+        if (n < images) {
+            look((long long)cdiv(images, n) * g.per, most);   // whole images
+        } else {
+            int j = (int)std::min<long long>(n / images, group);   // equal parts of an image
+            while (group % j) --j;
+            look(g.per / j, most);
+        }
+    }
+    // (large images: runs as short as their offsets need)
+    return tz_cut(g, ni, best == 0 ? 8 : best) && tz_blocks(g) <= 0x7fffffffLL;
+}
+
+// The geometry but for the runs (false: not covered).
 template <int K, int NPC, int CS>
-static bool tz_make_geom(TzGeom& g, long long& nblocks, bool add, int B, int H, int W, int C, int PH, int PW, bool flip,
-                         const TzGate* gate) {
+static bool tz_make_geom(TzGeom& g, bool add, int B, int H, int W, int C, int PH, int PW, bool flip, const TzGate* gate) {
     using Sh = TzShape<K, NPC, CS>;
     g.B = B, g.H = H, g.W = W, g.C = C, g.PH = PH, g.PW = PW, g.flip = flip ? 1 : 0;
     g.OH = H + 2 * PH - K + 1, g.OW = W + 2 * PW - K + 1;
@@ -561,11 +755,12 @@ static bool tz_make_geom(TzGeom& g, long long& nblocks, bool add, int B, int H, 
     g.YC = gate ? gate->ldy : C, g.ych = gate ? gate->ych : 0, g.gs = gate ? gate->gs : 1.f;
     if (gate && (add || flip || C % 16 != 0 || gate->ldy < gate->ych + C / 2 || (gate->ldy | gate->ych) % 8 != 0)) return false;
     if ((long long)H * W * C * Sh::NI > 0x1fffffffLL || (long long)g.OH * g.OW * g.YC * Sh::NI > 0x1fffffffLL) return false;
-    g.BR = tz_pick_band<K, NPC, CS>(B, g.OH, g.OW, C);
-    if (g.BR < 4) return false;
-    g.nbands = cdiv(g.OH, g.BR), g.ncolt = cdiv(g.OW, Sh::TW), g.nslices = cdiv(C, CS);
-    nblocks = (long long)cdiv(B, Sh::NI) * g.nbands * g.ncolt * g.nslices;
-    return nblocks <= 0x7fffffffLL;
+    // the windows of a run's first and last rows of an image reach PH rows before it and K - 1 - PH after: zeros
+    g.per = H + PH > g.OH ? H + PH : g.OH;
+    g.per = (g.per + 7) / 8 * 8;
+    if ((long long)(cdiv(B, Sh::NI) - 1) * g.per + g.OH + g.per + 64 > 0x7fffffffLL) return false;
+    g.ncolt = cdiv(g.OW, Sh::TW), g.nslices = cdiv(C, CS);
+    return true;
 }
 
 template <typename T, int K, int NPC, int CS>
@@ -573,8 +768,7 @@ static int launch_tz(const void* x, const void* w, const void* add, void* pool, 
                      int PH, int PW, bool flip, const TzGate* gate, hipStream_t s) {
     using Sh = TzShape<K, NPC, CS>;
     TzGeom g;
-    long long nblocks;
-    if (!tz_make_geom<K, NPC, CS>(g, nblocks, add != nullptr, B, H, W, C, PH, PW, flip, gate)) return -1;
+    if (!tz_make_geom<K, NPC, CS>(g, add != nullptr, B, H, W, C, PH, PW, flip, gate) || !tz_cut_alone(g, Sh::NI)) return -1;
     const size_t lds = Sh::lds_bytes;
     const int mode = (add ? 1 : 0) | (pool ? 2 : 0) | (gate ? 4 : 0);
     auto kern = dwconv_tz_k<T, K, NPC, CS, 0>;
@@ -587,7 +781,7 @@ static int launch_tz(const void* x, const void* w, const void* add, void* pool, 
     if (mode == 3 || mode == 5 || mode == 7 || (mode == 6 && CS != 16)) return -1;
     static std::once_flag attr_once[8];
     std::call_once(attr_once[mode], [&] { (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); });
-    hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(Sh::NT), lds, s, (const T*)x, (const T*)w, (const T*)add,
+    hipLaunchKernelGGL(kern, dim3((unsigned)tz_blocks(g)), dim3(Sh::NT), lds, s, (const T*)x, (const T*)w, (const T*)add,
                        (T*)pool, (T*)y, g);
     return check_launch("dwconv_tz");
 }

@@ -342,7 +342,9 @@ inline bool wgrad_ph_cut(WgPhPlan& p, int n) {
 
 // Estimated time of a run, us, on a chip full of them: start-up (16 gy rows, two round trips to memory, the partial), then
 // passes of 8 rows.
-inline double wgrad_ph_run_cost(int K, int passes) { return (K <= 9 ? 6.0 : 7.0) + (K <= 9 ? 1.15 : 1.35) * passes; }
+constexpr double kWgPhStart = 7.0;
+inline double wgrad_ph_step(int K) { return K <= 9 ? 1.15 : 1.35; }
+inline double wgrad_ph_run_cost(int K, int passes) { return kWgPhStart + wgrad_ph_step(K) * passes; }
 
 // Covered: 16-bit types (the caller checks), C % 8 == 0, K <= 15, 16-byte aligned tensors.
 inline WgPhPlan wgrad_ph_plan(int B, int H, int W, int C, int K, int PH, int PW) {

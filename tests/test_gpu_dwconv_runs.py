@@ -1,0 +1,28 @@
+"""The 16-bit forward and input gradient where their runs of rows start and end: batches stacked into one column of rows, runs
+that begin inside an image, cross several, or end between two; odd batches of narrow images (two side by side); paddings on
+either side of a multiple of 8 rows."""
+import pytest
+import torch
+
+from parity import TOL, randn, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shape,k,pad", [((40, 9, 40, 16), 5, 2), ((37, 7, 7, 136), 9, 4), ((300, 3, 20, 8), 3, 1),
+                                         ((66, 20, 36, 64), 13, 6), ((5, 57, 61, 24), 17, 8), ((9, 16, 64, 272), 7, 3),
+                                         ((3, 24, 112, 48), 15, 7), ((130, 8, 33, 8), 11, 5), ((6, 17, 30, 24), 9, 0),
+                                         ((4, 12, 13, 40), 5, 11)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_runs_over_stacked_images(oracle, shape, k, pad, dtype):
+    from pyramidconvblock_amd.dwconv import dwconv_dgrad, dwconv_forward
+
+    B, H, W, C = shape
+    gen = torch.Generator().manual_seed(k + H)
+    x, w = randn(gen, *shape).to(dtype), (randn(gen, k, k, C) / k).to(dtype)
+    gy = randn(gen, B, H + 2 * pad - k + 1, W + 2 * pad - k + 1, C).to(dtype)
+    geo = ((1, 1), (pad, pad), (1, 1))
+    want = oracle.dwconv_fwd(x.double().numpy(), w.double().numpy(), 1, (pad, pad), 1)
+    assert rel_err(dwconv_forward(x.cuda(), w.cuda(), *geo), want) <= TOL[dtype]
+    want = oracle.dwconv_dgrad(gy.double().numpy(), w.double().numpy(), (H, W), 1, (pad, pad), 1)
+    assert rel_err(dwconv_dgrad(gy.cuda(), w.cuda(), shape, *geo), want) <= TOL[dtype]
