@@ -293,13 +293,16 @@ int backward(const Shape& s, const Saved& v, const BwdWork& g, const void* gy, c
         if (int e = pdw_dense_bwd_pair(gy, w_out, v.cat, g.dcat, gparts, gw_out, g.ws_po, g.b_po, nullptr, 1, s.N, s.D, s.I, dt, stream))
             return e;
     } else {
+        const int both = colsum ? -1 : dense_bwd_both_launch(gy, w_out, v.cat, g.dcat, gw_out, g.ws_po, g.b_po, nullptr, 1, s.N, s.D, s.I, dt, st);
+        if (both != 0 && both != -1) return both;
         if (colsum) {
             gparts = g.gparts;
             if (int e = pdw_dense_fwd_colsum(gy, w_out, 1, nullptr, nullptr, g.dcat, gparts, s.N, s.D, s.I, 1, dt, stream)) return e;
-        } else if (int e = pdw_dense_fwd(gy, w_out, 1, nullptr, nullptr, g.dcat, s.N, s.D, s.I, 1, dt, stream)) {
-            return e;
+        } else if (both == -1) {
+            if (int e = pdw_dense_fwd(gy, w_out, 1, nullptr, nullptr, g.dcat, s.N, s.D, s.I, 1, dt, stream)) return e;
         }
-        if (int e = pdw_dense_wgrad(gy, v.cat, gw_out, g.ws_po, g.b_po, s.N, s.D, s.I, dt, stream)) return e;
+        if (both == -1)
+            if (int e = pdw_dense_wgrad(gy, v.cat, gw_out, g.ws_po, g.b_po, s.N, s.D, s.I, dt, stream)) return e;
     }
     // the gates and the mean branch
     reduce_defer_compact(0, 0);
@@ -355,6 +358,10 @@ int backward(const Shape& s, const Saved& v, const BwdWork& g, const void* gy, c
     reduce_defer_compact(seg * s.D, val * s.D);
     if (dx && s.P >= 32 && pdw_dense_bwd_pair_supported(s.I, s.D, dt))
         return pdw_dense_bwd_pair(g.da, w_up, x, dx, nullptr, gw_up, g.ws_pu, g.b_pu, g.dmean, s.P, s.N, s.I, s.D, dt, stream);
+    if (dx) {
+        const int both = dense_bwd_both_launch(g.da, w_up, x, dx, gw_up, g.ws_pu, g.b_pu, g.dmean, s.P, s.N, s.I, s.D, dt, st);
+        if (both != -1) return both;
+    }
     if (int e = pdw_dense_wgrad(g.da, x, gw_up, g.ws_pu, g.b_pu, s.N, s.I, s.D, dt, stream)) return e;
     if (!dx) return 0;
     // (the summations recorded so far ride in the last kernel of the pass)

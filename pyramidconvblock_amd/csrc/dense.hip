@@ -1280,6 +1280,12 @@ int dense_wgrad_launch(const void* a, const void* b, void* dw, void* ws, long lo
     return dense_wgrad_t<bf16_t>(a, b, dw, ws, N, M, NO, s);
 }
 
+int dense_bwd_both_launch(const void* gy, const void* w, const void* b, void* dx, void* dw, void* ws, size_t ws_bytes, const float* rowbias,
+                          int P, long long N, int M, int NO, int dtype, hipStream_t s) {
+    if (dense_dims_ok(M, NO, dtype) || dense_wgrad_tiled_ok(M, NO, dtype) || ws_bytes < dense_wgrad_workspace(N, M, NO)) return -1;
+    return dense_wide_bwd_pair_launch(gy, w, b, dx, dw, ws, rowbias, P, N, M, NO, dtype, dense_wgrad_parts(N, M, NO), s);
+}
+
 static bool pair_exact(int O, int I) {
     return (O == 128 && I == 64) || (O == 64 && I == 128) || (O == 64 && I == 32) || (O == 32 && I == 64) ||
            (O == 96 && I == 48) || (O == 48 && I == 96);

@@ -22,6 +22,7 @@
 #include <mutex>
 
 #include "common.h"
+#include "dense_any_wgrad.h"
 #include "kernels.h"
 #include "reduce_parts.h"
 #include "tile_common.h"
@@ -30,9 +31,6 @@ namespace pdw {
 
 namespace {
 
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef short v8s __attribute__((ext_vector_type(8)));
@@ -41,7 +39,6 @@ typedef __attribute__((address_space(3))) char lds_char;
 constexpr int kRowBytes = 128;              // inner bytes per stage: 64 values of 16 bits, 32 of fp32
 template <typename T>
 constexpr int kBK = kRowBytes / (int)sizeof(T);
-constexpr uint32_t kPast = 0x80000000u;     // an offset past the end of any descriptor used here
 
 __device__ __forceinline__ v16f mfma(v8s a, v8s b, v16f c, bf16_t) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
@@ -162,7 +159,7 @@ template <typename T, int BM, int BN>
 constexpr int kWideOccupancy = sizeof(T) == 4 ? (BM * BN <= 64 * 64 ? 4 : BM * BN <= 128 * 64 ? 3 : 2) : 2;
 
 template <typename T, int BM, int BN, bool TA, bool TB, bool PART>
-__global__ __launch_bounds__(256, (kWideOccupancy<T, BM, BN>)) void wide_gemm_k(WideArgs g) {
+__device__ __forceinline__ void wide_gemm_body(const WideArgs& g, int blk, int nblk) {
     typedef Operand<T, BM, TA> OpA;
     typedef Operand<T, BN, TB> OpB;
     constexpr int BK = kBK<T>, KK = 4;          // inner values of a stage; fragments of it
@@ -173,7 +170,7 @@ __global__ __launch_bounds__(256, (kWideOccupancy<T, BM, BN>)) void wide_gemm_k(
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave & 1, wn = wave >> 1;
     // tiles of one row range next to each other on one XCD: they read the same rows
-    int id = xcd_remap(blockIdx.x, gridDim.x);
+    int id = xcd_remap(blk, nblk);
     const int tn = id % g.nt;
     id /= g.nt;
     const int tm = id % g.mt, sp = id / g.mt;
@@ -278,9 +275,51 @@ __global__ __launch_bounds__(256, (kWideOccupancy<T, BM, BN>)) void wide_gemm_k(
 }
 
 template <typename T, int BM, int BN, bool TA, bool TB, bool PART>
-int wide_go(const WideArgs& g, hipStream_t s) {
+__global__ __launch_bounds__(256, (kWideOccupancy<T, BM, BN>)) void wide_gemm_k(WideArgs g) {
+    wide_gemm_body<T, BM, BN, TA, TB, PART>(g, blockIdx.x, gridDim.x);
+}
+
+// Both products that read the gradient of a layer's output, as one launch: the weight gradient's nw workgroups (tiles of WM x WN
+// of this file; WM = 0: the kernel without LDS, dense_any_wgrad.h), which are the longer ones, then the input gradient's.  A
+// launch of its own leaves part of the chip idle in its last round and pays the ramp; together they are dealt as one.
+// us, two launches -> one: [100352,128] <- 64 fp32 44.7 -> 41.0, 64 <- 128 48.4 -> 43.0 (153 and 180 MB); [10431,200] <- 104 bf16 13.4
+// -> 8.8; [16384,1152] <- 576 fp16 66.5 -> 61.4, 576 <- 1152 71.7 -> 68.1; [2048,64] <- 32 fp32 8.6 -> 4.9.
+template <typename T, int BM, int BN, int WM, int WN>
+__global__ __launch_bounds__(256, (kWideOccupancy<T, BM, BN>)) void wide_pair_k(WideArgs rows, WideArgs wgrad, AnyWgradArgs any, int nw) {
+    const int blk = blockIdx.x;
+    if (blk >= nw) {
+        wide_gemm_body<T, BM, BN, false, true, false>(rows, blk - nw, gridDim.x - nw);
+    } else if constexpr (WM != 0) {
+        wide_gemm_body<T, WM, WN, true, true, true>(wgrad, blk, nw);
+    } else {
+        const int group = blk / any.chunks;
+        dense_any_wgrad_body<T>(any, blk - group * any.chunks, group);
+    }
+}
+
+template <typename T, int BM, int BN, bool PART>
+constexpr size_t wide_lds() {
     constexpr size_t stages = (size_t)2 * (BM + BN) * kRowBytes, out = PART ? 0 : (size_t)BM * (BN * sizeof(T) + 16);
-    constexpr size_t lds = stages > out ? stages : out;
+    return stages > out ? stages : out;
+}
+
+template <typename T, int BM, int BN, int WM, int WN>
+int pair_go(const WideArgs& rows, const WideArgs& wgrad, const AnyWgradArgs& any, int nw, hipStream_t s) {
+    constexpr size_t a = wide_lds<T, BM, BN, false>(), b = WM != 0 ? wide_lds<T, WM, WN, true>() : 0, lds = a > b ? a : b;
+    if constexpr (lds > 64 * 1024) {
+        static std::once_flag once;
+        std::call_once(once, [] {
+            (void)hipFuncSetAttribute((const void*)wide_pair_k<T, BM, BN, WM, WN>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        });
+    }
+    if ((long long)nw + (long long)rows.mt * rows.nt > 0x7fffffffLL) return -1;
+    hipLaunchKernelGGL((wide_pair_k<T, BM, BN, WM, WN>), dim3((unsigned)(nw + rows.mt * rows.nt)), dim3(256), lds, s, rows, wgrad, any, nw);
+    return check_launch("wide_pair");
+}
+
+template <typename T, int BM, int BN, bool TA, bool TB, bool PART>
+int wide_go(const WideArgs& g, hipStream_t s) {
+    constexpr size_t lds = wide_lds<T, BM, BN, PART>();
     if constexpr (lds > 64 * 1024) {
         static std::once_flag once;
         std::call_once(once, [] {
@@ -328,21 +367,19 @@ bool dense_wide_ok(int K, int NO, int dtype) {
     return K >= v && NO >= v && K % v == 0 && NO % v == 0;
 }
 
-// -1: not covered (widths, alignment, offsets of 2^31 bytes within a tile or a weight).
-int dense_wide_rows_launch(const void* x, const void* w, int w_kmajor, const void* bias, const float* rowbias, void* y,
-                           long long N, int K, int NO, int P, int dtype, hipStream_t s) {
+// Arguments and tiles of the row product; false: not covered (widths, alignment, offsets of 2^31 bytes within a tile or a weight).
+static bool wide_rows_plan(WideArgs& g, int& bm, int& bn, const void* x, const void* w, int w_kmajor, const void* bias, const float* rowbias,
+                           void* y, long long N, int K, int NO, int P, int dtype) {
     const int es = dtype == kF32 ? 4 : 2;
     if (!dense_wide_ok(K, NO, dtype) || N > 0x7fffffffLL || (long long)K * NO * es > 0x7fffffffLL || K > (1 << 21) || NO > (1 << 21))
-        return -1;
+        return false;
     if (!aligned16(x) || !aligned16(w) || !aligned16(y) || !aligned16(rowbias) || (reinterpret_cast<uintptr_t>(bias) & (es == 4 ? 15 : 7)))
-        return -1;
-    if (N == 0) return 0;
-    WideArgs g{x, w, bias, rowbias, y, N, K, NO, K, w_kmajor ? NO : K, P > 0 ? P : 1, 0, 0, 1, (long long)cdiv(K, 64) * 64};
-    int bm, bn;
+        return false;
+    g = WideArgs{x, w, bias, rowbias, y, N, K, NO, K, w_kmajor ? NO : K, P > 0 ? P : 1, 0, 0, 1, (long long)cdiv(K, 64) * 64};
     if (es == 4) {
         // small tiles, four to a compute unit ([100352,128] -> 64: 22.8 us, 128 x 64 26.9, 128 x 128 41.7; never slower where
         // it matters), but not for many rows of a short sum, which is a stream ([50000,16] -> 32: 6.4 here, 5.6 in dense_any.hip)
-        if (K < 32 && N >= 16384 && NO <= 256) return -1;
+        if (K < 32 && N >= 16384 && NO <= 256) return false;
         bm = bn = 64;
     } else {
         // tiles of 64 rows where 128-row tiles would leave compute units without work
@@ -354,10 +391,19 @@ int dense_wide_rows_launch(const void* x, const void* w, int w_kmajor, const voi
         if (bm == 128 && bn == 128 && K >= 256 && rounds(192) * 4 < rounds(128) * 3) bn = 192;
     }
     g.mt = cdiv(N, bm), g.nt = cdiv(NO, bn);
-    if ((long long)g.mt * g.nt > 0x7fffffffLL) return -1;
+    return (long long)g.mt * g.nt <= 0x7fffffffLL;
+}
+
+// -1: not covered.
+int dense_wide_rows_launch(const void* x, const void* w, int w_kmajor, const void* bias, const float* rowbias, void* y,
+                           long long N, int K, int NO, int P, int dtype, hipStream_t s) {
+    WideArgs g;
+    int bm, bn;
+    if (!wide_rows_plan(g, bm, bn, x, w, w_kmajor, bias, rowbias, y, N, K, NO, P, dtype)) return -1;
+    if (N == 0) return 0;
 #define PDW_WIDE_T(T, BM, BN) (w_kmajor ? wide_go<T, BM, BN, false, true, false>(g, s) : wide_go<T, BM, BN, false, false, false>(g, s))
 #define PDW_WIDE(BM, BN) (dtype == kF16 ? PDW_WIDE_T(f16_t, BM, BN) : PDW_WIDE_T(bf16_t, BM, BN))
-    if (es == 4) return PDW_WIDE_T(float, 64, 64);
+    if (dtype == kF32) return PDW_WIDE_T(float, 64, 64);
     if (bn == 192) return PDW_WIDE(128, 192);
     if (bm == 64) return bn == 64 ? PDW_WIDE(64, 64) : PDW_WIDE(64, 128);
     return bn == 64 ? PDW_WIDE(128, 64) : PDW_WIDE(128, 128);
@@ -392,6 +438,47 @@ int dense_wide_wgrad_launch(const void* a, const void* b, void* dw, void* ws, lo
     if (dtype == kF32) return wgrad_reduce_launch<float>((const float*)ws, dw, p.splits, M * NO, s);
     if (dtype == kF16) return wgrad_reduce_launch<f16_t>((const float*)ws, dw, p.splits, M * NO, s);
     return wgrad_reduce_launch<bf16_t>((const float*)ws, dw, p.splits, M * NO, s);
+}
+
+// dx[N,NO] = gy[N,M] W (+ rowbias), W stored [M][NO], and dW[M][NO] = gy^T b, in one launch; -1: not covered, or products that
+// other kernels make (the caller makes them one by one).  max_chunks: partials the workspace holds.
+int dense_wide_bwd_pair_launch(const void* gy, const void* w, const void* b, void* dx, void* dw, void* ws, const float* rowbias, int P,
+                               long long N, int M, int NO, int dtype, int max_chunks, hipStream_t s) {
+    WideArgs rows, wg{};
+    AnyWgradArgs any{};
+    int bm, bn, nw, nparts;
+    if (N < 1 || !aligned16(b) || !aligned16(ws) || !dense_wide_ok(M, NO, dtype)) return -1;
+    if (!wide_rows_plan(rows, bm, bn, gy, w, 1, nullptr, rowbias, dx, N, M, NO, P, dtype)) return -1;
+    const int es = dtype == kF32 ? 4 : 2;
+    WgradPlan p{};
+    const bool small = es == 4 && M <= 256 && NO <= 256;   // (as dense_wide_wgrad_launch chooses)
+    if (small) {
+        if (!any_wgrad_args(any, gy, b, ws, N, M, NO, dtype, max_chunks)) return -1;
+        nw = any.chunks * any_wgrad_groups(any), nparts = any.chunks;
+    } else {
+        p = wgrad_plan(N, M, NO, es);
+        if (p.kper * (M > NO ? M : NO) * es > 0x7fffffffLL) return -1;
+        wg = WideArgs{gy, b, nullptr, nullptr, ws, M, N, NO, M, NO, 1, p.mt, p.nt, p.splits, p.kper};
+        nw = p.mt * p.nt * p.splits, nparts = p.splits;
+    }
+    int e = -1;
+    if (es == 4) {
+        if (small) e = pair_go<float, 64, 64, 0, 0>(rows, wg, any, nw, s);
+        else if (p.bm == 64 && p.bn == 64) e = pair_go<float, 64, 64, 64, 64>(rows, wg, any, nw, s);
+    } else if (p.bm == 128 && p.bn == 128) {
+        auto go = [&](auto t) {
+            using T = decltype(t);
+            if (bn == 192) return pair_go<T, 128, 192, 128, 128>(rows, wg, any, nw, s);
+            if (bm == 64 && bn == 128) return pair_go<T, 64, 128, 128, 128>(rows, wg, any, nw, s);
+            if (bm == 128 && bn == 128) return pair_go<T, 128, 128, 128, 128>(rows, wg, any, nw, s);
+            return -1;
+        };
+        e = dtype == kF16 ? go(f16_t{}) : go(bf16_t{});
+    }
+    if (e) return e;
+    if (dtype == kF32) return wgrad_reduce_launch<float>((const float*)ws, dw, nparts, M * NO, s);
+    if (dtype == kF16) return wgrad_reduce_launch<f16_t>((const float*)ws, dw, nparts, M * NO, s);
+    return wgrad_reduce_launch<bf16_t>((const float*)ws, dw, nparts, M * NO, s);
 }
 
 }  // namespace pdw
