@@ -506,7 +506,9 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
             __builtin_amdgcn_raw_buffer_store_b64(v2u{o.x, o.y}, yrsrc, (int)yoff[n], (int)stored, 0);
         } else {
             typedef unsigned v4u __attribute__((ext_vector_type(4)));
-            __builtin_amdgcn_raw_buffer_store_b128(v4u{v.x, v.y, v.z, v.w}, yrsrc, (int)yoff[n], (int)stored, 0);
+            // (No scalar offset in a 16-byte store: with one the compiler leaves no wait state between the store and a vector
+            // instruction that overwrites its data registers, and the last quarter of a row of lanes then stores the new value.)
+            __builtin_amdgcn_raw_buffer_store_b128(v4u{v.x, v.y, v.z, v.w}, yrsrc, (int)(yoff[n] + stored), 0, 0);
         }
     };
 
