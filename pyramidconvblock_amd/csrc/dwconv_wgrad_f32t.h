@@ -6,18 +6,22 @@
 // position 4g + t of the block for lane group g in instruction t, so that a lane's four xw values are one aligned
 // 16-byte LDS read, and its four gy values two 8-byte pairs at any element offset.
 //
-// What bounds it: the matrix pipe (32 cycles an instruction; its operands cost the LDS half of that).  Every position of a
+// What bounds it: the matrix pipe (32 cycles an instruction; its operands cost the LDS half of that), and next to it the vector
+// instructions of the staging, which do not overlap with fp32 products (dwconv_f32t.h): a tick has about 45 of them for 64
+// products (157 with every offset and ring row computed per thread).  Every position of a
 // row block costs the same whatever the filter, and a row block computes 16 positions of which 8 per tile are margin.
 //
 // A workgroup (8 wavefronts, one channel each) takes `U` units (image, row band, column tile) of one 8-channel slice one
 // after the other as one stream: a tick brings four window rows of x and four rows of gy into LDS rings (requested two
 // ticks ahead, across units as well) while the previous ones are multiplied, so only the first unit of a workgroup waits
-// for memory.  The taps leave through LDS as 16-byte stores into the workgroup's partial; fixed-order summation, no atomics.
+// for memory.  The taps leave through LDS as 16-byte stores into the workgroup's partial; fixed-order summation, no atomics;
+// every four ticks the accumulators are added to a total, so that the error does not grow with a workgroup's share ([32,56,56,64]
+// filter 13, against 64 bits: 2.6e-7 of the norm; 4.7e-7 without, 3.5e-7 in halves of an image without).
 //
-// Measured with the summation at [32,56,56,64]: filter 13 55 us for 78 on the vector ALU (dwconv_wgrad_tiled.h), 17 95 for
-// 177; [32,28,28,64]: filter 3 24 for 43, 13 27 for 33.  The products alone are 29 and the staging alone 29 of the 51 us
-// (filter 13, without the summation): the matrix pipe is 57 % busy.  16 channels a workgroup for whole 64-byte requests
-// measured the same.
+// Measured with the summation (us, before the waits by buffer name, the scalar offsets and the plan below -> with them):
+// [32,56,56,64] filter 13 52.7 -> 42.2 (products alone 29; vector ALU, dwconv_wgrad_tiled.h, 78), [3,57,61,100] filter 15 26.9 ->
+// 17.9, [8,112,112,48] filter 17 78 -> 63.8, [4,64,64,576] filter 13 110.6 -> 92.2, [100,14,14,64] filter 15 40.9 -> 29.6,
+// [6,90,90,32] filter 17 55.8 -> 30.9.  16 channels a workgroup for whole 64-byte requests measured the same.
 #pragma once
 #include <mutex>
 
@@ -56,7 +60,7 @@ struct WgF32Shape {
     static constexpr int CHX = wg_f32t_chx(K, NBI, NI), CHG = wg_f32t_chg(NBI, NI);
     static constexpr size_t lds_bytes = (size_t)CS * (CHX + CHG);
     static constexpr int NLX = (4 * XC * NQ + NT - 1) / NT, NLG = (4 * NI * TW * NQ + NT - 1) / NT;
-    static_assert(lds_bytes <= 160 * 1024 && NLG == 1 && (size_t)K * K * CS * 4 <= lds_bytes, "sizes");
+    static_assert(XC % 8 == 0 && TW % 8 == 0 && lds_bytes <= 160 * 1024 && NLG == 1 && (size_t)K * K * CS * 4 <= lds_bytes, "sizes");
 };
 
 struct WgF32Geom {
@@ -73,7 +77,7 @@ __device__ __forceinline__ void dwconv_wgrad_f32_body(const float* __restrict__ 
     extern __shared__ uint32_t smem[];
     char* const xl = reinterpret_cast<char*>(smem);
     char* const gl = xl + CS * CHX;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int bid = xcd_remap(blk, nblk);
     const int sl = bid % g.nslices, chunk = bid / g.nslices, c0 = sl * CS;
     const int u0 = chunk * g.U, u1 = min(u0 + g.U, g.units);
@@ -99,33 +103,63 @@ __device__ __forceinline__ void dwconv_wgrad_f32_body(const float* __restrict__ 
 
     // the unit and group that is requested next
     struct Cursor {
-        int u, gi, ng, rows, orow0, ocol0, cols;
+        int u, ct, band, b, gi, ng, rows, orow0;
         __amdgpu_buffer_rsrc_t xr, gr;
     } cur;
-    auto open = [&](int u) {
-        cur.u = u, cur.gi = 0;
-        const int ct = u % g.ncolt, t = u / g.ncolt, band = t % g.nbands, b = t / g.nbands * NI;
-        const int nimg = u < u1 ? min(NI, g.B - b) : 0;
-        cur.orow0 = band * g.BR, cur.ocol0 = ct * TW;
-        cur.rows = min(g.BR, g.OH - cur.orow0), cur.cols = min(TW, g.OW - cur.ocol0);
-        cur.ng = (cur.rows + 4) / 4 + XG - 1;   // steps over rows 0 .. rows, and the groups ahead of the first
-        cur.xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x + (nimg ? b : 0) * img_x), (short)0, (int)(nimg * img_x * 4), 0x00020000);
-        cur.gr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(gy + (nimg ? b : 0) * img_g), (short)0, (int)(nimg * img_g * 4), 0x00020000);
+    uint32_t xoff[NLX], goff;   // a thread's items in the unit: bytes from the group's first row, or kNoRow
+    auto steps = [&](int band) { return (min(g.BR, g.OH - band * g.BR) + 4) / 4 + XG - 1; };   // over rows 0 .. rows, and the groups ahead of the first
+    auto open = [&]() {
+        const int ocol0 = cur.ct * TW, nimg = min(NI, g.B - cur.b);
+        cur.orow0 = cur.band * g.BR;
+        cur.rows = min(g.BR, g.OH - cur.orow0);
+        cur.gi = 0, cur.ng = steps(cur.band);
+        cur.xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x + cur.b * img_x), (short)0, (int)(nimg * img_x * 4), 0x00020000);
+        cur.gr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(gy + cur.b * img_g), (short)0, (int)(nimg * img_g * 4), 0x00020000);
+#pragma unroll
+        for (int l = 0; l < NLX; ++l) {
+            const int ic = ocol0 - g.PW + xcol[l];
+            const bool ok = qok && xrow[l] < 4 && ic >= 0 && ic < g.W;
+            xoff[l] = ok ? ((uint32_t)((xrow[l] * g.W + ic) * g.C) + ximg[l]) * 4u : kNoRow;
+        }
+        const bool ok = qok && grow < 4 && gcol < min(TW, g.OW - ocol0);
+        goff = ok ? ((uint32_t)((grow * g.OW + ocol0 + gcol) * g.C) + gimg) * 4u : kNoRow;
     };
     f4 bx[2][NLX], bg[2];
     auto issue = [&](f4 (&dx)[NLX], f4& dg) {
+        const int xr0 = cur.orow0 - g.PH + 4 * cur.gi, gr0 = 4 * (cur.gi - (XG - 1));
+        const int xrow_at = xr0 * g.W * g.C * 4, grow_at = (cur.orow0 + gr0) * g.OW * g.C * 4;
+        // where all four rows exist, nothing to compute per thread
+        uint32_t xo[NLX], go = goff;
+        int xs = xrow_at, gs = grow_at;
 #pragma unroll
-        for (int l = 0; l < NLX; ++l) {
-            const int ic = cur.ocol0 - g.PW + xcol[l], ir = cur.orow0 - g.PH + 4 * cur.gi + xrow[l];
-            const bool ok = qok && xrow[l] < 4 && ic >= 0 && ic < g.W && ir >= 0 && ir < g.H;
-            const uint32_t off = ok ? ((uint32_t)((ir * g.W + ic) * g.C) + ximg[l]) * 4u : kNoRow;
-            dx[l] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(cur.xr, (int)off, 0, 0));
+        for (int l = 0; l < NLX; ++l) xo[l] = xoff[l];
+        if (xr0 < 0 || xr0 + 3 >= g.H) {   // (uniform, as the next)
+            xs = 0;
+#pragma unroll
+            for (int l = 0; l < NLX; ++l) {
+                const bool ok = (int)xoff[l] >= 0 && (unsigned)(xr0 + xrow[l]) < (unsigned)g.H;
+                xo[l] = ok ? xoff[l] + (uint32_t)xrow_at : kNoRow;
+            }
         }
-        const int r = 4 * (cur.gi - (XG - 1)) + grow;
-        const bool ok = qok && grow < 4 && gcol < cur.cols && r >= 0 && r < cur.rows;
-        const uint32_t off = ok ? ((uint32_t)(((cur.orow0 + r) * g.OW + cur.ocol0 + gcol) * g.C) + gimg) * 4u : kNoRow;
-        dg = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(cur.gr, (int)off, 0, 0));
-        if (++cur.gi == cur.ng) open(cur.u + 1);   // (uniform; past the last unit: empty descriptors)
+        if (gr0 < 0 || gr0 + 3 >= cur.rows) {
+            const bool ok = (int)goff >= 0 && (unsigned)(gr0 + grow) < (unsigned)cur.rows;
+            gs = 0, go = ok ? goff + (uint32_t)grow_at : kNoRow;
+        }
+#pragma unroll
+        for (int l = 0; l < NLX; ++l) dx[l] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(cur.xr, (int)xo[l], xs, 0));
+        dg = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(cur.gr, (int)go, gs, 0));
+        if (++cur.gi == cur.ng) {   // (uniform)
+            if (++cur.u < u1) {
+                if (++cur.ct == g.ncolt) {
+                    cur.ct = 0;
+                    if (++cur.band == g.nbands) cur.band = 0, cur.b += NI;
+                }
+                open();
+            } else {   // past the last unit: empty descriptors
+                cur.xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x), (short)0, 0, 0x00020000);
+                cur.gr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(gy), (short)0, 0, 0x00020000);
+            }
+        }
     };
     auto put = [&](char* d, int ch, const f4& v) {
         const float e0 = v.x, e1 = v.y, e2 = v.z, e3 = v.w;
@@ -135,127 +169,138 @@ __device__ __forceinline__ void dwconv_wgrad_f32_body(const float* __restrict__ 
     auto commit = [&](const f4 (&dx)[NLX], const f4& dg, int xslot, int grow0) {   // grow0: ring row of the group's first gy row
 #pragma unroll
         for (int l = 0; l < NLX; ++l)
-            if (xrow[l] < 4) put(xl + xdst[l] + xslot * 4 * RPX, CHX, dx[l]);
+            if (wv * 64 + l * NT < 4 * XC * NQ) put(xl + xdst[l] + xslot * 4 * RPX, CHX, dx[l]);   // (whole wavefronts)
         int r = grow0 + (grow & 3);
         r -= r >= NRG ? NRG : 0;
-        if (grow < 4) put(gl + gdst + r * RPG, CHG, dg);
+        if (wv * 64 < 4 * NI * TW * NQ) put(gl + gdst + r * RPG, CHG, dg);
     };
     auto lds_barrier = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-    open(u0);
+    cur.u = u0, cur.ct = u0 % g.ncolt, cur.band = u0 / g.ncolt % g.nbands, cur.b = u0 / g.ncolt / g.nbands * NI;
+    int ct = cur.ct, band = cur.band;   // of the unit that is multiplied
+    open();
     issue(bx[0], bg[0]);
     issue(bx[1], bg[1]);
-    // the zero margins of gy: everything but the tiles' own columns
-    for (int i = tid; i < CS * NRG * (RPG / 4); i += NT) {
-        const int c = i % (RPG / 4), row = i / (RPG / 4) % NRG, ch = i / (RPG / 4) / NRG;
-        if (c >= NI * GCI || c % GCI < 8 || c % GCI >= 8 + TW) *reinterpret_cast<float*>(gl + ch * CHG + row * RPG + c * 4) = 0.f;
-    }
+    for (int i = tid; i < CS * CHG / 16; i += NT) reinterpret_cast<f4*>(gl)[i] = f4{0.f, 0.f, 0.f, 0.f};   // (gy's zero margins stay)
+    lds_barrier();
     commit(bx[0], bg[0], 0, 0);
     issue(bx[0], bg[0]);
 
     // ---- operands of this wavefront's channel: lane = (m or n, k group kg)
     const int ln = lane & 15, kg = lane >> 4;
-    int arow[NMF];
+    uint32_t arow[NMF];   // bytes from the window's first row
     const char* abase[NMF];
 #pragma unroll
     for (int f = 0; f < NMF; ++f) {
         const int mi = min(ln + 16 * f, COMB - 1);
-        arow[f] = 2 * (mi / NBV);
+        arow[f] = (uint32_t)(2 * (mi / NBV) * RPX);
         abase[f] = xl + wv * CHX + (8 * (mi % NBV) + 4 * kg) * 4;
     }
     const int du = ln >> 3, dv = ln & 7;
-    const char* const bbase = gl + wv * CHG + (8 + 4 * kg - dv) * 4;
-    f4 acc[NMF][4];
+    const uint32_t bbase = (uint32_t)(CS * CHX + wv * CHG + (8 + 4 * kg - dv) * 4 - du * RPG);   // bytes in LDS
+    const uint32_t bwrap = du ? NRG * RPG : 0;
+    f4 acc[NMF][4], sum[NMF];   // of the last kFlush ticks; of all before
 #pragma unroll
-    for (int f = 0; f < NMF; ++f)
+    for (int f = 0; f < NMF; ++f) {
+        sum[f] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int t = 0; t < 4; ++t) acc[f][t] = f4{0.f, 0.f, 0.f, 0.f};
-    // With one product a position, a row's operands are read while the previous row is multiplied (left to itself the
-    // compiler reads a block's operands, waits for them and multiplies); with two (K = 17) the operands of a row would not
-    // fit the registers, and the second product covers the reads.
-    struct Row {
-        f4 a[NBI * NI][NMF];
-        float b[NBI * NI][4];
+    }
+    auto flush = [&]() {
+#pragma unroll
+        for (int f = 0; f < NMF; ++f) {
+            sum[f] += (acc[f][0] + acc[f][1]) + (acc[f][2] + acc[f][3]);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) acc[f][t] = f4{0.f, 0.f, 0.f, 0.f};
+        }
+    };
+    // A block of 16 positions is a piece: the operands of the piece kAhead further on are read while one is multiplied.
+    constexpr int NB = NBI * NI, kAhead = 1, kFlush = 4;
+    struct Piece {
+        f4 a[NMF];
+        float b[4];
     };
     auto compute = [&](int xslot, int grow0) {   // where the tick's own groups (the newest) lie
         int xr0 = 4 * (xslot - (XG - 1));
         xr0 += xr0 < 0 ? NRX : 0;
-        auto fetch = [&](Row& o, int ii) {
-            int gr = grow0 + ii - du;
-            gr += gr < 0 ? NRG : 0;
-            gr -= gr >= NRG ? NRG : 0;
-            const char* bp = bbase + gr * RPG;
-#pragma unroll
-            for (int nb = 0; nb < NBI * NI; ++nb)
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-                    o.b[nb][t] = *reinterpret_cast<const float*>(bp + 4 * (nb / NBI * GCI + nb % NBI * 16) + 4 * t);
-#pragma unroll
-            for (int f = 0; f < NMF; ++f) {
-                int r = xr0 + ii + arow[f];
-                r -= r >= NRX ? NRX : 0;
-                const char* ap = abase[f] + r * RPX;
-#pragma unroll
-                for (int nb = 0; nb < NBI * NI; ++nb) o.a[nb][f] = *reinterpret_cast<const f4*>(ap + 4 * (nb / NBI * XCI + nb % NBI * 16));
-            }
-        };
-        auto multiply = [&](const Row& o) {
-#pragma unroll
-            for (int nb = 0; nb < NBI * NI; ++nb)
+        uint32_t bp = 0;
+        const char* ap[NMF] = {};
+        auto fetch = [&](Piece& o, int p) {
+            const int ii = p / NB, nb = p % NB;
+            if (nb == 0) {
+                // gy row grow0 + ii - du of the ring: one further up where that is row -1
+                const int gr = grow0 + ii - (grow0 + ii >= NRG ? NRG : 0);
+                bp = bbase + (uint32_t)(gr * RPG) + (bwrap & (gr == 0 ? ~0u : 0u));
+                asm("" : "+v"(bp));   // (whole in a register: with the planes' offset left to the reads, each adds it again)
+                // window row xr0 + ii + 2a of the ring, whose rows come in pairs
 #pragma unroll
                 for (int f = 0; f < NMF; ++f) {
-                    const float a0 = o.a[nb][f].x, a1 = o.a[nb][f].y, a2 = o.a[nb][f].z, a3 = o.a[nb][f].w;
-                    acc[f][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, o.b[nb][0], acc[f][0], 0, 0, 0);
-                    acc[f][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, o.b[nb][1], acc[f][1], 0, 0, 0);
-                    acc[f][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(a2, o.b[nb][2], acc[f][2], 0, 0, 0);
-                    acc[f][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(a3, o.b[nb][3], acc[f][3], 0, 0, 0);
+                    if (ii % 2 == 0) {
+                        const uint32_t r = arow[f] + (uint32_t)((xr0 + ii) * RPX);
+                        ap[f] = abase[f] + min(r, r - (uint32_t)(NRX * RPX));
+                    } else {
+                        ap[f] += RPX;
+                    }
                 }
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t) o.b[t] = *reinterpret_cast<const float*>(xl + bp + 4 * (nb / NBI * GCI + nb % NBI * 16) + 4 * t);
+#pragma unroll
+            for (int f = 0; f < NMF; ++f) o.a[f] = *reinterpret_cast<const f4*>(ap[f] + 4 * (nb / NBI * XCI + nb % NBI * 16));
         };
-        Row row[NMF == 1 ? 2 : 1];
-        if constexpr (NMF == 1) {
-            fetch(row[0], 0);
+        auto multiply = [&](const Piece& o) {
 #pragma unroll
-            for (int ii = 0; ii < 4; ++ii) {
-                if (ii < 3) fetch(row[(ii + 1) & 1], ii + 1);
-                __builtin_amdgcn_sched_barrier(0);
-                multiply(row[ii & 1]);
-                __builtin_amdgcn_sched_barrier(0);
+            for (int f = 0; f < NMF; ++f) {
+                const float a0 = o.a[f].x, a1 = o.a[f].y, a2 = o.a[f].z, a3 = o.a[f].w;
+                acc[f][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, o.b[0], acc[f][0], 0, 0, 0);
+                acc[f][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, o.b[1], acc[f][1], 0, 0, 0);
+                acc[f][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(a2, o.b[2], acc[f][2], 0, 0, 0);
+                acc[f][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(a3, o.b[3], acc[f][3], 0, 0, 0);
             }
-        } else {
+        };
+        Piece pc[kAhead + 1];
 #pragma unroll
-            for (int ii = 0; ii < 4; ++ii) {
-                fetch(row[0], ii);
-                multiply(row[0]);
-            }
+        for (int p = 0; p < kAhead; ++p) fetch(pc[p], p);
+#pragma unroll
+        for (int p = 0; p < 4 * NB; ++p) {
+            if (p + kAhead < 4 * NB) fetch(pc[(p + kAhead) % (kAhead + 1)], p + kAhead);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(pc[p % (kAhead + 1)]);
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
-    // ---- ticks: group gi of unit u is in place; the products follow once XG groups of the unit are
-    int xslot = 0, gslot = 0, par = 1;   // (gslot: ring row)
-    for (int u = u0; u < u1; ++u) {
-        const int band = u / g.ncolt % g.nbands;
-        const int ng = (min(g.BR, g.OH - band * g.BR) + 4) / 4 + XG - 1;
-        for (int gi = 0; gi < ng; ++gi) {
-            lds_barrier();
-            const int xn = xslot + 1 == XG + 1 ? 0 : xslot + 1, gn = gslot + 4 >= NRG ? gslot + 4 - NRG : gslot + 4;
-            const bool mul = gi >= XG - 1;
-            if (wv < CS / 2 && mul) compute(xslot, gslot);
-            if (par) {   // (uniform)
-                commit(bx[1], bg[1], xn, gn);
-                issue(bx[1], bg[1]);
-            } else {
-                commit(bx[0], bg[0], xn, gn);
-                issue(bx[0], bg[0]);
+    // ---- ticks: group gi of a unit is in place; the products follow once XG groups of the unit are
+    int xslot = 0, gslot = 0, gi = 0, u = u0, ng = steps(band);   // (gslot: ring row)
+    auto tick = [&](f4 (&dx)[NLX], f4& dg) {   // (one past the last unit's: zeros into the rings)
+        lds_barrier();
+        if (gi % kFlush == 0) flush();   // (short chains of additions, however many units a workgroup takes)
+        const int xn = xslot + 1 == XG + 1 ? 0 : xslot + 1, gn = gslot + 4 >= NRG ? gslot + 4 - NRG : gslot + 4;
+        const bool mul = gi >= XG - 1 && u < u1;
+        if (wv < CS / 2 && mul) compute(xslot, gslot);
+        commit(dx, dg, xn, gn);
+        issue(dx, dg);
+        if (wv >= CS / 2 && mul) compute(xslot, gslot);
+        xslot = xn, gslot = gn;
+        if (++gi == ng) {
+            if (++ct == g.ncolt) {
+                ct = 0;
+                if (++band == g.nbands) band = 0;
             }
-            if (wv >= CS / 2 && mul) compute(xslot, gslot);
-            xslot = xn, gslot = gn, par ^= 1;
+            gi = 0, ng = steps(band), ++u;
         }
-    }
+    };
+    // (the two buffers by name and no way out between them: the compiler can then tell which requests are the newest, and a
+    // commit waits for its own alone)
+    do {
+        tick(bx[1], bg[1]);
+        tick(bx[0], bg[0]);
+    } while (u < u1);
+    flush();
     // ---- taps through LDS: [tap][channel], then 16-byte stores
     lds_barrier();
     float* const tl = reinterpret_cast<float*>(xl);
 #pragma unroll
     for (int f = 0; f < NMF; ++f) {
-        const f4 s = (acc[f][0] + acc[f][1]) + (acc[f][2] + acc[f][3]);
-        const float e[4] = {s.x, s.y, s.z, s.w};
+        const float e[4] = {sum[f].x, sum[f].y, sum[f].z, sum[f].w};
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int mi = 16 * f + 4 * kg + r, u = 2 * (mi / NBV) + du, v = 8 * (mi % NBV) + dv;
@@ -311,21 +356,36 @@ inline WgF32Plan wgrad_f32t_plan(int B, int H, int W, int C, int K, int PH, int 
     const int ni = p.nbi > 2 ? 1 : 4 / p.nbi;
     if ((long long)H * W * C * ni > 0x1fffffffLL || (long long)g.OH * g.OW * C * ni > 0x1fffffffLL) return p;
     g.ncolt = cdiv(g.OW, 16 * p.nbi - 8), g.nslices = cdiv(C, 8);
-    // two workgroups for every compute unit: several units each, or row bands of at least 12 rows (5 where those would not
-    // give every compute unit one: the chain of a band's steps is all there is to wait for)
-    const int want = 512;
-    const long long whole = (long long)cdiv(B, ni) * g.ncolt * g.nslices;
-    g.BR = g.OH;
-    if (whole >= 2 * want) {
-        g.U = (int)(whole / want);
-    } else if (whole < want) {
-        int nb = (int)(want / whole);
-        const int least_rows = whole * (g.OH / 12) >= 256 ? 12 : 5;
-        if (nb > g.OH / least_rows) nb = g.OH / least_rows;
-        if (nb > 1) g.BR = (cdiv(g.OH, nb) + 1 + 3) / 4 * 4 - 1;   // (rows + 1 whole groups of four)
+    // One, two or three workgroups for every compute unit: bands of an image, or several units each; the cheapest by the
+    // cycles of a unit's ticks (with products: 4 rows of the tile by two wavefronts and what the other workgroup's products do
+    // not cover of the staging; without: 800) and of the start-up (9000, half for each further round), the fewer workgroups
+    // where they tie.  As one of a pair, which is how a block runs it, a problem leaves the compute units that it does not fill
+    // to the other, so that half of its price is its work and half its longest unit (us of the pair, two workgroups each -> by
+    // this rule: [32,56,56,64] filter 13 62.9 -> 55.6, [16,28,28,96] filter 9 29.8 -> 27.0, [64,40,40,32] filter 9 75 -> 63).
+    // The same plan by itself and in a pair: the results are then the same to the bit.
+    const int units = cdiv(B, ni) * g.ncolt, nmf = ((K + 1) / 2 * ((K + 7) / 8) + 15) / 16, xg = (4 + 2 * ((K + 1) / 2 - 1) + 3) / 4;
+    const int held = 8 * (wg_f32t_chx(K, p.nbi, ni) + wg_f32t_chg(p.nbi, ni)) <= 80 * 1024 ? 2 : 1;
+    double least_cost = -1;
+    for (int n = 1; n <= 3; ++n) {
+        int c = 256 * n / g.nslices, br = g.OH, u = 1;   // chunks of a slice
+        if (c < 1) c = 1;
+        if (c > units) {
+            int nb = c / units;
+            if (nb > cdiv(g.OH, 4)) nb = cdiv(g.OH, 4);
+            if (nb > 1) br = (cdiv(g.OH, nb) + 1 + 3) / 4 * 4 - 1;   // (rows + 1 whole groups of four)
+        } else {
+            u = cdiv(units, c);
+        }
+        const int nbands = cdiv(g.OH, br), chunks = cdiv(units * nbands, u);
+        const long long each = cdiv((long long)chunks * g.nslices, 256);   // workgroups of a compute unit
+        const double fill = (double)((long long)chunks * g.nslices) / 256;
+        const double cost = 0.5 * (each + (fill > 0.8 ? fill : 0.8)) * u * (((br + 4) / 4) * (1024 * p.nbi * ni * nmf + 400) + (xg - 1) * 800) +
+                            4500.0 * (1 + cdiv(each, held));
+        if (least_cost < 0 || cost < 0.98 * least_cost) least_cost = cost, g.BR = br, g.U = u;
     }
+    if (const char* e = tune_env("PDW_WGF")) sscanf(e, "%d,%d", &g.BR, &g.U);
     g.nbands = cdiv(g.OH, g.BR);
-    g.units = cdiv(B, ni) * g.ncolt * g.nbands;
+    g.units = units * g.nbands;
     p.nchunks = cdiv(g.units, g.U);
     p.ok = (long long)p.nchunks * g.nslices <= 0x7fffffffLL;
     return p;
@@ -359,9 +419,9 @@ int launch_wgrad_f32t(const void* x, const void* gy, void* dw, void* ws, int B, 
 }
 
 // The weight gradients of two problems (a block's scales) in one grid, each in the tile of its plan: neither depends on the
-// other, and at the sizes where one of them leaves compute units without work the launch takes as long as the longer one
-// ([2,32,32,32] and its half scale, filter 7, us: 10.6 + 12.4 -> 12.6; [3,57,61,100], filter 15: 25.2 + 12.0 -> 26.0;
-// [32,56,56,64], filter 13, where both fill the chip: 57.5 + 25.6 -> 76.1).
+// other, and where one of them leaves compute units without work the launch takes as long as the longer one (us with the
+// summations, at the start of both and now: [2,32,32,32] and its half scale, filter 7, 16.1 -> 13.8; [3,57,61,100], filter 15,
+// 29.9 -> 23.6; [32,56,56,64], filter 13, 77 -> 55.6; [4,64,64,576], filter 13, 126.5 -> 106.7).
 struct WgF32Problem {
     const float *x, *gy;
     float* part;
