@@ -7,7 +7,12 @@
 //     B[(r, 4j+g)][n]       = window[r][4n + 4j + g]      64 consecutive floats of a staged row: one conflict-free LDS read
 // A window row belongs to up to PER = ceil(IC/4) patch rows, whose accumulators are all live: a B operand is read once and
 // feeds PER products of 32 cycles each, so the matrix pipe is what bounds the kernel (LDS is under 10 % busy), a row
-// is dead after its step, and the window in LDS is two groups of four rows whatever the filter (20 KB).
+// is dead after its step, and the window in LDS is two groups of four rows whatever the filter (20 KB).  Vector instructions do
+// not overlap with fp32 products (measured with products by one wavefront of a SIMD and additions by another: 124 and 172 us
+// alone, 289 together), so what the staging computes per thread is added to the products' time: offsets are those of a
+// workgroup plus a scalar row offset wherever all rows of a group exist, and the accumulators rotate by the products' own
+// addend operand.  A step in which all accumulators are live runs without a branch, the products of a row alternating
+// between them.
 //
 // A workgroup (8 wavefronts, one channel each) owns a band of output rows x 4 NPC columns x NI images of 8 channels.  A step is
 // four window rows: the wavefronts multiply them, commit the next four from registers (16 bytes = 4 channels of a pixel,
@@ -15,8 +20,9 @@
 // (through a pixel-major tile in LDS, 16 bytes a thread).  One barrier a step; wavefronts 0-3 multiply first and 4-7 last, so
 // that of a SIMD's two wavefronts one always feeds the matrix pipe.
 //
-// Measured at [32,56,56,64] against the vector-ALU kernel (dwconv_tiled.h): filter 9 28 us for 37, 13 40 for 77, 17 57 for 90
-// (the products of filter 13 alone 24); [32,28,28,64]: filter 13 15 for 41; [4,112,112,128]: filter 9 28 for 49, 13 39 for 75.
+// Measured at [32,56,56,64], filter 13: 35.1 us (36.7 with the conditions per thread and per product; the products alone 27 at
+// the clock that they leave, vector-ALU kernel (dwconv_tiled.h) 77); [3,57,61,100] filter 15 14.9 (15.9); [8,112,112,48] filter
+// 17 38.3 (41.0); [1,5,90,36] filter 17 8.5 (9.7).
 //
 // ADD: the input gradient of a tensor that was also average-pooled to (AH, AW): y += the pool's gradient, from the one bin of
 // a pixel where the pool halved both extents (1), gathered from the at most 2 x 2 bins that a pixel lies in (2).
@@ -80,7 +86,7 @@ __device__ __forceinline__ void dwconv_f32_body(const float* __restrict__ x, con
     extern __shared__ uint32_t smem[];
     char* const xl = reinterpret_cast<char*>(smem);
     char* const r2 = xl + NI * CS * CHP;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     int bid = xcd_remap(blk, nblk);
     const int sl = bid % g.nslices;
     bid /= g.nslices;
@@ -101,10 +107,10 @@ __device__ __forceinline__ void dwconv_f32_body(const float* __restrict__ x, con
         wval[i] = *reinterpret_cast<const f4*>(w + (idx >> 1) * g.C + min(c0 + 4 * (idx & 1), g.C - 4));
     }
     // ---- staging: offsets past the descriptor's end (images beyond the batch, the markers) read as zero
-    constexpr uint32_t kNoCol = 0x40000000u, kNoRow = 0x80000000u;
+    constexpr uint32_t kNoRow = 0x80000000u;
     const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float*>(x + (long long)b0 * img_in), (short)0, (int)(min(NI, g.B - b0) * img_in * 4), 0x00020000);
-    uint32_t icol[NLD];
+    uint32_t xoff[NLD];   // bytes from the group's first row, or kNoRow
     int irow[NLD], idst[NLD];
 #pragma unroll
     for (int l = 0; l < NLD; ++l) {
@@ -112,25 +118,33 @@ __device__ __forceinline__ void dwconv_f32_body(const float* __restrict__ x, con
         irow[l] = (idx >> 1) / WCOLS / NI;
         const int ic = ocol0 - g.PW + col;
         const bool ok = irow[l] < 4 && c0 + 4 * q < g.C && ic >= 0 && ic < g.W;
-        icol[l] = ok ? ((uint32_t)img * (uint32_t)img_in + (uint32_t)(ic * g.C + c0 + 4 * q)) * 4u : kNoCol;
+        xoff[l] = ok ? ((uint32_t)img * (uint32_t)img_in + (uint32_t)((irow[l] * g.W + ic) * g.C + c0 + 4 * q)) * 4u : kNoRow;
         idst[l] = (img * CS + 4 * q) * CHP + (irow[l] & 3) * RP + col * 4;
     }
     f4 buf[2][NLD];
     auto issue = [&](f4 (&bf)[NLD], int s) {
+        const int ir0 = orow0 - g.PH + 4 * s, row_at = ir0 * g.W * g.C * 4;
+        uint32_t xo[NLD];
+        int so = row_at;
 #pragma unroll
-        for (int l = 0; l < NLD; ++l) {
-            const int ir = orow0 - g.PH + 4 * s + irow[l];
-            const uint32_t r = s < nsteps && ir >= 0 && ir < g.H ? (uint32_t)(ir * g.W * g.C) * 4u : kNoRow;
-            bf[l] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(xrsrc, (int)(r + icol[l]), 0, 0));
+        for (int l = 0; l < NLD; ++l) xo[l] = xoff[l];
+        if (s >= nsteps || ir0 < 0 || ir0 + 3 >= g.H) {   // (uniform; where all four rows exist, nothing to compute per thread)
+            so = 0;
+#pragma unroll
+            for (int l = 0; l < NLD; ++l) {
+                const bool ok = (int)xoff[l] >= 0 && s < nsteps && (unsigned)(ir0 + irow[l]) < (unsigned)g.H;
+                xo[l] = ok ? xoff[l] + (uint32_t)row_at : kNoRow;
+            }
         }
+#pragma unroll
+        for (int l = 0; l < NLD; ++l) bf[l] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(xrsrc, (int)xo[l], so, 0));
     };
-    auto commit = [&](const f4 (&bf)[NLD], int s) {
-        char* const half = xl + (s & 1) * 4 * RP;
+    auto commit = [&](const f4 (&bf)[NLD], int half) {   // half of the window: 0 or 1
 #pragma unroll
         for (int l = 0; l < NLD; ++l) {
-            if (irow[l] < 4) {
+            if (wv * 64 + l * NT < 8 * NI * WCOLS && ((l + 1) * NT <= 8 * NI * WCOLS || irow[l] < 4)) {
                 const float e0 = bf[l].x, e1 = bf[l].y, e2 = bf[l].z, e3 = bf[l].w;
-                char* d = half + idst[l];
+                char* d = xl + idst[l] + half * 4 * RP;
                 *reinterpret_cast<float*>(d) = e0;
                 *reinterpret_cast<float*>(d + CHP) = e1;
                 *reinterpret_cast<float*>(d + 2 * CHP) = e2;
@@ -170,7 +184,15 @@ __device__ __forceinline__ void dwconv_f32_body(const float* __restrict__ x, con
     }
     lds_barrier();   // (the table's space becomes the result tiles)
     const int pimg = ln / NPC, pc = ln % NPC;
-    const char* const xb = xl + (pimg * CS + wv) * CHP + (4 * pc + kg) * 4;
+    // Rows 0 .. 7 of the window at a lane, in three registers: as offsets from one they are out of a paired read's reach, and
+    // each read would add its own (vector instructions do not overlap with fp32 products: 124 us of products and 172 us of
+    // additions by another wavefront take 289 us).
+    uint32_t xb[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        xb[i] = (uint32_t)((pimg * CS + wv) * CHP + (4 * pc + kg) * 4 + 3 * i * RP);
+        asm("" : "+v"(xb[i]));
+    }
     // result of a lane: patch ln, row kg, columns 4 pc .. + 3 (the four registers)
     char* const olw = r2 + (pimg * 4 + kg) * OROWP + pc * (4 * 32 + 4) + wv * 4;
     const int sq = tid & 1, scol = (tid >> 1) % TW, srow = (tid >> 1) / TW % 4, simg = (tid >> 1) / TW / 4;
@@ -178,22 +200,24 @@ __device__ __forceinline__ void dwconv_f32_body(const float* __restrict__ x, con
     const char* const olr = r2 + (simg * 4 + srow) * OROWP + scol * 32 + (scol >> 2) * 4 + 16 * sq;
     const __amdgpu_buffer_rsrc_t yrsrc = __builtin_amdgcn_make_buffer_rsrc(
         y + (long long)b0 * img_out, (short)0, (int)(min(NI, g.B - b0) * img_out * 4), 0x00020000);
-    const uint32_t ycol = (uint32_t)simg * (uint32_t)img_out + (uint32_t)((ocol0 + scol) * g.C + c0 + 4 * sq);
+    const uint32_t yoff = s_ok ? ((uint32_t)simg * (uint32_t)img_out + (uint32_t)((srow * g.OW + ocol0 + scol) * g.C + c0 + 4 * sq)) * 4u : kNoRow;
     __amdgpu_buffer_rsrc_t arsrc = xrsrc;
     int jb0 = 0;
+    uint32_t aoff = 0;
     float wj0 = 0.f, wj1 = 0.f, wi0 = 0.f, wi1 = 0.f;
     f4 addv[ADD == 2 ? 4 : 1];
     if constexpr (ADD) {
         arsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(add + (long long)b0 * g.AH * g.AW * g.C), (short)0,
                                                   (int)((long long)min(NI, g.B - b0) * g.AH * g.AW * g.C * 4), 0x00020000);
         if constexpr (ADD == 2) pool_bins(min(ocol0 + scol, g.OW - 1), g.OW, g.AW, jb0, wj0, wj1);
-        else jb0 = (ocol0 + scol) >> 1;
+        else aoff = s_ok ? ((uint32_t)((simg * g.AH + (srow >> 1)) * g.AW + ((ocol0 + scol) >> 1)) * (uint32_t)g.C + (uint32_t)(c0 + 4 * sq)) * 4u : kNoRow;
     }
     auto add_fetch = [&](int pr) {   // the bins of patch row pr's pixels
         if constexpr (ADD == 1) {
-            const bool ok = s_ok && pr >= 0 && 4 * pr + srow < rows_valid;
-            const uint32_t off = ok ? ((uint32_t)((simg * g.AH + ((orow0 + 4 * pr + srow) >> 1)) * g.AW + jb0) * (uint32_t)g.C + (uint32_t)(c0 + 4 * sq)) * 4u : kNoRow;
-            addv[0] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(arsrc, (int)off, 0, 0));
+            uint32_t o = aoff;
+            if (pr < 0 || 4 * pr + 3 >= rows_valid) o = pr >= 0 && 4 * pr + srow < rows_valid ? o : kNoRow;
+            const int at = pr >= 0 ? ((orow0 + 4 * pr) >> 1) * g.AW * g.C * 4 : 0;
+            addv[0] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(arsrc, (int)o, at, 0));
         } else if constexpr (ADD == 2) {
             int ib0;
             const int row = orow0 + 4 * pr + srow;
@@ -223,83 +247,86 @@ __device__ __forceinline__ void dwconv_f32_body(const float* __restrict__ x, con
             for (int e = 0; e < 4; ++e)
                 v[e] += fmaf(k11, addv[3][e], fmaf(k10, addv[2][e], fmaf(k01, addv[1][e], k00 * addv[0][e])));
         }
-        const bool ok = s_ok && pr >= 0 && 4 * pr + srow < rows_valid;
-        const uint32_t off = ok ? (ycol + (uint32_t)((orow0 + 4 * pr + srow) * g.OW * g.C)) * 4u : kNoRow;
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, f4{v[0], v[1], v[2], v[3]}), yrsrc, (int)off, 0, 0);
+        uint32_t o = yoff;
+        if (pr < 0 || 4 * pr + 3 >= rows_valid) o = pr >= 0 && 4 * pr + srow < rows_valid ? o : kNoRow;   // (uniform)
+        const int at = pr >= 0 ? (orow0 + 4 * pr) * g.OW * g.C * 4 : 0;   // (no scalar offset in a 16-byte store: see dwconv_tz.h)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, f4{v[0], v[1], v[2], v[3]}), yrsrc, (int)(o + (uint32_t)at), 0, 0);
     };
+    // acc[q]: the patch row whose q-th group of window rows was multiplied last.  Step s multiplies window rows 4 s .. 4 s + 3
+    // for patch rows s - q and finishes patch row s - PER + 1; every patch row moves one accumulator up in its first product.
     f4 acc[PER];
 #pragma unroll
     for (int q = 0; q < PER; ++q) acc[q] = f4{0.f, 0.f, 0.f, 0.f};
-    // step s multiplies window rows 4 s .. 4 s + 3 (for patch rows s - PER + 1 .. s) and finishes patch row s - PER + 1
-    auto compute = [&](int ps, int s) {   // ps = s mod PER
-        const char* rowp = xb + (s & 1) * 4 * RP;
-        float bv[2][JB];   // the next row's operands are read while a row is multiplied
-        auto fetch = [&](int r) {
+    auto compute = [&](int half, int s) {
+        auto fetch = [&](float (&bv)[JB], int r) {
+            const int row = half * 4 + r;
 #pragma unroll
-            for (int j = 0; j < JB; ++j) bv[r & 1][j] = *reinterpret_cast<const float*>(rowp + r * RP + 16 * j);
+            for (int j = 0; j < JB; ++j) bv[j] = *reinterpret_cast<const float*>(xl + xb[row / 3] + row % 3 * RP + 16 * j);
         };
-        fetch(0);
+        if (s >= PER - 1 && s < npr) {   // (uniform) all of them: row by row, the next row's operands read meanwhile
+            float bv[2][JB];
+            fetch(bv[0], 0);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            if (r < 3) fetch(r + 1);
+            for (int r = 0; r < 4; ++r) {
+                if (r < 3) fetch(bv[(r + 1) & 1], r + 1);
 #pragma unroll
-            for (int q = 0; q < PER; ++q) {
-                if (4 * q + r >= IC) continue;
-                if (s - q >= 0 && s - q < npr) {   // (uniform)
-                    f4& a = acc[(ps - q + PER) % PER];
+                for (int j = 0; j < JB; ++j) {
 #pragma unroll
-                    for (int j = 0; j < JB; ++j) a = __builtin_amdgcn_mfma_f32_16x16x4f32(A[4 * q + r < IC ? 4 * q + r : 0][j], bv[r & 1][j], a, 0, 0, 0);
+                    for (int q = PER - 1; q >= 0; --q) {
+                        if (4 * q + r >= IC) continue;
+                        const f4 c = r == 0 && j == 0 ? (q > 0 ? acc[q > 0 ? q - 1 : 0] : f4{0.f, 0.f, 0.f, 0.f}) : acc[q];
+                        acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[4 * q + r < IC ? 4 * q + r : 0][j], bv[r & 1][j], c, 0, 0, 0);
+                    }
                 }
             }
+        } else {   // the first and last patch rows: one after the other
+#pragma unroll
+            for (int q = PER - 1; q >= 0; --q) {
+                if (s < q || s - q >= npr) continue;   // (uniform)
+                f4 a = q > 0 ? acc[q > 0 ? q - 1 : 0] : f4{0.f, 0.f, 0.f, 0.f};
+                float bv[2][JB];
+                fetch(bv[0], 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (4 * q + r >= IC) continue;
+                    if (r < 3) fetch(bv[(r + 1) & 1], r + 1);
+#pragma unroll
+                    for (int j = 0; j < JB; ++j)
+                        a = __builtin_amdgcn_mfma_f32_16x16x4f32(A[4 * q + r < IC ? 4 * q + r : 0][j], bv[r & 1][j], a, 0, 0, 0);
+                }
+                acc[q] = a;
+            }
         }
-        f4& done = acc[(ps + 1) % PER];
         const int pr = s - PER + 1;
-        if (pr >= 0) {
+        if (pr >= 0 && pr < npr) {
             char* d = olw + (pr & 1) * OLB;
-            const float e0 = done.x, e1 = done.y, e2 = done.z, e3 = done.w;
+            const float e0 = acc[PER - 1].x, e1 = acc[PER - 1].y, e2 = acc[PER - 1].z, e3 = acc[PER - 1].w;
             *reinterpret_cast<float*>(d) = e0;
             *reinterpret_cast<float*>(d + 32) = e1;
             *reinterpret_cast<float*>(d + 64) = e2;
             *reinterpret_cast<float*>(d + 96) = e3;
         }
-        done = f4{0.f, 0.f, 0.f, 0.f};
     };
-    auto stage = [&](int par, int s) {   // par: the buffer that the rows of step s came from
+    auto step = [&](f4 (&bf)[NLD], int half, int s) {   // bf: holds the rows of step s + 1
+        lds_barrier();   // the rows of step s are in place, and everybody is done with those of s - 1
+        if (wv < 4 && s < nsteps) compute(half, s);
         store(s - PER);                      // (finished by step s - 1)
         add_fetch(s - PER + 1);              // for the next step's store
-        commit(buf[par ^ 1], s + 1);
-        issue(buf[par ^ 1], s + 3);
+        commit(bf, half ^ 1);
+        issue(bf, s + 3);
+        if (wv >= 4 && s < nsteps) compute(half, s);
     };
-    // trips of PER steps: accumulators and buffers by constant index (an odd trip leaves the two buffers swapped)
     add_fetch(-1);
-    bool left = false;
-    for (int s0 = 0; !left; s0 += PER) {
-#pragma unroll
-        for (int t = 0; t < PER; ++t) {
-            const int s = s0 + t;
-            if (s >= nsteps) {   // (uniform)
-                left = true;
-                break;
-            }
-            lds_barrier();   // the rows of step s are in place, and everybody is done with those of s - 1
-            if (wv < 4) {
-                compute(t, s);
-                stage(t & 1, s);
-            } else {
-                stage(t & 1, s);
-                compute(t, s);
-            }
-        }
-        if constexpr (PER % 2 == 1) {
-#pragma unroll
-            for (int l = 0; l < NLD; ++l) {
-                const f4 v = buf[0][l];
-                buf[0][l] = buf[1][l], buf[1][l] = v;
-            }
-        }
-    }
+    // (the two buffers by name and no way out between them: the compiler can then tell which requests are the newest, and a
+    // commit waits for its own alone)
+    int s = 0;
+    do {
+        step(buf[1], 0, s);
+        step(buf[0], 1, s + 1);
+        s += 2;
+    } while (s < nsteps);
     lds_barrier();
-    store(nsteps - PER);
+    if (s == nsteps) store(nsteps - PER);   // (else the step past the last did)
 }
 
 // Register bound: two workgroups on a compute unit where the filter's operands leave room, so that one's start-up
@@ -348,11 +375,10 @@ int f32t_band(long long per_band, int OH) {
 }
 
 // Where the vector-ALU kernel (dwconv_tiled.h) stays, unless the pooled gradient rides here (which saves a pass over y):
-// - filters 3 and 7 once the tensor is more than a round of workgroups ([32,28,28,64]: 8.3 and 11.1 us here, 7.4 and 10.3
-//   there; [40,112,112,64]: 86 and 98, 69 and 87; [4,16,37,32]: 5.6 and 6.8, 5.9 and 7.7), 5 there unless the images fill
-//   the tiles ([40,70,70,64]: 32 here, 45 there);
-// - filters 9 and 11 on images that leave half of a tile's columns empty ([100,7,7,1152] filter 9: 66 here, 47 there; filter
-//   13 130 and 144).
+// - filters 3 and 7 once the tensor is more than a round of workgroups ([40,14,14,256] filter 7: 14.5 us here, 11.9 there), whose
+//   values that are not finite reach no further than the filter there; 5 there unless the images fill the tiles
+//   ([40,70,70,64]: 30 here, 45 there);
+// - filters 9 and 11 on images that leave half of a tile's columns empty ([100,7,7,1152] filter 9: 61 here, 46 there).
 template <int K>
 bool f32t_pays(long long outputs, int OW, int npc, bool add) {
     if (K >= 13 || add) return true;
