@@ -444,9 +444,14 @@ template <typename T, int KW>
 static int launch_best(const void* x, const void* w, void* y, int B, int H, int W, int C, int KH, int PH, int PW,
                        bool flip, hipStream_t s) {
     const int OH = H + 2 * PH - KH + 1, OW = W + 2 * PW - KW + 1;
-    const TiledPlan p0 = plan_tiled<T, KW, 8, 2, 32>(OH, OW, KH, B, C);
-    const TiledPlan p1 = plan_tiled<T, KW, 14, 1, 32>(OH, OW, KH, B, C);
-    const TiledPlan p2 = plan_tiled<T, KW, 14, 2, 32>(OH, OW, KH, B, C);
+    // (the search takes 25 to 100 us, two to six times the kernel: kept by shape.  [32,28,28,64] filter 3 46 -> 8 us a call,
+    // [32,56,56,64] filter 7 45 -> 24)
+    using Key = std::array<int, 5>;
+    static PlanCache<Key, std::array<TiledPlan, 3>> cache;
+    const auto [p0, p1, p2] = cache.get(Key{OH, OW, KH, B, C}, [&] {
+        return std::array<TiledPlan, 3>{plan_tiled<T, KW, 8, 2, 32>(OH, OW, KH, B, C), plan_tiled<T, KW, 14, 1, 32>(OH, OW, KH, B, C),
+                                        plan_tiled<T, KW, 14, 2, 32>(OH, OW, KH, B, C)};
+    });
     int pick = -1;
     double best = -1;
     const TiledPlan* ps[3] = {&p0, &p1, &p2};

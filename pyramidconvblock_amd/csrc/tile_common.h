@@ -1,9 +1,30 @@
 // Device helpers shared by the LDS-tiled depthwise-convolution kernels: the 16-bit pair
 // packing, the dot2 wrappers, the XCD-aware work order and the tile staging routine.
 #pragma once
+#include <array>
+#include <map>
+#include <mutex>
+
 #include "common.h"
 
 namespace pdw {
+
+// Launch plans by shape, for planners whose search costs more than a kernel (bounded; any thread).
+template <typename Key, typename Plan>
+class PlanCache {
+public:
+    template <typename F>
+    Plan get(const Key& key, F make) {
+        std::lock_guard<std::mutex> lock(mu_);
+        if (auto it = plans_.find(key); it != plans_.end()) return it->second;
+        if (plans_.size() >= kPlanCacheMax) plans_.clear();
+        return plans_[key] = make();
+    }
+
+private:
+    std::mutex mu_;
+    std::map<Key, Plan> plans_;
+};
 
 template <typename T>
 struct PackOf {
