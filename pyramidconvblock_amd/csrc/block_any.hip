@@ -338,18 +338,25 @@ int backward(const Shape& s, const Saved& v, const BwdWork& g, const void* gy, c
     const int r = dwconv_bwd3_launch(g.gcf, w_dw0, s.exact ? g.dxp : nullptr, g.da, v.a, gw_dw0, g.ws_w0, v.xp, g.gch, gw_dw1, g.ws_w1,
                                      s.B, s.H, s.W, s.h, s.w, s.I, s.K, dt, st, nullptr, waiting ? &mean : nullptr);
     if (r != 0 && r != -1) return r;
+    // in fp32 both weight gradients, with the mean branch's backward, and then the full scale's input gradient
+    int pair = -1;
+    if (r == -1 && dt == kF32)
+        pair = dwconv_wgrad_f32t_pair_launch(v.a, g.gcf, gw_dw0, g.ws_w0, s.H, s.W, v.xp, g.gch, gw_dw1, g.ws_w1, s.h, s.w, s.B,
+                                             s.I, s.K, pad, st, waiting ? &mean : nullptr);
+    if (pair != 0 && pair != -1) return pair;
     if (waiting) {
         reduce_defer_compact(0, 0);
-        if (int e = r == 0 ? mean_bwd_defer(mean, gb0, gb1, gw_pool, dt, st) : mean_bwd_launch(mean, gb0, gb1, gw_pool, dt, st)) return e;
+        if (int e = r == 0 || pair == 0 ? mean_bwd_defer(mean, gb0, gb1, gw_pool, dt, st) : mean_bwd_launch(mean, gb0, gb1, gw_pool, dt, st)) return e;
         reduce_defer_compact(seg, val);
     }
     if (r == 0) {
         if (!s.exact)
             if (int e = avgpool_bwd_launch(g.dxp, g.da, s.B, s.H, s.W, s.I, s.h, s.w, 1, dt, st)) return e;
     } else {
-        if (int e = pdw_dwconv_wgrad_pair(v.a, g.gcf, gw_dw0, g.ws_w0, g.b_w0, s.H, s.W, v.xp, g.gch, gw_dw1, g.ws_w1, g.b_w1,
-                                          s.h, s.w, s.B, s.I, s.K, dt, stream))
-            return e;
+        if (pair == -1)
+            if (int e = pdw_dwconv_wgrad_pair(v.a, g.gcf, gw_dw0, g.ws_w0, g.b_w0, s.H, s.W, v.xp, g.gch, gw_dw1, g.ws_w1, g.b_w1,
+                                              s.h, s.w, s.B, s.I, s.K, dt, stream))
+                return e;
         if (int e = pdw_dwconv_dgrad_addpool(g.gcf, w_dw0, g.dxp, g.da, s.B, s.H, s.W, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, s.h,
                                              s.w, dt, stream))
             return e;

@@ -27,6 +27,7 @@
 
 #include "common.h"
 #include "kernels.h"
+#include "mean_any.h"
 #include "tile_common.h"
 
 namespace pdw {
@@ -430,7 +431,8 @@ struct WgF32Problem {
 };
 struct WgF32Pair {
     WgF32Problem p[2];
-};
+    MeanJob mean;   // workgroups behind both problems: the backward of the block's mean branch, which needs nothing of this
+};                  // launch and whose result is read after it (by a launch of its own 5.1 us at [32,56,56,128], 3.1 at [2,32,32,64])
 
 // Tiles that leave room for two workgroups on a compute unit: the pair is for those.
 template <int K>
@@ -443,6 +445,10 @@ constexpr bool wg_f32t_pairs(int nbi) {
 
 template <int K>
 __global__ __launch_bounds__(512, 4) void dwconv_wgrad_f32t_pair_k(const WgF32Pair a) {
+    if ((int)blockIdx.x >= a.p[0].n + a.p[1].n) {
+        extern __shared__ uint32_t smem[];
+        return mean_bwd_body<float, 512>(a.mean, (int)blockIdx.x - a.p[0].n - a.p[1].n, reinterpret_cast<float*>(smem));
+    }
     const bool first = (int)blockIdx.x < a.p[0].n;
     const float *x = first ? a.p[0].x : a.p[1].x, *gy = first ? a.p[0].gy : a.p[1].gy;
     float* const part = first ? a.p[0].part : a.p[1].part;
@@ -461,7 +467,7 @@ __global__ __launch_bounds__(512, 4) void dwconv_wgrad_f32t_pair_k(const WgF32Pa
 // -1: not covered (the caller makes two launches).
 template <int K>
 int launch_wgrad_f32t_pair(const void* x0, const void* gy0, void* dw0, void* ws0, int H0, int W0, const void* x1, const void* gy1,
-                           void* dw1, void* ws1, int H1, int W1, int B, int C, int P, hipStream_t s) {
+                           void* dw1, void* ws1, int H1, int W1, int B, int C, int P, hipStream_t s, const MeanJob* mean) {
     const WgF32Plan plan[2] = {wgrad_f32t_plan(B, H0, W0, C, K, P, P), wgrad_f32t_plan(B, H1, W1, C, K, P, P)};
     const void *const x[2] = {x0, x1}, *const gy[2] = {gy0, gy1};
     void *const dw[2] = {dw0, dw1}, *const ws[2] = {ws0, ws1};
@@ -481,6 +487,12 @@ int launch_wgrad_f32t_pair(const void* x0, const void* gy0, void* dw0, void* ws0
                             : p.nbi == 2 ? WgF32Shape<K, 2, 2>::lds_bytes
                                          : WgF32Shape<K, 1, 4>::lds_bytes;
         if (need > lds) lds = need;
+    }
+    if (mean) {
+        const size_t need = mean_lds(mean->D, 512);
+        if (need > 80 * 1024) return -1;   // (two workgroups on a compute unit)
+        if (need > lds) lds = need;
+        a.mean = *mean, n += (long long)mean->B * mean_slices(mean->D);
     }
     if (n > 0x7fffffffLL) return -1;
     static std::once_flag once;

@@ -137,7 +137,7 @@ int dwconv_wgrad_pair_launch(const void* xa, const void* gya, void* dwa, void* w
                              const void* gyb, void* dwb, void* wsb, int Hb, int Wb, int B, int C, int K, int PH, int PW,
                              int dtype, hipStream_t s) {
     if (dtype == kF32 && PH == K / 2 && PW == PH)
-        return dwconv_wgrad_f32t_pair_launch(xa, gya, dwa, wsa, Ha, Wa, xb, gyb, dwb, wsb, Hb, Wb, B, C, K, PH, s);
+        return dwconv_wgrad_f32t_pair_launch(xa, gya, dwa, wsa, Ha, Wa, xb, gyb, dwb, wsb, Hb, Wb, B, C, K, PH, s, nullptr);
     if (!wgrad_mfma_enabled(dtype) || tune_env("PDW_NO_WGRAD_PAIR")) return -1;
     if (wgrad_tz_enabled() && dwconv_wgrad_tz_workspace(B, Ha, Wa, C, K, PH, PW, dtype) &&
         dwconv_wgrad_tz_workspace(B, Hb, Wb, C, K, PH, PW, dtype)) {
