@@ -111,17 +111,19 @@ struct LaunchPart {
     int total, least;                        // steps of the whole problem; fewest of a run
     std::function<long long(int)> blocks;    // workgroups when cut so
 };
-constexpr double kMeanCost = 5.0;   // us of one of the mean branch's workgroups
+constexpr double kMeanCost = 8.0;   // us of one of the mean branch's workgroups beside these
 
 // (Measured against plans in several rounds that are estimated equal: backward of [128,56,56,64], filter 13, 72.7 us in 252
 // workgroups, 80.2 in 428.  The mean branch's count too: forward of [8,112,112,48], filter 17, 17 us with units left for its 8
-// workgroups, 21.8 without.)
+// workgroups, 21.8 without.  Each of them takes a unit for a whole turn: forward of [32,56,56,64], filter 13, with 32 of them,
+// 15.8 us on 224 workgroups, 18.7 on 268 by a share of 5 us each, which left the last 12 a unit only when the convolutions ended.)
 // Steps per run with which all problems end together, as early as 256 compute units with one workgroup each allow, the mean
 // branch's nmean short workgroups one after another on the units left over; false: they do not fit in one round.
 template <int N>
 inline bool launch_balance(const LaunchPart (&p)[N], int nmean, int (&steps)[N]) {
     auto fits = [&](double t, int (&s)[N]) {
-        double units = nmean * kMeanCost / t;
+        const int turns = t < 2 * kMeanCost ? 1 : (int)(t / kMeanCost);   // of a unit, within the launch
+        double units = (nmean + turns - 1) / turns;
         for (int i = 0; i < N; ++i) {
             const double most = (t - p[i].start) / p[i].step;
             s[i] = most >= p[i].total ? p[i].total : (int)most;
