@@ -168,16 +168,17 @@ int pdw_dwconv_wgrad_pair(const void *x0, const void *gy0, void *dw0, void *work
  * [B,H/2,W/2,C].  Square odd filter, stride 1, padding K/2, even H and W; workspaces as for the two pdw_dwconv_wgrad
  * calls.  Status 3 (nothing launched) when the fused kernel does not cover the case (fp32, C % 16, images narrower than
  * 33 columns...): the caller then makes the three calls.  dx is bitwise that of the separate call; the weight gradients
- * are the same sums taken over other bands of the images (the launch chooses its own band heights: as few bands as fill
- * the chip together with the other two problems), so they can differ from pdw_dwconv_wgrad's in the last bit, and are
+ * are the same sums taken over other pieces of the images (the launch cuts its three problems in its own way, into one
+ * round of the chip where that is possible), so they can differ from pdw_dwconv_wgrad's in the last bit, and are
  * the same from call to call.  Between pdw_reduce_defer_begin/flush the two summations are recorded like any other. */
 int pdw_dwconv_bwd3(const void *gy0, const void *w0, const void *gp, void *dx, const void *x0, void *dw0,
                     void *workspace0, size_t workspace0_bytes, const void *x1, const void *gy1, void *dw1,
                     void *workspace1, size_t workspace1_bytes, int B, int H, int W, int C, int K, int dtype,
                     void *stream);
 /* Host only: the cut pdw_dwconv_bwd3 would choose for these extents (launch planning of the same call sites; no
- * reference counterpart, the Triton grid is fixed at dwconv_triton.py:318-333).  bands[0..2] receive the number of row
- * bands per image of the input gradient, the full scale's and the half scale's weight gradient (each >= 1).  Returns 0,
+ * reference counterpart, the Triton grid is fixed at dwconv_triton.py:318-333).  bands[0..2] receive the number of
+ * pieces per image (rounded up: a piece may span images) of the input gradient, the full scale's and the half scale's
+ * weight gradient (each >= 1).  Returns 0,
  * 3 when pdw_dwconv_bwd3 does not cover the case, 1 on invalid arguments.  Touches no device. */
 int pdw_dwconv_bwd3_plan(int B, int H, int W, int C, int K, int dtype, int *bands);
 
