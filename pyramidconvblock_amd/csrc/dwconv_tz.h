@@ -18,9 +18,11 @@
 // lane) for NM instructions.  That is what makes the kernel a stream: per step and channel 2 LDS reads, 8 MFMAs.
 //
 // A workgroup (8 wavefronts, CS = 8 CPW channels) owns 4 NPC columns of NI images side by side and a run of output rows.  The
-// images of a batch are stacked into one column of rows, `per` rows apart with at least PH rows of zeros between them, and a
-// run starts and ends anywhere (at multiples of 8 rows): as many workgroups as the chip holds at once, whatever the extents,
-// each with one start-up.  The input window is streamed through LDS, channel-major: xl[image][channel][row][column] as 16-bit
+// images of a batch are stacked into one column of rows, `per` rows apart with zeros between them, and a run starts and ends
+// anywhere (at multiples of 8 rows): as many workgroups as the chip holds at once, whatever the extents, each with one
+// start-up.  There are at least PH rows of zeros, and more where the last patch of an image needs them: its operands cover
+// OPR >= K + 3 window rows, of which those beyond the K + 3 (and those below an image's last output) meet zeros of A, and zero
+// times an infinity of the next image would be NaN.  Runs that are parts of one image read nothing of another.  The input window is streamed through LDS, channel-major: xl[image][channel][row][column] as 16-bit
 // values, so that 8 consecutive columns of a channel are 16 contiguous bytes.  Threads load 4 pixels of a row x 8 channels (four
 // 16-byte loads), interleave columns with byte permutes and write 8 bytes per channel; the passes of this copy are requested two
 // ahead and committed only as far as the next step needs.  Results are rounded once, transposed through a small
@@ -78,6 +80,7 @@ struct TzShape {
     static constexpr int NKG = IC * ICB;              // k groups of a patch
     static constexpr int NM = (NKG + 3) / 4;          // MFMAs per patch (group of 16) and channel
     static constexpr int PER = (NM + ICB - 1) / ICB;  // row groups (of 4 rows) an operand ring spans
+    static constexpr int OPR = (4 * NM + ICB - 1) / ICB;  // window rows that a patch's operands cover (those from IC on meet zeros of A)
     static constexpr int RING = PER * ICB;            // operands in the ring
     static constexpr int NI = 16 / NPC;               // images side by side in one instruction
     static constexpr int TW = 4 * NPC;                // output columns of a workgroup
@@ -111,16 +114,21 @@ struct TzShape {
 // 2^32 / d rounded up (0 for 1): n / d = the high half of n times this while n d < 2^32.  (A division costs a wavefront about
 // 150 cycles, and a workgroup cannot request its first rows before it has made a handful.)
 inline uint32_t tz_inverse(int d) { return d == 1 ? 0u : (uint32_t)(((1ULL << 32) + d - 1) / (uint32_t)d); }
+// Rows to the next image for a run that knows its own only: further than it reaches, and the inverse that makes all of its rows
+// lie in image 0 (n * 1 / 2^32).
+constexpr int kTzAlone = 0x40000000;
+constexpr uint32_t kTzAloneInverse = 1;
 __device__ __forceinline__ int tz_quotient(int n, uint32_t inverse) { return inverse ? (int)__umulhi((uint32_t)n, inverse) : n; }
 
 struct TzGeom {
     int B, H, W, C;    // input extents
     int OH, OW;        // output extents
     int PH, PW;        // padding
-    int per;           // rows from one image to the next in the stack of a batch's images (a multiple of 8)
+    int per;           // rows from one image to the next in the stack of a batch's images (a multiple of 8); kTzAlone if rpi
     int run;           // stacked rows of a workgroup (a multiple of 8)
-    int rpi;           // 0: runs follow one another; else they start anew with every image, rpi of them to one
+    int rpi;           // 0: runs follow one another through the stack; else they are parts of an image, rpi of them to one
     int nruns, ncolt, nslices;
+    int part, stack;   // (host) rows that runs by image divide; rows from one image to the next in the stack
     uint32_t per_inv, rpi_inv, ncolt_inv, nslices_inv;   // tz_inverse of these
     int flip;          // 1: 180-degree rotated filter (input gradient)
     int AH, AW;        // extents of the half-resolution addend / pooled output
@@ -181,12 +189,14 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
     const int ct = rest - bid * g.ncolt;
     const int c0 = sl * CS, ocol0 = ct * TW;
     auto images_in = [&](int v) { return tz_quotient(v, g.per_inv); };   // (v >= 0)
-    // the run's output rows: g.run of the stack, without the rows between images at its ends
+    // the run's output rows: a part of an image, or g.run of the stack without the rows between images at its ends
     int b0, orow0, rows_valid;
-    {
-        const int image = g.rpi ? tz_quotient(bid, g.rpi_inv) : 0;
-        const int first = g.rpi ? image * g.per + (bid - image * g.rpi) * g.run : bid * g.run;
-        b0 = g.rpi ? image : images_in(first), orow0 = first - b0 * g.per;
+    if (g.rpi) {
+        const int image = tz_quotient(bid, g.rpi_inv);
+        orow0 = (bid - image * g.rpi) * g.run, rows_valid = min(g.run, g.OH - orow0), b0 = image * NI;
+    } else {
+        const int first = bid * g.run;
+        b0 = images_in(first), orow0 = first - b0 * g.per;
         int end = orow0 + min(g.run, ((g.B + NI - 1) / NI - 1) * g.per + g.OH - first);   // (from image b0's first row on)
         if (orow0 >= g.OH) ++b0, orow0 = 0, end -= g.per;
         if (end <= 0) return;     // (uniform) all of them between two images
@@ -273,7 +283,7 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
         prsrc = __builtin_amdgcn_make_buffer_rsrc(pool + (long long)b0 * g.AH * g.AW * g.C, (short)0,
                                                   (int)((long long)images * g.AH * g.AW * g.C * 2), 0x00020000);
     // Window row r of the run is stacked row orow0 - PH + r, counted from b0's first: where it lies (image group, row in it).
-    // Rows between images and above the first are zeros; per >= H + PH keeps the windows of neighbouring images apart.
+    // Rows between images and above the first are zeros; the host's `stack` keeps the windows of neighbouring images apart.
     const uint32_t row_in = (uint32_t)(g.W * g.C) * 2u, group_in = (uint32_t)img_in * (uint32_t)NI * 2u;
     auto locate = [&](int v, int& group, int& row) {
         group = images_in(max(v, 0)), row = v - group * g.per;   // (v < 0: row < 0)
@@ -669,20 +679,20 @@ inline bool tz_wide_tile(int B, int OW) {
     return (long long)cdiv(OW, 64) * 64 * B <= (long long)cdiv(OW, 32) * 32 * cdiv(B, 2) * 2;
 }
 
-// Cuts the stack into runs of `run` rows (a multiple of 8), by the image where that divides an image's part of the stack; false:
-// a run's images are beyond 32-bit offsets.
+// Cuts the stack into runs of `run` rows (a multiple of 8), by the image where that divides its rows; false: a run's images are
+// beyond 32-bit offsets.
 inline bool tz_cut(TzGeom& g, int ni, long long run) {
-    const int images = cdiv(g.B, ni), total = (images - 1) * g.per + g.OH;
+    const int images = cdiv(g.B, ni), total = (images - 1) * g.stack + g.OH;
     if (run > total) run = (total + 7) / 8 * 8;
-    g.run = (int)run, g.rpi = g.per % g.run == 0 ? cdiv(g.OH, g.run) : 0;
+    g.run = (int)run, g.rpi = g.part % g.run == 0 ? cdiv(g.OH, g.run) : 0;
     if ((long long)images * g.rpi > 0x7fffffffLL) return false;
     g.nruns = g.rpi ? images * g.rpi : cdiv(total, g.run);
-    const long long reach = ((long long)(g.per + g.run + 64) / g.per + 1) * ni, most = reach < g.B ? reach : g.B;
+    const long long reach = g.rpi ? ni : ((long long)(g.stack + g.run + 64) / g.stack + 1) * ni, most = reach < g.B ? reach : g.B;
     const long long in = (long long)g.H * g.W * g.C, out = (long long)g.OH * g.OW * g.YC;
     // the kernel's quotients: rows of the stack by per, workgroups by slices, tiles and runs
     const int by = std::max(std::max(g.nslices, g.ncolt), g.rpi);
-    if ((long long)(total + g.run + g.per + 128) * g.per > 0xffffffffLL || (long long)g.nruns * g.ncolt * g.nslices * by > 0xffffffffLL) return false;
-    g.per_inv = tz_inverse(g.per), g.rpi_inv = tz_inverse(std::max(g.rpi, 1));
+    if ((long long)(total + g.run + g.stack + 128) * g.stack > 0xffffffffLL || (long long)g.nruns * g.ncolt * g.nslices * by > 0xffffffffLL) return false;
+    g.per = g.rpi ? kTzAlone : g.stack, g.per_inv = g.rpi ? kTzAloneInverse : tz_inverse(g.stack), g.rpi_inv = tz_inverse(std::max(g.rpi, 1));
     g.ncolt_inv = tz_inverse(g.ncolt), g.nslices_inv = tz_inverse(g.nslices);
     return most * (in > out ? in : out) <= 0x1fffffffLL;
 }
@@ -690,8 +700,8 @@ inline long long tz_blocks(const TzGeom& g) { return (long long)g.nruns * g.ncol
 
 // Steps of 8 rows of the longest run: those between images at a run's end are left out.
 inline int tz_steps(const TzGeom& g) {
-    if (g.run % g.per == 0) return (g.run - g.per + g.OH + 7) / 8;
-    return (g.rpi && g.OH < g.run ? g.OH + 7 : g.run) / 8;
+    if (g.rpi) return (std::min(g.run, g.OH) + 7) / 8;
+    return (g.run % g.stack == 0 ? g.run - g.stack + g.OH + 7 : g.run) / 8;
 }
 
 // Estimated time of a workgroup, us, on a chip full of them: a start-up (first windows, filter table, operand set-up), then
@@ -709,12 +719,15 @@ inline bool tz_cut_steps(TzGeom& g, int ni, int steps) {
         const long long n = tz_blocks(g);
         if (best == 0 || n < best_blocks || (n == best_blocks && tz_steps(g) < best_steps)) best = run, best_blocks = n, best_steps = tz_steps(g);
     };
-    const int per_image = cdiv(g.OH, 8), group = g.per / 8;
+    const int per_image = cdiv(g.OH, 8), group = g.part / 8;
     look(8LL * steps);
-    if (steps >= per_image) look((long long)((steps - per_image) / group + 1) * g.per);
+    if (steps >= per_image) {
+        const long long n = (steps - per_image) / (g.stack / 8) + 1;
+        look(n == 1 ? g.part : n * g.stack);
+    }
     for (int j = 2; j <= group; ++j)
         if (group % j == 0 && group / j <= steps) {
-            look(g.per / j);
+            look(g.part / j);
             break;
         }
     return best != 0 && tz_cut(g, ni, best);
@@ -724,7 +737,7 @@ inline bool tz_cut_steps(TzGeom& g, int ni, int steps) {
 // end first; false: not covered.  (Each call plans anew: a handful of cuts, a fraction of a microsecond.)
 inline bool tz_cut_alone(TzGeom& g, int ni) {
     const long long per_run = (long long)g.ncolt * g.nslices;
-    const int images = cdiv(g.B, ni), total = cdiv((long long)(images - 1) * g.per + g.OH, 8), group = g.per / 8;
+    const int images = cdiv(g.B, ni), total = cdiv((long long)(images - 1) * g.stack + g.OH, 8), group = g.part / 8;
     long long best = 0;
     double best_cost = 0;
     auto look = [&](long long run, long long most) {
@@ -736,11 +749,11 @@ inline bool tz_cut_alone(TzGeom& g, int ni) {
         const long long most = 256LL * rounds, want = most / per_run, n = want < 1 ? 1 : want > total ? total : want;
         look(8LL * cdiv(total, n), most);
         if (n < images) {
-            look((long long)cdiv(images, n) * g.per, most);   // whole images
+            look((long long)cdiv(images, n) * g.stack, most);   // whole images
         } else {
             int j = (int)std::min<long long>(n / images, group);   // equal parts of an image
             while (group % j) --j;
-            look(g.per / j, most);
+            look(g.part / j, most);
         }
     }
     // (large images: runs as short as their offsets need)
@@ -757,10 +770,11 @@ static bool tz_make_geom(TzGeom& g, bool add, int B, int H, int W, int C, int PH
     g.YC = gate ? gate->ldy : C, g.ych = gate ? gate->ych : 0, g.gs = gate ? gate->gs : 1.f;
     if (gate && (add || flip || C % 16 != 0 || gate->ldy < gate->ych + C / 2 || (gate->ldy | gate->ych) % 8 != 0)) return false;
     if ((long long)H * W * C * Sh::NI > 0x1fffffffLL || (long long)g.OH * g.OW * g.YC * Sh::NI > 0x1fffffffLL) return false;
-    // the windows of a run's first and last rows of an image reach PH rows before it and K - 1 - PH after: zeros
-    g.per = H + PH > g.OH ? H + PH : g.OH;
-    g.per = (g.per + 7) / 8 * 8;
-    if ((long long)(cdiv(B, Sh::NI) - 1) * g.per + g.OH + g.per + 64 > 0x7fffffffLL) return false;
+    g.part = (std::max(H + PH, g.OH) + 7) / 8 * 8;
+    // the windows of an image's first patches reach PH rows above it, and the operands of its last, output rows 4 * ((OH - 1) / 4)
+    // on, OPR rows from PH above those: none of them the neighbour's
+    g.stack = std::max(g.part, (4 * ((g.OH - 1) / 4) - PH + Sh::OPR + 7) / 8 * 8);
+    if ((long long)(cdiv(B, Sh::NI) - 1) * g.stack + g.OH + g.stack + 64 > 0x7fffffffLL) return false;
     g.ncolt = cdiv(g.OW, Sh::TW), g.nslices = cdiv(C, CS);
     return true;
 }

@@ -126,3 +126,104 @@ def test_weight_gradient_other_channels_unaffected(oracle, shape, k, dtype):
     ref_bad = ~np.isfinite(bad)
     assert ref_bad[:, :, [5, 9]].any() and not ref_bad[:, :, others].any()
     assert (~np.isfinite(got[ref_bad])).all()
+
+
+# Images never meet: whatever one holds, the others' results are bitwise those of the clean batch.  (The 16-bit kernels walk a
+# batch as one column of rows, and the last patch of an image multiplies up to three rows beyond its last window by zeros.)
+HURT = 2   # an image with neighbours on both sides, in a batch side by side in pairs too
+ODD = [3, 5, 7, 9, 11, 13, 15, 17]
+
+
+def _hurt(t):
+    t = t.clone()
+    t[HURT] = float("nan")
+    t[HURT, ..., ::2] = float("inf")
+    return t
+
+
+def _apart(what, got, want):
+    others = [b for b in range(want.shape[0]) if b != HURT]
+    assert torch.isfinite(want).all(), what
+    assert torch.equal(got[others], want[others]), f"{what}: another image's values changed"
+
+
+def _conv_results(x, w, pad):
+    """Forward and input gradient, and both with the pool of the input or its gradient where the extents are even."""
+    from pyramidconvblock_amd.dwconv import dwconv_dgrad, dwconv_forward
+
+    geo = ((1, 1), (pad, pad), (1, 1))
+    k, (B, H, W, C) = w.shape[0], x.shape
+    res = {"forward": dwconv_forward(x, w, *geo)}
+    if H + k - 1 - 2 * pad >= 1 and W + k - 1 - 2 * pad >= 1:   # (x as the gradient of a result)
+        res["input gradient"] = dwconv_dgrad(x, w, (B, H + k - 1 - 2 * pad, W + k - 1 - 2 * pad, C), *geo)
+    if 2 * pad == k - 1 and H % 2 == 0 and W % 2 == 0:
+        res["forward of a pool"], res["pool"] = dwconv_forward(x, w, *geo, pool_to=(H // 2, W // 2))
+        res["input gradient of a pool"] = dwconv_dgrad(x, w, (B, H, W, C), *geo, pooled_grad=x[:, ::2, ::2].contiguous())
+    return res
+
+
+@pytest.mark.parametrize("k", ODD)
+@pytest.mark.parametrize("B,W,C,dtype", [(5, 20, 16, torch.bfloat16), (4, 44, 24, torch.float16), (4, 13, 20, torch.bfloat16),
+                                         (5, 18, 12, torch.float32)])
+def test_images_stay_apart(k, B, W, C, dtype):
+    """Every height modulo 8, a run of rows to a part of an image; 20: two images side by side."""
+    gen = torch.Generator().manual_seed(k + C)
+    w = (randn(gen, k, k, C) / k).to(dtype).cuda()
+    for H in [*range(1, 18), *range(22, 30)]:
+        x = randn(gen, B, H, W, C).to(dtype).cuda()
+        for pad in sorted({k // 2, 0, k - 1, k // 2 + 1}):
+            if H + 2 * pad < k or W + 2 * pad < k:
+                continue
+            clean, hurt = _conv_results(x, w, pad), _conv_results(_hurt(x), w, pad)
+            for name in clean:
+                _apart(f"{name} k={k} H={H} pad={pad}", hurt[name], clean[name])
+
+
+# heights after which a window row beyond the last one counts, by the filter, and one height of each filter where none does
+LAST_ROWS = [(3, 5), (3, 6), (3, 7), (3, 14), (3, 8), (5, 13), (5, 14), (5, 12), (7, 13), (7, 16), (11, 9), (11, 10), (11, 11), (11, 28),
+             (13, 9), (13, 58), (13, 40), (15, 57), (15, 17), (15, 20), (9, 14), (17, 14)]
+
+
+@pytest.mark.parametrize("k,H", LAST_ROWS)
+@pytest.mark.parametrize("B,W,C", [(40, 10, 136), (43, 36, 136), (4, 36, 16)])
+def test_images_of_a_run_stay_apart(oracle, k, H, B, W, C):
+    """The same where a run of rows crosses several images (more images x slices of channels than compute units), with the
+    values of the other images against the clean oracle."""
+    dtype, pad = torch.bfloat16, k // 2
+    gen = torch.Generator().manual_seed(k + H)
+    x, w = randn(gen, B, H, W, C).to(dtype), (randn(gen, k, k, C) / k).to(dtype)
+    first, second = _conv_results(x.cuda(), w.cuda(), pad), _conv_results(_hurt(x).cuda(), w.cuda(), pad)
+    for name in first:
+        _apart(name, second[name], first[name])
+    some = [b for b in (0, 1, 3, B - 1) if b < B]
+    xs, ws = x[some].double().numpy(), w.double().numpy()
+    for name, want in (("forward", oracle.dwconv_fwd(xs, ws, 1, (pad, pad), 1)),
+                       ("input gradient", oracle.dwconv_dgrad(xs, ws, (H, W), 1, (pad, pad), 1))):
+        got = second[name][some].double().cpu().numpy()
+        assert np.abs(got - want).max() / np.abs(want).max() <= TOL[dtype], name
+
+
+@pytest.mark.parametrize("shape,k", [((5, 14, 44, 64), 3), ((5, 28, 60, 64), 5), ((9, 13, 40, 64), 7), ((4, 18, 48, 128), 11), ((4, 58, 60, 128), 13),
+                                     ((4, 57, 61, 64), 15), ((5, 34, 36, 64), 17), ((80, 14, 14, 256), 3), ((40, 7, 7, 520), 3)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_images_of_a_block_stay_apart(shape, k, dtype):
+    """The shared launches of both scales, gates and mean branch, forward, backward and at inference."""
+    import pyramidconvblock_amd as pcb
+
+    torch.manual_seed(k)
+    block = pcb.ConvBlock(dim=shape[3], kernel_size=k).to(dtype).cuda()
+    gen = torch.Generator().manual_seed(k + shape[1])
+    x, g = randn(gen, *shape).to(dtype).cuda(), randn(gen, *shape).to(dtype).cuda()
+
+    def results(x, g):
+        with torch.no_grad():
+            inferred = block(x)
+        x = x.clone().requires_grad_()
+        y = block(x)
+        torch.autograd.backward(y, g)
+        return {"inference": inferred, "forward": y.detach(), "input gradient": x.grad}
+
+    clean = results(x, g)
+    for hurt in (results(_hurt(x), g), results(x, _hurt(g))):
+        for name in clean:
+            _apart(name, hurt[name], clean[name])
