@@ -236,6 +236,9 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
     constexpr int RWMAX = RW01 > 8 ? RW01 : 8;
     constexpr int WCQ = Sh::WCOLS / IC;
     constexpr int NLD = (RWMAX / IR * NI * (Sh::WCOLS / IC) * NH + NT - 1) / NT;  // items per thread and pass
+    // A step has too few products to put the staging between them: the previous step's tiles leave before them instead (us:
+    // [32,56,56,128] filter 3 14.4 -> 13.4, [64,28,28,256] 15.5 -> 14.8; the tiles behind the staging: 14.6 and 16.4).
+    constexpr bool FEW = NM <= 2;
     constexpr int UNRF = PER % 4 == 0 ? PER / 2 : (PER % 2 == 0 ? PER : 2 * PER);  // steps per trip: even, PER | 2 UNRF
     auto first_row = [&](int pass) { return pass < 2 ? pass * RW01 : 2 * RW01 + 8 * (pass - 2); };
     // Loads go through a buffer descriptor over the workgroup's images: an offset past its end (an image beyond the
@@ -341,11 +344,15 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
         next_group(rb, ob, rb, ob);
     };
     // A pass into the window: the columns of channels 2j and 2j + 1 of the items' rows at ring byte offset cring[l].  No
-    // branch, so that the products around it can be interleaved: lanes without an item write behind the planes.
+    // branch, so that the products around it can be interleaved: lanes without an item write behind the planes (with FEW
+    // products there is nothing to interleave, and wavefronts without an item write nothing).
     int cring[NLD];
+    constexpr int ITEMS = RWMAX / IR * NI * WCQ * NH;
+    const int wave0 = __builtin_amdgcn_readfirstlane(tid) & ~63;   // the wavefront's first thread
     auto commit_part = [&](const uint4 (&bf)[NLD][IC * IR], int j) {
 #pragma unroll
-        for (int l = 0; l < NLD; ++l)
+        for (int l = 0; l < NLD; ++l) {
+            if (FEW && wave0 + l * NT >= ITEMS) continue;   // (uniform)
 #pragma unroll
             for (int r = 0; r < IR; ++r) {
                 auto d = [&](int k) { const uint4& u = bf[l][IC * r + k]; return j == 0 ? u.x : j == 1 ? u.y : j == 2 ? u.z : u.w; };
@@ -360,6 +367,7 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
                         *reinterpret_cast<uint32_t*>(dst + (2 * j + odd) * CHP) = lo;
                 }
             }
+        }
     };
     auto commit_next = [&]() {   // 8 rows on (passes from 2 on)
 #pragma unroll
@@ -562,15 +570,25 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
 
 #pragma unroll
     for (int j = 0; j < PER - 1; ++j) load_group(j, 4 * j * RP);
-    // A step is two row groups (8 output rows).  Trips of UNRF steps (the ring's period in steps), left after the run's last step
-    // by a uniform exit between steps.
+    // A step is two row groups (8 output rows), UNRF steps (the ring's period in steps) a trip.
     const int nfat = (nsteps + 1) >> 1;
-    int fdone = 0;
-    bool left = false;
     auto step = [&](int jf, int f) {
         // the two row groups this step adds to the ring; the second goes to the slot of the step's own first group, once the
         // first tile's products with that are issued (LATE), or waits in registers where those are nearly all there are
         constexpr bool LATE = PER >= 3;
+        uint4 out[NG];
+        auto tiles_read = [&]() {
+#pragma unroll
+            for (int n = 0; n < NG; ++n) out[n] = tile_read(jf + 1, n);
+        };
+        auto tiles_store = [&]() {
+#pragma unroll
+            for (int n = 0; n < NG; ++n) tile_store(out[n], n);
+        };
+        if constexpr (FEW) {
+            tiles_read();
+            __builtin_amdgcn_sched_barrier(0x6);
+        }
         load_group((2 * jf + PER - 1) % PER, ((2 * f + PER - 1) % NR) * (4 * RP));
         const int late_off = ((2 * f + PER) % NR) * (4 * RP);
         uint4 late[CPW][ICB];
@@ -580,9 +598,13 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
 #pragma unroll
                 for (int i = 0; i < ICB; ++i) late[q][i] = read16(xb[q][i] + late_off);
         }
-        uint4 out[NG];
-#pragma unroll
-        for (int n = 0; n < NG; ++n) out[n] = tile_read(jf + 1, n);
+        if constexpr (FEW) {
+            __builtin_amdgcn_sched_barrier(0x6);
+            tiles_store();
+            __builtin_amdgcn_sched_barrier(0x6);
+        } else {
+            tiles_read();
+        }
         tz_f32x4 acc[2][CPW];
 #pragma unroll
         for (int gi = 0; gi < 2; ++gi)
@@ -612,10 +634,7 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
                     write_pool(buf[jf % 2], f + 2);
                     issue(buf[jf % 2], f + 4);
                 }
-                if (piece == 0) {
-#pragma unroll
-                    for (int n = 0; n < NG; ++n) tile_store(out[n], n);
-                }
+                if (piece == 0 && !FEW) tiles_store();
                 if (piece == 1) place();
                 __builtin_amdgcn_sched_barrier(0x6);   // (vector and scalar arithmetic may cross)
             }
@@ -644,24 +663,39 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
             }
         }
     };
-    for (int f0 = 0; f0 < nfat; f0 += UNRF) {
-#pragma unroll
-        for (int jf = 0; jf < UNRF; ++jf) {
-            const int f = f0 + jf;
+    if constexpr (UNRF == 2) {
+        // A run's odd last step by itself: with a way out between the two steps of a trip the compiler no longer knows which
+        // requests are the newest, and every other commit waited for those of the step before as well (us: [32,56,56,128] filter
+        // 13 17.0 -> 16.6, [16,32,32,64] 7.25 -> 6.85, [1,56,56,64] 6.35 -> 6.0).
+        int f = 0;
+        for (; f + 2 <= nfat; f += 2) {
             lds_barrier();  // the previous step's tiles are complete, its window reads done
-            step(jf, f);
-            if (f + 1 >= nfat) {   // the run's last step (uniform): its tiles are stored after the loop
-                left = true;
-                fdone = f + 1;
-                break;
-            }
+            step(0, f);
+            lds_barrier();
+            step(1, f + 1);
         }
-        if (left) break;
-        fdone = f0 + UNRF;
+        if (f < nfat) {
+            lds_barrier();
+            step(0, f);
+        }
+    } else {   // left after the run's last step by a uniform exit between steps
+        bool left = false;
+        for (int f0 = 0; f0 < nfat; f0 += UNRF) {
+#pragma unroll
+            for (int jf = 0; jf < UNRF; ++jf) {
+                lds_barrier();
+                step(jf, f0 + jf);
+                if (f0 + jf + 1 >= nfat) {
+                    left = true;
+                    break;
+                }
+            }
+            if (left) break;
+        }
     }
     lds_barrier();
 #pragma unroll
-    for (int n = 0; n < NG; ++n) tile_store(tile_read(fdone - 1, n), n);
+    for (int n = 0; n < NG; ++n) tile_store(tile_read(nfat - 1, n), n);
 }
 
 template <typename T, int K, int NPC, int CS, int MODE>
