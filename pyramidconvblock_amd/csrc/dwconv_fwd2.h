@@ -146,7 +146,7 @@ inline bool launch_balance(const LaunchPart (&p)[N], int nmean, int (&steps)[N])
 
 // (a tile of two images starts later)
 inline LaunchPart tz_part(const TzGeom& g, int ni, double start, double step) {
-    return {start + 1.3 * (ni - 1), step, cdiv((long long)(cdiv(g.B, ni) - 1) * g.stack + g.OH, 8), 1, [g, ni](int steps) {
+    return {start + 1.3 * (ni - 1), step, cdiv(tz_rows(g, ni), 8), 1, [g, ni](int steps) {
                 TzGeom c = g;
                 return tz_cut_steps(c, ni, steps) ? tz_blocks(c) : 1LL << 40;
             }};

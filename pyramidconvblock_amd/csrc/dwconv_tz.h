@@ -128,7 +128,7 @@ struct TzGeom {
     int run;           // stacked rows of a workgroup (a multiple of 8)
     int rpi;           // 0: runs follow one another through the stack; else they are parts of an image, rpi of them to one
     int nruns, ncolt, nslices;
-    int part, stack;   // (host) rows that runs by image divide; rows from one image to the next in the stack
+    int part, stack;   // (host) rows that runs by image divide; rows from one image to the next in the stack (0: no stack)
     uint32_t per_inv, rpi_inv, ncolt_inv, nslices_inv;   // tz_inverse of these
     int flip;          // 1: 180-degree rotated filter (input gradient)
     int AH, AW;        // extents of the half-resolution addend / pooled output
@@ -713,19 +713,22 @@ inline bool tz_wide_tile(int B, int OW) {
     return (long long)cdiv(OW, 64) * 64 * B <= (long long)cdiv(OW, 32) * 32 * cdiv(B, 2) * 2;
 }
 
-// Cuts the stack into runs of `run` rows (a multiple of 8), by the image where that divides its rows; false: a run's images are
-// beyond 32-bit offsets.
+// Rows of the stack (of one image where there is none).
+inline int tz_rows(const TzGeom& g, int ni) { return g.stack ? (cdiv(g.B, ni) - 1) * g.stack + g.OH : g.OH; }
+
+// Cuts the stack into runs of `run` rows (a multiple of 8), by the image where that divides its rows or there is no stack; false:
+// a run's images are beyond 32-bit offsets.
 inline bool tz_cut(TzGeom& g, int ni, long long run) {
-    const int images = cdiv(g.B, ni), total = (images - 1) * g.stack + g.OH;
+    const int images = cdiv(g.B, ni), total = tz_rows(g, ni);
     if (run > total) run = (total + 7) / 8 * 8;
-    g.run = (int)run, g.rpi = g.part % g.run == 0 ? cdiv(g.OH, g.run) : 0;
+    g.run = (int)run, g.rpi = !g.stack || g.part % g.run == 0 ? cdiv(g.OH, g.run) : 0;
     if ((long long)images * g.rpi > 0x7fffffffLL) return false;
     g.nruns = g.rpi ? images * g.rpi : cdiv(total, g.run);
     const long long reach = g.rpi ? ni : ((long long)(g.stack + g.run + 64) / g.stack + 1) * ni, most = reach < g.B ? reach : g.B;
     const long long in = (long long)g.H * g.W * g.C, out = (long long)g.OH * g.OW * g.YC;
-    // the kernel's quotients: rows of the stack by per, workgroups by slices, tiles and runs
+    // the kernel's quotients of workgroups: by slices, tiles and runs
     const int by = std::max(std::max(g.nslices, g.ncolt), g.rpi);
-    if ((long long)(total + g.run + g.stack + 128) * g.stack > 0xffffffffLL || (long long)g.nruns * g.ncolt * g.nslices * by > 0xffffffffLL) return false;
+    if ((long long)g.nruns * g.ncolt * g.nslices * by > 0xffffffffLL) return false;
     g.per = g.rpi ? kTzAlone : g.stack, g.per_inv = g.rpi ? kTzAloneInverse : tz_inverse(g.stack), g.rpi_inv = tz_inverse(std::max(g.rpi, 1));
     g.ncolt_inv = tz_inverse(g.ncolt), g.nslices_inv = tz_inverse(g.nslices);
     return most * (in > out ? in : out) <= 0x1fffffffLL;
@@ -756,7 +759,7 @@ inline bool tz_cut_steps(TzGeom& g, int ni, int steps) {
     const int per_image = cdiv(g.OH, 8), group = g.part / 8;
     look(8LL * steps);
     if (steps >= per_image) {
-        const long long n = (steps - per_image) / (g.stack / 8) + 1;
+        const long long n = g.stack ? (steps - per_image) / (g.stack / 8) + 1 : 1;
         look(n == 1 ? g.part : n * g.stack);
     }
     for (int j = 2; j <= group; ++j)
@@ -771,7 +774,8 @@ inline bool tz_cut_steps(TzGeom& g, int ni, int steps) {
 // end first; false: not covered.  (Each call plans anew: a handful of cuts, a fraction of a microsecond.)
 inline bool tz_cut_alone(TzGeom& g, int ni) {
     const long long per_run = (long long)g.ncolt * g.nslices;
-    const int images = cdiv(g.B, ni), total = cdiv((long long)(images - 1) * g.stack + g.OH, 8), group = g.part / 8;
+    const int images = cdiv(g.B, ni), group = g.part / 8;
+    const long long total = cdiv(tz_rows(g, ni), 8) * (g.stack ? 1LL : images);
     long long best = 0;
     double best_cost = 0;
     auto look = [&](long long run, long long most) {
@@ -783,7 +787,7 @@ inline bool tz_cut_alone(TzGeom& g, int ni) {
         const long long most = 256LL * rounds, want = most / per_run, n = want < 1 ? 1 : want > total ? total : want;
         look(8LL * cdiv(total, n), most);
         if (n < images) {
-            look((long long)cdiv(images, n) * g.stack, most);   // whole images
+            look(g.stack ? (long long)cdiv(images, n) * g.stack : g.part, most);   // whole images
         } else {
             int j = (int)std::min<long long>(n / images, group);   // equal parts of an image
             while (group % j) --j;
@@ -808,7 +812,10 @@ static bool tz_make_geom(TzGeom& g, bool add, int B, int H, int W, int C, int PH
     // the windows of an image's first patches reach PH rows above it, and the operands of its last, output rows 4 * ((OH - 1) / 4)
     // on, OPR rows from PH above those: none of them the neighbour's
     g.stack = std::max(g.part, (4 * ((g.OH - 1) / 4) - PH + Sh::OPR + 7) / 8 * 8);
-    if ((long long)(cdiv(B, Sh::NI) - 1) * g.stack + g.OH + g.stack + 64 > 0x7fffffffLL) return false;
+    // the kernel's quotients of rows of the stack by this are exact up to 2^32 / stack; images too tall for that are walked one by
+    // one (a run of one such image is thousands of steps: nothing is lost)
+    const long long rows = (long long)cdiv(B, Sh::NI) * g.stack;
+    if (rows > 0x3fffffffLL || (2 * rows + g.stack + 128) * g.stack > 0xffffffffLL) g.stack = 0;
     g.ncolt = cdiv(g.OW, Sh::TW), g.nslices = cdiv(C, CS);
     return true;
 }

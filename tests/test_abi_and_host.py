@@ -152,6 +152,19 @@ def test_bwd3_planner_strip_shaped_inputs(shape):
     assert L.pdw_dwconv_bwd3_plan(B, H, W, C, K, 2, None) == 1
 
 
+@pytest.mark.parametrize("shape", [(64, 8192, 34, 16, 5), (2, 65536, 34, 16, 13), (3, 40000, 36, 32, 7), (256, 4096, 34, 16, 3)])
+def test_bwd3_planner_tall_images(shape):
+    """Batches of tall images, whose rows one below the other are more than the kernel's quotients by an image's rows are exact
+    for, are walked image by image (host code, no device touched)."""
+    from pyramidconvblock_amd import _lib
+
+    bands = (ctypes.c_int * 3)(-1, -1, -1)
+    rc = _lib.lib().pdw_dwconv_bwd3_plan(*shape, _lib.dtype_code(torch.bfloat16), ctypes.addressof(bands))
+    assert rc == 0, _lib.lib().pdw_last_error()
+    B, H, _, C, _ = shape
+    assert all(1 <= n <= H for n in bands) and B * bands[0] * C // 16 >= 48, list(bands)   # (a useful share of the chip)
+
+
 def test_module_structure_and_seeded_init_match_reference_recipe():
     import pyramid_dwconv
     from oracle import torch_path

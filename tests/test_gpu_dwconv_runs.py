@@ -26,3 +26,20 @@ def test_runs_over_stacked_images(oracle, shape, k, pad, dtype):
     assert rel_err(dwconv_forward(x.cuda(), w.cuda(), *geo), want) <= TOL[dtype]
     want = oracle.dwconv_dgrad(gy.double().numpy(), w.double().numpy(), (H, W), 1, (pad, pad), 1)
     assert rel_err(dwconv_dgrad(gy.cuda(), w.cuda(), shape, *geo), want) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("shape,k,pad", [((3, 30011, 9, 8), 5, 2), ((1, 40003, 33, 16), 3, 1), ((2, 65530, 7, 8), 9, 4), ((5, 29990, 11, 24), 7, 0)])
+def test_tall_images_run_by_image(oracle, shape, k, pad):
+    """Images too tall for a stack: runs are parts of an image of any length, the last one shorter."""
+    from pyramidconvblock_amd.dwconv import dwconv_dgrad, dwconv_forward
+
+    dtype = torch.bfloat16
+    gen = torch.Generator().manual_seed(k)
+    x, w = randn(gen, *shape).to(dtype), (randn(gen, k, k, shape[3]) / k).to(dtype)
+    B, H, W, C = shape
+    gy = randn(gen, B, H + 2 * pad - k + 1, W + 2 * pad - k + 1, C).to(dtype)
+    geo = ((1, 1), (pad, pad), (1, 1))
+    want = oracle.dwconv_fwd(x.double().numpy(), w.double().numpy(), 1, (pad, pad), 1)
+    assert rel_err(dwconv_forward(x.cuda(), w.cuda(), *geo), want) <= TOL[dtype]
+    want = oracle.dwconv_dgrad(gy.double().numpy(), w.double().numpy(), (H, W), 1, (pad, pad), 1)
+    assert rel_err(dwconv_dgrad(gy.cuda(), w.cuda(), shape, *geo), want) <= TOL[dtype]
