@@ -120,16 +120,21 @@ constexpr int kTzAlone = 0x40000000;
 constexpr uint32_t kTzAloneInverse = 1;
 __device__ __forceinline__ int tz_quotient(int n, uint32_t inverse) { return inverse ? (int)__umulhi((uint32_t)n, inverse) : n; }
 
-struct TzGeom {
-    int B, H, W, C;    // input extents
-    int OH, OW;        // output extents
-    int PH, PW;        // padding
+// How a problem is cut into workgroups (tz_cut).
+struct TzRuns {
     int per;           // rows from one image to the next in the stack of a batch's images (a multiple of 8); kTzAlone if rpi
     int run;           // stacked rows of a workgroup (a multiple of 8)
     int rpi;           // 0: runs follow one another through the stack; else they are parts of an image, rpi of them to one
-    int nruns, ncolt, nslices;
-    int part, stack;   // (host) rows that runs by image divide; rows from one image to the next in the stack (0: no stack)
+    int nruns;         // (0: not covered)
     uint32_t per_inv, rpi_inv, ncolt_inv, nslices_inv;   // tz_inverse of these
+};
+
+struct TzGeom : TzRuns {
+    int B, H, W, C;    // input extents
+    int OH, OW;        // output extents
+    int PH, PW;        // padding
+    int ncolt, nslices;
+    int part, stack;   // (host) rows that runs by image divide; rows from one image to the next in the stack (0: no stack)
     int flip;          // 1: 180-degree rotated filter (input gradient)
     int AH, AW;        // extents of the half-resolution addend / pooled output
     int YC, ych;       // output pixel stride in channels, first output channel
@@ -771,7 +776,7 @@ inline bool tz_cut_steps(TzGeom& g, int ni, int steps) {
 }
 
 // Runs of a launch of its own: the shortest with which 256 compute units are filled 1..4 times, whichever number is estimated to
-// end first; false: not covered.  (Each call plans anew: a handful of cuts, a fraction of a microsecond.)
+// end first; false: not covered.
 inline bool tz_cut_alone(TzGeom& g, int ni) {
     const long long per_run = (long long)g.ncolt * g.nslices;
     const int images = cdiv(g.B, ni), group = g.part / 8;
@@ -825,7 +830,14 @@ static int launch_tz(const void* x, const void* w, const void* add, void* pool, 
                      int PH, int PW, bool flip, const TzGate* gate, hipStream_t s) {
     using Sh = TzShape<K, NPC, CS>;
     TzGeom g;
-    if (!tz_make_geom<K, NPC, CS>(g, add != nullptr, B, H, W, C, PH, PW, flip, gate) || !tz_cut_alone(g, Sh::NI)) return -1;
+    if (!tz_make_geom<K, NPC, CS>(g, add != nullptr, B, H, W, C, PH, PW, flip, gate)) return -1;
+    // (the search takes a quarter of a microsecond of the call, which a short kernel does not hide: 0.21-0.26 us, kept 0.02)
+    static PlanCache<std::array<int, 7>, TzRuns> plans;
+    static_cast<TzRuns&>(g) = plans.get({B, H, W, C, PH, PW, g.YC}, [g]() mutable {
+        if (!tz_cut_alone(g, Sh::NI)) g.nruns = 0;
+        return static_cast<TzRuns>(g);
+    });
+    if (g.nruns == 0) return -1;
     const size_t lds = Sh::lds_bytes;
     const int mode = (add ? 1 : 0) | (pool ? 2 : 0) | (gate ? 4 : 0);
     auto kern = dwconv_tz_k<T, K, NPC, CS, 0>;

@@ -43,3 +43,21 @@ def test_tall_images_run_by_image(oracle, shape, k, pad):
     assert rel_err(dwconv_forward(x.cuda(), w.cuda(), *geo), want) <= TOL[dtype]
     want = oracle.dwconv_dgrad(gy.double().numpy(), w.double().numpy(), (H, W), 1, (pad, pad), 1)
     assert rel_err(dwconv_dgrad(gy.cuda(), w.cuda(), shape, *geo), want) <= TOL[dtype]
+
+
+def test_plans_are_kept_by_shape():
+    """More shapes than are kept, twice over and from two threads: every batch gives the results of the whole one."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    from pyramidconvblock_amd.dwconv import dwconv_forward
+
+    gen = torch.Generator().manual_seed(0)
+    geo = ((1, 1), (1, 1), (1, 1))
+    x, w = randn(gen, 300, 5, 7, 16).to(torch.bfloat16).cuda(), randn(gen, 3, 3, 16).to(torch.bfloat16).cuda()
+    whole = dwconv_forward(x, w, geo[0], geo[1], geo[2])
+
+    def batches(order):
+        return all(torch.equal(dwconv_forward(x[:b], w, *geo), whole[:b]) for b in order for _ in range(2))
+
+    with ThreadPoolExecutor(2) as pool:
+        assert all(pool.map(batches, [range(1, 301), range(300, 0, -1)]))
