@@ -577,6 +577,7 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
     for (int j = 0; j < PER - 1; ++j) load_group(j, 4 * j * RP);
     // A step is two row groups (8 output rows), UNRF steps (the ring's period in steps) a trip.
     const int nfat = (nsteps + 1) >> 1;
+    int last = nfat - 1;
     auto step = [&](int jf, int f) {
         // the two row groups this step adds to the ring; the second goes to the slot of the step's own first group, once the
         // first tile's products with that are issued (LATE), or waits in registers where those are nearly all there are
@@ -685,22 +686,24 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
         }
     } else {   // left after the run's last step by a uniform exit between steps
         bool left = false;
+        last = -1;   // (set where a trip is left, with its parity known there: 188 registers at filter 17, 231 with nfat - 1)
         for (int f0 = 0; f0 < nfat; f0 += UNRF) {
 #pragma unroll
             for (int jf = 0; jf < UNRF; ++jf) {
                 lds_barrier();
                 step(jf, f0 + jf);
                 if (f0 + jf + 1 >= nfat) {
-                    left = true;
+                    left = true, last = f0 + jf;
                     break;
                 }
             }
             if (left) break;
+            last = f0 + UNRF - 1;
         }
     }
     lds_barrier();
 #pragma unroll
-    for (int n = 0; n < NG; ++n) tile_store(tile_read(nfat - 1, n), n);
+    for (int n = 0; n < NG; ++n) tile_store(tile_read(last, n), n);
 }
 
 template <typename T, int K, int NPC, int CS, int MODE>
