@@ -71,7 +71,7 @@ def conv_issue(k):
     ic = k + 3
     icb = (ic + 7) // 8
     nm = (ic * icb + 3) // 4
-    return dict(fwd=nm * 32, wgrad=256 if k <= 14 else None, useful=k * k)
+    return dict(fwd=nm * 32, wgrad=256 if k <= 15 else None, useful=k * k)
 
 
 # ------------------------------------------------------------------------------------------------
@@ -739,7 +739,7 @@ def main():
             "traffic": traffic.get(dom["kernel"]), "avg_us": dom["seconds"] * 1e6,
             "flops_per_byte": ai, "machine_flops_per_byte": MFMA_PEAK / HBM_PEAK,
             "mfma_issue_frac": (dom["issued_flops"] / dom["seconds"] / MFMA_PEAK) if dom["issued_flops"] else None,
-            "limiter": "not the roofline: LDS operand reads and exposed load latency (profiles/)",
+            "limiter": "not the roofline: LDS traffic and exposed latency, no unit busy half of the time (profiles/)",
             "timed": "HIP events around graph replays over rotating buffers; for dwconv_bwd3 the graph holds the launch "
                      "alone (its summations are recorded during the capture and run outside the graph; `call_us` in the "
                      "kernels row includes them), graph launch gaps included",

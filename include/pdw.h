@@ -27,8 +27,8 @@
  *     is a function of the arguments.
  *   - Non-finite inputs: the matrix-core convolution kernels multiply a window of input pixels somewhat larger
  *     than the filter by zero-padded filter operands, so an Inf or NaN input pixel can turn outputs up to
- *     PDW_NONFINITE_REACH pixels beyond the filter's own footprint into NaN (0 * Inf).  Outputs further away, and
- *     all outputs for finite inputs, are unaffected.  The reference masks its loads (dwconv_triton.py:55-86), so
+ *     PDW_NONFINITE_REACH pixels beyond the filter's own footprint into NaN (0 * Inf).  Outputs further away, those of
+ *     the batch's other images, and all outputs for finite inputs, are unaffected.  The reference masks its loads (dwconv_triton.py:55-86), so
  *     there the value reaches the footprint only.
  */
 #ifndef PDW_H_

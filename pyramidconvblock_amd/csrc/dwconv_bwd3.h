@@ -3,8 +3,8 @@
 // gradients of both scales) as one launch: on a compute unit a band of each runs back to back, without two drains and
 // launch gaps in between.  Every problem runs in the tile that its width fills better: by template where both full-scale
 // problems' are the wide ones, the pool halved the extents and no mean branch rides along (each workgroup starts with one
-// problem's arguments; chosen at run time as for the others, us: [32,56,56,64] filter 13 30.8 for 30.6, 9 32.4 for 31.6,
-// 17 50.1 for 49.6; [128,56,56,64] filter 13 98.8 for 97.6), at run time per problem elsewhere.
+// problem's arguments), at run time per problem elsewhere.  (With bands of one image the template was 0.2 to 1.2 us faster; with runs
+// both take as long: [32,56,56,64] filter 9 26.0 and 25.9 us, 13 28.6 and 28.7, 17 50.0 and 49.8, [128,56,56,64] filter 13 76.0 and 76.5.)
 // The kernel template and its per-filter-size launcher; dwconv_bwd3_k<K>.hip instantiate it, one file per size.
 #pragma once
 #include "dwconv_fwd2.h"
@@ -99,9 +99,11 @@ __global__ __launch_bounds__(512, 1) void dwconv_bwd3_k(const Bwd3Args<K> a) {
 // costs a start-up (first rows, operand set-up) that does not depend on how many rows it takes, so unlike a launch of its
 // own, which has to fill the chip, a problem here is best cut into as few pieces as the other problems leave room for: all
 // three in one round of the chip, ending together, where that is possible; else each candidate (runs of several lengths; bands
-// per image for the weight gradients of dwconv_wgrad_tz.h)
-// is priced by dealing its workgroups, longest problem first (the grid order), to the compute units.  us with the summations,
-// against whole-image bands of one image: [32,56,56,64] filter 13 31 -> 27, 15 42 -> 32.5, 9 32 -> 25; [128,56,56,64] 98 -> 73.
+// per image for the weight gradients of dwconv_wgrad_tz.h) is priced by dealing its workgroups, longest problem first (the grid
+// order), to the compute units.  us a call with its two summations, 20 of them in a graph, against whole-image bands of one
+// image: [32,56,56,64] filter 9 32.8 -> 25.9, 13 32.3 -> 28.5, 15 43.5 -> 33.9, 17 (bands still) 51.1 -> 49.2; [128,56,56,64] filter 13
+// 100.5 -> 75.8, 17 167 -> 156.  What the runs cost: the two problems that share gy read it at different times, and [32,56,56,64]
+// filter 13 fetches and writes 67.3 MB where bands moved 51.6 (48.2 are needed).
 struct Bwd3Plan {
     int n[3];         // rows of the input gradient's runs; runs or bands of the full scale's and the half scale's weight gradient
     char order[4];    // 'D', 'F', 'H' in grid order
@@ -120,7 +122,9 @@ static Bwd3Plan bwd3_plan(int B, const TzGeom& gd, int npcd, const P& p0, const 
     const Key key{B, gd.OH, gd.OW, p1.g.OH, p1.g.OW, gd.C, nmean};
     std::lock_guard<std::mutex> lock(mu);
     if (auto it = cache.find(key); it != cache.end()) return it->second;
-    constexpr double kStart = 5.0, kStep = 1.15;   // of the input gradient here (its store adds the pooled gradient)
+    // Prices of the input gradient here: its store adds the pooled gradient, and its runs have the chip and its memory to share with
+    // the weight gradients' (256 of them alone: 6.1 + 1.8 a step at filter 13).
+    constexpr double kStart = 5.0, kStep = 1.15;
     const int ni = 16 / npcd;
     Bwd3Plan best{{8, 1, 1}, "DFH"};
     bool balanced = false;

@@ -2,12 +2,13 @@
 // y1 = conv(x1, w1) at the pooled one (x1 being the average pool of x0, made before the launch), neither
 // depending on the other.  A compute unit holds one workgroup of these kernels at a time and a run of rows costs a start-up
 // that does not depend on its length, so a launch of its own cuts a problem into enough runs to fill the chip; here each
-// scale gets the part of the chip that lets both end together (us at [32,56,56,64], filter 13: 14.0 for the launch against 13.9
-// + 7.9 and a gap; [128,56,56,64] 31; with bands of one image instead of runs 14.4 and 36.3).  Each scale runs in the tile
+// scale gets the part of the chip that lets both end together.  us a launch, 20 of them in a graph: [32,56,56,64] filter 13 15.1
+// (bands of one image instead of runs 15.4), 17 20.1 (22.8), [128,56,56,64] filter 13 39 (41), 17 55.5 (68); the two launches
+// one by one at [32,56,56,64] filter 13 12.2 + 8.0 and a gap.  Each scale runs in the tile
 // (16 or 8 patches side by side) that its width fills better: by template where the full scale's is the wide one and slices
 // are 16 channels (each workgroup starts with one problem's arguments and no choice between the fields of two; at run time,
-// us: filter 13 14.2 for 14.0), at run time elsewhere (with the mean branch, filters 15 and 17: 24.7 and 24.6, by template 24.9
-// and 24.8).
+// us: filter 13 15.4 for 15.0, 9 14.2 for 13.95), at run time elsewhere (filters 15 and 17, whose slices are 8 channels: by
+// template no faster when measured with bands).
 // The kernel template and its per-filter-size launcher; dwconv_fwd2_k<K>.hip instantiate it, one file per size.
 #pragma once
 #include <algorithm>

@@ -29,13 +29,12 @@
 // double-buffered LDS tile (pixel-major, one dword of padding per 4 pixels keeps the 4-byte scatter free of bank conflicts) and
 // leave as 16-byte stores, one step behind the MFMAs.
 //
-// What bounds it: the instructions that move data.  A step of 8 rows (of 64 columns and 16 channels) is 1024 cycles of products
-// on a SIMD, about 1100 of LDS accesses on the compute unit and, with two wavefronts to a SIMD that wait for one another,
-// whatever vector arithmetic a wavefront has: dependent instructions are 8 cycles apart.  Hence rows are counted with scalars
-// (images a multiple of 8 rows apart, so that a step or pass meets a boundary as a whole), LDS writes are 8 bytes with constant
-// offsets, and the pieces that move data are written between the products.  115 vector instructions a step became 64 and
-// [8,56,56,64], filter 13, in 8 long runs 1.15 us a step 0.97; what does not overlap yet is the LDS round trips either side of
-// the barrier.
+// What bounds it: the instructions that move data, and waiting.  By the counters ([128,56,56,64] filter 13, 47 k cycles) the LDS is
+// busy 41 % of the cycles, the matrix pipe 33 and the vector ALU 31, and a wavefront, two to a SIMD, waits for data or a barrier a
+// third of its time and for its turn to issue another third.  Hence rows are counted with scalars (images a multiple of 8 rows
+// apart, so that a step or pass meets a boundary as a whole), LDS writes are 8 bytes with constant offsets, and the pieces that
+// move data are written between the products.  115 vector instructions a step became 64 and [8,56,56,64], filter 13, in 8 long
+// runs 1.15 us a step 0.97; what does not overlap yet is the LDS round trips either side of the barrier.
 //
 // MODE is a set of bits.
 // 1 (input gradient of a tensor that was also average-pooled 2x2): y += add[i/2, j/2] / 4 in the store.
@@ -50,7 +49,7 @@
 // halves of its piece.
 //
 // Zero entries of A multiply real pixels of the window (and the window is wider than K+3 where (K+3) % 8 != 0), so a
-// non-finite input value reaches outputs up to 3 + 8 ICB - (K+3) pixels beyond its K x K footprint as NaN.
+// non-finite input value reaches outputs of its own image up to 3 + 8 ICB - (K+3) pixels beyond its K x K footprint as NaN.
 #pragma once
 #include <algorithm>
 #include <mutex>
@@ -749,8 +748,9 @@ inline int tz_steps(const TzGeom& g) {
     return (g.run % g.stack == 0 ? g.run - g.stack + g.OH + 7 : g.run) / 8;
 }
 
-// Estimated time of a workgroup, us, on a chip full of them: a start-up (first windows, filter table, operand set-up), then
-// steps of 8 rows.
+// Price of a workgroup to the planners, us: a start-up (first windows, filter table, operand set-up), then steps of 8 rows.  (The
+// step is that of runs which have the memory to themselves.  256 equal runs at once take 6.1 + 1.47 a step at [64,H,56,64] filter 13,
+// 5.5 + 1.36 at filter 9, 5.9 + 1.2 at filter 15 with its 8 channels; with the pooled gradient 6.1 + 1.8, 5.7 + 1.6 and 6.1 + 1.35.)
 constexpr double kTzStart = 7.0, kTzStep = 0.9;
 inline double tz_run_cost(const TzGeom& g) { return kTzStart + kTzStep * tz_steps(g); }
 

@@ -8,11 +8,13 @@
 // vectors: A holds X_{r+v} (index v, k group = one of 4 phases), B holds G_r of 16 rows (index = row mod 16).  One
 // accumulator of 4 registers holds all taps of a channel, a row takes 2 products (8 phases) per channel.
 //
-// What bounds it: LDS reads.  B stays in registers: from one row of x to the next only the gy row that enters changes (GR rows
-// at a time, one read and four selects), so that a product costs one 16-byte LDS read per lane (4 cycles) instead of three
-// (the form of dwconv_wgrad_tz.h: 11 cycles).  The index of a gy row in B is fixed while u = rho - row moves with rho: there
-// are 8 accumulators, by rho mod 8, whose lanes are rotated against each other when they are added at the end (DPP row
-// rotates), and B itself is rotated by 8 lanes once in 8 rows.
+// What bounds it: the LDS before anything else.  By the counters ([128,56,56,64] filter 13, 16 passes a run) it is busy 51 % of the
+// cycles, a quarter of that bank conflicts, the vector ALU 26 % and the matrix pipe 21 %; wavefronts wait for their turn at the
+// LDS a fifth of their time and for data or a barrier a third.  B stays in registers: from one row of x to the next only the
+// gy row that enters changes (GR rows at a time, one read and four selects), so that a product costs one 16-byte LDS read per
+// lane (4 cycles) instead of three (the form of dwconv_wgrad_tz.h: 11 cycles).  The index of a gy row in B is fixed while
+// u = rho - row moves with rho: there are 8 accumulators, by rho mod 8, whose lanes are rotated against each other when they are
+// added at the end (DPP row rotates), and B itself is rotated by 8 lanes once in 8 rows.
 //
 // Rows are streamed through LDS in passes of 8 (double-buffered, requested two passes ahead).  The images of a batch are
 // stacked into one column of rows, `per` rows apart with at least PH rows of zeros between them, and a workgroup takes a
@@ -20,10 +22,10 @@
 // Tiles of 64 columns of an image, or of 32 columns of two images side by side (the halves of the vectors).
 // Fixed-order summation of the workgroups' partials (wgrad_reduce_parts), no atomics.
 //
-// us with the summation, against the form of dwconv_wgrad_tz.h: [8,64,64,1152] filter 9 133 -> 47 (its tiles are 56 columns
-// wide, 1152 workgroups of one start-up each; 151 MB at 3.6 TB/s now), [32,56,56,64] filter 13 19.2 -> 17.7, [128,56,56,64]
-// 50 -> 37, [128,7,7,1152] filter 3 163 -> 37.  A pass costs 1.3 us (filters 10-15, of it LDS reads 0.6, the staging's writes
-// and shuffles 0.4, what of the products does not overlap 0.1) or 1.05 (up to 9), a run 4-7 us besides.
+// us of the kernel (the summation is 4 more), against the form of dwconv_wgrad_tz.h: [8,64,64,1152] filter 9 139 -> 47 (its tiles are
+// 56 columns wide, 1152 workgroups of one start-up each; 151 MB at 3.2 TB/s now), [32,56,56,64] filter 13 17.6 -> 15.4,
+// [128,56,56,64] 50 -> 37, [128,7,7,1152] filter 3 166 -> 34.  With all of the chip in such runs a pass takes 1.8 us and a run 8 besides
+// (4, 16 and 23 passes of 64 columns in the first three).
 #pragma once
 #include <mutex>
 
@@ -340,8 +342,8 @@ inline bool wgrad_ph_cut(WgPhPlan& p, int n) {
     return most * big <= 0x1fffffffLL && p.nblocks <= 0x7fffffffLL && (long long)g.nchunks * g.ncolt <= 0x7fffffffLL;
 }
 
-// Estimated time of a run, us, on a chip full of them: start-up (16 gy rows, two round trips to memory, the partial), then
-// passes of 8 rows.
+// Price of a run to the planners, us: start-up (16 gy rows, two round trips to memory, the partial), then passes of 8 rows.  (Of runs
+// that share the chip with other problems; see the top for a chip full of them.)
 constexpr double kWgPhStart = 7.0;
 inline double wgrad_ph_step(int K) { return K <= 9 ? 1.15 : 1.35; }
 inline double wgrad_ph_run_cost(int K, int passes) { return kWgPhStart + wgrad_ph_step(K) * passes; }
