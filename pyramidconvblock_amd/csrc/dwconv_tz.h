@@ -53,6 +53,7 @@
 #pragma once
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "common.h"
 #include "kernels.h"
@@ -164,6 +165,14 @@ __device__ __forceinline__ uint2 tz_gate(uint2 a, uint2 b, float s) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) uo.t[i] = from_f32<T>(gate_f32(to_f32(ua.t[i]), to_f32(ub.t[i]), s));
     return uo.u;
+}
+
+// f(0), f(1), ... f(N - 1) with constants, until one of them answers false.
+template <int J, int N, typename F>
+__device__ __forceinline__ void tz_in_turn(F& f) {
+    if constexpr (J < N) {
+        if (f(std::integral_constant<int, J>())) tz_in_turn<J + 1, N>(f);
+    }
 }
 
 // One workgroup's run: `blk` of the problem's `nblk` workgroups.
@@ -576,8 +585,7 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
     for (int j = 0; j < PER - 1; ++j) load_group(j, 4 * j * RP);
     // A step is two row groups (8 output rows), UNRF steps (the ring's period in steps) a trip.
     const int nfat = (nsteps + 1) >> 1;
-    int last = nfat - 1;
-    auto step = [&](int jf, int f) {
+    auto step = [&](int jf, int f) __attribute__((always_inline)) {
         // the two row groups this step adds to the ring; the second goes to the slot of the step's own first group, once the
         // first tile's products with that are issued (LATE), or waits in registers where those are nearly all there are
         constexpr bool LATE = PER >= 3;
@@ -668,30 +676,30 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
             }
         }
     };
-    if constexpr (UNRF == 2) {
-        // A run's odd last step by itself: with a way out between the two steps of a trip the compiler no longer knows which
-        // requests are the newest, and every other commit waited for those of the step before as well (us: [32,56,56,128] filter
-        // 13 17.0 -> 16.6, [16,32,32,64] 7.25 -> 6.85, [1,56,56,64] 6.35 -> 6.0).
-        int f = 0;
-        for (; f + 2 <= nfat; f += 2) {
-            lds_barrier();  // the previous step's tiles are complete, its window reads done
-            step(0, f);
-            lds_barrier();
-            step(1, f + 1);
-        }
-        if (f < nfat) {
-            lds_barrier();
-            step(0, f);
-        }
-    } else {   // left after the run's last step by a uniform exit between steps
+    auto any = [&](int jf, int f) __attribute__((always_inline)) {
+        lds_barrier();  // the previous step's tiles are complete, its window reads done
+        step(jf, f);
+    };
+    int last = 0;   // (the parity known where it is set: 188 registers at filter 17, 231 with nfat - 1)
+    if constexpr (UNRF <= 6) {
+        // Whole trips, then what is left of the run by itself: with a way out between the steps of a trip the compiler no longer
+        // knows which requests are the newest, and commits waited for those of the step before as well (us: [32,56,56,128] filter 13
+        // 17.0 -> 16.6, 9 15.5 -> 15.0, 7 15.3 -> 14.8; [16,32,32,64] 7.25 -> 6.9, 6.6 -> 6.3, 6.4 -> 6.15).  In turn and not by the
+        // compiler's unrolling, which gives up on a loop with so many ways out.
+        int f0 = 0;
+        auto trip = [&](auto jf) { return any(jf, f0 + jf), last = f0 + jf, true; };
+        auto left = [&](auto jf) { return f0 + jf < nfat && trip(jf); };   // (uniform)
+        for (; f0 + UNRF <= nfat; f0 += UNRF) tz_in_turn<0, UNRF>(trip);
+        tz_in_turn<0, UNRF - 1>(left);
+    } else {
+        // Ten steps a trip, left after the run's last step: few runs take a second one, and nine more steps of code cost more than
+        // the waits (us, [32,56,56,128] filter 17 25.6 and 25.8, [32,28,28,64] 9.15 and 9.35).
         bool left = false;
-        last = -1;   // (set where a trip is left, with its parity known there: 188 registers at filter 17, 231 with nfat - 1)
         for (int f0 = 0; f0 < nfat; f0 += UNRF) {
 #pragma unroll
             for (int jf = 0; jf < UNRF; ++jf) {
-                lds_barrier();
-                step(jf, f0 + jf);
-                if (f0 + jf + 1 >= nfat) {
+                any(jf, f0 + jf);
+                if (f0 + jf + 1 >= nfat) {   // (uniform)
                     left = true, last = f0 + jf;
                     break;
                 }
