@@ -134,7 +134,7 @@ struct TzGeom : TzRuns {
     int OH, OW;        // output extents
     int PH, PW;        // padding
     int ncolt, nslices;
-    int part, stack;   // (host) rows that runs by image divide; rows from one image to the next in the stack (0: no stack)
+    int stack;         // (host) rows from one image to the next in the stack (0: no stack)
     int flip;          // 1: 180-degree rotated filter (input gradient)
     int AH, AW;        // extents of the half-resolution addend / pooled output
     int YC, ych;       // output pixel stride in channels, first output channel
@@ -731,14 +731,18 @@ inline bool tz_wide_tile(int B, int OW) {
 // Rows of the stack (of one image where there is none).
 inline int tz_rows(const TzGeom& g, int ni) { return g.stack ? (cdiv(g.B, ni) - 1) * g.stack + g.OH : g.OH; }
 
-// Cuts the stack into runs of `run` rows (a multiple of 8), by the image where that divides its rows or there is no stack; false:
-// a run's images are beyond 32-bit offsets.
+// Cuts the stack into runs of `run` rows (a multiple of 8), or every image by itself where that makes no more of them (its last
+// run may be shorter, and none needs the rows between two images) or there is no stack; false: a run's images are beyond 32-bit
+// offsets.  (us, by the image only where the run divided the image's rows of the stack, and now: [32,28,28,64] filter 17 9.4 -> 8.5,
+// 15 9.4 -> 8.55; both scales of [8,112,112,48], filter 17, 16.1 -> 15.2; elsewhere the same.)
 inline bool tz_cut(TzGeom& g, int ni, long long run) {
     const int images = cdiv(g.B, ni), total = tz_rows(g, ni);
     if (run > total) run = (total + 7) / 8 * 8;
-    g.run = (int)run, g.rpi = !g.stack || g.part % g.run == 0 ? cdiv(g.OH, g.run) : 0;
-    if ((long long)images * g.rpi > 0x7fffffffLL) return false;
-    g.nruns = g.rpi ? images * g.rpi : cdiv(total, g.run);
+    g.run = (int)run, g.rpi = cdiv(g.OH, g.run);
+    const long long alone = (long long)images * g.rpi;
+    if (g.stack && alone > cdiv(total, g.run)) g.rpi = 0;
+    if (g.rpi && alone > 0x7fffffffLL) return false;
+    g.nruns = g.rpi ? (int)alone : cdiv(total, g.run);
     const long long reach = g.rpi ? ni : ((long long)(g.stack + g.run + 64) / g.stack + 1) * ni, most = reach < g.B ? reach : g.B;
     const long long in = (long long)g.H * g.W * g.C, out = (long long)g.OH * g.OW * g.YC;
     // the kernel's quotients of workgroups: by slices, tiles and runs
@@ -763,7 +767,7 @@ constexpr double kTzStart = 7.0, kTzStep = 0.9;
 inline double tz_run_cost(const TzGeom& g) { return kTzStart + kTzStep * tz_steps(g); }
 
 // The cut with the fewest workgroups whose runs have at most `steps` steps (of equal ones the shorter runs): runs of any length,
-// whole images, or equal parts of an image (those that start with an image need no steps for the rows between two).
+// whole images, or equal parts of an image.
 inline bool tz_cut_steps(TzGeom& g, int ni, int steps) {
     long long best = 0, best_blocks = 0;
     int best_steps = 0;
@@ -772,17 +776,14 @@ inline bool tz_cut_steps(TzGeom& g, int ni, int steps) {
         const long long n = tz_blocks(g);
         if (best == 0 || n < best_blocks || (n == best_blocks && tz_steps(g) < best_steps)) best = run, best_blocks = n, best_steps = tz_steps(g);
     };
-    const int per_image = cdiv(g.OH, 8), group = g.part / 8;
+    const int per_image = cdiv(g.OH, 8);
     look(8LL * steps);
-    if (steps >= per_image) {
+    if (steps < per_image) {
+        look(8LL * cdiv(per_image, cdiv(per_image, steps)));
+    } else {
         const long long n = g.stack ? (steps - per_image) / (g.stack / 8) + 1 : 1;
-        look(n == 1 ? g.part : n * g.stack);
+        look(n == 1 ? 8LL * per_image : n * g.stack);
     }
-    for (int j = 2; j <= group; ++j)
-        if (group % j == 0 && group / j <= steps) {
-            look(g.part / j);
-            break;
-        }
     return best != 0 && tz_cut(g, ni, best);
 }
 
@@ -790,7 +791,7 @@ inline bool tz_cut_steps(TzGeom& g, int ni, int steps) {
 // end first; false: not covered.
 inline bool tz_cut_alone(TzGeom& g, int ni) {
     const long long per_run = (long long)g.ncolt * g.nslices;
-    const int images = cdiv(g.B, ni), group = g.part / 8;
+    const int images = cdiv(g.B, ni), per_image = cdiv(g.OH, 8);
     const long long total = cdiv(tz_rows(g, ni), 8) * (g.stack ? 1LL : images);
     long long best = 0;
     double best_cost = 0;
@@ -803,11 +804,9 @@ inline bool tz_cut_alone(TzGeom& g, int ni) {
         const long long most = 256LL * rounds, want = most / per_run, n = want < 1 ? 1 : want > total ? total : want;
         look(8LL * cdiv(total, n), most);
         if (n < images) {
-            look(g.stack ? (long long)cdiv(images, n) * g.stack : g.part, most);   // whole images
+            look(g.stack ? (long long)cdiv(images, n) * g.stack : 8LL * per_image, most);   // whole images
         } else {
-            int j = (int)std::min<long long>(n / images, group);   // equal parts of an image
-            while (group % j) --j;
-            look(g.part / j, most);
+            look(8LL * cdiv(per_image, std::min<long long>(n / images, per_image)), most);   // equal parts of an image
         }
     }
     // (large images: runs as short as their offsets need)
@@ -824,10 +823,9 @@ static bool tz_make_geom(TzGeom& g, bool add, int B, int H, int W, int C, int PH
     g.YC = gate ? gate->ldy : C, g.ych = gate ? gate->ych : 0, g.gs = gate ? gate->gs : 1.f;
     if (gate && (add || flip || C % 16 != 0 || gate->ldy < gate->ych + C / 2 || (gate->ldy | gate->ych) % 8 != 0)) return false;
     if ((long long)H * W * C * Sh::NI > 0x1fffffffLL || (long long)g.OH * g.OW * g.YC * Sh::NI > 0x1fffffffLL) return false;
-    g.part = (std::max(H + PH, g.OH) + 7) / 8 * 8;
     // the windows of an image's first patches reach PH rows above it, and the operands of its last, output rows 4 * ((OH - 1) / 4)
     // on, OPR rows from PH above those: none of them the neighbour's
-    g.stack = std::max(g.part, (4 * ((g.OH - 1) / 4) - PH + Sh::OPR + 7) / 8 * 8);
+    g.stack = (std::max(std::max(H + PH, g.OH), 4 * ((g.OH - 1) / 4) - PH + Sh::OPR) + 7) / 8 * 8;
     // the kernel's quotients of rows of the stack by this are exact up to 2^32 / stack; images too tall for that are walked one by
     // one (a run of one such image is thousands of steps: nothing is lost)
     const long long rows = (long long)cdiv(B, Sh::NI) * g.stack;
