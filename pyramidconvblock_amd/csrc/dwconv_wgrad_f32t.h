@@ -156,9 +156,8 @@ __device__ __forceinline__ void dwconv_wgrad_f32_body(const float* __restrict__ 
                     if (++cur.band == g.nbands) cur.band = 0, cur.b += NI;
                 }
                 open();
-            } else {   // past the last unit: empty descriptors
-                cur.xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x), (short)0, 0, 0x00020000);
-                cur.gr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(gy), (short)0, 0, 0x00020000);
+            } else {   // past the last unit (at most four more requests): rows that no image has, which take no scalar offset
+                cur.orow0 = g.PH - 64, cur.rows = 0, cur.gi = 0;
             }
         }
     };

@@ -15,6 +15,8 @@ pytestmark = pytest.mark.gpu
     ((7, 35, 61, 300), 15),    # two column tiles an image, several chunks of both
     ((2, 70, 25, 16), 17),     # bands of one image, two products a position
     ((1, 5, 90, 12), 11),      # fewer rows than the filter
+    ((1, 90, 8, 16), 15),      # a workgroup's last rows end inside an image, and three of a tile's four images are missing
+    ((3, 120, 20, 8), 13),     # ... the second of two
 ])
 def test_several_units_in_a_workgroup(oracle, shape, k):
     from pyramidconvblock_amd.dwconv import dwconv_wgrad
