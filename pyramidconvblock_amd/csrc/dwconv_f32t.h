@@ -216,7 +216,8 @@ __device__ __forceinline__ void dwconv_f32_body(const float* __restrict__ x, con
         if constexpr (ADD == 1) {
             uint32_t o = aoff;
             if (pr < 0 || 4 * pr + 3 >= rows_valid) o = pr >= 0 && 4 * pr + srow < rows_valid ? o : kNoRow;
-            const int at = pr >= 0 ? ((orow0 + 4 * pr) >> 1) * g.AW * g.C * 4 : 0;
+            // (below the band no scalar offset either: it could lie past the descriptor's end, from which the range check subtracts it)
+            const int at = pr >= 0 && 4 * pr < rows_valid ? ((orow0 + 4 * pr) >> 1) * g.AW * g.C * 4 : 0;
             addv[0] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(arsrc, (int)o, at, 0));
         } else if constexpr (ADD == 2) {
             int ib0;

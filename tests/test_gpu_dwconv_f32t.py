@@ -46,3 +46,17 @@ def test_weight_gradients_of_two_scales_in_one_launch(k, shape, hw):
     geo = ((1, 1), (k // 2, k // 2), (1, 1))
     d0, d1 = dwconv_wgrad_pair(x0, g0, x1, g1, (k, k, C))
     assert torch.equal(d0, dwconv_wgrad(x0, g0, (k, k, C), *geo)) and torch.equal(d1, dwconv_wgrad(x1, g1, (k, k, C), *geo))
+
+
+@pytest.mark.parametrize("k", [3, 9, 17])
+@pytest.mark.parametrize("shape", [(1, 2, 64, 4), (1, 6, 8, 12), (3, 10, 30, 8), (1, 50, 16, 20)])
+def test_pooled_gradient_below_the_last_row(oracle, k, shape):
+    """Exact halves whose last patch row, and those requested after it, lie below the pooled gradient's last row."""
+    from pyramidconvblock_amd.dwconv import dwconv_dgrad
+
+    B, H, W, C = shape
+    gen = torch.Generator().manual_seed(k + H)
+    g, gp, w = randn(gen, *shape), randn(gen, B, H // 2, W // 2, C), randn(gen, k, k, C) / k
+    dx = dwconv_dgrad(g.cuda(), w.cuda(), shape, (1, 1), (k // 2, k // 2), (1, 1), pooled_grad=gp.cuda())
+    want = oracle.dwconv_dgrad(g.double().numpy(), w.double().numpy(), (H, W), 1, k // 2, 1)
+    assert_close(dx, want + oracle.avgpool_bwd(gp.double().numpy(), (H, W)), torch.float32)
