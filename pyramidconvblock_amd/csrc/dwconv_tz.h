@@ -500,15 +500,17 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
         alane[n] = s_ok ? (uint32_t)(((simg * g.AH + (r >> 1)) * g.AW + ((ocol0 + scol) >> 1)) * g.C + c0 + 8 * sh) * 2u : kNoRow;
         yoff[n] = kNoRow, addv[n] = make_uint4(0u, 0u, 0u, 0u);
     }
-    auto place = [&]() {   // the next step: the offsets its tiles are stored at, and the addends
+    // The next step: the offsets its tiles are stored at, and the addends.  (A step between images moves nothing and takes no scalar
+    // offset: behind images of one to three rows it could lie past the descriptor's end, from which the range check subtracts it.)
+    auto place = [&]() {
         const int lim = min(g.OH - orow, rleft);
 #pragma unroll
         for (int n = 0; n < NG; ++n) {
             const bool ok = 4 * tile_of(n) + srow < lim;
             yoff[n] = ok ? ylane[n] : kNoRow;
-            if constexpr (ADD) addv[n] = xload_from(arsrc, ok ? alane[n] : kNoRow, aoff);
+            if constexpr (ADD) addv[n] = xload_from(arsrc, ok ? alane[n] : kNoRow, lim > 0 ? aoff : 0);
         }
-        stored = ooff;
+        stored = lim > 0 ? ooff : 0;
         rleft -= 8, orow += 8;
         const bool wrap = orow >= g.per;
         ooff += wrap ? group_out - (uint32_t)(orow - 8) * row_out : 8u * row_out;

@@ -45,6 +45,32 @@ def test_tall_images_run_by_image(oracle, shape, k, pad):
     assert rel_err(dwconv_dgrad(gy.cuda(), w.cuda(), shape, *geo), want) <= TOL[dtype]
 
 
+@pytest.mark.parametrize("shape", [(9, 2, 12, 32), (40, 2, 40, 64), (5, 3, 7, 48), (70, 3, 64, 32)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_images_shorter_than_a_step(oracle, shape, dtype):
+    """Stacks with whole steps of 8 rows between images of two and three, where the runs' offsets pass the last image: the input
+    gradient with a pooled one, and the gated convolutions of inference."""
+    import pyramidconvblock_amd as pcb
+    from pyramidconvblock_amd.dwconv import dwconv_dgrad
+
+    B, H, W, C = shape
+    gen = torch.Generator().manual_seed(H + W)
+    for k in (15, 17):
+        geo = ((1, 1), (k // 2, k // 2), (1, 1))
+        if H % 2 == 0:
+            gy, gp, w = randn(gen, *shape).to(dtype), randn(gen, B, H // 2, W // 2, C).to(dtype), (randn(gen, k, k, C) / k).to(dtype)
+            want = oracle.dwconv_dgrad(gy.double().numpy(), w.double().numpy(), (H, W), 1, k // 2, 1)
+            got = dwconv_dgrad(gy.cuda(), w.cuda(), shape, *geo, pooled_grad=gp.cuda())
+            assert rel_err(got, want + oracle.avgpool_bwd(gp.double().numpy(), (H, W))) <= TOL[dtype]
+        torch.manual_seed(k)
+        m = pcb.ConvBlock(dim=C, kernel_size=k).to(dtype)
+        x = randn(gen, *shape).to(dtype)
+        params = {n: p.detach().double().numpy() for n, p in m.state_dict().items()}
+        want, _ = oracle.convblock_fwd(x.double().numpy(), params)
+        with torch.no_grad():
+            assert rel_err(m.cuda()(x.cuda()), want) <= TOL[dtype]
+
+
 def test_plans_are_kept_by_shape():
     """More shapes than are kept, twice over and from two threads: every batch gives the results of the whole one."""
     from concurrent.futures import ThreadPoolExecutor
