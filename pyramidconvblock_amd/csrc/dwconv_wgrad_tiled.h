@@ -256,16 +256,16 @@ static WgradPlan plan_wgrad(int B, int H, int W, int C, int PH, int PW) {
 }
 
 // plan_wgrad by shape: the search takes longer than most of the kernels, and every workspace query makes it.
-template <typename T, int K>
+template <typename T, int K, int R>
 static WgradPlan wgrad_plan_of(int B, int H, int W, int C, int PH, int PW) {
     using Key = std::array<int, 6>;
     static PlanCache<Key, WgradPlan> cache;
-    return cache.get(Key{B, H, W, C, PH, PW}, [&] { return plan_wgrad<T, K, WgradCfg<T, K>::R>(B, H, W, C, PH, PW); });
+    return cache.get(Key{B, H, W, C, PH, PW}, [&] { return plan_wgrad<T, K, R>(B, H, W, C, PH, PW); });
 }
 
 template <typename T, int K>
 static size_t wgrad_tiled_workspace_t(int B, int H, int W, int C, int PH, int PW) {
-    const WgradPlan p = wgrad_plan_of<T, K>(B, H, W, C, PH, PW);
+    const WgradPlan p = wgrad_plan_of<T, K, WgradCfg<T, K>::R>(B, H, W, C, PH, PW);
     return p.ok ? (size_t)p.g.nchunks * K * K * C * sizeof(float) : 0;
 }
 
@@ -274,8 +274,7 @@ static int wgrad_tiled_launch_t(const void* x, const void* gy, void* dw, void* w
                                 int PW, hipStream_t s) {
     constexpr int R = WgradCfg<T, K>::R;
     constexpr int USPLIT = WgradCfg<T, K>::USPLIT;
-    static_assert(R == WgradCfg<T, K>::R, "the plan is kept for one patch width");
-    WgradPlan p = wgrad_plan_of<T, K>(B, H, W, C, PH, PW);
+    WgradPlan p = wgrad_plan_of<T, K, R>(B, H, W, C, PH, PW);
     if (!p.ok) return -1;
     WgradGeom& g = p.g;
     const void* ptrs[2] = {x, gy};
