@@ -20,9 +20,9 @@
  *   - Callable from several host threads at once.  The library keeps four pieces of state: the per-thread
  *     error text, the per-thread list of summations recorded between pdw_reduce_defer_begin() and
  *     pdw_reduce_defer_flush(), a once-per-process set-up of each large kernel's LDS limit (guarded by
- *     std::call_once), and a bounded cache of launch plans per shape for the launches that hold several problems (behind a
- *     mutex, emptied when it reaches 256 shapes; a plan is a function of the shape alone, so the cache changes no
- *     result).  The no-allocation entry point
+ *     std::call_once), and bounded caches of launch plans per shape (of the shared launches, the 16-bit matrix-core convolutions and
+ *     the vector-ALU kernels with their workspace queries; each behind a mutex and emptied when it reaches 256 shapes; a plan is a
+ *     function of the shape alone, so they change no result).  The no-allocation entry point
  *     has a device buffer of its own, described there.  The library reads no environment variables: every launch plan
  *     is a function of the arguments.
  *   - Non-finite inputs: the matrix-core convolution kernels multiply a window of input pixels somewhat larger

@@ -2,8 +2,8 @@
 // the kernel launchers.  No allocation, no synchronisation; the only state is the per-thread
 // error text here, the per-thread list of deferred summations (dwconv_direct.hip), the
 // once-per-process LDS-limit set-up next to each large kernel's launcher, the bounded per-shape
-// launch-plan caches of the shared conv launches (dwconv_fwd2.h, dwconv_bwd3.h: a std::map behind a
-// mutex each, emptied at kPlanCacheMax entries) and the per-device address of the static scratch array.
+// launch-plan caches (dwconv_fwd2.h, dwconv_bwd3.h, and PlanCache of tile_common.h in dwconv_tz.h, dwconv_tiled.h,
+// dwconv_wgrad_tiled.h: a std::map behind a mutex each, emptied at kPlanCacheMax entries) and the per-device address of the static scratch array.
 #include <stdarg.h>
 #include <stdio.h>
 
