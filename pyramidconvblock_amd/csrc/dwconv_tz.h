@@ -105,10 +105,16 @@ struct TzShape {
     static constexpr int NR = PER + 1 > 4 ? PER + 1 : 4;
     static constexpr int NRR = 4 * NR;
     static constexpr int CHP = NRR * RP % 16 == 8 ? NRR * RP : NRR * RP + 8;  // bytes per channel plane, = 8 mod 16
-    // behind the planes and the result tiles: where staging lanes without an item write (8 planes apart like an item)
-    static constexpr int SPARE = NI * CS * CHP + R2B;
-    static constexpr size_t lds_bytes = (size_t)SPARE + 7 * CHP + RP + 16;
-    static_assert(lds_bytes <= 160 * 1024, "LDS");
+    static_assert(CHP == NRR * RP + 8, "the spare bytes of a plane");
+    // Where staging lanes without an item write, 8 planes apart like an item: the 8 bytes behind a plane's rows, which nobody reads;
+    // where the pool is written, whose items are two rows, space of its own behind the result tiles.  (With that everywhere a workgroup
+    // of filters 3 and 5, 64 columns wide, had no room for a second one beside it: launches of 257 .. 512 workgroups took 1.13 times as
+    // long, of up to 1024 1.2, beyond 1.36.)
+    static constexpr int ENDS = NI * CS * CHP + R2B;
+    static constexpr int spare(bool pool) { return pool ? ENDS : NRR * RP; }
+    static constexpr size_t lds_bytes = ENDS, lds_bytes_pool = (size_t)ENDS + 7 * CHP + RP + 16;
+    static_assert(lds_bytes_pool <= 160 * 1024, "LDS");
+    static_assert(K > 5 || lds_bytes <= 80 * 1024, "two workgroups on a compute unit");
 };
 
 // 2^32 / d rounded up (0 for 1): n / d = the high half of n times this while n d < 2^32.  (A division costs a wavefront about
@@ -357,7 +363,7 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
         next_group(rb, ob, rb, ob);
     };
     // A pass into the window: the columns of channels 2j and 2j + 1 of the items' rows at ring byte offset cring[l].  No
-    // branch, so that the products around it can be interleaved: lanes without an item write behind the planes (with FEW
+    // branch, so that the products around it can be interleaved: lanes without an item write to spare bytes (with FEW
     // products there is nothing to interleave, and wavefronts without an item write nothing).
     int cring[NLD];
     constexpr int ITEMS = RWMAX / IR * NI * WCQ * NH;
@@ -418,7 +424,7 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
     };
     auto commit_first = [&](const uint4 (&bf)[NLD][IC * IR], int pass) {   // passes 0 and 1
 #pragma unroll
-        for (int l = 0; l < NLD; ++l) cring[l] = irw[l] < RW01 ? idst[l] + (pass * RW01 + irw[l]) % NRR * RP : Sh::SPARE;
+        for (int l = 0; l < NLD; ++l) cring[l] = irw[l] < RW01 ? idst[l] + (pass * RW01 + irw[l]) % NRR * RP : Sh::spare(POOL);
 #pragma unroll
         for (int j = 0; j < 4; ++j) commit_part(bf, j);
         write_pool(bf, pass);
@@ -562,7 +568,7 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
     commit_first(buf[1], 1);
     issue(buf[1], 3);
 #pragma unroll
-    for (int l = 0; l < NLD; ++l) cring[l] = irw[l] < 8 ? idst[l] + (2 * RW01 + irw[l]) % NRR * RP : Sh::SPARE;
+    for (int l = 0; l < NLD; ++l) cring[l] = irw[l] < 8 ? idst[l] + (2 * RW01 + irw[l]) % NRR * RP : Sh::spare(POOL);
     lds_barrier();
     // ---- this wavefront's A operands: lane = (m = 4 di + dj, k group kg); operand t covers k groups 4t .. 4t+3
     uint4 A[CPW][NM];
@@ -849,7 +855,7 @@ static int launch_tz(const void* x, const void* w, const void* add, void* pool, 
         return static_cast<TzRuns>(g);
     });
     if (g.nruns == 0) return -1;
-    const size_t lds = Sh::lds_bytes;
+    const size_t lds = pool ? Sh::lds_bytes_pool : Sh::lds_bytes;
     const int mode = (add ? 1 : 0) | (pool ? 2 : 0) | (gate ? 4 : 0);
     auto kern = dwconv_tz_k<T, K, NPC, CS, 0>;
     if (mode == 1) kern = dwconv_tz_k<T, K, NPC, CS, 1>;
