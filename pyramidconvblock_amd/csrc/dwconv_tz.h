@@ -768,11 +768,11 @@ inline int tz_steps(const TzGeom& g) {
     return (g.run % g.stack == 0 ? g.run - g.stack + g.OH + 7 : g.run) / 8;
 }
 
-// Price of a workgroup to the planners, us: a start-up (first windows, filter table, operand set-up), then steps of 8 rows.  (The
-// step is that of runs which have the memory to themselves.  256 equal runs at once take 6.1 + 1.47 a step at [64,H,56,64] filter 13,
-// 5.5 + 1.36 at filter 9, 5.9 + 1.2 at filter 15 with its 8 channels; with the pooled gradient 6.1 + 1.8, 5.7 + 1.6 and 6.1 + 1.35.)
+// Price of a workgroup to the planners of shared launches, us: a start-up (first windows, filter table, operand set-up), then steps of
+// 8 rows.  (The step is that of runs which have the memory to themselves.  256 equal runs at once take 6.1 + 1.47 a step at
+// [64,H,56,64] filter 13, 5.5 + 1.36 at filter 9, 5.9 + 1.2 at filter 15 with its 8 channels; with the pooled gradient 6.1 + 1.8, 5.7 +
+// 1.6 and 6.1 + 1.35.)
 constexpr double kTzStart = 7.0, kTzStep = 0.9;
-inline double tz_run_cost(const TzGeom& g) { return kTzStart + kTzStep * tz_steps(g); }
 
 // The cut with the fewest workgroups whose runs have at most `steps` steps (of equal ones the shorter runs): runs of any length,
 // whole images, or equal parts of an image.
@@ -795,28 +795,36 @@ inline bool tz_cut_steps(TzGeom& g, int ni, int steps) {
     return best != 0 && tz_cut(g, ni, best);
 }
 
-// Runs of a launch of its own: the shortest with which 256 compute units are filled 1..4 times, whichever number is estimated to
-// end first; false: not covered.
-inline bool tz_cut_alone(TzGeom& g, int ni) {
+// Time of a launch of equal runs by itself, in steps of one that has its compute unit to itself, to its planner: what a unit takes of
+// them, one after the other, each with a start-up; with `pairs` (filters 3 and 5) a unit holds two, which take less than twice as long
+// (us, [1725,8,9,56] filter 3: 27 steps in 256 workgroups 26.5, 13 in 496 22.9, 9 in 768 25.0).
+inline double tz_alone_cost(long long blocks, int steps, bool pairs) {
+    if (!pairs) return (double)cdiv(blocks, 256) * (5.0 + steps);
+    return blocks <= 256 ? 5.0 + steps : 7.5 + 0.8 * steps * cdiv(blocks, 256) + 2.5 * (cdiv(blocks, 512) - 1);
+}
+
+// Runs of a launch of its own: the cut estimated to end first of those that fill 256 compute units 1..8 times, the equal parts of
+// an image and numbers of whole images; false: not covered.  (480 random shapes with all of about 20 cuts timed: the choice is 0.2 %
+// behind the fastest, 0.6 % at filters 3 and 5; at a price of eight steps a start-up, four fillings, and parts or whole images only next
+// to those it was 3 %, 38 % at worst.  us: [16,77,76,232] filter 15 62.8 -> 51, 5 28.9 -> 24.8, [144,8,7,1112] filter 3 43.1 -> 33.)
+inline bool tz_cut_alone(TzGeom& g, int ni, bool pairs = false) {
     const long long per_run = (long long)g.ncolt * g.nslices;
     const int images = cdiv(g.B, ni), per_image = cdiv(g.OH, 8);
     const long long total = cdiv(tz_rows(g, ni), 8) * (g.stack ? 1LL : images);
     long long best = 0;
     double best_cost = 0;
-    auto look = [&](long long run, long long most) {
-        if (!tz_cut(g, ni, run) || (tz_blocks(g) > most && most >= per_run)) return;
-        const double cost = cdiv(tz_blocks(g), 256) * tz_run_cost(g);
+    auto look = [&](long long run) {
+        if (!tz_cut(g, ni, run)) return;
+        const double cost = tz_alone_cost(tz_blocks(g), tz_steps(g), pairs);
         if (best == 0 || cost < best_cost) best = run, best_cost = cost;
     };
-    for (int rounds = 1; rounds <= 4; ++rounds) {
-        const long long most = 256LL * rounds, want = most / per_run, n = want < 1 ? 1 : want > total ? total : want;
-        look(8LL * cdiv(total, n), most);
-        if (n < images) {
-            look(g.stack ? (long long)cdiv(images, n) * g.stack : 8LL * per_image, most);   // whole images
-        } else {
-            look(8LL * cdiv(per_image, std::min<long long>(n / images, per_image)), most);   // equal parts of an image
-        }
+    for (int rounds = 1; rounds <= 8; ++rounds) {
+        const long long want = 256LL * rounds / per_run, n = want < 1 ? 1 : want > total ? total : want;
+        look(8LL * cdiv(total, n));
     }
+    for (int parts = 1; parts <= std::min(per_image, 16); ++parts) look(8LL * cdiv(per_image, parts));
+    if (g.stack)
+        for (int n = 1; n <= std::min(images, 16); ++n) look((long long)n * g.stack);
     // (large images: runs as short as their offsets need)
     return tz_cut(g, ni, best == 0 ? 8 : best) && tz_blocks(g) <= 0x7fffffffLL;
 }
@@ -849,9 +857,10 @@ static int launch_tz(const void* x, const void* w, const void* add, void* pool, 
     TzGeom g;
     if (!tz_make_geom<K, NPC, CS>(g, add != nullptr, B, H, W, C, PH, PW, flip, gate)) return -1;
     // (the search takes a quarter of a microsecond of the call, which a short kernel does not hide: 0.21-0.26 us, kept 0.02)
-    static PlanCache<std::array<int, 7>, TzRuns> plans;
-    static_cast<TzRuns&>(g) = plans.get({B, H, W, C, PH, PW, g.YC}, [g]() mutable {
-        if (!tz_cut_alone(g, Sh::NI)) g.nruns = 0;
+    const bool pairs = K <= 5 && !pool;
+    static PlanCache<std::array<int, 8>, TzRuns> plans;
+    static_cast<TzRuns&>(g) = plans.get({B, H, W, C, PH, PW, g.YC, pairs}, [=]() mutable {
+        if (!tz_cut_alone(g, Sh::NI, pairs)) g.nruns = 0;
         return static_cast<TzRuns>(g);
     });
     if (g.nruns == 0) return -1;
