@@ -47,6 +47,7 @@
 // With 8 channels per workgroup (filters from 15 on) the slice is 4 channels of each half: every 16-byte load of the
 // staging and of the filter becomes two 8-byte loads C bytes apart, and a pixel's one store thread gates the two
 // halves of its piece.
+// 8: with any of these but the pool, runs of no more than tz_short(K) steps.
 //
 // Zero entries of A multiply real pixels of the window (and the window is wider than K+3 where (K+3) % 8 != 0), so a
 // non-finite input value reaches outputs of its own image up to 3 + 8 ICB - (K+3) pixels beyond its K x K footprint as NaN.
@@ -173,6 +174,13 @@ __device__ __forceinline__ uint2 tz_gate(uint2 a, uint2 b, float s) {
     return uo.u;
 }
 
+// Steps of a run up to which MODE 8 is there (0: never).  A run's last steps request passes past its window, which move nothing
+// but take their turn at the address unit, in front of the run's result stores; left out as constants, since with a branch the compiler
+// no longer knows which requests are the newest, and not beside the general code, which then has 36 registers more (us: [108,10,13,40]
+// filter 5, two steps, 5.8 -> 5.3, [2,33,44,440] filter 3 6.0 -> 5.6; [18,7,7,224] filter 15, one step, 6.45 -> 5.95, [4,8,10,176]
+// filter 17 6.15 -> 6.05; with bands of one image, which requested nothing past a window, 5.35, 5.65, 6.15 and 6.0).
+constexpr int tz_short(int K) { return K <= 5 ? 2 : K >= 15 ? 1 : 0; }
+
 // f(0), f(1), ... f(N - 1) with constants, until one of them answers false.
 template <int J, int N, typename F>
 __device__ __forceinline__ void tz_in_turn(F& f) {
@@ -191,7 +199,9 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
     constexpr int NI = Sh::NI, TW = Sh::TW, NH = Sh::NH, CPW = Sh::CPW, RP = Sh::RP, OPX = Sh::OPX, OROWP = Sh::OROWP;
     constexpr int OLB = Sh::OLB, WTH = Sh::WTH, WTW = Sh::WTW, NR = Sh::NR, NRR = Sh::NRR, CHP = Sh::CHP;
     constexpr bool ADD = (MODE & 1) != 0, POOL = (MODE & 2) != 0, GATE = (MODE & 4) != 0;
+    constexpr int SHORT = (MODE & 8) != 0 ? tz_short(K) : 0, PASSES = SHORT ? SHORT + 1 : 4;   // steps of a run at most; passes before them
     static_assert(!GATE || !ADD, "the gate is a forward mode");
+    static_assert(!(SHORT && POOL), "short runs do not write the pool");
     // the gate pairs channel c with channel C/2 + c: a 16-channel slice is 8 channels of each half of C (its two
     // 8-channel pieces), an 8-channel slice 4 of each (the halves of its one piece, moved as two 8-byte accesses)
     constexpr bool G8 = GATE && CS == 8;
@@ -564,9 +574,9 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
     };
     // the passes the first step reads, then the ring's first PER - 1 row groups
     commit_first(buf[0], 0);
-    issue(buf[0], 2);
+    if constexpr (PASSES > 2) issue(buf[0], 2);
     commit_first(buf[1], 1);
-    issue(buf[1], 3);
+    if constexpr (PASSES > 3) issue(buf[1], 3);
 #pragma unroll
     for (int l = 0; l < NLD; ++l) cring[l] = irw[l] < 8 ? idst[l] + (2 * RW01 + irw[l]) % NRR * RP : Sh::spare(POOL);
     lds_barrier();
@@ -593,7 +603,9 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
     for (int j = 0; j < PER - 1; ++j) load_group(j, 4 * j * RP);
     // A step is two row groups (8 output rows), UNRF steps (the ring's period in steps) a trip.
     const int nfat = (nsteps + 1) >> 1;
-    auto step = [&](int jf, int f) __attribute__((always_inline)) {
+    // (commits: a step follows; issues: passes from f + 4 on may lie in the window)
+    auto step = [&](int jf, int f, auto commits, auto issues) __attribute__((always_inline)) {
+        constexpr bool COMMITS = decltype(commits)::value, ISSUES = decltype(issues)::value;
         // the two row groups this step adds to the ring; the second goes to the slot of the step's own first group, once the
         // first tile's products with that are issued (LATE), or waits in registers where those are nearly all there are
         constexpr bool LATE = PER >= 3;
@@ -649,11 +661,11 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
 #pragma unroll
             for (int piece = 0; piece < 7; ++piece) {
                 if (t != (piece * MOVE < NM - 1 ? piece * MOVE : NM - 1)) continue;
-                if (piece >= 2 && piece < 6) commit_part(buf[jf % 2], piece - 2);   // pass f + 2 sits in buffer f % 2 = jf % 2 (UNRF is even)
-                if (piece == 6) {
+                if (COMMITS && piece >= 2 && piece < 6) commit_part(buf[jf % 2], piece - 2);   // pass f + 2 sits in buffer f % 2 = jf % 2 (UNRF is even)
+                if (COMMITS && piece == 6) {
                     commit_next();
                     write_pool(buf[jf % 2], f + 2);
-                    issue(buf[jf % 2], f + 4);
+                    if constexpr (ISSUES) issue(buf[jf % 2], f + 4);
                 }
                 if (piece == 0 && !FEW) tiles_store();
                 if (piece == 1) place();
@@ -684,18 +696,25 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
             }
         }
     };
-    auto any = [&](int jf, int f) __attribute__((always_inline)) {
+    constexpr std::true_type yes;
+    constexpr std::false_type no;
+    auto any = [&](int jf, int f, auto commits, auto issues) __attribute__((always_inline)) {
         lds_barrier();  // the previous step's tiles are complete, its window reads done
-        step(jf, f);
+        step(jf, f, commits, issues);
     };
     int last = 0;   // (the parity known where it is set: 188 registers at filter 17, 231 with nfat - 1)
-    if constexpr (UNRF <= 6) {
+    if constexpr (SHORT == 2) {
+        if (nfat == 2) any(0, 0, yes, no), any(1, 1, no, no), last = 1;   // (uniform)
+        else any(0, 0, no, no);
+    } else if constexpr (SHORT == 1) {
+        any(0, 0, no, no);
+    } else if constexpr (UNRF <= 6) {
         // Whole trips, then what is left of the run by itself: with a way out between the steps of a trip the compiler no longer
         // knows which requests are the newest, and commits waited for those of the step before as well (us: [32,56,56,128] filter 13
         // 17.0 -> 16.6, 9 15.5 -> 15.0, 7 15.3 -> 14.8; [16,32,32,64] 7.25 -> 6.9, 6.6 -> 6.3, 6.4 -> 6.15).  In turn and not by the
         // compiler's unrolling, which gives up on a loop with so many ways out.
         int f0 = 0;
-        auto trip = [&](auto jf) { return any(jf, f0 + jf), last = f0 + jf, true; };
+        auto trip = [&](auto jf) { return any(jf, f0 + jf, yes, yes), last = f0 + jf, true; };
         auto left = [&](auto jf) { return f0 + jf < nfat && trip(jf); };   // (uniform)
         for (; f0 + UNRF <= nfat; f0 += UNRF) tz_in_turn<0, UNRF>(trip);
         tz_in_turn<0, UNRF - 1>(left);
@@ -706,7 +725,7 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
         for (int f0 = 0; f0 < nfat; f0 += UNRF) {
 #pragma unroll
             for (int jf = 0; jf < UNRF; ++jf) {
-                any(jf, f0 + jf);
+                any(jf, f0 + jf, yes, yes);
                 if (f0 + jf + 1 >= nfat) {   // (uniform)
                     left = true, last = f0 + jf;
                     break;
@@ -865,7 +884,8 @@ static int launch_tz(const void* x, const void* w, const void* add, void* pool, 
     });
     if (g.nruns == 0) return -1;
     const size_t lds = pool ? Sh::lds_bytes_pool : Sh::lds_bytes;
-    const int mode = (add ? 1 : 0) | (pool ? 2 : 0) | (gate ? 4 : 0);
+    const bool brief = !pool && tz_steps(g) <= tz_short(K);
+    const int mode = (add ? 1 : 0) | (pool ? 2 : 0) | (gate ? 4 : 0) | (brief ? 8 : 0);
     auto kern = dwconv_tz_k<T, K, NPC, CS, 0>;
     if (mode == 1) kern = dwconv_tz_k<T, K, NPC, CS, 1>;
     if (mode == 2) kern = dwconv_tz_k<T, K, NPC, CS, 2>;
@@ -873,8 +893,13 @@ static int launch_tz(const void* x, const void* w, const void* add, void* pool, 
     if constexpr (CS == 16) {
         if (mode == 6) kern = dwconv_tz_k<T, K, NPC, CS, 6>;
     }
-    if (mode == 3 || mode == 5 || mode == 7 || (mode == 6 && CS != 16)) return -1;
-    static std::once_flag attr_once[8];
+    if constexpr (tz_short(K) != 0) {
+        if (mode == 8) kern = dwconv_tz_k<T, K, NPC, CS, 8>;
+        if (mode == 9) kern = dwconv_tz_k<T, K, NPC, CS, 9>;
+        if (mode == 12) kern = dwconv_tz_k<T, K, NPC, CS, 12>;
+    }
+    if ((mode & 7) == 3 || (mode & 7) == 5 || (mode & 7) == 7 || (mode == 6 && CS != 16)) return -1;
+    static std::once_flag attr_once[16];
     std::call_once(attr_once[mode], [&] { (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); });
     hipLaunchKernelGGL(kern, dim3((unsigned)tz_blocks(g)), dim3(Sh::NT), lds, s, (const T*)x, (const T*)w, (const T*)add,
                        (T*)pool, (T*)y, g);

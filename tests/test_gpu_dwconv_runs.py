@@ -71,6 +71,47 @@ def test_images_shorter_than_a_step(oracle, shape, dtype):
             assert rel_err(m.cuda()(x.cuda()), want) <= TOL[dtype]
 
 
+@pytest.mark.parametrize("k", [3, 5, 15, 17])
+@pytest.mark.parametrize("H,W,C", [(2, 12, 16), (6, 64, 24), (7, 40, 8), (8, 20, 48), (9, 9, 16), (16, 70, 40), (14, 14, 264)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_short_runs(k, H, W, C, dtype):
+    """Few images, whose runs are one or two steps long, by themselves and in a batch of long runs: the same bits."""
+    from pyramidconvblock_amd.dwconv import dwconv_dgrad, dwconv_forward
+
+    B, few = 12000 * 64 // (H * W * C) * 16 + 40, 5
+    gen = torch.Generator().manual_seed(k + H)
+    w, geo = (randn(gen, k, k, C) / k).to(dtype).cuda(), ((1, 1), (k // 2, k // 2), (1, 1))
+    gen = torch.Generator("cuda").manual_seed(k + H)
+    x = torch.randn(B, H, W, C, generator=gen, device="cuda").to(dtype)
+    assert torch.equal(dwconv_forward(x[:few], w, *geo), dwconv_forward(x, w, *geo)[:few])
+    assert torch.equal(dwconv_dgrad(x[:few], w, x[:few].shape, *geo), dwconv_dgrad(x, w, x.shape, *geo)[:few])
+    if H % 2 == 0 and W % 2 == 0:
+        gp = torch.randn(B, H // 2, W // 2, C, generator=gen, device="cuda").to(dtype)
+        whole = dwconv_dgrad(x, w, x.shape, *geo, pooled_grad=gp)
+        assert torch.equal(dwconv_dgrad(x[:few], w, x[:few].shape, *geo, pooled_grad=gp[:few]), whole[:few])
+
+
+@pytest.mark.parametrize("k", [3, 5, 15, 17])
+@pytest.mark.parametrize("H,W,C", [(2, 12, 16), (7, 40, 48), (8, 20, 32), (13, 64, 16)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_short_gated_runs(k, H, W, C, dtype):
+    """The same of the convolution with the gate in its store."""
+    from pyramidconvblock_amd import _lib
+
+    L = _lib.lib()
+    B, few = 12000 * 64 // (H * W * C) * 16 + 40, 5
+    gen = torch.Generator("cuda").manual_seed(k + H)
+    x, w = torch.randn(B, H, W, C, generator=gen, device="cuda").to(dtype), (torch.randn(k, k, C, generator=gen, device="cuda") / k).to(dtype)
+
+    def gated(x):
+        y = torch.empty(*x.shape[:3], C // 2, device="cuda", dtype=dtype)
+        _lib.check(L.pdw_dwconv_fwd_gate(x.data_ptr(), w.data_ptr(), y.data_ptr(), None, len(x), H, W, C, k, k // 2, 0, 0, _lib.dtype_code(dtype),
+                                         _lib.stream_ptr(x.device)))
+        return y
+
+    assert torch.equal(gated(x[:few]), gated(x)[:few])
+
+
 def test_plans_are_kept_by_shape():
     """More shapes than are kept, twice over and from two threads: every batch gives the results of the whole one."""
     from concurrent.futures import ThreadPoolExecutor
