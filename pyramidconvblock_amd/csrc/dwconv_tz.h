@@ -815,10 +815,11 @@ inline bool tz_cut_steps(TzGeom& g, int ni, int steps) {
 }
 
 // Time of a launch of equal runs by itself, in steps of one that has its compute unit to itself, to its planner: what a unit takes of
-// them, one after the other, each with a start-up; with `pairs` (filters 3 and 5) a unit holds two, which take less than twice as long
+// them, one after the other, each with a start-up of 4.5 (of 5 it tied 18 steps in 435 workgroups with 10 in 696 at [16,81,78,232]
+// filter 17: 64 and 54 us; what 256 equal runs at once take says 4.0 to 4.9); with `pairs` (filters 3 and 5) a unit holds two, which take less than twice as long
 // (us, [1725,8,9,56] filter 3: 27 steps in 256 workgroups 26.5, 13 in 496 22.9, 9 in 768 25.0).
 inline double tz_alone_cost(long long blocks, int steps, bool pairs) {
-    if (!pairs) return (double)cdiv(blocks, 256) * (5.0 + steps);
+    if (!pairs) return (double)cdiv(blocks, 256) * (4.5 + steps);
     return blocks <= 256 ? 5.0 + steps : 7.5 + 0.8 * steps * cdiv(blocks, 256) + 2.5 * (cdiv(blocks, 512) - 1);
 }
 
