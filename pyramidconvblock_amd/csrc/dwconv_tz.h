@@ -876,7 +876,7 @@ static int launch_tz(const void* x, const void* w, const void* add, void* pool, 
     using Sh = TzShape<K, NPC, CS>;
     TzGeom g;
     if (!tz_make_geom<K, NPC, CS>(g, add != nullptr, B, H, W, C, PH, PW, flip, gate)) return -1;
-    // (the search takes a quarter of a microsecond of the call, which a short kernel does not hide: 0.21-0.26 us, kept 0.02)
+    // (the search takes 0.66 us of the call, which a short kernel does not hide; kept 0.02)
     const bool pairs = K <= 5 && !pool;
     static PlanCache<std::array<int, 8>, TzRuns> plans;
     static_cast<TzRuns&>(g) = plans.get({B, H, W, C, PH, PW, g.YC, pairs}, [=]() mutable {
