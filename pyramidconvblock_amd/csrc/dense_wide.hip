@@ -6,7 +6,8 @@
 //
 // What bounds it: the matrix pipe from a width of about 600 on, HBM below.  A stage is 128 bytes of the inner dimension
 // (64 values, in fp32 32) of both operands, moved by the direct global-to-LDS loads (16 bytes a lane, no registers in between) into one of two
-// buffers while the other is multiplied; one barrier a stage.  Operands whose inner dimension is not the contiguous one
+// buffers while the other is multiplied; one barrier a stage.  Where a launch leaves compute units with one workgroup each there are
+// four such buffers, since nothing else covers a stage's trip to memory.  Operands whose inner dimension is not the contiguous one
 // (both of the weight gradient, the weight of the input gradient) are staged as they lie and read with
 // ds_read_b64_tr_b16, which hands every lane four values down a column, so there is no transposing pass over memory and
 // no byte shuffling.  The 16-byte pieces of a staged row are permuted by the row (the loads' lanes choose the global piece,
@@ -19,7 +20,9 @@
 // Out-of-range rows, columns and the inner tail read as zero through the buffer descriptors; nothing is branched around.
 #include <stdint.h>
 
+#include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "common.h"
 #include "dense_any_wgrad.h"
@@ -142,6 +145,66 @@ struct Operand {
     }
 };
 
+// Fragments read by hand, for the loop that keeps requests in flight across LDS reads (the compiler would let each such read wait
+// for all of them: it cannot tell the stages apart); the waits are that loop's own.
+template <typename T, int R, bool TR>
+struct HandFragments {
+    typedef Operand<T, R, TR> Op;
+    static constexpr int ES = (int)sizeof(T);
+    static constexpr int READS = TR ? (ES == 4 ? 4 : 2) : 1;   // LDS instructions of a fragment
+    // per lane and in a stage, but for constants: (TR) where fragment t's values of kk = 0 lie, else those of kk = n and t = 0
+    static constexpr int ADDRESSES = TR ? R / 32 : 4;
+    static __device__ __forceinline__ uint32_t at(int n, int lane) {
+        if constexpr (!TR) {
+            const int row = lane & 31;
+            return (uint32_t)(row * kRowBytes + Op::swz(row, 2 * n + (lane >> 5)) * 16);
+        } else if constexpr (ES == 4) {
+            const int col = 32 * n + (lane & 31), row = 4 * (lane >> 5);
+            return (uint32_t)(row * (R * 4) + Op::swz(row, col >> 2) * 16 + (col & 3) * 4);
+        } else {
+            const int g = lane >> 4, i = lane & 15, col = 32 * n + 16 * (g & 1) + 4 * (i & 3), row = 8 * (g >> 1) + (i >> 2);
+            return (uint32_t)(row * (R * 2) + Op::swz(row, col >> 3) * 16 + (col & 7) * 2);
+        }
+    }
+    template <int TILE, int KK>
+    static __device__ __forceinline__ v8s read(uint32_t p) {   // p: stage + at
+        if constexpr (!TR) {
+            v8s f;
+            asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(f) : "v"(p), "n"(TILE * 32 * kRowBytes));
+            return f;
+        } else if constexpr (ES == 4) {
+            float e0, e1, e2, e3;
+            asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(e0) : "v"(p), "n"(8 * KK * R * 4));
+            asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(e1) : "v"(p), "n"((8 * KK + 1) * R * 4));
+            asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(e2) : "v"(p), "n"((8 * KK + 2) * R * 4));
+            asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(e3) : "v"(p), "n"((8 * KK + 3) * R * 4));
+            const v4f v = {e0, e1, e2, e3};
+            return __builtin_bit_cast(v8s, v);
+        } else {
+            v4s h0, h1;
+            asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(h0) : "v"(p), "n"(16 * KK * R * 2));
+            asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(h1) : "v"(p), "n"((16 * KK + 4) * R * 2));
+            return __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+    }
+};
+
+// Until all but the newest N LDS instructions are done, from when on what the others read may be used.
+template <int N, int FM, int FN>
+__device__ __forceinline__ void wait_fragments(v8s (&a)[FM], v8s (&b)[FN]) {
+    asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N < 15 ? N : 15));
+#pragma unroll
+    for (int i = 0; i < FM; ++i) asm volatile("" : "+v"(a[i]));
+#pragma unroll
+    for (int j = 0; j < FN; ++j) asm volatile("" : "+v"(b[j]));
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void for_each(F f) {   // f(0) .. f(N - 1), the index a constant
+    if constexpr (I < N) f(std::integral_constant<int, I>()), for_each<N, I + 1>(f);
+}
+
 struct WideArgs {
     const void *a, *b, *bias;
     const float* rowbias;
@@ -158,7 +221,7 @@ struct WideArgs {
 template <typename T, int BM, int BN>
 constexpr int kWideOccupancy = sizeof(T) == 4 ? (BM * BN <= 64 * 64 ? 4 : BM * BN <= 128 * 64 ? 3 : 2) : 2;
 
-template <typename T, int BM, int BN, bool TA, bool TB, bool PART>
+template <typename T, int BM, int BN, bool TA, bool TB, bool PART, int STAGES = 2>
 __device__ __forceinline__ void wide_gemm_body(const WideArgs& g, int blk, int nblk) {
     typedef Operand<T, BM, TA> OpA;
     typedef Operand<T, BN, TB> OpB;
@@ -189,51 +252,110 @@ __device__ __forceinline__ void wide_gemm_body(const WideArgs& g, int blk, int n
         for (int j = 0; j < FN; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-    a.request(sm, 0, left);
-    b.request(sm + OpA::BYTES, 0, left);
-    for (int st = 0; st < nst; ++st) {
-        lds_char* const cur = sm + (st & 1) * STAGE;
-        lds_char* const nxt = sm + ((st & 1) ^ 1) * STAGE;
-        // this stage has arrived, and every wavefront is done with the buffer that the next one goes to
-        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-        // all fragments of the stage first, then the next stage's requests, then the products: an LDS read behind a
-        // request in program order would wait for it (the compiler cannot tell the two buffers apart)
-        v8s fa[KK][FM], fb[KK][FN];
+    if constexpr (STAGES == 2) {
+        a.request(sm, 0, left);
+        b.request(sm + OpA::BYTES, 0, left);
+        for (int st = 0; st < nst; ++st) {
+            lds_char* const cur = sm + (st & 1) * STAGE;
+            lds_char* const nxt = sm + ((st & 1) ^ 1) * STAGE;
+            // this stage has arrived, and every wavefront is done with the buffer that the next one goes to
+            asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+            // all fragments of the stage first, then the next stage's requests, then the products: an LDS read behind a
+            // request in program order would wait for it (the compiler cannot tell the two buffers apart)
+            v8s fa[KK][FM], fb[KK][FN];
 #pragma unroll
-        for (int kk = 0; kk < KK; ++kk) {
+            for (int kk = 0; kk < KK; ++kk) {
 #pragma unroll
-            for (int i = 0; i < FM; ++i) fa[kk][i] = OpA::frag(cur, wm * FM + i, kk, lane);
+                for (int i = 0; i < FM; ++i) fa[kk][i] = OpA::frag(cur, wm * FM + i, kk, lane);
 #pragma unroll
-            for (int j = 0; j < FN; ++j) fb[kk][j] = OpB::frag(cur + OpA::BYTES, wn * FN + j, kk, lane);
+                for (int j = 0; j < FN; ++j) fb[kk][j] = OpB::frag(cur + OpA::BYTES, wn * FN + j, kk, lane);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (st + 1 < nst) {
+                a.request(nxt, st + 1, left - (st + 1) * BK);
+                b.request(nxt + OpA::BYTES, st + 1, left - (st + 1) * BK);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j) acc[i][j] = mfma(fb[kk][j], fa[kk][i], acc[i][j], T());
         }
-        __builtin_amdgcn_sched_barrier(0);
-        if (st + 1 < nst) {
-            a.request(nxt, st + 1, left - (st + 1) * BK);
-            b.request(nxt + OpA::BYTES, st + 1, left - (st + 1) * BK);
+    } else {
+        // STAGES in LDS and all but two of them on their way: a launch that leaves compute units with one workgroup each has
+        // nothing else to cover a trip to memory with.  Fragments are read one product ahead, across the stages too.
+        typedef HandFragments<T, BM, TA> HA;
+        typedef HandFragments<T, BN, TB> HB;
+        constexpr int LOADS = OpA::NL + OpB::NL, READS = FM * HA::READS + FN * HB::READS, NA = TA ? FM : KK, NB = TB ? FN : KK;
+        static_assert(STAGES > 2 && (STAGES - 2) * LOADS < 64, "requests in flight");
+        const uint32_t lds0 = (uint32_t)(uintptr_t)sm;
+        uint32_t ata[NA], atb[NB];
+#pragma unroll
+        for (int n = 0; n < NA; ++n) ata[n] = lds0 + (TA ? HA::at(wm * FM + n, lane) : HA::at(n, lane) + (uint32_t)(wm * FM * 32 * kRowBytes));
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+            atb[n] = lds0 + OpA::BYTES + (TB ? HB::at(wn * FN + n, lane) : HB::at(n, lane) + (uint32_t)(wn * FN * 32 * kRowBytes));
+        auto request = [&](int st, int slot) {   // (past the last stage: zeros, so that every stage has its requests)
+            a.request(sm + slot * STAGE, st, left - st * BK);
+            b.request(sm + slot * STAGE + OpA::BYTES, st, left - st * BK);
+        };
+        v8s fa[2][FM], fb[2][FN];
+        auto fragments = [&](int slot, auto kk) {
+            const uint32_t buf = (uint32_t)(slot * STAGE);
+            for_each<FM>([&](auto i) { fa[kk & 1][i] = HA::template read<TA ? 0 : i, kk>(buf + ata[TA ? i : kk]); });
+            for_each<FN>([&](auto j) { fb[kk & 1][j] = HB::template read<TB ? 0 : j, kk>(buf + atb[TB ? j : kk]); });
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        constexpr std::integral_constant<int, 0> first;
+#pragma unroll
+        for (int st = 0; st < STAGES - 1; ++st) request(st, st);
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((STAGES - 2) * LOADS) : "memory");
+        fragments(0, first);
+        int slot = 0;
+        for (int st = 0; st < nst; ++st) {
+            const int next = slot + 1 == STAGES ? 0 : slot + 1, before = slot == 0 ? STAGES - 1 : slot - 1;
+            for_each<KK>([&](auto kk) {
+                if constexpr (kk + 1 < KK) {
+                    fragments(slot, std::integral_constant<int, kk + 1>());
+                } else {
+                    // the next stage has arrived, and every wavefront is done with the one before this, whose place is requested into
+                    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((STAGES - 3) * LOADS) : "memory");
+                    fragments(next, first);
+                    request(st + STAGES - 1, before);
+                }
+                wait_fragments<READS>(fa[kk & 1], fb[kk & 1]);
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j) acc[i][j] = mfma(fb[kk & 1][j], fa[kk & 1][i], acc[i][j], T());
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            slot = next;
         }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int kk = 0; kk < KK; ++kk)
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int j = 0; j < FN; ++j) acc[i][j] = mfma(fb[kk][j], fa[kk][i], acc[i][j], T());
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     }
     if constexpr (PART) {
-        float* const out = (float*)g.y + (size_t)sp * g.M * g.N;
+        // through LDS: as they lie in registers a store would write 16 bytes of each of 32 rows
+        constexpr int TP = BN + 4, CPR = BN / 4;
+        __syncthreads();
+        float* const tile = reinterpret_cast<float*>(dsm);
 #pragma unroll
-        for (int i = 0; i < FM; ++i) {
-            const long long m = m0 + (wm * FM + i) * 32 + l32;
-            if (m >= g.M) continue;
+        for (int i = 0; i < FM; ++i)
 #pragma unroll
             for (int j = 0; j < FN; ++j)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int n = n0 + (wn * FN + j) * 32 + 8 * q + 4 * h;
-                    if (n < g.N)
-                        *reinterpret_cast<float4*>(out + m * g.N + n) =
-                            make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
-                }
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<float4*>(tile + ((wm * FM + i) * 32 + l32) * TP + (wn * FN + j) * 32 + 8 * q + 4 * h) =
+                        make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+        __syncthreads();
+        float* const out = (float*)g.y + (size_t)sp * g.M * g.N;
+#pragma unroll
+        for (int j = 0; j < BM * CPR / 256; ++j) {
+            const int s = j * 256 + tid, row = s / CPR, c = s % CPR;
+            if (m0 + row < g.M && n0 + c * 4 < g.N)
+                *reinterpret_cast<float4*>(out + (m0 + row) * g.N + n0 + c * 4) = *reinterpret_cast<const float4*>(tile + row * TP + c * 4);
         }
     } else {
         // bias and per-image row in fp32, then through LDS so that the stores are whole 16-byte pieces in order
@@ -274,9 +396,9 @@ __device__ __forceinline__ void wide_gemm_body(const WideArgs& g, int blk, int n
     }
 }
 
-template <typename T, int BM, int BN, bool TA, bool TB, bool PART>
-__global__ __launch_bounds__(256, (kWideOccupancy<T, BM, BN>)) void wide_gemm_k(WideArgs g) {
-    wide_gemm_body<T, BM, BN, TA, TB, PART>(g, blockIdx.x, gridDim.x);
+template <typename T, int BM, int BN, bool TA, bool TB, bool PART, int STAGES>
+__global__ __launch_bounds__(256, (STAGES == 2 ? kWideOccupancy<T, BM, BN> : 1)) void wide_gemm_k(WideArgs g) {
+    wide_gemm_body<T, BM, BN, TA, TB, PART, STAGES>(g, blockIdx.x, gridDim.x);
 }
 
 // Both products that read the gradient of a layer's output, as one launch: the weight gradient's nw workgroups (tiles of WM x WN
@@ -284,78 +406,116 @@ __global__ __launch_bounds__(256, (kWideOccupancy<T, BM, BN>)) void wide_gemm_k(
 // launch of its own leaves part of the chip idle in its last round and pays the ramp; together they are dealt as one.
 // us, two launches -> one: [100352,128] <- 64 fp32 44.7 -> 41.0, 64 <- 128 48.4 -> 43.0 (153 and 180 MB); [10431,200] <- 104 bf16 13.4
 // -> 8.8; [16384,1152] <- 576 fp16 66.5 -> 61.4, 576 <- 1152 71.7 -> 68.1; [2048,64] <- 32 fp32 8.6 -> 4.9.
-template <typename T, int BM, int BN, int WM, int WN>
-__global__ __launch_bounds__(256, (kWideOccupancy<T, BM, BN>)) void wide_pair_k(WideArgs rows, WideArgs wgrad, AnyWgradArgs any, int nw) {
+template <typename T, int BM, int BN, int WM, int WN, int STAGES>
+__global__ __launch_bounds__(256, (STAGES == 2 ? kWideOccupancy<T, BM, BN> : 1)) void wide_pair_k(WideArgs rows, WideArgs wgrad, AnyWgradArgs any, int nw) {
     const int blk = blockIdx.x;
     if (blk >= nw) {
-        wide_gemm_body<T, BM, BN, false, true, false>(rows, blk - nw, gridDim.x - nw);
+        wide_gemm_body<T, BM, BN, false, true, false, STAGES>(rows, blk - nw, gridDim.x - nw);
     } else if constexpr (WM != 0) {
-        wide_gemm_body<T, WM, WN, true, true, true>(wgrad, blk, nw);
+        wide_gemm_body<T, WM, WN, true, true, true, STAGES>(wgrad, blk, nw);
     } else {
         const int group = blk / any.chunks;
         dense_any_wgrad_body<T>(any, blk - group * any.chunks, group);
     }
 }
 
-template <typename T, int BM, int BN, bool PART>
+template <typename T, int BM, int BN, bool PART, int STAGES>
 constexpr size_t wide_lds() {
-    constexpr size_t stages = (size_t)2 * (BM + BN) * kRowBytes, out = PART ? 0 : (size_t)BM * (BN * sizeof(T) + 16);
+    constexpr size_t stages = (size_t)STAGES * (BM + BN) * kRowBytes, out = (size_t)BM * (BN * (PART ? 4 : sizeof(T)) + 16);
     return stages > out ? stages : out;
 }
 
-template <typename T, int BM, int BN, int WM, int WN>
+// Launches that kDeep stages in LDS are for: 16-bit ones whose workgroups are all on the chip at once with them, and whose sums have
+// `least` stages or more (us, two stages -> four: [2128,920] -> 464, 136 workgroups of 15 stages, 12.0 -> 9.65, [1568,1024] -> 512 11.8 -> 9.2,
+// [3136,768] -> 384 10.1 -> 8.2; of five stages or fewer the same or up to 0.4 more, and in fp32, where the products take longer, 40.5 -> 41.2).
+constexpr int kDeep = 4;
+template <typename T>
+constexpr bool goes_deep(long long n, size_t lds, long long inner, int least) {
+    return sizeof(T) == 2 && inner >= least * kBK<T> && n <= 256LL * (long long)(160 * 1024 / lds);
+}
+
+template <typename T, int BM, int BN, int WM, int WN, int STAGES>
 int pair_go(const WideArgs& rows, const WideArgs& wgrad, const AnyWgradArgs& any, int nw, hipStream_t s) {
-    constexpr size_t a = wide_lds<T, BM, BN, false>(), b = WM != 0 ? wide_lds<T, WM, WN, true>() : 0, lds = a > b ? a : b;
+    constexpr size_t a = wide_lds<T, BM, BN, false, STAGES>(), b = WM != 0 ? wide_lds<T, WM, WN, true, STAGES>() : 0, lds = a > b ? a : b;
+    const long long n = (long long)nw + (long long)rows.mt * rows.nt;
+    if (n > 0x7fffffffLL) return -1;
+    if constexpr (STAGES == kDeep) {
+        if (!goes_deep<T>(n, lds, rows.Kd, 4)) return pair_go<T, BM, BN, WM, WN, 2>(rows, wgrad, any, nw, s);
+    }
     if constexpr (lds > 64 * 1024) {
         static std::once_flag once;
         std::call_once(once, [] {
-            (void)hipFuncSetAttribute((const void*)wide_pair_k<T, BM, BN, WM, WN>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+            (void)hipFuncSetAttribute((const void*)wide_pair_k<T, BM, BN, WM, WN, STAGES>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         });
     }
-    if ((long long)nw + (long long)rows.mt * rows.nt > 0x7fffffffLL) return -1;
-    hipLaunchKernelGGL((wide_pair_k<T, BM, BN, WM, WN>), dim3((unsigned)(nw + rows.mt * rows.nt)), dim3(256), lds, s, rows, wgrad, any, nw);
+    hipLaunchKernelGGL((wide_pair_k<T, BM, BN, WM, WN, STAGES>), dim3((unsigned)n), dim3(256), lds, s, rows, wgrad, any, nw);
     return check_launch("wide_pair");
 }
 
-template <typename T, int BM, int BN, bool TA, bool TB, bool PART>
+template <typename T, int BM, int BN, bool TA, bool TB, bool PART, int STAGES = kDeep>
 int wide_go(const WideArgs& g, hipStream_t s) {
-    constexpr size_t lds = wide_lds<T, BM, BN, PART>();
+    constexpr size_t lds = wide_lds<T, BM, BN, PART, STAGES>();
+    if constexpr (STAGES == kDeep) {
+        if (!goes_deep<T>((long long)g.mt * g.nt * g.splits, lds, PART ? g.kper : g.Kd, PART ? 3 : 6)) return wide_go<T, BM, BN, TA, TB, PART, 2>(g, s);
+    }
     if constexpr (lds > 64 * 1024) {
         static std::once_flag once;
         std::call_once(once, [] {
-            (void)hipFuncSetAttribute((const void*)wide_gemm_k<T, BM, BN, TA, TB, PART>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+            (void)hipFuncSetAttribute((const void*)wide_gemm_k<T, BM, BN, TA, TB, PART, STAGES>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         });
     }
-    hipLaunchKernelGGL((wide_gemm_k<T, BM, BN, TA, TB, PART>), dim3((unsigned)(g.mt * g.nt * g.splits)), dim3(256), lds, s, g);
+    hipLaunchKernelGGL((wide_gemm_k<T, BM, BN, TA, TB, PART, STAGES>), dim3((unsigned)(g.mt * g.nt * g.splits)), dim3(256), lds, s, g);
     return check_launch("wide_gemm");
 }
 
-// Tiles and row ranges of the weight gradient: tiles of 64 where a width is no more than that, and enough ranges for
-// two workgroups on every compute unit, of at least four stages each, whose partials (written and read once more in
-// fp32) are not more traffic than the operands.
+// Tiles and row ranges of the weight gradient: tiles of 64 where a width is no more than that, and the number of ranges that is
+// estimated to end first: a compute unit's stages (0.6 us one of 128 x 128 results, whether it has one workgroup or two in turn), and
+// the partials, written and read once more in fp32.  (With no more partials than are the operands' traffic, 512 workgroups at most,
+// [2128,920]^T [2128,464] was 32 workgroups of 34 stages.  us with the summation, bf16: that product 33.6 -> 15.3, [1568,1024]^T [1568,512]
+// 26.5 -> 16.4, [3136,768]^T [3136,384] 20.3 -> 14.8, [25088,384]^T [25088,192] 19.2 -> 16.5, [16384,1152]^T [16384,576] 42.3 and 42.6; fp32:
+// [2002,1032]^T [2002,516] 40.7 -> 31.6, [1000,512]^T [1000,256] 15.8 -> 9.5.)
 struct WgradPlan {
     int bm, bn, mt, nt, splits;
     long long kper;
 };
-WgradPlan wgrad_plan(long long N, int M, int NO, int es) {
+WgradPlan wgrad_make_plan(long long N, int M, int NO, int es) {
     WgradPlan p{M <= 64 ? 64 : 128, NO <= 64 ? 64 : 128, 0, 0, 0, 0};
-    const long long by_rows = es == 4 ? N / 128 : N / 256, by_traffic = es * N * (M + NO) / (8LL * M * NO);
+    const int bk = kRowBytes / es;
+    const double stage = es == 4 ? 0.5 / (64 * 64) : 0.6 / (128 * 128), partial = 8.0 * M * NO / 3.5e6;   // us: a result's stage, a range's partials
+    const double alone = es == 4 ? 1.3 : 1.0;   // (fp32: of one workgroup a compute unit)
+    double least;
     auto cut = [&] {
         p.mt = cdiv(M, p.bm), p.nt = cdiv(NO, p.bn);
-        long long s = 512 / ((long long)p.mt * p.nt);
-        if (s > by_rows) s = by_rows;
-        if (s > by_traffic) s = by_traffic;
-        return s < 1 ? 1 : s;
+        const long long tiles = (long long)p.mt * p.nt, most = std::min(N / (2 * bk), std::max(1024 / tiles, 1LL));
+        long long best = 1;
+        for (long long s = 1; s <= most || s == 1; s += s < 16 ? 1 : s / 8) {
+            const long long inner = cdiv(cdiv(N, s), bk);
+            const double c = (double)cdiv(tiles * s, 256) * (tiles * s <= 256 ? alone : 1.0) * inner * p.bm * p.bn * stage + partial * s;
+            if (s == 1 || c < least) least = c, best = s;
+        }
+        return best;
     };
     long long s = cut();
-    // fp32, bound by the matrix pipe and not by what the tiles read: smaller ones where these would be too few
-    if (es == 4 && s * p.mt * p.nt < 512) p.bm = p.bn = 64, s = cut();
+    // fp32, bound by the matrix pipe and not by what the tiles read: smaller ones where these are no slower
+    if (es == 4 && (p.bm > 64 || p.bn > 64)) {
+        const WgradPlan large = p;
+        const double before = least;
+        const long long was = s;
+        p.bm = p.bn = 64, s = cut();
+        if (least > before) p = large, s = was;
+    }
     // no range longer than its 32-bit offsets reach (operands of more than 2 GiB, widths that alone fill the chip)
     const long long most = 0x7fffffffLL / ((long long)(M > NO ? M : NO) * es) / 64 * 64;
     if (most > 0 && s < (N + most - 1) / most) s = (N + most - 1) / most;
     p.kper = ((N + s - 1) / s + 63) / 64 * 64;
     p.splits = (int)((N + p.kper - 1) / p.kper);
     return p;
+}
+
+// (asked for five times a call, the workspace's size among them, and microseconds to make)
+WgradPlan wgrad_plan(long long N, int M, int NO, int es) {
+    static PlanCache<std::array<long long, 4>, WgradPlan> plans;
+    return plans.get({N, M, NO, es}, [=] { return wgrad_make_plan(N, M, NO, es); });
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -403,11 +563,14 @@ int dense_wide_rows_launch(const void* x, const void* w, int w_kmajor, const voi
     if (N == 0) return 0;
 #define PDW_WIDE_T(T, BM, BN) (w_kmajor ? wide_go<T, BM, BN, false, true, false>(g, s) : wide_go<T, BM, BN, false, false, false>(g, s))
 #define PDW_WIDE(BM, BN) (dtype == kF16 ? PDW_WIDE_T(f16_t, BM, BN) : PDW_WIDE_T(bf16_t, BM, BN))
-    if (dtype == kF32) return PDW_WIDE_T(float, 64, 64);
-    if (bn == 192) return PDW_WIDE(128, 192);
+#define PDW_WIDE2(BM, BN) (dtype == kF16 ? PDW_WIDE2_T(f16_t, BM, BN) : PDW_WIDE2_T(bf16_t, BM, BN))   /* (tiles of launches that fill the chip) */
+#define PDW_WIDE2_T(T, BM, BN) (w_kmajor ? wide_go<T, BM, BN, false, true, false, 2>(g, s) : wide_go<T, BM, BN, false, false, false, 2>(g, s))
+    if (dtype == kF32) return PDW_WIDE2_T(float, 64, 64);
+    if (bn == 192) return PDW_WIDE2(128, 192);
     if (bm == 64) return bn == 64 ? PDW_WIDE(64, 64) : PDW_WIDE(64, 128);
-    return bn == 64 ? PDW_WIDE(128, 64) : PDW_WIDE(128, 128);
+    return bn == 64 ? PDW_WIDE(128, 64) : PDW_WIDE2(128, 128);
 #undef PDW_WIDE
+#undef PDW_WIDE2
 #undef PDW_WIDE_T
 }
 
@@ -428,7 +591,7 @@ int dense_wide_wgrad_launch(const void* a, const void* b, void* dw, void* ws, lo
     if (p.kper * (M > NO ? M : NO) * es > 0x7fffffffLL) return -1;
     WideArgs g{a, b, nullptr, nullptr, ws, M, N, NO, M, NO, 1, p.mt, p.nt, p.splits, p.kper};
 #define PDW_WIDE_W(BM, BN)                                                 \
-    (dtype == kF32   ? wide_go<float, BM, BN, true, true, true>(g, s)      \
+    (dtype == kF32   ? wide_go<float, BM, BN, true, true, true, 2>(g, s)   \
      : dtype == kF16 ? wide_go<f16_t, BM, BN, true, true, true>(g, s)      \
                      : wide_go<bf16_t, BM, BN, true, true, true>(g, s))
     const int e = p.bm == 64 ? (p.bn == 64 ? PDW_WIDE_W(64, 64) : PDW_WIDE_W(64, 128))
@@ -463,14 +626,14 @@ int dense_wide_bwd_pair_launch(const void* gy, const void* w, const void* b, voi
     }
     int e = -1;
     if (es == 4) {
-        if (small) e = pair_go<float, 64, 64, 0, 0>(rows, wg, any, nw, s);
-        else if (p.bm == 64 && p.bn == 64) e = pair_go<float, 64, 64, 64, 64>(rows, wg, any, nw, s);
+        if (small) e = pair_go<float, 64, 64, 0, 0, 2>(rows, wg, any, nw, s);
+        else if (p.bm == 64 && p.bn == 64) e = pair_go<float, 64, 64, 64, 64, 2>(rows, wg, any, nw, s);
     } else if (p.bm == 128 && p.bn == 128) {
         auto go = [&](auto t) {
             using T = decltype(t);
-            if (bn == 192) return pair_go<T, 128, 192, 128, 128>(rows, wg, any, nw, s);
-            if (bm == 64 && bn == 128) return pair_go<T, 64, 128, 128, 128>(rows, wg, any, nw, s);
-            if (bm == 128 && bn == 128) return pair_go<T, 128, 128, 128, 128>(rows, wg, any, nw, s);
+            if (bn == 192) return pair_go<T, 128, 192, 128, 128, 2>(rows, wg, any, nw, s);
+            if (bm == 64 && bn == 128) return pair_go<T, 64, 128, 128, 128, kDeep>(rows, wg, any, nw, s);
+            if (bm == 128 && bn == 128) return pair_go<T, 128, 128, 128, 128, 2>(rows, wg, any, nw, s);
             return -1;
         };
         e = dtype == kF16 ? go(f16_t{}) : go(bf16_t{});

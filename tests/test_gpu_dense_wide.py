@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from parity import assert_close, randn
+from test_gpu_block import _block_case
 
 pytestmark = pytest.mark.gpu
 
@@ -37,6 +38,21 @@ def test_dense_wide_layers(dtype, K, NO, N, P):
 def test_dense_wide_fp32_layers(K, NO, N, P):
     """Every tile (70001 rows: 128 high), remainders of 4 in both widths, ranges of rows that end within a stage."""
     _layers(torch.float32, K, NO, N, P)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K,NO", [(376, 136), (384, 64), (392, 72), (448, 920), (1152, 144)])
+@pytest.mark.parametrize("N", [1, 65, 191, 320, 2128])
+def test_few_workgroups_of_long_sums(dtype, K, NO, N):
+    """Four stages in flight: sums just below and from six stages on (of three in a weight gradient's range), remainders of a stage,
+    every tile."""
+    _layers(dtype, K, NO, N, N)
+
+
+@pytest.mark.parametrize("dim,shape", [(920, (2, 9, 8, 920)), (520, (3, 14, 13, 520)), (264, (1, 6, 5, 264))])
+def test_few_workgroups_of_both_products(oracle, dim, shape):
+    """The same in the launch that makes both gradients of a block's layers."""
+    _block_case(oracle, dim, 3, shape, torch.float16)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
