@@ -336,8 +336,24 @@ __device__ __forceinline__ void wide_gemm_body(const WideArgs& g, int blk, int n
         }
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     }
-    if constexpr (PART) {
-        // through LDS: as they lie in registers a store would write 16 bytes of each of 32 rows
+    if constexpr (PART && sizeof(T) == 4) {   // (tiles of 64, four to a compute unit: nothing to win by the other way)
+        float* const out = (float*)g.y + (size_t)sp * g.M * g.N;
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+            const long long m = m0 + (wm * FM + i) * 32 + l32;
+            if (m >= g.M) continue;
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int n = n0 + (wn * FN + j) * 32 + 8 * q + 4 * h;
+                    if (n < g.N)
+                        *reinterpret_cast<float4*>(out + m * g.N + n) =
+                            make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+                }
+        }
+    } else if constexpr (PART) {
+        // through LDS: as they lie in registers a store would write 16 bytes of each of 32 rows ([3136,768]^T [3136,384] 18.6 -> 17.5 us)
         constexpr int TP = BN + 4, CPR = BN / 4;
         __syncthreads();
         float* const tile = reinterpret_cast<float*>(dsm);
@@ -496,13 +512,14 @@ WgradPlan wgrad_make_plan(long long N, int M, int NO, int es) {
         return best;
     };
     long long s = cut();
-    // fp32, bound by the matrix pipe and not by what the tiles read: smaller ones where these are no slower
+    // fp32, bound by the matrix pipe and not by what the tiles read: smaller ones (which the shared launch takes) unless these are
+    // clearly faster
     if (es == 4 && (p.bm > 64 || p.bn > 64)) {
         const WgradPlan large = p;
         const double before = least;
         const long long was = s;
         p.bm = p.bn = 64, s = cut();
-        if (least > before) p = large, s = was;
+        if (least > 1.15 * before) p = large, s = was;
     }
     // no range longer than its 32-bit offsets reach (operands of more than 2 GiB, widths that alone fill the chip)
     const long long most = 0x7fffffffLL / ((long long)(M > NO ? M : NO) * es) / 64 * 64;

@@ -220,7 +220,9 @@ static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* 
     };
     auto p0 = plan_of(H, W), p1 = plan_of(h, w);
     if (!p0.ok || !p1.ok) return -1;
-    const int nmean = mean ? mean->B * mean_slices(mean->D) : 0;
+    MeanJob job{};
+    if (mean) job = *mean, job.shared = mean_shared(job.B, job.D);
+    const int nmean = mean ? mean_bwd_workgroups(job) : 0;
     Bwd3Plan plan = bwd3_plan<K, CS>(B, a.gd, a.npcd, p0, p1, nmean);
     if (const char* e = tune_env("PDW_BWD3_BANDS")) {   // e.g. "64,31,8,DHF": cuts of D, F, H and the grid order
         if (sscanf(e, "%d,%d,%d,%3s", &plan.n[0], &plan.n[1], &plan.n[2], plan.order) != 4) return -1;
@@ -254,7 +256,7 @@ static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* 
     a.p[0].x = x0, a.p[0].gy = gyf, a.p[0].part = (float*)ws0;
     a.p[1].x = x1, a.p[1].gy = gy1, a.p[1].part = (float*)ws1;
     a.nd = (int)nd, a.nmean = nmean;
-    if (mean) a.mean = *mean;
+    a.mean = job;
     {
         // order of the three problems in the grid: a permutation of D (input gradient), H (half scale), F (full scale)
         const char* ord = plan.order;
@@ -271,7 +273,7 @@ static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* 
     } else {
         for (const Bwd3Wgrad<K>& p : a.p) lds = std::max(lds, p.ncb == 8 ? WgTzShape<8>::lds_bytes : WgTzShape<5>::lds_bytes);
     }
-    if (nmean) lds = std::max(lds, mean_lds(mean->D, 512));
+    if (nmean) lds = std::max(lds, mean_lds(job.D, 512, job.shared ? kMeanImages : 1));
     const unsigned grid = (unsigned)(nd + p0.nblocks + p1.nblocks + nmean);
     auto go = [&](auto t) {
         using T = decltype(t);

@@ -491,7 +491,7 @@ int launch_wgrad_f32t_pair(const void* x0, const void* gy0, void* dw0, void* ws0
         const size_t need = mean_lds(mean->D, 512);
         if (need > 80 * 1024) return -1;   // (two workgroups on a compute unit)
         if (need > lds) lds = need;
-        a.mean = *mean, n += (long long)mean->B * mean_slices(mean->D);
+        a.mean = *mean, n += mean_bwd_workgroups(*mean);
     }
     if (n > 0x7fffffffLL) return -1;
     static std::once_flag once;

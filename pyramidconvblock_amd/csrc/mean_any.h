@@ -117,7 +117,35 @@ __device__ __forceinline__ void image_sums(const float* __restrict__ pp, int n, 
     __syncthreads();
 }
 
+// The same for `images` <= IM images after one another (partials of few ranges: many images), into sm[image][D].
+template <int NT, int IM>
+__device__ __forceinline__ void images_sums(const float* __restrict__ pp, int n, int D, int images, float* sm) {
+    const int d4 = D / 4;
+    for (int i = threadIdx.x; i < IM * d4; i += NT) {
+        const int im = i / d4, c = i - im * d4;
+        float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (im < images) {
+            const float* p = pp + (long long)im * n * D + c * 4;
+            int q = 0;
+            for (; q + 3 < n; q += 4) {
+                float4 v[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) v[u] = *reinterpret_cast<const float4*>(p + (long long)(q + u) * D);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) s.x += v[u].x, s.y += v[u].y, s.z += v[u].z, s.w += v[u].w;
+            }
+            for (; q < n; ++q) {
+                const float4 v = *reinterpret_cast<const float4*>(p + (long long)q * D);
+                s.x += v.x, s.y += v.y, s.z += v.z, s.w += v.w;
+            }
+        }
+        *reinterpret_cast<float4*>(sm + i * 4) = s;
+    }
+    __syncthreads();
+}
+
 constexpr int kMeanOut = 64;   // features of a workgroup of the products
+constexpr int kMeanImages = 4; // images of one in the backward, where there would be many
 
 struct MeanJob {
     const float* part;   // [B][n][D]
@@ -127,11 +155,18 @@ struct MeanJob {
     void* m;             // forward: the mean
     float* rowbias;      // forward: m Wp^T + bp + bo
     float *gs, *dmean;   // backward: the sums of the gradient, their product with Wp over P
+    bool shared;         // backward: kMeanImages images to a workgroup
 };
 
 inline int mean_slices(int D) { return cdiv(D, kMeanOut); }
+// Whether a workgroup of the backward takes four images: where one each would make more workgroups than the convolutions' shared
+// launch, which holds one workgroup a compute unit, has units left for.  They read the layer's weight once and take less than twice as long.  Training
+// steps, us: [102,10,13,608] filter 9 bf16 (1020 workgroups -> 260) 248 -> 228, [40,7,7,1152] filter 5 184 -> 151, [20,14,14,1024] filter 5 (320
+// -> 80) 147 -> 137, [64,20,20,256] (256 -> 64) 117 -> 113; with eight images [12,28,28,768] (144 -> 24) 156 -> 179.
+inline bool mean_shared(int B, int D) { return (long long)B * mean_slices(D) > 192 && D > 128 && D <= 2048; }
+inline int mean_bwd_workgroups(const MeanJob& j) { return cdiv(j.B, j.shared ? kMeanImages : 1) * mean_slices(j.D); }
 // sums; scratch of 32 bytes a thread (backward, 16-bit) or less
-inline size_t mean_lds(int D, int nt = 256) { return (size_t)D * sizeof(float) + (size_t)nt * 32; }
+inline size_t mean_lds(int D, int nt = 256, int images = 1) { return (size_t)images * D * sizeof(float) + (size_t)nt * 32; }
 
 template <typename T>
 __device__ __forceinline__ void mean_fwd_body(const MeanJob& j, int wg, float* sm) {
@@ -180,45 +215,59 @@ __device__ __forceinline__ void mean_fwd_body(const MeanJob& j, int wg, float* s
 }
 
 // By a workgroup of NT threads.
-template <typename T, int NT>
-__device__ __forceinline__ void mean_bwd_body(const MeanJob& j, int wg, float* sm) {
+template <typename T, int NT, int IM>
+__device__ __forceinline__ void mean_bwd_images(const MeanJob& j, int wg, float* sm) {
     constexpr int V = 16 / (int)sizeof(T), CL = kMeanOut / V, OL = NT / CL;   // column lanes, row lanes
-    const int slices = (j.D + kMeanOut - 1) / kMeanOut, b = wg / slices, sl = wg - b * slices, D = j.D, tid = threadIdx.x;
-    float* red = sm + D;   // [OL][64]
-    image_sums<NT>(j.part + (long long)b * j.n * D, j.n, D, sm, reinterpret_cast<float4*>(red));
+    const int slices = (j.D + kMeanOut - 1) / kMeanOut, b0 = wg / slices * IM, sl = wg % slices, D = j.D, tid = threadIdx.x;
+    const int images = min(IM, j.B - b0);
+    float* red = sm + IM * D;   // [OL][64]
+    const float* const part = j.part + (long long)b0 * j.n * D;
+    if constexpr (IM == 1) image_sums<NT>(part, j.n, D, sm, reinterpret_cast<float4*>(red));
+    else images_sums<NT, IM>(part, j.n, D, images, sm);
     if (sl == 0)
-        for (int c = tid; c < D; c += NT) j.gs[(long long)b * D + c] = sm[c];
+        for (int c = tid; c < images * D; c += NT) j.gs[(long long)b0 * D + c] = sm[c];
     const int cv = tid % CL, ol = tid / CL, c = sl * kMeanOut + cv * V;
-    float acc[V];
+    float acc[IM][V];
 #pragma unroll
-    for (int e = 0; e < V; ++e) acc[e] = 0.f;
+    for (int i = 0; i < IM; ++i)
+#pragma unroll
+        for (int e = 0; e < V; ++e) acc[i][e] = 0.f;
     if (c < D) {
         const T* wc = (const T*)j.wp + c;
+        auto add = [&](const ChanVec<T, V>& wv, int o) {
+#pragma unroll
+            for (int i = 0; i < IM; ++i)
+#pragma unroll
+                for (int e = 0; e < V; ++e) acc[i][e] = fmaf(sm[i * D + o], to_f32(wv.v[e]), acc[i][e]);
+        };
         int o = ol;
         for (; o + 7 * OL < D; o += 8 * OL) {
             ChanVec<T, V> wv[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u) wv[u] = *reinterpret_cast<const ChanVec<T, V>*>(wc + (long long)(o + u * OL) * D);
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
-#pragma unroll
-                for (int e = 0; e < V; ++e) acc[e] = fmaf(sm[o + u * OL], to_f32(wv[u].v[e]), acc[e]);
+            for (int u = 0; u < 8; ++u) add(wv[u], o + u * OL);
         }
-        for (; o < D; o += OL) {
-            float wv[V];
-            load_f32<T, V>(wc + (long long)o * D, wv);
-#pragma unroll
-            for (int e = 0; e < V; ++e) acc[e] = fmaf(sm[o], wv[e], acc[e]);
-        }
+        for (; o < D; o += OL) add(*reinterpret_cast<const ChanVec<T, V>*>(wc + (long long)o * D), o);
     }
 #pragma unroll
-    for (int e = 0; e < V; ++e) red[ol * kMeanOut + cv * V + e] = acc[e];
-    __syncthreads();
-    if (tid < kMeanOut && sl * kMeanOut + tid < D) {
-        float t = 0.f;
-        for (int q = 0; q < OL; ++q) t += red[q * kMeanOut + tid];
-        j.dmean[(long long)b * D + sl * kMeanOut + tid] = t * j.inv_p;
+    for (int i = 0; i < IM; ++i) {
+        if (i > 0) __syncthreads();
+#pragma unroll
+        for (int e = 0; e < V; ++e) red[ol * kMeanOut + cv * V + e] = acc[i][e];
+        __syncthreads();
+        if (tid < kMeanOut && sl * kMeanOut + tid < D && i < images) {
+            float t = 0.f;
+            for (int q = 0; q < OL; ++q) t += red[q * kMeanOut + tid];
+            j.dmean[(long long)(b0 + i) * D + sl * kMeanOut + tid] = t * j.inv_p;
+        }
     }
+}
+
+template <typename T, int NT>
+__device__ __forceinline__ void mean_bwd_body(const MeanJob& j, int wg, float* sm) {
+    if (j.shared) mean_bwd_images<T, NT, kMeanImages>(j, wg, sm);   // (uniform)
+    else mean_bwd_images<T, NT, 1>(j, wg, sm);
 }
 
 // Whether the bodies take the case (host side).

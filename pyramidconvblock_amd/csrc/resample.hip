@@ -1529,8 +1529,8 @@ int gate_pair_colsum_bwd_launch(const void* gy, const void* xf, const void* xh, 
 }
 
 int mean_bwd_launch(const MeanJob& mean, void* gbias, void* gbias2, void* gwp, int dtype, hipStream_t s) {
-    const int B = mean.B, D = mean.D;
-    const dim3 grid((unsigned)(B * mean_slices(D)));
+    const int D = mean.D;
+    const dim3 grid((unsigned)mean_bwd_workgroups(mean));
     switch (dtype) {
         case kF32: hipLaunchKernelGGL((mean_bwd_k<float>), grid, dim3(256), mean_lds(D), s, mean); break;
         case kF16: hipLaunchKernelGGL((mean_bwd_k<f16_t>), grid, dim3(256), mean_lds(D), s, mean); break;

@@ -21,6 +21,8 @@ def test_padded_inner_channels(oracle, dtype, dim, k, shape):
 @pytest.mark.parametrize("dtype,dim,k,shape", [
     (torch.bfloat16, 16, 5, (5, 11, 13, 16)), (torch.float16, 72, 3, (2, 90, 90, 72)), (torch.bfloat16, 1032, 3, (1, 7, 9, 1032)),
     (torch.float32, 36, 5, (3, 17, 12, 36)), (torch.float32, 252, 3, (40, 9, 8, 252)), (torch.float16, 256, 3, (70, 6, 6, 256)),
+    # four images to a workgroup of its backward: a rest of one and of two, sums of one and of several ranges
+    (torch.bfloat16, 264, 3, (41, 6, 6, 264)), (torch.float16, 136, 3, (66, 5, 6, 136)), (torch.bfloat16, 520, 3, (22, 16, 18, 520)),
 ])
 def test_mean_branch_of_any_width(oracle, dtype, dim, k, shape):
     """The mean branch riding in the pool's and the gates' launches (csrc/mean_any.h): widths of less than one, of several
