@@ -140,8 +140,13 @@ static thread_local int t_seg = 0, t_val = 0;
 
 void reduce_defer_compact(int seg, int val) { t_seg = t_defer ? seg : 0, t_val = val; }
 
-// Part lanes of a stand-alone summation: 32 when 8 would need more than one round of loads.
-static int standalone_part_lanes(int nparts) { return nparts > 128 ? 32 : 8; }
+// Part lanes of a stand-alone summation: 32 when 8 would need more than one round of loads; one when that has no more than two and the
+// outputs are many (training steps as graphs, us: [4,64,64,1152] filter 13 fp16, 11 parts of 660 000 outputs, 336.5 -> 328.5, [102,10,13,608]
+// filter 9 bf16 230 -> 223, [20,14,14,1024] filter 5 135 -> 130; from 8192 outputs on 225 and 132).
+static int standalone_part_lanes(int nparts, int n) {
+    if (nparts <= 32 && n >= 65536) return 1;
+    return nparts > 128 ? 32 : 8;
+}
 
 // A launch of its own has the whole chip's slots: the jobs that were laid out for riding (few workgroups, 8 part
 // lanes) are laid out again with as many part lanes as make their loads a single round.
@@ -151,7 +156,7 @@ int reduce_jobs_launch(const ReduceJobs& recorded, hipStream_t s) {
     for (int j = 0; j < jobs.njobs; ++j) {
         int nb = recorded.first_block[j + 1] - recorded.first_block[j];
         if (recorded.vec[j] != 0) {
-            jobs.ql[j] = standalone_part_lanes(jobs.nparts[j]);
+            jobs.ql[j] = standalone_part_lanes(jobs.nparts[j], jobs.n[j]);
             nb = cdiv(jobs.n[j], reduce_block_outputs(jobs.vec[j], jobs.ql[j]));
         }
         jobs.first_block[j + 1] = jobs.first_block[j] + nb;
@@ -292,7 +297,7 @@ int wgrad_reduce_launch(const float* part, void* dw, int nparts, int n, hipStrea
         t_jobs.first_block[j + 1] = t_jobs.first_block[j] + cdiv(n, reduce_block_outputs(vec, 8));
         return 0;
     }
-    const int ql = standalone_part_lanes(nparts);
+    const int ql = standalone_part_lanes(nparts, n);
     hipLaunchKernelGGL((wgrad_reduce_parts<T>), dim3(cdiv(n, reduce_block_outputs(vec, ql))), dim3(256), 0, s, part,
                        (T*)dw, nparts, n, vec, ql);
     return check_launch("wgrad_reduce_parts");

@@ -10,7 +10,8 @@ namespace pdw {
 // 16-byte loads), part lane q adds parts q, q + QL, ... with up to sixteen loads in flight, and the QL lanes are
 // combined through LDS, so the reads of one part are contiguous and many parts are in flight.  The pass is pure
 // latency.  QL = 8 keeps the workgroups few (they ride in other kernels' grids, where resident slots are scarce);
-// QL = 32 takes 256 parts in one round of loads, for the stand-alone launch.  V = 4 needs n % 4 == 0 and 16-byte
+// QL = 32 takes 256 parts in one round of loads, for the stand-alone launch; QL = 1 few parts of many outputs, where eight lanes have
+// two or three loads each and the launch is a long row of such workgroups.  V = 4 needs n % 4 == 0 and 16-byte
 // aligned partials (reduce_vec_ok).  The order of the additions, and so the result, depends on QL.
 constexpr int kReduceVec = 4;
 constexpr int kReduceLds = 8 * 32 * kReduceVec;  // floats of LDS a workgroup needs
@@ -67,9 +68,11 @@ __device__ __forceinline__ void reduce_parts_block(const float* __restrict__ par
             for (int i = 0; i < V; ++i) s0[i] += a[i];
         }
     }
+    if constexpr (QL > 1) {
 #pragma unroll
-    for (int i = 0; i < V; ++i) red[q * ROW + el * V + i] = s0[i] + s1[i];
-    __syncthreads();
+        for (int i = 0; i < V; ++i) red[q * ROW + el * V + i] = s0[i] + s1[i];
+        __syncthreads();
+    }
     if constexpr (QL == 32) {  // 32 rows -> 8, by the threads of the first 8 part lanes
         if (q < 8) {
 #pragma unroll
@@ -86,8 +89,9 @@ __device__ __forceinline__ void reduce_parts_block(const float* __restrict__ par
 #pragma unroll
         for (int i = 0; i < V; ++i) {
             const int c = el * V + i;
-            o[i] = ((red[c] + red[ROW + c]) + (red[2 * ROW + c] + red[3 * ROW + c])) +
-                   ((red[4 * ROW + c] + red[5 * ROW + c]) + (red[6 * ROW + c] + red[7 * ROW + c]));
+            if constexpr (QL == 1) o[i] = s0[i] + s1[i];
+            else o[i] = ((red[c] + red[ROW + c]) + (red[2 * ROW + c] + red[3 * ROW + c])) +
+                        ((red[4 * ROW + c] + red[5 * ROW + c]) + (red[6 * ROW + c] + red[7 * ROW + c]));
         }
         if (seg == 0) {
             store_f32<T, V>(dw + e, o);
@@ -113,10 +117,12 @@ template <typename T>
 __device__ __forceinline__ void reduce_parts_any(const float* part, T* dw, int nparts, int n, int blk, int vec, int ql,
                                                  float* red, int seg = 0, int val = 0) {
     if (vec == kReduceVec) {
-        if (ql == 32) reduce_parts_block<T, kReduceVec, 32>(part, dw, nparts, n, blk, red, seg, val);
+        if (ql == 1) reduce_parts_block<T, kReduceVec, 1>(part, dw, nparts, n, blk, red, seg, val);
+        else if (ql == 32) reduce_parts_block<T, kReduceVec, 32>(part, dw, nparts, n, blk, red, seg, val);
         else reduce_parts_block<T, kReduceVec, 8>(part, dw, nparts, n, blk, red, seg, val);
     } else {
-        if (ql == 32) reduce_parts_block<T, 1, 32>(part, dw, nparts, n, blk, red, seg, val);
+        if (ql == 1) reduce_parts_block<T, 1, 1>(part, dw, nparts, n, blk, red, seg, val);
+        else if (ql == 32) reduce_parts_block<T, 1, 32>(part, dw, nparts, n, blk, red, seg, val);
         else reduce_parts_block<T, 1, 8>(part, dw, nparts, n, blk, red, seg, val);
     }
 }
@@ -166,7 +172,7 @@ struct ReduceJobs {
     const void* aux[kMaxReduceJobs];  // outer products: the second factor (element type of `out`)
     int nparts[kMaxReduceJobs], n[kMaxReduceJobs], dtype[kMaxReduceJobs];
     int vec[kMaxReduceJobs];  // outputs per lane: kReduceVec or 1; 0 = outer product (n = D * D, nparts = B)
-    int ql[kMaxReduceJobs];   // part lanes: 8 or 32
+    int ql[kMaxReduceJobs];   // part lanes: 1, 8 or 32
     int dim[kMaxReduceJobs];  // outer products: D
     int seg[kMaxReduceJobs], val[kMaxReduceJobs];  // outputs without their padding (reduce_defer_compact); seg = 0: all of them
     int first_block[kMaxReduceJobs + 1];

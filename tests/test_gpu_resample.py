@@ -456,6 +456,22 @@ def test_sum_parts_is_the_fp32_sum_rounded_once(shape, dtype):
     assert bool(((out.double().cpu() - ref).abs() <= tol).all())
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("shape", [(1, 65536), (2, 65532), (16, 65540), (17, 70001), (32, 65536), (33, 65536)])
+def test_sum_of_few_parts_of_many_outputs(shape, dtype):
+    """One lane to an output group: up to 32 parts of 65536 outputs or more, remainders of a workgroup and of four outputs."""
+    from pyramidconvblock_amd import ops
+
+    gen = torch.Generator().manual_seed(shape[0])
+    parts = torch.randn(*shape, generator=gen, dtype=torch.float32)
+    out = ops.sum_parts(parts.cuda(), dtype)
+    ref = parts.double().sum(0)
+    eps = {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -8}[dtype]
+    tol = eps * ref.abs() + shape[0] * 2.0 ** -24 * parts.abs().double().sum(0) + 1e-7
+    assert bool(((out.double().cpu() - ref).abs() <= tol).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("with_cat", [True, False])
 @pytest.mark.parametrize("case", [(32, 56, 56, 64, 128), (1, 4, 8, 64, 128), (3, 8, 16, 64, 128), (2, 12, 40, 64, 128),
