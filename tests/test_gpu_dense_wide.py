@@ -62,6 +62,86 @@ def test_dense_wide_columns_of_192(dtype, K, NO):
     _layers(dtype, K, NO, 257 * 128 + 5, 257 * 128 + 5)
 
 
+@pytest.mark.parametrize("K,NO,N,P", [(196, 196, 13100, 13100), (516, 200, 7001, 700), (200, 516, 7001, 7001), (1028, 260, 2000, 63), (704, 352, 10816, 10816),
+                                      (192, 192, 13564, 6782), (260, 1028, 2000, 2000)])
+def test_fp32_layers_on_split_operands(K, NO, N, P):
+    """Large fp32 products (csrc/dense_split.h): both tiles, remainders of 4 results and inner values, an odd number of stages, ranges of
+    rows; no further from float64 than fp32 products and sums of that length are (their partial sums random: sqrt(K) roundings)."""
+    from pyramidconvblock_amd import ops
+
+    _layers(torch.float32, K, NO, N, P)
+    gen = torch.Generator().manual_seed(K)
+    x, w = randn(gen, N, K), randn(gen, NO, K)
+    y = ops.dense_forward(x.cuda(), w.cuda())
+    want = x.double() @ w.double().t()
+    assert float((y.double().cpu() - want).norm() / want.norm()) <= 2.0 ** -24 * K ** 0.5
+    dw = ops.dense_wgrad(y, x.cuda())
+    want = y.double().cpu().t() @ x.double()
+    assert float((dw.double().cpu() - want).norm() / want.norm()) <= 2.0 ** -24 * N ** 0.5
+
+
+def test_fp32_split_operands_and_values_that_are_not_finite():
+    """Results are those of fp32 arithmetic where an operand has no three bf16 parts: infinities of a sign, NaN, and values that round
+    up to infinity in bf16; the others are as without them."""
+    from pyramidconvblock_amd import ops
+
+    K, NO, N = 260, 256, 8000
+    gen = torch.Generator().manual_seed(1)
+    x, w, g = randn(gen, N, K), randn(gen, NO, K), randn(gen, N, NO)
+    clean = ops.dense_forward(x.cuda(), w.cuda()).cpu()
+    dclean = ops.dense_wgrad(g.cuda(), x.cuda()).cpu()
+    xp = x.clone()
+    xp[5, 7], xp[300, 9], xp[4000, 0] = float("inf"), float("nan"), -float("inf")
+    xp[700, 11] = 3.4e38
+    y = ops.dense_forward(xp.cuda(), (w * 1e-3).cuda()).cpu()
+    want = xp.double() @ (w * 1e-3).double().t()
+    for r in (5, 4000):
+        assert torch.equal(y[r].double(), want[r])   # infinities of the weights' signs
+    assert torch.isnan(y[300]).all()
+    assert torch.isfinite(y[700]).all() and float(((y[700].double() - want[700]) / want[700].abs().max()).abs().max()) < 1e-6
+    others = torch.ones(N, dtype=torch.bool)
+    others[[5, 300, 700, 4000]] = False
+    assert torch.isfinite(y[others]).all() and float((y[others].double() - want[others]).norm() / want[others].norm()) < 1e-6
+    dw = ops.dense_wgrad(g.cuda(), xp.cuda()).cpu()
+    for c, r in ((7, 5), (0, 4000)):
+        assert torch.equal(dw[:, c].double(), (g[r].double() * xp[r, c].double()))
+    assert torch.isnan(dw[:, 9]).all()
+    cols = torch.ones(K, dtype=torch.bool)
+    cols[[0, 7, 9, 11]] = False
+    assert float((dw[:, cols] - dclean[:, cols]).norm() / dclean.norm()) < 1e-6
+    wp = w.clone()
+    wp[3, 4] = float("inf")
+    y = ops.dense_forward(x.cuda(), wp.cuda()).cpu()
+    assert torch.equal(y[:, 3].double(), x[:, 4].double() * float("inf"))
+    keep = torch.ones(NO, dtype=torch.bool)
+    keep[3] = False
+    assert float((y[:, keep] - clean[:, keep]).norm() / clean.norm()) < 1e-6
+
+
+@pytest.mark.parametrize("scale", [1e-29, 1e-34, 1e-37])
+def test_fp32_split_operands_near_the_smallest_values(scale):
+    """Values whose parts bf16 cannot hold: no less precise than others."""
+    from pyramidconvblock_amd import ops
+
+    gen = torch.Generator().manual_seed(2)
+    x, w = randn(gen, 8000, 256), randn(gen, 256, 256) * 1e4
+    x[:1000] *= scale   # (beside rows of ordinary values, in tiles of their own and in one with them)
+    y = ops.dense_forward(x.cuda(), w.cuda()).cpu().double()
+    want = x.double() @ w.double().t()
+    for rows in (slice(0, 1000), slice(1000, None)):
+        assert float((y[rows] - want[rows]).norm() / want[rows].norm()) <= 2.0 ** -24 * 16
+    g = randn(gen, 8000, 256) * scale
+    dw = ops.dense_wgrad(g.cuda(), x[1000:].repeat(2, 1)[:8000].cuda()).cpu().double()
+    want = g.double().t() @ x[1000:].repeat(2, 1)[:8000].double()
+    assert float((dw - want).norm() / want.norm()) <= 2.0 ** -24 * 8000 ** 0.5
+
+
+@pytest.mark.parametrize("dim,shape", [(400, (3, 47, 45, 400)), (712, (1, 50, 41, 712))])
+def test_fp32_block_on_split_operands(oracle, dim, shape):
+    """Both products of a layer's backward on split operands, in one launch."""
+    _block_case(oracle, dim, 3, shape, torch.float32)
+
+
 @pytest.mark.parametrize("dtype,N", [(torch.bfloat16, 270000), (torch.float32, 140000)])
 def test_weight_gradient_of_more_than_2_gib(dtype, N):
     """A layer whose tiles alone fill the chip, over operands that one range's 32-bit offsets do not reach."""
