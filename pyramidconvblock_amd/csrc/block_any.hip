@@ -64,45 +64,7 @@ Shape shape_of(int B, int H, int W, int h, int w, int D, int I, int K, int dtype
 
 bool layer_ok(int K, int NO, int dtype) { return pdw_dense_supported(K, NO, dtype) != 0 || dense_wide_ok(K, NO, dtype); }
 
-// The four weights with inner channels in the padded layout, eight values to a thread: conv_up's rows, conv_out's
-// columns, the filters' channels.  A few hundred KB at most: launch latency.
-struct PackArgs {
-    const uint16_t *up, *out, *dw0, *dw1;
-    uint16_t *up_p, *out_p, *dw0_p, *dw1_p;
-    int D, G, Gp, KK;
-    int n_up, n_out, n_dw;   // vectors of 8 in each region
-};
-
-__global__ __launch_bounds__(256) void pack_weights_k(const PackArgs g) {
-    int v = blockIdx.x * 256 + threadIdx.x;
-    const int I = 2 * g.G, Ip = 2 * g.Gp;
-    if (v < g.n_up) {
-        const int per = g.D / 8, row = v / per, c = v - row * per;
-        const int hi = row >= g.Gp, r = row - hi * g.Gp;
-        uint4 x = make_uint4(0, 0, 0, 0);
-        if (r < g.G) x = *reinterpret_cast<const uint4*>(g.up + (long long)(hi * g.G + r) * g.D + c * 8);
-        *reinterpret_cast<uint4*>(g.up_p + (long long)v * 8) = x;
-        return;
-    }
-    v -= g.n_up;
-    const uint16_t* src = g.out;
-    uint16_t* dst = g.out_p;
-    if (v >= g.n_out) {
-        v -= g.n_out;
-        src = g.dw0, dst = g.dw0_p;
-        if (v >= g.n_dw) {
-            v -= g.n_dw;
-            src = g.dw1, dst = g.dw1_p;
-            if (v >= g.n_dw) return;
-        }
-    }
-    const int per = Ip / 8, row = v / per, c = (v - row * per) * 8;
-    const int hi = c >= g.Gp, r = c - hi * g.Gp;
-    ChanVec<uint16_t, 8> o;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) o.v[i] = r + i < g.G ? src[(long long)row * I + hi * g.G + r + i] : (uint16_t)0;
-    *reinterpret_cast<ChanVec<uint16_t, 8>*>(dst + (long long)v * 8) = o;
-}
+__global__ __launch_bounds__(256) void pack_weights_k(const PackArgs g) { pack_weights_body(g, blockIdx.x); }
 
 // The block's inner weights as its kernels read them.
 struct Weights {
@@ -176,34 +138,52 @@ BwdWork bwd_layout(const Shape& s, void* base) {
     return r;
 }
 
-int pack_weights(const Shape& s, const Saved& v, Weights* w, hipStream_t stream) {
-    PackArgs g{(const uint16_t*)w->up, (const uint16_t*)w->out, (const uint16_t*)w->dw0, (const uint16_t*)w->dw1,
-               (uint16_t*)v.up_p,      (uint16_t*)v.out_p,      (uint16_t*)v.dw0_p,      (uint16_t*)v.dw1_p,
-               s.D,                    s.G,                     s.Gp,                    s.K * s.K,
-               s.I * s.D / 8,          s.I * s.D / 8,           s.K * s.K * s.I / 8};
-    hipLaunchKernelGGL(pack_weights_k, dim3(cdiv(g.n_up + g.n_out + 2 * g.n_dw, 256)), dim3(256), 0, stream, g);
-    *w = {v.up_p, v.out_p, v.dw0_p, v.dw1_p};
+PackArgs pack_args(const Shape& s, const Saved& v, const Weights& w) {
+    return PackArgs{(const uint16_t*)w.up, (const uint16_t*)w.out, (const uint16_t*)w.dw0, (const uint16_t*)w.dw1,
+                    (uint16_t*)v.up_p,     (uint16_t*)v.out_p,     (uint16_t*)v.dw0_p,     (uint16_t*)v.dw1_p,
+                    s.D,                   s.G,                    s.Gp,
+                    s.I * s.D / 8,         s.I * s.D / 8,          s.K * s.K * s.I / 8};
+}
+
+int pack_weights(const PackArgs& g, hipStream_t stream) {
+    hipLaunchKernelGGL(pack_weights_k, dim3(pack_workgroups(g)), dim3(256), 0, stream, g);
     return check_launch("pack_weights");
 }
 
 bool rows_whole_tiles(const Shape& s) { return s.P % pdw_dense_colsum_rows() == 0; }
 
-int forward(const Shape& s, const Saved& v, const void* x, const Weights& wt, const void* w_pool, const void* b_pool,
+int forward(const Shape& s, const Saved& v, const void* x, const Weights& given, const void* w_pool, const void* b_pool,
             const void* b_out, void* y, void* stream) {
-    const void *const w_up = wt.up, *const w_out = wt.out, *const w_dw0 = wt.dw0, *const w_dw1 = wt.dw1;
     const hipStream_t st = (hipStream_t)stream;
+    const Weights wt = s.padded() ? Weights{v.up_p, v.out_p, v.dw0_p, v.dw1_p} : given;
+    const void *const w_up = wt.up, *const w_out = wt.out, *const w_dw0 = wt.dw0, *const w_dw1 = wt.dw1;
+    // conv_up reads its weights as they were given where it can, and all four are packed by the launch of the pool
+    const PackArgs pack = s.padded() ? pack_args(s, v, given) : PackArgs{};
+    bool unpacked = s.padded();
     const int pad = s.K / 2, dt = s.dtype;
     const bool two = s.exact && dt != kF32 && pdw_dwconv_fwd2_supported(s.B, s.H, s.W, s.I, s.K, dt);
     // conv_up, where its kernel can with the sums of x per row tile (for the mean branch) and the 2x2 pool of its result
     const float* parts = nullptr;
     int nparts = 0;
     bool pooled = false;
-    if (two) {
+    if (two && !s.padded()) {
         const int r = pdw_dense_fwd_colsum_pool(x, w_up, nullptr, v.a, v.xparts, v.xp, s.B, s.H, s.W, s.D, s.I, dt, stream);
         if (r != 0 && r != 3) return r;
         pooled = r == 0;
     }
-    if (pooled) {
+    if (s.padded()) {
+        const RowMap map{s.Gp, s.G};
+        float* const sums = rows_whole_tiles(s) && pdw_dense_colsum_supported(s.D, s.I, dt) ? v.xparts : nullptr;
+        int r = dense_rows_launch(x, given.up, 0, nullptr, nullptr, v.a, s.N, s.D, s.I, s.P, dt, st, sums, nullptr, &map);
+        if (r == -1) {
+            if (int e = pack_weights(pack, st)) return e;
+            unpacked = false;
+            r = sums ? pdw_dense_fwd_colsum(x, w_up, 0, nullptr, nullptr, v.a, sums, s.N, s.D, s.I, s.P, dt, stream)
+                     : pdw_dense_fwd(x, w_up, 0, nullptr, nullptr, v.a, s.N, s.D, s.I, s.P, dt, stream);
+        }
+        if (r) return r;
+        if (sums) parts = sums, nparts = s.P / pdw_dense_colsum_rows();
+    } else if (pooled) {
         parts = v.xparts, nparts = s.P / 32;
     } else if (rows_whole_tiles(s) && pdw_dense_colsum_supported(s.D, s.I, dt)) {
         if (int e = pdw_dense_fwd_colsum(x, w_up, 0, nullptr, nullptr, v.a, v.xparts, s.N, s.D, s.I, s.P, dt, stream)) return e;
@@ -214,10 +194,12 @@ int forward(const Shape& s, const Saved& v, const void* x, const Weights& wt, co
     // the pool, with the sums of x where conv_up's kernel did not leave any
     const bool any_mean = mean_any_ok(x, w_pool, v.m, s.D, s.es);
     auto pool = [&]() -> int {
-        if (parts || !any_mean) return avgpool_fwd_launch(v.a, v.xp, s.B, s.H, s.W, s.I, s.h, s.w, dt, st);
+        const PackArgs* const with = unpacked ? &pack : nullptr;
+        unpacked = false;
+        if (parts || !any_mean) return avgpool_with_launch(v.a, v.xp, s.B, s.H, s.W, s.I, s.h, s.w, nullptr, with, dt, st);
         const ColsumJob sums = colsum_plan(x, (float*)v.ws, s.B, s.P, s.D, s.es);
         parts = sums.part, nparts = sums.n;
-        return avgpool_colsum_launch(v.a, v.xp, s.B, s.H, s.W, s.I, s.h, s.w, sums, dt, st);
+        return avgpool_with_launch(v.a, v.xp, s.B, s.H, s.W, s.I, s.h, s.w, &sums, with, dt, st);
     };
     // the convolutions of both scales                                                         (conv_block.py:14-17)
     bool convs = false, mean = false;
@@ -235,7 +217,7 @@ int forward(const Shape& s, const Saved& v, const void* x, const Weights& wt, co
         convs = r == 0;
         if (!convs)
             if (int e = pdw_dwconv_fwd(v.a, w_dw0, v.c0, s.B, s.H, s.W, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, dt, stream)) return e;
-    } else if (parts || !any_mean) {
+    } else if ((parts || !any_mean) && !unpacked) {
         if (int e = pdw_dwconv_fwd_pool(v.a, w_dw0, v.c0, v.xp, s.B, s.H, s.W, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, s.h, s.w, dt, stream))
             return e;
     } else {
@@ -416,10 +398,7 @@ int pdw_block_fwd(const void* x, const void* w_up, const void* w_dw0, const void
     if (s.single)
         return convblock_fwd_launch(x, w_up, w_dw0, w_dw1, w_pool, b_pool, w_out, b_out, v.a, v.c0, v.xp, v.c1, v.cat, v.m, y,
                                     v.xparts, v.yp, B, H, W, D, I, K, dtype, stream);
-    Weights wt{w_up, w_out, w_dw0, w_dw1};
-    if (s.padded())
-        if (int e = pack_weights(s, v, &wt, (hipStream_t)stream)) return e;
-    return forward(s, v, x, wt, w_pool, b_pool, b_out, y, stream);
+    return forward(s, v, x, Weights{w_up, w_out, w_dw0, w_dw1}, w_pool, b_pool, b_out, y, stream);
 }
 
 size_t pdw_block_bwd_workspace_bytes(int B, int H, int W, int h, int w, int D, int I, int K, int dtype) {

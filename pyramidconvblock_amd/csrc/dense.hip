@@ -215,7 +215,7 @@ __device__ __forceinline__ void dense_rows_body(const T* __restrict__ X, const T
                                                 T* __restrict__ Y, float* __restrict__ colsum, long long N, int Kd,
                                                 int NOd, int P, int nktd, int nntd, int bid, int nblocks,
                                                 uint32_t* dsm, T* __restrict__ pool = nullptr, int Himg = 0,
-                                                int Wimg = 0, const MidRows* mid = nullptr) {
+                                                int Wimg = 0, const MidRows* mid = nullptr, const RowMap map = {}) {
     constexpr bool STATIC = SK > 0 && SNO > 0;
     static_assert(!POOL || (STATIC && !KMAJOR), "pooled output: layers with their extents as constants");
     static_assert(MID == 0 || (((STATIC && SK <= 64) || (SK == 0 && SNO == 0)) && !KMAJOR && !COLSUM && !POOL),
@@ -252,7 +252,7 @@ __device__ __forceinline__ void dense_rows_body(const T* __restrict__ X, const T
     // this lane's four bias values: an unconditional 8-byte load (of the weights when there is no bias), converted
     // where the table is written, so that nothing waits for it before the weights and the first tile are requested
     const ChanVec<T, 4> braw = *reinterpret_cast<const ChanVec<T, 4>*>(bias && bcol < NO ? bias + bcol : W);
-    if (K != KP || NO != NOP) {  // uniform
+    if (K != KP || NO != NOP || (!STATIC && map.seg)) {  // uniform
         for (int i = tid; i < NOP * ldw / 8; i += 256) reinterpret_cast<uint4*>(wl)[i] = make_uint4(0u, 0u, 0u, 0u);
         __syncthreads();
     }
@@ -377,6 +377,14 @@ __device__ __forceinline__ void dense_rows_body(const T* __restrict__ X, const T
         int src[ITW], wdst[ITW];
         strided_offsets<ITW>(tid, 256, kv, K, 8, NO, src);
         strided_offsets<ITW>(tid, 256, kv, ldw, 8, NO, wdst);
+        if (!STATIC && MID == 0 && map.seg) {   // (uniform)
+#pragma unroll
+            for (int it = 0; it < ITW; ++it) {
+                const int row = (it * 256 + tid) / kv, hi = row >= map.seg;
+                if (src[it] >= 0) src[it] -= hi * (map.seg - map.val) * K;
+                if (row - hi * map.seg >= map.val) src[it] = wdst[it] = -1;   // (the zeros of above stay)
+            }
+        }
 #pragma unroll
         for (int it = 0; it < ITW; ++it) wv[it] = *reinterpret_cast<const Frag*>(W + (src[it] >= 0 ? src[it] : 0));
         if (gw < ntiles) load_tile(gw);
@@ -721,10 +729,10 @@ template <typename T, bool KMAJOR, bool COLSUM, int SK, int SNO>
 __global__ __launch_bounds__(256, 2) void dense_rows_k(const T* __restrict__ X, const T* __restrict__ W,
                                                     const T* __restrict__ bias, const float* __restrict__ rowbias,
                                                     T* __restrict__ Y, float* __restrict__ colsum, long long N, int K,
-                                                    int NO, int P, int nkt, int nnt) {
+                                                    int NO, int P, int nkt, int nnt, const RowMap map) {
     extern __shared__ uint32_t dsm[];
     dense_rows_body<T, KMAJOR, COLSUM, SK, SNO>(X, W, bias, rowbias, Y, colsum, N, K, NO, P, nkt, nnt, blockIdx.x,
-                                                gridDim.x, dsm);
+                                                gridDim.x, dsm, nullptr, 0, 0, nullptr, map);
 }
 
 // The 128 -> 64 layer over the pixels of [B, Himg, Wimg] images with the tile sums of X and the 2x2 average pool of Y
@@ -1005,7 +1013,8 @@ int dense_colsum_supported(int K, int NO, int dtype) { return dense_dims_ok(K, N
 
 int dense_rows_launch(const void* x, const void* w, int w_kmajor, const void* bias, const float* rowbias, void* y,
                       long long N, int K, int NO, int P, int dtype, hipStream_t s, float* colsum,
-                      const ReduceJobs* rider) {
+                      const ReduceJobs* rider, const RowMap* map) {
+    if (map && (w_kmajor || bias || rowbias || rider || dtype == kF32 || NO != 2 * map->seg)) return -1;
     if (!dense_dims_ok(K, NO, dtype)) {
         // fp32 and the widths the tiled kernels do not take: no tile sums there, and summations that were to ride
         // in this launch get one of their own
@@ -1013,8 +1022,8 @@ int dense_rows_launch(const void* x, const void* w, int w_kmajor, const void* bi
         if (rider)
             if (int e = reduce_jobs_launch(*rider, s)) return e;
         // (wide against any, 16-bit, us: [10431,200] -> 112 7.0 / 12.7, [50000,256] -> 128 9.7 / 24)
-        const int r = dense_wide_rows_launch(x, w, w_kmajor, bias, rowbias, y, N, K, NO, P, dtype, s);
-        if (r != -1) return r;
+        const int r = dense_wide_rows_launch(x, w, w_kmajor, bias, rowbias, y, N, K, NO, P, dtype, s, map);
+        if (r != -1 || map) return r;
         return dense_any_rows_launch(x, w, w_kmajor, bias, rowbias, y, N, K, NO, P, dtype, s);
     }
     if (rider && colsum) return -1;
@@ -1044,7 +1053,7 @@ int dense_rows_launch(const void* x, const void* w, int w_kmajor, const void* bi
     if (blocks < 1) blocks = 1;
     const size_t lds = ((size_t)nnt * 32 * ((nkt > 4 ? 128 : 64) + 8) + 4 * 32 * ((K > NO ? K : NO) + 8)) * 2 +
                        ((bias || rowbias) ? (size_t)4 * 2 * nnt * 32 * sizeof(float) : 0);
-    const int shape = tune_env("PDW_DENSE_GENERIC") ? 0 : (K == 128 && NO == 64) ? 1 : (K == 64 && NO == 128) ? 2 : 0;
+    const int shape = map || tune_env("PDW_DENSE_GENERIC") ? 0 : (K == 128 && NO == 64) ? 1 : (K == 64 && NO == 128) ? 2 : 0;
     if (rider) {
         // The summations come first in the grid and take resident slots of their own from the start (the slots
         // are two per compute unit; waiting for finished row workgroups would put their latency behind the
@@ -1075,7 +1084,7 @@ int dense_rows_launch(const void* x, const void* w, int w_kmajor, const void* bi
     }
 #define PDW_GO(T, KM, CSUM, SK, SNO)                                                                             \
     hipLaunchKernelGGL((dense_rows_k<T, KM, CSUM, SK, SNO>), dim3((unsigned)blocks), dim3(256), lds, s, (const T*)x, \
-                       (const T*)w, (const T*)bias, rowbias, (T*)y, colsum, N, K, NO, P > 0 ? P : 1, nkt, nnt)
+                       (const T*)w, (const T*)bias, rowbias, (T*)y, colsum, N, K, NO, P > 0 ? P : 1, nkt, nnt, map ? *map : RowMap{})
 #define PDW_GO_S(T, KM, CSUM)             \
     if (shape == 1)                       \
         PDW_GO(T, KM, CSUM, 128, 64);     \
@@ -1090,9 +1099,9 @@ int dense_rows_launch(const void* x, const void* w, int w_kmajor, const void* bi
         PDW_GO_S(T, KM, false);           \
     }
     // conv_up of a 96- or 64-feature pyramid block (with the tile sums): its extents as constants, too
-    if (K == 96 && NO == 48 && colsum && !w_kmajor && !tune_env("PDW_DENSE_GENERIC")) {
+    if (K == 96 && NO == 48 && colsum && !w_kmajor && !map && !tune_env("PDW_DENSE_GENERIC")) {
         if (dtype == kF16) PDW_GO(f16_t, false, true, 96, 48); else PDW_GO(bf16_t, false, true, 96, 48);
-    } else if (K == 64 && NO == 32 && colsum && !w_kmajor && !tune_env("PDW_DENSE_GENERIC")) {
+    } else if (K == 64 && NO == 32 && colsum && !w_kmajor && !map && !tune_env("PDW_DENSE_GENERIC")) {
         if (dtype == kF16) PDW_GO(f16_t, false, true, 64, 32); else PDW_GO(bf16_t, false, true, 64, 32);
     } else
     if (dtype == kF16) {

@@ -109,6 +109,19 @@ struct Operand {
             }
         }
     }
+    // results of a tensor that leaves some out (RowMap): result c at its row c % seg + val (c / seg), zero where c % seg >= val
+    __device__ __forceinline__ void init(const char* p, int ld, long long r0, long long nres, long long kb, long long ke, const RowMap& map) {
+        static_assert(!TR, "stored by results");
+        rsrc = rsrc_of(p + kb * ES, (uint32_t)((2 * map.val - 1) * ld + (ke - kb)) * ES);
+        step = kRowBytes;
+#pragma unroll
+        for (int j = 0; j < NL; ++j) {
+            const int slot = j * 256 + (int)threadIdx.x, row = slot / CPR, c = swz(row, slot % CPR);
+            const int res = (int)r0 + row, hi = res >= map.seg, r = res - hi * map.seg;
+            kc[j] = c * VE;
+            off[j] = r < map.val && res < nres ? (uint32_t)((r + hi * map.val) * ld + c * VE) * ES : kPast;
+        }
+    }
     // requests stage `st` (inner values left from its start: left) into buf
     __device__ __forceinline__ void request(lds_char* buf, int st, int left) const {
         const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -215,6 +228,7 @@ struct WideArgs {
     int N, lda, ldb, P;   // results along b
     int mt, nt, splits;
     long long kper;       // inner values per split (a multiple of 64)
+    RowMap map;           // of b's results (16-bit rows, stored by results)
 };
 
 // Results [M][N] = sum over k of a(m,k) b(n,k).  The b operand is the matrix instruction's first, so that a lane holds
@@ -245,7 +259,12 @@ __device__ __forceinline__ void wide_gemm_body(const WideArgs& g, int blk, int n
     OpA a;
     OpB b;
     a.init((const char*)g.a, g.lda, m0, g.M, kb, ke);
-    b.init((const char*)g.b, g.ldb, n0, g.N, kb, ke);
+    if constexpr (!TB && !PART && sizeof(T) == 2) {
+        if (g.map.seg) b.init((const char*)g.b, g.ldb, n0, g.N, kb, ke, g.map);   // (uniform)
+        else b.init((const char*)g.b, g.ldb, n0, g.N, kb, ke);
+    } else {
+        b.init((const char*)g.b, g.ldb, n0, g.N, kb, ke);
+    }
     const int left = (int)(ke - kb), nst = (left + BK - 1) / BK;
     v16f acc[FM][FN];
 #pragma unroll
@@ -628,11 +647,13 @@ static bool wide_rows_plan(WideArgs& g, int& bm, int& bn, const void* x, const v
 
 // -1: not covered.
 int dense_wide_rows_launch(const void* x, const void* w, int w_kmajor, const void* bias, const float* rowbias, void* y,
-                           long long N, int K, int NO, int P, int dtype, hipStream_t s) {
+                           long long N, int K, int NO, int P, int dtype, hipStream_t s, const RowMap* map) {
     WideArgs g;
     int bm, bn;
+    if (map && (w_kmajor || dtype == kF32)) return -1;
     if (!wide_rows_plan(g, bm, bn, x, w, w_kmajor, bias, rowbias, y, N, K, NO, P, dtype)) return -1;
     if (N == 0) return 0;
+    if (map) g.map = *map;
 #define PDW_WIDE_T(T, BM, BN) (w_kmajor ? wide_go<T, BM, BN, false, true, false>(g, s) : wide_go<T, BM, BN, false, false, false>(g, s))
 #define PDW_WIDE(BM, BN) (dtype == kF16 ? PDW_WIDE_T(f16_t, BM, BN) : PDW_WIDE_T(bf16_t, BM, BN))
 #define PDW_WIDE2(BM, BN) (dtype == kF16 ? PDW_WIDE2_T(f16_t, BM, BN) : PDW_WIDE2_T(bf16_t, BM, BN))   /* (tiles of launches that fill the chip) */

@@ -105,9 +105,14 @@ int pool_branch_bwd_launch(const void* gy, const void* m, const void* wp, void* 
 // dense.hip: thin dense layers on the matrix cores (16-bit types, inner dims <= 128); -1 = not covered
 int dense_rows_supported(int K, int NO, int dtype);
 // colsum (optional, fp32 [ceil(N/R)][K], K = 64 or 128, R = dense_colsum_rows()): sums of x over groups of R rows
+// map: result columns that the weights leave out.  Column c has the weights of row c % seg + val (c / seg) where c % seg < val (two
+// segments: NO = 2 seg), and is zero elsewhere; w_kmajor = 0, no bias, no rowbias, 16-bit types, else -1
+struct RowMap {
+    int seg = 0, val = 0;
+};
 int dense_rows_launch(const void* x, const void* w, int w_kmajor, const void* bias, const float* rowbias, void* y,
                       long long N, int K, int NO, int P, int dtype, hipStream_t s, float* colsum = nullptr,
-                      const struct ReduceJobs* rider = nullptr);
+                      const struct ReduceJobs* rider = nullptr, const RowMap* map = nullptr);
 // the 128 -> 64 layer over the pixels of [B, H, W] images with the tile sums of x (tiles of 4 rows x 8 columns) and the
 // 2x2 average pool of y; -1 = not covered
 int dense_rows_pool_launch(const void* x, const void* w, const void* bias, void* y, float* colsum, void* pool, int B,
@@ -150,7 +155,7 @@ int dense_any_wgrad_launch(const void* a, const void* b, void* dw, void* ws, lon
 // dense_wide.hip: tiles of 128 x 128 results, widths that are multiples of 16 bytes; -1 = not covered
 bool dense_wide_ok(int K, int NO, int dtype);
 int dense_wide_rows_launch(const void* x, const void* w, int w_kmajor, const void* bias, const float* rowbias, void* y,
-                           long long N, int K, int NO, int P, int dtype, hipStream_t s);
+                           long long N, int K, int NO, int P, int dtype, hipStream_t s, const RowMap* map = nullptr);
 size_t dense_wide_wgrad_workspace(long long N, int M, int NO);
 int dense_wide_bwd_pair_launch(const void* gy, const void* w, const void* b, void* dx, void* dw, void* ws, const float* rowbias, int P,
                                long long N, int M, int NO, int dtype, int max_chunks, hipStream_t s);

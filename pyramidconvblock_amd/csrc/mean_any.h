@@ -7,6 +7,7 @@
 // launches that this replaces (two sums, two products with up to 128 partials an image) took 10 + 24 + 10 + 52 us.
 #pragma once
 #include "common.h"
+#include "pack_weights.h"
 
 namespace pdw {
 
@@ -277,8 +278,9 @@ inline bool mean_any_ok(const void* x, const void* wp, const void* m, int D, int
 }
 
 // resample.hip: the launches that they ride in.
-// xp = adaptive average pool of a to (h, w), with the column sums
-int avgpool_colsum_launch(const void* a, void* xp, int B, int H, int W, int C, int h, int w, const ColsumJob& sums, int dtype, hipStream_t s);
+// xp = adaptive average pool of a to (h, w), with the column sums and the packing of weights that are given
+int avgpool_with_launch(const void* a, void* xp, int B, int H, int W, int C, int h, int w, const ColsumJob* sums, const PackArgs* pack,
+                        int dtype, hipStream_t s);
 // gate_pair_fwd_launch with the mean branch's forward
 int gate_pair_mean_fwd_launch(const void* xf, const void* xh, void* y, int B, int H, int W, int h, int w, int I, int ldy,
                               const MeanJob& mean, int dtype, hipStream_t s, int gw);

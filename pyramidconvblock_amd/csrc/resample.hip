@@ -89,13 +89,15 @@ __global__ __launch_bounds__(256) void avgpool_fwd_k(const T* __restrict__ x, T*
     if (idx < total) avgpool_fwd_item<T, VEC>(x, y, H, W, C, h, w, idx);
 }
 
-// The same with the column sums of another tensor (mean_any.h) in the first workgroups: both are bandwidth.
+// The same with the column sums of another tensor (mean_any.h) and the packing of weights (pack_weights.h) in the first
+// workgroups: all are bandwidth.
 template <typename T, int VEC>
-__global__ __launch_bounds__(256) void avgpool_colsum_k(const T* __restrict__ x, T* __restrict__ y, int H, int W, int C,
-                                                        int h, int w, long long total, const ColsumJob sums, int nsums) {
+__global__ __launch_bounds__(256) void avgpool_with_k(const T* __restrict__ x, T* __restrict__ y, int H, int W, int C, int h,
+                                                      int w, long long total, const ColsumJob sums, int nsums, const PackArgs pack, int npack) {
     extern __shared__ float sm[];
     if ((int)blockIdx.x < nsums) return colsum_body<T>(sums, blockIdx.x, sm);
-    const long long idx = (long long)(blockIdx.x - nsums) * blockDim.x + threadIdx.x;
+    if ((int)blockIdx.x - nsums < npack) return pack_weights_body(pack, blockIdx.x - nsums);
+    const long long idx = (long long)(blockIdx.x - nsums - npack) * blockDim.x + threadIdx.x;
     if (idx < total) avgpool_fwd_item<T, VEC>(x, y, H, W, C, h, w, idx);
 }
 
@@ -1356,19 +1358,22 @@ int avgpool_fwd_launch(const void* x, void* y, int B, int H, int W, int C, int h
     return check_launch("avgpool_fwd");
 }
 
-int avgpool_colsum_launch(const void* a, void* xp, int B, int H, int W, int C, int h, int w, const ColsumJob& sums, int dtype,
-                          hipStream_t s) {
+int avgpool_with_launch(const void* a, void* xp, int B, int H, int W, int C, int h, int w, const ColsumJob* sums,
+                        const PackArgs* pack, int dtype, hipStream_t s) {
+    if (!sums && !pack) return avgpool_fwd_launch(a, xp, B, H, W, C, h, w, dtype, s);
     const void* ptrs[2] = {a, xp};
     const int vec = pick_vec(C, esize(dtype), ptrs, 2);
     const long long total = (long long)B * h * w * (C / vec);
-    const int nsums = colsum_workgroups(sums);
+    const int nsums = sums ? colsum_workgroups(*sums) : 0, npack = pack ? pack_workgroups(*pack) : 0;
     unsigned blocks;
-    if (!grid_for(total, &blocks) || (unsigned long long)blocks + nsums > 0x7fffffffULL) return 1;
-    const size_t lds = 256 * 16 / esize(dtype) * sizeof(float);
-#define CALL(T, V) hipLaunchKernelGGL((avgpool_colsum_k<T, V>), dim3(blocks + nsums), dim3(256), lds, s, (const T*)a, (T*)xp, H, W, C, h, w, total, sums, nsums);
+    if (!grid_for(total, &blocks) || (unsigned long long)blocks + nsums + npack > 0x7fffffffULL) return 1;
+    const size_t lds = sums ? 256 * 16 / esize(dtype) * sizeof(float) : 0;
+#define CALL(T, V)                                                                                                                       \
+    hipLaunchKernelGGL((avgpool_with_k<T, V>), dim3(blocks + nsums + npack), dim3(256), lds, s, (const T*)a, (T*)xp, H, W, C, h, w, total, \
+                       sums ? *sums : ColsumJob{}, nsums, pack ? *pack : PackArgs{}, npack);
     PDW_TYPE_SWITCH(dtype, vec, CALL)
 #undef CALL
-    return check_launch("avgpool_colsum");
+    return check_launch("avgpool_with");
 }
 
 int avgpool_bwd_launch(const void* gy, void* gx, int B, int H, int W, int C, int h, int w, int accumulate, int dtype,

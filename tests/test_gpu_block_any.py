@@ -4,6 +4,7 @@ and the small tensors that run unpadded."""
 import pytest
 import torch
 
+from parity import assert_close
 from test_gpu_block import _block_case
 
 pytestmark = pytest.mark.gpu
@@ -16,6 +17,35 @@ pytestmark = pytest.mark.gpu
 ])
 def test_padded_inner_channels(oracle, dtype, dim, k, shape):
     _block_case(oracle, dim, k, shape, dtype)
+
+
+@pytest.mark.parametrize("dim,inter,k,shape,shift", [
+    # conv_up on tiles of whole images with their sums (a width that fills the tiles, and one that does not), on others, on
+    # wide tiles of 64 and 128 results, and on weights that it does not read in place (8 bytes off the alignment)
+    (128, 124, 5, (2, 32, 32), 0), (72, 36, 7, (2, 32, 32), 0), (104, 52, 7, (1, 30, 34), 0), (136, 68, 5, (2, 32, 32), 0),
+    (264, 132, 3, (1, 9, 11), 0), (392, 196, 3, (1, 7, 12), 0), (104, 52, 7, (1, 30, 34), 4), (264, 132, 3, (1, 9, 11), 4),
+])
+def test_weights_read_as_given_and_packed_beside_the_pool(oracle, dim, inter, k, shape, shift):
+    """Padded halves: conv_up skips the rows that its weights do not have, the pool's launch packs all four."""
+    import pyramid_dwconv
+
+    dtype = torch.bfloat16
+    torch.manual_seed(3)
+    m = pyramid_dwconv.ConvBlock(dim=dim, kernel_size=k, inter_ratio=inter / dim).to(dtype)
+    x, g = (torch.randn(*shape, dim).to(dtype) for _ in range(2))
+    params = {n: p.detach().double().numpy() for n, p in m.state_dict().items()}
+    yo, cache = oracle.convblock_fwd(x.double().numpy(), params)
+    dxo, go = oracle.convblock_bwd(cache, g.double().numpy())
+    m = m.cuda()
+    w = m.conv_up.weight
+    w.data = torch.cat([w.data.new_zeros(shift), w.data.flatten()])[shift:].view_as(w)
+    xd = x.cuda().requires_grad_()
+    y = m(xd)
+    assert_close(y, yo, dtype, "y")
+    torch.autograd.backward(y, g.cuda())
+    assert_close(xd.grad, dxo, dtype, "dx")
+    for n, p in m.named_parameters():
+        assert_close(p.grad, go[n], dtype, "grad " + n)
 
 
 @pytest.mark.parametrize("dtype,dim,k,shape", [
