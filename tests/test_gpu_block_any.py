@@ -1,6 +1,6 @@
 """16-bit blocks whose inner width is not a multiple of 8 (laid out with padded halves, weights packed, gradients
 unpacked: csrc/block_any.hip) against the float64 block oracle: gate widths 2, 6, 10, 50 and 132 + 2, even and odd extents,
-and the small tensors that run unpadded."""
+small tensors and large ones."""
 import pytest
 import torch
 
@@ -14,6 +14,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("dim,k,shape", [
     (8, 17, (2, 60, 60, 8)), (24, 9, (3, 33, 40, 24)), (40, 15, (4, 13, 13, 40)), (88, 13, (2, 28, 32, 88)),
     (200, 5, (1, 57, 61, 200)), (264, 7, (2, 20, 24, 264)), (536, 3, (1, 7, 9, 536)), (40, 3, (2, 9, 8, 40)),
+    (8, 3, (1, 2, 2, 8)), (24, 17, (1, 7, 7, 24)), (56, 5, (2, 3, 16, 56)), (136, 9, (1, 2, 31, 136)), (248, 13, (1, 7, 8, 248)),
 ])
 def test_padded_inner_channels(oracle, dtype, dim, k, shape):
     _block_case(oracle, dim, k, shape, dtype)
