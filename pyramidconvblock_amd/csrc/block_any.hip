@@ -48,11 +48,15 @@ struct Shape {
 // dense tiles take them, and the padding would cost more than 8-byte instead of 16-byte gates (108 against 101 us for a training step
 // at [41,16,17,80]).  Others are padded at any size, since the matrix-core convolutions and shared launches take those only: as
 // graphs, unpadded and padded, training [1,8,8,40] filter 3 69.4 and 52.2 us, filter 17 125.9 and 57, [2,20,20,136] filter 9 100 and 58,
-// inference [1,8,8,40] filter 3 28.3 and 25.3, [1,40,40,248] filter 5 36.1 and 28.4.
-int padded_half(int D, int I, int dtype) { return dtype == kF32 || D % 8 != 0 || I % 8 == 0 ? I / 2 : (I / 2 + 7) / 8 * 8; }
+// inference [1,8,8,40] filter 3 28.3 and 25.3, [1,40,40,248] filter 5 36.1 and 28.4.  Filters beyond 17 run on the vector ALU both
+// ways and are padded where the tensor is large ([1,14,14,40], filter 19: 284 and 332).
+int padded_half(long long N, int D, int I, int K, int dtype) {
+    const bool as_is = dtype == kF32 || D % 8 != 0 || I % 8 == 0 || (K > 17 && D <= 256 && N * I * K * K < 2000000);
+    return as_is ? I / 2 : (I / 2 + 7) / 8 * 8;
+}
 
 Shape shape_of(int B, int H, int W, int h, int w, int D, int I, int K, int dtype) {
-    const int G = I / 2, Gp = padded_half(D, I, dtype);
+    const int G = I / 2, Gp = padded_half((long long)B * H * W, D, I, K, dtype);
     Shape s{B, H, W, h, w, D, 2 * Gp, K, dtype, dtype == kF32 ? 4 : 2, H * W, G, Gp, (long long)B * H * W, (long long)B * h * w, false, false};
     s.exact = H == 2 * h && W == 2 * w;
     s.single = s.exact && !s.padded() && pdw_convblock_supported(B, H, W, D, I, K, dtype) != 0;
@@ -367,7 +371,7 @@ int pdw_block_supported(int B, int H, int W, int h, int w, int D, int I, int K, 
         !(H == 2 * h && W == 2 * w && pdw_convblock_supported(B, H, W, D, I, K, dtype)))
         return 0;
     if ((long long)B * h * w * I > 0x7fffffffLL) return 0;
-    const int Il = 2 * padded_half(D, I, dtype);
+    const int Il = 2 * padded_half((long long)B * H * W, D, I, K, dtype);
     if (Il * (long long)B * H * W > 0x7fffffffLL) return 0;
     return layer_ok(D, Il, dtype) && layer_ok(Il, D, dtype) ? 1 : 0;
 }
