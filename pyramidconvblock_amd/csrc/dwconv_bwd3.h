@@ -1,8 +1,8 @@
 // The three convolution launches at the end of a two-scale block's backward pass that do not depend on one another
 // (the full-scale input gradient, with the pooled branch's gradient added where the pool halved the extents, and the weight
 // gradients of both scales) as one launch: on a compute unit a band of each runs back to back, without two drains and
-// launch gaps in between.  Every problem runs in the tile that its width fills better: by template where both full-scale
-// problems' are the wide ones, the pool halved the extents and no mean branch rides along (each workgroup starts with one
+// launch gaps in between.  Every problem runs in the tile that its width fills better: by template where the input
+// gradient's is the wide one, the pool halved the extents and no mean branch rides along (each workgroup starts with one
 // problem's arguments), at run time per problem elsewhere.  (With bands of one image the template was 0.2 to 1.2 us faster; with runs
 // both take as long: [32,56,56,64] filter 9 26.0 and 25.9 us, 13 28.6 and 28.7, 17 50.0 and 49.8, [128,56,56,64] filter 13 76.0 and 76.5.)
 // The kernel template and its per-filter-size launcher; dwconv_bwd3_k<K>.hip instantiate it, one file per size.
@@ -10,7 +10,6 @@
 #include "dwconv_fwd2.h"
 #include "dwconv_tz.h"
 #include "dwconv_wgrad_ph.h"
-#include "dwconv_wgrad_tz.h"
 #include <algorithm>
 #include <map>
 #include <tuple>
@@ -22,53 +21,41 @@
 
 namespace pdw {
 
-// The weight gradient's kernel by filter size: phase-major (dwconv_wgrad_ph.h) up to 15, dwconv_wgrad_tz.h beyond.
-constexpr bool bwd3_phases(int K) { return K <= kWgPhMaxK; }
-template <int K>
-using Bwd3Geom = std::conditional_t<bwd3_phases(K), WgPhGeom, WgTzGeom>;
-
-template <int K>
 struct Bwd3Wgrad {
     const void *x, *gy;
     float* part;
-    Bwd3Geom<K> g;
-    int ncb;       // column blocks of a tile (8 or 5; filters beyond 15)
+    WgPhGeom g;
     int start, n;  // first workgroup and number of workgroups
 };
 
-template <int K>
 struct Bwd3Args {
     const void *gy, *w, *add;   // input gradient: dx = conv^T(gy, w) (+ add / 4 over 2x2 blocks)
     void* dx;
     TzGeom gd;
     int npcd;                   // patches of its tile side by side (16 or 8)
     int sd, nd;
-    Bwd3Wgrad<K> p[2];          // full scale, pooled scale
+    Bwd3Wgrad p[2];          // full scale, pooled scale
     MeanJob mean;               // nmean workgroups behind the others: the backward of the block's mean branch, which needs
     int nmean;                  // nothing of this launch and whose result is read after it
 };
 
-template <typename T, int K, int NCB>
-__device__ __forceinline__ void bwd3_wgrad(const void* x, const void* gy, float* part, const Bwd3Geom<K>& g, int blk, int nblk) {
-    if constexpr (bwd3_phases(K))
-        dwconv_wgrad_ph_body<T, wgrad_ph_ncopy(K), wgrad_ph_gr(K)>((const T*)x, (const T*)gy, part, g, blk, nblk);
-    else
-        dwconv_wgrad_tz_body<T, NCB>((const T*)x, (const T*)gy, part, g, blk, nblk);
+template <typename T, int K>
+__device__ __forceinline__ void bwd3_wgrad(const void* x, const void* gy, float* part, const WgPhGeom& g, int blk, int nblk) {
+    dwconv_wgrad_ph_body<T, wgrad_ph_ncopy(K), wgrad_ph_gr(K)>((const T*)x, (const T*)gy, part, g, blk, nblk);
 }
 
 // Each problem's workgroups are a contiguous range of the grid, in the order the launcher chose.
-// NCB1: column blocks of the pooled scale's tile (filters beyond 15; else 8), the input gradient's tile being 16 patches, the
-// full scale's 8 blocks, and no mean branch; 0: all as the arguments say.
-template <typename T, int K, int CS, int NCB1, int MODE>
-__global__ __launch_bounds__(512, 1) void dwconv_bwd3_k(const Bwd3Args<K> a) {
+// WIDE: the input gradient's tile is 16 patches, and no mean branch; else as the arguments say.
+template <typename T, int K, int CS, bool WIDE, int MODE>
+__global__ __launch_bounds__(512, 1) void dwconv_bwd3_k(const Bwd3Args a) {
     const int blk = blockIdx.x;
-    if constexpr (NCB1 != 0) {
+    if constexpr (WIDE) {
         if ((unsigned)(blk - a.sd) < (unsigned)a.nd)
             dwconv_tz_body<T, K, 16, CS, MODE>((const T*)a.gy, (const T*)a.w, (const T*)a.add, nullptr, (T*)a.dx, a.gd, blk - a.sd, a.nd);
         else if ((unsigned)(blk - a.p[1].start) < (unsigned)a.p[1].n)
-            bwd3_wgrad<T, K, NCB1>(a.p[1].x, a.p[1].gy, a.p[1].part, a.p[1].g, blk - a.p[1].start, a.p[1].n);
+            bwd3_wgrad<T, K>(a.p[1].x, a.p[1].gy, a.p[1].part, a.p[1].g, blk - a.p[1].start, a.p[1].n);
         else
-            bwd3_wgrad<T, K, 8>(a.p[0].x, a.p[0].gy, a.p[0].part, a.p[0].g, blk - a.p[0].start, a.p[0].n);
+            bwd3_wgrad<T, K>(a.p[0].x, a.p[0].gy, a.p[0].part, a.p[0].g, blk - a.p[0].start, a.p[0].n);
     } else {
         if (blk >= a.nd + a.p[0].n + a.p[1].n) {
             extern __shared__ uint32_t smem[];
@@ -84,33 +71,26 @@ __global__ __launch_bounds__(512, 1) void dwconv_bwd3_k(const Bwd3Args<K> a) {
         const bool full = (unsigned)(blk - a.p[0].start) < (unsigned)a.p[0].n;
         const void *x = full ? a.p[0].x : a.p[1].x, *gy = full ? a.p[0].gy : a.p[1].gy;
         float* const part = full ? a.p[0].part : a.p[1].part;
-        const Bwd3Geom<K> g = full ? a.p[0].g : a.p[1].g;
-        const int at = blk - (full ? a.p[0].start : a.p[1].start), n = full ? a.p[0].n : a.p[1].n;
-        if constexpr (bwd3_phases(K)) {
-            bwd3_wgrad<T, K, 8>(x, gy, part, g, at, n);
-        } else {
-            if ((full ? a.p[0].ncb : a.p[1].ncb) == 8) bwd3_wgrad<T, K, 8>(x, gy, part, g, at, n);
-            else bwd3_wgrad<T, K, 5>(x, gy, part, g, at, n);
-        }
+        const WgPhGeom g = full ? a.p[0].g : a.p[1].g;
+        bwd3_wgrad<T, K>(x, gy, part, g, blk - (full ? a.p[0].start : a.p[1].start), full ? a.p[0].n : a.p[1].n);
     }
 }
 
 // Cuts and grid order of the three problems.  A compute unit holds one workgroup of this launch at a time, and a workgroup
 // costs a start-up (first rows, operand set-up) that does not depend on how many rows it takes, so unlike a launch of its
 // own, which has to fill the chip, a problem here is best cut into as few pieces as the other problems leave room for: all
-// three in one round of the chip, ending together, where that is possible; else each candidate (runs of several lengths; bands
-// per image for the weight gradients of dwconv_wgrad_tz.h) is priced by dealing its workgroups, longest problem first (the grid
+// three in one round of the chip, ending together, where that is possible; else each candidate (runs of several lengths)
+// is priced by dealing its workgroups, longest problem first (the grid
 // order), to the compute units.  us a call with its two summations, 20 of them in a graph, against whole-image bands of one
-// image: [32,56,56,64] filter 9 32.8 -> 25.9, 13 32.3 -> 28.5, 15 43.5 -> 33.9, 17 (bands still) 51.1 -> 49.2; [128,56,56,64] filter 13
-// 100.5 -> 75.8, 17 167 -> 156.  What the runs cost: the two problems that share gy read it at different times, and [32,56,56,64]
+// image: [32,56,56,64] filter 9 32.8 -> 25.9, 13 32.3 -> 28.5, 15 43.5 -> 33.9; [128,56,56,64] filter 13 100.5 -> 75.8.  What the runs cost: the two problems that share gy read it at different times, and [32,56,56,64]
 // filter 13 fetches and writes 67.3 MB where bands moved 51.6 (48.2 are needed).
 struct Bwd3Plan {
-    int n[3];         // rows of the input gradient's runs; runs or bands of the full scale's and the half scale's weight gradient
+    int n[3];         // rows of the input gradient's runs; runs of the full scale's and the half scale's weight gradient
     char order[4];    // 'D', 'F', 'H' in grid order
 };
 
-template <int K, int CS, typename P>
-static Bwd3Plan bwd3_plan(int B, const TzGeom& gd, int npcd, const P& p0, const P& p1, int nmean) {
+template <int K>
+static Bwd3Plan bwd3_plan(int B, const TzGeom& gd, int npcd, const WgPhPlan& p0, const WgPhPlan& p1, int nmean) {
     static std::mutex mu;
     struct Key {
         int B, H, W, h, w, C, nmean;
@@ -127,40 +107,22 @@ static Bwd3Plan bwd3_plan(int B, const TzGeom& gd, int npcd, const P& p0, const 
     constexpr double kStart = 5.0, kStep = 1.15;
     const int ni = 16 / npcd;
     Bwd3Plan best{{8, 1, 1}, "DFH"};
-    bool balanced = false;
-    if constexpr (bwd3_phases(K)) {
-        auto part = [](const P& p) { return LaunchPart{kWgPhStart, wgrad_ph_step(K), p.total, p.g.passes, [p](int s) { return p.per_chunk * cdiv(p.total, s); }}; };
-        const LaunchPart parts[3] = {tz_part(gd, ni, kStart, kStep), part(p0), part(p1)};
-        int steps[3];
-        if ((balanced = launch_balance(parts, nmean, steps))) {
-            TzGeom c = gd;
-            tz_cut_steps(c, ni, steps[0]);
-            best = Bwd3Plan{{c.run, cdiv(p0.total, steps[1]), cdiv(p1.total, steps[2])}, "DFH"};
-        }
-    }
-    if (!balanced) {
+    auto part = [](const WgPhPlan& p) { return LaunchPart{kWgPhStart, wgrad_ph_step(K), p.total, p.g.passes, [p](int s) { return p.per_chunk * cdiv(p.total, s); }}; };
+    const LaunchPart parts[3] = {tz_part(gd, ni, kStart, kStep), part(p0), part(p1)};
+    int steps[3];
+    if (launch_balance(parts, nmean, steps)) {
+        TzGeom c = gd;
+        tz_cut_steps(c, ni, steps[0]);
+        best = Bwd3Plan{{c.run, cdiv(p0.total, steps[1]), cdiv(p1.total, steps[2])}, "DFH"};
+    } else {
         std::vector<LaunchCut> cuts[3];
         tz_cuts(cuts[0], gd, ni, kStart, kStep);
         for (int i = 1; i < 3; ++i) {
-            P p = i == 1 ? p0 : p1;
-            if constexpr (bwd3_phases(K)) {
-                const int most = p.g.nchunks;
-                for (int e = 8; e >= 1; --e) {
-                    if (!wgrad_ph_cut(p, std::max(1, most * e / 8)) || (!cuts[i].empty() && cuts[i].back().n == p.g.nchunks)) continue;
-                    cuts[i].push_back({p.g.nchunks, wgrad_ph_run_cost(K, p.g.passes), p.nblocks});
-                }
-            } else {
-                const long long per_band = (long long)B * p.g.ncolt * p.g.nslices;
-                for (int pick : {1, 2, 4, 0}) {   // 0: the stand-alone planner's number
-                    // with many times more whole-image bands than compute units the chip is full whatever the cut: fewest start-ups
-                    if (per_band > 1024 && pick != 1) continue;
-                    int nb = pick ? pick : p.g.nbands;
-                    // (the partials must fit the workspace sized for the stand-alone plan)
-                    if (pick && (nb > std::max(1, p.g.OH / 4) || nb > p.g.nbands)) continue;
-                    const int br = (cdiv(p.g.OH, nb) + 3) / 4 * 4;
-                    nb = cdiv(p.g.OH, br);
-                    cuts[i].push_back({nb, 3.0 + 3.0 * (p.ncb == 8 ? 1.0 : 0.9) * ((br + 4) / 4), per_band * nb});
-                }
+            WgPhPlan p = i == 1 ? p0 : p1;
+            const int most = p.g.nchunks;
+            for (int e = 8; e >= 1; --e) {
+                if (!wgrad_ph_cut(p, std::max(1, most * e / 8)) || (!cuts[i].empty() && cuts[i].back().n == p.g.nchunks)) continue;
+                cuts[i].push_back({p.g.nchunks, wgrad_ph_run_cost(K, p.g.passes), p.nblocks});
             }
         }
         const LaunchCut mean{0, kMeanCost, nmean};
@@ -187,9 +149,9 @@ static Bwd3Plan bwd3_plan(int B, const TzGeom& gd, int npcd, const P& p0, const 
     return best;
 }
 
-template <typename T, int K, int CS, int NCB1, int MODE>
-static void bwd3_go(const Bwd3Args<K>& a, unsigned grid, size_t lds, hipStream_t s) {
-    auto kern = dwconv_bwd3_k<T, K, CS, NCB1, MODE>;
+template <typename T, int K, int CS, bool WIDE, int MODE>
+static void bwd3_go(const Bwd3Args& a, unsigned grid, size_t lds, hipStream_t s) {
+    auto kern = dwconv_bwd3_k<T, K, CS, WIDE, MODE>;
     static std::once_flag once;
     std::call_once(once, [&] { (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); });
     hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, s, a);
@@ -209,21 +171,17 @@ static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* 
         for (const void* p : {gyf, w0, (const void*)dx, x0, (const void*)ws0, x1, gy1, (const void*)ws1})
             if (!p || (reinterpret_cast<uintptr_t>(p) & 15)) return -1;
     if (reinterpret_cast<uintptr_t>(addp) & 15) return -1;
-    Bwd3Args<K> a{};
+    Bwd3Args a{};
     a.npcd = tz_wide_tile(B, W) ? 16 : 8;
     if (!(a.npcd == 16 ? tz_make_geom<K, 16, CS>(a.gd, true, B, H, W, C, K - 1 - P, K - 1 - P, true, nullptr)
                        : tz_make_geom<K, 8, CS>(a.gd, true, B, H, W, C, K - 1 - P, K - 1 - P, true, nullptr)))
         return -1;
-    auto plan_of = [&](int hh, int ww) {
-        if constexpr (bwd3_phases(K)) return wgrad_ph_plan(B, hh, ww, C, K, P, P);
-        else return wgrad_tz_plan(B, hh, ww, C, K, P, P);
-    };
-    auto p0 = plan_of(H, W), p1 = plan_of(h, w);
+    WgPhPlan p0 = wgrad_ph_plan(B, H, W, C, K, P, P), p1 = wgrad_ph_plan(B, h, w, C, K, P, P);
     if (!p0.ok || !p1.ok) return -1;
     MeanJob job{};
     if (mean) job = *mean, job.shared = mean_shared(job.B, job.D);
     const int nmean = mean ? mean_bwd_workgroups(job) : 0;
-    Bwd3Plan plan = bwd3_plan<K, CS>(B, a.gd, a.npcd, p0, p1, nmean);
+    Bwd3Plan plan = bwd3_plan<K>(B, a.gd, a.npcd, p0, p1, nmean);
     if (const char* e = tune_env("PDW_BWD3_BANDS")) {   // e.g. "64,31,8,DHF": cuts of D, F, H and the grid order
         if (sscanf(e, "%d,%d,%d,%3s", &plan.n[0], &plan.n[1], &plan.n[2], plan.order) != 4) return -1;
     }
@@ -235,16 +193,9 @@ static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* 
     const long long nd = tz_blocks(a.gd);
     int parts[2], per_image[2];   // partials of the weight gradients, pieces of an image
     for (int i = 0; i < 2; ++i) {
-        auto& p = i == 0 ? p0 : p1;
-        if constexpr (bwd3_phases(K)) {
-            if (!wgrad_ph_cut(p, plan.n[1 + i])) return -1;
-            parts[i] = p.parts(), per_image[i] = cdiv(p.g.nchunks, cdiv(B, p.g.ni));
-        } else {
-            p.g.BR = (cdiv(p.g.OH, plan.n[1 + i]) + 3) / 4 * 4, p.g.nbands = cdiv(p.g.OH, p.g.BR);
-            p.nblocks = (long long)B * p.g.nslices * p.g.ncolt * p.g.nbands;
-            parts[i] = B * p.g.nbands * p.g.ncolt, per_image[i] = p.g.nbands;
-            a.p[i].ncb = p.ncb;
-        }
+        WgPhPlan& p = i == 0 ? p0 : p1;
+        if (!wgrad_ph_cut(p, plan.n[1 + i])) return -1;
+        parts[i] = p.parts(), per_image[i] = cdiv(p.g.nchunks, cdiv(B, p.g.ni));
         a.p[i].g = p.g, a.p[i].n = (int)p.nblocks;
     }
     if (nd + p0.nblocks + p1.nblocks + nmean > 0x7fffffffLL) return -1;
@@ -268,22 +219,14 @@ static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* 
         }
     }
     size_t lds = a.npcd == 16 ? TzShape<K, 16, CS>::lds_bytes : TzShape<K, 8, CS>::lds_bytes;
-    if constexpr (bwd3_phases(K)) {
-        lds = std::max(lds, WgPhShape<wgrad_ph_ncopy(K), wgrad_ph_gr(K)>::lds_bytes);
-    } else {
-        for (const Bwd3Wgrad<K>& p : a.p) lds = std::max(lds, p.ncb == 8 ? WgTzShape<8>::lds_bytes : WgTzShape<5>::lds_bytes);
-    }
+    lds = std::max(lds, WgPhShape<wgrad_ph_ncopy(K), wgrad_ph_gr(K)>::lds_bytes);
     if (nmean) lds = std::max(lds, mean_lds(job.D, 512, job.shared ? kMeanImages : 1));
     const unsigned grid = (unsigned)(nd + p0.nblocks + p1.nblocks + nmean);
     auto go = [&](auto t) {
         using T = decltype(t);
-        const bool wide = a.npcd == 16 && nmean == 0 && (bwd3_phases(K) || a.p[0].ncb == 8);
-        if (!addp) return bwd3_go<T, K, CS, 0, 0>(a, grid, lds, s);
-        if (!wide) return bwd3_go<T, K, CS, 0, 1>(a, grid, lds, s);
-        if constexpr (!bwd3_phases(K)) {
-            if (a.p[1].ncb != 8) return bwd3_go<T, K, CS, 5, 1>(a, grid, lds, s);
-        }
-        bwd3_go<T, K, CS, 8, 1>(a, grid, lds, s);
+        if (!addp) bwd3_go<T, K, CS, false, 0>(a, grid, lds, s);
+        else if (a.npcd == 16 && nmean == 0) bwd3_go<T, K, CS, true, 1>(a, grid, lds, s);
+        else bwd3_go<T, K, CS, false, 1>(a, grid, lds, s);
     };
     if (dtype == kF16) go(f16_t{});
     else go(bf16_t{});

@@ -1,6 +1,6 @@
 // Depthwise weight gradient in fp32 on the fp32 matrix cores: stride 1, dilation 1, odd square filters 3 .. 17.
 //
-// As in dwconv_wgrad_tz.h, with u = 2a + du, v = 8b + dv:  dw[2a+du][8b+dv] = sum over p of xw[p + (2a,8b)] gy[p - (du,dv)],
+// With u = 2a + du, v = 8b + dv:  dw[2a+du][8b+dv] = sum over p of xw[p + (2a,8b)] gy[p - (du,dv)],
 // one v_mfma_f32_16x16x4_f32 with m = (a,b), n = (du,dv), k = 4 positions: an accumulator of 4 registers holds all taps of a
 // channel (filter 17: 27 (a,b), two instructions that share the gy operand).  Four instructions take 16 positions of a row:
 // position 4g + t of the block for lane group g in instruction t, so that a lane's four xw values are one aligned

@@ -1,5 +1,5 @@
 // Depthwise-convolution weight gradient on the dense matrix cores, phase-major (16-bit types, stride 1, dilation 1, square
-// filters up to 15):     dw[u,v,c] = sum_{b,i,j} gy[b,i,j,c] * xw[b, i+u, j+v, c],   xw[r][s] = x[r-PH][s-PW].
+// filters up to 17):     dw[u,v,c] = sum_{b,i,j} gy[b,i,j,c] * xw[b, i+u, j+v, c],   xw[r][s] = x[r-PH][s-PW].
 //
 // A row of 64 gy columns j = 8q + r is kept as 8 vectors G_r, r = j mod 8, of the 8 values q = 0..7, and a row of x as the
 // vectors X_p[q] = xw[8q + p], p = 0 .. 7 + K-1.  A column offset of v is then another vector instead of a shift inside one,
@@ -12,7 +12,7 @@
 // cycles, a quarter of that bank conflicts, the vector ALU 26 % and the matrix pipe 21 %; wavefronts wait for their turn at the
 // LDS a fifth of their time and for data or a barrier a third.  B stays in registers: from one row of x to the next only the
 // gy row that enters changes (GR rows at a time, one read and four selects), so that a product costs one 16-byte LDS read per
-// lane (4 cycles) instead of three (the form of dwconv_wgrad_tz.h: 11 cycles).  The index of a gy row in B is fixed while
+// lane (4 cycles) instead of the 11 cycles of an aligned operand and one at single-element offsets.  The index of a gy row in B is fixed while
 // u = rho - row moves with rho: there are 8 accumulators, by rho mod 8, whose lanes are rotated against each other when they are
 // added at the end (DPP row rotates), and B itself is rotated by 8 lanes once in 8 rows.
 //
@@ -22,10 +22,17 @@
 // Tiles of 64 columns of an image, or of 32 columns of two images side by side (the halves of the vectors).
 // Fixed-order summation of the workgroups' partials (wgrad_reduce_parts), no atomics.
 //
-// us of the kernel (the summation is 4 more), against the form of dwconv_wgrad_tz.h: [8,64,64,1152] filter 9 139 -> 47 (its tiles are
+// us of the kernel (the summation is 4 more), against tiles of one image, gy shifted by elements: [8,64,64,1152] filter 9 139 -> 47 (its tiles are
 // 56 columns wide, 1152 workgroups of one start-up each; 151 MB at 3.2 TB/s now), [32,56,56,64] filter 13 17.6 -> 15.4,
 // [128,56,56,64] 50 -> 37, [128,7,7,1152] filter 3 166 -> 34.  With all of the chip in such runs a pass takes 1.8 us and a run 8 besides
 // (4, 16 and 23 passes of 64 columns in the first three).
+//
+// Filters 16 and 17 have one more column and row than the indices.  The 16 rows of B are then those before x's row (u = 1 .. 16), and
+// the rest comes from 8 products a pass besides the 32 of a channel: column 16 with the pass's 8 rows of x as A's index, row 0 with
+// the vectors p against the phases r and the rows as k groups (both as differences of their indices, added up at the end).
+// Such a pass takes 2.5 us.  us of kernel and summation against a kernel of two accumulators over bands of single images (two 1 KB
+// operands a product): [32,56,56,64] 29.6 -> 23.7, [128,56,56,64] 81 -> 52, [5,47,51,1000] 67 -> 36, [79,7,7,264] 55 -> 24, [1,28,28,64]
+// 10.2 -> 11.2 (within the block's launch, where it runs beside others, no longer: 54.9 and 55.0 its training step).
 #pragma once
 #include <mutex>
 
@@ -36,8 +43,9 @@
 
 namespace pdw {
 
-// NCOPY: 8-vector groups of an x row (p < 8 NCOPY: 2 up to K = 9, 3 up to 15); GR: gy rows that enter B at a time
-// (K + GR - 1 <= 16: a row that is in B too early multiplies into taps beyond the filter).
+// NCOPY: 8-vector groups of an x row (p < 8 NCOPY: 2 up to K = 9, 3 beyond); GR: gy rows that enter B at a time
+// (K + GR - 1 <= 16: a row that is in B too early multiplies into taps beyond the filter).  8: filters 16 and 17, the pass's rows are
+// read at once and enter one by one, each after its own row of x.
 template <int NCOPY, int GR>
 struct WgPhShape {
     static constexpr int NT = 512, CS = 16, CPW = 2;
@@ -47,7 +55,7 @@ struct WgPhShape {
     static constexpr int HALF = 128;   // channels 8..15 sit 32 banks further: a staging write's two 8-channel pieces differ
     static constexpr int XBUF = CS * XPL + HALF, GBUF = CS * GPL + HALF;
     static constexpr size_t lds_bytes = 2 * (size_t)(XBUF + GBUF);
-    static_assert((NCOPY == 2 || NCOPY == 3) && (GR == 2 || GR == 4), "vector groups, rows per update");
+    static_assert((NCOPY == 2 || NCOPY == 3) && (GR == 2 || GR == 4 || GR == 8), "vector groups, rows per update");
     static_assert(XPL % 256 == 0 && GPL % 128 == 0 && lds_bytes <= 160 * 1024, "LDS");
 };
 
@@ -67,6 +75,7 @@ __device__ __forceinline__ void dwconv_wgrad_ph_body(const T* __restrict__ x, co
                                                      float* __restrict__ part, const WgPhGeom& g, int blk, int nblk) {
     using Sh = WgPhShape<NCOPY, GR>;
     constexpr int NT = Sh::NT, CS = Sh::CS, CPW = Sh::CPW, XROW = Sh::XROW, XPL = Sh::XPL, GROW = Sh::GROW, GPL = Sh::GPL;
+    constexpr bool EDGE = GR == 8;   // filters 16 and 17
     extern __shared__ uint32_t smem[];
     char* const xl = reinterpret_cast<char*>(smem);   // [buffer][channel][row][vector p][q] of T
     char* const gl = xl + 2 * Sh::XBUF;               // [buffer][channel][row][phase][q]
@@ -194,53 +203,122 @@ __device__ __forceinline__ void dwconv_wgrad_ph_body(const T* __restrict__ x, co
 #pragma unroll
         for (int t = 0; t < 8; ++t) acc[q][t] = tz_f32x4{0.f, 0.f, 0.f, 0.f};
 
+    // EDGE: column 16 and row 0 of the filter, which a product of 16 columns with the 16 rows before does not hold.
+    // Column 16: products of the pass's 8 rows of x (index) with the 16 gy rows before the pass, and with its own 8:
+    // u = m - n + 16 (n >= m: others lie beyond the filter) and m - n (n <= m).  Row 0: products of the vectors p (index, 0 .. 15 and
+    // 8 .. 23) with the phases r, four rows of x and gy at a time as the k groups: v = p - r.
+    tz_f32x4 before[EDGE ? CPW : 1], own[EDGE ? CPW : 1], row0[EDGE ? CPW : 1][2];
+    if constexpr (EDGE) {
+#pragma unroll
+        for (int q = 0; q < CPW; ++q) before[q] = own[q] = row0[q][0] = row0[q][1] = tz_f32x4{0.f, 0.f, 0.f, 0.f};
+    }
     // One pass from LDS buffer `buffer`, and the next one from registers into the other.
     auto pass_step = [&](int buffer, int pass) {
         const char* const xa = xlane + buffer * Sh::XBUF;
         const char* const ga = glane + buffer * Sh::GBUF;
-        // blocks of 2 rows, the reads of a block ahead of the products of the one before it (left to itself the compiler
-        // requests the whole pass at once and spills)
-        uint4 a[2][2][2][CPW], n[CPW][2];
-        auto read_rows = [&](int blk) {
-            if (2 * blk % GR == 0) {
-#pragma unroll
-                for (int q = 0; q < CPW; ++q)
-#pragma unroll
-                    for (int f = 0; f < 2; ++f) n[q][f] = read16(ga + q * GPL + 2 * blk * GROW + 64 * f);
-            }
-#pragma unroll
-            for (int r = 0; r < 2; ++r)
+        if constexpr (EDGE) {
+            // a row at a time (blocks of two spill), its reads ahead of the products of the one before it
+            uint4 a[2][2][CPW], n[CPW][2], ea[CPW][2], eb;
+            auto read_row = [&](int row) {
 #pragma unroll
                 for (int f = 0; f < 2; ++f)
 #pragma unroll
-                    for (int q = 0; q < CPW; ++q) a[blk % 2][r][f][q] = read16(xa + q * XPL + (2 * blk + r) * XROW + 64 * f);
-        };
-        read_rows(0);
+                    for (int q = 0; q < CPW; ++q) a[row % 2][f][q] = read16(xa + q * XPL + row * XROW + 64 * f);
+            };
+            const char* const xe = xl + plane * XPL + hoff + buffer * Sh::XBUF;
+            const char* const ge = gl + plane * GPL + hoff + buffer * Sh::GBUF;
+            auto read_row0 = [&](int i) {   // channel i % 2, rows 4 (i / 2) ..
+                const int q = i % 2, r = 4 * (i / 2);
 #pragma unroll
-        for (int blk = 0; blk < 4; ++blk) {
-            if (2 * blk % GR == 0) {
-                const bool enters = ln / GR == 2 * blk / GR;
+                for (int t = 0; t < 2; ++t) ea[0][t] = read16(xe + q * XPL + (r + kg) * XROW + (8 * t + ln) * 16);
+                eb = read16(ge + q * GPL + (r + kg) * GROW + (ln & 7) * 16);
+            };
+#pragma unroll
+            for (int q = 0; q < CPW; ++q)
+#pragma unroll
+                for (int f = 0; f < 2; ++f) {
+                    n[q][f] = read16(ga + q * GPL + 64 * f);
+                    ea[q][f] = read16(xe + q * XPL + (ln & 7) * XROW + (16 + 4 * f + kg) * 16);
+                }
+            read_row(0);
+#pragma unroll
+            for (int q = 0; q < CPW; ++q)
+#pragma unroll
+                for (int f = 0; f < 2; ++f) {
+                    before[q] = mfma16(ea[q][f], bop[q][f], before[q], T());
+                    own[q] = mfma16(ea[q][f], n[q][f], own[q], T());
+                }
+#pragma unroll
+            for (int row = 0; row < 8; ++row) {
+                if (row < 7) read_row(row + 1);
+                if (row < 4) read_row0(row);
+                commit(buf[1 - buffer], 1 - buffer, row);
+                __builtin_amdgcn_sched_barrier(0x7);
+#pragma unroll
+                for (int f = 0; f < 2; ++f)
+#pragma unroll
+                    for (int q = 0; q < CPW; ++q) acc[q][row] = mfma16(a[row % 2][f][q], bop[q][f], acc[q][row], T());
+                if (row < 4) {
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) row0[row % 2][t] = mfma16(ea[0][t], eb, row0[row % 2][t], T());
+                }
+                // the pass's gy row `row`, which index `row` of n holds
 #pragma unroll
                 for (int q = 0; q < CPW; ++q)
 #pragma unroll
                     for (int f = 0; f < 2; ++f) {
                         uint4& b = bop[q][f];
-                        b.x = enters ? n[q][f].x : b.x, b.y = enters ? n[q][f].y : b.y;
-                        b.z = enters ? n[q][f].z : b.z, b.w = enters ? n[q][f].w : b.w;
+                        b.x = ln == row ? n[q][f].x : b.x, b.y = ln == row ? n[q][f].y : b.y;
+                        b.z = ln == row ? n[q][f].z : b.z, b.w = ln == row ? n[q][f].w : b.w;
                     }
+                __builtin_amdgcn_sched_barrier(0x7);
+                if (row == 5) commit_copies(buf[1 - buffer], 1 - buffer);
             }
-            if (blk < 3) read_rows(blk + 1);
-            commit(buf[1 - buffer], 1 - buffer, 2 * blk), commit(buf[1 - buffer], 1 - buffer, 2 * blk + 1);
-            __builtin_amdgcn_sched_barrier(0x7);
-#pragma unroll
-            for (int r = 0; r < 2; ++r)
-#pragma unroll
-                for (int f = 0; f < 2; ++f)
+        } else {
+            // blocks of 2 rows, the reads of a block ahead of the products of the one before it (left to itself the compiler
+            // requests the whole pass at once and spills)
+            uint4 a[2][2][2][CPW], n[CPW][2];
+            auto read_rows = [&](int blk) {
+                if (2 * blk % GR == 0) {
 #pragma unroll
                     for (int q = 0; q < CPW; ++q)
-                        acc[q][2 * blk + r] = mfma16(a[blk % 2][r][f][q], bop[q][f], acc[q][2 * blk + r], T());
-            __builtin_amdgcn_sched_barrier(0x7);
-            if (blk == 1) commit_copies(buf[1 - buffer], 1 - buffer);
+#pragma unroll
+                        for (int f = 0; f < 2; ++f) n[q][f] = read16(ga + q * GPL + 2 * blk * GROW + 64 * f);
+                }
+#pragma unroll
+                for (int r = 0; r < 2; ++r)
+#pragma unroll
+                    for (int f = 0; f < 2; ++f)
+#pragma unroll
+                        for (int q = 0; q < CPW; ++q) a[blk % 2][r][f][q] = read16(xa + q * XPL + (2 * blk + r) * XROW + 64 * f);
+            };
+            read_rows(0);
+#pragma unroll
+            for (int blk = 0; blk < 4; ++blk) {
+                if (2 * blk % GR == 0) {
+                    const bool enters = ln / GR == 2 * blk / GR;
+#pragma unroll
+                    for (int q = 0; q < CPW; ++q)
+#pragma unroll
+                        for (int f = 0; f < 2; ++f) {
+                            uint4& b = bop[q][f];
+                            b.x = enters ? n[q][f].x : b.x, b.y = enters ? n[q][f].y : b.y;
+                            b.z = enters ? n[q][f].z : b.z, b.w = enters ? n[q][f].w : b.w;
+                        }
+                }
+                if (blk < 3) read_rows(blk + 1);
+                commit(buf[1 - buffer], 1 - buffer, 2 * blk), commit(buf[1 - buffer], 1 - buffer, 2 * blk + 1);
+                __builtin_amdgcn_sched_barrier(0x7);
+#pragma unroll
+                for (int r = 0; r < 2; ++r)
+#pragma unroll
+                    for (int f = 0; f < 2; ++f)
+#pragma unroll
+                        for (int q = 0; q < CPW; ++q)
+                            acc[q][2 * blk + r] = mfma16(a[blk % 2][r][f][q], bop[q][f], acc[q][2 * blk + r], T());
+                __builtin_amdgcn_sched_barrier(0x7);
+                if (blk == 1) commit_copies(buf[1 - buffer], 1 - buffer);
+            }
         }
         issue(buf[1 - buffer], pass + 3);
         // in the next pass a row's index counts from 8 rows further
@@ -281,7 +359,7 @@ __device__ __forceinline__ void dwconv_wgrad_ph_body(const T* __restrict__ x, co
     lds_barrier();
     float* const ep = reinterpret_cast<float*>(smem);   // [tap][channel], 20 floats a tap
     constexpr int EPP = 20;
-    const int u = (16 - ln) & 15;
+    const int u = EDGE ? 16 - ln : (16 - ln) & 15;   // (EDGE: the rows 16 .. 1 before)
 #pragma unroll
     for (int q = 0; q < CPW; ++q)
 #pragma unroll
@@ -289,6 +367,35 @@ __device__ __forceinline__ void dwconv_wgrad_ph_body(const T* __restrict__ x, co
             const int v = 4 * kg + r;
             if (u < g.K && v < g.K) ep[(u * g.K + v) * EPP + plane + q] = tot[q][r];
         }
+    if constexpr (EDGE) {
+        // per channel [8][24] products of column 16 (n of before, n of own) and [8 phases][24 vectors] of row 0; a tap is the sum of
+        // eight of them, added in this order
+        constexpr int EW = 24, ECH = 2 * 8 * EW + 1;
+        float* const ee = ep + 17 * 17 * EPP;
+        static_assert((17 * 17 * EPP + CS * ECH) * 4 <= Sh::lds_bytes, "LDS");
+#pragma unroll
+        for (int q = 0; q < CPW; ++q) {
+            float* const e = ee + (plane + q) * ECH;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int m = 4 * kg + r;
+                if (m < 8) e[m * EW + ln] = before[q][r];
+                if (m < 8 && ln < 8) e[m * EW + 16 + ln] = own[q][r];
+                if (ln < 8) e[(8 + ln) * EW + m] = row0[q][0][r];
+                if (m >= 8 && ln < 8) e[(8 + ln) * EW + 8 + m] = row0[q][1][r];
+            }
+        }
+        __syncthreads();
+        for (int i = tid; i < 33 * CS; i += NT) {
+            const int c = i % CS, tap = i / CS;   // 0 .. 16: (tap, 16); 17 .. 32: (0, tap - 17)
+            const float* const e = ee + c * ECH;
+            float sum = 0.f;
+#pragma unroll
+            for (int m = 0; m < 8; ++m) sum += tap < 17 ? e[m * EW + (m < tap ? m - tap + 16 : 16 + m - tap)] : e[(8 + m) * EW + tap - 17 + m];
+            const int tu = tap < 17 ? tap : 0, tv = tap < 17 ? 16 : tap - 17;
+            if (tu < g.K && tv < g.K) ep[(tu * g.K + tv) * EPP + c] = sum;
+        }
+    }
     __syncthreads();
     float* const pc = part + (long long)(chunk * g.ncolt + ct) * g.K * g.K * g.C;
     for (int i = tid; i < g.K * g.K * (CS / 4); i += NT) {
@@ -318,10 +425,9 @@ __global__ __launch_bounds__(512, 1) void dwconv_wgrad_ph_pair_k(const T* __rest
 // ------------------------------------------------------------------------------------------------
 // Host side
 
-// Beyond 15 (with two rows entering at a time) the taps of a row or column are more than the 16 of an operand's index.
-constexpr int kWgPhMaxK = 15;
+constexpr int kWgPhMaxK = 17;
 constexpr int wgrad_ph_ncopy(int K) { return K <= 9 ? 2 : 3; }
-constexpr int wgrad_ph_gr(int K) { return K <= 13 ? 4 : 2; }
+constexpr int wgrad_ph_gr(int K) { return K <= 13 ? 4 : K <= 15 ? 2 : 8; }
 
 struct WgPhPlan {
     bool ok = false;
@@ -343,12 +449,13 @@ inline bool wgrad_ph_cut(WgPhPlan& p, int n) {
 }
 
 // Price of a run to the planners, us: start-up (16 gy rows, two round trips to memory, the partial), then passes of 8 rows.  (Of runs
-// that share the chip with other problems; see the top for a chip full of them.)
+// that share the chip with other problems; see the top for a chip full of them.  Beyond 15: training steps of [8,112,112,96], [128,56,56,128]
+// and [26,106,105,80] with filter 17, us, at 1.35 126, 460, 295; 1.85 124, 442, 288; 2.5 122, 434, 286; 3.3 128, 451, 288.)
 constexpr double kWgPhStart = 7.0;
-inline double wgrad_ph_step(int K) { return K <= 9 ? 1.15 : 1.35; }
+inline double wgrad_ph_step(int K) { return K <= 9 ? 1.15 : K <= 15 ? 1.35 : 2.5; }
 inline double wgrad_ph_run_cost(int K, int passes) { return kWgPhStart + wgrad_ph_step(K) * passes; }
 
-// Covered: 16-bit types (the caller checks), C % 8 == 0, K <= 15, 16-byte aligned tensors.
+// Covered: 16-bit types (the caller checks), C % 8 == 0, K <= 17, 16-byte aligned tensors.
 inline WgPhPlan wgrad_ph_plan(int B, int H, int W, int C, int K, int PH, int PW) {
     WgPhPlan p;
     WgPhGeom& g = p.g;

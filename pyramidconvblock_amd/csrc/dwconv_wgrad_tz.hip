@@ -1,8 +1,6 @@
-// Depthwise-convolution weight gradient on the dense matrix cores, 16-bit types: filters up to 15 phase-major
-// (dwconv_wgrad_ph.h), 16 and 17 with all taps over two accumulators (dwconv_wgrad_tz.h).  Instantiations, workspace query and
-// launchers, for one problem and for two of the same filter size in one launch.
+// Depthwise-convolution weight gradient on the dense matrix cores, 16-bit types, phase-major (dwconv_wgrad_ph.h).  Instantiations,
+// workspace query and launchers, for one problem and for two of the same filter size in one launch.
 #include "dwconv_wgrad_ph.h"
-#include "dwconv_wgrad_tz.h"
 
 #include "reduce_parts.h"
 
@@ -10,8 +8,8 @@ namespace pdw {
 
 size_t dwconv_wgrad_tz_workspace(int B, int H, int W, int C, int K, int PH, int PW, int dtype) {
     if (dtype == kF32) return 0;
-    if (const WgPhPlan p = wgrad_ph_plan(B, H, W, C, K, PH, PW); p.ok) return (size_t)p.parts() * K * K * C * sizeof(float);
-    return wgrad_tz_workspace(B, H, W, C, K, PH, PW);
+    const WgPhPlan p = wgrad_ph_plan(B, H, W, C, K, PH, PW);
+    return p.ok ? (size_t)p.parts() * K * K * C * sizeof(float) : 0;
 }
 
 static bool aligned(std::initializer_list<const void*> ptrs) {
@@ -28,7 +26,9 @@ static int reduce(const void* ws, void* dw, int nparts, int n, int dtype, hipStr
 template <typename T>
 static int wgrad_ph_go(const WgPhPlan& p, const void* x, const void* gy, void* ws, hipStream_t s) {
     if (wgrad_ph_ncopy(p.g.K) == 2) return launch_wgrad_ph<T, 2, 4>(p, x, gy, ws, s);
-    return wgrad_ph_gr(p.g.K) == 4 ? launch_wgrad_ph<T, 3, 4>(p, x, gy, ws, s) : launch_wgrad_ph<T, 3, 2>(p, x, gy, ws, s);
+    return wgrad_ph_gr(p.g.K) == 4   ? launch_wgrad_ph<T, 3, 4>(p, x, gy, ws, s)
+           : wgrad_ph_gr(p.g.K) == 2 ? launch_wgrad_ph<T, 3, 2>(p, x, gy, ws, s)
+                                     : launch_wgrad_ph<T, 3, 8>(p, x, gy, ws, s);
 }
 
 template <typename T>
@@ -36,29 +36,19 @@ static int wgrad_ph_pair_go(const WgPhPlan& p0, const void* x0, const void* gy0,
                             const void* gy1, void* ws1, hipStream_t s) {
     const int K = p0.g.K;
     if (wgrad_ph_ncopy(K) == 2) return launch_wgrad_ph_pair<T, 2, 4>(p0, x0, gy0, ws0, p1, x1, gy1, ws1, s);
-    return wgrad_ph_gr(K) == 4 ? launch_wgrad_ph_pair<T, 3, 4>(p0, x0, gy0, ws0, p1, x1, gy1, ws1, s)
-                               : launch_wgrad_ph_pair<T, 3, 2>(p0, x0, gy0, ws0, p1, x1, gy1, ws1, s);
+    return wgrad_ph_gr(K) == 4   ? launch_wgrad_ph_pair<T, 3, 4>(p0, x0, gy0, ws0, p1, x1, gy1, ws1, s)
+           : wgrad_ph_gr(K) == 2 ? launch_wgrad_ph_pair<T, 3, 2>(p0, x0, gy0, ws0, p1, x1, gy1, ws1, s)
+                                 : launch_wgrad_ph_pair<T, 3, 8>(p0, x0, gy0, ws0, p1, x1, gy1, ws1, s);
 }
 
 // -1: not covered (the caller falls back to the other weight-gradient kernels).
 int dwconv_wgrad_tz_launch(const void* x, const void* gy, void* dw, void* ws, int B, int H, int W, int C, int K, int PH,
                            int PW, int dtype, hipStream_t s) {
     if (dtype == kF32 || !aligned({x, gy, ws})) return -1;
-    int r, nparts;
-    if (const WgPhPlan p = wgrad_ph_plan(B, H, W, C, K, PH, PW); p.ok) {
-        r = dtype == kF16 ? wgrad_ph_go<f16_t>(p, x, gy, ws, s) : wgrad_ph_go<bf16_t>(p, x, gy, ws, s);
-        nparts = p.parts();
-    } else {
-        const WgTzPlan q = wgrad_tz_plan(B, H, W, C, K, PH, PW);
-        if (!q.ok) return -1;
-        auto go = [&](auto t) {
-            using T = decltype(t);
-            return q.ncb == 8 ? launch_wgrad_tz<T, 8>(q, x, gy, ws, s) : launch_wgrad_tz<T, 5>(q, x, gy, ws, s);
-        };
-        r = dtype == kF16 ? go(f16_t{}) : go(bf16_t{});
-        nparts = B * q.g.nbands * q.g.ncolt;
-    }
-    return r != 0 ? r : reduce(ws, dw, nparts, K * K * C, dtype, s);
+    const WgPhPlan p = wgrad_ph_plan(B, H, W, C, K, PH, PW);
+    if (!p.ok) return -1;
+    const int r = dtype == kF16 ? wgrad_ph_go<f16_t>(p, x, gy, ws, s) : wgrad_ph_go<bf16_t>(p, x, gy, ws, s);
+    return r != 0 ? r : reduce(ws, dw, p.parts(), K * K * C, dtype, s);
 }
 
 // -1: not covered (the caller runs the two problems one by one).  Problem 0 is the wider one.
@@ -66,23 +56,11 @@ int dwconv_wgrad_tz_pair_launch(const void* x0, const void* gy0, void* dw0, void
                                 const void* gy1, void* dw1, void* ws1, int H1, int W1, int B, int C, int K, int PH, int PW,
                                 int dtype, hipStream_t s) {
     if (dtype == kF32 || !aligned({x0, gy0, ws0, x1, gy1, ws1})) return -1;
-    int r, n0, n1;
     const WgPhPlan p0 = wgrad_ph_plan(B, H0, W0, C, K, PH, PW), p1 = wgrad_ph_plan(B, H1, W1, C, K, PH, PW);
-    if (p0.ok && p1.ok) {
-        r = dtype == kF16 ? wgrad_ph_pair_go<f16_t>(p0, x0, gy0, ws0, p1, x1, gy1, ws1, s)
-                          : wgrad_ph_pair_go<bf16_t>(p0, x0, gy0, ws0, p1, x1, gy1, ws1, s);
-        n0 = p0.parts(), n1 = p1.parts();
-    } else {
-        const WgTzPlan q0 = wgrad_tz_plan(B, H0, W0, C, K, PH, PW), q1 = wgrad_tz_plan(B, H1, W1, C, K, PH, PW);
-        if (!q0.ok || !q1.ok || q0.ncb != 8) return -1;
-        auto go = [&](auto t) {
-            using T = decltype(t);
-            return q1.ncb == 8 ? launch_wgrad_tz_pair<T, 8, 8>(q0, x0, gy0, ws0, q1, x1, gy1, ws1, s)
-                               : launch_wgrad_tz_pair<T, 8, 5>(q0, x0, gy0, ws0, q1, x1, gy1, ws1, s);
-        };
-        r = dtype == kF16 ? go(f16_t{}) : go(bf16_t{});
-        n0 = B * q0.g.nbands * q0.g.ncolt, n1 = B * q1.g.nbands * q1.g.ncolt;
-    }
+    if (!p0.ok || !p1.ok) return -1;
+    const int r = dtype == kF16 ? wgrad_ph_pair_go<f16_t>(p0, x0, gy0, ws0, p1, x1, gy1, ws1, s)
+                                : wgrad_ph_pair_go<bf16_t>(p0, x0, gy0, ws0, p1, x1, gy1, ws1, s);
+    const int n0 = p0.parts(), n1 = p1.parts();
     if (r != 0) return r;
     if (int e = reduce(ws0, dw0, n0, K * K * C, dtype, s)) return e;
     return reduce(ws1, dw1, n1, K * K * C, dtype, s);

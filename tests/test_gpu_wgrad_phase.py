@@ -46,12 +46,16 @@ def test_even_filters(oracle, shape, k, dtype):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("shape,k", [((1, 8, 64, 16), 3), ((2, 9, 65, 24), 9), ((3, 57, 61, 8), 13), ((5, 16, 32, 40), 15),
                                      ((3, 7, 7, 16), 11), ((4, 33, 31, 16), 5), ((2, 15, 112, 24), 7), ((7, 24, 63, 16), 13),
-                                     ((1, 1, 1, 8), 15), ((9, 3, 33, 8), 1), ((40, 28, 28, 32), 13), ((2, 70, 20, 136), 9)])
+                                     ((1, 1, 1, 8), 15), ((9, 3, 33, 8), 1), ((40, 28, 28, 32), 13), ((2, 70, 20, 136), 9),
+                                     # one column and row more than an operand's 16
+                                     ((1, 8, 64, 16), 17), ((3, 57, 61, 8), 17), ((5, 16, 32, 40), 17), ((1, 1, 1, 8), 17),
+                                     ((40, 28, 28, 32), 17), ((2, 15, 112, 24), 17), ((3, 7, 7, 16), 17), ((2, 70, 20, 136), 17)])
 def test_tiles_and_runs(oracle, shape, k, dtype):
     _check(oracle, shape, k, (k // 2, k // 2), dtype, k + shape[1])
 
 
 @pytest.mark.parametrize("shape,k,pad", [((3, 20, 40, 16), 13, (0, 0)), ((2, 18, 34, 24), 9, (8, 8)), ((2, 17, 33, 8), 5, (7, 6)),
-                                         ((3, 16, 70, 16), 15, (14, 3)), ((2, 13, 13, 16), 11, (1, 10))])
+                                         ((3, 16, 70, 16), 15, (14, 3)), ((2, 13, 13, 16), 11, (1, 10)),
+                                         ((2, 18, 34, 16), 17, (16, 0)), ((3, 20, 40, 16), 17, (3, 16)), ((2, 17, 70, 24), 16, (0, 15))])
 def test_paddings_other_than_same(oracle, shape, k, pad):
     _check(oracle, shape, k, pad, torch.bfloat16, k + pad[0])
