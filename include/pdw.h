@@ -136,6 +136,14 @@ int pdw_dwconv_wgrad(const void *x, const void *gy, void *dw, void *workspace, s
                      int B, int H, int W, int C, int KH, int KW, int SH, int SW, int PH, int PW, int DH,
                      int DW, int dtype, void *stream);
 
+/* pdw_dwconv_dgrad and pdw_dwconv_wgrad of one convolution as one call (dwconv_triton.py:334-387): dx from gy and w, dw from x and gy,
+ * workspace as for pdw_dwconv_wgrad.  16-bit types with an odd square filter up to 17, stride 1 and padding K/2 run as one launch
+ * where that is estimated to end sooner, everything else as the two calls.  dx is bitwise that of pdw_dwconv_dgrad; dw is the same sum
+ * taken over other pieces of the images, so it can differ from pdw_dwconv_wgrad's in the last bit, and is the same from call to call. */
+int pdw_dwconv_bwd(const void *gy, const void *w, const void *x, void *dx, void *dw, void *workspace, size_t workspace_bytes,
+                   int B, int H, int W, int C, int KH, int KW, int SH, int SW, int PH, int PW, int DH, int DW, int dtype,
+                   void *stream);
+
 /* pdw_dwconv_wgrad for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc): same arguments and bitwise the same result, but the fp32 partial sums
  * go to a buffer of pdw_static_scratch_bytes() (32 MiB) that is part of the library's device image instead of a

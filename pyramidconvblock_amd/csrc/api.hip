@@ -230,6 +230,23 @@ int pdw_dwconv_wgrad(const void* x, const void* gy, void* dw, void* workspace, s
                                       (hipStream_t)stream);
 }
 
+int pdw_dwconv_bwd(const void* gy, const void* w, const void* x, void* dx, void* dw, void* workspace, size_t workspace_bytes, int B, int H,
+                   int W, int C, int KH, int KW, int SH, int SW, int PH, int PW, int DH, int DW, int dtype, void* stream) {
+    if (int e = check_conv("pdw_dwconv_bwd", gy, w, dx, B, H, W, C, KH, KW, SH, SW, PH, PW, DH, DW, dtype)) return e;
+    if (int e = check_conv("pdw_dwconv_bwd", x, gy, dw, B, H, W, C, KH, KW, SH, SW, PH, PW, DH, DW, dtype)) return e;
+    if (!dw) return set_error("pdw_dwconv_bwd: null dw"), 1;
+    const size_t need = pdw_dwconv_wgrad_workspace_bytes(B, H, W, C, KH, KW, SH, SW, PH, PW, DH, DW, dtype);
+    if (!workspace || workspace_bytes < need)
+        return set_error("pdw_dwconv_bwd: workspace of %zu bytes given, %zu needed", workspace_bytes, need), 1;
+    if (B > 0 && SH == 1 && SW == 1 && DH == 1 && DW == 1 && KH == KW && (KH & 1) && PH == KH / 2 && PW == PH) {
+        const int r = dwconv_bwd3_launch(gy, w, nullptr, dx, x, dw, workspace, nullptr, nullptr, nullptr, nullptr, B, H, W, 0, 0, C, KH,
+                                         dtype, (hipStream_t)stream);
+        if (r != -1) return r;
+    }
+    if (int e = pdw_dwconv_dgrad(gy, w, dx, B, H, W, C, KH, KW, SH, SW, PH, PW, DH, DW, dtype, stream)) return e;
+    return pdw_dwconv_wgrad(x, gy, dw, workspace, workspace_bytes, B, H, W, C, KH, KW, SH, SW, PH, PW, DH, DW, dtype, stream);
+}
+
 size_t pdw_static_scratch_bytes(void) { return kStaticScratchBytes; }
 
 int pdw_static_scratch_init(void) {

@@ -11,6 +11,7 @@
 #include "dwconv_tz.h"
 #include "dwconv_wgrad_ph.h"
 #include <algorithm>
+#include <array>
 #include <map>
 #include <tuple>
 #include <type_traits>
@@ -149,6 +150,64 @@ static Bwd3Plan bwd3_plan(int B, const TzGeom& gd, int npcd, const WgPhPlan& p0,
     return best;
 }
 
+// The same for the input gradient and the weight gradient of one convolution by itself (no second scale): the cuts that are
+// estimated to end first, of one round or several; n[0] = 0 where a launch each is estimated to take no longer.  Together they save a launch and
+// fill the rounds that 72 slices, say, leave open (2 x 216 workgroups, or 288 + 216 in two rounds); apart, each side has the chip and its
+// memory to itself and its steps are shorter ([64,56,56,128] filter 13 in one round 83.7 us, apart 70.1, [39,45,45,216] filter 17 117
+// and 87).  Prices fitted to both of 160 random shapes with cold buffers; with them 180 others
+// take 1.12 times less, the slowest 1.05 times more ([74,17,17,896] filter 9 76.8 -> 80.7).  us with the summation, apart and together:
+// [8,64,64,1152] filter 9 84 -> 70, [32,28,28,256] filter 13 33.8 -> 28.8, [2,20,20,64] filter 7 13.2 -> 8.6, [11,74,74,688] filter 9 137 -> 109.
+template <int K>
+static Bwd3Plan bwd2_plan(const TzGeom& gd, int npcd, const WgPhPlan& p0) {
+    static std::mutex mu;
+    static std::map<std::array<int, 4>, Bwd3Plan> cache;
+    const std::array<int, 4> key{gd.B, gd.OH, gd.OW, gd.C};
+    std::lock_guard<std::mutex> lock(mu);
+    if (auto it = cache.find(key); it != cache.end()) return it->second;
+    // us of a run's start and of its steps in a launch of its own, the input gradient's (filters 15 and 17: 8 channels) and the weight
+    // gradient's; their steps side by side, in one round and in several (which are full of either side most of the time); what an
+    // estimate of one round has to be ahead by (launch_makespan adds its own to several)
+    constexpr double kStartD = 5.5, kStepD = K <= 9 ? 1.25 : K <= 13 ? 1.4 : 1.2, kStartF = kWgPhStart, kStepF = K <= 9 ? 1.25 : K <= 15 ? 1.8 : 2.5,
+                     kLaunch = 2.8, kShareOne = K <= 5 ? 1.15 : K <= 9 ? 1.17 : 1.2, kShareMore = K <= 5 ? 1.15 : K <= 9 ? 1.1 : 1.2, kAhead = 1.04;
+    const int ni = 16 / npcd;
+    std::vector<LaunchCut> cuts[2];
+    TzGeom g = gd;
+    double apart = kLaunch + cdiv(p0.nblocks, 256) * (kStartF + kStepF * p0.g.passes);
+    if (tz_cut_alone(g, ni, K <= 5)) {
+        const double steps = tz_alone_cost(tz_blocks(g), tz_steps(g), K <= 5);
+        apart += K <= 5 ? kStepD * steps : cdiv(tz_blocks(g), 256) * kStartD + kStepD * (steps - cdiv(tz_blocks(g), 256) * 4.5);
+        const int runs = g.nruns;
+        int last = 0;
+        for (int e = 2; e <= 16; ++e) {
+            const int most = cdiv(cdiv(tz_rows(gd, ni), 8) * (gd.stack ? 1 : cdiv(gd.B, ni)), std::max(1, runs * e / 8));
+            if (most != last && tz_cut_steps(g, ni, most)) cuts[0].push_back({g.run, kStepD * tz_steps(g), tz_blocks(g)});
+            last = most;
+        }
+    }
+    WgPhPlan p = p0;
+    for (int e = 16; e >= 1; --e) {   // (no more runs than by itself: the workspace is sized for those)
+        if (!wgrad_ph_cut(p, std::max(1, p0.g.nchunks * e / 16)) || (!cuts[1].empty() && cuts[1].back().n == p.g.nchunks)) continue;
+        cuts[1].push_back({p.g.nchunks, kStepF * p.g.passes, p.nblocks});
+    }
+    Bwd3Plan best{{0, 1, 0}, "DF"};
+    for (const LaunchCut& dc : cuts[0])
+        for (const LaunchCut& fc : cuts[1]) {
+            const bool single = dc.count + fc.count <= 256;
+            const double share = single ? kShareOne : kShareMore;
+            const LaunchCut d{dc.n, kStartD + share * dc.cost, dc.count}, f{fc.n, kStartF + share * fc.cost, fc.count};
+            const LaunchCut* const pick[2] = {&d, &f};
+            const int ord[2] = {d.cost >= f.cost ? 0 : 1, d.cost >= f.cost ? 1 : 0};
+            const double t = (single ? kAhead : 1.0) * launch_makespan(pick, ord);
+            if (t >= apart) continue;
+            apart = t;
+            best.n[0] = d.n, best.n[1] = f.n;
+            best.order[0] = "DF"[ord[0]], best.order[1] = "DF"[ord[1]];
+        }
+    if (cache.size() >= kPlanCacheMax) cache.clear();
+    cache[key] = best;
+    return best;
+}
+
 template <typename T, int K, int CS, bool WIDE, int MODE>
 static void bwd3_go(const Bwd3Args& a, unsigned grid, size_t lds, hipStream_t s) {
     auto kern = dwconv_bwd3_k<T, K, CS, WIDE, MODE>;
@@ -159,16 +218,18 @@ static void bwd3_go(const Bwd3Args& a, unsigned grid, size_t lds, hipStream_t s)
 
 // -1: not covered (the caller makes the three launches).  16-bit types, C % 8 == 0, padding K / 2; the full scale
 // [B, H, W, C], the pooled one [B, h, w, C].  addp (optional, H = 2 h and W = 2 w): the pooled branch's gradient.
+// x1 = nullptr and h = 0: no pooled scale (a convolution by itself; -1 also where two launches take no longer).
 template <int K>
 static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* dx, const void* x0, void* dw0, void* ws0,
                        const void* x1, const void* gy1, void* dw1, void* ws1, int B, int H, int W, int h, int w, int C, int dtype,
                        hipStream_t s, int* plan_out, const MeanJob* mean) {
     constexpr int CS = (2 * 4 * TzShape<K, 16, 16>::NM + 2 * 4 * TzShape<K, 16, 16>::RING) <= 160 ? 16 : 8;
-    if (dtype == kF32 || C % 8 != 0 || B < 1 || H < 1 || W < 1 || h < 1 || w < 1) return -1;
+    const bool one = h == 0;
+    if (dtype == kF32 || C % 8 != 0 || B < 1 || H < 1 || W < 1 || (!one && (h < 1 || w < 1))) return -1;
     if (addp && (H != 2 * h || W != 2 * w)) return -1;
     const int P = K / 2;
     if (!plan_out)
-        for (const void* p : {gyf, w0, (const void*)dx, x0, (const void*)ws0, x1, gy1, (const void*)ws1})
+        for (const void* p : {gyf, w0, (const void*)dx, x0, (const void*)ws0, one ? x0 : x1, one ? gyf : gy1, (const void*)(one ? ws0 : ws1)})
             if (!p || (reinterpret_cast<uintptr_t>(p) & 15)) return -1;
     if (reinterpret_cast<uintptr_t>(addp) & 15) return -1;
     Bwd3Args a{};
@@ -176,29 +237,31 @@ static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* 
     if (!(a.npcd == 16 ? tz_make_geom<K, 16, CS>(a.gd, true, B, H, W, C, K - 1 - P, K - 1 - P, true, nullptr)
                        : tz_make_geom<K, 8, CS>(a.gd, true, B, H, W, C, K - 1 - P, K - 1 - P, true, nullptr)))
         return -1;
-    WgPhPlan p0 = wgrad_ph_plan(B, H, W, C, K, P, P), p1 = wgrad_ph_plan(B, h, w, C, K, P, P);
-    if (!p0.ok || !p1.ok) return -1;
+    WgPhPlan p0 = wgrad_ph_plan(B, H, W, C, K, P, P), p1;
+    if (!one) p1 = wgrad_ph_plan(B, h, w, C, K, P, P);
+    if (!p0.ok || (!one && !p1.ok)) return -1;
     MeanJob job{};
     if (mean) job = *mean, job.shared = mean_shared(job.B, job.D);
     const int nmean = mean ? mean_bwd_workgroups(job) : 0;
-    Bwd3Plan plan = bwd3_plan<K>(B, a.gd, a.npcd, p0, p1, nmean);
+    Bwd3Plan plan = one ? bwd2_plan<K>(a.gd, a.npcd, p0) : bwd3_plan<K>(B, a.gd, a.npcd, p0, p1, nmean);
     if (const char* e = tune_env("PDW_BWD3_BANDS")) {   // e.g. "64,31,8,DHF": cuts of D, F, H and the grid order
         if (sscanf(e, "%d,%d,%d,%3s", &plan.n[0], &plan.n[1], &plan.n[2], plan.order) != 4) return -1;
     }
     if (tune_env("PDW_BWD3_PRINT"))
         fprintf(stderr, "bwd3 plan B=%d H=%d W=%d C=%d K=%d: cuts D %d F %d H %d order %s\n", B, H, W, C, K, plan.n[0],
                 plan.n[1], plan.n[2], plan.order);
-    if (plan.n[0] < 1 || plan.n[1] < 1 || plan.n[2] < 1) return -1;
+    if (plan.n[0] < 1 || plan.n[1] < 1 || (!one && plan.n[2] < 1)) return -1;
     if (!tz_cut(a.gd, 16 / a.npcd, plan.n[0])) return -1;
     const long long nd = tz_blocks(a.gd);
-    int parts[2], per_image[2];   // partials of the weight gradients, pieces of an image
-    for (int i = 0; i < 2; ++i) {
+    int parts[2] = {}, per_image[2] = {};   // partials of the weight gradients, pieces of an image
+    for (int i = 0; i < (one ? 1 : 2); ++i) {
         WgPhPlan& p = i == 0 ? p0 : p1;
         if (!wgrad_ph_cut(p, plan.n[1 + i])) return -1;
         parts[i] = p.parts(), per_image[i] = cdiv(p.g.nchunks, cdiv(B, p.g.ni));
         a.p[i].g = p.g, a.p[i].n = (int)p.nblocks;
     }
-    if (nd + p0.nblocks + p1.nblocks + nmean > 0x7fffffffLL) return -1;
+    const long long grid_all = nd + p0.nblocks + (one ? 0 : p1.nblocks) + nmean;
+    if (grid_all > 0x7fffffffLL) return -1;
     if (plan_out) {
         plan_out[0] = cdiv(a.gd.nruns, cdiv(B, 16 / a.npcd)), plan_out[1] = per_image[0], plan_out[2] = per_image[1];
         return 0;
@@ -212,7 +275,7 @@ static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* 
         // order of the three problems in the grid: a permutation of D (input gradient), H (half scale), F (full scale)
         const char* ord = plan.order;
         int at = 0;
-        for (int i = 0; i < 3; ++i) {
+        for (int i = 0; i < 3 && ord[i]; ++i) {
             if (ord[i] == 'D') a.sd = at, at += a.nd;
             if (ord[i] == 'H') a.p[1].start = at, at += a.p[1].n;
             if (ord[i] == 'F') a.p[0].start = at, at += a.p[0].n;
@@ -221,7 +284,7 @@ static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* 
     size_t lds = a.npcd == 16 ? TzShape<K, 16, CS>::lds_bytes : TzShape<K, 8, CS>::lds_bytes;
     lds = std::max(lds, WgPhShape<wgrad_ph_ncopy(K), wgrad_ph_gr(K)>::lds_bytes);
     if (nmean) lds = std::max(lds, mean_lds(job.D, 512, job.shared ? kMeanImages : 1));
-    const unsigned grid = (unsigned)(nd + p0.nblocks + p1.nblocks + nmean);
+    const unsigned grid = (unsigned)grid_all;
     auto go = [&](auto t) {
         using T = decltype(t);
         if (!addp) bwd3_go<T, K, CS, false, 0>(a, grid, lds, s);
@@ -234,10 +297,10 @@ static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* 
     const int n0 = parts[0], n1 = parts[1];
     if (dtype == kF16) {
         if (int e = wgrad_reduce_launch<f16_t>((const float*)ws0, dw0, n0, K * K * C, s)) return e;
-        return wgrad_reduce_launch<f16_t>((const float*)ws1, dw1, n1, K * K * C, s);
+        return one ? 0 : wgrad_reduce_launch<f16_t>((const float*)ws1, dw1, n1, K * K * C, s);
     }
     if (int e = wgrad_reduce_launch<bf16_t>((const float*)ws0, dw0, n0, K * K * C, s)) return e;
-    return wgrad_reduce_launch<bf16_t>((const float*)ws1, dw1, n1, K * K * C, s);
+    return one ? 0 : wgrad_reduce_launch<bf16_t>((const float*)ws1, dw1, n1, K * K * C, s);
 }
 
 }  // namespace pdw

@@ -170,7 +170,8 @@ int dense_bwd_pair_launch(const void* gy, const void* w, const void* xin, void* 
 
 // dwconv_bwd3.hip: input gradient (+ pooled branch's where the pool halved the extents, else addp = nullptr) of the full scale
 // and the weight gradients of both scales of a two-scale block in one launch, with the backward of its mean branch
-// (optional); -1 = not covered
+// (optional); -1 = not covered.  x1 = nullptr with h = 0: both gradients of a convolution by itself, -1 also where a launch each
+// takes no longer
 bool dwconv_bwd3_covers(int B, int W, int C);
 int dwconv_bwd3_launch(const void* gyf, const void* w0, const void* addp, void* dx, const void* x0, void* dw0, void* ws0,
                        const void* x1, const void* gy1, void* dw1, void* ws1, int B, int H, int W, int h, int w, int C, int K,

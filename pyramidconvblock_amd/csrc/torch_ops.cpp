@@ -225,25 +225,24 @@ struct ConvNode : public torch::autograd::Node {
         void* const stream = stream_of(xd);
         const auto xs = xd.sizes(), ws = wd.sizes();
         const bool empty = xd.numel() == 0 || gy.numel() == 0;
-        if (task_should_compute_output(0)) {
-            Tensor dx = at::empty(xs, xd.options());
-            if (empty)
-                dx.zero_();
-            else
-                check(pdw_dwconv_dgrad(ptr(gy), ptr(wd), ptr(dx), PDW_CONV(xs, ws, g), dt, stream), "pdw_dwconv_dgrad");
-            out[0] = dx.to(x_type);
+        const bool want_x = task_should_compute_output(0), want_w = task_should_compute_output(1);
+        Tensor dx, dw, work;
+        if (want_x) dx = at::empty(xs, xd.options());
+        if (want_w) dw = at::empty(ws, wd.options());
+        if (want_w && !empty) work = bytes(pdw_dwconv_wgrad_workspace_bytes(PDW_CONV(xs, ws, g), dt) + 4, xd);
+        if (empty) {
+            if (want_x) dx.zero_();
+            if (want_w) dw.zero_();
+        } else if (want_x && want_w) {
+            check(pdw_dwconv_bwd(ptr(gy), ptr(wd), ptr(xd), ptr(dx), ptr(dw), ptr(work), work.numel(), PDW_CONV(xs, ws, g), dt, stream),
+                  "pdw_dwconv_bwd");
+        } else if (want_x) {
+            check(pdw_dwconv_dgrad(ptr(gy), ptr(wd), ptr(dx), PDW_CONV(xs, ws, g), dt, stream), "pdw_dwconv_dgrad");
+        } else if (want_w) {
+            check(pdw_dwconv_wgrad(ptr(xd), ptr(gy), ptr(dw), ptr(work), work.numel(), PDW_CONV(xs, ws, g), dt, stream), "pdw_dwconv_wgrad");
         }
-        if (task_should_compute_output(1)) {
-            Tensor dw = at::empty(ws, wd.options());
-            if (empty) {
-                dw.zero_();
-            } else {
-                const Tensor work = bytes(pdw_dwconv_wgrad_workspace_bytes(PDW_CONV(xs, ws, g), dt) + 4, xd);
-                check(pdw_dwconv_wgrad(ptr(xd), ptr(gy), ptr(dw), ptr(work), work.numel(), PDW_CONV(xs, ws, g), dt, stream),
-                      "pdw_dwconv_wgrad");
-            }
-            out[1] = dw;
-        }
+        if (want_x) out[0] = dx.to(x_type);
+        if (want_w) out[1] = dw;
         return out;
     }
 };
