@@ -7,7 +7,8 @@
 // as it lies and read with ds_read_b64_tr_b16, as in dense_wide.hip.
 //
 // A value without such parts (infinite, NaN, or beyond 2^81) makes its workgroup's results again by plain multiply-adds, so that
-// they are what fp32 arithmetic gives.  So do values that a lane holds of one stored row (TR: of four results) and that are all below
+// they are what fp32 arithmetic gives.  So does a result that is not finite: where x1 y1 overflows, x2 y1 may do so the other way, and
+// an infinity would come out as NaN.  So do values that a lane holds of one stored row (TR: of four results) and that are all below
 // 2^-100 and not all zero: the matrix cores take a bf16 value below 2^-126 as zero, which beside a value from 2^-100 on is at
 // most 2^-26 of it and less than fp32's smallest normal value, and alone would be what the results consist of.
 #pragma once
@@ -212,11 +213,21 @@ __device__ __forceinline__ void wide_split_body(const Args& g, int blk, int nblk
             ((float*)g.y)[m * g.N + n] = s + add;
         }
     };
+    float finite = 0.f;   // (stays 0 while all results are)
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                if constexpr (PART) acc[i][j][r] += total[i][j][r];
+                finite = fmaf(acc[i][j][r], 0.f, finite);
+            }
     volatile uint32_t* const failed = reinterpret_cast<uint32_t*>(dsm);
     __syncthreads();
     if (tid == 0) *failed = 0;
     __syncthreads();
-    if (split_failed(seen) || OpA::tiny(topa) || OpB::tiny(topb)) *failed = 1;
+    if (split_failed(seen) || !(finite == 0.f) || OpA::tiny(topa) || OpB::tiny(topb)) *failed = 1;
     __syncthreads();
     if (*failed != 0) {   // (uniform)
         for (int r = tid; r < BM * BN; r += NT) {
@@ -232,12 +243,6 @@ __device__ __forceinline__ void wide_split_body(const Args& g, int blk, int nblk
         return;
     }
     if constexpr (PART) {
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[i][j][r] += total[i][j][r];
         float* const out = (float*)g.y + (size_t)sp * g.M * g.N;
 #pragma unroll
         for (int i = 0; i < FM; ++i) {

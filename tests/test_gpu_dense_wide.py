@@ -118,6 +118,26 @@ def test_fp32_split_operands_and_values_that_are_not_finite():
     assert float((y[:, keep] - clean[:, keep]).norm() / clean.norm()) < 1e-6
 
 
+def test_fp32_split_operands_whose_products_overflow():
+    """Infinities as fp32 products give them, not the NaN of parts that overflow in opposite directions."""
+    from pyramidconvblock_amd import ops
+
+    gen = torch.Generator().manual_seed(3)
+    x, w, g = randn(gen, 8000, 256), randn(gen, 256, 256), randn(gen, 8000, 256)
+    clean = ops.dense_forward(x.cuda(), w.cuda()).cpu()
+    xp, wp = x.clone(), w.clone()
+    xp[5], wp[7] = (x[5].abs() + 1) * 1e23, (w[7].abs() + 1) * 1e23
+    y = ops.dense_forward(xp.cuda(), wp.cuda()).cpu()
+    assert y[5, 7] == float("inf")
+    assert torch.isfinite(y[5, :7]).all() and torch.isfinite(y[:5, 7]).all()
+    y[5], y[:, 7] = clean[5], clean[:, 7]
+    assert float((y - clean).norm() / clean.norm()) < 1e-6
+    xc, gc = x.clone(), g.clone()
+    xc[:, 9], gc[:, 11] = (x[:, 9].abs() + 1) * 1e23, -(g[:, 11].abs() + 1) * 1e23
+    dw = ops.dense_wgrad(gc.cuda(), xc.cuda()).cpu()
+    assert dw[11, 9] == -float("inf") and int(torch.isfinite(dw).logical_not().sum()) == 1
+
+
 @pytest.mark.parametrize("scale", [1e-29, 1e-34, 1e-37])
 def test_fp32_split_operands_near_the_smallest_values(scale):
     """Values whose parts bf16 cannot hold: no less precise than others."""
