@@ -165,17 +165,13 @@ struct Operand {
 template <typename T, int R, bool TR>
 struct HandFragments {
     typedef Operand<T, R, TR> Op;
-    static constexpr int ES = (int)sizeof(T);
-    static constexpr int READS = TR ? (ES == 4 ? 4 : 2) : 1;   // LDS instructions of a fragment
+    static_assert(sizeof(T) == 2, "16-bit values");
+    static constexpr int READS = TR ? 2 : 1;   // LDS instructions of a fragment
     // per lane and in a stage, but for constants: (TR) where fragment t's values of kk = 0 lie, else those of kk = n and t = 0
-    static constexpr int ADDRESSES = TR ? R / 32 : 4;
     static __device__ __forceinline__ uint32_t at(int n, int lane) {
         if constexpr (!TR) {
             const int row = lane & 31;
             return (uint32_t)(row * kRowBytes + Op::swz(row, 2 * n + (lane >> 5)) * 16);
-        } else if constexpr (ES == 4) {
-            const int col = 32 * n + (lane & 31), row = 4 * (lane >> 5);
-            return (uint32_t)(row * (R * 4) + Op::swz(row, col >> 2) * 16 + (col & 3) * 4);
         } else {
             const int g = lane >> 4, i = lane & 15, col = 32 * n + 16 * (g & 1) + 4 * (i & 3), row = 8 * (g >> 1) + (i >> 2);
             return (uint32_t)(row * (R * 2) + Op::swz(row, col >> 3) * 16 + (col & 7) * 2);
@@ -187,14 +183,6 @@ struct HandFragments {
             v8s f;
             asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(f) : "v"(p), "n"(TILE * 32 * kRowBytes));
             return f;
-        } else if constexpr (ES == 4) {
-            float e0, e1, e2, e3;
-            asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(e0) : "v"(p), "n"(8 * KK * R * 4));
-            asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(e1) : "v"(p), "n"((8 * KK + 1) * R * 4));
-            asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(e2) : "v"(p), "n"((8 * KK + 2) * R * 4));
-            asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(e3) : "v"(p), "n"((8 * KK + 3) * R * 4));
-            const v4f v = {e0, e1, e2, e3};
-            return __builtin_bit_cast(v8s, v);
         } else {
             v4s h0, h1;
             asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(h0) : "v"(p), "n"(16 * KK * R * 2));
@@ -515,7 +503,8 @@ constexpr size_t wide_lds() {
 
 // Launches that kDeep stages in LDS are for: 16-bit ones whose workgroups are all on the chip at once with them, and whose sums have
 // `least` stages or more (us, two stages -> four: [2128,920] -> 464, 136 workgroups of 15 stages, 12.0 -> 9.65, [1568,1024] -> 512 11.8 -> 9.2,
-// [3136,768] -> 384 10.1 -> 8.2; of five stages or fewer the same or up to 0.4 more, and in fp32, where the products take longer, 40.5 -> 41.2).
+// [3136,768] -> 384 10.1 -> 8.2; of five stages or fewer the same or up to 0.4 more.  fp32's products take
+// longer than a stage's trip: [10431,200] -> 100 11.7 -> 12.5, [12544,256] -> 128 12.7 -> 13.2, [2048,96] -> 48 4.6 -> 4.9).
 constexpr int kDeep = 4;
 template <typename T>
 constexpr bool goes_deep(long long n, size_t lds, long long inner, int least) {
