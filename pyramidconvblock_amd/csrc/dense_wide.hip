@@ -614,7 +614,9 @@ static bool wide_rows_plan(WideArgs& g, int& bm, int& bn, const void* x, const v
         // it matters), but not for many rows of a short sum, which is a stream ([50000,16] -> 32: 6.4 here, 5.6 in dense_any.hip)
         if (K < 32 && N >= 16384 && NO <= 256) return false;
         bm = bn = 64;
-        if (wide_split(N, K, NO)) {
+        // not where those of 64 are one to a compute unit, which has the matrix pipe to itself (us, these and split: [1922,856] -> 428, 217 tiles,
+        // 21.5 and 25.8, [3000,640] -> 320, 235 tiles, 15.6 and 18.3; [2400,856] -> 428, 266 tiles, 32.2 and 24.2)
+        if (wide_split(N, K, NO) && (long long)cdiv(N, 64) * cdiv(NO, 64) > 256) {
             // 128 x 128 (one to a compute unit) or 128 x 64 (two): start-ups and stages of 32, us
             const long long narrow = (long long)cdiv(N, 128) * cdiv(NO, 64), broad = (long long)cdiv(N, 128) * cdiv(NO, 128);
             const double st = cdiv(K, kSplitBK), fill = narrow <= 512 ? 1.0 : narrow / 512.0;

@@ -63,10 +63,10 @@ def test_dense_wide_columns_of_192(dtype, K, NO):
 
 
 @pytest.mark.parametrize("K,NO,N,P", [(196, 196, 13100, 13100), (516, 200, 7001, 700), (200, 516, 7001, 7001), (1028, 260, 2000, 63), (704, 352, 10816, 10816),
-                                      (192, 192, 13564, 6782), (260, 1028, 2000, 2000)])
+                                      (192, 192, 13564, 6782), (260, 1028, 2000, 2000), (768, 512, 2048, 2048), (768, 512, 2049, 2049)])
 def test_fp32_layers_on_split_operands(K, NO, N, P):
     """Large fp32 products (csrc/dense_split.h): both tiles, remainders of 4 results and inner values, an odd number of stages, ranges of
-    rows; no further from float64 than fp32 products and sums of that length are (their partial sums random: sqrt(K) roundings)."""
+    rows, and either side of 256 fp32 tiles; no further from float64 than fp32 products and sums of that length are (their partial sums random: sqrt(K) roundings)."""
     from pyramidconvblock_amd import ops
 
     _layers(torch.float32, K, NO, N, P)
