@@ -343,7 +343,9 @@ __device__ __forceinline__ void wide_gemm_body(const WideArgs& g, int blk, int n
             });
             slot = next;
         }
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        // (the last turn has read fragments that nothing uses: their registers are given away only behind this wait)
+        wait_fragments<0>(fa[0], fb[0]);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     if constexpr (PART && sizeof(T) == 4) {   // (tiles of 64, four to a compute unit: nothing to win by the other way)
         float* const out = (float*)g.y + (size_t)sp * g.M * g.N;
