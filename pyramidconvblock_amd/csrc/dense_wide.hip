@@ -16,8 +16,7 @@
 // (48), its weight gradient 32 + its share of the summation (a batched product over 128 slabs and their sum: 160 + 150).
 // fp32 (v_mfma_f32_32x32x2_f32, a sixteenth of the rate, so that the LDS and its reads down a column value by value are no
 // matter), us, dense_any.hip -> here: [100352,128] -> 64 28.7 -> 22.8, its input gradient 32.3 -> 25.6 (77 MB, 10.5 us of matrix
-// pipe); [10431,200] -> 100 16.0 -> 11.4; [20000,256] -> 128 26.5 -> 18.7; [2048,64] -> 32 5.1 -> 3.8.  Large fp32 products, which that
-// rate bounds, run on operands split into three bf16 values each (dense_split.h).
+// pipe); [10431,200] -> 100 16.0 -> 11.4; [20000,256] -> 128 26.5 -> 18.7; [2048,64] -> 32 5.1 -> 3.8.
 // Out-of-range rows, columns and the inner tail read as zero through the buffer descriptors; nothing is branched around.
 #include <stdint.h>
 
@@ -27,7 +26,6 @@
 
 #include "common.h"
 #include "dense_any_wgrad.h"
-#include "dense_split.h"
 #include "kernels.h"
 #include "reduce_parts.h"
 #include "tile_common.h"
@@ -428,57 +426,6 @@ __global__ __launch_bounds__(256, (STAGES == 2 ? kWideOccupancy<T, BM, BN> : 1))
     wide_gemm_body<T, BM, BN, TA, TB, PART, STAGES>(g, blockIdx.x, gridDim.x);
 }
 
-// fp32 tiles of dense_split.h: 128 x 128 and 128 x 64 results by eight wavefronts, 64 x 64 by four.
-template <int BM, int BN>
-struct SplitTile {
-    static constexpr int WM = BM == 128 && BN == 64 ? 4 : 2, WN = BN == 128 ? 4 : 2, NT = 64 * WM * WN;
-    static constexpr int WAVES = BM * BN == 128 * 128 ? 2 : BM * BN == 128 * 64 ? 4 : 3;   // of a SIMD, by the LDS
-};
-
-template <int BM, int BN, bool TA, bool TB, bool PART>
-__device__ __forceinline__ void split_body(const WideArgs& g, int blk, int nblk) {
-    wide_split_body<BM, BN, SplitTile<BM, BN>::WM, SplitTile<BM, BN>::WN, TA, TB, PART>(g, blk, nblk);
-}
-
-template <int BM, int BN, bool TA, bool TB, bool PART>
-__global__ __launch_bounds__((SplitTile<BM, BN>::NT), (SplitTile<BM, BN>::WAVES)) void wide_split_k(WideArgs g) {
-    split_body<BM, BN, TA, TB, PART>(g, blockIdx.x, gridDim.x);
-}
-
-// As wide_pair_k, below: the weight gradient's nw workgroups first.
-template <int BN>
-__global__ __launch_bounds__(512, 2) void wide_split_pair_k(WideArgs rows, WideArgs wgrad, int nw) {
-    const int blk = blockIdx.x;
-    if (blk < nw) split_body<128, 128, true, true, true>(wgrad, blk, nw);
-    else split_body<128, BN, false, true, false>(rows, blk - nw, gridDim.x - nw);
-}
-
-template <int BM, int BN, bool TA, bool TB, bool PART>
-int split_go(const WideArgs& g, hipStream_t s) {
-    constexpr size_t lds = split_lds<BM, BN, PART>();
-    if constexpr (lds > 64 * 1024) {
-        static std::once_flag once;
-        std::call_once(once, [] {
-            (void)hipFuncSetAttribute((const void*)wide_split_k<BM, BN, TA, TB, PART>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        });
-    }
-    hipLaunchKernelGGL((wide_split_k<BM, BN, TA, TB, PART>), dim3((unsigned)(g.mt * g.nt * g.splits)), dim3(SplitTile<BM, BN>::NT), lds, s, g);
-    return check_launch("wide_split");
-}
-
-template <int BN>
-int split_pair_go(const WideArgs& rows, const WideArgs& wgrad, int nw, hipStream_t s) {
-    constexpr size_t lds = std::max(split_lds<128, 128, true>(), split_lds<128, BN, false>());
-    const long long n = (long long)nw + (long long)rows.mt * rows.nt;
-    if (n > 0x7fffffffLL) return -1;
-    static std::once_flag once;
-    std::call_once(once, [] {
-        (void)hipFuncSetAttribute((const void*)wide_split_pair_k<BN>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    });
-    hipLaunchKernelGGL(wide_split_pair_k<BN>, dim3((unsigned)n), dim3(512), lds, s, rows, wgrad, nw);
-    return check_launch("wide_split_pair");
-}
-
 // Both products that read the gradient of a layer's output, as one launch: the weight gradient's nw workgroups (tiles of WM x WN
 // of this file; WM = 0: the kernel without LDS, dense_any_wgrad.h), which are the longer ones, then the input gradient's.  A
 // launch of its own leaves part of the chip idle in its last round and pays the ramp; together they are dealt as one.
@@ -547,13 +494,6 @@ int wide_go(const WideArgs& g, hipStream_t s) {
     return check_launch("wide_gemm");
 }
 
-// Whether fp32 products over N rows, M and NO wide, run on split operands (dense_split.h): where the matrix pipe is what bounds
-// them.  us a product: [10816,704] -> 352 54.7 -> 38.2, its input gradient 53.3 -> 41.0, weight gradient 62.0 -> 43.6; [2002,1032] -> 516 40.6 ->
-// 30.4, 32.4 -> 26.2, 40.5 -> 28.3; [40000,400] -> 200 80 -> 65, 76 -> 66, 90 -> 63.  Smaller ones are chains of stages, which take longer
-// here ([1000,512] -> 256 12.5 -> 15), narrower ones bound by memory; and the chip's clock drops under 16-bit products (1.9 GHz for 2.3),
-// which the kernels after them feel: [25600,288] -> 144 36.7 -> 30.8 by itself, and its block's step 324 -> 333.
-bool wide_split(long long N, int M, int NO) { return std::min(M, NO) >= 192 && N * M * NO >= 500000000LL; }
-
 // Tiles and row ranges of the weight gradient: tiles of 64 where a width is no more than that, and the number of ranges that is
 // estimated to end first: a compute unit's stages (0.6 us one of 128 x 128 results, whether it has one workgroup or two in turn), and
 // the partials, written and read once more in fp32.  (With no more partials than are the operands' traffic, 512 workgroups at most,
@@ -566,18 +506,30 @@ struct WgradPlan {
 };
 WgradPlan wgrad_make_plan(long long N, int M, int NO, int es) {
     WgradPlan p{M <= 64 ? 64 : 128, NO <= 64 ? 64 : 128, 0, 0, 0, 0};
-    const int bk = es == 4 ? 32 : kRowBytes / es;
-    if (es == 4) p.bm = p.bn = wide_split(N, M, NO) ? 128 : 64;
-    // us: a stage of a tile, a range's partials
-    const double stage = es == 2 ? 0.6 / (128 * 128) * p.bm * p.bn : p.bm == 128 ? 1.4 : 0.5, partial = 8.0 * M * NO / (es == 4 ? 2.0e6 : 3.5e6);
-    const double alone = es == 4 && p.bm == 64 ? 1.3 : 1.0;   // (of one workgroup a compute unit)
-    p.mt = cdiv(M, p.bm), p.nt = cdiv(NO, p.bn);
-    const long long tiles = (long long)p.mt * p.nt, ranges = std::min(N / (2 * bk), std::max(1024 / tiles, 1LL));
-    long long s = 1;
-    double least = 0;
-    for (long long n = 1; n <= ranges || n == 1; n += n < 16 ? 1 : n / 8) {
-        const double c = (double)cdiv(tiles * n, 256) * (tiles * n <= 256 ? alone : 1.0) * cdiv(cdiv(N, n), bk) * stage + partial * n;
-        if (n == 1 || c < least) least = c, s = n;
+    const int bk = kRowBytes / es;
+    const double stage = es == 4 ? 0.5 / (64 * 64) : 0.6 / (128 * 128), partial = 8.0 * M * NO / 3.5e6;   // us: a result's stage, a range's partials
+    const double alone = es == 4 ? 1.3 : 1.0;   // (fp32: of one workgroup a compute unit)
+    double least;
+    auto cut = [&] {
+        p.mt = cdiv(M, p.bm), p.nt = cdiv(NO, p.bn);
+        const long long tiles = (long long)p.mt * p.nt, most = std::min(N / (2 * bk), std::max(1024 / tiles, 1LL));
+        long long best = 1;
+        for (long long s = 1; s <= most || s == 1; s += s < 16 ? 1 : s / 8) {
+            const long long inner = cdiv(cdiv(N, s), bk);
+            const double c = (double)cdiv(tiles * s, 256) * (tiles * s <= 256 ? alone : 1.0) * inner * p.bm * p.bn * stage + partial * s;
+            if (s == 1 || c < least) least = c, best = s;
+        }
+        return best;
+    };
+    long long s = cut();
+    // fp32, bound by the matrix pipe and not by what the tiles read: smaller ones (which the shared launch takes) unless these are
+    // clearly faster
+    if (es == 4 && (p.bm > 64 || p.bn > 64)) {
+        const WgradPlan large = p;
+        const double before = least;
+        const long long was = s;
+        p.bm = p.bn = 64, s = cut();
+        if (least > 1.15 * before) p = large, s = was;
     }
     // no range longer than its 32-bit offsets reach (operands of more than 2 GiB, widths that alone fill the chip)
     const long long most = 0x7fffffffLL / ((long long)(M > NO ? M : NO) * es) / 64 * 64;
@@ -616,15 +568,6 @@ static bool wide_rows_plan(WideArgs& g, int& bm, int& bn, const void* x, const v
         // it matters), but not for many rows of a short sum, which is a stream ([50000,16] -> 32: 6.4 here, 5.6 in dense_any.hip)
         if (K < 32 && N >= 16384 && NO <= 256) return false;
         bm = bn = 64;
-        // not where those of 64 are one to a compute unit, which has the matrix pipe to itself (us, these and split: [1922,856] -> 428, 217 tiles,
-        // 21.5 and 25.8, [3000,640] -> 320, 235 tiles, 15.6 and 18.3; [2400,856] -> 428, 266 tiles, 32.2 and 24.2)
-        if (wide_split(N, K, NO) && (long long)cdiv(N, 64) * cdiv(NO, 64) > 256) {
-            // 128 x 128 (one to a compute unit) or 128 x 64 (two): start-ups and stages of 32, us
-            const long long narrow = (long long)cdiv(N, 128) * cdiv(NO, 64), broad = (long long)cdiv(N, 128) * cdiv(NO, 128);
-            const double st = cdiv(K, kSplitBK), fill = narrow <= 512 ? 1.0 : narrow / 512.0;
-            bm = 128;
-            if (cdiv(broad, 256) * (3.5 + 1.2 * st) < (narrow <= 256 ? 3.5 + 0.72 * st : fill * (3.5 + 1.37 * st))) bn = 128;
-        }
     } else {
         // tiles of 64 rows where 128-row tiles would leave compute units without work
         bm = (long long)cdiv(N, 128) * cdiv(NO, 128) < 256 ? 64 : 128, bn = NO <= 64 ? 64 : 128;
@@ -651,12 +594,7 @@ int dense_wide_rows_launch(const void* x, const void* w, int w_kmajor, const voi
 #define PDW_WIDE(BM, BN) (dtype == kF16 ? PDW_WIDE_T(f16_t, BM, BN) : PDW_WIDE_T(bf16_t, BM, BN))
 #define PDW_WIDE2(BM, BN) (dtype == kF16 ? PDW_WIDE2_T(f16_t, BM, BN) : PDW_WIDE2_T(bf16_t, BM, BN))   /* (tiles of launches that fill the chip) */
 #define PDW_WIDE2_T(T, BM, BN) (w_kmajor ? wide_go<T, BM, BN, false, true, false, 2>(g, s) : wide_go<T, BM, BN, false, false, false, 2>(g, s))
-    if (dtype == kF32) {
-#define PDW_SPLIT(BM, BN) (w_kmajor ? split_go<BM, BN, false, true, false>(g, s) : split_go<BM, BN, false, false, false>(g, s))
-        if (bm == 128) return bn == 64 ? PDW_SPLIT(128, 64) : PDW_SPLIT(128, 128);
-#undef PDW_SPLIT
-        return PDW_WIDE2_T(float, 64, 64);
-    }
+    if (dtype == kF32) return PDW_WIDE2_T(float, 64, 64);
     if (bn == 192) return PDW_WIDE2(128, 192);
     if (bm == 64) return bn == 64 ? PDW_WIDE(64, 64) : PDW_WIDE(64, 128);
     return bn == 64 ? PDW_WIDE(128, 64) : PDW_WIDE2(128, 128);
@@ -681,10 +619,12 @@ int dense_wide_wgrad_launch(const void* a, const void* b, void* dw, void* ws, lo
     const WgradPlan p = wgrad_plan(N, M, NO, es);
     if (p.kper * (M > NO ? M : NO) * es > 0x7fffffffLL) return -1;
     WideArgs g{a, b, nullptr, nullptr, ws, M, N, NO, M, NO, 1, p.mt, p.nt, p.splits, p.kper};
-#define PDW_WIDE_W(BM, BN) (dtype == kF16 ? wide_go<f16_t, BM, BN, true, true, true>(g, s) : wide_go<bf16_t, BM, BN, true, true, true>(g, s))
-    const int e = dtype == kF32 ? (p.bm == 64 ? wide_go<float, 64, 64, true, true, true, 2>(g, s) : split_go<128, 128, true, true, true>(g, s))
-                  : p.bm == 64  ? (p.bn == 64 ? PDW_WIDE_W(64, 64) : PDW_WIDE_W(64, 128))
-                                : (p.bn == 64 ? PDW_WIDE_W(128, 64) : PDW_WIDE_W(128, 128));
+#define PDW_WIDE_W(BM, BN)                                                 \
+    (dtype == kF32   ? wide_go<float, BM, BN, true, true, true, 2>(g, s)   \
+     : dtype == kF16 ? wide_go<f16_t, BM, BN, true, true, true>(g, s)      \
+                     : wide_go<bf16_t, BM, BN, true, true, true>(g, s))
+    const int e = p.bm == 64 ? (p.bn == 64 ? PDW_WIDE_W(64, 64) : PDW_WIDE_W(64, 128))
+                             : (p.bn == 64 ? PDW_WIDE_W(128, 64) : PDW_WIDE_W(128, 128));
 #undef PDW_WIDE_W
     if (e) return e;
     if (dtype == kF32) return wgrad_reduce_launch<float>((const float*)ws, dw, p.splits, M * NO, s);
@@ -715,12 +655,8 @@ int dense_wide_bwd_pair_launch(const void* gy, const void* w, const void* b, voi
     }
     int e = -1;
     if (es == 4) {
-        // (both products on one kind of tile)
-        bm = !small && p.bm == 128 ? 128 : 64, bn = bm == 128 && (long long)cdiv(N, 128) * cdiv(NO, 128) >= 200 ? 128 : 64;
-        rows.mt = cdiv(N, bm), rows.nt = cdiv(NO, bn);
         if (small) e = pair_go<float, 64, 64, 0, 0, 2>(rows, wg, any, nw, s);
-        else if (bm == 64) e = pair_go<float, 64, 64, 64, 64, 2>(rows, wg, any, nw, s);
-        else e = bn == 128 ? split_pair_go<128>(rows, wg, nw, s) : split_pair_go<64>(rows, wg, nw, s);
+        else if (p.bm == 64 && p.bn == 64) e = pair_go<float, 64, 64, 64, 64, 2>(rows, wg, any, nw, s);
     } else if (p.bm == 128 && p.bn == 128) {
         auto go = [&](auto t) {
             using T = decltype(t);

@@ -64,9 +64,9 @@ def test_dense_wide_columns_of_192(dtype, K, NO):
 
 @pytest.mark.parametrize("K,NO,N,P", [(196, 196, 13100, 13100), (516, 200, 7001, 700), (200, 516, 7001, 7001), (1028, 260, 2000, 63), (704, 352, 10816, 10816),
                                       (192, 192, 13564, 6782), (260, 1028, 2000, 2000), (768, 512, 2048, 2048), (768, 512, 2049, 2049)])
-def test_fp32_layers_on_split_operands(K, NO, N, P):
-    """Large fp32 products (csrc/dense_split.h): both tiles, remainders of 4 results and inner values, an odd number of stages, ranges of
-    rows, and either side of 256 fp32 tiles; no further from float64 than fp32 products and sums of that length are (their partial sums random: sqrt(K) roundings)."""
+def test_large_fp32_layers(K, NO, N, P):
+    """Large fp32 products: remainders of 4 results and inner values, an odd number of stages, ranges of rows, and either side of 256
+    tiles; no further from float64 than fp32 products and sums of that length are (their partial sums random: sqrt(K) roundings)."""
     from pyramidconvblock_amd import ops
 
     _layers(torch.float32, K, NO, N, P)
@@ -80,9 +80,8 @@ def test_fp32_layers_on_split_operands(K, NO, N, P):
     assert float((dw.double().cpu() - want).norm() / want.norm()) <= 2.0 ** -24 * N ** 0.5
 
 
-def test_fp32_split_operands_and_values_that_are_not_finite():
-    """Results are those of fp32 arithmetic where an operand has no three bf16 parts: infinities of a sign, NaN, and values that round
-    up to infinity in bf16; the others are as without them."""
+def test_fp32_values_that_are_not_finite():
+    """Infinities of a sign, NaN, and values near fp32's largest give what fp32 arithmetic gives; the other results are as without them."""
     from pyramidconvblock_amd import ops
 
     K, NO, N = 260, 256, 8000
@@ -118,12 +117,13 @@ def test_fp32_split_operands_and_values_that_are_not_finite():
     assert float((y[:, keep] - clean[:, keep]).norm() / clean.norm()) < 1e-6
 
 
-def test_fp32_split_operands_whose_products_overflow():
-    """Infinities as fp32 products give them, not the NaN of parts that overflow in opposite directions."""
+@pytest.mark.parametrize("K", [256, 260])   # (weight gradients up to 256 wide run dense_any.hip)
+def test_fp32_values_whose_products_overflow(K):
+    """Infinities, and no NaN."""
     from pyramidconvblock_amd import ops
 
     gen = torch.Generator().manual_seed(3)
-    x, w, g = randn(gen, 8000, 256), randn(gen, 256, 256), randn(gen, 8000, 256)
+    x, w, g = randn(gen, 8000, K), randn(gen, 256, K), randn(gen, 8000, 256)
     clean = ops.dense_forward(x.cuda(), w.cuda()).cpu()
     xp, wp = x.clone(), w.clone()
     xp[5], wp[7] = (x[5].abs() + 1) * 1e23, (w[7].abs() + 1) * 1e23
@@ -138,13 +138,14 @@ def test_fp32_split_operands_whose_products_overflow():
     assert dw[11, 9] == -float("inf") and int(torch.isfinite(dw).logical_not().sum()) == 1
 
 
+@pytest.mark.parametrize("K", [256, 260])
 @pytest.mark.parametrize("scale", [1e-29, 1e-34, 1e-37])
-def test_fp32_split_operands_near_the_smallest_values(scale):
-    """Values whose parts bf16 cannot hold: no less precise than others."""
+def test_fp32_values_near_the_smallest(scale, K):
+    """No less precise than others."""
     from pyramidconvblock_amd import ops
 
     gen = torch.Generator().manual_seed(2)
-    x, w = randn(gen, 8000, 256), randn(gen, 256, 256) * 1e4
+    x, w = randn(gen, 8000, K), randn(gen, 256, K) * 1e4
     x[:1000] *= scale   # (beside rows of ordinary values, in tiles of their own and in one with them)
     y = ops.dense_forward(x.cuda(), w.cuda()).cpu().double()
     want = x.double() @ w.double().t()
@@ -157,9 +158,69 @@ def test_fp32_split_operands_near_the_smallest_values(scale):
 
 
 @pytest.mark.parametrize("dim,shape", [(400, (3, 47, 45, 400)), (712, (1, 50, 41, 712))])
-def test_fp32_block_on_split_operands(oracle, dim, shape):
-    """Both products of a layer's backward on split operands, in one launch."""
+def test_large_fp32_products_of_a_block(oracle, dim, shape):
+    """Both products of a layer's backward, in one launch."""
     _block_case(oracle, dim, 3, shape, torch.float32)
+
+
+def test_fp32_results_of_one_term_are_rounded_once():
+    """A sum of zeros and one product is that product rounded to fp32: operands keep all their bits, and so do their products."""
+    from pyramidconvblock_amd import ops
+
+    N, K, NO = 10816, 704, 352
+    gen = torch.Generator().manual_seed(4)
+    at = torch.randint(0, K, (N,), generator=gen)
+    v, w, g = randn(gen, N), randn(gen, NO, K), randn(gen, N, NO)
+    x = torch.zeros(N, K)
+    x[torch.arange(N), at] = v
+    y = ops.dense_forward(x.cuda(), w.cuda()).cpu()
+    assert torch.equal(y, v[:, None] * w.t()[at])
+    dx = ops.dense_forward(x.cuda(), w.t().contiguous().cuda(), w_kmajor=True).cpu()
+    assert torch.equal(dx, y)
+    rows = torch.randint(0, N, (K,), generator=gen)
+    x = torch.zeros(N, K)
+    x[rows, torch.arange(K)] = v[:K]
+    dw = ops.dense_wgrad(g.cuda(), x.cuda()).cpu()
+    assert torch.equal(dw, (g[rows] * v[:K, None]).t())
+
+
+def test_fp32_small_values_beside_ordinary_ones():
+    """A column near fp32's smallest values among ordinary ones, and small values that meet large ones: as precise as the others."""
+    from pyramidconvblock_amd import ops
+
+    N, K, NO = 10816, 704, 352
+    gen = torch.Generator().manual_seed(5)
+    x, g, w = randn(gen, N, K), randn(gen, N, NO), randn(gen, NO, K)
+    x[:, 5] *= 1e-36
+    dw = ops.dense_wgrad(g.cuda(), x.cuda()).cpu().double()
+    want = g.double().t() @ x.double()
+    assert float((dw[:, 5] - want[:, 5]).norm() / want[:, 5].norm()) <= 2.0 ** -24 * N ** 0.5
+    w[:, :] = 0
+    w[:, 5] = 1e30
+    y = ops.dense_forward(x.cuda(), w.cuda()).cpu().double()
+    want = x.double() @ w.double().t()
+    assert float((y - want).norm() / want.norm()) <= 2.0 ** -24
+
+
+def test_fp32_products_take_as_long_whatever_the_values():
+    """A NaN in every tile does not slow a product down (a bound far above what timings scatter by: a fifth at most)."""
+    from pyramidconvblock_amd import ops
+
+    x, w = torch.randn(10816, 704, device="cuda"), torch.randn(352, 704, device="cuda")
+    bad = x.clone()
+    bad[::64, 3] = float("nan")
+
+    def ms(a):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        ops.dense_forward(a, w), ops.dense_wgrad(a, a)
+        start.record()
+        for _ in range(20):
+            ops.dense_forward(a, w), ops.dense_wgrad(a, a)
+        end.record()
+        end.synchronize()
+        return start.elapsed_time(end)
+
+    assert min(ms(bad) for _ in range(3)) < 4 * min(ms(x) for _ in range(3))
 
 
 @pytest.mark.parametrize("dtype,N", [(torch.bfloat16, 270000), (torch.float32, 140000)])
