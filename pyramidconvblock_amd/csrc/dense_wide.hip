@@ -597,7 +597,7 @@ int dense_wide_rows_launch(const void* x, const void* w, int w_kmajor, const voi
     if (dtype == kF32) return PDW_WIDE2_T(float, 64, 64);
     if (bn == 192) return PDW_WIDE2(128, 192);
     if (bm == 64) return bn == 64 ? PDW_WIDE(64, 64) : PDW_WIDE(64, 128);
-    return bn == 64 ? PDW_WIDE(128, 64) : PDW_WIDE2(128, 128);
+    return bn == 64 ? PDW_WIDE2(128, 64) : PDW_WIDE2(128, 128);
 #undef PDW_WIDE
 #undef PDW_WIDE2
 #undef PDW_WIDE_T

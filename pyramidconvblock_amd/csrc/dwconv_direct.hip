@@ -129,7 +129,7 @@ __global__ __launch_bounds__(256) void wgrad_reduce_parts(const float* __restric
 
 __global__ __launch_bounds__(256) void wgrad_reduce_many(const ReduceJobs jobs) {
     __shared__ float red[kReduceLds];
-    reduce_jobs_block(jobs, blockIdx.x, red);
+    reduce_jobs_block<false>(jobs, blockIdx.x, red);
 }
 
 // Deferred mode (per host thread): between reduce_defer_begin and reduce_defer_flush the reductions are only
