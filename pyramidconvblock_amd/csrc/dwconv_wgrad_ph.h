@@ -29,10 +29,10 @@
 //
 // Filters 16 and 17 have one more column and row than the indices.  The 16 rows of B are then those before x's row (u = 1 .. 16), and
 // the rest comes from 8 products a pass besides the 32 of a channel: column 16 with the pass's 8 rows of x as A's index, row 0 with
-// the vectors p against the phases r and the rows as k groups (both as differences of their indices, added up at the end).
-// Such a pass takes 2.5 us.  us of kernel and summation against a kernel of two accumulators over bands of single images (two 1 KB
-// operands a product): [32,56,56,64] 29.6 -> 23.7, [128,56,56,64] 81 -> 52, [5,47,51,1000] 67 -> 36, [79,7,7,264] 55 -> 24, [1,28,28,64]
-// 10.2 -> 11.2 (within the block's launch, where it runs beside others, no longer: 54.9 and 55.0 its training step).
+// the vectors p against the phases r and the rows as k groups (both as differences of their indices, added up at the end by lane
+// rotations: 10.1 us of the smallest launch, 10.9 through LDS).  us of kernel and summation against a kernel of two accumulators over bands
+// of single images (two 1 KB operands a product): [32,56,56,64] 26.6 -> 19.9, [128,56,56,64] 77.4 -> 45.7, [5,47,51,1000] 64.3 -> 31.9,
+// [79,7,7,264] 53.7 -> 21.1, [1,28,28,64] 10.0 -> 9.5.
 #pragma once
 #include <mutex>
 
@@ -205,8 +205,8 @@ __device__ __forceinline__ void dwconv_wgrad_ph_body(const T* __restrict__ x, co
 
     // EDGE: column 16 and row 0 of the filter, which a product of 16 columns with the 16 rows before does not hold.
     // Column 16: products of the pass's 8 rows of x (index) with the 16 gy rows before the pass, and with its own 8:
-    // u = m - n + 16 (n >= m: others lie beyond the filter) and m - n (n <= m).  Row 0: products of the vectors p (index, 0 .. 15 and
-    // 8 .. 23) with the phases r, four rows of x and gy at a time as the k groups: v = p - r.
+    // u = m - n + 16 (n >= m: others lie beyond the filter) and m - n (n <= m).  Row 0: products of the phases r (index) with the
+    // vectors p (0 .. 15 and 8 .. 23), four rows of x and gy at a time as the k groups: v = p - r.  A tap is a sum along a diagonal of both.
     tz_f32x4 before[EDGE ? CPW : 1], own[EDGE ? CPW : 1], row0[EDGE ? CPW : 1][2];
     if constexpr (EDGE) {
 #pragma unroll
@@ -225,20 +225,25 @@ __device__ __forceinline__ void dwconv_wgrad_ph_body(const T* __restrict__ x, co
 #pragma unroll
                     for (int q = 0; q < CPW; ++q) a[row % 2][f][q] = read16(xa + q * XPL + row * XROW + 64 * f);
             };
+            // (the lane's part of these addresses is made in every pass: kept, they cost registers that others are spilled for,
+            // [128,56,56,64] 48.8 us for 45.7)
+            int here = lane;
+            asm volatile("" : "+v"(here));
+            const int en = here & 15, ek = here >> 4;
             const char* const xe = xl + plane * XPL + hoff + buffer * Sh::XBUF;
             const char* const ge = gl + plane * GPL + hoff + buffer * Sh::GBUF;
             auto read_row0 = [&](int i) {   // channel i % 2, rows 4 (i / 2) ..
                 const int q = i % 2, r = 4 * (i / 2);
 #pragma unroll
-                for (int t = 0; t < 2; ++t) ea[0][t] = read16(xe + q * XPL + (r + kg) * XROW + (8 * t + ln) * 16);
-                eb = read16(ge + q * GPL + (r + kg) * GROW + (ln & 7) * 16);
+                for (int t = 0; t < 2; ++t) ea[0][t] = read16(xe + q * XPL + (r + ek) * XROW + (8 * t + en) * 16);
+                eb = read16(ge + q * GPL + (r + ek) * GROW + (en & 7) * 16);
             };
 #pragma unroll
             for (int q = 0; q < CPW; ++q)
 #pragma unroll
                 for (int f = 0; f < 2; ++f) {
                     n[q][f] = read16(ga + q * GPL + 64 * f);
-                    ea[q][f] = read16(xe + q * XPL + (ln & 7) * XROW + (16 + 4 * f + kg) * 16);
+                    ea[q][f] = read16(xe + q * XPL + (en & 7) * XROW + (16 + 4 * f + ek) * 16);
                 }
             read_row(0);
 #pragma unroll
@@ -260,7 +265,7 @@ __device__ __forceinline__ void dwconv_wgrad_ph_body(const T* __restrict__ x, co
                     for (int q = 0; q < CPW; ++q) acc[q][row] = mfma16(a[row % 2][f][q], bop[q][f], acc[q][row], T());
                 if (row < 4) {
 #pragma unroll
-                    for (int t = 0; t < 2; ++t) row0[row % 2][t] = mfma16(ea[0][t], eb, row0[row % 2][t], T());
+                    for (int t = 0; t < 2; ++t) row0[row % 2][t] = mfma16(eb, ea[0][t], row0[row % 2][t], T());
                 }
                 // the pass's gy row `row`, which index `row` of n holds
 #pragma unroll
@@ -368,32 +373,30 @@ __device__ __forceinline__ void dwconv_wgrad_ph_body(const T* __restrict__ x, co
             if (u < g.K && v < g.K) ep[(u * g.K + v) * EPP + plane + q] = tot[q][r];
         }
     if constexpr (EDGE) {
-        // per channel [8][24] products of column 16 (n of before, n of own) and [8 phases][24 vectors] of row 0; a tap is the sum of
-        // eight of them, added in this order
-        constexpr int EW = 24, ECH = 2 * 8 * EW + 1;
-        float* const ee = ep + 17 * 17 * EPP;
-        static_assert((17 * 17 * EPP + CS * ECH) * 4 <= Sh::lds_bytes, "LDS");
+        // sum of at_m[(lane + m) mod 16] over m < 8, at_m[n] being above[m] where n >= m and below[m] else; every lane group has it
+        int here = tid;
+        asm volatile("" : "+v"(here));   // (what follows from it is not worth registers during the passes)
+        here &= 63;
+        const int n = here & 15, group = here >> 4, first = n - 4 * (group & 1);   // m = 4 (group mod 2) + r
+        auto diagonal = [&](const tz_f32x4& above, const tz_f32x4& below) {
+            float t = first >= 0 ? above[0] : below[0];
+#define PDW_ROT(r)                                                                             \
+    t += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(first >= r ? above[r] : below[r]), 0x120 + 16 - r, 0xf, 0xf, true));
+            PDW_ROT(1) PDW_ROT(2) PDW_ROT(3)
+#undef PDW_ROT
+            t = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(t), __float_as_int(t), 0x120 + 12, 0xa, 0xf, false));
+            return t + __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(t), 0x401f));   // (lanes 16 apart)
+        };
 #pragma unroll
         for (int q = 0; q < CPW; ++q) {
-            float* const e = ee + (plane + q) * ECH;
+            const float column = diagonal(before[q], own[q]), corner = diagonal(own[q], own[q]);   // (16 - lane, 16); lane 0: (0, 16)
+            tz_f32x4 far;   // the vectors 16 .. 23 at the lanes 0 .. 7
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int m = 4 * kg + r;
-                if (m < 8) e[m * EW + ln] = before[q][r];
-                if (m < 8 && ln < 8) e[m * EW + 16 + ln] = own[q][r];
-                if (ln < 8) e[(8 + ln) * EW + m] = row0[q][0][r];
-                if (m >= 8 && ln < 8) e[(8 + ln) * EW + 8 + m] = row0[q][1][r];
-            }
-        }
-        __syncthreads();
-        for (int i = tid; i < 33 * CS; i += NT) {
-            const int c = i % CS, tap = i / CS;   // 0 .. 16: (tap, 16); 17 .. 32: (0, tap - 17)
-            const float* const e = ee + c * ECH;
-            float sum = 0.f;
-#pragma unroll
-            for (int m = 0; m < 8; ++m) sum += tap < 17 ? e[m * EW + (m < tap ? m - tap + 16 : 16 + m - tap)] : e[(8 + m) * EW + tap - 17 + m];
-            const int tu = tap < 17 ? tap : 0, tv = tap < 17 ? 16 : tap - 17;
-            if (tu < g.K && tv < g.K) ep[(tu * g.K + tv) * EPP + c] = sum;
+            for (int r = 0; r < 4; ++r)
+                far[r] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(row0[q][1][r]), 0x128, 0xf, 0xf, true));
+            const float row = diagonal(row0[q][0], far);   // (0, lane)
+            const int tu = group == 0 ? 16 - n : 0, tv = group == 1 ? n : 16;
+            if ((group < 2 || here == 32) && tu < g.K && tv < g.K) ep[(tu * g.K + tv) * EPP + plane + q] = group == 0 ? column : group == 1 ? row : corner;
         }
     }
     __syncthreads();
@@ -449,10 +452,11 @@ inline bool wgrad_ph_cut(WgPhPlan& p, int n) {
 }
 
 // Price of a run to the planners, us: start-up (16 gy rows, two round trips to memory, the partial), then passes of 8 rows.  (Of runs
-// that share the chip with other problems; see the top for a chip full of them.  Beyond 15: training steps of [8,112,112,96], [128,56,56,128]
-// and [26,106,105,80] with filter 17, us, at 1.35 126, 460, 295; 1.85 124, 442, 288; 2.5 122, 434, 286; 3.3 128, 451, 288.)
+// that share the chip with other problems; see the top for a chip full of them.  Beyond 15: training steps of [128,56,56,128],
+// [16,40,40,256] and [26,106,105,80] with filter 17, us, at 2.1 437.2, 119.5, 280.6; 2.3 434.0, 119.7, 280.7; 2.5 432.8, 121.7, 282.1; 2.7 433.0,
+// 121.6, 281.8.)
 constexpr double kWgPhStart = 7.0;
-inline double wgrad_ph_step(int K) { return K <= 9 ? 1.15 : K <= 15 ? 1.35 : 2.5; }
+inline double wgrad_ph_step(int K) { return K <= 9 ? 1.15 : K <= 15 ? 1.35 : 2.3; }
 inline double wgrad_ph_run_cost(int K, int passes) { return kWgPhStart + wgrad_ph_step(K) * passes; }
 
 // Covered: 16-bit types (the caller checks), C % 8 == 0, K <= 17, 16-byte aligned tensors.
