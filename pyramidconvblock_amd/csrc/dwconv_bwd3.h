@@ -154,8 +154,12 @@ static Bwd3Plan bwd3_plan(int B, const TzGeom& gd, int npcd, const WgPhPlan& p0,
 // estimated to end first, of one round or several; n[0] = 0 where a launch each is estimated to take no longer.  Together they save a launch and
 // fill the rounds that 72 slices, say, leave open (2 x 216 workgroups, or 288 + 216 in two rounds); apart, each side has the chip and its
 // memory to itself and its steps are shorter ([64,56,56,128] filter 13 in one round 83.7 us, apart 70.1, [39,45,45,216] filter 17 117
-// and 87).  Prices fitted to both of 160 random shapes with cold buffers; with them 180 others
-// take 1.12 times less, the slowest 1.05 times more ([74,17,17,896] filter 9 76.8 -> 80.7).  us with the summation, apart and together:
+// and 87).  Prices fitted to both of 160 random shapes with cold buffers.  What they do not see: in several rounds, runs of either side longer than
+// by itself leave both sides short of memory all the time (with the estimate 0 to 10 % ahead [97,10,11,896] filter 9 64.7 -> 71.6, [75,12,12,624]
+// filter 7 42.0 -> 44.8; as long as by itself, 220 such plans 0.98 to 1.5 times as fast), so these have to be estimated further ahead.
+// (One round of filters 3 and 5 alike would lose more than it gains: [92,7,7,448] filter 5 29.0 for 26.8 apart, but [27,29,28,640] 43.6 for 49.4,
+// [42,11,11,1008] filter 3 27.1 for 30.5.)  300 other shapes take 1.18 times less, the slowest 1.04 times more ([11,64,64,432] filter 7).
+// us with the summation, apart and together:
 // [8,64,64,1152] filter 9 84 -> 70, [32,28,28,256] filter 13 33.8 -> 28.8, [2,20,20,64] filter 7 13.2 -> 8.6, [11,74,74,688] filter 9 137 -> 109.
 template <int K>
 static Bwd3Plan bwd2_plan(const TzGeom& gd, int npcd, const WgPhPlan& p0) {
@@ -166,17 +170,20 @@ static Bwd3Plan bwd2_plan(const TzGeom& gd, int npcd, const WgPhPlan& p0) {
     if (auto it = cache.find(key); it != cache.end()) return it->second;
     // us of a run's start and of its steps in a launch of its own, the input gradient's (filters 15 and 17: 8 channels) and the weight
     // gradient's; their steps side by side, in one round and in several (which are full of either side most of the time); what an
-    // estimate of one round has to be ahead by (launch_makespan adds its own to several)
+    // estimate of one round has to be ahead by, and one of several with longer runs than by itself (launch_makespan adds its own to all of these)
     constexpr double kStartD = 5.5, kStepD = K <= 9 ? 1.25 : K <= 13 ? 1.4 : 1.2, kStartF = kWgPhStart, kStepF = K <= 9 ? 1.25 : K <= 15 ? 1.8 : 2.5,
-                     kLaunch = 2.8, kShareOne = K <= 5 ? 1.15 : K <= 9 ? 1.17 : 1.2, kShareMore = K <= 5 ? 1.15 : K <= 9 ? 1.1 : 1.2, kAhead = 1.04;
+                     kLaunch = 2.8, kShareOne = K <= 5 ? 1.15 : K <= 9 ? 1.17 : 1.2, kShareMore = K <= 5 ? 1.15 : K <= 9 ? 1.1 : 1.2, kAhead = 1.04,
+                     kAheadLonger = 1.1;
     const int ni = 16 / npcd;
     std::vector<LaunchCut> cuts[2];
     TzGeom g = gd;
     double apart = kLaunch + cdiv(p0.nblocks, 256) * (kStartF + kStepF * p0.g.passes);
+    long long alone = 0;   // workgroups of the input gradient by itself
     if (tz_cut_alone(g, ni, K <= 5)) {
         const double steps = tz_alone_cost(tz_blocks(g), tz_steps(g), K <= 5);
         apart += K <= 5 ? kStepD * steps : cdiv(tz_blocks(g), 256) * kStartD + kStepD * (steps - cdiv(tz_blocks(g), 256) * 4.5);
         const int runs = g.nruns;
+        alone = tz_blocks(g);
         int last = 0;
         for (int e = 2; e <= 16; ++e) {
             const int most = cdiv(cdiv(tz_rows(gd, ni), 8) * (gd.stack ? 1 : cdiv(gd.B, ni)), std::max(1, runs * e / 8));
@@ -197,7 +204,8 @@ static Bwd3Plan bwd2_plan(const TzGeom& gd, int npcd, const WgPhPlan& p0) {
             const LaunchCut d{dc.n, kStartD + share * dc.cost, dc.count}, f{fc.n, kStartF + share * fc.cost, fc.count};
             const LaunchCut* const pick[2] = {&d, &f};
             const int ord[2] = {d.cost >= f.cost ? 0 : 1, d.cost >= f.cost ? 1 : 0};
-            const double t = (single ? kAhead : 1.0) * launch_makespan(pick, ord);
+            const bool longer = dc.count < alone || fc.count < p0.nblocks;
+            const double t = (single ? kAhead : longer ? kAheadLonger : 1.0) * launch_makespan(pick, ord);
             if (t >= apart) continue;
             apart = t;
             best.n[0] = d.n, best.n[1] = f.n;

@@ -1,5 +1,7 @@
 """Both gradients of a stand-alone depthwise convolution as one call (csrc/dwconv_bwd3.h without a pooled scale): against the float64
 oracle and the two separate calls, with the partial sums inside the workspace that the size query names."""
+import ctypes
+
 import pytest
 import torch
 
@@ -57,6 +59,45 @@ def test_cuts(shape, k):
     x, gy = (torch.randn(shape, generator=gen, device="cuda").bfloat16() for _ in range(2))
     w = torch.randn(k, k, shape[3], generator=gen, device="cuda").bfloat16()
     _same(*_both(x, gy, w, (*shape, k, k, 1, 1, k // 2, k // 2, 1, 1)))
+
+
+def _launches(x, gy, w, geo):
+    """Kernels that a call of pdw_dwconv_bwd launches: the nodes of a graph that it is captured into (and that is not replayed)."""
+    from pyramidconvblock_amd import _lib
+
+    L, code = _lib.lib(), _lib.dtype_code(x.dtype)
+    need = L.pdw_dwconv_wgrad_workspace_bytes(*geo, code)
+    ws, dx, dw = torch.empty(need // 4 + 1, device="cuda"), torch.empty_like(x), torch.empty_like(w)
+    stream = torch.cuda.Stream()
+
+    def call():
+        _lib.check(L.pdw_dwconv_bwd(gy.data_ptr(), w.data_ptr(), x.data_ptr(), dx.data_ptr(), dw.data_ptr(), ws.data_ptr(), need, *geo, code,
+                                    stream.cuda_stream), "pdw_dwconv_bwd")
+
+    torch.cuda.synchronize()
+    call()
+    torch.cuda.synchronize()
+    hip = ctypes.CDLL("libamdhip64.so")
+    handle, graph, nodes = ctypes.c_void_p(stream.cuda_stream), ctypes.c_void_p(), ctypes.c_size_t()
+    assert hip.hipStreamBeginCapture(handle, 1) == 0   # (calls of this thread)
+    try:
+        call()
+    finally:
+        ended = hip.hipStreamEndCapture(handle, ctypes.byref(graph))
+    assert ended == 0 and hip.hipGraphGetNodes(graph, None, ctypes.byref(nodes)) == 0
+    assert hip.hipGraphDestroy(graph) == 0
+    return nodes.value
+
+
+# the shared launch and its summation, in one round of workgroups and in several (72, 69 and 66 slices); two launches and the summation where the
+# shared one takes as long or longer: runs of the weight gradient twice as long to make room (45 slices), chips full of either side
+@pytest.mark.parametrize("shape,k,launches", [((2, 20, 20, 64), 7, 2), ((32, 28, 28, 256), 13, 2), ((8, 64, 64, 1152), 9, 2), ((8, 19, 19, 1096), 7, 2),
+                                              ((10, 16, 16, 1056), 9, 2), ((74, 17, 17, 896), 9, 3), ((40, 15, 15, 712), 13, 3),
+                                              ((64, 56, 56, 128), 13, 3), ((39, 45, 45, 216), 17, 3)])
+def test_launches(shape, k, launches):
+    x, w = torch.zeros(shape, device="cuda", dtype=torch.bfloat16), torch.zeros(k, k, shape[3], device="cuda", dtype=torch.bfloat16)
+    n = _launches(x, torch.zeros_like(x), w, (*shape, k, k, 1, 1, k // 2, k // 2, 1, 1))
+    assert n == launches
 
 
 # what the shared launch does not take runs as the two calls
