@@ -252,7 +252,7 @@ __device__ __forceinline__ void dense_rows_body(const T* __restrict__ X, const T
     // this lane's four bias values: an unconditional 8-byte load (of the weights when there is no bias), converted
     // where the table is written, so that nothing waits for it before the weights and the first tile are requested
     const ChanVec<T, 4> braw = *reinterpret_cast<const ChanVec<T, 4>*>(bias && bcol < NO ? bias + bcol : W);
-    if (K != KP || NO != NOP || (!STATIC && map.seg)) {  // uniform
+    if (K != KP || NO != NOP || (!STATIC && !KMAJOR && map.seg)) {  // uniform
         for (int i = tid; i < NOP * ldw / 8; i += 256) reinterpret_cast<uint4*>(wl)[i] = make_uint4(0u, 0u, 0u, 0u);
         __syncthreads();
     }

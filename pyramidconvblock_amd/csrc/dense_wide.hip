@@ -223,7 +223,7 @@ struct WideArgs {
 template <typename T, int BM, int BN>
 constexpr int kWideOccupancy = sizeof(T) == 4 ? (BM * BN <= 64 * 64 ? 4 : BM * BN <= 128 * 64 ? 3 : 2) : 2;
 
-template <typename T, int BM, int BN, bool TA, bool TB, bool PART, int STAGES = 2>
+template <typename T, int BM, int BN, bool TA, bool TB, bool PART, int STAGES = 2, bool MAP = false>
 __device__ __forceinline__ void wide_gemm_body(const WideArgs& g, int blk, int nblk) {
     typedef Operand<T, BM, TA> OpA;
     typedef Operand<T, BN, TB> OpB;
@@ -245,12 +245,9 @@ __device__ __forceinline__ void wide_gemm_body(const WideArgs& g, int blk, int n
     OpA a;
     OpB b;
     a.init((const char*)g.a, g.lda, m0, g.M, kb, ke);
-    if constexpr (!TB && !PART && sizeof(T) == 2) {
-        if (g.map.seg) b.init((const char*)g.b, g.ldb, n0, g.N, kb, ke, g.map);   // (uniform)
-        else b.init((const char*)g.b, g.ldb, n0, g.N, kb, ke);
-    } else {
-        b.init((const char*)g.b, g.ldb, n0, g.N, kb, ke);
-    }
+    // (a kernel of its own for a RowMap: chosen inside one, the two cost other layers up to 0.6 us of 10)
+    if constexpr (MAP) b.init((const char*)g.b, g.ldb, n0, g.N, kb, ke, g.map);
+    else b.init((const char*)g.b, g.ldb, n0, g.N, kb, ke);
     const int left = (int)(ke - kb), nst = (left + BK - 1) / BK;
     v16f acc[FM][FN];
 #pragma unroll
@@ -421,9 +418,9 @@ __device__ __forceinline__ void wide_gemm_body(const WideArgs& g, int blk, int n
     }
 }
 
-template <typename T, int BM, int BN, bool TA, bool TB, bool PART, int STAGES>
+template <typename T, int BM, int BN, bool TA, bool TB, bool PART, int STAGES, bool MAP = false>
 __global__ __launch_bounds__(256, (STAGES == 2 ? kWideOccupancy<T, BM, BN> : 1)) void wide_gemm_k(WideArgs g) {
-    wide_gemm_body<T, BM, BN, TA, TB, PART, STAGES>(g, blockIdx.x, gridDim.x);
+    wide_gemm_body<T, BM, BN, TA, TB, PART, STAGES, MAP>(g, blockIdx.x, gridDim.x);
 }
 
 // Both products that read the gradient of a layer's output, as one launch: the weight gradient's nw workgroups (tiles of WM x WN
@@ -478,19 +475,19 @@ int pair_go(const WideArgs& rows, const WideArgs& wgrad, const AnyWgradArgs& any
     return check_launch("wide_pair");
 }
 
-template <typename T, int BM, int BN, bool TA, bool TB, bool PART, int STAGES = kDeep>
+template <typename T, int BM, int BN, bool TA, bool TB, bool PART, int STAGES = kDeep, bool MAP = false>
 int wide_go(const WideArgs& g, hipStream_t s) {
     constexpr size_t lds = wide_lds<T, BM, BN, PART, STAGES>();
     if constexpr (STAGES == kDeep) {
-        if (!goes_deep<T>((long long)g.mt * g.nt * g.splits, lds, PART ? g.kper : g.Kd, PART ? 3 : 6)) return wide_go<T, BM, BN, TA, TB, PART, 2>(g, s);
+        if (!goes_deep<T>((long long)g.mt * g.nt * g.splits, lds, PART ? g.kper : g.Kd, PART ? 3 : 6)) return wide_go<T, BM, BN, TA, TB, PART, 2, MAP>(g, s);
     }
     if constexpr (lds > 64 * 1024) {
         static std::once_flag once;
         std::call_once(once, [] {
-            (void)hipFuncSetAttribute((const void*)wide_gemm_k<T, BM, BN, TA, TB, PART, STAGES>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+            (void)hipFuncSetAttribute((const void*)wide_gemm_k<T, BM, BN, TA, TB, PART, STAGES, MAP>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         });
     }
-    hipLaunchKernelGGL((wide_gemm_k<T, BM, BN, TA, TB, PART, STAGES>), dim3((unsigned)(g.mt * g.nt * g.splits)), dim3(256), lds, s, g);
+    hipLaunchKernelGGL((wide_gemm_k<T, BM, BN, TA, TB, PART, STAGES, MAP>), dim3((unsigned)(g.mt * g.nt * g.splits)), dim3(256), lds, s, g);
     return check_launch("wide_gemm");
 }
 
@@ -590,17 +587,22 @@ int dense_wide_rows_launch(const void* x, const void* w, int w_kmajor, const voi
     if (!wide_rows_plan(g, bm, bn, x, w, w_kmajor, bias, rowbias, y, N, K, NO, P, dtype)) return -1;
     if (N == 0) return 0;
     if (map) g.map = *map;
-#define PDW_WIDE_T(T, BM, BN) (w_kmajor ? wide_go<T, BM, BN, false, true, false>(g, s) : wide_go<T, BM, BN, false, false, false>(g, s))
+#define PDW_WIDE_S(T, BM, BN, STAGES)                              \
+    (w_kmajor ? wide_go<T, BM, BN, false, true, false, STAGES>(g, s) \
+     : map    ? wide_go<T, BM, BN, false, false, false, STAGES, true>(g, s) : wide_go<T, BM, BN, false, false, false, STAGES>(g, s))
+#define PDW_WIDE_T(T, BM, BN) PDW_WIDE_S(T, BM, BN, kDeep)
 #define PDW_WIDE(BM, BN) (dtype == kF16 ? PDW_WIDE_T(f16_t, BM, BN) : PDW_WIDE_T(bf16_t, BM, BN))
 #define PDW_WIDE2(BM, BN) (dtype == kF16 ? PDW_WIDE2_T(f16_t, BM, BN) : PDW_WIDE2_T(bf16_t, BM, BN))   /* (tiles of launches that fill the chip) */
-#define PDW_WIDE2_T(T, BM, BN) (w_kmajor ? wide_go<T, BM, BN, false, true, false, 2>(g, s) : wide_go<T, BM, BN, false, false, false, 2>(g, s))
-    if (dtype == kF32) return PDW_WIDE2_T(float, 64, 64);
+#define PDW_WIDE2_T(T, BM, BN) PDW_WIDE_S(T, BM, BN, 2)
+    if (dtype == kF32) return w_kmajor ? wide_go<float, 64, 64, false, true, false, 2>(g, s) : wide_go<float, 64, 64, false, false, false, 2>(g, s);
     if (bn == 192) return PDW_WIDE2(128, 192);
     if (bm == 64) return bn == 64 ? PDW_WIDE(64, 64) : PDW_WIDE(64, 128);
     return bn == 64 ? PDW_WIDE2(128, 64) : PDW_WIDE2(128, 128);
 #undef PDW_WIDE
 #undef PDW_WIDE2
 #undef PDW_WIDE_T
+#undef PDW_WIDE2_T
+#undef PDW_WIDE_S
 }
 
 // (of either type)
