@@ -491,6 +491,17 @@ int wide_go(const WideArgs& g, hipStream_t s) {
     return check_launch("wide_gemm");
 }
 
+// Tiles of the 16-bit row product.
+void rows_tiles(long long N, int K, int NO, int& bm, int& bn) {
+    // tiles of 64 rows where 128-row tiles would leave compute units without work
+    bm = (long long)cdiv(N, 128) * cdiv(NO, 128) < 256 ? 64 : 128, bn = NO <= 64 ? 64 : 128;
+    // 192 columns (a sixth fewer bytes staged per product, longer tiles) where they save a whole round of the 512 tiles
+    // that the chip holds; a third longer each ([16384,1152] -> 576, one round instead of two, 35.0 -> 27.4 us; 576 ->
+    // 1152, two instead of three, 32.7 -> 29.8; [100000,192] -> 384, four instead of five, would be 31.1 -> 35.7)
+    auto rounds = [&](int n) { return cdiv((long long)cdiv(N, 128) * cdiv(NO, n), 512); };
+    if (bm == 128 && bn == 128 && K >= 256 && rounds(192) * 4 < rounds(128) * 3) bn = 192;
+}
+
 // Tiles and row ranges of the weight gradient: tiles of 64 where a width is no more than that, and the number of ranges that is
 // estimated to end first: a compute unit's stages (0.6 us one of 128 x 128 results, whether it has one workgroup or two in turn), and
 // the partials, written and read once more in fp32.  (With no more partials than are the operands' traffic, 512 workgroups at most,
@@ -531,8 +542,25 @@ WgradPlan wgrad_make_plan(long long N, int M, int NO, int es) {
     // no range longer than its 32-bit offsets reach (operands of more than 2 GiB, widths that alone fill the chip)
     const long long most = 0x7fffffffLL / ((long long)(M > NO ? M : NO) * es) / 64 * 64;
     if (most > 0 && s < (N + most - 1) / most) s = (N + most - 1) / most;
-    p.kper = ((N + s - 1) / s + 63) / 64 * 64;
-    p.splits = (int)((N + p.kper - 1) / p.kper);
+    auto cut_in = [&](long long n) {
+        p.kper = ((N + n - 1) / n + 63) / 64 * 64;
+        p.splits = (int)((N + p.kper - 1) / p.kper);
+    };
+    cut_in(s);
+    // The launch that it shares with the input gradient (16-bit, two workgroups a compute unit; both make the same ranges, so that their results
+    // are the same): fewer, where all of that launch is then on the chip at once and a range gets fewer stages more than an input gradient's workgroup
+    // has, which otherwise start when the first others end.  (Training steps as graphs, filter 5 bf16, us, without and with this: [1,64,64,1152] 149.9 and
+    // 131.9, [1,76,75,776] 145.9 and 136.1, [1,88,88,672] 132.5 and 124.4, [3,57,61,400] 119.6 and 113.2; [11,51,50,200], where a range would have 12
+    // stages for 7 and the others have 2 and 4, 114.4 and 116.5, [15,56,57,368], 34 for 19 and 6, 230.9 and 234.3.)
+    if (es == 2 && p.bm == 128 && p.bn == 128) {
+        int bm, bn;
+        rows_tiles(N, M, NO, bm, bn);
+        const long long tiles = (long long)p.mt * p.nt, rows = (long long)cdiv(N, bm) * cdiv(NO, bn), fit = (512 - rows) / tiles, was = p.kper;
+        if (rows + tiles * p.splits > 512 && fit >= 1) {
+            cut_in(fit);
+            if ((p.kper - was) / bk >= cdiv(M, bk)) cut_in(s);
+        }
+    }
     return p;
 }
 
@@ -566,13 +594,7 @@ static bool wide_rows_plan(WideArgs& g, int& bm, int& bn, const void* x, const v
         if (K < 32 && N >= 16384 && NO <= 256) return false;
         bm = bn = 64;
     } else {
-        // tiles of 64 rows where 128-row tiles would leave compute units without work
-        bm = (long long)cdiv(N, 128) * cdiv(NO, 128) < 256 ? 64 : 128, bn = NO <= 64 ? 64 : 128;
-        // 192 columns (a sixth fewer bytes staged per product, longer tiles) where they save a whole round of the 512 tiles
-        // that the chip holds; a third longer each ([16384,1152] -> 576, one round instead of two, 35.0 -> 27.4 us; 576 ->
-        // 1152, two instead of three, 32.7 -> 29.8; [100000,192] -> 384, four instead of five, would be 31.1 -> 35.7)
-        auto rounds = [&](int n) { return cdiv((long long)cdiv(N, 128) * cdiv(NO, n), 512); };
-        if (bm == 128 && bn == 128 && K >= 256 && rounds(192) * 4 < rounds(128) * 3) bn = 192;
+        rows_tiles(N, K, NO, bm, bn);
     }
     g.mt = cdiv(N, bm), g.nt = cdiv(NO, bn);
     return (long long)g.mt * g.nt <= 0x7fffffffLL;

@@ -55,6 +55,12 @@ def test_few_workgroups_of_both_products(oracle, dim, shape):
     _block_case(oracle, dim, 3, shape, torch.float16)
 
 
+@pytest.mark.parametrize("dim,shape", [(400, (3, 57, 61, 400)), (1048, (1, 64, 67, 1048)), (200, (11, 51, 50, 200))])
+def test_row_ranges_that_make_room(oracle, dim, shape):
+    """Fewer row ranges for the launch of both products to be on the chip at once, one less (400) and one and two (1048), and as many as are estimated best (200)."""
+    _block_case(oracle, dim, 3, shape, torch.bfloat16)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("K,NO", [(264, 136), (320, 200), (256, 384)])
 def test_dense_wide_columns_of_192(dtype, K, NO):
