@@ -547,18 +547,19 @@ WgradPlan wgrad_make_plan(long long N, int M, int NO, int es) {
         p.splits = (int)((N + p.kper - 1) / p.kper);
     };
     cut_in(s);
-    // The launch that it shares with the input gradient (16-bit, two workgroups a compute unit; both make the same ranges, so that their results
-    // are the same): fewer, where all of that launch is then on the chip at once and a range gets fewer stages more than an input gradient's workgroup
-    // has, which otherwise start when the first others end.  (Training steps as graphs, filter 5 bf16, us, without and with this: [1,64,64,1152] 149.9 and
-    // 131.9, [1,76,75,776] 145.9 and 136.1, [1,88,88,672] 132.5 and 124.4, [3,57,61,400] 119.6 and 113.2; [11,51,50,200], where a range would have 12
-    // stages for 7 and the others have 2 and 4, 114.4 and 116.5, [15,56,57,368], 34 for 19 and 6, 230.9 and 234.3.)
-    if (es == 2 && p.bm == 128 && p.bn == 128) {
-        int bm, bn;
-        rows_tiles(N, M, NO, bm, bn);
-        const long long tiles = (long long)p.mt * p.nt, rows = (long long)cdiv(N, bm) * cdiv(NO, bn), fit = (512 - rows) / tiles, was = p.kper;
-        if (rows + tiles * p.splits > 512 && fit >= 1) {
+    // The launch that it shares with the input gradient (both make the same ranges, so that their results are the same): fewer, where it then is a round
+    // less, of two workgroups a compute unit (fp32: one, the matrix pipe being what bounds them), and the stages that the ranges are longer by are
+    // fewer than those of an input gradient's workgroup, which would be that round.  Training steps as graphs, filter 5, us, without and with this: bf16
+    // [1,64,64,1152] 149.9 and 131.9, [1,88,88,672] 132.5 and 122.9, [3,57,61,400] 119.6 and 111.5, but [11,51,50,200], where a range would have 12 stages
+    // for 7 and the others have 2 and 4, 114.4 and 116.5; fp32 [32,11,11,552] 204.3 and 196.3, [2,28,28,744] 155.1 and 148.3, [6,15,15,352] 109.4 and 105.4.
+    if (es == 2 ? p.bm == 128 && p.bn == 128 : p.bm == 64 && p.bn == 64 && (M > 256 || NO > 256)) {
+        int bm = 64, bn = 64;
+        if (es == 2) rows_tiles(N, M, NO, bm, bn);
+        const long long round = es == 2 ? 512 : 256, tiles = (long long)p.mt * p.nt, rows = (long long)cdiv(N, bm) * cdiv(NO, bn), was = p.kper,
+                        fit = (round * (cdiv(rows + tiles * p.splits, round) - 1) - rows) / tiles;
+        if (fit >= 1) {
             cut_in(fit);
-            if ((p.kper - was) / bk >= cdiv(M, bk)) cut_in(s);
+            if ((p.kper - was) / bk * cdiv(tiles * fit, round) >= cdiv(M, bk)) cut_in(s);
         }
     }
     return p;

@@ -55,10 +55,12 @@ def test_few_workgroups_of_both_products(oracle, dim, shape):
     _block_case(oracle, dim, 3, shape, torch.float16)
 
 
-@pytest.mark.parametrize("dim,shape", [(400, (3, 57, 61, 400)), (1048, (1, 64, 67, 1048)), (200, (11, 51, 50, 200))])
-def test_row_ranges_that_make_room(oracle, dim, shape):
-    """Fewer row ranges for the launch of both products to be on the chip at once, one less (400) and one and two (1048), and as many as are estimated best (200)."""
-    _block_case(oracle, dim, 3, shape, torch.bfloat16)
+@pytest.mark.parametrize("dtype,dim,shape", [(torch.bfloat16, 400, (3, 57, 61, 400)), (torch.bfloat16, 1048, (1, 64, 67, 1048)), (torch.bfloat16, 200, (11, 51, 50, 200)),
+                                             (torch.float32, 352, (6, 15, 15, 352)), (torch.float32, 872, (3, 21, 20, 872)), (torch.float32, 384, (3, 12, 15, 384))])
+def test_row_ranges_that_make_room(oracle, dtype, dim, shape):
+    """Fewer row ranges for the launch of both products to be a round less, by one (400) and more (1048; 352, one round; 872, two), and as many as are estimated
+    best by themselves (200, 384)."""
+    _block_case(oracle, dim, 3, shape, dtype)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
