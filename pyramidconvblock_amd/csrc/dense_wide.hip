@@ -541,7 +541,8 @@ WgradPlan wgrad_make_plan(long long N, int M, int NO, int es) {
     }
     // no range longer than its 32-bit offsets reach (operands of more than 2 GiB, widths that alone fill the chip)
     const long long most = 0x7fffffffLL / ((long long)(M > NO ? M : NO) * es) / 64 * 64;
-    if (most > 0 && s < (N + most - 1) / most) s = (N + most - 1) / most;
+    const long long fewest = most > 0 ? (N + most - 1) / most : 1;
+    s = std::max(s, fewest);
     auto cut_in = [&](long long n) {
         p.kper = ((N + n - 1) / n + 63) / 64 * 64;
         p.splits = (int)((N + p.kper - 1) / p.kper);
@@ -557,7 +558,7 @@ WgradPlan wgrad_make_plan(long long N, int M, int NO, int es) {
         if (es == 2) rows_tiles(N, M, NO, bm, bn);
         const long long round = es == 2 ? 512 : 256, tiles = (long long)p.mt * p.nt, rows = (long long)cdiv(N, bm) * cdiv(NO, bn), was = p.kper,
                         fit = (round * (cdiv(rows + tiles * p.splits, round) - 1) - rows) / tiles;
-        if (fit >= 1) {
+        if (fit >= fewest) {
             cut_in(fit);
             if ((p.kper - was) / bk * cdiv(tiles * fit, round) >= cdiv(M, bk)) cut_in(s);
         }

@@ -104,7 +104,8 @@ def test_block_buffers_hold_no_scratch_beyond_its_use(B, H, W, D, K, dtype):
         assert b"overlaps" in L.pdw_last_error()
 
 
-@pytest.mark.parametrize("N,M,NO", [(458752, 4096, 2048), (458752, 2048, 4096), (1 << 20, 2040, 1020), (1 << 17, 16376, 64)])
+@pytest.mark.parametrize("N,M,NO", [(458752, 4096, 2048), (458752, 2048, 4096), (1 << 20, 2040, 1020), (1 << 17, 16376, 64),
+                                    (8490, 63592, 168), (136435, 32464, 64)])   # (fewer ranges would save the launch of both products a round)
 def test_wide_weight_gradient_ranges_fit_32_bit_offsets(N, M, NO):
     """pdw_dense_wgrad of wide layers cuts the rows into ranges whose operands 32-bit offsets reach, also where the layer's
     tiles alone fill the chip: the workspace holds a partial result for each."""
