@@ -60,7 +60,7 @@ __global__ __launch_bounds__(512, 1) void dwconv_bwd3_k(const Bwd3Args a) {
     } else {
         if (blk >= a.nd + a.p[0].n + a.p[1].n) {
             extern __shared__ uint32_t smem[];
-            mean_bwd_body<T, 512>(a.mean, blk - a.nd - a.p[0].n - a.p[1].n, reinterpret_cast<float*>(smem));
+            mean_bwd_body<T, 512, true>(a.mean, blk - a.nd - a.p[0].n - a.p[1].n, reinterpret_cast<float*>(smem));
             return;
         }
         if ((unsigned)(blk - a.sd) < (unsigned)a.nd) {

@@ -446,7 +446,7 @@ template <int K>
 __global__ __launch_bounds__(512, 4) void dwconv_wgrad_f32t_pair_k(const WgF32Pair a) {
     if ((int)blockIdx.x >= a.p[0].n + a.p[1].n) {
         extern __shared__ uint32_t smem[];
-        return mean_bwd_body<float, 512>(a.mean, (int)blockIdx.x - a.p[0].n - a.p[1].n, reinterpret_cast<float*>(smem));
+        return mean_bwd_body<float, 512, false>(a.mean, (int)blockIdx.x - a.p[0].n - a.p[1].n, reinterpret_cast<float*>(smem));
     }
     const bool first = (int)blockIdx.x < a.p[0].n;
     const float *x = first ? a.p[0].x : a.p[1].x, *gy = first ? a.p[0].gy : a.p[1].gy;
@@ -491,7 +491,7 @@ int launch_wgrad_f32t_pair(const void* x0, const void* gy0, void* dw0, void* ws0
         const size_t need = mean_lds(mean->D, 512);
         if (need > 80 * 1024) return -1;   // (two workgroups on a compute unit)
         if (need > lds) lds = need;
-        a.mean = *mean, n += mean_bwd_workgroups(*mean);
+        a.mean = *mean, n += (long long)mean->B * mean_slices(mean->D);
     }
     if (n > 0x7fffffffLL) return -1;
     static std::once_flag once;

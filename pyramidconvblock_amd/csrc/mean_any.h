@@ -156,7 +156,7 @@ struct MeanJob {
     void* m;             // forward: the mean
     float* rowbias;      // forward: m Wp^T + bp + bo
     float *gs, *dmean;   // backward: the sums of the gradient, their product with Wp over P
-    bool shared;         // backward: kMeanImages images to a workgroup
+    bool shared;         // backward in dwconv_bwd3_k: kMeanImages images to a workgroup
 };
 
 inline int mean_slices(int D) { return cdiv(D, kMeanOut); }
@@ -265,9 +265,10 @@ __device__ __forceinline__ void mean_bwd_images(const MeanJob& j, int wg, float*
     }
 }
 
-template <typename T, int NT>
+// SHARED: where a job may have kMeanImages images to a workgroup (twice the instructions of one that never has).
+template <typename T, int NT, bool SHARED>
 __device__ __forceinline__ void mean_bwd_body(const MeanJob& j, int wg, float* sm) {
-    if (j.shared) mean_bwd_images<T, NT, kMeanImages>(j, wg, sm);   // (uniform)
+    if (SHARED && j.shared) mean_bwd_images<T, NT, kMeanImages>(j, wg, sm);   // (uniform)
     else mean_bwd_images<T, NT, 1>(j, wg, sm);
 }
 

@@ -818,7 +818,7 @@ __global__ __launch_bounds__(256) void gate_pair_colsum_bwd_k(const T* __restric
 template <typename T>
 __global__ __launch_bounds__(256) void mean_bwd_k(const MeanJob mean) {
     extern __shared__ float sm[];
-    mean_bwd_body<T, 256>(mean, blockIdx.x, sm);
+    mean_bwd_body<T, 256, false>(mean, blockIdx.x, sm);
 }
 
 // ---------------------------------------------------------------- per-image column sums and broadcast add
@@ -1535,7 +1535,7 @@ int gate_pair_colsum_bwd_launch(const void* gy, const void* xf, const void* xh, 
 
 int mean_bwd_launch(const MeanJob& mean, void* gbias, void* gbias2, void* gwp, int dtype, hipStream_t s) {
     const int D = mean.D;
-    const dim3 grid((unsigned)mean_bwd_workgroups(mean));
+    const dim3 grid((unsigned)(mean.B * mean_slices(D)));
     switch (dtype) {
         case kF32: hipLaunchKernelGGL((mean_bwd_k<float>), grid, dim3(256), mean_lds(D), s, mean); break;
         case kF16: hipLaunchKernelGGL((mean_bwd_k<f16_t>), grid, dim3(256), mean_lds(D), s, mean); break;
