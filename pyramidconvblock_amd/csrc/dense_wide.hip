@@ -502,68 +502,74 @@ void rows_tiles(long long N, int K, int NO, int& bm, int& bn) {
     if (bm == 128 && bn == 128 && K >= 256 && rounds(192) * 4 < rounds(128) * 3) bn = 192;
 }
 
-// Tiles and row ranges of the weight gradient: tiles of 64 where a width is no more than that, and the number of ranges that is
-// estimated to end first: a compute unit's stages (0.6 us one of 128 x 128 results, whether it has one workgroup or two in turn), and
-// the partials, written and read once more in fp32.  (With no more partials than are the operands' traffic, 512 workgroups at most,
-// [2128,920]^T [2128,464] was 32 workgroups of 34 stages.  us with the summation, bf16: that product 33.6 -> 15.3, [1568,1024]^T [1568,512]
-// 26.5 -> 16.4, [3136,768]^T [3136,384] 20.3 -> 14.8, [25088,384]^T [25088,192] 19.2 -> 16.5, [16384,1152]^T [16384,576] 42.3 and 42.6; fp32:
-// [2002,1032]^T [2002,516] 40.7 -> 31.6, [1000,512]^T [1000,256] 15.8 -> 9.5.)
+// Tiles and row ranges of the weight gradient: tiles of 64 where a width is no more than that, and the number of ranges whose product by
+// itself and with the input gradient, in the launch that they share (both make the same ranges, so that their results are the same), are
+// estimated to end first, the latter counting twice.  By itself a compute unit's stages, less each where workgroups take turns.  The shared launch,
+// where it is all on the chip at once: the most that a unit is dealt, in order and the ranges first; else all work evenly and part of a
+// range's and of a row tile's, which are the last ones.  In both the partials, written and read once more in fp32, and the start of a further round.
+// Prices fitted to 1320 random layers of 136 to 1152 channels with every number of ranges (us, MI355X): the ranges chosen take 2.1 % longer than the best
+// by themselves and 1.9 % in the shared launch, in fp32 3.1 and 1.9 % (there both cannot be had: [1038,704]^T [1038,352] 17.1 and 20.4 us with two
+// ranges, 14.3 and 26.4 with three, since a compute unit's matrix pipe serves one workgroup at a time and 256 are a round).
+// us by itself and shared, against 512 workgroups with no more partials than are the operands' traffic, and two stages in LDS: bf16
+// [2128,920]^T [2128,464] 29.8 -> 15.1, 34.0 -> 16.0, [1568,1024]^T [1568,512] 22.7 -> 14.3, 24.3 -> 15.6, [16384,1152]^T [16384,576] 36.7 -> 38.9, 59.0 -> 60.2;
+// fp32 [2002,1032]^T [2002,516] 40.3 -> 31.0, 58.5 -> 53.7, [1000,512]^T [1000,256] 15.4 -> 11.2, 15.7 -> 16.6.  1370 other random layers 1.14 and 1.13
+// times as fast in bf16, 1.09 and 1.04 in fp32 (of the shared launches one in 40 is more than 5 % slower in bf16, one in 23 in fp32).
 struct WgradPlan {
     int bm, bn, mt, nt, splits;
     long long kper;
 };
 WgradPlan wgrad_make_plan(long long N, int M, int NO, int es) {
-    WgradPlan p{M <= 64 ? 64 : 128, NO <= 64 ? 64 : 128, 0, 0, 0, 0};
+    const bool f32 = es == 4;
     const int bk = kRowBytes / es;
-    const double stage = es == 4 ? 0.5 / (64 * 64) : 0.6 / (128 * 128), partial = 8.0 * M * NO / 3.5e6;   // us: a result's stage, a range's partials
-    const double alone = es == 4 ? 1.3 : 1.0;   // (fp32: of one workgroup a compute unit)
-    double least;
-    auto cut = [&] {
-        p.mt = cdiv(M, p.bm), p.nt = cdiv(NO, p.bn);
-        const long long tiles = (long long)p.mt * p.nt, most = std::min(N / (2 * bk), std::max(1024 / tiles, 1LL));
-        long long best = 1;
-        for (long long s = 1; s <= most || s == 1; s += s < 16 ? 1 : s / 8) {
-            const long long inner = cdiv(cdiv(N, s), bk);
-            const double c = (double)cdiv(tiles * s, 256) * (tiles * s <= 256 ? alone : 1.0) * inner * p.bm * p.bn * stage + partial * s;
-            if (s == 1 || c < least) least = c, best = s;
+    // us: a result's stage of a compute unit's only workgroup, of one of several, and of the input gradient; a range's partials
+    const double area = f32 ? 64 * 64 : 128 * 128, only = (f32 ? 0.6 : 0.52) / area, several = (f32 ? 0.55 : 0.355) / area,
+                 row = (f32 ? 0.55 : 0.44) / area, partial = (f32 ? 2.0e-6 : 1.8e-6) * M * NO + (f32 ? 0.03 : 0.005);
+    const double uneven = f32 ? 1.0 : 1.3, end = f32 ? 0.25 : 0.4, last = 0.5;   // shares of a unit's most work, a range's, and a row tile's
+    const double again = f32 ? 0.6 : 1.0;   // us: the start of another round of workgroups
+    const long long resident = f32 ? 1024 : 512;
+    // no range longer than its 32-bit offsets reach (operands of more than 2 GiB, widths that alone fill the chip)
+    const long long reach = 0x7fffffffLL / ((long long)(M > NO ? M : NO) * es) / 64 * 64, fewest = reach > 0 ? (N + reach - 1) / reach : 1;
+    int rm = 64, rn = 64;
+    if (!f32) rows_tiles(N, M, NO, rm, rn);
+    const long long rows = (long long)cdiv(N, rm) * cdiv(NO, rn);
+    const double row_work = (double)cdiv(M, bk) * rm * rn * row;
+    auto shared = [&](long long blocks, double work) {   // (without the partials)
+        const long long all = blocks + rows;
+        const double even = (blocks * work * several + rows * row_work) / 256;
+        if (all > resident) return even + end * work * several + last * row_work + again * (cdiv(all, resident) - 1);
+        double most = 0;
+        for (const long long unit : {0LL, blocks % 256, all % 256}) {   // (units alike up to the next of these)
+            const long long ranges = (blocks + 255 - unit) / 256, n = (all + 255 - unit) / 256;
+            most = std::max(most, (ranges * work * several + (n - ranges) * row_work) * (n == 1 ? only / several : 1.0));
+        }
+        return std::max(even, most * uneven);
+    };
+    struct Choice {
+        WgradPlan p;
+        double alone;
+    };
+    auto best_of = [&](int bm, int bn) {
+        Choice best{};
+        double least = 0;
+        const long long mt = cdiv(M, bm), nt = cdiv(NO, bn), tiles = mt * nt, most = std::max(fewest, std::min(N / 64, 1024 / tiles));
+        const bool paired = f32 ? bm == 64 && bn == 64 : bm == 128 && bn == 128;
+        for (long long s = fewest; s <= most || s == fewest; s += s < 16 ? 1 : s / 8) {
+            const long long kper = ((N + s - 1) / s + 63) / 64 * 64, n = (N + kper - 1) / kper, blocks = tiles * n;
+            const double work = (double)(kper / bk) * bm * bn;
+            const double alone = work * (blocks <= 256 ? only : cdiv(blocks, 256) * several) + again * (cdiv(blocks, resident) - 1) + partial * n;
+            const double cost = paired ? 0.5 * alone + shared(blocks, work) + partial * n : alone;
+            if (best.p.splits != 0 && cost >= least) continue;
+            least = cost;
+            best = {{bm, bn, (int)mt, (int)nt, (int)n, kper}, alone};
         }
         return best;
     };
-    long long s = cut();
-    // fp32, bound by the matrix pipe and not by what the tiles read: smaller ones (which the shared launch takes) unless these are
-    // clearly faster
-    if (es == 4 && (p.bm > 64 || p.bn > 64)) {
-        const WgradPlan large = p;
-        const double before = least;
-        const long long was = s;
-        p.bm = p.bn = 64, s = cut();
-        if (least > 1.15 * before) p = large, s = was;
-    }
-    // no range longer than its 32-bit offsets reach (operands of more than 2 GiB, widths that alone fill the chip)
-    const long long most = 0x7fffffffLL / ((long long)(M > NO ? M : NO) * es) / 64 * 64;
-    const long long fewest = most > 0 ? (N + most - 1) / most : 1;
-    s = std::max(s, fewest);
-    auto cut_in = [&](long long n) {
-        p.kper = ((N + n - 1) / n + 63) / 64 * 64;
-        p.splits = (int)((N + p.kper - 1) / p.kper);
-    };
-    cut_in(s);
-    // The launch that it shares with the input gradient (both make the same ranges, so that their results are the same): fewer, where it then is a round
-    // less, of two workgroups a compute unit (fp32: one, the matrix pipe being what bounds them), and the stages that the ranges are longer by are
-    // fewer than those of an input gradient's workgroup, which would be that round.  Training steps as graphs, filter 5, us, without and with this: bf16
-    // [1,64,64,1152] 149.9 and 131.9, [1,88,88,672] 132.5 and 122.9, [3,57,61,400] 119.6 and 111.5, but [11,51,50,200], where a range would have 12 stages
-    // for 7 and the others have 2 and 4, 114.4 and 116.5; fp32 [32,11,11,552] 204.3 and 196.3, [2,28,28,744] 155.1 and 148.3, [6,15,15,352] 109.4 and 105.4.
-    if (es == 2 ? p.bm == 128 && p.bn == 128 : p.bm == 64 && p.bn == 64 && (M > 256 || NO > 256)) {
-        int bm = 64, bn = 64;
-        if (es == 2) rows_tiles(N, M, NO, bm, bn);
-        const long long round = es == 2 ? 512 : 256, tiles = (long long)p.mt * p.nt, rows = (long long)cdiv(N, bm) * cdiv(NO, bn), was = p.kper,
-                        fit = (round * (cdiv(rows + tiles * p.splits, round) - 1) - rows) / tiles;
-        if (fit >= fewest) {
-            cut_in(fit);
-            if ((p.kper - was) / bk * cdiv(tiles * fit, round) >= cdiv(M, bk)) cut_in(s);
-        }
-    }
-    return p;
+    const Choice large = best_of(M <= 64 ? 64 : 128, NO <= 64 ? 64 : 128);
+    if (!f32) return large.p;
+    // fp32, bound by the matrix pipe and not by what the tiles read: tiles of 64 (which the shared launch takes) unless larger ones
+    // are clearly faster
+    const Choice small = best_of(64, 64);
+    return small.alone > 1.15 * large.alone ? large.p : small.p;
 }
 
 // (asked for five times a call, the workspace's size among them, and microseconds to make)

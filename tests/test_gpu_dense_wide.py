@@ -36,7 +36,7 @@ def test_dense_wide_layers(dtype, K, NO, N, P):
 @pytest.mark.parametrize("K,NO", [(4, 4), (132, 36), (100, 200), (128, 64), (64, 128), (260, 576)])
 @pytest.mark.parametrize("N,P", [(1, 1), (63, 7), (1000, 250), (4097, 4097), (70001, 35001)])
 def test_dense_wide_fp32_layers(K, NO, N, P):
-    """Every tile (70001 rows: 128 high), remainders of 4 in both widths, ranges of rows that end within a stage."""
+    """Remainders of 4 in both widths, ranges of rows that end within a stage, and many of them."""
     _layers(torch.float32, K, NO, N, P)
 
 
@@ -58,8 +58,8 @@ def test_few_workgroups_of_both_products(oracle, dim, shape):
 @pytest.mark.parametrize("dtype,dim,shape", [(torch.bfloat16, 400, (3, 57, 61, 400)), (torch.bfloat16, 1048, (1, 64, 67, 1048)), (torch.bfloat16, 200, (11, 51, 50, 200)),
                                              (torch.float32, 352, (6, 15, 15, 352)), (torch.float32, 872, (3, 21, 20, 872)), (torch.float32, 384, (3, 12, 15, 384))])
 def test_row_ranges_that_make_room(oracle, dtype, dim, shape):
-    """Fewer row ranges for the launch of both products to be a round less, by one (400) and more (1048; 352, one round; 872, two), and as many as are estimated
-    best by themselves (200, 384)."""
+    """Row ranges that are fewer than a weight gradient by itself would have: launches of both products that the chip holds at once (400; 352, 384 and 872), and
+    longer ones (200; 1048, one of its layers)."""
     _block_case(oracle, dim, 3, shape, dtype)
 
 
