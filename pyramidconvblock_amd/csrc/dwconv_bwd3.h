@@ -4,7 +4,7 @@
 // launch gaps in between.  Every problem runs in the tile that its width fills better: by template where the input
 // gradient's is the wide one, the pool halved the extents and no mean branch rides along (each workgroup starts with one
 // problem's arguments), at run time per problem elsewhere.  (With bands of one image the template was 0.2 to 1.2 us faster; with runs
-// both take as long: [32,56,56,64] filter 9 26.0 and 25.9 us, 13 28.6 and 28.7, 17 50.0 and 49.8, [128,56,56,64] filter 13 76.0 and 76.5.)
+// both take as long: [32,56,56,64] filter 9 26.0 and 25.9 us, 13 28.6 and 28.7, [128,56,56,64] filter 13 76.0 and 76.5.)
 // The kernel template and its per-filter-size launcher; dwconv_bwd3_k<K>.hip instantiate it, one file per size.
 #pragma once
 #include "dwconv_fwd2.h"
@@ -157,8 +157,9 @@ static Bwd3Plan bwd3_plan(int B, const TzGeom& gd, int npcd, const WgPhPlan& p0,
 // and 87).  Prices fitted to both of 160 random shapes with cold buffers.  What they do not see: in several rounds, runs of either side longer than
 // by itself leave both sides short of memory all the time (with the estimate 0 to 10 % ahead [97,10,11,896] filter 9 64.7 -> 71.6, [75,12,12,624]
 // filter 7 42.0 -> 44.8; as long as by itself, 220 such plans 0.98 to 1.5 times as fast), so these have to be estimated further ahead.
-// (One round of filters 3 and 5 alike would lose more than it gains: [92,7,7,448] filter 5 29.0 for 26.8 apart, but [27,29,28,640] 43.6 for 49.4,
-// [42,11,11,1008] filter 3 27.1 for 30.5.)  300 other shapes take 1.18 times less, the slowest 1.04 times more ([11,64,64,432] filter 7).
+// Filters 3 and 5 in one round with runs of the weight gradient more than two and a half times as long as by itself are estimated too short
+// ([92,7,7,448] filter 5, three times: 26.6 apart, 28.9 together).
+// An estimate less than 6 % ahead is as often behind ([11,64,64,432] filter 7 59.1 and 61.4, [124,8,8,432] filter 5 33.3 and 31.4).
 // us with the summation, apart and together:
 // [8,64,64,1152] filter 9 84 -> 70, [32,28,28,256] filter 13 33.8 -> 28.8, [2,20,20,64] filter 7 13.2 -> 8.6, [11,74,74,688] filter 9 137 -> 109.
 template <int K>
@@ -172,7 +173,7 @@ static Bwd3Plan bwd2_plan(const TzGeom& gd, int npcd, const WgPhPlan& p0) {
     // gradient's; their steps side by side, in one round and in several (which are full of either side most of the time); what an
     // estimate of one round has to be ahead by, and one of several with longer runs than by itself (launch_makespan adds its own to all of these)
     constexpr double kStartD = 5.5, kStepD = K <= 9 ? 1.25 : K <= 13 ? 1.4 : 1.2, kStartF = kWgPhStart, kStepF = K <= 9 ? 1.25 : K <= 15 ? 1.8 : 2.5,
-                     kLaunch = 2.8, kShareOne = K <= 5 ? 1.15 : K <= 9 ? 1.17 : 1.2, kShareMore = K <= 5 ? 1.15 : K <= 9 ? 1.1 : 1.2, kAhead = 1.04,
+                     kLaunch = 2.8, kShareOne = K <= 5 ? 1.15 : K <= 9 ? 1.17 : 1.2, kShareMore = K <= 5 ? 1.15 : K <= 9 ? 1.1 : 1.2, kAhead = 1.06,
                      kAheadLonger = 1.1;
     const int ni = 16 / npcd;
     std::vector<LaunchCut> cuts[2];
@@ -200,6 +201,7 @@ static Bwd3Plan bwd2_plan(const TzGeom& gd, int npcd, const WgPhPlan& p0) {
     for (const LaunchCut& dc : cuts[0])
         for (const LaunchCut& fc : cuts[1]) {
             const bool single = dc.count + fc.count <= 256;
+            if (K <= 5 && single && fc.count * 5 < p0.nblocks * 2) continue;
             const double share = single ? kShareOne : kShareMore;
             const LaunchCut d{dc.n, kStartD + share * dc.cost, dc.count}, f{fc.n, kStartF + share * fc.cost, fc.count};
             const LaunchCut* const pick[2] = {&d, &f};

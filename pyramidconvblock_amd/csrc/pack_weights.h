@@ -1,5 +1,5 @@
 // The four weights of a block whose halves of inner channels are padded to a multiple of 8 (block_any.hip), in the padded
-// layout, eight values to a thread: conv_up's rows, conv_out's columns, the filters' channels.  A few hundred KB at most: a launch of its
+// layout, eight values to a thread: conv_up's rows, conv_out's columns, the filters' channels.  A few hundred KB, 2.6 MB at 1144 channels: a launch of its
 // own was latency (us of inference as a graph, with it and in the launch of the pool, conv_up reading its weights as they are given:
 // [4,33,33,104] filter 9 37.1 -> 32.7, [3,57,61,200] filter 9 40.7 -> 36.4, [32,14,14,968] filter 3 71.2 -> 66.6).
 #pragma once
