@@ -89,10 +89,20 @@ __global__ __launch_bounds__(256) void avgpool_fwd_k(const T* __restrict__ x, T*
     if (idx < total) avgpool_fwd_item<T, VEC>(x, y, H, W, C, h, w, idx);
 }
 
-// The same with the column sums of another tensor (mean_any.h) and the packing of weights (pack_weights.h) in the first
-// workgroups: all are bandwidth.
+// The same with the column sums of another tensor (mean_any.h) in the first workgroups: both are bandwidth.
 template <typename T, int VEC>
-__global__ __launch_bounds__(256) void avgpool_with_k(const T* __restrict__ x, T* __restrict__ y, int H, int W, int C, int h,
+__global__ __launch_bounds__(256) void avgpool_colsum_k(const T* __restrict__ x, T* __restrict__ y, int H, int W, int C,
+                                                        int h, int w, long long total, const ColsumJob sums, int nsums) {
+    extern __shared__ float sm[];
+    if ((int)blockIdx.x < nsums) return colsum_body<T>(sums, blockIdx.x, sm);
+    const long long idx = (long long)(blockIdx.x - nsums) * blockDim.x + threadIdx.x;
+    if (idx < total) avgpool_fwd_item<T, VEC>(x, y, H, W, C, h, w, idx);
+}
+
+// And with the packing of weights (pack_weights.h) behind those, for blocks that pad their channels: a kernel of its own, since its
+// arguments and the branch cost the others 0.1 us.
+template <typename T, int VEC>
+__global__ __launch_bounds__(256) void avgpool_pack_k(const T* __restrict__ x, T* __restrict__ y, int H, int W, int C, int h,
                                                       int w, long long total, const ColsumJob sums, int nsums, const PackArgs pack, int npack) {
     extern __shared__ float sm[];
     if ((int)blockIdx.x < nsums) return colsum_body<T>(sums, blockIdx.x, sm);
@@ -1368,12 +1378,19 @@ int avgpool_with_launch(const void* a, void* xp, int B, int H, int W, int C, int
     unsigned blocks;
     if (!grid_for(total, &blocks) || (unsigned long long)blocks + nsums + npack > 0x7fffffffULL) return 1;
     const size_t lds = sums ? 256 * 16 / esize(dtype) * sizeof(float) : 0;
-#define CALL(T, V)                                                                                                                       \
-    hipLaunchKernelGGL((avgpool_with_k<T, V>), dim3(blocks + nsums + npack), dim3(256), lds, s, (const T*)a, (T*)xp, H, W, C, h, w, total, \
-                       sums ? *sums : ColsumJob{}, nsums, pack ? *pack : PackArgs{}, npack);
-    PDW_TYPE_SWITCH(dtype, vec, CALL)
+    if (!pack) {
+#define CALL(T, V) hipLaunchKernelGGL((avgpool_colsum_k<T, V>), dim3(blocks + nsums), dim3(256), lds, s, (const T*)a, (T*)xp, H, W, C, h, w, total, *sums, nsums);
+        PDW_TYPE_SWITCH(dtype, vec, CALL)
 #undef CALL
-    return check_launch("avgpool_with");
+        return check_launch("avgpool_colsum");
+    }
+    if (dtype == kF32) return set_error("packed weights are of 16-bit types"), 1;
+#define CALL(T, V)                                                                                                                       \
+    hipLaunchKernelGGL((avgpool_pack_k<T, V>), dim3(blocks + nsums + npack), dim3(256), lds, s, (const T*)a, (T*)xp, H, W, C, h, w, total, \
+                       sums ? *sums : ColsumJob{}, nsums, *pack, npack);
+    if (dtype == kF16) PDW_VEC_SWITCH(f16_t, vec, CALL) else PDW_VEC_SWITCH(bf16_t, vec, CALL)
+#undef CALL
+    return check_launch("avgpool_pack");
 }
 
 int avgpool_bwd_launch(const void* gy, void* gx, int B, int H, int W, int C, int h, int w, int accumulate, int dtype,
