@@ -773,7 +773,7 @@ __global__ __launch_bounds__(256, 2) void dense_rows_rider_k(const T* __restrict
     extern __shared__ uint32_t dsm[];
     const int nride = (int)gridDim.x - nblocks;
     if ((int)blockIdx.x < nride) {
-        reduce_jobs_block<true>(jobs, blockIdx.x, reinterpret_cast<float*>(dsm));
+        reduce_jobs_block<kLanesRiding>(jobs, blockIdx.x, reinterpret_cast<float*>(dsm));
     } else {
         dense_rows_body<T, KMAJOR, false, SK, SNO>(X, W, bias, rowbias, Y, nullptr, N, K, NO, P, nkt, nnt,
                                                    blockIdx.x - nride, nblocks, dsm);
@@ -954,7 +954,7 @@ __global__ __launch_bounds__(256, 2) void dense_wgrad_rider_k(const T* __restric
                                                               int nblocks, const ReduceJobs jobs) {
     extern __shared__ uint32_t dsm[];
     if ((int)blockIdx.x >= nblocks) {
-        reduce_jobs_block<true>(jobs, blockIdx.x - nblocks, reinterpret_cast<float*>(dsm));
+        reduce_jobs_block<kLanesRiding>(jobs, blockIdx.x - nblocks, reinterpret_cast<float*>(dsm));
         return;
     }
     dense_wgrad_body<T, MT, NT, EXACT>(A, Bm, part, N, M, NO, nblocks, dsm);

@@ -120,16 +120,17 @@ __global__ __launch_bounds__(256) void dwconv_wgrad_direct(const T* __restrict__
     }
 }
 
-template <typename T>
+template <typename T, ReduceLanes LANES>
 __global__ __launch_bounds__(256) void wgrad_reduce_parts(const float* __restrict__ part, T* __restrict__ dw,
                                                           int nparts, int n, int vec, int ql) {
     __shared__ float red[kReduceLds];
-    reduce_parts_any<T>(part, dw, nparts, n, blockIdx.x, vec, ql, red);
+    reduce_parts_any<T, LANES>(part, dw, nparts, n, blockIdx.x, vec, ql, red);
 }
 
+template <ReduceLanes LANES>
 __global__ __launch_bounds__(256) void wgrad_reduce_many(const ReduceJobs jobs) {
     __shared__ float red[kReduceLds];
-    reduce_jobs_block<false>(jobs, blockIdx.x, red);
+    reduce_jobs_block<LANES>(jobs, blockIdx.x, red);
 }
 
 // Deferred mode (per host thread): between reduce_defer_begin and reduce_defer_flush the reductions are only
@@ -143,8 +144,8 @@ void reduce_defer_compact(int seg, int val) { t_seg = t_defer ? seg : 0, t_val =
 // Part lanes of a stand-alone summation: 32 when 8 would need more than one round of loads; one when that has no more than two and the
 // outputs are many (training steps as graphs, us: [4,64,64,1152] filter 13 fp16, 11 parts of 660 000 outputs, 336.5 -> 328.5, [102,10,13,608]
 // filter 9 bf16 230 -> 223, [20,14,14,1024] filter 5 135 -> 130; from 8192 outputs on 225 and 132).
-static int standalone_part_lanes(int nparts, int n) {
-    if (nparts <= 32 && n >= 65536) return 1;
+static int standalone_part_lanes(int nparts, int n, int vec) {
+    if (nparts <= 32 && n >= 65536 && vec == kReduceVec) return 1;
     return nparts > 128 ? 32 : 8;
 }
 
@@ -153,15 +154,17 @@ static int standalone_part_lanes(int nparts, int n) {
 int reduce_jobs_launch(const ReduceJobs& recorded, hipStream_t s) {
     if (recorded.njobs == 0) return 0;
     ReduceJobs jobs = recorded;
+    bool few = false;
     for (int j = 0; j < jobs.njobs; ++j) {
         int nb = recorded.first_block[j + 1] - recorded.first_block[j];
         if (recorded.vec[j] != 0) {
-            jobs.ql[j] = standalone_part_lanes(jobs.nparts[j], jobs.n[j]);
+            jobs.ql[j] = standalone_part_lanes(jobs.nparts[j], jobs.n[j], jobs.vec[j]);
+            few = few || jobs.ql[j] == 1;
             nb = cdiv(jobs.n[j], reduce_block_outputs(jobs.vec[j], jobs.ql[j]));
         }
         jobs.first_block[j + 1] = jobs.first_block[j] + nb;
     }
-    hipLaunchKernelGGL(wgrad_reduce_many, dim3(jobs.first_block[jobs.njobs]), dim3(256), 0, s, jobs);
+    hipLaunchKernelGGL(few ? wgrad_reduce_many<kLanesFew> : wgrad_reduce_many<kLanesAlone>, dim3(jobs.first_block[jobs.njobs]), dim3(256), 0, s, jobs);
     return check_launch("wgrad_reduce_many");
 }
 
@@ -297,8 +300,8 @@ int wgrad_reduce_launch(const float* part, void* dw, int nparts, int n, hipStrea
         t_jobs.first_block[j + 1] = t_jobs.first_block[j] + cdiv(n, reduce_block_outputs(vec, 8));
         return 0;
     }
-    const int ql = standalone_part_lanes(nparts, n);
-    hipLaunchKernelGGL((wgrad_reduce_parts<T>), dim3(cdiv(n, reduce_block_outputs(vec, ql))), dim3(256), 0, s, part,
+    const int ql = standalone_part_lanes(nparts, n, vec);
+    hipLaunchKernelGGL((ql == 1 ? wgrad_reduce_parts<T, kLanesFew> : wgrad_reduce_parts<T, kLanesAlone>), dim3(cdiv(n, reduce_block_outputs(vec, ql))), dim3(256), 0, s, part,
                        (T*)dw, nparts, n, vec, ql);
     return check_launch("wgrad_reduce_parts");
 }
