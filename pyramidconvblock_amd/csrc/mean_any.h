@@ -162,8 +162,8 @@ struct MeanJob {
 inline int mean_slices(int D) { return cdiv(D, kMeanOut); }
 // Whether a workgroup of the backward takes four images: where one each would make more workgroups than the convolutions' shared
 // launch, which holds one workgroup a compute unit, has units left for.  They read the layer's weight once and take less than twice as long.  Training
-// steps, us: [102,10,13,608] filter 9 bf16 (1020 workgroups -> 260) 248 -> 228, [40,7,7,1152] filter 5 184 -> 151, [20,14,14,1024] filter 5 (320
-// -> 80) 147 -> 137, [64,20,20,256] (256 -> 64) 117 -> 113; with eight images [12,28,28,768] (144 -> 24) 156 -> 179.
+// steps, us: [102,10,13,608] filter 9 bf16 (1020 workgroups -> 260) 249 -> 230, [40,7,7,1152] filter 5 184 -> 151, [20,14,14,1024] filter 5 (320
+// -> 80) 147 -> 138, [64,20,20,256] (256 -> 64) 117 -> 113; with eight images [12,28,28,768] (144 -> 24) 156 -> 179.
 inline bool mean_shared(int B, int D) { return (long long)B * mean_slices(D) > 192 && D > 128 && D <= 2048; }
 inline int mean_bwd_workgroups(const MeanJob& j) { return cdiv(j.B, j.shared ? kMeanImages : 1) * mean_slices(j.D); }
 // sums; scratch of 32 bytes a thread (backward, 16-bit) or less
