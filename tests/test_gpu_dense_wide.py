@@ -40,6 +40,14 @@ def test_dense_wide_fp32_layers(K, NO, N, P):
     _layers(torch.float32, K, NO, N, P)
 
 
+# (a weight gradient's tiles are its output's width by its input's)
+@pytest.mark.parametrize("K,NO,N", [(448, 780, 848), (448, 780, 849), (4, 968, 5951), (28, 1048, 6829), (968, 4, 5951), (1048, 28, 6829)])
+def test_fp32_weight_gradients_in_larger_tiles(K, NO, N):
+    """128 x 128 and 128 x 64 results, where they are estimated to end clearly before 64 x 64 (the last two stay there): remainders of 4 and of
+    a stage."""
+    _layers(torch.float32, K, NO, N, N)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("K,NO", [(376, 136), (384, 64), (392, 72), (448, 920), (1152, 144)])
 @pytest.mark.parametrize("N", [1, 65, 191, 320, 2128])
