@@ -166,13 +166,26 @@ int forward(const Shape& s, const Saved& v, const void* x, const Weights& given,
     // conv_up, where its kernel can with the sums of x per row tile (for the mean branch) and the 2x2 pool of its result
     const float* parts = nullptr;
     int nparts = 0;
-    bool pooled = false;
+    bool pooled = false, first = false;
+    const bool any_mean = mean_any_ok(x, w_pool, v.m, s.D, s.es);
     if (two && !s.padded()) {
         const int r = pdw_dense_fwd_colsum_pool(x, w_up, nullptr, v.a, v.xparts, v.xp, s.B, s.H, s.W, s.D, s.I, dt, stream);
         if (r != 0 && r != 3) return r;
         pooled = r == 0;
     }
-    if (s.padded()) {
+    // wide layers and fp32 on exact halves: with the pool, the sums of x and the packing, in place of the pool's launch
+    if (!pooled && s.exact && any_mean && !pdw_dense_colsum_supported(s.D, s.I, dt)) {
+        ColsumJob sums;
+        if (dense_wide_first_plan(&sums, s.N, s.D, s.I, s.B, s.P, dt)) {
+            sums.x = x, sums.part = (float*)v.ws;
+            const int r = dense_wide_first_launch(x, given.up, v.a, v.xp, s.w, s.N, s.D, s.I, sums, s.padded() ? &pack : nullptr, dt, st);
+            if (r != 0 && r != -1) return r;
+            if (r == 0) pooled = first = true, unpacked = false, parts = sums.part, nparts = sums.n;
+        }
+    }
+    if (first) {
+        // (done)
+    } else if (s.padded()) {
         const RowMap map{s.Gp, s.G};
         float* const sums = rows_whole_tiles(s) && pdw_dense_colsum_supported(s.D, s.I, dt) ? v.xparts : nullptr;
         int r = dense_rows_launch(x, given.up, 0, nullptr, nullptr, v.a, s.N, s.D, s.I, s.P, dt, st, sums, nullptr, &map);
@@ -193,7 +206,6 @@ int forward(const Shape& s, const Saved& v, const void* x, const Weights& given,
         return e;
     }
     // the pool, with the sums of x where conv_up's kernel did not leave any
-    const bool any_mean = mean_any_ok(x, w_pool, v.m, s.D, s.es);
     auto pool = [&]() -> int {
         const PackArgs* const with = unpacked ? &pack : nullptr;
         unpacked = false;
@@ -218,11 +230,12 @@ int forward(const Shape& s, const Saved& v, const void* x, const Weights& given,
         convs = r == 0;
         if (!convs)
             if (int e = pdw_dwconv_fwd(v.a, w_dw0, v.c0, s.B, s.H, s.W, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, dt, stream)) return e;
-    } else if ((parts || !any_mean) && !unpacked) {
+    } else if ((parts || !any_mean) && !unpacked && !pooled) {
         if (int e = pdw_dwconv_fwd_pool(v.a, w_dw0, v.c0, v.xp, s.B, s.H, s.W, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, s.h, s.w, dt, stream))
             return e;
     } else {
-        if (int e = pool()) return e;
+        if (!pooled)
+            if (int e = pool()) return e;
         const int r = dt == kF32 ? dwconv_f32t_pair_launch(v.a, w_dw0, v.c0, s.H, s.W, v.xp, w_dw1, v.c1, s.h, s.w, s.B, s.I, s.K, st)
                                  : dwconv_fwd2_launch(v.a, w_dw0, v.c0, v.xp, w_dw1, v.c1, s.B, s.H, s.W, s.h, s.w, s.I, s.K, dt, st);
         if (r != 0 && r != -1) return r;

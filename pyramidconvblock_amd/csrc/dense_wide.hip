@@ -27,6 +27,7 @@
 #include "common.h"
 #include "dense_any_wgrad.h"
 #include "kernels.h"
+#include "mean_any.h"
 #include "reduce_parts.h"
 #include "tile_common.h"
 
@@ -62,6 +63,27 @@ __device__ __forceinline__ v16f mfma(v8s a, v8s b, v16f c, float) {
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void* p, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
 }
+
+// Rows of a tensor [images][2 h][2 w][] taken by quads, the 2 x 2 pixels of one pooled pixel: row 4 q + 2 dy + dx is pixel (2 y + dy, 2 x + dx)
+// of pooled pixel q, so that a tile of rows holds whole quads whatever the extents are.  (Images are stacked: H = 2 h.)
+struct QuadArgs {
+    void* pool;       // [images][h][w][]: the mean of each quad's results
+    int w;
+    uint32_t magic;   // 2^32 / w rounded up (w > 1): x / w for x w < 2^32
+};
+struct QuadRows {
+    uint32_t pix0, x0;   // first pixel of the row pair of the tile's first quad, and that quad's place in it
+    int w;
+    uint32_t magic;
+    __device__ __forceinline__ void init(const QuadArgs& g, long long quad0) {
+        const uint32_t pair = (uint32_t)quad0 / (uint32_t)g.w;
+        w = g.w, magic = g.magic, x0 = (uint32_t)quad0 - pair * (uint32_t)w, pix0 = 4 * pair * (uint32_t)w;
+    }
+    __device__ __forceinline__ uint32_t pixel(int row) const {   // of the tile's row, from pix0
+        const uint32_t t = x0 + (uint32_t)(row >> 2), dy = w == 1 ? t : __umulhi(t, magic), x = t - dy * (uint32_t)w;
+        return (2 * dy + (uint32_t)(row >> 1 & 1)) * 2 * (uint32_t)w + 2 * x + (uint32_t)(row & 1);
+    }
+};
 
 // One operand of a tile: R results wide, kBK inner values per stage, staged by the workgroup's 256 threads.
 // TR = false: stored [result][inner] (pitch ld): LDS rows of 128 bytes, 8 pieces each, piece c of row r at c ^ (r / 2 % 8).
@@ -118,6 +140,19 @@ struct Operand {
             const int res = (int)r0 + row, hi = res >= map.seg, r = res - hi * map.seg;
             kc[j] = c * VE;
             off[j] = r < map.val && res < nres ? (uint32_t)((r + hi * map.val) * ld + c * VE) * ES : kPast;
+        }
+    }
+    // rows by quads from `quad0` on, of `quads`
+    __device__ __forceinline__ void init(const char* p, int ld, const QuadRows& rows, long long quad0, long long quads, int inner) {
+        static_assert(!TR, "stored by results");
+        const long long bytes = (4 * quads - rows.pix0) * ld * ES;
+        rsrc = rsrc_of(p + (long long)rows.pix0 * ld * ES, (uint32_t)(bytes < 0x7fffffffLL ? bytes : 0x7fffffffLL));
+        step = kRowBytes;
+#pragma unroll
+        for (int j = 0; j < NL; ++j) {
+            const int slot = j * 256 + (int)threadIdx.x, row = slot / CPR, c = swz(row, slot % CPR);
+            kc[j] = c * VE;
+            off[j] = quad0 + (row >> 2) < quads ? (rows.pixel(row) * (uint32_t)ld + (uint32_t)(c * VE)) * ES : kPast;
         }
     }
     // requests stage `st` (inner values left from its start: left) into buf
@@ -223,8 +258,9 @@ struct WideArgs {
 template <typename T, int BM, int BN>
 constexpr int kWideOccupancy = sizeof(T) == 4 ? (BM * BN <= 64 * 64 ? 4 : BM * BN <= 128 * 64 ? 3 : 2) : 2;
 
-template <typename T, int BM, int BN, bool TA, bool TB, bool PART, int STAGES = 2, bool MAP = false>
-__device__ __forceinline__ void wide_gemm_body(const WideArgs& g, int blk, int nblk) {
+// QUAD: a's rows by quads (M of them), and the mean of each quad's results as they are stored.
+template <typename T, int BM, int BN, bool TA, bool TB, bool PART, int STAGES = 2, bool MAP = false, bool QUAD = false>
+__device__ __forceinline__ void wide_gemm_body(const WideArgs& g, int blk, int nblk, const QuadArgs& qa = QuadArgs{}) {
     typedef Operand<T, BM, TA> OpA;
     typedef Operand<T, BN, TB> OpB;
     constexpr int BK = kBK<T>, KK = 4;          // inner values of a stage; fragments of it
@@ -244,7 +280,13 @@ __device__ __forceinline__ void wide_gemm_body(const WideArgs& g, int blk, int n
     const long long kb = sp * g.kper, ke = kb + g.kper < g.Kd ? kb + g.kper : g.Kd;
     OpA a;
     OpB b;
-    a.init((const char*)g.a, g.lda, m0, g.M, kb, ke);
+    QuadRows quad;
+    if constexpr (QUAD) {
+        quad.init(qa, m0 / 4);
+        a.init((const char*)g.a, g.lda, quad, m0 / 4, g.M / 4, (int)g.Kd);
+    } else {
+        a.init((const char*)g.a, g.lda, m0, g.M, kb, ke);
+    }
     // (a kernel of its own for a RowMap: chosen inside one, the two cost other layers up to 0.6 us of 10)
     if constexpr (MAP) b.init((const char*)g.b, g.ldb, n0, g.N, kb, ke, g.map);
     else b.init((const char*)g.b, g.ldb, n0, g.N, kb, ke);
@@ -408,12 +450,29 @@ __device__ __forceinline__ void wide_gemm_body(const WideArgs& g, int blk, int n
         }
         __syncthreads();
         constexpr int CPR = BN / VE;
+        if constexpr (QUAD) {   // a quad's pieces by one thread, and their mean in avgpool_fwd_item's order
 #pragma unroll
-        for (int j = 0; j < BM * CPR / 256; ++j) {
-            const int s = j * 256 + tid, row = s / CPR, c = s % CPR;
-            if (m0 + row < g.M && n0 + c * VE < g.N)
-                *reinterpret_cast<uint4*>((T*)g.y + (m0 + row) * g.N + n0 + c * VE) =
-                    *reinterpret_cast<const uint4*>(tile + row * TP + c * VE);
+            for (int s = tid; s < BM / 4 * CPR; s += 256) {
+                const int row = s / CPR * 4, c = s % CPR;
+                if (m0 + row >= g.M || n0 + c * VE >= g.N) continue;
+                T* const y = (T*)g.y + (quad.pix0 + (long long)quad.pixel(row)) * g.N + n0 + c * VE;
+                ChanVec<T, VE> v[4];
+                float o[VE];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = *reinterpret_cast<const ChanVec<T, VE>*>(tile + (row + r) * TP + c * VE);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) *reinterpret_cast<ChanVec<T, VE>*>(y + (long long)((r >> 1) * 2 * quad.w + (r & 1)) * g.N) = v[r];
+#pragma unroll
+                for (int e = 0; e < VE; ++e) o[e] = (((to_f32(v[0].v[e]) + to_f32(v[1].v[e])) + to_f32(v[2].v[e])) + to_f32(v[3].v[e])) * 0.25f;
+                store_f32<T, VE>((T*)qa.pool + ((m0 + row) / 4) * g.N + n0 + c * VE, o);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < BM * CPR / 256; ++j) {
+                const int s = j * 256 + tid, row = s / CPR, c = s % CPR;
+                if (m0 + row < g.M && n0 + c * VE < g.N)
+                    *reinterpret_cast<uint4*>((T*)g.y + (m0 + row) * g.N + n0 + c * VE) = *reinterpret_cast<const uint4*>(tile + row * TP + c * VE);
+            }
         }
     }
 }
@@ -421,6 +480,32 @@ __device__ __forceinline__ void wide_gemm_body(const WideArgs& g, int blk, int n
 template <typename T, int BM, int BN, bool TA, bool TB, bool PART, int STAGES, bool MAP = false>
 __global__ __launch_bounds__(256, (STAGES == 2 ? kWideOccupancy<T, BM, BN> : 1)) void wide_gemm_k(WideArgs g) {
     wide_gemm_body<T, BM, BN, TA, TB, PART, STAGES, MAP>(g, blockIdx.x, gridDim.x);
+}
+
+// The first layer of a block whose pooled extents are exact halves: the pool of its result in the product's store, where it lies in LDS
+// anyway (its rows go by quads for that), and the column sums of its input (mean_any.h) by workgroups of their own behind the
+// product's.  Instead of a launch that reads both again and of its start-up: what bounds it is the product (matrix pipe or HBM), the pool and
+// the rows' order cost 2 us of 30, the sums 1 to 4.  us, the product and that launch -> this: [100352,128] -> 64 fp32 23.6 + 13.0 -> 28.7;
+// [25600,400] -> 200 fp32 53.1 + 12.9 -> 53.3; [16384,1152] -> 576 fp16 29.4 + 11.5 -> 30.8; [100352,256] -> 128 bf16 20.4 + 14.2 -> 25.2;
+// [3200,640] -> 320 8.3 + 4.0 -> 9.4; [2048,64] -> 32 fp32 4.5 + 2.9 -> 5.4.  Where the pool needs a launch of its own (odd extents) the sums stay
+// there: [10431,200] -> 100 fp32 11.2 + 6.1, riding here 12.2 + 5.4; [1500,920] -> 464 bf16 10.4 + 5.2 and 14.7 + 5.1 (two stages, not four).
+template <typename T, int BM, int BN, int STAGES>
+__global__ __launch_bounds__(256, (STAGES == 2 ? kWideOccupancy<T, BM, BN> : 1)) void wide_first_k(WideArgs g, QuadArgs qa, ColsumJob sums, int nrows) {
+    extern __shared__ __align__(16) char dsm[];
+    const int blk = blockIdx.x;
+    if (blk < nrows) wide_gemm_body<T, BM, BN, false, false, false, STAGES, false, true>(g, blk, nrows, qa);
+    else colsum_body<T>(sums, blk - nrows, (float*)dsm);
+}
+
+// With the weights by a RowMap, and their packing (pack_weights.h) last.
+template <typename T, int BM, int BN, int STAGES>
+__global__ __launch_bounds__(256, (STAGES == 2 ? kWideOccupancy<T, BM, BN> : 1)) void wide_first_pack_k(WideArgs g, QuadArgs qa, ColsumJob sums, int nrows,
+                                                                                                     int nsums, PackArgs pack) {
+    extern __shared__ __align__(16) char dsm[];
+    const int blk = blockIdx.x;
+    if (blk < nrows) wide_gemm_body<T, BM, BN, false, false, false, STAGES, true, true>(g, blk, nrows, qa);
+    else if (blk < nrows + nsums) colsum_body<T>(sums, blk - nrows, (float*)dsm);
+    else pack_weights_body(pack, blk - nrows - nsums);
 }
 
 // Both products that read the gradient of a layer's output, as one launch: the weight gradient's nw workgroups (tiles of WM x WN
@@ -634,6 +719,74 @@ int dense_wide_rows_launch(const void* x, const void* w, int w_kmajor, const voi
 #undef PDW_WIDE_T
 #undef PDW_WIDE2_T
 #undef PDW_WIDE_S
+}
+
+namespace {
+
+template <typename T, int BM, int BN, int STAGES>
+int first_go(const WideArgs& g, const QuadArgs& qa, const ColsumJob& sums, const PackArgs* pack, hipStream_t s) {
+    constexpr size_t stages = wide_lds<T, BM, BN, false, STAGES>(), red = 256 * 16 / sizeof(T) * sizeof(float), lds = stages > red ? stages : red;
+    const long long nrows = (long long)g.mt * g.nt, nsums = colsum_workgroups(sums), all = nrows + nsums + (pack ? pack_workgroups(*pack) : 0);
+    if (all > 0x7fffffffLL) return -1;
+    if constexpr (STAGES == kDeep) {
+        if (!goes_deep<T>(all, lds, g.Kd, 6)) return first_go<T, BM, BN, 2>(g, qa, sums, pack, s);
+    }
+    if constexpr (lds > 64 * 1024) {
+        static std::once_flag once;
+        std::call_once(once, [] {
+            (void)hipFuncSetAttribute((const void*)wide_first_k<T, BM, BN, STAGES>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+            if constexpr (sizeof(T) == 2) (void)hipFuncSetAttribute((const void*)wide_first_pack_k<T, BM, BN, STAGES>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        });
+    }
+    if constexpr (sizeof(T) == 2) {
+        if (pack) {
+            hipLaunchKernelGGL((wide_first_pack_k<T, BM, BN, STAGES>), dim3((unsigned)all), dim3(256), lds, s, g, qa, sums, (int)nrows, (int)nsums, *pack);
+            return check_launch("wide_first_pack");
+        }
+    }
+    hipLaunchKernelGGL((wide_first_k<T, BM, BN, STAGES>), dim3((unsigned)all), dim3(256), lds, s, g, qa, sums, (int)nrows);
+    return check_launch("wide_first");
+}
+
+}  // namespace
+
+// Whether dense_wide_first_launch takes the layer (its plan for the sums in *sums, without pointers).
+bool dense_wide_first_plan(ColsumJob* sums, long long N, int K, int NO, int B, int P, int dtype) {
+    const int es = dtype == kF32 ? 4 : 2;
+    WideArgs g;
+    int bm, bn;
+    alignas(16) static char any[16];
+    if (N < 1 || !wide_rows_plan(g, bm, bn, any, any, 0, nullptr, nullptr, any, N, K, NO, P, dtype)) return false;
+    // few workgroups of the sums, who read for as long as the product takes: more of them at once get in its way (us with 128, 256 and 512:
+    // [100352,256] -> 128 26.6, 28.6, 28.7, [21168,624] -> 312 26.5, 26.2, 28.1, [100352,128] -> 64 fp32 30.6, 29.2, 29.2)
+    const long long rows = (long long)g.mt * g.nt, spare = 256 - rows;
+    int n = 192;
+    if (es == 2 && spare >= 64 && spare < n) n = (int)spare;   // (a launch of one workgroup a compute unit, kDeep)
+    const int each = B * colsum_plan(nullptr, nullptr, B, P, K, es).slices;
+    *sums = colsum_plan(nullptr, nullptr, B, P, K, es, n > each ? n - each + 1 : 1);
+    return true;
+}
+
+// y[N][NO] = x W^T, W stored [NO][K] or, with pack, as given there (zero rows where the layout has padding), the column sums of x as
+// planned, and in pool the means of the 2 x 2 pixels of y, images of 2 w_half columns; -1: not covered.
+int dense_wide_first_launch(const void* x, const void* w, void* y, void* pool, int w_half, long long N, int K, int NO, const ColsumJob& sums,
+                            const PackArgs* pack, int dtype, hipStream_t s) {
+    WideArgs g;
+    int bm, bn;
+    const int es = dtype == kF32 ? 4 : 2;
+    if (N < 1 || (pack && dtype == kF32) || !wide_rows_plan(g, bm, bn, x, w, 0, nullptr, nullptr, y, N, K, NO, 1, dtype)) return -1;
+    // a tile of rows by quads reaches 32 quads and two pairs of image rows far: 32-bit offsets
+    if (!aligned16(pool) || (N & 3) || w_half < 1 || w_half > 32768 || (128LL + 8 * w_half) * K * es > 0x7fffffffLL) return -1;
+    if (pack) g.map = RowMap{pack->Gp, pack->G};
+    const QuadArgs qa{pool, w_half, w_half > 1 ? (uint32_t)((0x100000000ULL + w_half - 1) / w_half) : 0u};
+    auto go = [&](auto t) {
+        using T = decltype(t);
+        if (bn == 192) return first_go<T, 128, 192, 2>(g, qa, sums, pack, s);
+        if (bm == 64) return bn == 64 ? first_go<T, 64, 64, kDeep>(g, qa, sums, pack, s) : first_go<T, 64, 128, kDeep>(g, qa, sums, pack, s);
+        return bn == 64 ? first_go<T, 128, 64, 2>(g, qa, sums, pack, s) : first_go<T, 128, 128, 2>(g, qa, sums, pack, s);
+    };
+    if (dtype == kF32) return first_go<float, 64, 64, 2>(g, qa, sums, nullptr, s);
+    return dtype == kF16 ? go(f16_t{}) : go(bf16_t{});
 }
 
 // (of either type)

@@ -20,14 +20,14 @@ struct ColsumJob {
 
 inline int colsum_workgroups(const ColsumJob& j) { return j.B * j.n * j.slices; }
 
-// part = nullptr: only the plan (for the size of the partials).
-inline ColsumJob colsum_plan(const void* x, float* part, int B, int P, int C, int esize) {
+// part = nullptr: only the plan (for the size of the partials, which fewer workgroups never make larger).
+inline ColsumJob colsum_plan(const void* x, float* part, int B, int P, int C, int esize, int workgroups = 512) {
     const int V = 16 / esize, vecs = C / V;
     ColsumJob j{x, part, B, P, C, 1, P, 3, 1};
     while (j.lanes_log < 5 && (1 << j.lanes_log) < vecs) ++j.lanes_log;
     j.slices = cdiv(vecs, 1 << j.lanes_log);
     const int pl = 256 >> j.lanes_log;
-    int n = cdiv(512, (long long)B * j.slices);   // two workgroups per compute unit ...
+    int n = cdiv(workgroups, (long long)B * j.slices);   // two workgroups per compute unit ...
     if (n > P / (pl * 8)) n = P / (pl * 8);       // ... of at least eight positions a thread
     if (n > 32) n = 32;
     if (n < 1) n = 1;
@@ -278,6 +278,10 @@ inline bool mean_any_ok(const void* x, const void* wp, const void* m, int D, int
            (reinterpret_cast<uintptr_t>(m) & 15) == 0;
 }
 
+// dense_wide.hip: the block's first layer with the sums of its input and the 2 x 2 pool of its result
+bool dense_wide_first_plan(ColsumJob* sums, long long N, int K, int NO, int B, int P, int dtype);
+int dense_wide_first_launch(const void* x, const void* w, void* y, void* pool, int w_half, long long N, int K, int NO, const ColsumJob& sums,
+                            const PackArgs* pack, int dtype, hipStream_t s);
 // resample.hip: the launches that they ride in.
 // xp = adaptive average pool of a to (h, w), with the column sums and the packing of weights that are given
 int avgpool_with_launch(const void* a, void* xp, int B, int H, int W, int C, int h, int w, const ColsumJob* sums, const PackArgs* pack,

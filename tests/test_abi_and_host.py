@@ -240,3 +240,13 @@ def test_the_host_extension_is_bound_to_its_torch(monkeypatch):
     assert asked == ["99.1.0+rocm9"]
     names = {build.ext_path(v) for v in ("2.10.0+rocm7.0", "2.10.0", "2.11.0+rocm7.0")}
     assert len(names) == 3 and all(os.path.dirname(n) == build.HERE for n in names)
+
+
+def test_quotients_of_quads():
+    """x / w as the high half of x * ceil(2^32 / w) (QuadRows of csrc/dense_wide.hip): exact for every x < w + 32 and w up to 32768."""
+    import numpy as np
+
+    for w in [*range(2, 700), *range(701, 32768, 97), 32767, 32768]:
+        x = np.arange(w + 32, dtype=np.uint64)
+        magic = np.uint64((2 ** 32 + w - 1) // w)
+        assert ((x * magic) >> np.uint64(32) == x // np.uint64(w)).all(), w

@@ -85,3 +85,43 @@ def test_fp32_convolutions_of_two_scales(oracle, k, dim, shape):
 def test_sums_of_x_in_the_result_or_behind_the_saved(oracle, dtype, shape):
     """The forward's sums of x, in y until it is written, or (images of a few pixels) in the buffer of the saved tensors."""
     _block_case(oracle, shape[3], 3, shape, dtype)
+
+
+@pytest.mark.parametrize("dtype,dim,k,shape", [
+    # pairs of image rows of one quad and of many, quads that end within a tile of 64 or 128 rows and an image that ends within one
+    (torch.float32, 64, 3, (3, 2, 2, 64)), (torch.float32, 132, 3, (5, 6, 10, 132)), (torch.float32, 200, 5, (2, 34, 2, 200)),
+    (torch.float32, 32, 3, (1, 2, 66, 32)), (torch.bfloat16, 144, 3, (3, 2, 2, 144)), (torch.float16, 264, 3, (5, 6, 10, 264)),
+    (torch.bfloat16, 400, 3, (2, 34, 2, 400)), (torch.float16, 640, 3, (1, 2, 66, 640)),
+    # four stages in flight; packed weights; tiles of 128 rows
+    (torch.bfloat16, 528, 3, (3, 14, 14, 528)), (torch.float16, 136, 3, (2, 10, 6, 136)), (torch.bfloat16, 424, 3, (3, 4, 8, 424)),
+])
+def test_pool_in_the_first_layers_store(oracle, dtype, dim, k, shape):
+    """Wide and fp32 blocks on exact halves: conv_up's rows by 2 x 2 quads, their mean in its store (csrc/dense_wide.hip)."""
+    _block_case(oracle, dim, k, shape, dtype)
+
+
+@pytest.mark.parametrize("dtype,dim,shape", [
+    (torch.bfloat16, 288, (11, 56, 56, 288)), (torch.float16, 576, (7, 70, 50, 576)), (torch.float16, 1152, (4, 64, 64, 1152)),
+    (torch.bfloat16, 808, (4, 66, 62, 808)), (torch.float32, 128, (12, 56, 54, 128)),
+])
+def test_pool_in_the_first_layers_store_large(monkeypatch, dtype, dim, shape):
+    """The same on tiles of 128 x 128 and 128 x 192 results, with padded halves too, against the separate launches: the same roundings, but for
+    sums of x and of the output's gradient over other ranges (a rounding of the mean and what follows from it)."""
+    import pyramid_dwconv
+    from pyramidconvblock_amd import conv_block
+
+    torch.manual_seed(1)
+    m = pyramid_dwconv.ConvBlock(dim=dim, kernel_size=3).to(dtype).cuda()
+    x, g = (torch.randn(*shape, device="cuda").to(dtype) for _ in range(2))
+
+    def step():
+        xd = x.clone().requires_grad_()
+        m.zero_grad(set_to_none=True)
+        y = m(xd)
+        torch.autograd.backward(y, g)
+        return [y.detach(), xd.grad, *[p.grad for p in m.parameters()]]
+
+    got = step()
+    monkeypatch.setattr(conv_block, "FORCE_STEPWISE", True)
+    for a, b in zip(got, step()):
+        assert_close(a, b.double().cpu().numpy(), dtype, "block", 0.5)
