@@ -151,6 +151,12 @@ int pack_weights(const PackArgs& g, hipStream_t stream) {
     return check_launch("pack_weights");
 }
 
+// Bytes of gy from which its column sums ride in the launch of conv_out's gradients, which are bound by their matrix products more than by
+// memory, instead of that of the gates.  us of the two launches: [32,56,56,128] fp32 (51 MB) 65.9 -> 61.5, [4,64,64,1152] fp16 (38 MB)
+// 81.7 -> 79.5, [8,112,112,256] bf16 (51 MB) 58.4 -> 55.9, [104,27,28,280] 68.6 -> 66.9, [8,48,48,256] fp32 (19 MB) 40.3 -> 37.8,
+// [6,56,56,256] bf16 (9.6 MB) 18.8 -> 18.7; [2,40,40,640] bf16 (4.1 MB) 17.6 -> 17.9, [3,25,20,920] bf16 (2.8 MB) 20.3 -> 20.5.
+constexpr size_t kRidingSums = 8 << 20;
+
 bool rows_whole_tiles(const Shape& s) { return s.P % pdw_dense_colsum_rows() == 0; }
 
 int forward(const Shape& s, const Saved& v, const void* x, const Weights& given, const void* w_pool, const void* b_pool,
@@ -284,13 +290,20 @@ int backward(const Shape& s, const Saved& v, const BwdWork& g, const void* gy, c
     const bool colsum = rows_whole_tiles(s) && pdw_dense_colsum_supported(s.D, s.I, dt);
     const bool pair_cs = colsum && pdw_dense_bwd_pair_colsum_supported(s.D, s.I, dt);
     float* gparts = nullptr;
+    const bool any_mean = mean_any_ok(gy, w_pool, v.m, s.D, s.es);
+    ColsumJob sums = colsum_plan(gy, (float*)g.ws_pool, s.B, s.P, s.D, s.es);
+    // ... or, where it is large, by workgroups of their own behind those gradients' (else in the gates' launch, as a part of which they take no time)
+    const bool ride = any_mean && (size_t)s.N * s.D * s.es >= kRidingSums;
+    bool summed = false;
     if (pair_cs || pdw_dense_bwd_pair_supported(s.D, s.I, dt)) {
         if (pair_cs) gparts = g.gparts;
         if (int e = pdw_dense_bwd_pair(gy, w_out, v.cat, g.dcat, gparts, gw_out, g.ws_po, g.b_po, nullptr, 1, s.N, s.D, s.I, dt, stream))
             return e;
     } else {
-        const int both = colsum ? -1 : dense_bwd_both_launch(gy, w_out, v.cat, g.dcat, gw_out, g.ws_po, g.b_po, nullptr, 1, s.N, s.D, s.I, dt, st);
+        const int both = colsum ? -1 : dense_bwd_both_launch(gy, w_out, v.cat, g.dcat, gw_out, g.ws_po, g.b_po, nullptr, 1, s.N, s.D, s.I, dt, st,
+                                                           ride ? &sums : nullptr);
         if (both != 0 && both != -1) return both;
+        summed = both == 0 && ride;
         if (colsum) {
             gparts = g.gparts;
             if (int e = pdw_dense_fwd_colsum(gy, w_out, 1, nullptr, nullptr, g.dcat, gparts, s.N, s.D, s.I, 1, dt, stream)) return e;
@@ -313,11 +326,10 @@ int backward(const Shape& s, const Saved& v, const BwdWork& g, const void* gy, c
                                    gb0, gb1, gw_pool, g.dmean, (float*)g.ws_pool, s.P, s.D, dt, st, s.gw());
         if (mid != 0 && mid != -1) return mid;
     }
-    if (mid == -1 && mean_any_ok(gy, w_pool, v.m, s.D, s.es) && reduce_defer_room() >= 5) {
-        ColsumJob sums = colsum_plan(gy, (float*)g.ws_pool, s.B, s.P, s.D, s.es);
+    if (mid == -1 && any_mean && reduce_defer_room() >= 5) {
         float* const gs = (float*)((char*)g.ws_pool + up256((size_t)s.B * sums.n * s.D * 4));
-        if (int e = gparts ? gate_pair_bwd_launch(g.dcat, v.c0, v.c1, g.gcf, g.gch, s.B, s.H, s.W, s.h, s.w, s.I, s.I, dt, st, s.gw())
-                           : gate_pair_colsum_bwd_launch(g.dcat, v.c0, v.c1, g.gcf, g.gch, s.B, s.H, s.W, s.h, s.w, s.I, s.I, sums, dt, st, s.gw()))
+        if (int e = gparts || summed ? gate_pair_bwd_launch(g.dcat, v.c0, v.c1, g.gcf, g.gch, s.B, s.H, s.W, s.h, s.w, s.I, s.I, dt, st, s.gw())
+                                     : gate_pair_colsum_bwd_launch(g.dcat, v.c0, v.c1, g.gcf, g.gch, s.B, s.H, s.W, s.h, s.w, s.I, s.I, sums, dt, st, s.gw()))
             return e;
         mean = MeanJob{gparts ? gparts : sums.part, gparts ? nparts : sums.n, s.B, s.D, 1.f / (float)s.P, w_pool, nullptr, nullptr, v.m,
                        nullptr, gs, g.dmean};

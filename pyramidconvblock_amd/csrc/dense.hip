@@ -1290,9 +1290,9 @@ int dense_wgrad_launch(const void* a, const void* b, void* dw, void* ws, long lo
 }
 
 int dense_bwd_both_launch(const void* gy, const void* w, const void* b, void* dx, void* dw, void* ws, size_t ws_bytes, const float* rowbias,
-                          int P, long long N, int M, int NO, int dtype, hipStream_t s) {
+                          int P, long long N, int M, int NO, int dtype, hipStream_t s, ColsumJob* sums) {
     if (dense_dims_ok(M, NO, dtype) || dense_wgrad_tiled_ok(M, NO, dtype) || ws_bytes < dense_wgrad_workspace(N, M, NO)) return -1;
-    return dense_wide_bwd_pair_launch(gy, w, b, dx, dw, ws, rowbias, P, N, M, NO, dtype, dense_wgrad_parts(N, M, NO), s);
+    return dense_wide_bwd_pair_launch(gy, w, b, dx, dw, ws, rowbias, P, N, M, NO, dtype, dense_wgrad_parts(N, M, NO), s, sums);
 }
 
 static bool pair_exact(int O, int I) {

@@ -526,6 +526,24 @@ __global__ __launch_bounds__(256, (STAGES == 2 ? kWideOccupancy<T, BM, BN> : 1))
     }
 }
 
+// And with the column sums of the gradient (mean_any.h) behind them.
+template <typename T, int BM, int BN, int WM, int WN, int STAGES>
+__global__ __launch_bounds__(256, (STAGES == 2 ? kWideOccupancy<T, BM, BN> : 1)) void wide_pair_sums_k(WideArgs rows, WideArgs wgrad, AnyWgradArgs any, int nw,
+                                                                                                    ColsumJob sums, int nrows) {
+    extern __shared__ __align__(16) char dsm[];
+    const int blk = blockIdx.x;
+    if (blk >= nw + nrows) {
+        colsum_body<T>(sums, blk - nw - nrows, (float*)dsm);
+    } else if (blk >= nw) {
+        wide_gemm_body<T, BM, BN, false, true, false, STAGES>(rows, blk - nw, nrows);
+    } else if constexpr (WM != 0) {
+        wide_gemm_body<T, WM, WN, true, true, true, STAGES>(wgrad, blk, nw);
+    } else {
+        const int group = blk / any.chunks;
+        dense_any_wgrad_body<T>(any, blk - group * any.chunks, group);
+    }
+}
+
 template <typename T, int BM, int BN, bool PART, int STAGES>
 constexpr size_t wide_lds() {
     constexpr size_t stages = (size_t)STAGES * (BM + BN) * kRowBytes, out = (size_t)BM * (BN * (PART ? 4 : sizeof(T)) + 16);
@@ -543,18 +561,23 @@ constexpr bool goes_deep(long long n, size_t lds, long long inner, int least) {
 }
 
 template <typename T, int BM, int BN, int WM, int WN, int STAGES>
-int pair_go(const WideArgs& rows, const WideArgs& wgrad, const AnyWgradArgs& any, int nw, hipStream_t s) {
+int pair_go(const WideArgs& rows, const WideArgs& wgrad, const AnyWgradArgs& any, int nw, const ColsumJob* sums, hipStream_t s) {
     constexpr size_t a = wide_lds<T, BM, BN, false, STAGES>(), b = WM != 0 ? wide_lds<T, WM, WN, true, STAGES>() : 0, lds = a > b ? a : b;
-    const long long n = (long long)nw + (long long)rows.mt * rows.nt;
+    const long long nrows = (long long)rows.mt * rows.nt, n = nw + nrows + (sums ? colsum_workgroups(*sums) : 0);
     if (n > 0x7fffffffLL) return -1;
     if constexpr (STAGES == kDeep) {
-        if (!goes_deep<T>(n, lds, rows.Kd, 4)) return pair_go<T, BM, BN, WM, WN, 2>(rows, wgrad, any, nw, s);
+        if (!goes_deep<T>(n, lds, rows.Kd, 4)) return pair_go<T, BM, BN, WM, WN, 2>(rows, wgrad, any, nw, sums, s);
     }
     if constexpr (lds > 64 * 1024) {
         static std::once_flag once;
         std::call_once(once, [] {
-            (void)hipFuncSetAttribute((const void*)wide_pair_k<T, BM, BN, WM, WN, STAGES>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+            for (const void* k : {(const void*)wide_pair_k<T, BM, BN, WM, WN, STAGES>, (const void*)wide_pair_sums_k<T, BM, BN, WM, WN, STAGES>})
+                (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         });
+    }
+    if (sums) {
+        hipLaunchKernelGGL((wide_pair_sums_k<T, BM, BN, WM, WN, STAGES>), dim3((unsigned)n), dim3(256), lds, s, rows, wgrad, any, nw, *sums, (int)nrows);
+        return check_launch("wide_pair_sums");
     }
     hipLaunchKernelGGL((wide_pair_k<T, BM, BN, WM, WN, STAGES>), dim3((unsigned)n), dim3(256), lds, s, rows, wgrad, any, nw);
     return check_launch("wide_pair");
@@ -664,6 +687,14 @@ WgradPlan wgrad_plan(long long N, int M, int NO, int es) {
     return plans.get({N, M, NO, es}, [=] { return wgrad_make_plan(N, M, NO, es); });
 }
 
+// Column sums that ride behind `blocks` workgroups of products: few, who read for as long as those take; more of them get in the
+// products' way.  No more than compute units are left in a launch of one workgroup each (kDeep).
+ColsumJob riding_sums(const ColsumJob& j, long long blocks, int es) {
+    const long long spare = 256 - blocks;
+    const int n = es == 2 && spare >= 64 && spare < 192 ? (int)spare : 192, each = j.B * j.slices;
+    return colsum_plan(j.x, j.part, j.B, j.P, j.C, es, n > each ? n - each + 1 : 1);
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 }  // namespace
@@ -757,13 +788,7 @@ bool dense_wide_first_plan(ColsumJob* sums, long long N, int K, int NO, int B, i
     int bm, bn;
     alignas(16) static char any[16];
     if (N < 1 || !wide_rows_plan(g, bm, bn, any, any, 0, nullptr, nullptr, any, N, K, NO, P, dtype)) return false;
-    // few workgroups of the sums, who read for as long as the product takes: more of them at once get in its way (us with 128, 256 and 512:
-    // [100352,256] -> 128 26.6, 28.6, 28.7, [21168,624] -> 312 26.5, 26.2, 28.1, [100352,128] -> 64 fp32 30.6, 29.2, 29.2)
-    const long long rows = (long long)g.mt * g.nt, spare = 256 - rows;
-    int n = 192;
-    if (es == 2 && spare >= 64 && spare < n) n = (int)spare;   // (a launch of one workgroup a compute unit, kDeep)
-    const int each = B * colsum_plan(nullptr, nullptr, B, P, K, es).slices;
-    *sums = colsum_plan(nullptr, nullptr, B, P, K, es, n > each ? n - each + 1 : 1);
+    *sums = riding_sums(colsum_plan(nullptr, nullptr, B, P, K, es), (long long)g.mt * g.nt, es);
     return true;
 }
 
@@ -820,8 +845,9 @@ int dense_wide_wgrad_launch(const void* a, const void* b, void* dw, void* ws, lo
 
 // dx[N,NO] = gy[N,M] W (+ rowbias), W stored [M][NO], and dW[M][NO] = gy^T b, in one launch; -1: not covered, or products that
 // other kernels make (the caller makes them one by one).  max_chunks: partials the workspace holds.
+// sums (optional): of gy, planned here within what it was given as.
 int dense_wide_bwd_pair_launch(const void* gy, const void* w, const void* b, void* dx, void* dw, void* ws, const float* rowbias, int P,
-                               long long N, int M, int NO, int dtype, int max_chunks, hipStream_t s) {
+                               long long N, int M, int NO, int dtype, int max_chunks, hipStream_t s, ColsumJob* sums) {
     WideArgs rows, wg{};
     AnyWgradArgs any{};
     int bm, bn, nw, nparts;
@@ -839,16 +865,17 @@ int dense_wide_bwd_pair_launch(const void* gy, const void* w, const void* b, voi
         wg = WideArgs{gy, b, nullptr, nullptr, ws, M, N, NO, M, NO, 1, p.mt, p.nt, p.splits, p.kper};
         nw = p.mt * p.nt * p.splits, nparts = p.splits;
     }
+    if (sums) *sums = riding_sums(*sums, nw + (long long)rows.mt * rows.nt, es);
     int e = -1;
     if (es == 4) {
-        if (small) e = pair_go<float, 64, 64, 0, 0, 2>(rows, wg, any, nw, s);
-        else if (p.bm == 64 && p.bn == 64) e = pair_go<float, 64, 64, 64, 64, 2>(rows, wg, any, nw, s);
+        if (small) e = pair_go<float, 64, 64, 0, 0, 2>(rows, wg, any, nw, sums, s);
+        else if (p.bm == 64 && p.bn == 64) e = pair_go<float, 64, 64, 64, 64, 2>(rows, wg, any, nw, sums, s);
     } else if (p.bm == 128 && p.bn == 128) {
         auto go = [&](auto t) {
             using T = decltype(t);
-            if (bn == 192) return pair_go<T, 128, 192, 128, 128, 2>(rows, wg, any, nw, s);
-            if (bm == 64 && bn == 128) return pair_go<T, 64, 128, 128, 128, kDeep>(rows, wg, any, nw, s);
-            if (bm == 128 && bn == 128) return pair_go<T, 128, 128, 128, 128, 2>(rows, wg, any, nw, s);
+            if (bn == 192) return pair_go<T, 128, 192, 128, 128, 2>(rows, wg, any, nw, sums, s);
+            if (bm == 64 && bn == 128) return pair_go<T, 64, 128, 128, 128, kDeep>(rows, wg, any, nw, sums, s);
+            if (bm == 128 && bn == 128) return pair_go<T, 128, 128, 128, 128, 2>(rows, wg, any, nw, sums, s);
             return -1;
         };
         e = dtype == kF16 ? go(f16_t{}) : go(bf16_t{});

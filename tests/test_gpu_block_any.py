@@ -103,10 +103,12 @@ def test_pool_in_the_first_layers_store(oracle, dtype, dim, k, shape):
 @pytest.mark.parametrize("dtype,dim,shape", [
     (torch.bfloat16, 288, (11, 56, 56, 288)), (torch.float16, 576, (7, 70, 50, 576)), (torch.float16, 1152, (4, 64, 64, 1152)),
     (torch.bfloat16, 808, (4, 66, 62, 808)), (torch.float32, 128, (12, 56, 54, 128)),
+    # odd extents: the sums of the output's gradient only
+    (torch.bfloat16, 304, (3, 71, 67, 304)), (torch.float32, 264, (2, 67, 65, 264)), (torch.float16, 1040, (1, 65, 63, 1040)),
 ])
-def test_pool_in_the_first_layers_store_large(monkeypatch, dtype, dim, shape):
-    """The same on tiles of 128 x 128 and 128 x 192 results, with padded halves too, against the separate launches: the same roundings, but for
-    sums of x and of the output's gradient over other ranges (a rounding of the mean and what follows from it)."""
+def test_pool_and_sums_beside_large_products(monkeypatch, dtype, dim, shape):
+    """The same on tiles of 128 x 128 and 128 x 192 results, with padded halves too, and the sums of the output's gradient beside conv_out's gradients,
+    against the separate launches: the same roundings, but for sums of x and of the output's gradient over other ranges (a rounding of the mean and what follows from it)."""
     import pyramid_dwconv
     from pyramidconvblock_amd import conv_block
 
