@@ -342,15 +342,19 @@ int backward(const Shape& s, const Saved& v, const BwdWork& g, const void* gy, c
     }
     // the convolutions: the pooled scale's input gradient, then the rest (one launch where that is covered, the mean branch in it)
     reduce_defer_compact(seg, val);
-    if (int e = pdw_dwconv_dgrad(g.gch, w_dw1, g.dxp, s.B, s.h, s.w, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, dt, stream)) return e;
-    const int r = dwconv_bwd3_launch(g.gcf, w_dw0, s.exact ? g.dxp : nullptr, g.da, v.a, gw_dw0, g.ws_w0, v.xp, g.gch, gw_dw1, g.ws_w1,
+    // (fp32: that gradient together with both weight gradients and the mean branch's backward, then the full scale's input gradient)
+    auto f32_pair = [&](const void* w1, void* dx1) {
+        return dt != kF32 ? -1 : dwconv_wgrad_f32t_pair_launch(v.a, g.gcf, gw_dw0, g.ws_w0, s.H, s.W, v.xp, g.gch, gw_dw1, g.ws_w1, s.h, s.w, s.B, s.I,
+                                                               s.K, pad, st, waiting ? &mean : nullptr, w1, dx1);
+    };
+    int pair = f32_pair(w_dw1, g.dxp);
+    if (pair != 0 && pair != -1) return pair;
+    if (pair == -1)
+        if (int e = pdw_dwconv_dgrad(g.gch, w_dw1, g.dxp, s.B, s.h, s.w, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, dt, stream)) return e;
+    const int r = pair == 0 ? -1 : dwconv_bwd3_launch(g.gcf, w_dw0, s.exact ? g.dxp : nullptr, g.da, v.a, gw_dw0, g.ws_w0, v.xp, g.gch, gw_dw1, g.ws_w1,
                                      s.B, s.H, s.W, s.h, s.w, s.I, s.K, dt, st, nullptr, waiting ? &mean : nullptr);
     if (r != 0 && r != -1) return r;
-    // in fp32 both weight gradients, with the mean branch's backward, and then the full scale's input gradient
-    int pair = -1;
-    if (r == -1 && dt == kF32)
-        pair = dwconv_wgrad_f32t_pair_launch(v.a, g.gcf, gw_dw0, g.ws_w0, s.H, s.W, v.xp, g.gch, gw_dw1, g.ws_w1, s.h, s.w, s.B,
-                                             s.I, s.K, pad, st, waiting ? &mean : nullptr);
+    if (r == -1 && pair == -1) pair = f32_pair(nullptr, nullptr);
     if (pair != 0 && pair != -1) return pair;
     if (waiting) {
         reduce_defer_compact(0, 0);

@@ -466,30 +466,31 @@ __global__ __launch_bounds__(512, (f32t_waves<K, 0>())) void dwconv_f32t_pair_k(
     else dwconv_f32_body<K, 4, 0>(x, w, nullptr, y, g, at, n);
 }
 
+// One problem of a launch of several, padding K / 2 (flip: the input gradient): its workgroups, and the LDS that it needs at least;
+// false: not covered.
+template <int K>
+bool f32t_problem(F32Problem& p, long long& n, size_t& lds, const void* x, const void* w, void* y, int B, int H, int W, int C, bool flip) {
+    if (!f32t_geom<K>(p.g, p.npc, n, B, H, W, C, K / 2, K / 2, flip)) return false;
+    if (!f32t_pays<K>((long long)B * H * W * C, W, p.npc, false)) return false;
+    for (const void* q : {x, w, (const void*)y})
+        if (reinterpret_cast<uintptr_t>(q) & 15) return false;
+    p.x = (const float*)x, p.w = (const float*)w, p.y = (float*)y, p.n = (int)n;
+    const size_t need = p.npc == 16 ? F32Shape<K, 16>::lds_bytes : p.npc == 8 ? F32Shape<K, 8>::lds_bytes : F32Shape<K, 4>::lds_bytes;
+    if (need > lds) lds = need;
+    return true;
+}
+
 // -1: not covered (the caller makes two launches).  Padding K / 2.
 template <int K>
 int launch_f32t_pair(const void* x0, const void* w0, void* y0, int H0, int W0, const void* x1, const void* w1, void* y1, int H1,
                      int W1, int B, int C, hipStream_t s) {
-    const void *const x[2] = {x0, x1}, *const w[2] = {w0, w1};
-    void* const y[2] = {y0, y1};
-    const int H[2] = {H0, H1}, W[2] = {W0, W1};
     F32Pair a{};
     size_t lds = 0;
-    long long total = 0;
-    for (int i = 0; i < 2; ++i) {
-        long long n;
-        F32Problem& p = a.p[i];
-        if (!f32t_geom<K>(p.g, p.npc, n, B, H[i], W[i], C, K / 2, K / 2, false)) return -1;
-        if (!f32t_pays<K>((long long)B * H[i] * W[i] * C, W[i], p.npc, false)) return -1;
-        for (const void* q : {x[i], w[i], (const void*)y[i]})
-            if (reinterpret_cast<uintptr_t>(q) & 15) return -1;
-        p.x = (const float*)x[i], p.w = (const float*)w[i], p.y = (float*)y[i];
-        total += n;
-        if (total > 0x7fffffffLL) return -1;
-        p.n = (int)n;
-        const size_t need = p.npc == 16 ? F32Shape<K, 16>::lds_bytes : p.npc == 8 ? F32Shape<K, 8>::lds_bytes : F32Shape<K, 4>::lds_bytes;
-        if (need > lds) lds = need;
-    }
+    long long n0, n1;
+    if (!f32t_problem<K>(a.p[0], n0, lds, x0, w0, y0, B, H0, W0, C, false) || !f32t_problem<K>(a.p[1], n1, lds, x1, w1, y1, B, H1, W1, C, false))
+        return -1;
+    const long long total = n0 + n1;
+    if (total > 0x7fffffffLL) return -1;
     static std::once_flag once;
     std::call_once(once, [] {
         (void)hipFuncSetAttribute((const void*)dwconv_f32t_pair_k<K>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);

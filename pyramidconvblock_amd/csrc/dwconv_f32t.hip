@@ -12,7 +12,7 @@ namespace pdw {
                                int PW, hipStream_t s);                                                                     \
     int dwconv_wgrad_f32t_pair_k##K(const void* x0, const void* gy0, void* dw0, void* ws0, int H0, int W0, const void* x1, \
                                     const void* gy1, void* dw1, void* ws1, int H1, int W1, int B, int C, int P, hipStream_t s,        \
-                                    const MeanJob* mean);
+                                    const MeanJob* mean, const void* w1, void* dx1);
 PDW_DECL(3) PDW_DECL(5) PDW_DECL(7) PDW_DECL(9) PDW_DECL(11) PDW_DECL(13) PDW_DECL(15) PDW_DECL(17)
 #undef PDW_DECL
 
@@ -57,8 +57,8 @@ int dwconv_wgrad_f32t_launch(const void* x, const void* gy, void* dw, void* ws, 
 
 int dwconv_wgrad_f32t_pair_launch(const void* x0, const void* gy0, void* dw0, void* ws0, int H0, int W0, const void* x1,
                                   const void* gy1, void* dw1, void* ws1, int H1, int W1, int B, int C, int K, int P, hipStream_t s,
-                                  const MeanJob* mean) {
-#define CALL(N) dwconv_wgrad_f32t_pair_k##N(x0, gy0, dw0, ws0, H0, W0, x1, gy1, dw1, ws1, H1, W1, B, C, P, s, mean)
+                                  const MeanJob* mean, const void* w1, void* dx1) {
+#define CALL(N) dwconv_wgrad_f32t_pair_k##N(x0, gy0, dw0, ws0, H0, W0, x1, gy1, dw1, ws1, H1, W1, B, C, P, s, mean, w1, dx1)
     PDW_BY_SIZE(CALL)
 #undef CALL
 }

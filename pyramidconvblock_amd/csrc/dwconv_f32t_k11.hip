@@ -23,8 +23,8 @@ int dwconv_wgrad_f32t_k11(const void* x, const void* gy, void* dw, void* ws, int
 
 int dwconv_wgrad_f32t_pair_k11(const void* x0, const void* gy0, void* dw0, void* ws0, int H0, int W0, const void* x1,
                               const void* gy1, void* dw1, void* ws1, int H1, int W1, int B, int C, int P, hipStream_t s,
-                              const MeanJob* mean) {
-    return launch_wgrad_f32t_pair<11>(x0, gy0, dw0, ws0, H0, W0, x1, gy1, dw1, ws1, H1, W1, B, C, P, s, mean);
+                              const MeanJob* mean, const void* w1, void* dx1) {
+    return launch_wgrad_f32t_pair<11>(x0, gy0, dw0, ws0, H0, W0, x1, gy1, dw1, ws1, H1, W1, B, C, P, s, mean, w1, dx1);
 }
 
 }  // namespace pdw

@@ -26,6 +26,7 @@
 #include <mutex>
 
 #include "common.h"
+#include "dwconv_f32t.h"
 #include "kernels.h"
 #include "mean_any.h"
 #include "tile_common.h"
@@ -443,16 +444,12 @@ constexpr bool wg_f32t_pairs(int nbi) {
 }
 
 template <int K>
-__global__ __launch_bounds__(512, 4) void dwconv_wgrad_f32t_pair_k(const WgF32Pair a) {
-    if ((int)blockIdx.x >= a.p[0].n + a.p[1].n) {
-        extern __shared__ uint32_t smem[];
-        return mean_bwd_body<float, 512, false>(a.mean, (int)blockIdx.x - a.p[0].n - a.p[1].n, reinterpret_cast<float*>(smem));
-    }
-    const bool first = (int)blockIdx.x < a.p[0].n;
+__device__ __forceinline__ void wgrad_f32t_pair_body(const WgF32Pair& a, int blk) {
+    const bool first = blk < a.p[0].n;
     const float *x = first ? a.p[0].x : a.p[1].x, *gy = first ? a.p[0].gy : a.p[1].gy;
     float* const part = first ? a.p[0].part : a.p[1].part;
     const WgF32Geom g = first ? a.p[0].g : a.p[1].g;
-    const int nbi = first ? a.p[0].nbi : a.p[1].nbi, at = (int)blockIdx.x - (first ? 0 : a.p[0].n), n = first ? a.p[0].n : a.p[1].n;
+    const int nbi = first ? a.p[0].nbi : a.p[1].nbi, at = blk - (first ? 0 : a.p[0].n), n = first ? a.p[0].n : a.p[1].n;
     if constexpr (wg_f32t_pairs<K>(4))
         if (nbi == 4) return dwconv_wgrad_f32_body<K, 4, 1>(x, gy, part, g, at, n);
     if constexpr (wg_f32t_pairs<K>(3))
@@ -463,10 +460,38 @@ __global__ __launch_bounds__(512, 4) void dwconv_wgrad_f32t_pair_k(const WgF32Pa
         if (nbi == 1) return dwconv_wgrad_f32_body<K, 1, 4>(x, gy, part, g, at, n);
 }
 
-// -1: not covered (the caller makes two launches).
+template <int K>
+__global__ __launch_bounds__(512, 4) void dwconv_wgrad_f32t_pair_k(const WgF32Pair a) {
+    if ((int)blockIdx.x >= a.p[0].n + a.p[1].n) {
+        extern __shared__ uint32_t smem[];
+        return mean_bwd_body<float, 512, false>(a.mean, (int)blockIdx.x - a.p[0].n - a.p[1].n, reinterpret_cast<float*>(smem));
+    }
+    wgrad_f32t_pair_body<K>(a, blockIdx.x);
+}
+
+// And with the input gradient of the second problem (dwconv_f32t.h), which the launch behind this one adds: by itself one workgroup a compute
+// unit with half of its time in start-up and last steps.  It lies where the weight gradients' workgroups end and fills the places of their
+// last round, or in front (d0 = 0) where that is (nearly) full, since it would be a round of its own then: as its shorter workgroups
+// end, places come free one after the other.  us, the input gradient + the weight gradients -> this: [2,32,32,32] filter 7 (its half scale's)
+// 5.8 + 9.7 -> 9.6; [2,92,92,104] filter 11 9.5 + 24.2 -> 26.4 (in front 29.9); [64,28,28,48] filter 13 10.3 + 45.7 -> 46.8 (50.4);
+// [32,56,56,64] filter 13 15.7 + 56.4 -> 66.5 (behind 74.7); [16,56,56,64] 37.3 (43.4).
+template <int K>
+__global__ __launch_bounds__(512, 4) void dwconv_bwd_f32t_half_k(const WgF32Pair a, const F32Problem d, int d0) {
+    const int blk = (int)blockIdx.x, at = blk - d0, nw = a.p[0].n + a.p[1].n;
+    if (blk >= nw + d.n) {
+        extern __shared__ uint32_t smem[];
+        return mean_bwd_body<float, 512, false>(a.mean, blk - nw - d.n, reinterpret_cast<float*>(smem));
+    }
+    if (at < 0 || at >= d.n) return wgrad_f32t_pair_body<K>(a, at < 0 ? blk : blk - d.n);
+    if (d.npc == 16) dwconv_f32_body<K, 16, 0>(d.x, d.w, nullptr, d.y, d.g, at, d.n);
+    else if (d.npc == 8) dwconv_f32_body<K, 8, 0>(d.x, d.w, nullptr, d.y, d.g, at, d.n);
+    else dwconv_f32_body<K, 4, 0>(d.x, d.w, nullptr, d.y, d.g, at, d.n);
+}
+
+// -1: not covered (the caller makes two launches).  w1, dx1 (optional): the second problem's filter and input gradient.
 template <int K>
 int launch_wgrad_f32t_pair(const void* x0, const void* gy0, void* dw0, void* ws0, int H0, int W0, const void* x1, const void* gy1,
-                           void* dw1, void* ws1, int H1, int W1, int B, int C, int P, hipStream_t s, const MeanJob* mean) {
+                           void* dw1, void* ws1, int H1, int W1, int B, int C, int P, hipStream_t s, const MeanJob* mean, const void* w1, void* dx1) {
     const WgF32Plan plan[2] = {wgrad_f32t_plan(B, H0, W0, C, K, P, P), wgrad_f32t_plan(B, H1, W1, C, K, P, P)};
     const void *const x[2] = {x0, x1}, *const gy[2] = {gy0, gy1};
     void *const dw[2] = {dw0, dw1}, *const ws[2] = {ws0, ws1};
@@ -493,12 +518,23 @@ int launch_wgrad_f32t_pair(const void* x0, const void* gy0, void* dw0, void* ws0
         if (need > lds) lds = need;
         a.mean = *mean, n += (long long)mean->B * mean_slices(mean->D);
     }
+    F32Problem d{};
+    if (dx1) {
+        long long nd;
+        if (K > 13 || !f32t_problem<K>(d, nd, lds, gy1, w1, dx1, B, H1, W1, C, true)) return -1;   // (larger filters' operands: no second workgroup)
+        n += nd;
+    }
+    const long long nw = a.p[0].n + a.p[1].n;
+    const int d0 = (nw + 511) % 512 + 1 >= 448 ? 0 : (int)nw;   // (two workgroups a compute unit: 512 a round)
     if (n > 0x7fffffffLL) return -1;
     static std::once_flag once;
     std::call_once(once, [] {
         (void)hipFuncSetAttribute((const void*)dwconv_wgrad_f32t_pair_k<K>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if constexpr (K <= 13) (void)hipFuncSetAttribute((const void*)dwconv_bwd_f32t_half_k<K>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     });
-    hipLaunchKernelGGL(dwconv_wgrad_f32t_pair_k<K>, dim3((unsigned)n), dim3(512), lds, s, a);
+    if (!dx1) hipLaunchKernelGGL(dwconv_wgrad_f32t_pair_k<K>, dim3((unsigned)n), dim3(512), lds, s, a);
+    if constexpr (K <= 13)
+        if (dx1) hipLaunchKernelGGL(dwconv_bwd_f32t_half_k<K>, dim3((unsigned)n), dim3(512), lds, s, a, d, d0);
     if (int e = check_launch("dwconv_wgrad_f32t_pair")) return e;
     for (int i = 0; i < 2; ++i)
         if (int e = wgrad_reduce_launch<float>((const float*)ws[i], (float*)dw[i], plan[i].nchunks, K * K * C, s)) return e;

@@ -141,10 +141,11 @@ int dwconv_f32t_pair_launch(const void* x0, const void* w0, void* y0, int H0, in
 size_t dwconv_wgrad_f32t_workspace(int B, int H, int W, int C, int K, int PH, int PW);
 int dwconv_wgrad_f32t_launch(const void* x, const void* gy, void* dw, void* ws, int B, int H, int W, int C, int K, int PH, int PW,
                              hipStream_t s);
-// two problems of one batch and channel count, padding P, in one launch, with (optional) the mean branch's backward
+// two problems of one batch and channel count, padding P, in one launch, with (optional) the mean branch's backward and the input
+// gradient dx1 of the second, whose filter is w1
 int dwconv_wgrad_f32t_pair_launch(const void* x0, const void* gy0, void* dw0, void* ws0, int H0, int W0, const void* x1,
                                   const void* gy1, void* dw1, void* ws1, int H1, int W1, int B, int C, int K, int P, hipStream_t s,
-                                  const struct MeanJob* mean);
+                                  const struct MeanJob* mean, const void* w1 = nullptr, void* dx1 = nullptr);
 // dense_any.hip: one 32 x 32 tile per wavefront, any dtype, widths that are multiples of 4 (inner width <= 256)
 bool dense_any_dims_ok(int K, int NO);
 int dense_any_rows_launch(const void* x, const void* w, int w_kmajor, const void* bias, const float* rowbias, void* y,

@@ -127,3 +127,13 @@ def test_pool_and_sums_beside_large_products(monkeypatch, dtype, dim, shape):
     monkeypatch.setattr(conv_block, "FORCE_STEPWISE", True)
     for a, b in zip(got, step()):
         assert_close(a, b.double().cpu().numpy(), dtype, "block", 0.5)
+
+
+@pytest.mark.parametrize("k,dim,shape", [
+    # the pooled scale's input gradient behind the weight gradients and in front (448 to 512 of their workgroups), in tiles of one, two and four images
+    (3, 16, (2, 24, 26, 16)), (5, 24, (3, 26, 30, 24)), (7, 40, (1, 31, 29, 40)), (11, 72, (2, 40, 26, 72)), (13, 8, (5, 26, 27, 8)), (13, 64, (2, 24, 130, 64)),
+    (9, 128, (3, 30, 30, 128)), (3, 128, (16, 30, 26, 128)), (3, 128, (16, 48, 26, 128)),
+])
+def test_fp32_half_scale_beside_the_weight_gradients(oracle, k, dim, shape):
+    """Both weight gradients and the pooled scale's input gradient as one launch (csrc/dwconv_wgrad_f32t.h)."""
+    _block_case(oracle, dim, k, shape, torch.float32)
