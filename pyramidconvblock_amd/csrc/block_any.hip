@@ -300,8 +300,8 @@ int backward(const Shape& s, const Saved& v, const BwdWork& g, const void* gy, c
         if (int e = pdw_dense_bwd_pair(gy, w_out, v.cat, g.dcat, gparts, gw_out, g.ws_po, g.b_po, nullptr, 1, s.N, s.D, s.I, dt, stream))
             return e;
     } else {
-        const int both = colsum ? -1 : dense_bwd_both_launch(gy, w_out, v.cat, g.dcat, gw_out, g.ws_po, g.b_po, nullptr, 1, s.N, s.D, s.I, dt, st,
-                                                           ride ? &sums : nullptr);
+        const int both = colsum ? -1 : dense_bwd_both_sums_launch(gy, w_out, v.cat, g.dcat, gw_out, g.ws_po, g.b_po, nullptr, 1, s.N, s.D, s.I, dt, st,
+                                                                ride ? &sums : nullptr);
         if (both != 0 && both != -1) return both;
         summed = both == 0 && ride;
         if (colsum) {

@@ -1289,10 +1289,15 @@ int dense_wgrad_launch(const void* a, const void* b, void* dw, void* ws, long lo
     return dense_wgrad_t<bf16_t>(a, b, dw, ws, N, M, NO, s);
 }
 
-int dense_bwd_both_launch(const void* gy, const void* w, const void* b, void* dx, void* dw, void* ws, size_t ws_bytes, const float* rowbias,
-                          int P, long long N, int M, int NO, int dtype, hipStream_t s, ColsumJob* sums) {
+int dense_bwd_both_sums_launch(const void* gy, const void* w, const void* b, void* dx, void* dw, void* ws, size_t ws_bytes, const float* rowbias,
+                               int P, long long N, int M, int NO, int dtype, hipStream_t s, ColsumJob* sums) {
     if (dense_dims_ok(M, NO, dtype) || dense_wgrad_tiled_ok(M, NO, dtype) || ws_bytes < dense_wgrad_workspace(N, M, NO)) return -1;
     return dense_wide_bwd_pair_launch(gy, w, b, dx, dw, ws, rowbias, P, N, M, NO, dtype, dense_wgrad_parts(N, M, NO), s, sums);
+}
+
+int dense_bwd_both_launch(const void* gy, const void* w, const void* b, void* dx, void* dw, void* ws, size_t ws_bytes, const float* rowbias,
+                          int P, long long N, int M, int NO, int dtype, hipStream_t s) {
+    return dense_bwd_both_sums_launch(gy, w, b, dx, dw, ws, ws_bytes, rowbias, P, N, M, NO, dtype, s, nullptr);
 }
 
 static bool pair_exact(int O, int I) {

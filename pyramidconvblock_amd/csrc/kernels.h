@@ -162,7 +162,10 @@ int dense_wide_bwd_pair_launch(const void* gy, const void* w, const void* b, voi
                                long long N, int M, int NO, int dtype, int max_chunks, hipStream_t s, struct ColsumJob* sums = nullptr);
 // dense.hip: that for the widths whose products both run there; -1 = not covered (the caller makes the two products)
 int dense_bwd_both_launch(const void* gy, const void* w, const void* b, void* dx, void* dw, void* ws, size_t ws_bytes, const float* rowbias,
-                          int P, long long N, int M, int NO, int dtype, hipStream_t s, struct ColsumJob* sums = nullptr);
+                          int P, long long N, int M, int NO, int dtype, hipStream_t s);
+// and with the column sums of gy as planned, or fewer ranges of them (mean_any.h), by workgroups of their own
+int dense_bwd_both_sums_launch(const void* gy, const void* w, const void* b, void* dx, void* dw, void* ws, size_t ws_bytes, const float* rowbias,
+                               int P, long long N, int M, int NO, int dtype, hipStream_t s, struct ColsumJob* sums);
 int dense_wide_wgrad_launch(const void* a, const void* b, void* dw, void* ws, long long N, int M, int NO, int dtype, hipStream_t s);
 int dense_bwd_pair_supported(int O, int I, int dtype);
 int dense_bwd_pair_colsum_supported(int O, int I, int dtype);
