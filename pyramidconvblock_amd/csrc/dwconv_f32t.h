@@ -3,7 +3,8 @@
 //
 // The block-Toeplitz product of dwconv_tz.h on v_mfma_f32_16x16x4_f32: for one channel m = the 16 outputs of a 4 x 4 patch,
 // n = 16 patches four columns apart (in NI = 16 / NPC images), k = 4 consecutive columns of one window row.
-//     A[(di,dj)][(r, 4j+g)] = w[r - di][4j + g - dj]     in registers, IC * JB of them (IC = K+3 rows, JB column blocks)
+//     A[(di,dj)][(r, 4j+g)] = w[r - di][4j + g - dj]     IC * JB of them (IC = K+3 rows, JB column blocks), kept in registers as far as
+//                                                       two workgroups of a compute unit leave room (f32t_kept), else read from LDS
 //     B[(r, 4j+g)][n]       = window[r][4n + 4j + g]      64 consecutive floats of a staged row: one conflict-free LDS read
 // A window row belongs to up to PER = ceil(IC/4) patch rows, whose accumulators are all live: a B operand is read once and
 // feeds PER products of 32 cycles each, so the matrix pipe is what bounds the kernel (LDS is under 10 % busy), a row
@@ -35,7 +36,18 @@
 
 namespace pdw {
 
-template <int K, int NPC>
+// Column blocks of A operands that stay in registers, all of them or what leaves a wavefront 128 registers, so that two workgroups share a
+// compute unit; the others are read again from the filter table in LDS for every product (a fifth of its rate).  us, all in registers and one
+// workgroup a unit -> this: both scales of [32,56,56,64] filter 13 50.5 -> 45.5, [22,72,73,32] filter 13 36.6 -> 32.2, [3,57,61,100]
+// filter 15 24.2 -> 18.2, [16,56,56,64] filter 15 38.9 -> 33.3, [24,36,36,100] filter 17 57.0 -> 50.7, [2,20,20,32] filter 15 9.0 -> 8.5.  With the pooled
+// gradient added (ADD > 0), which the planner cuts into one workgroup a unit, all stay ([3,57,61,100] filter 15 21.5, 25.0 with two blocks kept),
+// and in launches of no more than that with long bands (ADD = -1: [32,56,56,64] filter 13 38.7, 39.7 with three blocks kept).
+template <int K, int ADD>
+constexpr int f32t_kept() {
+    return ADD != 0 || K <= 11 ? (K + 6) / 4 : K == 13 ? 3 : 2;
+}
+
+template <int K, int NPC, int ADD = 0>
 struct F32Shape {
     static constexpr int NT = 512, CS = 8;
     static constexpr int IC = K + 3, JB = (IC + 3) / 4, PER = (IC + 3) / 4, NI = 16 / NPC, TW = 4 * NPC;
@@ -52,7 +64,9 @@ struct F32Shape {
     static constexpr int OROWP = TW * 32 + NPC * 4;                // result tile: row pitch (4 bytes more every 4 pixels)
     static constexpr int OLB = NI * 4 * OROWP;
     static constexpr int WTH = K + 6, WTW = 4 * JB + 4;            // zero-bordered filter table of a channel
-    static constexpr int R2B = (2 * OLB > CS * WTH * WTW * 4 ? 2 * OLB : CS * WTH * WTW * 4 + 15) / 16 * 16;
+    static constexpr bool STREAM = f32t_kept<K, ADD>() < JB;       // the table stays, behind the result tiles
+    static constexpr int TAB = (CS * WTH * WTW * 4 + 15) / 16 * 16, OTB = (2 * OLB + 15) / 16 * 16;
+    static constexpr int R2B = STREAM ? OTB + TAB : OTB > TAB ? OTB : TAB;
     static constexpr size_t lds_bytes = (size_t)NI * CS * CHP + R2B;
     static constexpr int NLD = (4 * NI * WCOLS * 2 + NT - 1) / NT; // staging items per thread and step
     static_assert(lds_bytes <= 80 * 1024 && NLD <= 2, "sizes");
@@ -78,8 +92,9 @@ template <int K, int NPC, int ADD>
 __device__ __forceinline__ void dwconv_f32_body(const float* __restrict__ x, const float* __restrict__ w,
                                                 const float* __restrict__ add, float* __restrict__ y, const F32Geom& g, int blk,
                                                 int nblk) {
-    using Sh = F32Shape<K, NPC>;
+    using Sh = F32Shape<K, NPC, ADD>;
     constexpr int NT = Sh::NT, IC = Sh::IC, JB = Sh::JB, PER = Sh::PER, NI = Sh::NI, TW = Sh::TW, RP = Sh::RP, CHP = Sh::CHP;
+    constexpr int JR = f32t_kept<K, ADD>();
     constexpr int OROWP = Sh::OROWP, OLB = Sh::OLB, WTH = Sh::WTH, WTW = Sh::WTW, NLD = Sh::NLD, WCOLS = Sh::WCOLS, CS = Sh::CS;
     typedef float f4 __attribute__((ext_vector_type(4)));
     typedef unsigned u4 __attribute__((ext_vector_type(4)));
@@ -155,7 +170,7 @@ __device__ __forceinline__ void dwconv_f32_body(const float* __restrict__ x, con
     issue(buf[0], 0);
     issue(buf[1], 1);
     auto lds_barrier = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-    float* const wt = reinterpret_cast<float*>(r2);   // [channel][3 + u][3 + v]
+    float* const wt = reinterpret_cast<float*>(r2 + (Sh::STREAM ? Sh::OTB : 0));   // [channel][3 + u][3 + v]
     for (int i = tid; i < CS * WTH * WTW / 4; i += NT) reinterpret_cast<f4*>(wt)[i] = f4{0.f, 0.f, 0.f, 0.f};
     lds_barrier();
 #pragma unroll
@@ -173,16 +188,22 @@ __device__ __forceinline__ void dwconv_f32_body(const float* __restrict__ x, con
     lds_barrier();
     // ---- this wavefront's A operands
     const int ln = lane & 15, kg = lane >> 4;
-    float A[IC][JB];
-    {
-        const int di = ln >> 2, dj = ln & 3;
-        const float* wp = wt + (wv * WTH + 3 - di) * WTW + 3 + kg - dj;
+    float A[IC][JR];
+    const float* const wp = wt + (wv * WTH + 3 - (ln >> 2)) * WTW + 3 + kg - (ln & 3);
 #pragma unroll
-        for (int r = 0; r < IC; ++r)
+    for (int r = 0; r < IC; ++r)
 #pragma unroll
-            for (int j = 0; j < JB; ++j) A[r][j] = wp[r * WTW + 4 * j];
+        for (int j = 0; j < JR; ++j) A[r][j] = wp[r * WTW + 4 * j];
+    if constexpr (!Sh::STREAM) lds_barrier();   // (the table's space becomes the result tiles)
+    uint32_t wb[2] = {0, 0};   // rows 0 and 8 of this lane's table (as xb below)
+    if constexpr (Sh::STREAM) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            wb[i] = (uint32_t)(reinterpret_cast<const char*>(wp) - xl) + (uint32_t)(8 * i * WTW * 4);
+            asm("" : "+v"(wb[i]));
+        }
     }
-    lds_barrier();   // (the table's space becomes the result tiles)
+    auto weight = [&](int row, int j) { return *reinterpret_cast<const float*>(xl + wb[row / 8 < 2 ? row / 8 : 1] + ((row - (row < 8 ? 0 : 8)) * WTW + 4 * j) * 4); };
     const int pimg = ln / NPC, pc = ln % NPC;
     // Rows 0 .. 7 of the window at a lane, in three registers: as offsets from one they are out of a paired read's reach, and
     // each read would add its own (vector instructions do not overlap with fp32 products: 124 us of products and 172 us of
@@ -206,7 +227,7 @@ __device__ __forceinline__ void dwconv_f32_body(const float* __restrict__ x, con
     uint32_t aoff = 0;
     float wj0 = 0.f, wj1 = 0.f, wi0 = 0.f, wi1 = 0.f;
     f4 addv[ADD == 2 ? 4 : 1];
-    if constexpr (ADD) {
+    if constexpr (ADD > 0) {
         arsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(add + (long long)b0 * g.AH * g.AW * g.C), (short)0,
                                                   (int)((long long)min(NI, g.B - b0) * g.AH * g.AW * g.C * 4), 0x00020000);
         if constexpr (ADD == 2) pool_bins(min(ocol0 + scol, g.OW - 1), g.OW, g.AW, jb0, wj0, wj1);
@@ -265,18 +286,24 @@ __device__ __forceinline__ void dwconv_f32_body(const float* __restrict__ x, con
             for (int j = 0; j < JB; ++j) bv[j] = *reinterpret_cast<const float*>(xl + xb[row / 3] + row % 3 * RP + 16 * j);
         };
         if (s >= PER - 1 && s < npr) {   // (uniform) all of them: row by row, the next row's operands read meanwhile
-            float bv[2][JB];
+            float bv[2][JB], av[2][PER];   // (av: of the column blocks that are not kept, a block ahead)
             fetch(bv[0], 0);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 if (r < 3) fetch(bv[(r + 1) & 1], r + 1);
 #pragma unroll
                 for (int j = 0; j < JB; ++j) {
+                    if (j + 1 >= JR && j + 1 < JB) {
+#pragma unroll
+                        for (int q = PER - 1; q >= 0; --q)
+                            if (4 * q + r < IC) av[(j + 1) & 1][q] = weight(4 * q + r, j + 1);
+                    }
 #pragma unroll
                     for (int q = PER - 1; q >= 0; --q) {
                         if (4 * q + r >= IC) continue;
                         const f4 c = r == 0 && j == 0 ? (q > 0 ? acc[q > 0 ? q - 1 : 0] : f4{0.f, 0.f, 0.f, 0.f}) : acc[q];
-                        acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[4 * q + r < IC ? 4 * q + r : 0][j], bv[r & 1][j], c, 0, 0, 0);
+                        const float w = j < JR ? A[4 * q + r < IC ? 4 * q + r : 0][j < JR ? j : 0] : av[j & 1][q];
+                        acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, bv[r & 1][j], c, 0, 0, 0);
                     }
                 }
             }
@@ -285,15 +312,23 @@ __device__ __forceinline__ void dwconv_f32_body(const float* __restrict__ x, con
             for (int q = PER - 1; q >= 0; --q) {
                 if (s < q || s - q >= npr) continue;   // (uniform)
                 f4 a = q > 0 ? acc[q > 0 ? q - 1 : 0] : f4{0.f, 0.f, 0.f, 0.f};
-                float bv[2][JB];
+                float bv[2][JB], av[2][JB > JR ? JB - JR : 1];
+                auto weights = [&](float (&d)[JB > JR ? JB - JR : 1], int r) {
+#pragma unroll
+                    for (int j = JR; j < JB; ++j)
+                        if (4 * q + r < IC) d[j - JR] = weight(4 * q + r, j);
+                };
                 fetch(bv[0], 0);
+                weights(av[0], 0);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     if (4 * q + r >= IC) continue;
-                    if (r < 3) fetch(bv[(r + 1) & 1], r + 1);
+                    if (r < 3) fetch(bv[(r + 1) & 1], r + 1), weights(av[(r + 1) & 1], r + 1);
 #pragma unroll
-                    for (int j = 0; j < JB; ++j)
-                        a = __builtin_amdgcn_mfma_f32_16x16x4f32(A[4 * q + r < IC ? 4 * q + r : 0][j], bv[r & 1][j], a, 0, 0, 0);
+                    for (int j = 0; j < JB; ++j) {
+                        const float w = j < JR ? A[4 * q + r < IC ? 4 * q + r : 0][j < JR ? j : 0] : av[r & 1][j >= JR ? j - JR : 0];
+                        a = __builtin_amdgcn_mfma_f32_16x16x4f32(w, bv[r & 1][j], a, 0, 0, 0);
+                    }
                 }
                 acc[q] = a;
             }
@@ -334,7 +369,7 @@ __device__ __forceinline__ void dwconv_f32_body(const float* __restrict__ x, con
 // overlaps the other's products.
 template <int K, int ADD>
 constexpr int f32t_waves() {
-    return (K + 3) * ((K + 6) / 4) <= (ADD ? 36 : 56) ? 4 : 2;
+    return (K >= 13 && ADD == 0) || (K + 3) * ((K + 6) / 4) <= (ADD ? 36 : 56) ? 4 : 2;
 }
 
 template <int K, int NPC, int ADD>
@@ -362,14 +397,14 @@ inline int f32t_npc(int B, int OW) {
 // Band height: the fewest cycles for rounds of workgroups over 256 compute units (products of the band; start-up and the
 // window's first rows, which two workgroups of a unit overlap).
 template <int K>
-int f32t_band(long long per_band, int OH) {
+int f32t_band(long long per_band, int OH, bool add) {
     constexpr int NA = (K + 3) * ((K + 6) / 4);
     if (const char* e = tune_env("PDW_F32_BR")) return atoi(e);
     int best = 4;
     double cost = -1;
     for (int br = 4; br <= (OH + 3) / 4 * 4; br += 4) {
         const long long wgs = per_band * cdiv(OH, br);
-        const double c = (double)cdiv(wgs, 256) * (br / 4) * NA * 64 + (double)cdiv(wgs, f32t_waves<K, 0>() == 4 ? 512 : 256) * 9000;
+        const double c = (double)cdiv(wgs, 256) * (br / 4) * NA * 64 + (double)cdiv(wgs, f32t_waves<K, 0>() == 4 && (K < 13 || !add) ? 512 : 256) * 9000;
         if (cost < 0 || c <= cost) cost = c, best = br;
     }
     return best;
@@ -390,7 +425,7 @@ bool f32t_pays(long long outputs, int OW, int npc, bool add) {
 
 // false: not covered
 template <int K>
-bool f32t_geom(F32Geom& g, int& npc, long long& nblocks, int B, int H, int W, int C, int PH, int PW, bool flip) {
+bool f32t_geom(F32Geom& g, int& npc, long long& nblocks, int B, int H, int W, int C, int PH, int PW, bool flip, bool add = false) {
     g = F32Geom{B, H, W, C, H + 2 * PH - K + 1, W + 2 * PW - K + 1, PH, PW, 0, 0, 0, 0, flip ? 1 : 0, 0, 0};
     if (g.OH < 1 || g.OW < 1 || C % 4 != 0 || B < 1) return false;
     npc = f32t_npc(B, g.OW);
@@ -398,7 +433,7 @@ bool f32t_geom(F32Geom& g, int& npc, long long& nblocks, int B, int H, int W, in
     if ((long long)H * W * C * ni > 0x0fffffffLL || (long long)g.OH * g.OW * C * ni > 0x0fffffffLL) return false;
     g.ncolt = cdiv(g.OW, 4 * npc), g.nslices = cdiv(C, 8);
     const long long per_band = (long long)cdiv(B, ni) * g.ncolt * g.nslices;
-    g.BR = f32t_band<K>(per_band, g.OH), g.nbands = cdiv(g.OH, g.BR);
+    g.BR = f32t_band<K>(per_band, g.OH, add), g.nbands = cdiv(g.OH, g.BR);
     nblocks = per_band * g.nbands;
     return nblocks <= 0x7fffffffLL;
 }
@@ -410,7 +445,7 @@ int launch_f32t(const void* x, const void* w, const void* add, void* y, int B, i
     F32Geom g;
     int npc;
     long long nblocks;
-    if (!f32t_geom<K>(g, npc, nblocks, B, H, W, C, PH, PW, flip)) return -1;
+    if (!f32t_geom<K>(g, npc, nblocks, B, H, W, C, PH, PW, flip, add != nullptr)) return -1;
     if (!f32t_pays<K>((long long)B * g.OH * g.OW * C, g.OW, npc, add != nullptr)) return -1;
     for (const void* p : {x, w, (const void*)y, add})
         if (reinterpret_cast<uintptr_t>(p) & 15) return -1;
@@ -421,13 +456,13 @@ int launch_f32t(const void* x, const void* w, const void* add, void* y, int B, i
         auto kern = dwconv_f32t_k<K, NPC, A>;                                                                              \
         static std::once_flag once;                                                                                        \
         std::call_once(once, [&] { (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); }); \
-        constexpr size_t lds = F32Shape<K, NPC>::lds_bytes;                                                                \
+        constexpr size_t lds = F32Shape<K, NPC, A>::lds_bytes;                                                                \
         hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(512), lds, s, (const float*)x, (const float*)w,             \
                            (const float*)add, (float*)y, g);                                                               \
     }
-    const int mode = !add ? 0 : g.OH == 2 * AH && g.OW == 2 * AW ? 1 : 2;
+    const int mode = !add ? (K >= 13 && nblocks <= 256 && g.BR >= 40 ? -1 : 0) : g.OH == 2 * AH && g.OW == 2 * AW ? 1 : 2;
 #define PDW_F32T_M(NPC) \
-    if (mode == 0) PDW_F32T(NPC, 0) else if (mode == 1) PDW_F32T(NPC, 1) else PDW_F32T(NPC, 2)
+    if (mode == 0) PDW_F32T(NPC, 0) else if (mode == 1) PDW_F32T(NPC, 1) else if (mode == 2) PDW_F32T(NPC, 2) else PDW_F32T(NPC, (K >= 13 ? -1 : 0))
     if (npc == 16) {
         PDW_F32T_M(16)
     } else if (npc == 8) {

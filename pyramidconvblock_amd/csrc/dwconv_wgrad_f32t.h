@@ -474,7 +474,7 @@ __global__ __launch_bounds__(512, 4) void dwconv_wgrad_f32t_pair_k(const WgF32Pa
 // last round, or in front (d0 = 0) where that is (nearly) full, since it would be a round of its own then: as its shorter workgroups
 // end, places come free one after the other.  us, the input gradient + the weight gradients -> this: [2,32,32,32] filter 7 (its half scale's)
 // 5.8 + 9.7 -> 9.6; [2,92,92,104] filter 11 9.5 + 24.2 -> 26.4 (in front 29.9); [64,28,28,48] filter 13 10.3 + 45.7 -> 46.8 (50.4);
-// [32,56,56,64] filter 13 15.7 + 56.4 -> 66.5 (behind 74.7); [16,56,56,64] 37.3 (43.4).
+// [32,56,56,64] filter 13 15.7 + 56.4 -> 66.5 (behind 74.7); [16,56,56,64] 37.3 (43.4), filter 15 11.7 + 32.9 -> 40.3.
 template <int K>
 __global__ __launch_bounds__(512, 4) void dwconv_bwd_f32t_half_k(const WgF32Pair a, const F32Problem d, int d0) {
     const int blk = (int)blockIdx.x, at = blk - d0, nw = a.p[0].n + a.p[1].n;
@@ -521,7 +521,7 @@ int launch_wgrad_f32t_pair(const void* x0, const void* gy0, void* dw0, void* ws0
     F32Problem d{};
     if (dx1) {
         long long nd;
-        if (K > 13 || !f32t_problem<K>(d, nd, lds, gy1, w1, dx1, B, H1, W1, C, true)) return -1;   // (larger filters' operands: no second workgroup)
+        if (!f32t_problem<K>(d, nd, lds, gy1, w1, dx1, B, H1, W1, C, true)) return -1;
         n += nd;
     }
     const long long nw = a.p[0].n + a.p[1].n;
@@ -530,11 +530,10 @@ int launch_wgrad_f32t_pair(const void* x0, const void* gy0, void* dw0, void* ws0
     static std::once_flag once;
     std::call_once(once, [] {
         (void)hipFuncSetAttribute((const void*)dwconv_wgrad_f32t_pair_k<K>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        if constexpr (K <= 13) (void)hipFuncSetAttribute((const void*)dwconv_bwd_f32t_half_k<K>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        (void)hipFuncSetAttribute((const void*)dwconv_bwd_f32t_half_k<K>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     });
     if (!dx1) hipLaunchKernelGGL(dwconv_wgrad_f32t_pair_k<K>, dim3((unsigned)n), dim3(512), lds, s, a);
-    if constexpr (K <= 13)
-        if (dx1) hipLaunchKernelGGL(dwconv_bwd_f32t_half_k<K>, dim3((unsigned)n), dim3(512), lds, s, a, d, d0);
+    else hipLaunchKernelGGL(dwconv_bwd_f32t_half_k<K>, dim3((unsigned)n), dim3(512), lds, s, a, d, d0);
     if (int e = check_launch("dwconv_wgrad_f32t_pair")) return e;
     for (int i = 0; i < 2; ++i)
         if (int e = wgrad_reduce_launch<float>((const float*)ws[i], (float*)dw[i], plan[i].nchunks, K * K * C, s)) return e;

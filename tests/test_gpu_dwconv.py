@@ -346,3 +346,27 @@ def test_random_shapes_matrix_core_kernels(oracle, seed):
     C = 8 * int(rng.integers(1, 10))
     dtype = [torch.bfloat16, torch.float16][seed % 2]
     _run(oracle, (B, H, W, C), k, dtype, seed=seed)
+
+
+@pytest.mark.parametrize("k", [13, 15, 17])
+@pytest.mark.parametrize("shape", [
+    # operands read again from LDS: tiles of one, two and four images, a patch row, images shorter than a filter, many bands
+    (1, 3, 61, 8), (3, 41, 30, 12), (5, 9, 13, 20), (6, 40, 60, 72),
+    # one workgroup a compute unit in long bands, all operands in registers: 44 and 46 rows
+    (4, 44, 50, 512), (16, 46, 30, 256),
+])
+def test_fp32_operands_in_registers_and_in_lds(k, shape):
+    """fp32 on the matrix cores, filters whose operands two workgroups of a compute unit cannot both hold in registers (csrc/dwconv_f32t.h):
+    forward and input gradient against float64."""
+    import torch.nn.functional as F
+
+    from pyramidconvblock_amd.dwconv import dwconv_dgrad, dwconv_forward
+
+    gen = torch.Generator().manual_seed(k)
+    x, w = randn(gen, *shape).cuda(), (randn(gen, k, k, shape[3]) / k).cuda()
+    geo = ((1, 1), (k // 2, k // 2), (1, 1))
+    dense = lambda t, f: torch.cat([F.conv2d(t[b:b + 1].double().cpu().permute(0, 3, 1, 2), f.double().cpu().permute(2, 0, 1).unsqueeze(1), padding=k // 2,
+                                             groups=shape[3]) for b in (0, shape[0] - 1)]).permute(0, 2, 3, 1).numpy()
+    ends = lambda t: t[[0, -1]]
+    assert_close(ends(dwconv_forward(x, w, *geo)), dense(x, w), torch.float32, "y")
+    assert_close(ends(dwconv_dgrad(x, w, x.shape, *geo)), dense(x, w.flip(0, 1)), torch.float32, "dx")
