@@ -4,6 +4,8 @@
 // so every wavefront access is a contiguous run.  Both backward kernels are gathers:
 // each input element sums the few outputs that touch it, in a fixed order, so there are
 // no atomics and results are bit-reproducible.
+#include <type_traits>
+
 #include "common.h"
 #include "kernels.h"
 #include "mean_any.h"
@@ -69,13 +71,33 @@ __device__ __forceinline__ void avgpool_fwd_item(const T* __restrict__ x, T* __r
     float acc[VEC];
 #pragma unroll
     for (int v = 0; v < VEC; ++v) acc[v] = 0.f;
-    for (int ih = hs; ih < he; ++ih)
-        for (int iw = ws; iw < we; ++iw) {
-            float xv[VEC];
-            load_f32<T, VEC>(x + ((b * H + ih) * W + iw) * C + c, xv);
+    constexpr int NB = 3;
+    if (he - hs <= NB && we - ws <= NB) {   // bins of up to 3 x 3 (extents of two to three times the pooled ones): all loads in flight
+        // (us, with column sums: [2,15,15,96] bf16 4.7 -> 3.5, [27,15,15,624] 6.6 -> 4.8; [104,27,28,280], bandwidth, 17.4 -> 17.9)
+        const T* const p = x + ((b * H + hs) * W + ws) * C + c;
+        ChanVec<T, VEC> xv[NB][NB];
 #pragma unroll
-            for (int v = 0; v < VEC; ++v) acc[v] += xv[v];
-        }
+        for (int r = 0; r < NB; ++r)
+#pragma unroll
+            for (int k = 0; k < NB; ++k)
+                xv[r][k] = *reinterpret_cast<const ChanVec<T, VEC>*>(p + ((long long)min(r, he - hs - 1) * W + min(k, we - ws - 1)) * C);
+#pragma unroll
+        for (int r = 0; r < NB; ++r)
+#pragma unroll
+            for (int k = 0; k < NB; ++k)
+                if (r < he - hs && k < we - ws) {
+#pragma unroll
+                    for (int v = 0; v < VEC; ++v) acc[v] += to_f32(xv[r][k].v[v]);
+                }
+    } else {
+        for (int ih = hs; ih < he; ++ih)
+            for (int iw = ws; iw < we; ++iw) {
+                float xv[VEC];
+                load_f32<T, VEC>(x + ((b * H + ih) * W + iw) * C + c, xv);
+#pragma unroll
+                for (int v = 0; v < VEC; ++v) acc[v] += xv[v];
+            }
+    }
     const float inv = 1.f / (float)((he - hs) * (we - ws));
 #pragma unroll
     for (int v = 0; v < VEC; ++v) acc[v] *= inv;
@@ -127,23 +149,48 @@ __global__ __launch_bounds__(256) void avgpool_bwd_k(const T* __restrict__ gy, T
     float acc[VEC];
 #pragma unroll
     for (int v = 0; v < VEC; ++v) acc[v] = 0.f;
-    for (int i = i0; i <= i1; ++i) {
-        const int kh = bin_end(i, H, h) - bin_start(i, H, h);
-        for (int j = j0; j <= j1; ++j) {
-            const int kw = bin_end(j, W, w) - bin_start(j, W, w);
-            const float inv = 1.f / (float)(kh * kw);
-            float gv[VEC];
-            load_f32<T, VEC>(gy + ((b * h + i) * w + j) * C + c, gv);
+    T* dst = gx + ((b * H + ih) * W + iw) * C + c;
+    ChanVec<T, VEC> old;
+    if (accumulate) old = *reinterpret_cast<const ChanVec<T, VEC>*>(dst);
+    if (i1 - i0 <= 1 && j1 - j0 <= 1) {   // (always where the pool shrinks) at most 2 x 2 bins: their loads in flight together
+        // (us: [3,57,61,200] bf16 5.7 -> 4.8, [2,15,15,96] 3.8 -> 3.3; [104,27,28,280] 16.3 -> 16.8)
+        ChanVec<T, VEC> gv[2][2];
 #pragma unroll
-            for (int v = 0; v < VEC; ++v) acc[v] = fmaf(gv[v], inv, acc[v]);
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+                gv[p][q] = *reinterpret_cast<const ChanVec<T, VEC>*>(gy + ((b * h + (p ? i1 : i0)) * w + (q ? j1 : j0)) * C + c);
+        int kh[2], kw[2];
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            const int i = p ? i1 : i0, j = p ? j1 : j0;
+            kh[p] = bin_end(i, H, h) - bin_start(i, H, h), kw[p] = bin_end(j, W, w) - bin_start(j, W, w);
+        }
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+                if (i0 + p <= i1 && j0 + q <= j1) {
+                    const float inv = 1.f / (float)(kh[p] * kw[q]);
+#pragma unroll
+                    for (int v = 0; v < VEC; ++v) acc[v] = fmaf(to_f32(gv[p][q].v[v]), inv, acc[v]);
+                }
+    } else {
+        for (int i = i0; i <= i1; ++i) {
+            const int kh = bin_end(i, H, h) - bin_start(i, H, h);
+            for (int j = j0; j <= j1; ++j) {
+                const int kw = bin_end(j, W, w) - bin_start(j, W, w);
+                const float inv = 1.f / (float)(kh * kw);
+                float gv[VEC];
+                load_f32<T, VEC>(gy + ((b * h + i) * w + j) * C + c, gv);
+#pragma unroll
+                for (int v = 0; v < VEC; ++v) acc[v] = fmaf(gv[v], inv, acc[v]);
+            }
         }
     }
-    T* dst = gx + ((b * H + ih) * W + iw) * C + c;
     if (accumulate) {  // gx += pooled gradient (fp32 add, one rounding)
-        float old[VEC];
-        load_f32<T, VEC>(dst, old);
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) acc[v] += old[v];
+        for (int v = 0; v < VEC; ++v) acc[v] += to_f32(old.v[v]);
     }
     store_f32<T, VEC>(dst, acc);
 }
@@ -273,6 +320,35 @@ __device__ __forceinline__ void bl_dst_range(int m, float scale, int out, int& l
     if (hi > out - 1) hi = out - 1;
 }
 
+// The run of destinations i0 .. i1 in which source m weighs, and their weights (zero beyond i1); false where it is longer than kRun or does
+// not lie where a ratio of about two puts it.  Eight candidates, each weight computed once: the search over the generous range of twelve,
+// every weight up to three times, was most of a gradient's instructions (us, gates and sums: [3,57,61,200] bf16
+// 9.1 -> 6.9, [2,15,15,96] 8.1 -> 5.8, [27,15,15,624] 8.8 -> 6.7, [3,57,61,200] fp32 9.4 -> 7.2).
+constexpr int kRun = 5;
+__device__ __forceinline__ bool bl_dst_run(int m, float scale, int in, int out, int& i0, int& i1, float (&wt)[kRun]) {
+    constexpr int NC = 8, SHIFT = NC - kRun + 1;
+    const float inv = 1.f / scale;
+    const int lo = m == 0 ? 0 : max((int)floorf(((float)m - 0.5f) * inv - 0.5f), 0);
+    const int hi = min((int)ceilf(((float)m + 1.5f) * inv - 0.5f), out - 1);
+    if (hi - lo >= NC) return false;
+    float c[NC];
+    int d = NC, e = -1;   // the first and the last that weigh
+#pragma unroll
+    for (int q = NC - 1; q >= 0; --q) {
+        c[q] = lo + q <= hi ? bl_weight(lo + q, scale, in, m) : 0.f;
+        if (c[q] != 0.f) d = q, e = max(e, q);
+    }
+    if (e < 0 || e - d >= kRun || d >= SHIFT) return false;
+    i0 = lo + d, i1 = lo + e;
+#pragma unroll
+    for (int q = 0; q < kRun; ++q) {
+        wt[q] = c[q];
+#pragma unroll
+        for (int k = 1; k < SHIFT; ++k) wt[q] = d == k ? c[q + k] : wt[q];
+    }
+    return true;
+}
+
 // Exactly doubled extents (H = 2h, W = 2w, the block's half-resolution gate): source m is read by the 4
 // destinations 2m-1 .. 2m+2 and no others, so the taps are fixed and all 16 loads go out together.  The weights
 // come from the same bl_weight as the general kernel (bit-identical results, borders included).
@@ -326,64 +402,55 @@ __global__ __launch_bounds__(256) void bilinear_bwd_x2_k(const T* __restrict__ g
 template <typename T, int VEC>
 __device__ __forceinline__ void bilinear_bwd_gather(const T* __restrict__ gb, int h, int w, int H, int W, int ldg, float sy,
                                                     float sx, int m, int n, float (&acc)[VEC]) {
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) acc[v] = 0.f;
+    // The destinations that weigh in are a contiguous run of about 2 * out/in in a range one wider on either side.  Up to NS of
+    // them per axis are handled without branches: weights beyond the run are zero and addresses clamped, so that the loads of two
+    // rows are issued together (a load behind a per-lane `continue` is a trip to memory of its own).
+    int i0, i1, j0, j1;
+    float wy[kRun], wx[kRun];
+    if (bl_dst_run(m, sy, h, H, i0, i1, wy) && bl_dst_run(n, sx, w, W, j0, j1, wx)) {
+        constexpr int NS = kRun;
+        int jo[NS];
+#pragma unroll
+        for (int q = 0; q < NS; ++q) jo[q] = min(j0 + q, j1) * ldg;
+        auto rows = [&](auto first, auto count) {
+            constexpr int P = decltype(first)::value, N = decltype(count)::value;
+            ChanVec<T, VEC> gv[N][NS];
+#pragma unroll
+            for (int p = 0; p < N; ++p) {
+                const T* gr = gb + (long long)min(i0 + P + p, i1) * W * ldg;
+#pragma unroll
+                for (int q = 0; q < NS; ++q) gv[p][q] = *reinterpret_cast<const ChanVec<T, VEC>*>(gr + jo[q]);
+            }
+#pragma unroll
+            for (int p = 0; p < N; ++p)
+#pragma unroll
+                for (int q = 0; q < NS; ++q) {
+                    const float ww = wy[P + p] * wx[q];
+#pragma unroll
+                    for (int v = 0; v < VEC; ++v) acc[v] = fmaf(ww, to_f32(gv[p][q].v[v]), acc[v]);
+                }
+        };
+        rows(std::integral_constant<int, 0>(), std::integral_constant<int, 2>());
+        rows(std::integral_constant<int, 2>(), std::integral_constant<int, 2>());
+        if (i1 - i0 >= 4) rows(std::integral_constant<int, 4>(), std::integral_constant<int, 1>());
+        return;
+    }
     int ilo, ihi, jlo, jhi;
     bl_dst_range(m, sy, H, ilo, ihi);
     bl_dst_range(n, sx, W, jlo, jhi);
+    for (int i = ilo; i <= ihi; ++i) {
+        const float wy = bl_weight(i, sy, h, m);
+        if (wy == 0.f) continue;
+        for (int j = jlo; j <= jhi; ++j) {
+            const float wx = bl_weight(j, sx, w, n);
+            if (wx == 0.f) continue;
+            float gv[VEC];
+            load_f32<T, VEC>(gb + ((long long)i * W + j) * ldg, gv);
+            const float ww = wy * wx;
 #pragma unroll
-    for (int v = 0; v < VEC; ++v) acc[v] = 0.f;
-    // The candidate ranges are generous (up to 11 wide when the output is about twice the input); the destinations
-    // that really weigh in are a contiguous run of about 2 * out/in.  Up to NS of them per axis are handled
-    // without branches: weights beyond the run are zero and addresses clamped, so the NS loads of a row are issued
-    // together (a load behind a per-lane `continue` is a trip to memory of its own).
-    constexpr int NC = 12, NS = 5;
-    int i0 = ihi + 1, i1 = ilo - 1, j0 = jhi + 1, j1 = jlo - 1;
-    if (ihi - ilo < NC && jhi - jlo < NC) {
-#pragma unroll
-        for (int q = NC - 1; q >= 0; --q) {
-            if (ilo + q <= ihi && bl_weight(ilo + q, sy, h, m) != 0.f) i0 = ilo + q;
-            if (jlo + q <= jhi && bl_weight(jlo + q, sx, w, n) != 0.f) j0 = jlo + q;
-        }
-#pragma unroll
-        for (int q = 0; q < NC; ++q) {
-            if (ilo + q <= ihi && bl_weight(ilo + q, sy, h, m) != 0.f) i1 = ilo + q;
-            if (jlo + q <= jhi && bl_weight(jlo + q, sx, w, n) != 0.f) j1 = jlo + q;
-        }
-    }
-    if (i1 - i0 < NS && j1 - j0 < NS && i1 >= i0 && j1 >= j0) {
-        float wy[NS], wx[NS];
-        int jo[NS];
-#pragma unroll
-        for (int q = 0; q < NS; ++q) {
-            wy[q] = i0 + q <= i1 ? bl_weight(i0 + q, sy, h, m) : 0.f;
-            wx[q] = j0 + q <= j1 ? bl_weight(j0 + q, sx, w, n) : 0.f;
-            jo[q] = min(j0 + q, j1) * ldg;
-        }
-#pragma unroll
-        for (int p = 0; p < NS; ++p) {
-            const T* gr = gb + (long long)min(i0 + p, i1) * W * ldg;
-            ChanVec<T, VEC> gv[NS];
-#pragma unroll
-            for (int q = 0; q < NS; ++q) gv[q] = *reinterpret_cast<const ChanVec<T, VEC>*>(gr + jo[q]);
-#pragma unroll
-            for (int q = 0; q < NS; ++q) {
-                const float ww = wy[p] * wx[q];
-#pragma unroll
-                for (int v = 0; v < VEC; ++v) acc[v] = fmaf(ww, to_f32(gv[q].v[v]), acc[v]);
-            }
-        }
-    } else {
-        for (int i = ilo; i <= ihi; ++i) {
-            const float wy = bl_weight(i, sy, h, m);
-            if (wy == 0.f) continue;
-            for (int j = jlo; j <= jhi; ++j) {
-                const float wx = bl_weight(j, sx, w, n);
-                if (wx == 0.f) continue;
-                float gv[VEC];
-                load_f32<T, VEC>(gb + ((long long)i * W + j) * ldg, gv);
-                const float ww = wy * wx;
-#pragma unroll
-                for (int v = 0; v < VEC; ++v) acc[v] = fmaf(ww, gv[v], acc[v]);
-            }
+            for (int v = 0; v < VEC; ++v) acc[v] = fmaf(ww, gv[v], acc[v]);
         }
     }
 }

@@ -581,3 +581,24 @@ def test_fwd2_mean_is_the_convolutions_and_the_mean_branch(dtype, case, biases):
     if rc == 0:
         assert torch.equal(ya, yb) and torch.equal(za, zb) and torch.equal(m2, m) and torch.equal(rb2, rowbias)
         assert torch.equal(ya, ops.gate_forward(convs[0])) and torch.equal(za, ops.gate_forward(convs[1]))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("big,small", [
+    # ratios of two and a bit, where loads go out together: runs of four and five destinations, bins of two and three, both borders; and of
+    # one, three, four and a half, eight and beyond, where they do not
+    (3, 1), (5, 2), (7, 3), (9, 4), (57, 28), (61, 30), (111, 55), (12, 5), (13, 5), (10, 10), (11, 9), (15, 5), (16, 5), (18, 4), (33, 4), (40, 2),
+])
+def test_any_ratio(oracle, dtype, big, small):
+    """Pool forward, its gradient and the resize's gradient against float64, one axis at the ratio and the other at twice 4."""
+    import pyramidconvblock_amd as P
+
+    for hw, out in (((big, 8), (small, 4)), ((8, big), (4, small))):
+        gen = torch.Generator().manual_seed(big)
+        x, p = randn(gen, 2, *hw, 16).to(dtype), randn(gen, 2, *out, 16).to(dtype)
+        xd, pd = x.cuda().requires_grad_(), p.cuda().requires_grad_()
+        y, u = P.OptimizedAdaptiveAvgPool2d(out)(xd), P.OptimizedBilinearInterp2d(hw)(pd)
+        assert_close(y, oracle.avgpool_fwd(x.double().numpy(), out), dtype, "pool")
+        torch.autograd.backward([y, u], [p.cuda(), x.cuda()])
+        assert_close(xd.grad, oracle.avgpool_bwd(p.double().numpy(), hw), dtype, "pool's gradient")
+        assert_close(pd.grad, oracle.bilinear_bwd(x.double().numpy(), out), dtype, "resize's gradient")
