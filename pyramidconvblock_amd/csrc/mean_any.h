@@ -215,6 +215,94 @@ __device__ __forceinline__ void mean_fwd_body(const MeanJob& j, int wg, float* s
     }
 }
 
+// The same by workgroups of half as many features each, with everything that can be in flight so: what takes the time is trips to memory one after the
+// other.  Sixteen partials at once, the first weights requested before them, and eight at a time.  124 registers: for launches whose other
+// workgroups are all on the chip with those too (gate_pair_mean_fwd_launch).
+constexpr int kMeanFew = 32;
+template <typename T>
+__device__ __forceinline__ void mean_fwd_deep_body(const MeanJob& j, int wg, float* sm) {
+    constexpr int V = 16 / (int)sizeof(T);
+    typedef ChanVec<T, V> Vec;
+    const int D = j.D, d4 = D / 4, slices = (D + kMeanFew - 1) / kMeanFew, b = wg / slices, sl = wg - b * slices, tid = threadIdx.x;
+    const int sub = tid & 7, nv = D / V, o = sl * kMeanFew + (tid >> 3);
+    // vector v of the thread's feature (past the end: the last one, which is not added)
+    auto weight = [&](int v) { return *reinterpret_cast<const Vec*>((const T*)j.wp + (uint32_t)(min(o, D - 1) * D + min(v, nv - 1) * V)); };
+    Vec pre[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) pre[u] = weight(sub + 8 * u);
+    // sums: two columns of four a thread (c, c + L) over every QL-th partial; past the end the last one, not added
+    {
+        float4* const red = reinterpret_cast<float4*>(sm + D);
+        const float* const pp = j.part + (long long)b * j.n * D;
+        const int n = j.n, L = min((d4 + 1) / 2, 256), QL = 256 / L, ql = tid / L, cl = tid - ql * L;
+        for (int c0 = 0; c0 < d4; c0 += 2 * L) {   // (more than once only where QL = 1)
+            float4 s[2] = {make_float4(0.f, 0.f, 0.f, 0.f), make_float4(0.f, 0.f, 0.f, 0.f)};
+            const int c1 = c0 + cl, c[2] = {min(c1, d4 - 1), min(c1 + L, d4 - 1)};
+            if (ql < QL)
+                for (int q = ql; q < n; q += 8 * QL) {
+                    float4 v[8][2];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+#pragma unroll
+                        for (int k = 0; k < 2; ++k) v[u][k] = *reinterpret_cast<const float4*>(pp + (uint32_t)(min(q + u * QL, n - 1) * D + c[k] * 4));
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        if (q + u * QL < n) {
+#pragma unroll
+                            for (int k = 0; k < 2; ++k) s[k].x += v[u][k].x, s[k].y += v[u][k].y, s[k].z += v[u][k].z, s[k].w += v[u][k].w;
+                        }
+                }
+            if (QL > 1) {
+                if (ql < QL) red[ql * 2 * L + cl] = s[0], red[(ql * 2 + 1) * L + cl] = s[1];
+                __syncthreads();
+                if (ql == 0)
+                    for (int q = 1; q < QL; ++q)
+#pragma unroll
+                        for (int k = 0; k < 2; ++k) {
+                            const float4 v = red[(q * 2 + k) * L + cl];
+                            s[k].x += v.x, s[k].y += v.y, s[k].z += v.z, s[k].w += v.w;
+                        }
+            }
+            if (ql == 0) {
+#pragma unroll
+                for (int k = 0; k < 2; ++k)
+                    if (c1 + k * L < min(d4, c0 + (k + 1) * L)) *reinterpret_cast<float4*>(sm + (c1 + k * L) * 4) = s[k];
+            }
+        }
+        __syncthreads();
+    }
+    for (int c = tid; c < D; c += 256) {
+        const T mv = from_f32<T>(sm[c] * j.inv_p);
+        if (sl == 0) ((T*)j.m)[(long long)b * D + c] = mv;
+        sm[c] = to_f32(mv);
+    }
+    __syncthreads();
+    float acc = 0.f;   // (mean_fwd_body's order)
+    auto add = [&](const Vec& w, int v) {
+        if (v < nv) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) acc = fmaf(sm[v * V + e], to_f32(w.v[e]), acc);
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < 4; ++u) add(pre[u], sub + 8 * u);
+    for (int v = sub + 32; v < nv; v += 64) {
+        Vec wv[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) wv[u] = weight(v + 8 * u);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) add(wv[u], v + 8 * u);
+    }
+    acc += __shfl_xor(acc, 1);
+    acc += __shfl_xor(acc, 2);
+    acc += __shfl_xor(acc, 4);
+    if (sub == 0 && o < D) {
+        if (j.bp) acc += to_f32(((const T*)j.bp)[o]);
+        if (j.bo) acc += to_f32(((const T*)j.bo)[o]);
+        j.rowbias[(long long)b * D + o] = acc;
+    }
+}
+
 // By a workgroup of NT threads.
 template <typename T, int NT, int IM>
 __device__ __forceinline__ void mean_bwd_images(const MeanJob& j, int wg, float* sm) {

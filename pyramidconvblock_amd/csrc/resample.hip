@@ -734,14 +734,17 @@ __global__ __launch_bounds__(256) void gate_pair_fwd_k(const T* __restrict__ xf,
 }
 
 // The same with the mean branch (mean_any.h) in the first workgroups.
-template <typename T, int VEC>
+template <typename T, int VEC, bool DEEP>
 __global__ __launch_bounds__(256) void gate_pair_mean_fwd_k(const T* __restrict__ xf, const T* __restrict__ xh,
                                                             T* __restrict__ y, int h, int w, int I, int H, int W, int ldy,
                                                             float sy, float sx, float s, unsigned nblk_full,
                                                             long long total_full, long long total_half, const MeanJob mean,
                                                             unsigned nmean) {
     extern __shared__ float sm[];
-    if (blockIdx.x < nmean) return mean_fwd_body<T>(mean, blockIdx.x, sm);
+    if (blockIdx.x < nmean) {
+        if constexpr (DEEP) return mean_fwd_deep_body<T>(mean, blockIdx.x, sm);
+        else return mean_fwd_body<T>(mean, blockIdx.x, sm);
+    }
     gate_pair_fwd_body<T, VEC>(xf, xh, y, h, w, I, H, W, ldy, sy, sx, s, nblk_full, total_full, total_half, blockIdx.x - nmean);
 }
 
@@ -1585,14 +1588,20 @@ int gate_pair_mean_fwd_launch(const void* xf, const void* xh, void* y, int B, in
     const long long tf = (long long)B * H * W * (I / 2 / vec);
     const long long th = (H == 2 * h && W == 2 * w) ? (long long)B * h * w * (I / 2 / vec) : tf;
     unsigned bf, bh;
-    const unsigned nmean = (unsigned)(B * mean_slices(mean.D));
-    if (!grid_for((tf + kGateItems - 1) / kGateItems, &bf) || !grid_for(th, &bh) ||
-        (unsigned long long)bf + bh + nmean > 0x7fffffffULL)
-        return 1;
+    if (!grid_for((tf + kGateItems - 1) / kGateItems, &bf) || !grid_for(th, &bh)) return 1;
+    // (us: [4,64,64,1152] fp16 17.5 -> 12.7, [2,15,15,960] bf16 11.1 -> 7.8, [4,27,27,992] fp32 13.4 -> 10.7, [2,40,40,640] 9.6 -> 7.5, [3,8,8,632]
+    // 6.0 -> 5.4; of several rounds, at fewer workgroups a unit, [27,15,15,624] 8.0 -> 9.2,
+    // [104,27,28,280] 17.4 -> 18.6; narrow, one trip either way, [2,32,32,64] fp32 4.0 -> 4.5)
+    const unsigned ndeep = (unsigned)B * (unsigned)cdiv(mean.D, kMeanFew);
+    const bool deep = mean.D >= 256 && (unsigned long long)bf + bh + ndeep <= 1024;   // (four to a compute unit)
+    const unsigned nmean = deep ? ndeep : (unsigned)(B * mean_slices(mean.D));
+    if ((unsigned long long)bf + bh + nmean > 0x7fffffffULL) return 1;
     const float sy = (float)h / (float)H, sx = (float)w / (float)W, sc = sqrtf((float)(gw > 0 ? gw : I / 2));
-#define CALL(T, V) hipLaunchKernelGGL((gate_pair_mean_fwd_k<T, V>), dim3(bf + bh + nmean), dim3(256), mean_lds(mean.D), s, (const T*)xf, (const T*)xh, (T*)y, h, w, I, H, W, ldy, sy, sx, sc, bf, tf, th, mean, nmean);
+#define GO(T, V, DEEP) hipLaunchKernelGGL((gate_pair_mean_fwd_k<T, V, DEEP>), dim3(bf + bh + nmean), dim3(256), mean_lds(mean.D), s, (const T*)xf, (const T*)xh, (T*)y, h, w, I, H, W, ldy, sy, sx, sc, bf, tf, th, mean, nmean)
+#define CALL(T, V) if (deep) GO(T, V, true); else GO(T, V, false);
     PDW_TYPE_SWITCH(dtype, vec, CALL)
 #undef CALL
+#undef GO
     return check_launch("gate_pair_mean_fwd");
 }
 

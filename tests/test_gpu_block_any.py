@@ -52,6 +52,9 @@ def test_weights_read_as_given_and_packed_beside_the_pool(oracle, dim, inter, k,
 @pytest.mark.parametrize("dtype,dim,k,shape", [
     (torch.bfloat16, 16, 5, (5, 11, 13, 16)), (torch.float16, 72, 3, (2, 90, 90, 72)), (torch.bfloat16, 1032, 3, (1, 7, 9, 1032)),
     (torch.float32, 36, 5, (3, 17, 12, 36)), (torch.float32, 252, 3, (40, 9, 8, 252)), (torch.float16, 256, 3, (70, 6, 6, 256)),
+    # the forward with everything in flight: a last slice of 4, 8 and 16 features, one partial and many, more columns than twice the threads
+    (torch.float32, 260, 3, (3, 9, 8, 260)), (torch.float16, 264, 3, (2, 30, 33, 264)), (torch.bfloat16, 272, 3, (1, 41, 64, 272)),
+    (torch.bfloat16, 2056, 3, (2, 5, 4, 2056)), (torch.float32, 2080, 3, (1, 4, 6, 2080)),
     # four images to a workgroup of its backward: a rest of one and of two, sums of one and of several ranges
     (torch.bfloat16, 264, 3, (41, 6, 6, 264)), (torch.float16, 136, 3, (66, 5, 6, 136)), (torch.bfloat16, 520, 3, (22, 16, 18, 520)),
 ])
