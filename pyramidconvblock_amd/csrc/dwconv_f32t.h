@@ -40,7 +40,8 @@ namespace pdw {
 // compute unit; the others are read again from the filter table in LDS for every product (a fifth of its rate).  us, all in registers and one
 // workgroup a unit -> this: both scales of [32,56,56,64] filter 13 50.5 -> 45.5, [22,72,73,32] filter 13 36.6 -> 32.2, [3,57,61,100]
 // filter 15 24.2 -> 18.2, [16,56,56,64] filter 15 38.9 -> 33.3, [24,36,36,100] filter 17 57.0 -> 50.7, [2,20,20,32] filter 15 9.0 -> 8.5.  With the pooled
-// gradient added (ADD > 0), which the planner cuts into one workgroup a unit, all stay ([3,57,61,100] filter 15 21.5, 25.0 with two blocks kept),
+// gradient added (ADD > 0), which the planner cuts into one workgroup a unit, all stay ([32,56,56,64] filter 13 38.3, 39.2 with three
+// blocks kept, [24,36,36,100] filter 17 35.8 and 36.6),
 // and in launches of no more than that with long bands (ADD = -1: [32,56,56,64] filter 13 38.7, 39.7 with three blocks kept).
 template <int K, int ADD>
 constexpr int f32t_kept() {
@@ -227,11 +228,21 @@ __device__ __forceinline__ void dwconv_f32_body(const float* __restrict__ x, con
     uint32_t aoff = 0;
     float wj0 = 0.f, wj1 = 0.f, wi0 = 0.f, wi1 = 0.f;
     f4 addv[ADD == 2 ? 4 : 1];
+    float* const bins = reinterpret_cast<float*>(xl + Sh::lds_bytes);   // ADD 2: (byte offset of the first bin, both weights) of the band's rows
     if constexpr (ADD > 0) {
         arsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(add + (long long)b0 * g.AH * g.AW * g.C), (short)0,
                                                   (int)((long long)min(NI, g.B - b0) * g.AH * g.AW * g.C * 4), 0x00020000);
-        if constexpr (ADD == 2) pool_bins(min(ocol0 + scol, g.OW - 1), g.OW, g.AW, jb0, wj0, wj1);
-        else aoff = s_ok ? ((uint32_t)((simg * g.AH + (srow >> 1)) * g.AW + ((ocol0 + scol) >> 1)) * (uint32_t)g.C + (uint32_t)(c0 + 4 * sq)) * 4u : kNoRow;
+        if constexpr (ADD == 2) {
+            // (read by the first add_fetch of a row in it behind the first step's barrier)
+            for (int i = tid; i < rows_valid; i += NT) {
+                int b;
+                float w0, w1;
+                pool_bins(orow0 + i, g.OH, g.AH, b, w0, w1);
+                bins[4 * i] = __builtin_bit_cast(float, (uint32_t)(b * g.AW * g.C) * 4u), bins[4 * i + 1] = w0, bins[4 * i + 2] = w1;
+            }
+            pool_bins(min(ocol0 + scol, g.OW - 1), g.OW, g.AW, jb0, wj0, wj1);
+            aoff = ((uint32_t)(simg * g.AH * g.AW + jb0) * (uint32_t)g.C + (uint32_t)(c0 + 4 * sq)) * 4u;
+        } else aoff = s_ok ? ((uint32_t)((simg * g.AH + (srow >> 1)) * g.AW + ((ocol0 + scol) >> 1)) * (uint32_t)g.C + (uint32_t)(c0 + 4 * sq)) * 4u : kNoRow;
     }
     auto add_fetch = [&](int pr) {   // the bins of patch row pr's pixels
         if constexpr (ADD == 1) {
@@ -241,11 +252,12 @@ __device__ __forceinline__ void dwconv_f32_body(const float* __restrict__ x, con
             const int at = pr >= 0 && 4 * pr < rows_valid ? ((orow0 + 4 * pr) >> 1) * g.AW * g.C * 4 : 0;
             addv[0] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(arsrc, (int)o, at, 0));
         } else if constexpr (ADD == 2) {
-            int ib0;
-            const int row = orow0 + 4 * pr + srow;
-            pool_bins(min(max(row, 0), g.OH - 1), g.OH, g.AH, ib0, wi0, wi1);
+            // (from the table: found anew for every row they were 600 cycles a step that no product covers; us: [3,57,61,100] filter 15 21.4 ->
+            // 19.2, [22,72,73,32] filter 13 33.4 -> 29.2, [8,47,48,128] filter 17 33.0 -> 29.0, [8,27,31,40] filter 11 11.7 -> 9.2)
+            const float4 bin = *reinterpret_cast<const float4*>(bins + 4 * min(max(4 * pr + srow, 0), rows_valid - 1));
+            wi0 = bin.y, wi1 = bin.z;
             const bool ok = s_ok && pr >= 0 && 4 * pr + srow < rows_valid;
-            const uint32_t o = ((uint32_t)((simg * g.AH + ib0) * g.AW + jb0) * (uint32_t)g.C + (uint32_t)(c0 + 4 * sq)) * 4u;
+            const uint32_t o = aoff + __builtin_bit_cast(uint32_t, bin.x);
             const uint32_t dx = (uint32_t)g.C * 4u, dy = (uint32_t)(g.AW * g.C) * 4u;
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
@@ -352,6 +364,7 @@ __device__ __forceinline__ void dwconv_f32_body(const float* __restrict__ x, con
         issue(bf, s + 3);
         if (wv >= 4 && s < nsteps) compute(half, s);
     };
+    if constexpr (ADD == 2) lds_barrier();   // (the bins)
     add_fetch(-1);
     // (the two buffers by name and no way out between them: the compiler can then tell which requests are the newest, and a
     // commit waits for its own alone)
@@ -456,7 +469,8 @@ int launch_f32t(const void* x, const void* w, const void* add, void* y, int B, i
         auto kern = dwconv_f32t_k<K, NPC, A>;                                                                              \
         static std::once_flag once;                                                                                        \
         std::call_once(once, [&] { (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); }); \
-        constexpr size_t lds = F32Shape<K, NPC, A>::lds_bytes;                                                                \
+        const size_t lds = F32Shape<K, NPC, A>::lds_bytes + (A == 2 ? (size_t)(g.BR < g.OH ? g.BR : g.OH) * 16 : 0);          \
+        if (lds > 160 * 1024) return -1;                                                                                   \
         hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(512), lds, s, (const float*)x, (const float*)w,             \
                            (const float*)add, (float*)y, g);                                                               \
     }
