@@ -227,7 +227,7 @@ static void bwd3_go(const Bwd3Args& a, unsigned grid, size_t lds, hipStream_t s)
 }
 
 // -1: not covered (the caller makes the three launches).  16-bit types, C % 8 == 0, padding K / 2; the full scale
-// [B, H, W, C], the pooled one [B, h, w, C].  addp (optional, H = 2 h and W = 2 w): the pooled branch's gradient.
+// [B, H, W, C], the pooled one [B, h, w, C].  addp (optional; H = 2 h and W = 2 w or dwconv_bwd3_adds_any): the pooled branch's gradient.
 // x1 = nullptr and h = 0: no pooled scale (a convolution by itself; -1 also where two launches take no longer).
 template <int K>
 static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* dx, const void* x0, void* dw0, void* ws0,
@@ -236,7 +236,8 @@ static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* 
     constexpr int CS = (2 * 4 * TzShape<K, 16, 16>::NM + 2 * 4 * TzShape<K, 16, 16>::RING) <= 160 ? 16 : 8;
     const bool one = h == 0;
     if (dtype == kF32 || C % 8 != 0 || B < 1 || H < 1 || W < 1 || (!one && (h < 1 || w < 1))) return -1;
-    if (addp && (H != 2 * h || W != 2 * w)) return -1;
+    const bool any = addp && (H != 2 * h || W != 2 * w);
+    if (any && (one || h > H || w > W || !dwconv_bwd3_adds_any(K))) return -1;
     const int P = K / 2;
     if (!plan_out)
         for (const void* p : {gyf, w0, (const void*)dx, x0, (const void*)ws0, one ? x0 : x1, one ? gyf : gy1, (const void*)(one ? ws0 : ws1)})
@@ -291,13 +292,17 @@ static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* 
             if (ord[i] == 'F') a.p[0].start = at, at += a.p[0].n;
         }
     }
+    if (any) a.gd.AH = h, a.gd.AW = w;
     size_t lds = a.npcd == 16 ? TzShape<K, 16, CS>::lds_bytes : TzShape<K, 8, CS>::lds_bytes;
+    if (any) lds = (size_t)(a.npcd == 16 ? TzShape<K, 16, CS>::bins_at : TzShape<K, 8, CS>::bins_at) + 16 * (size_t)H;
+    if (lds > 160 * 1024) return -1;
     lds = std::max(lds, WgPhShape<wgrad_ph_ncopy(K), wgrad_ph_gr(K)>::lds_bytes);
     if (nmean) lds = std::max(lds, mean_lds(job.D, 512, job.shared ? kMeanImages : 1));
     const unsigned grid = (unsigned)grid_all;
     auto go = [&](auto t) {
         using T = decltype(t);
         if (!addp) bwd3_go<T, K, CS, false, 0>(a, grid, lds, s);
+        else if (any) bwd3_go<T, K, CS, false, dwconv_bwd3_adds_any(K) ? 16 : 0>(a, grid, lds, s);
         else if (a.npcd == 16 && nmean == 0) bwd3_go<T, K, CS, true, 1>(a, grid, lds, s);
         else bwd3_go<T, K, CS, false, 1>(a, grid, lds, s);
     };

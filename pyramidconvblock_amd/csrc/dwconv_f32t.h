@@ -77,18 +77,6 @@ struct F32Geom {
     int B, H, W, C, OH, OW, PH, PW, BR, nbands, ncolt, nslices, flip, AH, AW;
 };
 
-// Bins of an adaptive average pool of `in` values to `out` <= in that value i lies in: the first, and the weights (one
-// over the bin's length; 0: no second bin).
-__device__ __forceinline__ void pool_bins(int i, int in, int out, int& b0, float& w0, float& w1) {
-    b0 = (int)((unsigned)(i * out) / (unsigned)in);
-    const int b1 = (int)((unsigned)((i + 1) * out + in - 1) / (unsigned)in) - 1;
-    auto len = [&](int b) {
-        return (int)((unsigned)((b + 1) * in + out - 1) / (unsigned)out) - (int)((unsigned)(b * in) / (unsigned)out);
-    };
-    w0 = 1.f / (float)len(b0);
-    w1 = b1 > b0 ? 1.f / (float)len(b1) : 0.f;
-}
-
 template <int K, int NPC, int ADD>
 __device__ __forceinline__ void dwconv_f32_body(const float* __restrict__ x, const float* __restrict__ w,
                                                 const float* __restrict__ add, float* __restrict__ y, const F32Geom& g, int blk,

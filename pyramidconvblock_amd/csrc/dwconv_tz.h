@@ -37,7 +37,8 @@
 // runs 1.15 us a step 0.97; what does not overlap yet is the LDS round trips either side of the barrier.
 //
 // MODE is a set of bits.
-// 1 (input gradient of a tensor that was also average-pooled 2x2): y += add[i/2, j/2] / 4 in the store.
+// 1 (input gradient of a tensor that was also average-pooled 2x2): y += add[i/2, j/2] / 4 in the store; 16: that of a pool
+// of any ratio down to AH x AW, from the at most 2 x 2 bins that a pixel lies in.
 // 2 (forward): the 2x2 average pool of x is written to `pool` by the staging threads, which hold exactly the
 // four pixels of a pool window in registers (needs even padding, so that windows do not straddle threads).
 // 4 (forward, inference): the gate of conv_block.py:18-19 in the store.  A workgroup's 16 channels are 8 of the first
@@ -113,6 +114,7 @@ struct TzShape {
     // long, of up to 1024 1.2, beyond 1.36.)
     static constexpr int ENDS = NI * CS * CHP + R2B;
     static constexpr int spare(bool pool) { return pool ? ENDS : NRR * RP; }
+    static constexpr int bins_at = (ENDS + 15) / 16 * 16;   // (MODE & 16) 16 bytes an output row
     static constexpr size_t lds_bytes = ENDS, lds_bytes_pool = (size_t)ENDS + 7 * CHP + RP + 16;
     static_assert(lds_bytes_pool <= 160 * 1024, "LDS");
     static_assert(K > 5 || lds_bytes <= 80 * 1024, "two workgroups on a compute unit");
@@ -161,6 +163,22 @@ __device__ __forceinline__ uint4 tz_add_quarter(uint4 a, uint4 b) {
     return uo.u;
 }
 
+// 8 values of T: a + the weighted gradients of up to four bins, in avgpool_bwd_k's order, rounded once more.
+template <typename T>
+__device__ __forceinline__ uint4 tz_add_bins(uint4 a, const uint4 (&b)[4], float w0, float w1, float w2, float w3) {
+    union U {
+        uint4 u;
+        T t[8];
+    } ua, ub[4], uo;
+    ua.u = a;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) ub[k].u = b[k];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        uo.t[i] = from_f32<T>(to_f32(ua.t[i]) + fmaf(to_f32(ub[3].t[i]), w3, fmaf(to_f32(ub[2].t[i]), w2, fmaf(to_f32(ub[1].t[i]), w1, to_f32(ub[0].t[i]) * w0))));
+    return uo.u;
+}
+
 // 4 values of T: a * b * s, rounded once (the arithmetic of the stand-alone gate kernel).
 template <typename T>
 __device__ __forceinline__ uint2 tz_gate(uint2 a, uint2 b, float s) {
@@ -198,7 +216,7 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
     constexpr int NT = Sh::NT, NG = Sh::NG, ICB = Sh::ICB, NKG = Sh::NKG, NM = Sh::NM, PER = Sh::PER, RING = Sh::RING;
     constexpr int NI = Sh::NI, TW = Sh::TW, NH = Sh::NH, CPW = Sh::CPW, RP = Sh::RP, OPX = Sh::OPX, OROWP = Sh::OROWP;
     constexpr int OLB = Sh::OLB, WTH = Sh::WTH, WTW = Sh::WTW, NR = Sh::NR, NRR = Sh::NRR, CHP = Sh::CHP;
-    constexpr bool ADD = (MODE & 1) != 0, POOL = (MODE & 2) != 0, GATE = (MODE & 4) != 0;
+    constexpr bool ANY = (MODE & 16) != 0, ADD = (MODE & 1) != 0 || ANY, POOL = (MODE & 2) != 0, GATE = (MODE & 4) != 0;
     constexpr int SHORT = (MODE & 8) != 0 ? tz_short(K) : 0, PASSES = SHORT ? SHORT + 1 : 4;   // steps of a run at most; passes before them
     static_assert(!GATE || !ADD, "the gate is a forward mode");
     static_assert(!(SHORT && POOL), "short runs do not write the pool");
@@ -502,19 +520,36 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
     if constexpr (ADD)
         arsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(add + (long long)b0 * g.AH * g.AW * g.C), (short)0,
                                                   (int)((long long)images * g.AH * g.AW * g.C * 2), 0x00020000);
-    uint4 addv[NG];
+    constexpr int NA = ANY ? 4 : 1;   // addends of a piece
+    uint4 addv[NG][NA];
+    // ANY: the bins of an image's rows in LDS (byte offset of the first, both weights), of the thread's column in registers
+    float* const bins = reinterpret_cast<float*>(xl + Sh::bins_at);
+    int jb0 = 0;
+    float wj0 = 0.f, wj1 = 0.f, wi0[NG] = {}, wi1[NG] = {};
+    if constexpr (ANY) {
+        for (int i = tid; i < g.OH; i += NT) {   // (read behind the barrier that publishes the first passes)
+            int b;
+            float w0, w1;
+            pool_bins(i, g.OH, g.AH, b, w0, w1);
+            bins[4 * i] = __builtin_bit_cast(float, (uint32_t)(b * g.AW * g.C) * 2u), bins[4 * i + 1] = w0, bins[4 * i + 2] = w1;
+        }
+        pool_bins(min(ocol0 + scol, g.OW - 1), g.OW, g.AW, jb0, wj0, wj1);
+    }
     // a step's 8 rows lie in one image (group): its first row there, and the byte offsets of that row in y and the addend
     int orow = orow0, rleft = rows_valid;   // rleft: rows of the run from this step on
     const uint32_t row_out = (uint32_t)(g.OW * g.YC) * 2u, group_out = (uint32_t)img_out * (uint32_t)NI * 2u;
     const uint32_t row_add = (uint32_t)(g.AW * g.C) * 2u, group_add = (uint32_t)(NI * g.AH) * row_add;
-    uint32_t ooff = (uint32_t)orow * row_out, aoff = (uint32_t)(orow >> 1) * row_add, stored = 0;   // stored: ooff of the step before
+    uint32_t ooff = (uint32_t)orow * row_out, aoff = ANY ? 0u : (uint32_t)(orow >> 1) * row_add, stored = 0;   // stored: ooff of the step before
     uint32_t ylane[NG], alane[NG], yoff[NG];   // the thread's piece from there (rows srow or srow + 4); yoff: or the marker
 #pragma unroll
     for (int n = 0; n < NG; ++n) {
         const int r = 4 * tile_of(n) + srow;
         ylane[n] = s_ok ? ycol * 2u + (uint32_t)r * row_out : kNoRow;
-        alane[n] = s_ok ? (uint32_t)(((simg * g.AH + (r >> 1)) * g.AW + ((ocol0 + scol) >> 1)) * g.C + c0 + 8 * sh) * 2u : kNoRow;
-        yoff[n] = kNoRow, addv[n] = make_uint4(0u, 0u, 0u, 0u);
+        if constexpr (ANY) alane[n] = (uint32_t)((simg * g.AH * g.AW + jb0) * g.C + c0 + 8 * sh) * 2u;
+        else alane[n] = s_ok ? (uint32_t)(((simg * g.AH + (r >> 1)) * g.AW + ((ocol0 + scol) >> 1)) * g.C + c0 + 8 * sh) * 2u : kNoRow;
+        yoff[n] = kNoRow;
+#pragma unroll
+        for (int t = 0; t < NA; ++t) addv[n][t] = make_uint4(0u, 0u, 0u, 0u);
     }
     // The next step: the offsets its tiles are stored at, and the addends.  (A step between images moves nothing and takes no scalar
     // offset: behind images of one to three rows it could lie past the descriptor's end, from which the range check subtracts it.)
@@ -524,13 +559,26 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
         for (int n = 0; n < NG; ++n) {
             const bool ok = 4 * tile_of(n) + srow < lim;
             yoff[n] = ok ? ylane[n] : kNoRow;
-            if constexpr (ADD) addv[n] = xload_from(arsrc, ok ? alane[n] : kNoRow, lim > 0 ? aoff : 0);
+            if constexpr (ANY) {
+                const bool in = ok && s_ok;
+                const float4 bin = *reinterpret_cast<const float4*>(bins + 4 * (ok ? orow + 4 * tile_of(n) + srow : 0));
+                const uint32_t o = alane[n] + __builtin_bit_cast(uint32_t, bin.x);
+                wi0[n] = bin.y, wi1[n] = bin.z;
+                const bool right = in && wj1 != 0.f, below = in && wi1[n] != 0.f;
+                const uint32_t at = lim > 0 ? aoff : 0;
+                addv[n][0] = xload_from(arsrc, in ? o : kNoRow, at);
+                addv[n][1] = xload_from(arsrc, right ? o + 2u * (uint32_t)g.C : kNoRow, at);
+                addv[n][2] = xload_from(arsrc, below ? o + row_add : kNoRow, at);
+                addv[n][3] = xload_from(arsrc, right && below ? o + row_add + 2u * (uint32_t)g.C : kNoRow, at);
+            } else if constexpr (ADD) {
+                addv[n][0] = xload_from(arsrc, ok ? alane[n] : kNoRow, lim > 0 ? aoff : 0);
+            }
         }
         stored = lim > 0 ? ooff : 0;
         rleft -= 8, orow += 8;
         const bool wrap = orow >= g.per;
         ooff += wrap ? group_out - (uint32_t)(orow - 8) * row_out : 8u * row_out;
-        aoff += wrap ? group_add - (uint32_t)((orow - 8) >> 1) * row_add : 4u * row_add;
+        aoff += ANY ? (wrap ? group_add : 0u) : wrap ? group_add - (uint32_t)((orow - 8) >> 1) * row_add : 4u * row_add;
         orow = wrap ? 0 : orow;
     };
     auto tile_read = [&](int f, int n) {
@@ -548,7 +596,8 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
         }
     };
     auto tile_store = [&](uint4 v, int n) {   // where place() put it
-        if constexpr (ADD) v = tz_add_quarter<T>(v, addv[n]);
+        if constexpr (ANY) v = tz_add_bins<T>(v, addv[n], wi0[n] * wj0, wi0[n] * wj1, wi1[n] * wj0, wi1[n] * wj1);
+        else if constexpr (ADD) v = tz_add_quarter<T>(v, addv[n][0]);
         if constexpr (GATE) {
             const uint2 o = tz_gate<T>(make_uint2(v.x, v.y), make_uint2(v.z, v.w), g.gs);
             typedef unsigned v2u __attribute__((ext_vector_type(2)));

@@ -67,6 +67,18 @@ __device__ __forceinline__ void pack_pairs(const ChanVec<T, V>& a, const ChanVec
     }
 }
 
+// Bins of an adaptive average pool of `in` values to `out` <= in that value i lies in: the first, and the weights (one
+// over the bin's length; 0: no second bin).
+__device__ __forceinline__ void pool_bins(int i, int in, int out, int& b0, float& w0, float& w1) {
+    b0 = (int)((unsigned)(i * out) / (unsigned)in);
+    const int b1 = (int)((unsigned)((i + 1) * out + in - 1) / (unsigned)in) - 1;
+    auto len = [&](int b) {
+        return (int)((unsigned)((b + 1) * in + out - 1) / (unsigned)out) - (int)((unsigned)(b * in) / (unsigned)out);
+    };
+    w0 = 1.f / (float)len(b0);
+    w1 = b1 > b0 ? 1.f / (float)len(b1) : 0.f;
+}
+
 // XCD-aware work order: consecutive workgroup ids go to the 8 XCDs round-robin, so give each
 // XCD a contiguous range of work items (neighbouring tiles of one image share an L2).
 __device__ __forceinline__ int xcd_remap(int bid, int nblocks) {

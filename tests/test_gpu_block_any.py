@@ -140,3 +140,33 @@ def test_pool_and_sums_beside_large_products(monkeypatch, dtype, dim, shape):
 def test_fp32_half_scale_beside_the_weight_gradients(oracle, k, dim, shape):
     """Both weight gradients and the pooled scale's input gradient as one launch (csrc/dwconv_wgrad_f32t.h)."""
     _block_case(oracle, dim, k, shape, torch.float32)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("k", [3, 5, 7, 9, 11, 15, 17])
+@pytest.mark.parametrize("shape,second", [
+    # one bin a pixel and two, on either axis; runs over images of fewer rows than a step and of many; narrow and wide tiles; a last slice
+    # of 8 channels; every pixel a bin of its own on one axis
+    ((3, 57, 61, 48), 0.5), ((5, 7, 9, 16), 0.5), ((33, 15, 15, 32), 0.5), ((2, 3, 70, 48), 0.5), ((3, 31, 32, 16), 1 / 3), ((2, 20, 23, 32), 0.75),
+    ((2, 9, 66, 16), 0.95),
+])
+def test_pooled_gradient_of_any_ratio_in_the_store(oracle, dtype, k, shape, second):
+    """16-bit blocks whose pooled extents are no exact halves: the pool's gradient is added where the full scale's input gradient is stored
+    (csrc/dwconv_tz.h, MODE 16; filter 11: by the launch behind it)."""
+    import pyramid_dwconv
+
+    torch.manual_seed(2)
+    dim = shape[3]
+    m = pyramid_dwconv.ConvBlock(dim=dim, kernel_size=k, scales=(1.0, second)).to(dtype)
+    x, g = (torch.randn(*shape).to(dtype) for _ in range(2))
+    params = {n: p.detach().double().numpy() for n, p in m.state_dict().items()}
+    yo, cache = oracle.convblock_fwd(x.double().numpy(), params, scales=(1.0, second))
+    dxo, go = oracle.convblock_bwd(cache, g.double().numpy())
+    m = m.cuda()
+    xd = x.cuda().requires_grad_()
+    y = m(xd)
+    assert_close(y, yo, dtype, "y")
+    torch.autograd.backward(y, g.cuda())
+    assert_close(xd.grad, dxo, dtype, "dx")
+    for n, p in m.named_parameters():
+        assert_close(p.grad, go[n], dtype, "grad " + n)
