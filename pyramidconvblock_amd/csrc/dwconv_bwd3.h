@@ -294,7 +294,7 @@ static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* 
     }
     if (any) a.gd.AH = h, a.gd.AW = w;
     size_t lds = a.npcd == 16 ? TzShape<K, 16, CS>::lds_bytes : TzShape<K, 8, CS>::lds_bytes;
-    if (any) lds = (size_t)(a.npcd == 16 ? TzShape<K, 16, CS>::bins_at : TzShape<K, 8, CS>::bins_at) + 16 * (size_t)H;
+    if (any) lds = (size_t)(a.npcd == 16 ? TzShape<K, 16, CS>::bins_at : TzShape<K, 8, CS>::bins_at) + 8 * (size_t)H;
     if (lds > 160 * 1024) return -1;
     lds = std::max(lds, WgPhShape<wgrad_ph_ncopy(K), wgrad_ph_gr(K)>::lds_bytes);
     if (nmean) lds = std::max(lds, mean_lds(job.D, 512, job.shared ? kMeanImages : 1));

@@ -114,7 +114,7 @@ struct TzShape {
     // long, of up to 1024 1.2, beyond 1.36.)
     static constexpr int ENDS = NI * CS * CHP + R2B;
     static constexpr int spare(bool pool) { return pool ? ENDS : NRR * RP; }
-    static constexpr int bins_at = (ENDS + 15) / 16 * 16;   // (MODE & 16) 16 bytes an output row
+    static constexpr int bins_at = (ENDS + 15) / 16 * 16;   // (MODE & 16) 8 bytes an output row
     static constexpr size_t lds_bytes = ENDS, lds_bytes_pool = (size_t)ENDS + 7 * CHP + RP + 16;
     static_assert(lds_bytes_pool <= 160 * 1024, "LDS");
     static_assert(K > 5 || lds_bytes <= 80 * 1024, "two workgroups on a compute unit");
@@ -163,7 +163,8 @@ __device__ __forceinline__ uint4 tz_add_quarter(uint4 a, uint4 b) {
     return uo.u;
 }
 
-// 8 values of T: a + the weighted gradients of up to four bins, in avgpool_bwd_k's order, rounded once more.
+// 8 values of T: a + the weighted gradients of up to four bins, rounded once more: avgpool_bwd_k's sum to the bit (bins that are not there are
+// zeros).
 template <typename T>
 __device__ __forceinline__ uint4 tz_add_bins(uint4 a, const uint4 (&b)[4], float w0, float w1, float w2, float w3) {
     union U {
@@ -175,7 +176,7 @@ __device__ __forceinline__ uint4 tz_add_bins(uint4 a, const uint4 (&b)[4], float
     for (int k = 0; k < 4; ++k) ub[k].u = b[k];
 #pragma unroll
     for (int i = 0; i < 8; ++i)
-        uo.t[i] = from_f32<T>(to_f32(ua.t[i]) + fmaf(to_f32(ub[3].t[i]), w3, fmaf(to_f32(ub[2].t[i]), w2, fmaf(to_f32(ub[1].t[i]), w1, to_f32(ub[0].t[i]) * w0))));
+        uo.t[i] = from_f32<T>(to_f32(ua.t[i]) + fmaf(to_f32(ub[3].t[i]), w3, fmaf(to_f32(ub[2].t[i]), w2, fmaf(to_f32(ub[1].t[i]), w1, fmaf(to_f32(ub[0].t[i]), w0, 0.f)))));
     return uo.u;
 }
 
@@ -522,18 +523,24 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
                                                   (int)((long long)images * g.AH * g.AW * g.C * 2), 0x00020000);
     constexpr int NA = ANY ? 4 : 1;   // addends of a piece
     uint4 addv[NG][NA];
-    // ANY: the bins of an image's rows in LDS (byte offset of the first, both weights), of the thread's column in registers
-    float* const bins = reinterpret_cast<float*>(xl + Sh::bins_at);
+    // ANY: the bins of an image's rows in LDS, as the byte offset of the first and bits: it is the longer of the two lengths that bins have, there is
+    // a second, that is the longer.  A bin's weight is one over its pixels, for a thread's column one of two by the row's bin (a product of one
+    // over each length is 7e-8 off for 3 x 3 pixels, where that is exact to 1e-8).
+    uint2* const bins = reinterpret_cast<uint2*>(xl + Sh::bins_at);
     int jb0 = 0;
-    float wj0 = 0.f, wj1 = 0.f, wi0[NG] = {}, wi1[NG] = {};
+    float wj[2][2] = {};   // [the row's bin is the longer][the column's first or second bin; 0: not there]
+    uint32_t wi[NG] = {};
     if constexpr (ANY) {
+        const int least = (g.OH + g.AH - 1) / g.AH;
         for (int i = tid; i < g.OH; i += NT) {   // (read behind the barrier that publishes the first passes)
-            int b;
-            float w0, w1;
-            pool_bins(i, g.OH, g.AH, b, w0, w1);
-            bins[4 * i] = __builtin_bit_cast(float, (uint32_t)(b * g.AW * g.C) * 2u), bins[4 * i + 1] = w0, bins[4 * i + 2] = w1;
+            int b, l0, l1;
+            pool_bin_lengths(i, g.OH, g.AH, b, l0, l1);
+            bins[i] = make_uint2((uint32_t)(b * g.AW * g.C) * 2u, (l0 > least ? 1u : 0u) | (l1 > 0 ? 2u : 0u) | (l1 > least ? 4u : 0u));
         }
-        pool_bins(min(ocol0 + scol, g.OW - 1), g.OW, g.AW, jb0, wj0, wj1);
+        int l0, l1;
+        pool_bin_lengths(min(ocol0 + scol, g.OW - 1), g.OW, g.AW, jb0, l0, l1);
+#pragma unroll
+        for (int p = 0; p < 2; ++p) wj[p][0] = 1.f / (float)((least + p) * l0), wj[p][1] = l1 > 0 ? 1.f / (float)((least + p) * l1) : 0.f;
     }
     // a step's 8 rows lie in one image (group): its first row there, and the byte offsets of that row in y and the addend
     int orow = orow0, rleft = rows_valid;   // rleft: rows of the run from this step on
@@ -561,10 +568,10 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
             yoff[n] = ok ? ylane[n] : kNoRow;
             if constexpr (ANY) {
                 const bool in = ok && s_ok;
-                const float4 bin = *reinterpret_cast<const float4*>(bins + 4 * (ok ? orow + 4 * tile_of(n) + srow : 0));
-                const uint32_t o = alane[n] + __builtin_bit_cast(uint32_t, bin.x);
-                wi0[n] = bin.y, wi1[n] = bin.z;
-                const bool right = in && wj1 != 0.f, below = in && wi1[n] != 0.f;
+                const uint2 bin = bins[ok ? orow + 4 * tile_of(n) + srow : 0];
+                const uint32_t o = alane[n] + bin.x;
+                wi[n] = bin.y;
+                const bool right = in && wj[0][1] != 0.f, below = in && (bin.y & 2u) != 0;
                 const uint32_t at = lim > 0 ? aoff : 0;
                 addv[n][0] = xload_from(arsrc, in ? o : kNoRow, at);
                 addv[n][1] = xload_from(arsrc, right ? o + 2u * (uint32_t)g.C : kNoRow, at);
@@ -596,8 +603,10 @@ __device__ __forceinline__ void dwconv_tz_body(const T* __restrict__ x, const T*
         }
     };
     auto tile_store = [&](uint4 v, int n) {   // where place() put it
-        if constexpr (ANY) v = tz_add_bins<T>(v, addv[n], wi0[n] * wj0, wi0[n] * wj1, wi1[n] * wj0, wi1[n] * wj1);
-        else if constexpr (ADD) v = tz_add_quarter<T>(v, addv[n][0]);
+        if constexpr (ANY) {
+            const bool top = (wi[n] & 1u) != 0, below = (wi[n] & 4u) != 0;
+            v = tz_add_bins<T>(v, addv[n], top ? wj[1][0] : wj[0][0], top ? wj[1][1] : wj[0][1], below ? wj[1][0] : wj[0][0], below ? wj[1][1] : wj[0][1]);
+        } else if constexpr (ADD) v = tz_add_quarter<T>(v, addv[n][0]);
         if constexpr (GATE) {
             const uint2 o = tz_gate<T>(make_uint2(v.x, v.y), make_uint2(v.z, v.w), g.gs);
             typedef unsigned v2u __attribute__((ext_vector_type(2)));

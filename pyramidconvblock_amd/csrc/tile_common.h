@@ -67,16 +67,24 @@ __device__ __forceinline__ void pack_pairs(const ChanVec<T, V>& a, const ChanVec
     }
 }
 
-// Bins of an adaptive average pool of `in` values to `out` <= in that value i lies in: the first, and the weights (one
-// over the bin's length; 0: no second bin).
-__device__ __forceinline__ void pool_bins(int i, int in, int out, int& b0, float& w0, float& w1) {
+// Bins of an adaptive average pool of `in` values to `out` <= in that value i lies in: the first, and the lengths (0: no
+// second bin).  A length is ceil(in / out) or one more.
+__device__ __forceinline__ void pool_bin_lengths(int i, int in, int out, int& b0, int& l0, int& l1) {
     b0 = (int)((unsigned)(i * out) / (unsigned)in);
     const int b1 = (int)((unsigned)((i + 1) * out + in - 1) / (unsigned)in) - 1;
     auto len = [&](int b) {
         return (int)((unsigned)((b + 1) * in + out - 1) / (unsigned)out) - (int)((unsigned)(b * in) / (unsigned)out);
     };
-    w0 = 1.f / (float)len(b0);
-    w1 = b1 > b0 ? 1.f / (float)len(b1) : 0.f;
+    l0 = len(b0);
+    l1 = b1 > b0 ? len(b1) : 0;
+}
+
+// The same with the weights of one axis (one over the bin's length; 0: no second bin).
+__device__ __forceinline__ void pool_bins(int i, int in, int out, int& b0, float& w0, float& w1) {
+    int l0, l1;
+    pool_bin_lengths(i, in, out, b0, l0, l1);
+    w0 = 1.f / (float)l0;
+    w1 = l1 > 0 ? 1.f / (float)l1 : 0.f;
 }
 
 // XCD-aware work order: consecutive workgroup ids go to the 8 XCDs round-robin, so give each

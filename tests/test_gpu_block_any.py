@@ -170,3 +170,37 @@ def test_pooled_gradient_of_any_ratio_in_the_store(oracle, dtype, k, shape, seco
     assert_close(xd.grad, dxo, dtype, "dx")
     for n, p in m.named_parameters():
         assert_close(p.grad, go[n], dtype, "grad " + n)
+
+
+@pytest.mark.parametrize("k,shape,pooled", [
+    # bins of 2 and 3 a side, of 3 and 4, of 1 and 2 on one axis with one pixel each on the other; one image and two side by side in a tile
+    (9, (3, 57, 61, 200), (28, 30)), (3, (2, 111, 70, 72), (55, 35)), (17, (4, 61, 50, 104), (20, 16)), (7, (66, 15, 15, 64), (7, 7)), (5, (4, 40, 41, 168), (30, 41)),
+    (15, (5, 33, 64, 96), (16, 31)),
+])
+def test_pooled_gradient_in_the_store_is_the_pools(k, shape, pooled):
+    """The same bits as the pool's gradient added by its own launch (fp16: of a million elements, some ten would round otherwise with weights
+    one rounding off)."""
+    import ctypes
+
+    from pyramidconvblock_amd import _lib
+
+    L, dt = _lib.lib(), torch.float16
+    both = L["_ZN3pdw18dwconv_bwd3_launchEPKvS1_S1_PvS1_S2_S2_S1_S1_S2_S2_iiiiiiiiP12ihipStream_tPiPKNS_7MeanJobE"]
+    pool = L["_ZN3pdw18avgpool_bwd_launchEPKvPviiiiiiiiP12ihipStream_t"]
+    B, H, W, C = shape
+    h, w = pooled
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    r = lambda *s: torch.randn(*s, generator=gen, device="cuda").to(dt)
+    gy, x, w0, add, gy1, x1 = r(*shape), r(*shape), r(k, k, C), r(B, h, w, C), r(B, h, w, C), r(B, h, w, C)
+    dw = torch.empty_like(w0)
+    ws = [torch.empty(L.pdw_dwconv_wgrad_workspace_bytes(B, *e, C, k, k, 1, 1, k // 2, k // 2, 1, 1, _lib.dtype_code(dt)) // 4 + 1, device="cuda")
+          for e in ((H, W), (h, w))]
+    at, s = lambda t: ctypes.c_void_p(t.data_ptr() if t is not None else 0), ctypes.c_void_p(_lib.stream_ptr(x.device))
+    dx = []
+    for a in (add, None):
+        dx.append(torch.full_like(x, float("nan")))
+        rc = both(at(gy), at(w0), at(a), at(dx[-1]), at(x), at(dw), at(ws[0]), at(x1), at(gy1), at(dw), at(ws[1]), B, H, W, h, w, C, k,
+                  _lib.dtype_code(dt), s, at(None), at(None))
+        assert rc == 0
+    assert pool(at(add), at(dx[1]), B, H, W, C, h, w, 1, _lib.dtype_code(dt), s) == 0
+    assert bool(dx[1].isfinite().all()) and torch.equal(*dx)
