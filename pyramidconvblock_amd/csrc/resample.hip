@@ -48,7 +48,8 @@ __device__ __forceinline__ int bin_end(int i, int in, int out) {
     return (int)((unsigned)((i + 1) * in + out - 1) / (unsigned)out);
 }
 
-template <typename T, int VEC>
+// FLIGHT: all loads of a bin of up to 3 x 3 in flight (pool_in_flight).
+template <typename T, int VEC, bool FLIGHT>
 __device__ __forceinline__ void avgpool_fwd_item(const T* __restrict__ x, T* __restrict__ y, int H, int W, int C, int h,
                                                  int w, long long idx) {
     const int CV = C / VEC;
@@ -72,8 +73,7 @@ __device__ __forceinline__ void avgpool_fwd_item(const T* __restrict__ x, T* __r
 #pragma unroll
     for (int v = 0; v < VEC; ++v) acc[v] = 0.f;
     constexpr int NB = 3;
-    if (he - hs <= NB && we - ws <= NB) {   // bins of up to 3 x 3 (extents of two to three times the pooled ones): all loads in flight
-        // (us, with column sums: [2,15,15,96] bf16 4.7 -> 3.5, [27,15,15,624] 6.6 -> 4.8; [104,27,28,280], bandwidth, 17.4 -> 17.9)
+    if (FLIGHT && he - hs <= NB && we - ws <= NB) {   // (extents of two to three times the pooled ones)
         const T* const p = x + ((b * H + hs) * W + ws) * C + c;
         ChanVec<T, VEC> xv[NB][NB];
 #pragma unroll
@@ -104,37 +104,40 @@ __device__ __forceinline__ void avgpool_fwd_item(const T* __restrict__ x, T* __r
     store_f32<T, VEC>(y + ((b * h + i) * w + j) * C + c, acc);
 }
 
-template <typename T, int VEC>
+template <typename T, int VEC, bool FLIGHT>
 __global__ __launch_bounds__(256) void avgpool_fwd_k(const T* __restrict__ x, T* __restrict__ y, int H, int W, int C,
                                                      int h, int w, long long total) {
     const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx < total) avgpool_fwd_item<T, VEC>(x, y, H, W, C, h, w, idx);
+    if (idx < total) avgpool_fwd_item<T, VEC, FLIGHT>(x, y, H, W, C, h, w, idx);
 }
 
 // The same with the column sums of another tensor (mean_any.h) in the first workgroups: both are bandwidth.
-template <typename T, int VEC>
+template <typename T, int VEC, bool FLIGHT>
 __global__ __launch_bounds__(256) void avgpool_colsum_k(const T* __restrict__ x, T* __restrict__ y, int H, int W, int C,
                                                         int h, int w, long long total, const ColsumJob sums, int nsums) {
     extern __shared__ float sm[];
     if ((int)blockIdx.x < nsums) return colsum_body<T>(sums, blockIdx.x, sm);
     const long long idx = (long long)(blockIdx.x - nsums) * blockDim.x + threadIdx.x;
-    if (idx < total) avgpool_fwd_item<T, VEC>(x, y, H, W, C, h, w, idx);
+    if (idx < total) avgpool_fwd_item<T, VEC, FLIGHT>(x, y, H, W, C, h, w, idx);
 }
 
 // And with the packing of weights (pack_weights.h) behind those, for blocks that pad their channels: a kernel of its own, since its
 // arguments and the branch cost the others 0.1 us.
-template <typename T, int VEC>
+template <typename T, int VEC, bool FLIGHT>
 __global__ __launch_bounds__(256) void avgpool_pack_k(const T* __restrict__ x, T* __restrict__ y, int H, int W, int C, int h,
                                                       int w, long long total, const ColsumJob sums, int nsums, const PackArgs pack, int npack) {
     extern __shared__ float sm[];
     if ((int)blockIdx.x < nsums) return colsum_body<T>(sums, blockIdx.x, sm);
     if ((int)blockIdx.x - nsums < npack) return pack_weights_body(pack, blockIdx.x - nsums);
     const long long idx = (long long)(blockIdx.x - nsums - npack) * blockDim.x + threadIdx.x;
-    if (idx < total) avgpool_fwd_item<T, VEC>(x, y, H, W, C, h, w, idx);
+    if (idx < total) avgpool_fwd_item<T, VEC, FLIGHT>(x, y, H, W, C, h, w, idx);
 }
 
-// Input row ih lies in bins i with floor(ih*h/H) <= i <= ceil((ih+1)*h/H) - 1.
-template <typename T, int VEC>
+// Input row ih lies in bins i with floor(ih*h/H) <= i <= ceil((ih+1)*h/H) - 1: NR of them at most where the pool shrinks (one where the pooled
+// extent divides the input's), NC on the other axis.  us, one load after the other -> NR x NC: [3,57,61,200] bf16 5.7 -> 4.8, [2,15,15,96] 3.8 -> 3.3,
+// [70,57,57,128] 22.7 -> 21.2; of one bin on an axis [104,27,28,280] 17.1 -> 15.5 (two there too
+// 17.5; 230 launches of more than four workgroups a compute unit 1.1 times as fast, with two 0.95).
+template <typename T, int VEC, int NR, int NC>
 __global__ __launch_bounds__(256) void avgpool_bwd_k(const T* __restrict__ gy, T* __restrict__ gx, int H, int W,
                                                      int C, int h, int w, int accumulate, long long total) {
     const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -152,24 +155,22 @@ __global__ __launch_bounds__(256) void avgpool_bwd_k(const T* __restrict__ gy, T
     T* dst = gx + ((b * H + ih) * W + iw) * C + c;
     ChanVec<T, VEC> old;
     if (accumulate) old = *reinterpret_cast<const ChanVec<T, VEC>*>(dst);
-    if (i1 - i0 <= 1 && j1 - j0 <= 1) {   // (always where the pool shrinks) at most 2 x 2 bins: their loads in flight together
-        // (us: [3,57,61,200] bf16 5.7 -> 4.8, [2,15,15,96] 3.8 -> 3.3; [104,27,28,280] 16.3 -> 16.8)
-        ChanVec<T, VEC> gv[2][2];
+    if (i1 - i0 < NR && j1 - j0 < NC) {   // (always where the pool shrinks) the loads of all bins in flight together
+        ChanVec<T, VEC> gv[NR][NC];
 #pragma unroll
-        for (int p = 0; p < 2; ++p)
+        for (int p = 0; p < NR; ++p)
 #pragma unroll
-            for (int q = 0; q < 2; ++q)
+            for (int q = 0; q < NC; ++q)
                 gv[p][q] = *reinterpret_cast<const ChanVec<T, VEC>*>(gy + ((b * h + (p ? i1 : i0)) * w + (q ? j1 : j0)) * C + c);
-        int kh[2], kw[2];
+        int kh[NR], kw[NC];
 #pragma unroll
-        for (int p = 0; p < 2; ++p) {
-            const int i = p ? i1 : i0, j = p ? j1 : j0;
-            kh[p] = bin_end(i, H, h) - bin_start(i, H, h), kw[p] = bin_end(j, W, w) - bin_start(j, W, w);
-        }
+        for (int p = 0; p < NR; ++p) kh[p] = bin_end(p ? i1 : i0, H, h) - bin_start(p ? i1 : i0, H, h);
 #pragma unroll
-        for (int p = 0; p < 2; ++p)
+        for (int q = 0; q < NC; ++q) kw[q] = bin_end(q ? j1 : j0, W, w) - bin_start(q ? j1 : j0, W, w);
 #pragma unroll
-            for (int q = 0; q < 2; ++q)
+        for (int p = 0; p < NR; ++p)
+#pragma unroll
+            for (int q = 0; q < NC; ++q)
                 if (i0 + p <= i1 && j0 + q <= j1) {
                     const float inv = 1.f / (float)(kh[p] * kw[q]);
 #pragma unroll
@@ -1425,6 +1426,14 @@ static bool grid_for(long long total, unsigned* blocks) {
     return true;
 }
 
+// Whether a pool's bins of up to 3 x 3 have all loads in flight: latency, but where bins have rows or columns of two (an axis of exact halves) a third
+// of the loads are of pixels that a bin does not have, which launches of more than a workgroup a compute unit, bound by their requests, take
+// longer for.  (A bin's length is the ratio rounded up or one more.)  us with column sums, one load after the other -> in flight: [2,15,15,96] bf16
+// 4.7 -> 3.5, [27,15,15,624] 6.6 -> 4.8, [70,57,57,128] 18.6 -> 17.1; one axis of halves, up to 256 workgroups [18,30,27,80] fp32 5.1 -> 4.6,
+// [51,39,39,48] bf16 5.1 -> 4.2, [22,40,39,112] 5.3 -> 4.1, more: [65,33,44,280] 20.5 and 21.4, [104,27,28,280] 17.4 and 17.9, [1,76,75,696] 6.1
+// and 6.8, [4,81,78,272] 7.3 and 7.8 (130 such launches in flight 0.99 times as fast, 90 of no such axis 1.05).
+static bool pool_in_flight(unsigned blocks, int H, int W, int h, int w) { return blocks <= 256 || (cdiv(H, h) == 3 && cdiv(W, w) == 3); }
+
 int avgpool_fwd_launch(const void* x, void* y, int B, int H, int W, int C, int h, int w, int dtype, hipStream_t s) {
     const void* ptrs[2] = {x, y};
     const int vec = pick_vec(C, esize(dtype), ptrs, 2);
@@ -1432,9 +1441,12 @@ int avgpool_fwd_launch(const void* x, void* y, int B, int H, int W, int C, int h
     unsigned blocks;
     if (total == 0) return 0;
     if (!grid_for(total, &blocks)) return 1;
-#define CALL(T, V) hipLaunchKernelGGL((avgpool_fwd_k<T, V>), dim3(blocks), dim3(256), 0, s, (const T*)x, (T*)y, H, W, C, h, w, total);
+    const bool flight = pool_in_flight(blocks, H, W, h, w);
+#define GO(T, V, F) hipLaunchKernelGGL((avgpool_fwd_k<T, V, F>), dim3(blocks), dim3(256), 0, s, (const T*)x, (T*)y, H, W, C, h, w, total)
+#define CALL(T, V) if (flight) GO(T, V, true); else GO(T, V, false);
     PDW_TYPE_SWITCH(dtype, vec, CALL)
 #undef CALL
+#undef GO
     return check_launch("avgpool_fwd");
 }
 
@@ -1448,17 +1460,20 @@ int avgpool_with_launch(const void* a, void* xp, int B, int H, int W, int C, int
     unsigned blocks;
     if (!grid_for(total, &blocks) || (unsigned long long)blocks + nsums + npack > 0x7fffffffULL) return 1;
     const size_t lds = sums ? 256 * 16 / esize(dtype) * sizeof(float) : 0;
+    const bool flight = pool_in_flight(blocks, H, W, h, w);
+#define CALL(T, V) if (flight) GO(T, V, true); else GO(T, V, false);
     if (!pack) {
-#define CALL(T, V) hipLaunchKernelGGL((avgpool_colsum_k<T, V>), dim3(blocks + nsums), dim3(256), lds, s, (const T*)a, (T*)xp, H, W, C, h, w, total, *sums, nsums);
+#define GO(T, V, F) hipLaunchKernelGGL((avgpool_colsum_k<T, V, F>), dim3(blocks + nsums), dim3(256), lds, s, (const T*)a, (T*)xp, H, W, C, h, w, total, *sums, nsums)
         PDW_TYPE_SWITCH(dtype, vec, CALL)
-#undef CALL
+#undef GO
         return check_launch("avgpool_colsum");
     }
     if (dtype == kF32) return set_error("packed weights are of 16-bit types"), 1;
-#define CALL(T, V)                                                                                                                       \
-    hipLaunchKernelGGL((avgpool_pack_k<T, V>), dim3(blocks + nsums + npack), dim3(256), lds, s, (const T*)a, (T*)xp, H, W, C, h, w, total, \
-                       sums ? *sums : ColsumJob{}, nsums, *pack, npack);
+#define GO(T, V, F)                                                                                                                         \
+    hipLaunchKernelGGL((avgpool_pack_k<T, V, F>), dim3(blocks + nsums + npack), dim3(256), lds, s, (const T*)a, (T*)xp, H, W, C, h, w, total, \
+                       sums ? *sums : ColsumJob{}, nsums, *pack, npack)
     if (dtype == kF16) PDW_VEC_SWITCH(f16_t, vec, CALL) else PDW_VEC_SWITCH(bf16_t, vec, CALL)
+#undef GO
 #undef CALL
     return check_launch("avgpool_pack");
 }
@@ -1480,9 +1495,12 @@ int avgpool_bwd_launch(const void* gy, void* gx, int B, int H, int W, int C, int
     const long long total = (long long)B * H * W * (C / vec);
     if (total == 0) return 0;
     if (!grid_for(total, &blocks)) return 1;
-#define CALL(T, V) hipLaunchKernelGGL((avgpool_bwd_k<T, V>), dim3(blocks), dim3(256), 0, s, (const T*)gy, (T*)gx, H, W, C, h, w, accumulate, total);
+    const int one = (H % h == 0 ? 1 : 0) + (W % w == 0 ? 2 : 0);
+#define GO(T, V, NR, NC) hipLaunchKernelGGL((avgpool_bwd_k<T, V, NR, NC>), dim3(blocks), dim3(256), 0, s, (const T*)gy, (T*)gx, H, W, C, h, w, accumulate, total)
+#define CALL(T, V) if (one == 0) GO(T, V, 2, 2); else if (one == 1) GO(T, V, 1, 2); else if (one == 2) GO(T, V, 2, 1); else GO(T, V, 1, 1);
     PDW_TYPE_SWITCH(dtype, vec, CALL)
 #undef CALL
+#undef GO
     return check_launch("avgpool_bwd");
 }
 

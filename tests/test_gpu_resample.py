@@ -602,3 +602,26 @@ def test_any_ratio(oracle, dtype, big, small):
         torch.autograd.backward([y, u], [p.cuda(), x.cuda()])
         assert_close(xd.grad, oracle.avgpool_bwd(p.double().numpy(), hw), dtype, "pool's gradient")
         assert_close(pd.grad, oracle.bilinear_bwd(x.double().numpy(), out), dtype, "resize's gradient")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("shape,out", [
+    # more than 256 workgroups: an axis of exact halves (one load after the other; one bin a pixel there), neither, and ratios of three and 4 / 3
+    ((2, 83, 80, 176), (41, 40)), ((2, 80, 83, 176), (40, 41)), ((2, 83, 81, 176), (41, 40)), ((3, 93, 90, 256), (31, 30)),
+    ((2, 72, 76, 128), (54, 57)),
+])
+def test_pools_of_many_workgroups(dtype, shape, out):
+    """Pool and its gradient where launches are more than a workgroup a compute unit, against float64."""
+    import torch.nn.functional as F
+
+    import pyramidconvblock_amd as P
+
+    gen = torch.Generator().manual_seed(shape[1])
+    x = randn(gen, *shape).to(dtype)
+    g = randn(gen, shape[0], *out, shape[3]).to(dtype)
+    xd, xr = x.cuda().requires_grad_(), x.double().permute(0, 3, 1, 2).requires_grad_()
+    y, yr = P.AdaptiveAvgPool2dFunction.apply(xd, out), F.adaptive_avg_pool2d(xr, out)
+    assert_close(y, yr.detach().permute(0, 2, 3, 1).numpy(), dtype, "pool")
+    y.backward(g.cuda())
+    yr.backward(g.double().permute(0, 3, 1, 2))
+    assert_close(xd.grad, xr.grad.permute(0, 2, 3, 1).numpy(), dtype, "pool's gradient")
