@@ -351,15 +351,18 @@ int backward(const Shape& s, const Saved& v, const BwdWork& g, const void* gy, c
     if (pair != 0 && pair != -1) return pair;
     if (pair == -1)
         if (int e = pdw_dwconv_dgrad(g.gch, w_dw1, g.dxp, s.B, s.h, s.w, s.I, s.K, s.K, 1, 1, pad, pad, 1, 1, dt, stream)) return e;
-    auto rest = [&](const void* pooled) {
+    auto rest = [&](const void* pooled, int* cuts) {
         return dwconv_bwd3_launch(g.gcf, w_dw0, pooled, g.da, v.a, gw_dw0, g.ws_w0, v.xp, g.gch, gw_dw1, g.ws_w1, s.B, s.H, s.W, s.h, s.w, s.I, s.K, dt,
-                                  st, nullptr, waiting ? &mean : nullptr);
+                                  st, cuts, waiting ? &mean : nullptr);
     };
     // (the pooled gradient is added where the full scale's is stored, or behind)
-    bool pool_rides = s.exact || (s.h <= s.H && s.w <= s.W && dwconv_bwd3_adds_any(s.K));
-    int r = -1;
-    if (pair == -1) r = rest(pool_rides ? g.dxp : nullptr);
-    if (pair == -1 && r == -1 && pool_rides && !s.exact) pool_rides = false, r = rest(nullptr);
+    bool pool_rides = s.exact;
+    int r = -1, cuts[3];
+    if (pair == -1) {
+        if (!s.exact && s.h <= s.H && s.w <= s.W && dwconv_bwd3_adds_any(s.K)) pool_rides = rest(g.dxp, cuts) == 0;
+        r = rest(pool_rides ? g.dxp : nullptr, nullptr);
+        if (r == -1 && pool_rides && !s.exact) pool_rides = false, r = rest(nullptr, nullptr);
+    }
     if (r != 0 && r != -1) return r;
     if (r == -1 && pair == -1) pair = f32_pair(nullptr, nullptr);
     if (pair != 0 && pair != -1) return pair;

@@ -30,7 +30,7 @@ struct Bwd3Wgrad {
 };
 
 struct Bwd3Args {
-    const void *gy, *w, *add;   // input gradient: dx = conv^T(gy, w) (+ add / 4 over 2x2 blocks)
+    const void *gy, *w, *add;   // input gradient: dx = conv^T(gy, w) (+ the gradient of a pool of dx's tensor: add / 4 over 2x2 blocks, or by bins)
     void* dx;
     TzGeom gd;
     int npcd;                   // patches of its tile side by side (16 or 8)
@@ -88,7 +88,33 @@ __global__ __launch_bounds__(512, 1) void dwconv_bwd3_k(const Bwd3Args a) {
 struct Bwd3Plan {
     int n[3];         // rows of the input gradient's runs; runs of the full scale's and the half scale's weight gradient
     char order[4];    // 'D', 'F', 'H' in grid order
+    bool any_pays;    // the gradient of a pool of other ratios than halves is best added in this launch
 };
+
+// Prices of the input gradient here: its store adds the pooled gradient, and its runs have the chip and its memory to share with
+// the weight gradients' (256 of them alone: 6.1 + 1.8 a step at filter 13).
+constexpr double kBwd3Start = 5.0, kBwd3Step = 1.15;
+
+// Whether the gradient of a pool of other ratios is better added in the input gradient's store (MODE 16) than by avgpool_bwd_k behind the
+// launch, which takes 2.8 us and 0.6 a MB of the gradient: a run starts 1 us later and its steps are longer by the bins' loads, which the launch
+// waits for as far as its runs are the last to end.  Of 327 random shapes, in the store always, 52 are slower than by two launches, by up to 18 %
+// (us, two launches and the store: [3,103,103,600] filter 17 76.6 and 90.6, [107,13,14,640] 93.7 and 110, [54,11,8,664] filter 9 31.1 and 33.6,
+// [3,66,65,448] filter 15 31.8 and 34.4); by this rule 4, by 1 % of the step's kernels at most, and the sum of all is 9 % less than by two
+// launches.  In the store, as chosen: [3,57,61,200] filter 9 16.7 -> 14.3, [70,57,57,128] filter 7 73.9 -> 54.7, [2,83,82,208] filter 15 20.0 -> 17.1.
+template <int K>
+static bool bwd3_any_pays(const Bwd3Plan& plan, TzGeom gd, int ni, WgPhPlan p0, WgPhPlan p1, int nmean) {
+    constexpr double kAny = K == 3 ? 0.65 : K == 5 ? 0.3 : K == 9 ? 0.7 : K == 15 ? 0.45 : 0.6;   // (us a step; a tenth less, and a few are slower)
+    if (!dwconv_bwd3_adds_any(K) || !tz_cut(gd, ni, plan.n[0]) || !wgrad_ph_cut(p0, plan.n[1]) || !wgrad_ph_cut(p1, plan.n[2])) return false;
+    auto end = [&](double start, double step) {
+        const LaunchCut d{0, start + 1.3 * (ni - 1) + step * tz_steps(gd), tz_blocks(gd)}, mean{0, kMeanCost, nmean};
+        const LaunchCut f{0, wgrad_ph_run_cost(K, p0.g.passes), p0.nblocks}, h{0, wgrad_ph_run_cost(K, p1.g.passes), p1.nblocks};
+        const LaunchCut* const pick[4] = {&d, &f, &h, &mean};
+        int ord[4] = {0, 0, 0, 3};
+        for (int i = 0; i < 3; ++i) ord[i] = plan.order[i] == 'D' ? 0 : plan.order[i] == 'F' ? 1 : 2;
+        return launch_makespan(pick, ord);
+    };
+    return end(kBwd3Start + 1.0, kBwd3Step + kAny) - end(kBwd3Start, kBwd3Step) < 2.8 + 0.6 * (2e-6 * gd.B * gd.OH * gd.OW * gd.C);
+}
 
 template <int K>
 static Bwd3Plan bwd3_plan(int B, const TzGeom& gd, int npcd, const WgPhPlan& p0, const WgPhPlan& p1, int nmean) {
@@ -103,21 +129,18 @@ static Bwd3Plan bwd3_plan(int B, const TzGeom& gd, int npcd, const WgPhPlan& p0,
     const Key key{B, gd.OH, gd.OW, p1.g.OH, p1.g.OW, gd.C, nmean};
     std::lock_guard<std::mutex> lock(mu);
     if (auto it = cache.find(key); it != cache.end()) return it->second;
-    // Prices of the input gradient here: its store adds the pooled gradient, and its runs have the chip and its memory to share with
-    // the weight gradients' (256 of them alone: 6.1 + 1.8 a step at filter 13).
-    constexpr double kStart = 5.0, kStep = 1.15;
     const int ni = 16 / npcd;
-    Bwd3Plan best{{8, 1, 1}, "DFH"};
+    Bwd3Plan best{{8, 1, 1}, "DFH", false};
     auto part = [](const WgPhPlan& p) { return LaunchPart{kWgPhStart, wgrad_ph_step(K), p.total, p.g.passes, [p](int s) { return p.per_chunk * cdiv(p.total, s); }}; };
-    const LaunchPart parts[3] = {tz_part(gd, ni, kStart, kStep), part(p0), part(p1)};
+    const LaunchPart parts[3] = {tz_part(gd, ni, kBwd3Start, kBwd3Step), part(p0), part(p1)};
     int steps[3];
     if (launch_balance(parts, nmean, steps)) {
         TzGeom c = gd;
         tz_cut_steps(c, ni, steps[0]);
-        best = Bwd3Plan{{c.run, cdiv(p0.total, steps[1]), cdiv(p1.total, steps[2])}, "DFH"};
+        best = Bwd3Plan{{c.run, cdiv(p0.total, steps[1]), cdiv(p1.total, steps[2])}, "DFH", false};
     } else {
         std::vector<LaunchCut> cuts[3];
-        tz_cuts(cuts[0], gd, ni, kStart, kStep);
+        tz_cuts(cuts[0], gd, ni, kBwd3Start, kBwd3Step);
         for (int i = 1; i < 3; ++i) {
             WgPhPlan p = i == 1 ? p0 : p1;
             const int most = p.g.nchunks;
@@ -145,6 +168,7 @@ static Bwd3Plan bwd3_plan(int B, const TzGeom& gd, int npcd, const WgPhPlan& p0,
                     }
                 }
     }
+    best.any_pays = bwd3_any_pays<K>(best, gd, ni, p0, p1, nmean);
     if (cache.size() >= kPlanCacheMax) cache.clear();   // callers with ever-changing shapes: a plan is cheap to redo
     cache[key] = best;
     return best;
@@ -197,7 +221,7 @@ static Bwd3Plan bwd2_plan(const TzGeom& gd, int npcd, const WgPhPlan& p0) {
         if (!wgrad_ph_cut(p, std::max(1, p0.g.nchunks * e / 16)) || (!cuts[1].empty() && cuts[1].back().n == p.g.nchunks)) continue;
         cuts[1].push_back({p.g.nchunks, kStepF * p.g.passes, p.nblocks});
     }
-    Bwd3Plan best{{0, 1, 0}, "DF"};
+    Bwd3Plan best{{0, 1, 0}, "DF", false};
     for (const LaunchCut& dc : cuts[0])
         for (const LaunchCut& fc : cuts[1]) {
             const bool single = dc.count + fc.count <= 256;
@@ -228,7 +252,8 @@ static void bwd3_go(const Bwd3Args& a, unsigned grid, size_t lds, hipStream_t s)
 
 // -1: not covered (the caller makes the three launches).  16-bit types, C % 8 == 0, padding K / 2; the full scale
 // [B, H, W, C], the pooled one [B, h, w, C].  addp (optional; H = 2 h and W = 2 w or dwconv_bwd3_adds_any): the pooled branch's gradient.
-// x1 = nullptr and h = 0: no pooled scale (a convolution by itself; -1 also where two launches take no longer).
+// x1 = nullptr and h = 0: no pooled scale (a convolution by itself; -1 also where two launches take no longer).  With plan_out and addp of other
+// ratios than halves, -1 also where adding it by a launch behind is estimated to take no longer.
 template <int K>
 static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* dx, const void* x0, void* dw0, void* ws0,
                        const void* x1, const void* gy1, void* dw1, void* ws1, int B, int H, int W, int h, int w, int C, int dtype,
@@ -261,6 +286,7 @@ static int launch_bwd3(const void* gyf, const void* w0, const void* addp, void* 
     if (tune_env("PDW_BWD3_PRINT"))
         fprintf(stderr, "bwd3 plan B=%d H=%d W=%d C=%d K=%d: cuts D %d F %d H %d order %s\n", B, H, W, C, K, plan.n[0],
                 plan.n[1], plan.n[2], plan.order);
+    if (plan_out && any && !plan.any_pays) return -1;
     if (plan.n[0] < 1 || plan.n[1] < 1 || (!one && plan.n[2] < 1)) return -1;
     if (!tz_cut(a.gd, 16 / a.npcd, plan.n[0])) return -1;
     const long long nd = tz_blocks(a.gd);

@@ -19,8 +19,8 @@ PDW_BWD3_DECL(17)
 #undef PDW_BWD3_DECL
 
 // -1: not covered (the caller makes the three launches).  With plan_out the launch is only planned: the band counts
-// of the input gradient, the full and the half scale's weight gradient go to plan_out[0..2], no pointer is looked at
-// and nothing is launched.
+// of the input gradient, the full and the half scale's weight gradient go to plan_out[0..2], no pointer is followed
+// and nothing is launched; -1 then also where a given addp is better added by a launch of its own.
 int dwconv_bwd3_launch(const void* gyf, const void* w0, const void* addp, void* dx, const void* x0, void* dw0, void* ws0,
                        const void* x1, const void* gy1, void* dw1, void* ws1, int B, int H, int W, int h, int w, int C, int K,
                        int dtype, hipStream_t s, int* plan_out, const MeanJob* mean) {

@@ -177,11 +177,9 @@ int dense_bwd_pair_launch(const void* gy, const void* w, const void* xin, void* 
 // (optional); -1 = not covered.  x1 = nullptr with h = 0: both gradients of a convolution by itself, -1 also where a launch each
 // takes no longer
 bool dwconv_bwd3_covers(int B, int W, int C);
-// Filters whose launch also adds the gradient of a pool of other ratios (h <= H, w <= W), up to four bins a pixel, in the store of the
-// input gradient, instead of a launch that reads it again.  Not those whose operands of 16 channels leave no registers for them (43 and 61
-// spilled).  us, the launch and that behind it -> this: [3,57,61,200] filter 9 11.4 + 5.4 -> 13.7, [1,106,105,808] 19.5 + 9.2 -> 22.2,
-// [1,111,111,1144] filter 15 37.9 + 13.9 -> 38.9, [27,15,15,624] filter 5 18.7 + 6.2 -> 19.4, [16,107,107,104] filter 17 55.7 + 19.7 -> 73.3;
-// [104,27,28,280] filter 11 47.0 + 16.6, 100 here.
+// Filters whose launch can also add the gradient of a pool of other ratios (h <= H, w <= W), up to four bins a pixel, in the store of the
+// input gradient, instead of a launch that reads it again (where that pays: bwd3_any_pays).  Not those whose operands of 16 channels leave no
+// registers for them (43 and 61 spilled; us, two launches and this: [104,27,28,280] filter 11 47.0 + 16.6 and 100).
 constexpr bool dwconv_bwd3_adds_any(int K) { return K != 11 && K != 13; }
 int dwconv_bwd3_launch(const void* gyf, const void* w0, const void* addp, void* dx, const void* x0, void* dw0, void* ws0,
                        const void* x1, const void* gy1, void* dw1, void* ws1, int B, int H, int W, int h, int w, int C, int K,

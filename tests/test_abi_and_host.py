@@ -250,3 +250,26 @@ def test_quotients_of_quads():
         x = np.arange(w + 32, dtype=np.uint64)
         magic = np.uint64((2 ** 32 + w - 1) // w)
         assert ((x * magic) >> np.uint64(32) == x // np.uint64(w)).all(), w
+
+
+@pytest.mark.parametrize("shape,k,stores", [
+    # us, two launches and in the store: 16.7 and 14.3, 73.9 and 54.7, 20.0 and 17.1; 93.7 and 110, 76.6 and 90.6, 31.1 and 33.6
+    ((3, 57, 61, 104), 9, True), ((70, 57, 57, 64), 7, True), ((2, 83, 82, 112), 15, True),
+    ((107, 13, 14, 320), 17, False), ((3, 103, 103, 304), 17, False), ((54, 11, 8, 336), 9, False),
+])
+def test_where_a_pooled_gradient_is_added(shape, k, stores):
+    """The plan of a block's convolution gradients says whether their launch adds the gradient of a pool of odd extents (bwd3_any_pays of
+    csrc/dwconv_bwd3.h)."""
+    from pyramidconvblock_amd import _lib
+
+    class Mean(ctypes.Structure):   # MeanJob of csrc/mean_any.h: sums of one range, twice the channels
+        _fields_ = [("part", ctypes.c_void_p), ("n", ctypes.c_int), ("B", ctypes.c_int), ("D", ctypes.c_int), ("inv_p", ctypes.c_float),
+                    ("pointers", ctypes.c_void_p * 7), ("shared", ctypes.c_bool)]
+
+    launch = _lib.lib()["_ZN3pdw18dwconv_bwd3_launchEPKvS1_S1_PvS1_S2_S2_S1_S1_S2_S2_iiiiiiiiP12ihipStream_tPiPKNS_7MeanJobE"]
+    B, H, W, C = shape
+    none, at, cuts, mean = ctypes.c_void_p(0), ctypes.c_void_p(256), (ctypes.c_int * 3)(), Mean(n=1, B=B, D=2 * C)
+    for add, want in ((None, 0), (at, 0 if stores else -1)):
+        assert launch(none, none, add, *[none] * 8, B, H, W, H // 2, W // 2, C, k, _lib.dtype_code(torch.bfloat16), none, cuts,
+                      ctypes.byref(mean)) == want
+    assert min(cuts) >= 1

@@ -204,3 +204,8 @@ def test_pooled_gradient_in_the_store_is_the_pools(k, shape, pooled):
         assert rc == 0
     assert pool(at(add), at(dx[1]), B, H, W, C, h, w, 1, _lib.dtype_code(dt), s) == 0
     assert bool(dx[1].isfinite().all()) and torch.equal(*dx)
+
+
+def test_pooled_gradient_behind_the_store(oracle):
+    """Odd extents where the pooled gradient is better added by a launch of its own (16 steps a run that ends last)."""
+    _block_case(oracle, 664, 9, (54, 11, 8, 664), torch.bfloat16)
