@@ -865,22 +865,25 @@ int dense_wide_bwd_pair_launch(const void* gy, const void* w, const void* b, voi
         wg = WideArgs{gy, b, nullptr, nullptr, ws, M, N, NO, M, NO, 1, p.mt, p.nt, p.splits, p.kper};
         nw = p.mt * p.nt * p.splits, nparts = p.splits;
     }
-    if (sums) *sums = riding_sums(*sums, nw + (long long)rows.mt * rows.nt, es);
+    ColsumJob riding{};
+    if (sums) riding = riding_sums(*sums, nw + (long long)rows.mt * rows.nt, es);
+    const ColsumJob* const ride = sums ? &riding : nullptr;
     int e = -1;
     if (es == 4) {
-        if (small) e = pair_go<float, 64, 64, 0, 0, 2>(rows, wg, any, nw, sums, s);
-        else if (p.bm == 64 && p.bn == 64) e = pair_go<float, 64, 64, 64, 64, 2>(rows, wg, any, nw, sums, s);
+        if (small) e = pair_go<float, 64, 64, 0, 0, 2>(rows, wg, any, nw, ride, s);
+        else if (p.bm == 64 && p.bn == 64) e = pair_go<float, 64, 64, 64, 64, 2>(rows, wg, any, nw, ride, s);
     } else if (p.bm == 128 && p.bn == 128) {
         auto go = [&](auto t) {
             using T = decltype(t);
-            if (bn == 192) return pair_go<T, 128, 192, 128, 128, 2>(rows, wg, any, nw, sums, s);
-            if (bm == 64 && bn == 128) return pair_go<T, 64, 128, 128, 128, kDeep>(rows, wg, any, nw, sums, s);
-            if (bm == 128 && bn == 128) return pair_go<T, 128, 128, 128, 128, 2>(rows, wg, any, nw, sums, s);
+            if (bn == 192) return pair_go<T, 128, 192, 128, 128, 2>(rows, wg, any, nw, ride, s);
+            if (bm == 64 && bn == 128) return pair_go<T, 64, 128, 128, 128, kDeep>(rows, wg, any, nw, ride, s);
+            if (bm == 128 && bn == 128) return pair_go<T, 128, 128, 128, 128, 2>(rows, wg, any, nw, ride, s);
             return -1;
         };
         e = dtype == kF16 ? go(f16_t{}) : go(bf16_t{});
     }
     if (e) return e;
+    if (sums) *sums = riding;   // (where no kernel takes the layer the caller's plan stands)
     if (dtype == kF32) return wgrad_reduce_launch<float>((const float*)ws, dw, nparts, M * NO, s);
     if (dtype == kF16) return wgrad_reduce_launch<f16_t>((const float*)ws, dw, nparts, M * NO, s);
     return wgrad_reduce_launch<bf16_t>((const float*)ws, dw, nparts, M * NO, s);

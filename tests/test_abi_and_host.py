@@ -273,3 +273,19 @@ def test_where_a_pooled_gradient_is_added(shape, k, stores):
         assert launch(none, none, add, *[none] * 8, B, H, W, H // 2, W // 2, C, k, _lib.dtype_code(torch.bfloat16), none, cuts,
                       ctypes.byref(mean)) == want
     assert min(cuts) >= 1
+
+
+@pytest.mark.parametrize("dtype,N,D,I", [(torch.bfloat16, 800, 256, 64), (torch.float16, 2000, 512, 64), (torch.float32, 848, 780, 448)])
+def test_plans_of_sums_that_do_not_ride(dtype, N, D, I):
+    """Where no launch takes both gradients of a layer, the column sums that would have ridden there keep the plan for where they run instead."""
+    from pyramidconvblock_amd import _lib
+
+    class Sums(ctypes.Structure):   # ColsumJob of csrc/mean_any.h
+        _fields_ = [("x", ctypes.c_void_p), ("part", ctypes.c_void_p)] + [(n, ctypes.c_int) for n in ("B", "P", "C", "n", "len", "lanes_log", "slices")]
+
+    both = _lib.lib()["_ZN3pdw26dense_bwd_both_sums_launchEPKvS1_S1_PvS2_S2_mPKfixiiiP12ihipStream_tPNS_9ColsumJobE"]
+    at, none = ctypes.c_void_p(4096), ctypes.c_void_p(0)
+    given = (4096, 4096, 1, N, D, 32, -(-N // 32), 5, -(-D // 128))
+    sums = Sums(*given)
+    r = both(at, at, at, at, at, at, ctypes.c_size_t(1 << 40), none, 1, ctypes.c_longlong(N), D, I, _lib.dtype_code(dtype), none, ctypes.byref(sums))
+    assert r == -1 and tuple(getattr(sums, n) for n, _ in Sums._fields_) == given
