@@ -494,7 +494,7 @@ __global__ __launch_bounds__(256, (STAGES == 2 ? kWideOccupancy<T, BM, BN> : 1))
     extern __shared__ __align__(16) char dsm[];
     const int blk = blockIdx.x;
     if (blk < nrows) wide_gemm_body<T, BM, BN, false, false, false, STAGES, false, true>(g, blk, nrows, qa);
-    else colsum_body<T>(sums, blk - nrows, (float*)dsm);
+    else colsum_body<T, true>(sums, blk - nrows, (float*)dsm);
 }
 
 // With the weights by a RowMap, and their packing (pack_weights.h) last.
@@ -504,7 +504,7 @@ __global__ __launch_bounds__(256, (STAGES == 2 ? kWideOccupancy<T, BM, BN> : 1))
     extern __shared__ __align__(16) char dsm[];
     const int blk = blockIdx.x;
     if (blk < nrows) wide_gemm_body<T, BM, BN, false, false, false, STAGES, true, true>(g, blk, nrows, qa);
-    else if (blk < nrows + nsums) colsum_body<T>(sums, blk - nrows, (float*)dsm);
+    else if (blk < nrows + nsums) colsum_body<T, true>(sums, blk - nrows, (float*)dsm);
     else pack_weights_body(pack, blk - nrows - nsums);
 }
 
@@ -533,7 +533,7 @@ __global__ __launch_bounds__(256, (STAGES == 2 ? kWideOccupancy<T, BM, BN> : 1))
     extern __shared__ __align__(16) char dsm[];
     const int blk = blockIdx.x;
     if (blk >= nw + nrows) {
-        colsum_body<T>(sums, blk - nw - nrows, (float*)dsm);
+        colsum_body<T, true>(sums, blk - nw - nrows, (float*)dsm);
     } else if (blk >= nw) {
         wide_gemm_body<T, BM, BN, false, true, false, STAGES>(rows, blk - nw, nrows);
     } else if constexpr (WM != 0) {
