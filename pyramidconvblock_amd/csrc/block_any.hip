@@ -151,12 +151,6 @@ int pack_weights(const PackArgs& g, hipStream_t stream) {
     return check_launch("pack_weights");
 }
 
-// Bytes of gy from which its column sums ride in the launch of conv_out's gradients, which are bound by their matrix products more than by
-// memory, instead of that of the gates.  us of the two launches: [32,56,56,128] fp32 (51 MB) 65.9 -> 61.5, [4,64,64,1152] fp16 (38 MB)
-// 81.7 -> 79.5, [8,112,112,256] bf16 (51 MB) 58.4 -> 55.9, [104,27,28,280] 68.6 -> 66.9, [8,48,48,256] fp32 (19 MB) 40.3 -> 37.8,
-// [6,56,56,256] bf16 (9.6 MB) 18.8 -> 18.7; [2,40,40,640] bf16 (4.1 MB) 17.6 -> 17.9, [3,25,20,920] bf16 (2.8 MB) 20.3 -> 20.5.
-constexpr size_t kRidingSums = 8 << 20;
-
 bool rows_whole_tiles(const Shape& s) { return s.P % pdw_dense_colsum_rows() == 0; }
 
 int forward(const Shape& s, const Saved& v, const void* x, const Weights& given, const void* w_pool, const void* b_pool,
@@ -292,8 +286,8 @@ int backward(const Shape& s, const Saved& v, const BwdWork& g, const void* gy, c
     float* gparts = nullptr;
     const bool any_mean = mean_any_ok(gy, w_pool, v.m, s.D, s.es);
     ColsumJob sums = colsum_plan(gy, (float*)g.ws_pool, s.B, s.P, s.D, s.es);
-    // ... or, where it is large, by workgroups of their own behind those gradients' (else in the gates' launch, as a part of which they take no time)
-    const bool ride = any_mean && (size_t)s.N * s.D * s.es >= kRidingSums;
+    // ... or, where that is faster, by workgroups of their own behind those gradients' (else in the gates' launch, as a part of which they take no time)
+    const bool ride = any_mean && dense_wide_sums_ride(s.N, s.D, s.I, dt);
     bool summed = false;
     if (pair_cs || pdw_dense_bwd_pair_supported(s.D, s.I, dt)) {
         if (pair_cs) gparts = g.gparts;

@@ -843,6 +843,23 @@ int dense_wide_wgrad_launch(const void* a, const void* b, void* dw, void* ws, lo
     return wgrad_reduce_launch<bf16_t>((const float*)ws, dw, p.splits, M * NO, s);
 }
 
+// Whether the column sums of gy, a tensor of N x M, are best made by workgroups of their own in the launch of both gradients of its layer, which is bound by
+// its matrix products more than by memory, instead of that of the gates, which has other bytes to move: where it is large, and twice that where 16-bit
+// products fill no more than one round of 512 workgroups, whose tiles were cut to end together and which the sums then outlast.  us of the two
+// launches: [32,56,56,128] fp32 (51 MB) 65.9 -> 61.5, [4,64,64,1152] fp16 (38 MB) 81.7 -> 79.5, [8,112,112,256] bf16 (51 MB) 58.4 -> 55.9, [104,27,28,280]
+// 68.6 -> 66.9, [8,48,48,256] fp32 (19 MB) 40.3 -> 37.8; [2,40,40,640] bf16 (4.1 MB) 17.6 and 17.9, [3,25,20,920] (2.8 MB) 20.3 and 20.5.  Sums over random
+// 16-bit layers: 8 to 16 MB, one round 71 of them 1842 and 1889, more 54 of them 1664 -> 1632; 16 to 30 MB, one round 32 of them 1059 -> 1041, more 62 of
+// them 2567 -> 2501; more than 30 MB 56 of them 4009 -> 3910 ([71,13,12,552] bf16, 12 MB in one round, 24.4 and 27.0).
+bool dense_wide_sums_ride(long long N, int M, int NO, int dtype) {
+    const int es = dtype == kF32 ? 4 : 2;
+    const long long bytes = N * M * es, large = 8 << 20;
+    if (bytes < large || bytes >= 2 * large || es == 4) return bytes >= large;
+    const WgradPlan p = wgrad_plan(N, M, NO, es);
+    int bm, bn;
+    rows_tiles(N, M, NO, bm, bn);
+    return (long long)p.mt * p.nt * p.splits + (long long)cdiv(N, bm) * cdiv(NO, bn) > 512;
+}
+
 // dx[N,NO] = gy[N,M] W (+ rowbias), W stored [M][NO], and dW[M][NO] = gy^T b, in one launch; -1: not covered, or products that
 // other kernels make (the caller makes them one by one).  max_chunks: partials the workspace holds.
 // sums (optional): of gy, planned here within what it was given as.

@@ -289,3 +289,19 @@ def test_plans_of_sums_that_do_not_ride(dtype, N, D, I):
     sums = Sums(*given)
     r = both(at, at, at, at, at, at, ctypes.c_size_t(1 << 40), none, 1, ctypes.c_longlong(N), D, I, _lib.dtype_code(dtype), none, ctypes.byref(sums))
     assert r == -1 and tuple(getattr(sums, n) for n, _ in Sums._fields_) == given
+
+
+@pytest.mark.parametrize("dtype,shape,inter,rides", [
+    # small; one round of products and more, of 8 to 16 MB; larger; fp32 by its size alone
+    (torch.bfloat16, (2, 40, 40, 640), 320, False), (torch.bfloat16, (71, 13, 12, 552), 288, False), (torch.float16, (105, 7, 7, 848), 432, False),
+    (torch.bfloat16, (8, 58, 59, 168), 96, True), (torch.float16, (4, 64, 64, 1152), 576, True), (torch.float32, (32, 56, 56, 128), 64, True),
+    (torch.float32, (2, 40, 40, 512), 256, False),
+])
+def test_where_column_sums_ride(dtype, shape, inter, rides):
+    """csrc/dense_wide.hip: the sums of an output gradient in its layer's launch, or (not) in that of the gates."""
+    from pyramidconvblock_amd import _lib
+
+    f = _lib.lib()["_ZN3pdw20dense_wide_sums_rideExiii"]
+    f.restype = ctypes.c_bool
+    B, H, W, C = shape
+    assert f(ctypes.c_longlong(B * H * W), C, inter, _lib.dtype_code(dtype)) == rides
