@@ -41,8 +41,11 @@ namespace pdw {
 // workgroup a unit -> this: both scales of [32,56,56,64] filter 13 50.5 -> 45.5, [22,72,73,32] filter 13 36.6 -> 32.2, [3,57,61,100]
 // filter 15 24.2 -> 18.2, [16,56,56,64] filter 15 38.9 -> 33.3, [24,36,36,100] filter 17 57.0 -> 50.7, [2,20,20,32] filter 15 9.0 -> 8.5.  With the pooled
 // gradient added (ADD > 0), which the planner cuts into one workgroup a unit, all stay ([32,56,56,64] filter 13 38.3, 39.2 with three
-// blocks kept, [24,36,36,100] filter 17 35.8 and 36.6),
-// and in launches of no more than that with long bands (ADD = -1: [32,56,56,64] filter 13 38.7, 39.7 with three blocks kept).
+// blocks kept, [24,36,36,100] filter 17 35.8 and 36.6), and in launches of no more than that whose bands are of three patch rows or more (ADD = -1),
+// where reading operands again outweighs the longer start-up: with two or three blocks kept -> all, by the rows of a band, 12: [77,10,10,80]
+// filter 15 12.9 -> 12.4, [40,25,25,312] 16.4 -> 15.7, [3,106,107,112] filter 17 17.4 -> 17.0; 16: [21,31,32,276] filter 17 23.1 -> 22.3; 24: [7,21,20,440]
+// filter 13 10.8 -> 10.5, [6,45,60,152] filter 15 26.5 -> 25.3; 48: [19,45,49,92] 16.9 -> 15.9; 56: [32,56,56,64] filter 13 39.7 -> 38.7, [1,106,106,496]
+// filter 17 22.3 -> 21.2 (25 such launches, all of them faster); 8: [34,16,16,60] filter 17 10.0 and 11.0; 4: [8,12,16,252] filter 13 8.0 and 8.4.
 template <int K, int ADD>
 constexpr int f32t_kept() {
     return ADD != 0 || K <= 11 ? (K + 6) / 4 : K == 13 ? 3 : 2;
@@ -221,7 +224,7 @@ __device__ __forceinline__ void dwconv_f32_body(const float* __restrict__ x, con
         arsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(add + (long long)b0 * g.AH * g.AW * g.C), (short)0,
                                                   (int)((long long)min(NI, g.B - b0) * g.AH * g.AW * g.C * 4), 0x00020000);
         if constexpr (ADD == 2) {
-            // (read by the first add_fetch of a row in it behind the first step's barrier)
+            // (read behind the barrier before the first add_fetch)
             for (int i = tid; i < rows_valid; i += NT) {
                 int b;
                 float w0, w1;
@@ -462,7 +465,7 @@ int launch_f32t(const void* x, const void* w, const void* add, void* y, int B, i
         hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(512), lds, s, (const float*)x, (const float*)w,             \
                            (const float*)add, (float*)y, g);                                                               \
     }
-    const int mode = !add ? (K >= 13 && nblocks <= 256 && g.BR >= 40 ? -1 : 0) : g.OH == 2 * AH && g.OW == 2 * AW ? 1 : 2;
+    const int mode = !add ? (K >= 13 && nblocks <= 256 && g.BR >= 12 ? -1 : 0) : g.OH == 2 * AH && g.OW == 2 * AW ? 1 : 2;
 #define PDW_F32T_M(NPC) \
     if (mode == 0) PDW_F32T(NPC, 0) else if (mode == 1) PDW_F32T(NPC, 1) else if (mode == 2) PDW_F32T(NPC, 2) else PDW_F32T(NPC, (K >= 13 ? -1 : 0))
     if (npc == 16) {

@@ -370,3 +370,13 @@ def test_fp32_operands_in_registers_and_in_lds(k, shape):
     ends = lambda t: t[[0, -1]]
     assert_close(ends(dwconv_forward(x, w, *geo)), dense(x, w), torch.float32, "y")
     assert_close(ends(dwconv_dgrad(x, w, x.shape, *geo)), dense(x, w.flip(0, 1)), torch.float32, "dx")
+
+
+@pytest.mark.parametrize("k", [13, 15, 17])
+@pytest.mark.parametrize("shape", [
+    # one workgroup a compute unit in bands of three patch rows and more, tiles of four images, two and one, a last band of one row
+    (77, 10, 10, 80), (21, 31, 14, 136), (6, 25, 30, 200), (9, 33, 61, 56),
+])
+def test_fp32_operands_in_registers_of_short_bands(k, shape):
+    """fp32 on the matrix cores, all operands kept (csrc/dwconv_f32t.h, ADD = -1): forward and input gradient against float64."""
+    test_fp32_operands_in_registers_and_in_lds(k, shape)
