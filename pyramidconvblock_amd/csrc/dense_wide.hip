@@ -143,7 +143,7 @@ struct Operand {
         }
     }
     // rows by quads from `quad0` on, of `quads`
-    __device__ __forceinline__ void init(const char* p, int ld, const QuadRows& rows, long long quad0, long long quads, int inner) {
+    __device__ __forceinline__ void init(const char* p, int ld, const QuadRows& rows, long long quad0, long long quads) {
         static_assert(!TR, "stored by results");
         const long long bytes = (4 * quads - rows.pix0) * ld * ES;
         rsrc = rsrc_of(p + (long long)rows.pix0 * ld * ES, (uint32_t)(bytes < 0x7fffffffLL ? bytes : 0x7fffffffLL));
@@ -283,7 +283,7 @@ __device__ __forceinline__ void wide_gemm_body(const WideArgs& g, int blk, int n
     QuadRows quad;
     if constexpr (QUAD) {
         quad.init(qa, m0 / 4);
-        a.init((const char*)g.a, g.lda, quad, m0 / 4, g.M / 4, (int)g.Kd);
+        a.init((const char*)g.a, g.lda, quad, m0 / 4, g.M / 4);
     } else {
         a.init((const char*)g.a, g.lda, m0, g.M, kb, ke);
     }
@@ -688,7 +688,10 @@ WgradPlan wgrad_plan(long long N, int M, int NO, int es) {
 }
 
 // Column sums that ride behind `blocks` workgroups of products: few, who read for as long as those take; more of them get in the
-// products' way.  No more than compute units are left in a launch of one workgroup each (kDeep).
+// products' way.  In 16 bits as many as a launch of one workgroup a compute unit (kDeep) leaves units, where those are 64 to 192 and the images'
+// slices make no more by themselves; such products go in two stages where these do, where fewer units are left and where weights are packed
+// beside them.  (us, four stages and the launch that pooled and summed -> two stages with both: [40,8,8,1024] bf16 14.2 -> 14.2, [3,14,14,920], packed, 15.6 -> 15.4,
+// [12,14,14,920] 15.6 -> 14.7.)
 ColsumJob riding_sums(const ColsumJob& j, long long blocks, int es) {
     const long long spare = 256 - blocks;
     const int n = es == 2 && spare >= 64 && spare < 192 ? (int)spare : 192, each = j.B * j.slices;

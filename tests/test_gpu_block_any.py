@@ -227,3 +227,92 @@ def test_error_of_riding_sums():
         for p in (p for n, p in m.named_parameters() if n.endswith("bias")):
             err.append(float((p.grad.double() - want).norm() / want.norm()))
     assert len(err) == 8 and sum(err) / 8 <= 1.66e-7, err
+
+
+@pytest.mark.parametrize("k,shape", [
+    # behind the weight gradients' workgroups and in front of them (448 to 512 of those), tiles of one, two and four images
+    (9, (3, 30, 30, 64)), (3, (16, 30, 26, 64)), (5, (16, 40, 64, 32)), (11, (2, 40, 64, 32)), (11, (16, 30, 64, 32)), (13, (2, 24, 130, 32)), (13, (16, 30, 64, 32)),
+    (15, (2, 60, 64, 32)), (15, (3, 57, 61, 100)), (15, (16, 30, 64, 32)), (17, (2, 60, 64, 32)), (17, (16, 30, 64, 32)),
+])
+def test_fp32_half_scale_in_the_weight_gradients_launch(k, shape):
+    """That launch by its name (csrc/dwconv_wgrad_f32t.h), which has to take the case: the pooled scale's input gradient and both weight gradients
+    against float64."""
+    import ctypes
+
+    import torch.nn.functional as F
+
+    from pyramidconvblock_amd import _lib
+
+    L, (B, H, W, C) = _lib.lib(), shape
+    joint = L["_ZN3pdw29dwconv_wgrad_f32t_pair_launchEPKvS1_PvS2_iiS1_S1_S2_S2_iiiiiiP12ihipStream_tPKNS_7MeanJobES1_S2_"]
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    r = lambda *s: torch.randn(*s, generator=gen, device="cuda")
+    ext = ((H, W), (H // 2, W // 2))
+    x, gy, w1 = [r(B, *e, C) for e in ext], [r(B, *e, C) for e in ext], r(k, k, C) / k
+    dw, dx1 = [torch.empty(k, k, C, device="cuda") for _ in ext], torch.empty_like(x[1])
+    ws = [torch.empty(L.pdw_dwconv_wgrad_workspace_bytes(B, *e, C, k, k, 1, 1, k // 2, k // 2, 1, 1, 0) // 4 + 1, device="cuda") for e in ext]
+    at = lambda t: ctypes.c_void_p(t.data_ptr())
+    none, s = ctypes.c_void_p(0), ctypes.c_void_p(_lib.stream_ptr(dx1.device))
+    assert _lib.dtype_code(torch.float32) == 0
+    assert joint(at(x[0]), at(gy[0]), at(dw[0]), at(ws[0]), *ext[0], at(x[1]), at(gy[1]), at(dw[1]), at(ws[1]), *ext[1], B, C, k, k // 2, s, none,
+                 at(w1), at(dx1)) == 0
+    nchw = lambda t: t.double().cpu().permute(0, 3, 1, 2)
+    oihw = lambda t: t.double().cpu().permute(2, 0, 1).unsqueeze(1)
+    for i in range(2):
+        xr, wr = nchw(x[i]).requires_grad_(), oihw(w1).requires_grad_()
+        F.conv2d(xr, wr, padding=k // 2, groups=C).backward(nchw(gy[i]))
+        assert_close(dw[i], wr.grad.squeeze(1).permute(1, 2, 0).numpy(), torch.float32, "grad w%d" % i)
+    assert_close(dx1, xr.grad.permute(0, 2, 3, 1).numpy(), torch.float32, "dx")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape,half,padded", [
+    # tiles of 64 x 64 in two stages and in four, 64 x 128, 128 x 64, 128 x 128, 128 x 192; an image that ends within a tile, tiles past the last row
+    ((2, 20, 22, 264), 32, 32), ((2, 20, 22, 400), 32, 32), ((3, 14, 18, 520), 72, 72), ((11, 56, 56, 136), 32, 32), ((4, 66, 62, 264), 72, 72), ((6, 62, 60, 256), 192, 192),
+    # the same with padded halves, whose weights are packed beside
+    ((2, 20, 22, 264), 30, 32), ((2, 20, 22, 400), 27, 32), ((3, 14, 18, 520), 66, 72), ((11, 56, 56, 136), 30, 32), ((4, 66, 62, 264), 66, 72), ((6, 62, 60, 256), 190, 192),
+])
+def test_first_layer_with_pool_and_sums(dtype, shape, half, padded):
+    """The first layer's launch by its name (csrc/dense_wide.hip) in every tile: its result and the sums of its input against float64, the pool and the packed weights
+    to the bit."""
+    import ctypes
+
+    from pyramidconvblock_amd import _lib
+
+    class Sums(ctypes.Structure):   # ColsumJob of csrc/mean_any.h
+        _fields_ = [("x", ctypes.c_void_p), ("part", ctypes.c_void_p)] + [(n, ctypes.c_int) for n in ("B", "P", "C", "n", "len", "lanes_log", "slices")]
+
+    class Pack(ctypes.Structure):   # PackArgs of csrc/pack_weights.h
+        _fields_ = [("p", ctypes.c_void_p * 8)] + [(n, ctypes.c_int) for n in ("D", "G", "Gp", "n_up", "n_out", "n_dw")]
+
+    L = _lib.lib()
+    plan = L["_ZN3pdw21dense_wide_first_planEPNS_9ColsumJobExiiiii"]
+    plan.restype = ctypes.c_bool
+    launch = L["_ZN3pdw23dense_wide_first_launchEPKvS1_PvS2_ixiiRKNS_9ColsumJobEPKNS_8PackArgsEiP12ihipStream_t"]
+    (B, H, W, D), NO, k = shape, 2 * padded, 3
+    N, dt = B * H * W, _lib.dtype_code(dtype)
+    gen = torch.Generator(device="cuda").manual_seed(D)
+    r = lambda *s: torch.randn(*s, generator=gen, device="cuda").to(dtype)
+    x, w = r(*shape), (r(2 * half, D) / 16).to(dtype)
+    given = [w, r(D, 2 * half), r(k, k, 2 * half), r(k, k, 2 * half)]
+    wide = [torch.zeros(NO, D, device="cuda", dtype=dtype), *[torch.zeros(*s, NO, device="cuda", dtype=dtype) for s in ((D,), (k, k), (k, k))]]
+    for i in range(2):
+        a, b = slice(i * half, (i + 1) * half), slice(i * padded, i * padded + half)
+        wide[0][b] = given[0][a]
+        for q, t in zip(wide[1:], given[1:]):
+            q[..., b] = t[..., a]
+    packed = [torch.full_like(t, float("nan")) for t in wide]
+    y, pool = torch.full((B, H, W, NO), float("nan"), device="cuda", dtype=dtype), torch.full((B, H // 2, W // 2, NO), float("nan"), device="cuda", dtype=dtype)
+    at, sums = lambda t: ctypes.c_void_p(t.data_ptr()), Sums()
+    assert plan(ctypes.byref(sums), ctypes.c_longlong(N), D, NO, B, H * W, dt)
+    part = torch.full((B, sums.n, D), float("nan"), device="cuda")
+    sums.x, sums.part = x.data_ptr(), part.data_ptr()
+    pack = Pack((ctypes.c_void_p * 8)(*[t.data_ptr() for t in given + packed]), D, half, padded, NO * D // 8, NO * D // 8, k * k * NO // 8)
+    assert launch(at(x), at(w), at(y), at(pool), W // 2, ctypes.c_longlong(N), D, NO, ctypes.byref(sums), ctypes.byref(pack) if half != padded else None, dt,
+                  ctypes.c_void_p(_lib.stream_ptr(x.device))) == 0
+    assert_close(y, (x.double().cpu().reshape(N, D) @ wide[0].double().cpu().t()).reshape(y.shape).numpy(), dtype, "y")
+    q = y.float().reshape(B, H // 2, 2, W // 2, 2, NO)
+    assert torch.equal(pool, ((((q[:, :, 0, :, 0] + q[:, :, 0, :, 1]) + q[:, :, 1, :, 0]) + q[:, :, 1, :, 1]) * 0.25).to(dtype))
+    assert_close(part.double().sum(1).float(), x.double().sum((1, 2)).cpu().numpy(), torch.float32, "sums")
+    if half != padded:
+        assert all(torch.equal(a, b) for a, b in zip(packed, wide))
