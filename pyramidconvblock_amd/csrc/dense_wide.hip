@@ -695,7 +695,9 @@ WgradPlan wgrad_plan(long long N, int M, int NO, int es) {
 ColsumJob riding_sums(const ColsumJob& j, long long blocks, int es) {
     const long long spare = 256 - blocks;
     const int n = es == 2 && spare >= 64 && spare < 192 ? (int)spare : 192, each = j.B * j.slices;
-    return colsum_plan(j.x, j.part, j.B, j.P, j.C, es, n > each ? n - each + 1 : 1);
+    ColsumJob r = colsum_plan(j.x, j.part, j.B, j.P, j.C, es, n > each ? n - each + 1 : 1);
+    r.pairs = r.len > j.len;
+    return r;
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }

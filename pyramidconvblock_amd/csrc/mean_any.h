@@ -16,6 +16,7 @@ struct ColsumJob {
     float* part;     // [B][n][C]
     int B, P, C, n, len;      // n ranges of len positions
     int lanes_log, slices;    // 1 << lanes_log vectors of a row to a workgroup, slices of them
+    bool pairs;               // colsum_body<T, true>: eight positions in pairs
 };
 
 inline int colsum_workgroups(const ColsumJob& j) { return j.B * j.n * j.slices; }
@@ -23,7 +24,7 @@ inline int colsum_workgroups(const ColsumJob& j) { return j.B * j.n * j.slices; 
 // part = nullptr: only the plan (for the size of the partials, which fewer workgroups never make larger).
 inline ColsumJob colsum_plan(const void* x, float* part, int B, int P, int C, int esize, int workgroups = 512) {
     const int V = 16 / esize, vecs = C / V;
-    ColsumJob j{x, part, B, P, C, 1, P, 3, 1};
+    ColsumJob j{x, part, B, P, C, 1, P, 3, 1, false};
     while (j.lanes_log < 5 && (1 << j.lanes_log) < vecs) ++j.lanes_log;
     j.slices = cdiv(vecs, 1 << j.lanes_log);
     const int pl = 256 >> j.lanes_log;
@@ -35,10 +36,10 @@ inline ColsumJob colsum_plan(const void* x, float* part, int B, int P, int C, in
     return j;
 }
 
-// red: 256 * V floats of LDS (V = values per 16 bytes).  PAIRS: of every eight positions pairs, then pairs of those, before they are added to the
-// sum (as many additions): where ranges are longer because fewer workgroups ride along, a thread's chain of roundings is shorter all the same
-// (error of the sums over 100352 rows of 128 in fp32, 2-norm: 512 workgroups 1.35e-7, 192 1.8e-7, 192 in pairs 1.24e-7; over 16384 of 1152
-// 1.5e-7, 2.0e-7, 1.3e-7).
+// red: 256 * V floats of LDS (V = values per 16 bytes).  PAIRS, for jobs that say so: of every eight positions pairs, then pairs of those, before
+// they are added to the sum (as many additions): where ranges are longer because fewer workgroups ride along, a thread's chain of roundings is
+// shorter all the same (error of the sums over 100352 rows of 128 in fp32, 2-norm: 512 workgroups 1.35e-7, 192 1.8e-7, 192 in pairs 1.24e-7; over
+// 16384 of 1152 1.5e-7, 2.0e-7, 1.3e-7).
 template <typename T, bool PAIRS = false>
 __device__ __forceinline__ void colsum_body(const ColsumJob& j, int wg, float* red) {
     constexpr int V = 16 / (int)sizeof(T);
@@ -56,7 +57,7 @@ __device__ __forceinline__ void colsum_body(const ColsumJob& j, int wg, float* r
             ChanVec<T, V> xv[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u) xv[u] = *reinterpret_cast<const ChanVec<T, V>*>(xb + (long long)(p + u * PL) * j.C);
-            if constexpr (PAIRS) {
+            if (PAIRS && j.pairs) {   // (uniform)
 #pragma unroll
                 for (int v = 0; v < V; ++v) {
                     auto two = [&](int u) { return to_f32(xv[u].v[v]) + to_f32(xv[u + 1].v[v]); };

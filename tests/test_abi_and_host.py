@@ -281,11 +281,12 @@ def test_plans_of_sums_that_do_not_ride(dtype, N, D, I):
     from pyramidconvblock_amd import _lib
 
     class Sums(ctypes.Structure):   # ColsumJob of csrc/mean_any.h
-        _fields_ = [("x", ctypes.c_void_p), ("part", ctypes.c_void_p)] + [(n, ctypes.c_int) for n in ("B", "P", "C", "n", "len", "lanes_log", "slices")]
+        _fields_ = [("x", ctypes.c_void_p), ("part", ctypes.c_void_p)] + [(n, ctypes.c_int) for n in ("B", "P", "C", "n", "len", "lanes_log", "slices")] \
+            + [("pairs", ctypes.c_bool)]
 
     both = _lib.lib()["_ZN3pdw26dense_bwd_both_sums_launchEPKvS1_S1_PvS2_S2_mPKfixiiiP12ihipStream_tPNS_9ColsumJobE"]
     at, none = ctypes.c_void_p(4096), ctypes.c_void_p(0)
-    given = (4096, 4096, 1, N, D, 32, -(-N // 32), 5, -(-D // 128))
+    given = (4096, 4096, 1, N, D, 32, -(-N // 32), 5, -(-D // 128), False)
     sums = Sums(*given)
     r = both(at, at, at, at, at, at, ctypes.c_size_t(1 << 40), none, 1, ctypes.c_longlong(N), D, I, _lib.dtype_code(dtype), none, ctypes.byref(sums))
     assert r == -1 and tuple(getattr(sums, n) for n, _ in Sums._fields_) == given

@@ -280,7 +280,8 @@ def test_first_layer_with_pool_and_sums(dtype, shape, half, padded):
     from pyramidconvblock_amd import _lib
 
     class Sums(ctypes.Structure):   # ColsumJob of csrc/mean_any.h
-        _fields_ = [("x", ctypes.c_void_p), ("part", ctypes.c_void_p)] + [(n, ctypes.c_int) for n in ("B", "P", "C", "n", "len", "lanes_log", "slices")]
+        _fields_ = [("x", ctypes.c_void_p), ("part", ctypes.c_void_p)] + [(n, ctypes.c_int) for n in ("B", "P", "C", "n", "len", "lanes_log", "slices")] \
+            + [("pairs", ctypes.c_bool)]
 
     class Pack(ctypes.Structure):   # PackArgs of csrc/pack_weights.h
         _fields_ = [("p", ctypes.c_void_p * 8)] + [(n, ctypes.c_int) for n in ("D", "G", "Gp", "n_up", "n_out", "n_dw")]
