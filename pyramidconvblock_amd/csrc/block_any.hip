@@ -287,7 +287,7 @@ int backward(const Shape& s, const Saved& v, const BwdWork& g, const void* gy, c
     const bool any_mean = mean_any_ok(gy, w_pool, v.m, s.D, s.es);
     ColsumJob sums = colsum_plan(gy, (float*)g.ws_pool, s.B, s.P, s.D, s.es);
     // ... or, where that is faster, by workgroups of their own behind those gradients' (else in the gates' launch, as a part of which they take no time)
-    const bool ride = any_mean && dense_wide_sums_ride(s.N, s.D, s.I, dt);
+    const bool ride = any_mean && dense_wide_sums_ride(sums, s.I, dt);
     bool summed = false;
     if (pair_cs || pdw_dense_bwd_pair_supported(s.D, s.I, dt)) {
         if (pair_cs) gparts = g.gparts;

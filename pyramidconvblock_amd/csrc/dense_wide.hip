@@ -848,21 +848,26 @@ int dense_wide_wgrad_launch(const void* a, const void* b, void* dw, void* ws, lo
     return wgrad_reduce_launch<bf16_t>((const float*)ws, dw, p.splits, M * NO, s);
 }
 
-// Whether the column sums of gy, a tensor of N x M, are best made by workgroups of their own in the launch of both gradients of its layer, which is bound by
-// its matrix products more than by memory, instead of that of the gates, which has other bytes to move: where it is large, and twice that where 16-bit
-// products fill no more than one round of 512 workgroups, whose tiles were cut to end together and which the sums then outlast.  us of the two
-// launches: [32,56,56,128] fp32 (51 MB) 65.9 -> 61.5, [4,64,64,1152] fp16 (38 MB) 81.7 -> 79.5, [8,112,112,256] bf16 (51 MB) 58.4 -> 55.9, [104,27,28,280]
-// 68.6 -> 66.9, [8,48,48,256] fp32 (19 MB) 40.3 -> 37.8; [2,40,40,640] bf16 (4.1 MB) 17.6 and 17.9, [3,25,20,920] (2.8 MB) 20.3 and 20.5.  Sums over random
-// 16-bit layers: 8 to 16 MB, one round 71 of them 1842 and 1889, more 54 of them 1664 -> 1632; 16 to 30 MB, one round 32 of them 1059 -> 1041, more 62 of
-// them 2567 -> 2501; more than 30 MB 56 of them 4009 -> 3910 ([71,13,12,552] bf16, 12 MB in one round, 24.4 and 27.0).
-bool dense_wide_sums_ride(long long N, int M, int NO, int dtype) {
+// Whether the column sums j of the gradient of a layer with NO inputs are best made by workgroups of their own in the launch of both its gradients, which is bound
+// by its matrix products more than by memory, instead of that of the gates, which has other bytes to move: where it is large, and twice that where 16-bit
+// products fill no more than one round of 512 workgroups, whose tiles were cut to end together and which the sums then outlast; not where an image and
+// slice is one workgroup's alone and its chain of positions is long beside the tiles' products.  us of the two launches: [32,56,56,128] fp32 (51 MB) 65.9 -> 61.5,
+// [4,64,64,1152] fp16 (38 MB) 81.7 -> 79.5, [8,112,112,256] bf16 (51 MB) 58.4 -> 55.9, [104,27,28,280] 68.6 -> 66.9, [8,48,48,256] fp32 (19 MB) 40.3 -> 37.8;
+// [2,40,40,640] bf16 (4.1 MB) 17.6 and 17.9, [3,25,20,920] (2.8 MB) 20.3 and 20.5.  Sums over random 16-bit layers: 8 to 16 MB, one round 71 of them 1842 and 1889,
+// more 54 of them 1664 -> 1632; 16 to 30 MB, one round 32 of them 1059 -> 1041, more 62 of them 2567 -> 2501; more than 30 MB 56 of them 4009 -> 3910
+// ([71,13,12,552] bf16, 12 MB in one round, 24.4 and 27.0).  One workgroup an image and slice, positions a thread over channels: [65,33,44,280] fp16
+// 182 / 280 84 and 94, [99,39,36,272] 176 / 272 119 and 126, [109,47,47,160] 276 / 160 98 and 109; [96,33,33,296] 136 / 296 95 -> 90, [54,40,40,344] 200 / 344 92 -> 89.
+bool dense_wide_sums_ride(const ColsumJob& j, int NO, int dtype) {
     const int es = dtype == kF32 ? 4 : 2;
-    const long long bytes = N * M * es, large = 8 << 20;
-    if (bytes < large || bytes >= 2 * large || es == 4) return bytes >= large;
-    const WgradPlan p = wgrad_plan(N, M, NO, es);
+    const long long N = (long long)j.B * j.P, bytes = N * j.C * es, large = 8 << 20;
+    if (bytes < large || es == 4) return bytes >= large;
+    const WgradPlan p = wgrad_plan(N, j.C, NO, es);
     int bm, bn;
-    rows_tiles(N, M, NO, bm, bn);
-    return (long long)p.mt * p.nt * p.splits + (long long)cdiv(N, bm) * cdiv(NO, bn) > 512;
+    rows_tiles(N, j.C, NO, bm, bn);
+    const long long blocks = (long long)p.mt * p.nt * p.splits + (long long)cdiv(N, bm) * cdiv(NO, bn);
+    if (bytes < 2 * large && blocks <= 512) return false;
+    const ColsumJob r = riding_sums(j, blocks, es);
+    return r.n > 1 || 5LL * r.len / (256 >> r.lanes_log) <= 3LL * j.C;
 }
 
 // dx[N,NO] = gy[N,M] W (+ rowbias), W stored [M][NO], and dW[M][NO] = gy^T b, in one launch; -1: not covered, or products that

@@ -160,7 +160,7 @@ int dense_wide_rows_launch(const void* x, const void* w, int w_kmajor, const voi
 size_t dense_wide_wgrad_workspace(long long N, int M, int NO);
 int dense_wide_bwd_pair_launch(const void* gy, const void* w, const void* b, void* dx, void* dw, void* ws, const float* rowbias, int P,
                                long long N, int M, int NO, int dtype, int max_chunks, hipStream_t s, struct ColsumJob* sums = nullptr);
-bool dense_wide_sums_ride(long long N, int M, int NO, int dtype);   // whether such sums are best made there
+bool dense_wide_sums_ride(const struct ColsumJob& j, int NO, int dtype);   // whether such sums are best made there
 // dense.hip: that for the widths whose products both run there; -1 = not covered (the caller makes the two products)
 int dense_bwd_both_launch(const void* gy, const void* w, const void* b, void* dx, void* dw, void* ws, size_t ws_bytes, const float* rowbias,
                           int P, long long N, int M, int NO, int dtype, hipStream_t s);

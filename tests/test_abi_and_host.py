@@ -292,17 +292,25 @@ def test_plans_of_sums_that_do_not_ride(dtype, N, D, I):
     assert r == -1 and tuple(getattr(sums, n) for n, _ in Sums._fields_) == given
 
 
+class _Sums(ctypes.Structure):   # ColsumJob of csrc/mean_any.h
+    _fields_ = [("x", ctypes.c_void_p), ("part", ctypes.c_void_p)] + [(n, ctypes.c_int) for n in ("B", "P", "C", "n", "len", "lanes_log", "slices")] \
+        + [("pairs", ctypes.c_bool)]
+
+
 @pytest.mark.parametrize("dtype,shape,inter,rides", [
-    # small; one round of products and more, of 8 to 16 MB; larger; fp32 by its size alone
+    # small; one round of products and more, of 8 to 16 MB; larger; fp32 by its size alone; one workgroup an image and slice, long and short chains
     (torch.bfloat16, (2, 40, 40, 640), 320, False), (torch.bfloat16, (71, 13, 12, 552), 288, False), (torch.float16, (105, 7, 7, 848), 432, False),
     (torch.bfloat16, (8, 58, 59, 168), 96, True), (torch.float16, (4, 64, 64, 1152), 576, True), (torch.float32, (32, 56, 56, 128), 64, True),
-    (torch.float32, (2, 40, 40, 512), 256, False),
+    (torch.float32, (2, 40, 40, 512), 256, False), (torch.float16, (65, 33, 44, 280), 144, False), (torch.float16, (109, 47, 47, 160), 80, False),
+    (torch.bfloat16, (96, 33, 33, 296), 160, True), (torch.float32, (34, 38, 38, 280), 140, True),
 ])
 def test_where_column_sums_ride(dtype, shape, inter, rides):
     """csrc/dense_wide.hip: the sums of an output gradient in its layer's launch, or (not) in that of the gates."""
     from pyramidconvblock_amd import _lib
 
-    f = _lib.lib()["_ZN3pdw20dense_wide_sums_rideExiii"]
+    f = _lib.lib()["_ZN3pdw20dense_wide_sums_rideERKNS_9ColsumJobEii"]
     f.restype = ctypes.c_bool
     B, H, W, C = shape
-    assert f(ctypes.c_longlong(B * H * W), C, inter, _lib.dtype_code(dtype)) == rides
+    vecs = C // (4 if dtype == torch.float32 else 8)
+    assert vecs > 16   # 32 vectors of a row to a workgroup
+    assert f(ctypes.byref(_Sums(0, 0, B, H * W, C, 4, -(-H * W // 4), 5, -(-vecs // 32), False)), inter, _lib.dtype_code(dtype)) == rides
