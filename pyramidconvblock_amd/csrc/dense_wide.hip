@@ -687,14 +687,16 @@ WgradPlan wgrad_plan(long long N, int M, int NO, int es) {
     return plans.get({N, M, NO, es}, [=] { return wgrad_make_plan(N, M, NO, es); });
 }
 
-// Column sums that ride behind `blocks` workgroups of products: few, who read for as long as those take; more of them get in the
-// products' way.  In 16 bits as many as a launch of one workgroup a compute unit (kDeep) leaves units, where those are 64 to 192 and the images'
-// slices make no more by themselves; such products go in two stages where these do, where fewer units are left and where weights are packed
-// beside them.  (us, four stages and the launch that pooled and summed -> two stages with both: [40,8,8,1024] bf16 14.2 -> 14.2, [3,14,14,920], packed, 15.6 -> 15.4,
-// [12,14,14,920] 15.6 -> 14.7.)
+// Column sums that ride behind `blocks` workgroups of products: as many workgroups as by themselves, which read while the products multiply.  (192 of them
+// are one or two more to a compute unit, but their longer chains outlast the products: us of both launches with the gates', by themselves, 192 and
+// all, 418 random 16-bit layers of 8 MB and more 21.2, 20.7 and 20.2 ms, 152 fp32 ones 10.2, 9.7 and 9.5; [65,33,44,280] fp16 84, 94 and 82.)  In 16 bits, where
+// a launch of one workgroup a compute unit (kDeep) leaves 64 units or more, no more than those, so that its products keep their four stages: us of the first
+// layer, nine of 144 to 180 tiles, by themselves 126, with all 98, with these 87.  (Weights packed beside them make it two stages all the same: [3,14,14,920]
+// bf16 15.6 -> 15.4, [12,14,14,920] 15.6 -> 14.7.)
 ColsumJob riding_sums(const ColsumJob& j, long long blocks, int es) {
     const long long spare = 256 - blocks;
-    const int n = es == 2 && spare >= 64 && spare < 192 ? (int)spare : 192, each = j.B * j.slices;
+    if (es == 4 || spare < 64 || colsum_workgroups(j) <= spare) return j;
+    const int n = (int)spare, each = j.B * j.slices;
     ColsumJob r = colsum_plan(j.x, j.part, j.B, j.P, j.C, es, n > each ? n - each + 1 : 1);
     r.pairs = r.len > j.len;
     return r;
@@ -850,24 +852,19 @@ int dense_wide_wgrad_launch(const void* a, const void* b, void* dw, void* ws, lo
 
 // Whether the column sums j of the gradient of a layer with NO inputs are best made by workgroups of their own in the launch of both its gradients, which is bound
 // by its matrix products more than by memory, instead of that of the gates, which has other bytes to move: where it is large, and twice that where 16-bit
-// products fill no more than one round of 512 workgroups, whose tiles were cut to end together and which the sums then outlast; not where an image and
-// slice is one workgroup's alone and its chain of positions is long beside the tiles' products.  us of the two launches: [32,56,56,128] fp32 (51 MB) 65.9 -> 61.5,
-// [4,64,64,1152] fp16 (38 MB) 81.7 -> 79.5, [8,112,112,256] bf16 (51 MB) 58.4 -> 55.9, [104,27,28,280] 68.6 -> 66.9, [8,48,48,256] fp32 (19 MB) 40.3 -> 37.8;
-// [2,40,40,640] bf16 (4.1 MB) 17.6 and 17.9, [3,25,20,920] (2.8 MB) 20.3 and 20.5.  Sums over random 16-bit layers: 8 to 16 MB, one round 71 of them 1842 and 1889,
-// more 54 of them 1664 -> 1632; 16 to 30 MB, one round 32 of them 1059 -> 1041, more 62 of them 2567 -> 2501; more than 30 MB 56 of them 4009 -> 3910
-// ([71,13,12,552] bf16, 12 MB in one round, 24.4 and 27.0).  One workgroup an image and slice, positions a thread over channels: [65,33,44,280] fp16
-// 182 / 280 84 and 94, [99,39,36,272] 176 / 272 119 and 126, [109,47,47,160] 276 / 160 98 and 109; [96,33,33,296] 136 / 296 95 -> 90, [54,40,40,344] 200 / 344 92 -> 89.
+// products fill no more than one round of 512 workgroups, whose tiles were cut to end together and which the sums then outlast.  us of the two launches: [32,56,56,128]
+// fp32 (51 MB) 65.9 -> 61.5, [4,64,64,1152] fp16 (38 MB) 81.7 -> 79.5, [8,112,112,256] bf16 (51 MB) 58.4 -> 55.9, [104,27,28,280] 68.6 -> 66.9, [8,48,48,256] fp32
+// (19 MB) 40.3 -> 37.8; [2,40,40,640] bf16 (4.1 MB) 17.6 and 17.9, [3,25,20,920] (2.8 MB) 20.3 and 20.5.  Sums over random 16-bit layers, ms: 8 to 17 MB, one round 116 of
+// them 3.07 and 3.06 (15 of them slower by 1 to 2.5 % of their step), more 116 of them 3.66 -> 3.51; 17 to 33 MB, one round 47 of them 1.63 -> 1.58, more 140 of them 6.13 -> 5.87; more
+// than 33 MB 163 of them 13.5 -> 12.8.
 bool dense_wide_sums_ride(const ColsumJob& j, int NO, int dtype) {
     const int es = dtype == kF32 ? 4 : 2;
     const long long N = (long long)j.B * j.P, bytes = N * j.C * es, large = 8 << 20;
-    if (bytes < large || es == 4) return bytes >= large;
+    if (bytes < large || bytes >= 2 * large || es == 4) return bytes >= large;
     const WgradPlan p = wgrad_plan(N, j.C, NO, es);
     int bm, bn;
     rows_tiles(N, j.C, NO, bm, bn);
-    const long long blocks = (long long)p.mt * p.nt * p.splits + (long long)cdiv(N, bm) * cdiv(NO, bn);
-    if (bytes < 2 * large && blocks <= 512) return false;
-    const ColsumJob r = riding_sums(j, blocks, es);
-    return r.n > 1 || 5LL * r.len / (256 >> r.lanes_log) <= 3LL * j.C;
+    return (long long)p.mt * p.nt * p.splits + (long long)cdiv(N, bm) * cdiv(NO, bn) > 512;
 }
 
 // dx[N,NO] = gy[N,M] W (+ rowbias), W stored [M][NO], and dW[M][NO] = gy^T b, in one launch; -1: not covered, or products that

@@ -38,8 +38,7 @@ inline ColsumJob colsum_plan(const void* x, float* part, int B, int P, int C, in
 
 // red: 256 * V floats of LDS (V = values per 16 bytes).  PAIRS, for jobs that say so: of every eight positions pairs, then pairs of those, before
 // they are added to the sum (as many additions): where ranges are longer because fewer workgroups ride along, a thread's chain of roundings is
-// shorter all the same (error of the sums over 100352 rows of 128 in fp32, 2-norm: 512 workgroups 1.35e-7, 192 1.8e-7, 192 in pairs 1.24e-7; over
-// 16384 of 1152 1.5e-7, 2.0e-7, 1.3e-7).
+// shorter all the same (error of the sums over 100352 rows of 128 in fp32, 2-norm: 512 workgroups 1.35e-7, 192 1.8e-7, 192 in pairs 1.24e-7).
 template <typename T, bool PAIRS = false>
 __device__ __forceinline__ void colsum_body(const ColsumJob& j, int wg, float* red) {
     constexpr int V = 16 / (int)sizeof(T);

@@ -212,9 +212,9 @@ def test_pooled_gradient_behind_the_store(oracle):
 
 
 def test_error_of_riding_sums():
-    """The sums of a large output gradient (100352 rows) are no further off in fp32 than by 512 workgroups: their chains of 25 values a thread, 8 threads,
-    16 ranges and 32 images make 2.53e-8 * sqrt(4.3e6 / 100352) in the 2-norm (a rounding's mean square for values spread over an octave, times the variances of all
-    sums that are rounded); one after the other in the 6 longer ranges that ride along, 1.9e-7."""
+    """The sums of a large output gradient (100352 rows) in fp32 are no further off than by 512 workgroups: their chains of 25 values a thread, 8 threads, 16 ranges
+    and 32 images make 2.53e-8 * sqrt(4.3e6 / 100352) in the 2-norm (a rounding's mean square for values spread over an octave, times the variances of all sums
+    that are rounded); one after the other in 6 longer ranges, 1.9e-7."""
     import pyramid_dwconv
 
     err = []
